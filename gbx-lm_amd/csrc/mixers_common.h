@@ -1,6 +1,7 @@
 // Device helpers shared by the translation units of libgbx_mixers.so.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -96,6 +97,14 @@ __host__ __device__ __forceinline__ int first_seen(int pos, int window, int chun
 // floats per (split, row, head) of the key-split partial sums of softmax attention: dv sums padded to a multiple of four (rows stay
 // 16-byte aligned), then two more pairs of which the last holds (running maximum, denominator)
 __host__ __device__ __forceinline__ int partial_width(int dv) { return (dv + 3) / 4 * 4 + 4; }
+
+// First use of something on each device (a kernel's attributes belong to the device that is current when they are set).
+struct OncePerDevice {
+  std::atomic<unsigned long long> seen{0};
+  unsigned long long bit() const { int d = 0; (void)hipGetDevice(&d); return 1ull << (d & 63); }
+  bool pending() const { return (seen.load(std::memory_order_acquire) & bit()) == 0; }
+  void done() { seen.fetch_or(bit(), std::memory_order_release); }
+};
 
 extern thread_local char g_err[512];
 int fail(int code, const char* fmt, ...);

@@ -8,6 +8,7 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -16,6 +17,11 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 // C[8 (e / 4) + 4 (l / 32) + e % 4][l % 32], e = 0..15.
 __device__ __forceinline__ f32x16 mfma_bf16(const u32x4& a, const u32x4& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// C[16 x 16] += A[16 x 32] B[32 x 16]: lane l gives A[l % 16][8 (l / 16) ..+8] and B[8 (l / 16) ..+8][l % 16] and holds
+// C[4 (l / 16) + e][l % 16], e = 0..3.
+__device__ __forceinline__ f32x4v mfma_bf16_16(const u32x4& a, const u32x4& b, const f32x4v& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 // two fp32 -> one packed bf16 pair, round to nearest even
 __device__ __forceinline__ unsigned pack2(float a, float b) {

@@ -3,18 +3,23 @@
 // 1. expert_sort_kernel: the step's (row, choice) pairs counted and bucketed by expert on the device (one workgroup, LDS counters):
 //    offsets[E + 1], the pair ids in expert order, and the table of row tiles (expert, first pair) the two products walk.  Nothing
 //    returns to the host.
-// 2. expert_up_kernel:   act[p] = silu(gate_e h) * (up_e h) for the pairs of expert e, 128 pairs x 128 hidden channels per workgroup (256
-//    where experts have no gate: the second weight fragment is then another block of 32 channels);
-// 3. expert_down_kernel: y[pair] = down_e act[p], 128 pairs x 256 output channels per workgroup.
+// 2. expert_group_kernel, first products: act[p] = silu(gate_e h) * (up_e h) (or another form) for the pairs of expert e, 256 pairs x 128 hidden
+//    channels per workgroup (256 channels where experts have no gate);
+// 3. expert_group_kernel<EXPERT_DOWN>: y[pair] = down_e act[p], 256 pairs x 256 output channels per workgroup.
 // Products are computed swapped -- C^T[channel, pair] = mfma(weight rows, activation rows) -- so a lane ends up with four consecutive
 // channels of one pair (8-byte stores) and the gate / up pair of a channel sits in the same lane for the activation.
-// Weight fragments are 16-byte loads straight from the row-major matrices (every wave has rows of its own); the activation tile,
-// which all four waves share, goes global -> registers (one chunk ahead) -> LDS once per workgroup: counters showed the version
-// in which every wave fetched it for itself waiting on L2 -> L1 traffic for more than half of its cycles.
-// The contraction runs in chunks of 64 elements (a 32-element tail when the size is not a multiple of 64); inside a chunk the lane
-// half hb takes the contiguous half [hb * C/2, (hb + 1) * C/2) and feeds it to the chunk's MFMA steps 8 elements at a time -- the
-// order of the contraction is free as long as both operands use the same one -- so a lane reads 64 contiguous bytes per chunk.
-// The grid is sized for the worst case sum_e ceil(n_e / 128) <= P / 128 + E; surplus workgroups leave at once.
+// What bounds it: a few hundred pairs per expert, so the weights are a stream of their own (1.2 GB at 128 experts of 3 x 2048 x 768: 0.24 ms)
+// beside about as much matrix-core work; both operands therefore go memory -> LDS by DMA, two stages of 64 elements, and a weight row
+// is fetched once per 256 pairs.  Eight waves, a wave 128 pairs x 64 weight rows (16 x 16 x 32 products); four phases a stage, two wave groups
+// a barrier apart, so that one group multiplies while the other reads fragments and issues requests.  Stages of 64 elements, because a row
+// piece is then a whole 128-byte line: 256 x 128 tiles with stages of 32 elements and two workgroups per CU spent their time on twice the L2
+// requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
+// Measured (us, first + second products with the sort; before: 128-pair tiles, weight fragments straight from the matrices):
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  1 027 -> 479 (548 TFLOP/s, 2.5 TB/s of weights)
+//   18 128 pairs of the same:                       794 -> 327 (3.7 TB/s)
+//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 856 -> 424
+//    8 192 pairs,   8 experts, 4096 x 2048 gated:   975 -> 472 (873 TFLOP/s)
+// The grid is sized for the worst case sum_e ceil(n_e / 256) <= P / 256 + E; surplus workgroups leave at once.
 // Steps with few pairs per expert (a batch that decodes) stream weights and little else: expert_skinny_kernel takes tiles of 32 pairs, a
 // wave per 32 output channels and no barrier.  A wave moves its own rows -- eight lanes to a row's 128 bytes, so an access touches eight
 // cache lines instead of the 64 that loads in fragment order would -- through registers (two chunks in flight) into LDS of its own.
@@ -24,8 +29,7 @@
 namespace gbxm {
 namespace {
 
-constexpr int RT = 128;         // pairs per workgroup tile
-constexpr int RS = 32;          // and per tile of the skinny form
+constexpr int RS = 32;          // pairs per tile of the skinny form
 constexpr int BROW = 128 + 16;  // LDS bytes per activation row of a chunk (+16: conflict-free 16-byte fragment reads)
 
 __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ idx, int* __restrict__ offsets, int* __restrict__ sorted,
@@ -58,6 +62,7 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
     }
     if (threadIdx.x == 0) {
       offsets[E] = run;
+      offsets[E + 1] = tiles;
       sm[3 * E] = tiles;
     }
   }
@@ -71,188 +76,197 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   for (int t = sm[3 * E] + threadIdx.x; t < n_tiles; t += 1024) tile_tab[2 * t] = -1;
 }
 
-// Workgroup ids go round-robin over the 8 XCDs, each with an L2 of its own: row tile = (id % 8) * (gridDim.x / 8) + id / 8 gives every
-// XCD a contiguous run of row tiles, so the row tiles of ONE expert, which read the same weights, run on one XCD next to each other.
-// (gridDim.x is a multiple of 8.)
-__device__ __forceinline__ int xcd_row_tile() { return (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8; }
+// Workgroup ids go round-robin over the 8 XCDs, each with an L2 of its own: every XCD gets a contiguous run of units (row tile, column
+// block), so the column blocks of ONE row tile, which read the same activation rows, and the row tiles of one expert, which read the
+// same weights, run on one XCD next to each other.  The runs are cut from the units that exist (the sort counted the tiles), not from
+// the worst case that the grid is sized for: surplus workgroups would otherwise all stand in the last XCDs' runs.
+__device__ __forceinline__ int xcd_unit(int units) {
+  const int per = (units + 7) / 8, j = blockIdx.x >> 3, u = (blockIdx.x & 7) * per + j;
+  return j < per && u < units ? u : -1;
+}
 
-// Activation tile of a chunk: 128 rows x C elements.  Thread t moves the 16-byte pieces t + 256 i (i < 4): row = piece / 8, column piece
-// = piece % 8 (only the first C / 8 column pieces exist in a 32-element tail).
-struct BTile {
-  const bf16_t* rowp[4];      // this thread's four rows (already offset by its column piece)
-  int lds_off[4];
-  int cpiece;
-  u32x4 regs[4];
-  __device__ __forceinline__ void fetch(int k0, int pieces) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) regs[i] = cpiece < pieces ? *reinterpret_cast<const u32x4*>(rowp[i] + k0) : u32x4{0, 0, 0, 0};
-  }
-  __device__ __forceinline__ void park(unsigned char* bl) const {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(bl + lds_off[i]) = regs[i];
-  }
+// (the gated activations are forms of their own: a tile's epilogue repeats its activation a hundred times over)
+enum { EXPERT_DOWN, EXPERT_UP, EXPERT_SILU, EXPERT_CLAMPED };
+
+#define GBXM_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
+// s_waitcnt: every LDS access done, at most n vector memory accesses outstanding
+__device__ __forceinline__ constexpr int lds_and_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }
+
+struct GroupArgs {
+  const bf16_t* in;            // activation rows [.][C]
+  const bf16_t* w;             // [E][N][C], gated: [E][2 N][C]
+  const int* offsets;          // [E + 1], then the number of row tiles
+  const int* sorted;
+  const int* tile_tab;
+  const float* scale;
+  bf16_t* out;
+  int N, C, E, top, cols;
+  float limit;
 };
 
-template <bool GATED>
-__global__ __launch_bounds__(256) void expert_up_kernel(const bf16_t* __restrict__ h, const bf16_t* __restrict__ first, const int* __restrict__ offsets,
-                                                       const int* __restrict__ sorted, const int* __restrict__ tile_tab, const float* __restrict__ scale,
-                                                       bf16_t* __restrict__ act, int K, int F, int top, int kind, float limit) {
-  __shared__ __attribute__((aligned(16))) unsigned char bl[RT * BROW];
-  const int bt = xcd_row_tile();
-  const int e = tile_tab[2 * bt];
-  if (e < 0) return;                                                  // (workgroup-uniform)
-  const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hb = lane >> 5;
-  const int f0 = GATED ? blockIdx.y * 128 + wave * 32 : blockIdx.y * 256 + wave * 64;
-  const bool live = f0 < F;                                           // a wave past the last channel still moves its share of the tile
-  const bool second = GATED || f0 + 32 < F;                           // (F is a multiple of 32)
-  const bf16_t* wgl = first + (static_cast<int64_t>(e) * (GATED ? 2 : 1) * F + (live ? f0 + r : 0)) * K;
-  const bf16_t* wul = GATED ? wgl + static_cast<int64_t>(F) * K : (second ? wgl + static_cast<int64_t>(32) * K : wgl);
-  BTile b;
-  b.cpiece = tid & 7;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = (tid >> 3) + 32 * i;
-    b.rowp[i] = h + static_cast<int64_t>(sorted[min(lo + row, hi - 1)] / top) * K + b.cpiece * 8;
-    b.lds_off[i] = row * BROW + b.cpiece * 16;
-  }
-  f32x16 ag[4], au[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) { ag[j] = f32x16{0}; au[j] = f32x16{0}; }
+constexpr int GR = 256;                      // pairs per row tile at most
+constexpr int GHALF = 128 * 128;             // LDS bytes of a half-tile: 64 elements of 128 rows
+constexpr int GSTAGE = 4 * GHALF;            // activation rows of wave rows 0 | 1, weight rows of wave columns 0, 1 | 2, 3
+constexpr int GLDS = 2 * GSTAGE + GR * 8;    // two stages, then the tile's pair ids and factors
+constexpr int PAST = -16;                    // byte offset (as unsigned) beyond every buffer: such lanes of a buffer load deliver zeros
 
-  auto chunk = [&](int k0, auto steps_c) {
-    constexpr int S = decltype(steps_c)::value;                         // MFMA steps of the chunk: 4 (64 elements) or 2 (32)
-    const int off = k0 + hb * (S * 8);
-    u32x4 fg[S], fu[S];                                                 // weight fragments: requested ahead of the tile hand-over
+// One tile of 32 NR pairs x 256 weight rows.  See the head of the file.
+template <int FORM, int NR>
+__device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* lds, int e, int lo, int hi, int col) {
+  constexpr bool GATED = FORM == EXPERT_SILU || FORM == EXPERT_CLAMPED;
+  constexpr int PA = (NR + 3) / 4;                                      // 16-byte activation pieces per thread and half-tile
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wc = wave & 3;
+  const int fr = lane & 15, fk = lane >> 4;
+  const int N = a.N, C = a.C, n = (C + 63) >> 6;
+  const int r0 = GATED ? col * 128 : col * 256;                         // the tile's and the wave's first output channel
+  const int c0 = r0 + wc * (GATED ? 32 : 64);
+  int* ids = reinterpret_cast<int*>(lds + 2 * GSTAGE);
+  float* factor = reinterpret_cast<float*>(ids + GR);
+  if (tid < 32 * NR) {
+    const int id = a.sorted[min(lo + tid, hi - 1)];
+    ids[tid] = id;
+    factor[tid] = FORM != EXPERT_DOWN && a.scale ? a.scale[id] : 1.f;
+  }
+  __syncthreads();
+  // DMA side: piece p = tid + 512 i of a half-tile is row p / 8, slot p % 8 of its LDS image and holds 16-byte column slot ^ ((row / 2) & 7):
+  // every group of 16 lanes that an LDS fragment read serves at a time then meets 16 different bank quads
+  const int lcol = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+  // (down: the rows of a tile are neighbours, their offsets start at the tile; up: anywhere in the step's rows)
+  const bf16_t* in0 = FORM == EXPERT_DOWN ? a.in + static_cast<int64_t>(lo) * C : a.in;
+  // (the weight rows that a wave fetches lie in one matrix: in a gated tile every wave column has 32 gate rows -- fetched by waves 0 to 3 --
+  //  over the up rows of the same channels -- waves 4 to 7; offsets start at the tile's first row)
+  const bf16_t* w0 = a.w + (static_cast<int64_t>(e) * (GATED ? 2 : 1) * N + (GATED ? wr * N : 0) + r0) * C;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(in0), 0, 0x7FFFFFFF, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w0), 0, 0x7FFFFFFF, 0x00020000);
+  int voa[2][PA], vob[2][2];
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      fg[i] = *reinterpret_cast<const u32x4*>(wgl + off + i * 8);
-      fu[i] = *reinterpret_cast<const u32x4*>(wul + off + i * 8);
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int row = h * 16 * NR + min((tid >> 3) + 64 * i, 16 * NR - 1);
+      voa[h][i] = (FORM == EXPERT_DOWN ? min(row, hi - lo - 1) : ids[row] / a.top) * C * 2 + lcol;
     }
-    __syncthreads();                                                    // the previous chunk's fragments have been read
-    b.park(bl);
-    __syncthreads();
-    const int kn = k0 + S * 16;
-    if (kn < K) b.fetch(kn, kn + 64 <= K ? 8 : 4);                      // the next chunk travels while this one is multiplied
-    if (!live) return;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x4 fb[S];
+    for (int i = 0; i < 2; ++i) {
+      const int b = h * 128 + (tid >> 3) + 64 * i;
+      vob[h][i] = min(GATED ? (b >> 6) * 32 + (b & 31) : b, N - 1 - r0) * C * 2 + lcol;
+    }
+  }
+  auto stage = [&](int t, int h) {                                      // half-tile h (0, 1 activations, 2, 3 weights) of stage t
+    const int tc = min(t, n - 1);                                       // past the end the last one again: every wait counts the same requests
+    const bool cut = tc * 64 + 32 == C && lcol >= 64;                   // the second half of a stage that the contraction does not fill
+    unsigned char* dst = lds + (t & 1) * GSTAGE + h * GHALF + wave * 1024;
+    if (h < 2) {
 #pragma unroll
-      for (int i = 0; i < S; ++i) fb[i] = *reinterpret_cast<const u32x4*>(bl + (j * 32 + r) * BROW + hb * (S * 16) + i * 16);
+      for (int i = 0; i < PA; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : voa[h][i], tc * 128, 0, 0);
+    } else {
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        ag[j] = mfma_bf16(fg[i], fb[i], ag[j]);
-        au[j] = mfma_bf16(fu[i], fb[i], au[j]);
-      }
+      for (int i = 0; i < 2; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : vob[h - 2][i], tc * 128, 0, 0);
     }
   };
-  b.fetch(0, K >= 64 ? 8 : 4);
-  int k0 = 0;
-  for (; k0 + 64 <= K; k0 += 64) chunk(k0, std::integral_constant<int, 4>{});
-  if (k0 < K) chunk(k0, std::integral_constant<int, 2>{});
-  if (!live) return;
+  const int sw = (fr >> 1) & 7, k0 = (fk ^ sw) * 16, k1 = ((4 + fk) ^ sw) * 16;
+  const int fa_off = wr * GHALF + fr * 128, fb_off = (2 + (wc >> 1)) * GHALF + ((wc & 1) * 64 + fr) * 128;
+  u32x4 fa[NR][2], fb[4][2];
+  auto read_a = [&](const unsigned char* buf, int half) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = lo + j * 32 + r;
-    if (row >= hi) continue;
-    const float sc = scale ? scale[sorted[row]] : 1.f;
-    bf16_t* ap = act + static_cast<int64_t>(row) * F + f0 + 4 * hb;
+    for (int i = half * (NR / 2); i < (half + 1) * (NR / 2); ++i) {
+      fa[i][0] = *reinterpret_cast<const u32x4*>(buf + fa_off + i * 2048 + k0);
+      fa[i][1] = *reinterpret_cast<const u32x4*>(buf + fa_off + i * 2048 + k1);
+    }
+  };
+  auto read_b = [&](const unsigned char* buf, int half) {
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      float v[4];
-      if constexpr (GATED) {
+    for (int j = half * 2; j < half * 2 + 2; ++j) {
+      fb[j][0] = *reinterpret_cast<const u32x4*>(buf + fb_off + j * 2048 + k0);
+      fb[j][1] = *reinterpret_cast<const u32x4*>(buf + fb_off + j * 2048 + k1);
+    }
+  };
+  f32x4v acc[NR][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = glu_act<true>(sc * ag[j][4 * q4 + i], sc * au[j][4 * q4 + i], kind, limit, 1.702f);
-        *reinterpret_cast<u32x2*>(ap + 8 * q4) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-      } else {
+  for (int i = 0; i < NR; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { const float z = fmaxf(sc * ag[j][4 * q4 + i], 0.f); v[i] = z * z; }
-        *reinterpret_cast<u32x2*>(ap + 8 * q4) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-        if (second) {
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4v{0};
+  auto quadrant = [&](int ah, int bh) {
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) { const float z = fmaxf(sc * au[j][4 * q4 + i], 0.f); v[i] = z * z; }
-          *reinterpret_cast<u32x2*>(ap + 32 + 8 * q4) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
-        }
+    for (int i = ah * (NR / 2); i < (ah + 1) * (NR / 2); ++i)
+#pragma unroll
+      for (int j = bh * 2; j < bh * 2 + 2; ++j) {
+        acc[i][j] = mfma_bf16_16(fb[j][0], fa[i][0], acc[i][j]);
+        acc[i][j] = mfma_bf16_16(fb[j][1], fa[i][1], acc[i][j]);
       }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto bar = [] { asm volatile("s_barrier" ::: "memory"); };
+#pragma unroll
+  for (int h = 0; h < 4; ++h) stage(0, h);
+  stage(1, 0);
+  stage(1, 1);
+  __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(2 * PA));                    // stage 0 has landed (this wave's share), two half-tiles of stage 1 may fly
+  bar();
+  if (wr == 1) bar();                                                   // the second wave group runs one barrier interval behind the first
+  for (int t = 0; t < n; ++t) {
+    const unsigned char* buf = lds + (t & 1) * GSTAGE;
+    read_b(buf, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(buf, 0);
+    stage(t + 1, 2);
+    bar();
+    quadrant(0, 0);
+    bar();
+    read_b(buf, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(buf, 1);
+    stage(t + 1, 3);
+    __builtin_amdgcn_s_waitcnt(0xC07F);                                 // lgkmcnt(0): the stage is in registers before the barrier that frees its slots
+    bar();
+    quadrant(0, 1);
+    bar();
+    stage(t + 2, 0);
+    bar();
+    quadrant(1, 1);
+    bar();
+    stage(t + 2, 1);
+    __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(2 * PA));                  // all of stage t + 1 has landed
+    bar();
+    quadrant(1, 0);
+    bar();
+  }
+  if (wr == 0) bar();                                                   // the groups' barrier counts match again
+  __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(0));                         // no LDS-DMA outlives the workgroup
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int at = wr * 16 * NR + i * 16 + fr, row = lo + at;
+    if (row >= hi) continue;
+    const float sc = factor[at];
+    bf16_t* op = a.out + static_cast<int64_t>(FORM == EXPERT_DOWN ? ids[at] : row) * N + c0 + 4 * fk;
+#pragma unroll
+    for (int j = 0; j < (GATED ? 2 : 4); ++j) {
+      if (c0 + j * 16 >= N) break;                                      // (N is a multiple of 32)
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (FORM == EXPERT_DOWN) v[q] = acc[i][j][q];
+        else if constexpr (FORM == EXPERT_UP) { const float z = fmaxf(sc * acc[i][j][q], 0.f); v[q] = z * z; }
+        else v[q] = glu_act<true>(sc * acc[i][j][q], sc * acc[i][j + 2][q], FORM == EXPERT_SILU ? GBXM_GLU_SILU : GBXM_GLU_CLAMPED_SWISH, a.limit, 1.702f);
+      }
+      *reinterpret_cast<u32x2*>(op + j * 16) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
     }
   }
 }
 
-__global__ __launch_bounds__(256) void expert_down_kernel(const bf16_t* __restrict__ act, const bf16_t* __restrict__ down, const int* __restrict__ offsets,
-                                                         const int* __restrict__ sorted, const int* __restrict__ tile_tab, bf16_t* __restrict__ y,
-                                                         int K, int F) {
-  __shared__ __attribute__((aligned(16))) unsigned char bl[RT * BROW];
-  const int bt = xcd_row_tile();
-  const int e = tile_tab[2 * bt];
-  if (e < 0) return;
-  const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hb = lane >> 5;
-  const int c0 = blockIdx.y * 256 + wave * 64;
-  const bool live = c0 < K;
-  const bool second = c0 + 32 < K;                                    // K is a multiple of 32: the wave's second channel block may not exist
-  const bf16_t* wl[2];
-  wl[0] = down + (static_cast<int64_t>(e) * K + (live ? c0 + r : 0)) * F;
-  wl[1] = second ? wl[0] + static_cast<int64_t>(32) * F : wl[0];
-  BTile b;
-  b.cpiece = tid & 7;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = (tid >> 3) + 32 * i;
-    b.rowp[i] = act + static_cast<int64_t>(min(lo + row, hi - 1)) * F + b.cpiece * 8;
-    b.lds_off[i] = row * BROW + b.cpiece * 16;
-  }
-  f32x16 acc[2][4];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[c][j] = f32x16{0};
-
-  auto chunk = [&](int f0_, auto steps_c) {
-    constexpr int S = decltype(steps_c)::value;
-    const int off = f0_ + hb * (S * 8);
-    u32x4 fa[2][S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) {
-      fa[0][i] = *reinterpret_cast<const u32x4*>(wl[0] + off + i * 8);
-      fa[1][i] = *reinterpret_cast<const u32x4*>(wl[1] + off + i * 8);
-    }
-    __syncthreads();
-    b.park(bl);
-    __syncthreads();
-    const int fn = f0_ + S * 16;
-    if (fn < F) b.fetch(fn, fn + 64 <= F ? 8 : 4);
-    if (!live) return;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x4 fb[S];
-#pragma unroll
-      for (int i = 0; i < S; ++i) fb[i] = *reinterpret_cast<const u32x4*>(bl + (j * 32 + r) * BROW + hb * (S * 16) + i * 16);
-#pragma unroll
-      for (int i = 0; i < S; ++i) {
-        acc[0][j] = mfma_bf16(fa[0][i], fb[i], acc[0][j]);
-        acc[1][j] = mfma_bf16(fa[1][i], fb[i], acc[1][j]);
-      }
-    }
-  };
-  b.fetch(0, F >= 64 ? 8 : 4);
-  int fc = 0;
-  for (; fc + 64 <= F; fc += 64) chunk(fc, std::integral_constant<int, 4>{});
-  if (fc < F) chunk(fc, std::integral_constant<int, 2>{});
-  if (!live) return;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = lo + j * 32 + r;
-    if (row >= hi) continue;
-    bf16_t* yp = y + static_cast<int64_t>(sorted[row]) * K + c0 + 4 * hb;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (c == 1 && !second) continue;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *reinterpret_cast<u32x2*>(yp + c * 32 + 8 * q4) =
-            u32x2{pack2(acc[c][j][4 * q4], acc[c][j][4 * q4 + 1]), pack2(acc[c][j][4 * q4 + 2], acc[c][j][4 * q4 + 3])};
-    }
+template <int FORM>
+__global__ __launch_bounds__(512) void expert_group_kernel(const GroupArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int u = xcd_unit(a.offsets[a.E + 1] * a.cols);
+  if (u < 0) return;                                                    // (workgroup-uniform, as everything that picks the tile)
+  const int bt = u / a.cols, col = u % a.cols;
+  const int e = a.tile_tab[2 * bt], lo = a.tile_tab[2 * bt + 1], hi = min(a.offsets[e + 1], lo + GR);
+  switch ((hi - lo + 63) / 64) {
+    case 1: group_tile<FORM, 2>(a, lds, e, lo, hi, col); break;
+    case 2: group_tile<FORM, 4>(a, lds, e, lo, hi, col); break;
+    case 3: group_tile<FORM, 6>(a, lds, e, lo, hi, col); break;
+    default: group_tile<FORM, 8>(a, lds, e, lo, hi, col); break;
   }
 }
 
@@ -265,7 +279,7 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
                                                            const int* __restrict__ sorted, const int* __restrict__ tile_tab, const float* __restrict__ scale,
                                                            bf16_t* __restrict__ out, int N, int C, int top, int kind, float limit) {
   constexpr bool TWO = FORM == SKINNY_GATED;
-  const int bt = xcd_row_tile();
+  const int bt = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;   // a contiguous run of row tiles per XCD (gridDim.x is a multiple of 8)
   const int e = tile_tab[2 * bt];
   if (e < 0) return;
   const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
@@ -350,10 +364,26 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
   }
 }
 
+template <int FORM>
+int launch_group(const GroupArgs& g, int tiles, hipStream_t s) {
+  static OncePerDevice once;                                            // (a kernel attribute belongs to the device it is set on)
+  if (once.pending()) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_group_kernel<FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, GLDS);
+    if (e != hipSuccess) return hip_fail(e, "expert_ff (grouped)");
+    once.done();
+  }
+  const int64_t units = static_cast<int64_t>(tiles) * g.cols;
+  expert_group_kernel<FORM><<<static_cast<unsigned>((units + 7) / 8 * 8), 512, GLDS, s>>>(g);
+  return after_launch("expert_ff (grouped)");
+}
+
 size_t align16(size_t n) { return (n + 15) & ~static_cast<size_t>(15); }
 constexpr int64_t MIN_PAIRS = 64;         // below this the weight-streaming row kernels read less
-constexpr int64_t SKINNY_PAIRS = 64;      // pairs per expert (on average) up to which the skinny form is taken
-int rows_of(int64_t P, int E) { return P <= SKINNY_PAIRS * E ? RS : RT; }
+// Pairs per expert (on average) up to which the skinny form is taken.  Measured at 4 | 8 | 16 | 64 pairs per expert, skinny against grouped, us:
+// 128 experts of 3 x 2048 x 768  231 | 248 | 297 | 459  against 235 | 243 | 243 | 277;  64 of 2 x 2048 x 2048  230 | 237 | 277 | 448  against
+// 254 | 256 | 258 | 276;  32 of 3 x 1024 x 512  31 | 30 | 33 | 42  against 29 | 29 | 30 | 35.
+constexpr int64_t SKINNY_PAIRS = 8;
+int rows_of(int64_t P, int E) { return P <= SKINNY_PAIRS * E ? RS : GR; }
 int tiles_of(int64_t P, int E) { return static_cast<int>((P / rows_of(P, E) + E + 7) / 8 * 8); }
 
 }  // namespace
@@ -361,10 +391,25 @@ int tiles_of(int64_t P, int E) { return static_cast<int>((P / rows_of(P, E) + E 
 size_t expert_grouped_workspace(int64_t T, int K, int F, int E, int top) {
   const int64_t P = T * top;
   if (P < MIN_PAIRS || K % 32 || F % 32 || E > 4096 || P > 0x3fffffff) return 0;
-  return align16(sizeof(int) * (E + 1)) + align16(sizeof(int) * P) + align16(sizeof(int) * 2 * tiles_of(P, E)) + align16(sizeof(bf16_t) * P * F);
+  return align16(sizeof(int) * (E + 2)) + align16(sizeof(int) * P) + align16(sizeof(int) * 2 * tiles_of(P, E)) + align16(sizeof(bf16_t) * P * F);
 }
 
 int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
+  // a tile finds its activation rows by 31-bit byte offsets: rows beyond 2 GB are steps of their own (they share nothing but the weights)
+  const int64_t most = (static_cast<int64_t>(1) << 31) / (2 * static_cast<int64_t>(a.K)) - 1;
+  if (a.act == GBXM_BF16 && a.K % 32 == 0 && a.T > most && most > 0) {
+    for (int64_t t = 0; t < a.T; t += most) {
+      gbxm_expert_args part = a;
+      part.T = a.T - t < most ? a.T - t : most;
+      part.h = static_cast<const bf16_t*>(a.h) + t * a.K;
+      part.y = static_cast<bf16_t*>(a.y) + t * a.top * a.K;
+      part.idx = a.idx + t * a.top;
+      part.scale = a.scale ? a.scale + t * a.top : nullptr;
+      const int rc = launch_expert_grouped(part, s);
+      if (rc != GBXM_OK) return rc;
+    }
+    return GBXM_OK;
+  }
   const int K = a.K, F = a.F, E = a.E, top = a.top;
   const size_t need = expert_grouped_workspace(a.T, K, F, E, top);
   if (need == 0) return GBXM_ERR_UNSUPPORTED;
@@ -376,7 +421,7 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
   const int tiles = tiles_of(P, E);
   unsigned char* w = static_cast<unsigned char*>(a.ws);
   int* offsets = reinterpret_cast<int*>(w);
-  w += align16(sizeof(int) * (E + 1));
+  w += align16(sizeof(int) * (E + 2));
   int* sorted = reinterpret_cast<int*>(w);
   w += align16(sizeof(int) * P);
   int* tile_tab = reinterpret_cast<int*>(w);
@@ -395,13 +440,12 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
                                                          static_cast<bf16_t*>(a.y), K, F, top, a.kind, a.limit);
     return after_launch("expert_ff (skinny groups)");
   }
-  if (a.kind == GBXM_EXPERT_RELU2)
-    expert_up_kernel<false><<<dim3(tiles, (F + 255) / 256), 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, K, F, top, a.kind, a.limit);
-  else
-    expert_up_kernel<true><<<dim3(tiles, (F + 127) / 128), 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, K, F, top, a.kind, a.limit);
-  expert_down_kernel<<<dim3(tiles, (K + 255) / 256), 256, 0, s>>>(act, static_cast<const bf16_t*>(a.down), offsets, sorted, tile_tab,
-                                                                   static_cast<bf16_t*>(a.y), K, F);
-  return after_launch("expert_ff (grouped)");
+  const bool gated = a.kind != GBXM_EXPERT_RELU2;
+  GroupArgs g{h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, gated ? (F + 127) / 128 : (F + 255) / 256, a.limit};
+  const int rc = !gated ? launch_group<EXPERT_UP>(g, tiles, s) : a.kind == GBXM_GLU_SILU ? launch_group<EXPERT_SILU>(g, tiles, s) : launch_group<EXPERT_CLAMPED>(g, tiles, s);
+  if (rc != GBXM_OK) return rc;
+  g = GroupArgs{act, static_cast<const bf16_t*>(a.down), offsets, sorted, tile_tab, nullptr, static_cast<bf16_t*>(a.y), K, F, E, top, (K + 255) / 256, a.limit};
+  return launch_group<EXPERT_DOWN>(g, tiles, s);
 }
 
 }  // namespace gbxm
