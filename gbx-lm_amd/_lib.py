@@ -348,6 +348,13 @@ class ExpertArgs(ctypes.Structure):
                 ("act", ctypes.c_int32), ("kind", ctypes.c_int32), ("limit", ctypes.c_float), ("ws", ctypes.c_void_p), ("ws_bytes", ctypes.c_size_t)]
 
 
+class PackedExpertsArgs(ctypes.Structure):
+    """Mirror of ``gbxm_packed_experts_args``."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "qweight", "scales", "zeros", "up_qweight", "up_scales", "up_zeros", "bias", "idx", "y")]
+                + [("pairs", ctypes.c_int64)] + [(n, ctypes.c_int32) for n in ("x_div", "E", "N", "K", "bits", "group", "f16")]
+                + [("ws", ctypes.c_void_p), ("ws_bytes", ctypes.c_size_t)])
+
+
 class RecurrentPrepArgs(ctypes.Structure):
     """Mirror of ``gbxm_recurrent_prep_args``."""
     _fields_ = [("y", ctypes.c_void_p), ("y_stride", ctypes.c_int64), ("a", ctypes.c_void_p), ("a_stride", ctypes.c_int64),
@@ -434,6 +441,8 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_glu.argtypes = [p, i64, p, i64, p, i64, i64, i32, i32, f32, f32, i32, p]
         L.gbxm_route_sigmoid_groups.argtypes = [p, p, p, p, i64, i32, i32, i32, i32, i32, f32, p]
         L.gbxm_expert_glu_act.argtypes = [p, p, p, p, p, i64, i32, i32, i32, i32, i32, i32, f32, p, sz, p]
+        L.gbxm_packed_experts_workspace.argtypes, L.gbxm_packed_experts_workspace.restype = [i64, i32, i32], sz
+        L.gbxm_packed_experts.argtypes = [ctypes.POINTER(PackedExpertsArgs), p]
         L.gbxm_expert_ff.argtypes = [ctypes.POINTER(ExpertArgs), p]
         L.gbxm_recurrent_prepare.argtypes = [ctypes.POINTER(RecurrentPrepArgs), p]
         L.gbxm_conv_tail_update.argtypes = [p, i64, p, p, i32, i32, i32, i32, p]

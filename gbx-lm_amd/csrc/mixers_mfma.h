@@ -35,4 +35,26 @@ __device__ __forceinline__ u32x2 lds_read_tr(const unsigned char* p) {
       (s16x4 __attribute__((address_space(3)))*)(__attribute__((address_space(3))) unsigned char*)p));
 }
 
+// LDS as the destination of a buffer load
+#define GBXM_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
+
+// Workgroup ids go round-robin over the 8 XCDs, each with an L2 of its own: every XCD gets a contiguous run of units (row tile, column
+// block), so the column blocks of ONE row tile, which read the same activation rows, and the row tiles of one expert, which read the
+// same weights, run on one XCD next to each other.  The runs are cut from the units that exist (the sort counted the tiles), not from
+// the worst case that the grid is sized for: surplus workgroups would otherwise all stand in the last XCDs' runs.
+__device__ __forceinline__ int xcd_unit(int units) {
+  const int per = (units + 7) / 8, j = blockIdx.x >> 3, u = (blockIdx.x & 7) * per + j;
+  return j < per && u < units ? u : -1;
+}
+
+// Pairs (row, choice) bucketed by expert on the device (mixers_moe_mfma.hip): offsets [E + 2] by bucket -- bucket E holds the pairs whose
+// index names no expert -- then the number of row tiles; the pair ids in bucket order; per row tile (of at most `rows` pairs) its bucket
+// and first place in that order (surplus tiles: bucket -1).  `tiles` bounds the tiles on the host.  `ws`: expert_buckets_bytes.
+struct ExpertBuckets {
+  int *offsets, *sorted, *tile_tab;
+  int tiles;
+};
+size_t expert_buckets_bytes(int64_t P, int rows, int E);
+int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBuckets* out, hipStream_t s);
+
 }  // namespace gbxm

@@ -32,27 +32,29 @@ namespace {
 constexpr int RS = 32;          // pairs per tile of the skinny form
 constexpr int BROW = 128 + 16;  // LDS bytes per activation row of a chunk (+16: conflict-free 16-byte fragment reads)
 
+// One workgroup; E1 = E + 1 buckets, the last for indices that name no expert.
 __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ idx, int* __restrict__ offsets, int* __restrict__ sorted,
-                                                          int* __restrict__ tile_tab, int n_tiles, int rt, int P, int E) {
-  extern __shared__ int sm[];                 // counts [E] | cursor [E] | first tile [E]
+                                                          int* __restrict__ tile_tab, int n_tiles, int rt, int P, int E1) {
+  extern __shared__ int sm[];                 // counts [E1] | cursor [E1] | first tile [E1] | tiles
   int* counts = sm;
-  int* cursor = sm + E;
-  int* first = sm + 2 * E;
-  for (int e = threadIdx.x; e < E; e += 1024) counts[e] = 0;
+  int* cursor = sm + E1;
+  int* first = sm + 2 * E1;
+  auto bucket = [&](int i) { return static_cast<int>(min(static_cast<unsigned>(idx[i]), static_cast<unsigned>(E1 - 1))); };
+  for (int e = threadIdx.x; e < E1; e += 1024) counts[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < P; i += 1024) atomicAdd(&counts[idx[i]], 1);
+  for (int i = threadIdx.x; i < P; i += 1024) atomicAdd(&counts[bucket(i)], 1);
   __syncthreads();
   if (threadIdx.x < 64) {                      // one wave: running sums of pairs and tiles, 64 experts at a time
     int run = 0, tiles = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + threadIdx.x, c = e < E ? counts[e] : 0, t = (c + rt - 1) / rt;
+    for (int e0 = 0; e0 < E1; e0 += 64) {
+      const int e = e0 + threadIdx.x, c = e < E1 ? counts[e] : 0, t = (c + rt - 1) / rt;
       int sc = c, st = t;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int uc = __shfl_up(sc, o, 64), ut = __shfl_up(st, o, 64);
         if (static_cast<int>(threadIdx.x) >= o) { sc += uc; st += ut; }
       }
-      if (e < E) {
+      if (e < E1) {
         cursor[e] = run + sc - c;
         offsets[e] = run + sc - c;
         first[e] = tiles + st - t;
@@ -61,41 +63,31 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
       tiles += __shfl(st, 63, 64);
     }
     if (threadIdx.x == 0) {
-      offsets[E] = run;
-      offsets[E + 1] = tiles;
-      sm[3 * E] = tiles;
+      offsets[E1] = run;
+      offsets[E1 + 1] = tiles;
+      sm[3 * E1] = tiles;
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < P; i += 1024) sorted[atomicAdd(&cursor[idx[i]], 1)] = i;
+  for (int i = threadIdx.x; i < P; i += 1024) sorted[atomicAdd(&cursor[bucket(i)], 1)] = i;
   __syncthreads();                             // every cursor now stands at its expert's end
-  for (int e = threadIdx.x; e < E; e += 1024) {
+  for (int e = threadIdx.x; e < E1; e += 1024) {
     const int nt = (counts[e] + rt - 1) / rt, lo = cursor[e] - counts[e];
     for (int t = 0; t < nt; ++t) { tile_tab[2 * (first[e] + t)] = e; tile_tab[2 * (first[e] + t) + 1] = lo + t * rt; }
   }
-  for (int t = sm[3 * E] + threadIdx.x; t < n_tiles; t += 1024) tile_tab[2 * t] = -1;
-}
-
-// Workgroup ids go round-robin over the 8 XCDs, each with an L2 of its own: every XCD gets a contiguous run of units (row tile, column
-// block), so the column blocks of ONE row tile, which read the same activation rows, and the row tiles of one expert, which read the
-// same weights, run on one XCD next to each other.  The runs are cut from the units that exist (the sort counted the tiles), not from
-// the worst case that the grid is sized for: surplus workgroups would otherwise all stand in the last XCDs' runs.
-__device__ __forceinline__ int xcd_unit(int units) {
-  const int per = (units + 7) / 8, j = blockIdx.x >> 3, u = (blockIdx.x & 7) * per + j;
-  return j < per && u < units ? u : -1;
+  for (int t = sm[3 * E1] + threadIdx.x; t < n_tiles; t += 1024) tile_tab[2 * t] = -1;
 }
 
 // (the gated activations are forms of their own: a tile's epilogue repeats its activation a hundred times over)
 enum { EXPERT_DOWN, EXPERT_UP, EXPERT_SILU, EXPERT_CLAMPED };
 
-#define GBXM_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
 // s_waitcnt: every LDS access done, at most n vector memory accesses outstanding
 __device__ __forceinline__ constexpr int lds_and_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }
 
 struct GroupArgs {
   const bf16_t* in;            // activation rows [.][C]
   const bf16_t* w;             // [E][N][C], gated: [E][2 N][C]
-  const int* offsets;          // [E + 1], then the number of row tiles
+  const int* offsets;          // expert_buckets' table
   const int* sorted;
   const int* tile_tab;
   const float* scale;
@@ -258,10 +250,11 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
 template <int FORM>
 __global__ __launch_bounds__(512) void expert_group_kernel(const GroupArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int u = xcd_unit(a.offsets[a.E + 1] * a.cols);
+  const int u = xcd_unit(a.offsets[a.E + 2] * a.cols);
   if (u < 0) return;                                                    // (workgroup-uniform, as everything that picks the tile)
   const int bt = u / a.cols, col = u % a.cols;
   const int e = a.tile_tab[2 * bt], lo = a.tile_tab[2 * bt + 1], hi = min(a.offsets[e + 1], lo + GR);
+  if (e >= a.E) return;                                                 // (pairs without an expert)
   switch ((hi - lo + 63) / 64) {
     case 1: group_tile<FORM, 2>(a, lds, e, lo, hi, col); break;
     case 2: group_tile<FORM, 4>(a, lds, e, lo, hi, col); break;
@@ -277,11 +270,11 @@ enum { SKINNY_DOWN = 0, SKINNY_UP = 1, SKINNY_GATED = 2 };
 template <int FORM>
 __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __restrict__ in, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
                                                            const int* __restrict__ sorted, const int* __restrict__ tile_tab, const float* __restrict__ scale,
-                                                           bf16_t* __restrict__ out, int N, int C, int top, int kind, float limit) {
+                                                           bf16_t* __restrict__ out, int N, int C, int E, int top, int kind, float limit) {
   constexpr bool TWO = FORM == SKINNY_GATED;
   const int bt = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;   // a contiguous run of row tiles per XCD (gridDim.x is a multiple of 8)
   const int e = tile_tab[2 * bt];
-  if (e < 0) return;
+  if (e < 0 || e >= E) return;
   const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, hb = lane >> 5;
   const int c0 = blockIdx.y * 128 + wave * 32;
@@ -384,14 +377,32 @@ constexpr int64_t MIN_PAIRS = 64;         // below this the weight-streaming row
 // 254 | 256 | 258 | 276;  32 of 3 x 1024 x 512  31 | 30 | 33 | 42  against 29 | 29 | 30 | 35.
 constexpr int64_t SKINNY_PAIRS = 8;
 int rows_of(int64_t P, int E) { return P <= SKINNY_PAIRS * E ? RS : GR; }
-int tiles_of(int64_t P, int E) { return static_cast<int>((P / rows_of(P, E) + E + 7) / 8 * 8); }
+
 
 }  // namespace
+
+int64_t expert_tiles(int64_t P, int rows, int E) { return (P / rows + E + 1 + 7) / 8 * 8; }
+
+size_t expert_buckets_bytes(int64_t P, int rows, int E) {
+  return align16(sizeof(int) * (E + 3)) + align16(sizeof(int) * P) + align16(sizeof(int) * 2 * expert_tiles(P, rows, E));
+}
+
+int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBuckets* out, hipStream_t s) {
+  unsigned char* w = static_cast<unsigned char*>(ws);
+  out->tiles = static_cast<int>(expert_tiles(P, rows, E));
+  out->offsets = reinterpret_cast<int*>(w);
+  w += align16(sizeof(int) * (E + 3));
+  out->sorted = reinterpret_cast<int*>(w);
+  w += align16(sizeof(int) * P);
+  out->tile_tab = reinterpret_cast<int*>(w);
+  expert_sort_kernel<<<1, 1024, (3 * (E + 1) + 1) * sizeof(int), s>>>(idx, out->offsets, out->sorted, out->tile_tab, out->tiles, rows, P, E + 1);
+  return after_launch("expert buckets");
+}
 
 size_t expert_grouped_workspace(int64_t T, int K, int F, int E, int top) {
   const int64_t P = T * top;
   if (P < MIN_PAIRS || K % 32 || F % 32 || E > 4096 || P > 0x3fffffff) return 0;
-  return align16(sizeof(int) * (E + 2)) + align16(sizeof(int) * P) + align16(sizeof(int) * 2 * tiles_of(P, E)) + align16(sizeof(bf16_t) * P * F);
+  return expert_buckets_bytes(P, rows_of(P, E), E) + align16(sizeof(bf16_t) * P * F);
 }
 
 int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
@@ -418,31 +429,26 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
        reinterpret_cast<uintptr_t>(a.ws)) % 16)
     return GBXM_ERR_UNSUPPORTED;
   const int P = static_cast<int>(a.T * top);
-  const int tiles = tiles_of(P, E);
-  unsigned char* w = static_cast<unsigned char*>(a.ws);
-  int* offsets = reinterpret_cast<int*>(w);
-  w += align16(sizeof(int) * (E + 2));
-  int* sorted = reinterpret_cast<int*>(w);
-  w += align16(sizeof(int) * P);
-  int* tile_tab = reinterpret_cast<int*>(w);
-  w += align16(sizeof(int) * 2 * tiles);
-  bf16_t* act = reinterpret_cast<bf16_t*>(w);
-  expert_sort_kernel<<<1, 1024, (3 * E + 1) * sizeof(int), s>>>(a.idx, offsets, sorted, tile_tab, tiles, rows_of(P, E), P, E);
+  ExpertBuckets k;
+  int rc = expert_buckets(a.idx, P, rows_of(P, E), E, a.ws, &k, s);
+  if (rc != GBXM_OK) return rc;
+  const int *offsets = k.offsets, *sorted = k.sorted, *tile_tab = k.tile_tab, tiles = k.tiles;
+  bf16_t* act = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(a.ws) + expert_buckets_bytes(P, rows_of(P, E), E));
   const bf16_t* h = static_cast<const bf16_t*>(a.h);
   const bf16_t* first = static_cast<const bf16_t*>(a.first);
   if (rows_of(P, E) == RS) {
     const dim3 up(tiles, (F + 127) / 128), dn(tiles, (K + 127) / 128);
     if (a.kind == GBXM_EXPERT_RELU2)
-      expert_skinny_kernel<SKINNY_UP><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, top, a.kind, a.limit);
+      expert_skinny_kernel<SKINNY_UP><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
     else
-      expert_skinny_kernel<SKINNY_GATED><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, top, a.kind, a.limit);
+      expert_skinny_kernel<SKINNY_GATED><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
     expert_skinny_kernel<SKINNY_DOWN><<<dn, 256, 0, s>>>(act, static_cast<const bf16_t*>(a.down), offsets, sorted, tile_tab, nullptr,
-                                                         static_cast<bf16_t*>(a.y), K, F, top, a.kind, a.limit);
+                                                         static_cast<bf16_t*>(a.y), K, F, E, top, a.kind, a.limit);
     return after_launch("expert_ff (skinny groups)");
   }
   const bool gated = a.kind != GBXM_EXPERT_RELU2;
   GroupArgs g{h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, gated ? (F + 127) / 128 : (F + 255) / 256, a.limit};
-  const int rc = !gated ? launch_group<EXPERT_UP>(g, tiles, s) : a.kind == GBXM_GLU_SILU ? launch_group<EXPERT_SILU>(g, tiles, s) : launch_group<EXPERT_CLAMPED>(g, tiles, s);
+  rc = !gated ? launch_group<EXPERT_UP>(g, tiles, s) : a.kind == GBXM_GLU_SILU ? launch_group<EXPERT_SILU>(g, tiles, s) : launch_group<EXPERT_CLAMPED>(g, tiles, s);
   if (rc != GBXM_OK) return rc;
   g = GroupArgs{act, static_cast<const bf16_t*>(a.down), offsets, sorted, tile_tab, nullptr, static_cast<bf16_t*>(a.y), K, F, E, top, (K + 255) / 256, a.limit};
   return launch_group<EXPERT_DOWN>(g, tiles, s);

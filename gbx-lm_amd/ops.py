@@ -6,6 +6,7 @@ gbx_lm/models/quantized_linear_gba.py:195-203): same argument names and meaning.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from typing import Optional
 
@@ -389,8 +390,9 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     QuantizedSwitchLinear calls it (gbx_lm/models/switch_layers.py:78-92), plus the optional ``bias[indices]``.
 
     x: [..., 1, 1, K] or [..., k, 1, K]; rhs_indices: [..., k] -> [..., k, 1, N].  Few (token, slot) pairs run the
-    expert-indexed decode GEMV in ONE launch; many pairs are grouped by expert on the host (one batched GEMM per
-    expert present -- the reference's ``sorted_indices`` hint needs no special handling)."""
+    expert-indexed decode GEMV in ONE launch; many pairs are bucketed by expert on the device and run as tiles of the matrix cores
+    (``_packed_experts``); what neither takes is grouped on the host (one batched GEMM per expert present).  The reference's
+    ``sorted_indices`` hint needs no special handling."""
     if not transpose:
         raise NotImplementedError("gather_quantized_matmul supports transpose=True only (the reference's only use)")
     for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases"), (rhs_indices, "rhs_indices")):
@@ -420,9 +422,14 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     xr = x.reshape(-1, K).contiguous()                  # [tokens, K] (shared) or [pairs, K]
     idx = rhs_indices.reshape(-1)
-    y = torch.empty((pairs, N), dtype=x.dtype, device=x.device)
     max_k = 512 * (64 if bits == 2 else 32)
-    if pairs <= 64 and K % 128 == 0 and K <= max_k:
+    few = pairs <= 64 and K % 128 == 0 and K <= max_k
+    if not few and pairs:
+        y = _packed_experts(xr, (w, scales, biases), None, bias, idx, k if shared else 1, E, N, K, bits, group_size)
+        if y is not None:
+            return y.reshape(*lead, k, 1, N)
+    y = torch.empty((pairs, N), dtype=x.dtype, device=x.device)
+    if few:
         idx32 = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         _lib.check(_lib.lib().gbx_gather_qlinear_forward(
             xr.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias.data_ptr() if bias is not None else None,
@@ -431,7 +438,7 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     else:                                               # grouped by expert (one host sync for the expert list)
         if torch.cuda.is_current_stream_capturing():
             raise NotCapturable(f"gather_quantized_matmul: {pairs} (token, expert) pairs / K={K} need the host-grouped path, which "
-                               "cannot be captured into a HIP graph (the expert-indexed launch covers <= 64 pairs, K % 128 == 0)")
+                               "cannot be captured into a HIP graph (the expert-indexed launches need K % 128 == 0)")
         ar = torch.arange(pairs, device=x.device)
         rows = ar // k if shared else ar
         for e in torch.unique(idx).tolist():
@@ -441,13 +448,43 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     return y.reshape(*lead, k, 1, N)
 
 
+def _packed_experts(xr: torch.Tensor, first, second, bias, idx: torch.Tensor, x_div: int, E: int, N: int, K: int, bits: int, group_size: int):
+    """Rows [pairs, N] of the chosen experts' products over many (token, slot) pairs (gbxm_packed_experts): ``first`` = (qweight, scales,
+    zeros) [E, ...]; with ``second`` alike, silu(first) * second.  None where the launch does not serve the shapes."""
+    L = _lib.mixers()
+    pairs = idx.numel()
+    nbytes = L.gbxm_packed_experts_workspace(pairs, K, E)
+    if not nbytes:
+        return None
+    idx = (idx if idx.dtype == torch.int32 else idx.to(torch.int32)).contiguous()
+    y = torch.empty((pairs, N), dtype=xr.dtype, device=xr.device)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=xr.device)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    a = _lib.PackedExpertsArgs(xr.data_ptr(), *(t.data_ptr() for t in first), *(ptr(t) for t in (second or (None, None, None))), ptr(bias), idx.data_ptr(),
+                               y.data_ptr(), pairs, x_div, E, N, K, bits, group_size, int(xr.dtype == torch.float16), ws.data_ptr(), nbytes)
+    rc = L.gbxm_packed_experts(ctypes.byref(a), _stream_ptr(xr.device))
+    if rc == _lib.GBX_ERR_UNSUPPORTED:
+        return None
+    _lib.check_mixers(rc)
+    return y
+
+
 def gather_swiglu(x: torch.Tensor, gate, up, rhs_indices: torch.Tensor):
-    """``silu(gate_proj(x, indices)) * up_proj(x, indices)`` of SwitchGLU for a decode-sized index set in ONE expert-indexed
-    launch (gbx_gather_swiglu_forward); ``gate`` / ``up`` are QuantizedSwitchLinear modules.  Returns None when the shapes
-    are outside that launch (the caller then runs the three ops)."""
+    """``silu(gate_proj(x, indices)) * up_proj(x, indices)`` of SwitchGLU in ONE expert-indexed launch for a decode-sized index set
+    (gbx_gather_swiglu_forward) or over bucketed pairs (gbxm_packed_experts); ``gate`` / ``up`` are QuantizedSwitchLinear modules.
+    Returns None when the shapes are outside both (the caller then runs the three ops)."""
     K, N, k = x.shape[-1], gate.output_dims, rhs_indices.shape[-1]
     pairs = rhs_indices.numel()
     max_k = 512 * (64 if gate.bits == 2 else 32)
+    if (x.is_cuda and x.dtype in _DT and (pairs > 64 or K > max_k) and pairs and x.shape[-2] == 1 and x.shape[-3] in (1, k)
+            and (gate.bits, gate.group_size, gate.output_dims, gate.input_dims) == (up.bits, up.group_size, up.output_dims, up.input_dims)
+            and gate.num_experts == up.num_experts and gate.input_dims == K
+            and getattr(gate, "bias", None) is None and getattr(up, "bias", None) is None
+            and gate.scales.dtype == x.dtype and up.scales.dtype == x.dtype and gate.zeros.dtype == x.dtype and up.zeros.dtype == x.dtype
+            and all(t.is_contiguous() for m in (gate, up) for t in (m.qweight, m.scales, m.zeros))):
+        y = _packed_experts(x.reshape(-1, K).contiguous(), (gate.qweight, gate.scales, gate.zeros), (up.qweight, up.scales, up.zeros), None,
+                            rhs_indices.reshape(-1), k if x.shape[-3] == 1 else 1, gate.num_experts, N, K, gate.bits, gate.group_size)
+        return None if y is None else y.reshape(*rhs_indices.shape[:-1], k, 1, N)
     if not (x.is_cuda and x.dtype in _DT and pairs <= 64 and K % 128 == 0 and K <= max_k and x.shape[-2] == 1 and x.shape[-3] in (1, k)
             and (gate.bits, gate.group_size, gate.output_dims, gate.input_dims) == (up.bits, up.group_size, up.output_dims, up.input_dims)
             and getattr(gate, "bias", None) is None and getattr(up, "bias", None) is None

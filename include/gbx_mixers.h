@@ -202,6 +202,25 @@ typedef struct {
 } gbxm_expert_args;
 int gbxm_expert_ff(const gbxm_expert_args* a, void* stream);
 
+/* Routed experts over packed weights (fields of `bits` = 2, 3, 4 bits, little-endian bit streams [E][N][K * bits / 32]; w = scale * q + zero, scale
+ * and zero [E][N][K / group] in the activation type: bf16, or fp16 with `f16`), K a multiple of 128:
+ *   y[p] = x[p / x_div] . w[idx[p]]^T (+ bias[idx[p]])                     up_qweight null
+ *   y[p] = silu(x . w[idx[p]]^T) * (x . up[idx[p]]^T), each result rounded  otherwise (qweight is the gate; no bias)
+ * for p < pairs.  For many pairs: they are bucketed by expert on the device.  An index outside 0 .. E - 1 gives a row of NaN. */
+typedef struct {
+  const void* x;
+  const uint32_t* qweight; const void *scales, *zeros;
+  const uint32_t* up_qweight; const void *up_scales, *up_zeros;
+  const void* bias;             /* [E][N] or null */
+  const int32_t* idx;
+  void* y;                      /* [pairs][N] */
+  int64_t pairs;
+  int32_t x_div, E, N, K, bits, group, f16;
+  void* ws; size_t ws_bytes;    /* gbxm_packed_experts_workspace (0: shape not served) */
+} gbxm_packed_experts_args;
+size_t gbxm_packed_experts_workspace(int64_t pairs, int32_t K, int32_t E);
+int gbxm_packed_experts(const gbxm_packed_experts_args* a, void* stream);
+
 /* ---- recurrent mixers: a decayed matrix state per head (gbx-lm_amd/models/recurrent_mixers.py) ---- */
 
 /* Row preparation, everything in fp32.  y rows hold q (G*dk) | k (G*dk) | v (H*dv) at off_q / off_k / off_v and optionally beta (H) at

@@ -1,0 +1,114 @@
+"""Routed experts over packed weights for many (row, choice) pairs (csrc/mixers_moe_packed.hip) at the edges of their tiles: experts with no
+pair, one, and one less / as many / one more than 16, 32 and 64; output rows off the 64 / 128 / 256 grid; contractions of one, two, three
+chunks; every width, group size and activation type.  Reference: float64 from the oracle's unpacking.  Tolerance: fields and activations
+enter exactly, sums are fp32 (K 2^-24 of the terms' absolute sum with the offset C = 128 or 1024 in every field), the result is rounded once:
+2^-8 (bf16) / 2^-11 (fp16) of its size."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+COUNTS = [1, 0, 15, 16, 17, 31, 32, 33, 63, 64, 65, 130]
+
+
+def make(oracle, E, N, K, bits, g, dt, seed):
+    rng = np.random.default_rng(seed)
+    qw = rng.integers(0, 2**32, (E, N, K * bits // 32), dtype=np.uint32)
+    qmax = float((1 << bits) - 1)
+    s = torch.from_numpy(((rng.random((E, N, K // g)) + 0.5) * (0.04 / qmax)).astype(np.float32)).to(dt)
+    z = (-s.float() * qmax / 2.0 + torch.from_numpy(rng.standard_normal(s.shape).astype(np.float32)) * 0.1 * s.float()).to(dt)
+    q = torch.from_numpy(np.stack([oracle.unpack(qw[e], bits) for e in range(E)]).astype(np.float64))
+    w = q * s.double().repeat_interleave(g, -1) + z.double().repeat_interleave(g, -1)
+    mag = (q + (128 if dt == torch.bfloat16 else 1024)) * s.double().repeat_interleave(g, -1) + z.double().abs().repeat_interleave(g, -1)
+    return torch.from_numpy(qw.view(np.int32)).view(torch.uint32).to(DEV), s.to(DEV), z.to(DEV), w.to(DEV), mag.to(DEV)
+
+
+def indices(seed):
+    idx = torch.cat([torch.full((n,), e) for e, n in enumerate(COUNTS)])
+    return idx[torch.randperm(idx.numel(), generator=torch.Generator().manual_seed(seed))]
+
+
+def rows(x, w, idx):
+    y = torch.empty((x.shape[0], w.shape[1]), dtype=torch.float64, device=DEV)
+    for e in idx.unique().tolist():
+        at = idx == e
+        y[at] = x[at] @ w[e].t()
+    return y
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_tiles_of_every_height(oracle, bits, g, dt):
+    from gbx_lm_amd import ops
+    E, eps = len(COUNTS), 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    for N, K in ((200, 128), (72, 384), (257, 256)):
+        qw, s, z, w, mag = make(oracle, E, N, K, bits, g, dt, seed=bits + g + N)
+        idx = indices(N).to(DEV)
+        P = idx.numel()
+        gen = torch.Generator(device=DEV).manual_seed(N)
+        x = torch.randn((P, 1, 1, K), device=DEV, generator=gen).to(dt)
+        bias = (torch.randn((E, N), device=DEV, generator=gen) * 0.1).to(dt)
+        want, room = rows(x.view(P, K).double(), w, idx), K * 2.0 ** -24 * rows(x.view(P, K).double().abs(), mag, idx)
+        got = ops.gather_quantized_matmul(x, qw, s, z, idx[:, None], group_size=g, bits=bits).view(P, N).double()
+        assert bool(((got - want).abs() <= eps * want.abs() + room + 1e-7).all()), (N, K)
+        got = ops.gather_quantized_matmul(x, qw, s, z, idx[:, None], group_size=g, bits=bits, bias=bias).view(P, N).double()
+        want = want + bias.double()[idx]                            # (the product is rounded in front of the bias, the sum once more)
+        assert bool(((got - want).abs() <= 2 * eps * (want.abs() + bias.double()[idx].abs()) + room + 1e-7).all()), (N, K)
+
+
+@pytest.mark.parametrize("bits,g", [(2, 64), (3, 128), (3, 32), (4, 128)])
+def test_gated_pairs_round_like_the_three_operations(oracle, bits, g):
+    """silu(gate) * up of shared rows (several choices per row) equals the separate products and ``ops.swiglu`` bit for bit."""
+    from gbx_lm_amd import ops
+    from gbx_lm_amd.models.switch_layers import QuantizedSwitchLinear
+    E, N, K, T, k = 7, 200, 256, 90, 3
+    mods = []
+    for seed in (1, 2):
+        qw, s, z, _, _ = make(oracle, E, N, K, bits, g, torch.bfloat16, seed)
+        m = QuantizedSwitchLinear(K, N, E, bias=False, group_size=g, bits=bits)
+        m._buffers["qweight"], m._buffers["scales"], m._buffers["zeros"] = qw, s, z
+        mods.append(m)
+    x = torch.randn((T, 1, 1, K), device=DEV).to(torch.bfloat16)
+    idx = torch.rand((T, E), device=DEV).topk(k, -1).indices.to(torch.int32)
+    got = ops.gather_swiglu(x, mods[0], mods[1], idx)
+    want = ops.swiglu(mods[0](x, idx), mods[1](x, idx))
+    assert got.shape == want.shape == (T, k, 1, N)
+    assert torch.equal(got, want)
+
+
+def test_index_without_an_expert_gives_no_number(oracle):
+    from gbx_lm_amd import ops
+    E, N, K = 5, 72, 128
+    qw, s, z, w, _ = make(oracle, E, N, K, 4, 64, torch.bfloat16, 9)
+    idx = torch.arange(100, device=DEV) % E
+    x = torch.randn((100, 1, 1, K), device=DEV).to(torch.bfloat16)
+    good = ops.gather_quantized_matmul(x, qw, s, z, idx[:, None], group_size=64, bits=4).view(100, N)
+    bad = idx.clone()
+    bad[3], bad[70] = E, -1
+    got = ops.gather_quantized_matmul(x, qw, s, z, bad[:, None], group_size=64, bits=4).view(100, N)
+    keep = bad == idx
+    assert torch.isnan(got[~keep].float()).all() and torch.equal(got[keep], good[keep])
+
+
+def test_replays_in_a_graph(oracle):
+    """A step whose pairs were grouped on the host could not be captured; the launches can."""
+    from gbx_lm_amd import graphs, ops
+    E, N, K = 6, 256, 256
+    qw, s, z, _, _ = make(oracle, E, N, K, 4, 128, torch.bfloat16, 4)
+    x = torch.randn((96, 1, 1, K), device=DEV).to(torch.bfloat16)
+    idx = torch.zeros((96, 1), dtype=torch.int32, device=DEV)
+    run = lambda: ops.gather_quantized_matmul(x, qw, s, z, idx, group_size=128, bits=4)
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with graphs.capture(graph):
+        y = run()
+    for seed in range(4):
+        gen = torch.Generator(device=DEV).manual_seed(seed)
+        x.copy_(torch.randn(x.shape, device=DEV, generator=gen))
+        idx.copy_(torch.randint(0, E, idx.shape, device=DEV, generator=gen))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, run())
