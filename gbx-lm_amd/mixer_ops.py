@@ -17,7 +17,7 @@ _DT = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32}
 
 
 def _stream(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def _act(t: torch.Tensor, name: str) -> int:

@@ -124,10 +124,11 @@ class QuantizedLinear(nn.Module):
 
     # ------------------------------------------------------------------ forward (:179-207)
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if self.scales is None or self.zeros is None:
+        scales, zeros = self.scales, self.zeros
+        if scales is None or zeros is None:
             raise RuntimeError("QuantizedLinear: double-quantised statistics not expanded; call prepare_scales_zeros")
         # channel_scale / q_perm are intentionally NOT applied (commented out in the reference, :187-192)
-        return ops.quantized_matmul(x, self.qweight, scales=self.scales, biases=self.zeros, transpose=True,
+        return ops.quantized_matmul(x, self.qweight, scales=scales, biases=zeros, transpose=True,
                                     group_size=self.group_size, bits=self.bits, bias=self.bias)
 
     # ------------------------------------------------------------------ loader hooks (:210-324)

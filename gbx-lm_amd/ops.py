@@ -18,7 +18,8 @@ _DT = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16, torch.float32
 
 
 def _stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of the device's current stream (the raw handle: building a Stream object around it costs 2 us a launch)."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def _require_cuda(t: torch.Tensor, name: str) -> None:
@@ -185,45 +186,58 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """
     if not transpose:
         raise NotImplementedError("quantized_matmul(transpose=False) is not on the QuantizedLinear path")
-    for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases")):
-        _require_cuda(t, nm)
-    if x.dtype not in (torch.float16, torch.bfloat16):
-        raise ValueError(f"activations must be float16 or bfloat16, got {x.dtype}")
+    if not (x.is_cuda and w.is_cuda and scales.is_cuda and biases.is_cuda):
+        for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases")):
+            _require_cuda(t, nm)
+    dt = x.dtype
+    act = _DT.get(dt)
+    if act is None:
+        raise ValueError(f"activations must be float16 or bfloat16, got {dt}")
     if w.dtype not in (torch.uint32, torch.int32):
         raise ValueError(f"packed weight must be uint32, got {w.dtype}")
-    if w.dim() != 2 or scales.dim() != 2 or biases.shape != scales.shape:
+    wshape, sshape, xshape = w.shape, scales.shape, x.shape
+    if len(wshape) != 2 or len(sshape) != 2 or biases.shape != sshape:
         raise ValueError("w must be [N, K*bits/32]; scales/biases must be [N, K/group_size]")
-    n = w.shape[0]
-    if (w.shape[1] * 32) % bits:
-        raise ValueError(f"packed row of {w.shape[1]} words is not a whole number of {bits}-bit fields")
-    k = w.shape[1] * 32 // bits
-    if x.shape[-1] != k:
-        raise ValueError(f"last dim of x ({x.shape[-1]}) != input_dims ({k}) implied by w and bits")
-    if k % group_size or scales.shape != (n, k // group_size):
-        raise ValueError(f"scales must be [{n}, {k}//{group_size}], got {tuple(scales.shape)}")
-    if scales.dtype != x.dtype:
-        scales = scales.to(x.dtype)
-    if biases.dtype != x.dtype:
-        biases = biases.to(x.dtype)
+    n, words = wshape
+    if (words * 32) % bits:
+        raise ValueError(f"packed row of {words} words is not a whole number of {bits}-bit fields")
+    k = words * 32 // bits
+    if xshape[-1] != k:
+        raise ValueError(f"last dim of x ({xshape[-1]}) != input_dims ({k}) implied by w and bits")
+    if k % group_size or sshape[0] != n or sshape[1] != k // group_size:
+        raise ValueError(f"scales must be [{n}, {k}//{group_size}], got {tuple(sshape)}")
+    if scales.dtype != dt:
+        scales = scales.to(dt)
+    if biases.dtype != dt:
+        biases = biases.to(dt)
+    src = (w, scales, biases)                           # the caller's tensor objects: identity of a resident dense image
     if bias is not None:
         _require_cuda(bias, "bias")
         if bias.shape != (n,):
             raise ValueError(f"bias must be [{n}]")
-        if bias.dtype != x.dtype:
-            bias = bias.to(x.dtype)
+        if bias.dtype != dt:
+            bias = bias.to(dt)
         bias = bias.contiguous()
-    x2 = x.reshape(-1, k).contiguous()
+    x2 = (x if len(xshape) == 2 else x.reshape(-1, k)).contiguous()
     m = x2.shape[0]
-    src = (w, scales, biases)                           # the caller's tensor objects: identity of a resident dense image
-    w = w.contiguous()
-    scales = scales.contiguous()
-    biases = biases.contiguous()
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
     if out is None:
-        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    elif out.shape != (m, n) or out.dtype != x.dtype or not out.is_contiguous():
+        out = x2.new_empty((m, n))
+    elif out.shape != (m, n) or out.dtype != dt or not out.is_contiguous():
         raise ValueError("out must be a contiguous [M, N] tensor of the activation dtype")
+    bias_ptr = bias.data_ptr() if bias is not None else None
     L = _lib.lib()
+    # scratch: decode batches / short prompts split k across workgroups, long prompts dequantise once
     need = L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) if (2 <= m <= 32 or m > 64) else 0
+    if m < 256:                                         # no resident images at these sizes: nothing more to decide
+        args = (x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits, group_size, act)
+        if need:
+            ws = torch.empty((need,), dtype=torch.uint8, device=x.device)      # caller-owned (caching allocator: no sync)
+            rc = L.gbx_qlinear_forward_ws(*args, ws.data_ptr(), need, _stream_ptr(x.device))
+        else:
+            rc = L.gbx_qlinear_forward(*args, _stream_ptr(x.device))
+        _lib.check(rc)
+        return out if len(xshape) == 2 else out.reshape(*xshape[:-1], n)
     dense_path = m >= 1024 and need >= n * k * 2 and 31 <= L.gbx_qlinear_kernel_id(m, n, k, bits, group_size, 1) <= 33
     cacheable = (dense_path and _dense_cache.budget >= n * k * 2 and m <= 61440 and all(a is b for a, b in zip((w, scales, biases), src))
                  and not torch.cuda.is_current_stream_capturing())
@@ -256,19 +270,19 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                                         m, n, k, _DT[x.dtype], scratch.data_ptr() if part else None, part, _stream_ptr(x.device))
             if rc == _lib.GBX_OK:
                 return out.reshape(*x.shape[:-1], n)
-    if need:                                            # decode batches / short prompts: k split across workgroups; long prompts: dequantise once
-        ws = torch.empty((need,), dtype=torch.uint8, device=x.device)      # caller-owned scratch (caching allocator: no sync)
+    if need:
+        ws = torch.empty((need,), dtype=torch.uint8, device=x.device)
         rc = L.gbx_qlinear_forward_ws(
             x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(),
-            bias.data_ptr() if bias is not None else None, out.data_ptr(),
-            m, n, k, bits, group_size, _DT[x.dtype], ws.data_ptr(), need, _stream_ptr(x.device))
+            bias_ptr, out.data_ptr(),
+            m, n, k, bits, group_size, act, ws.data_ptr(), need, _stream_ptr(x.device))
     else:
         rc = L.gbx_qlinear_forward(
             x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(),
-            bias.data_ptr() if bias is not None else None, out.data_ptr(),
-            m, n, k, bits, group_size, _DT[x.dtype], _stream_ptr(x.device))
+            bias_ptr, out.data_ptr(),
+            m, n, k, bits, group_size, act, _stream_ptr(x.device))
     _lib.check(rc)
-    return out.reshape(*x.shape[:-1], n)
+    return out.reshape(*xshape[:-1], n)
 
 
 def unpack(w: torch.Tensor, bits: int) -> torch.Tensor:
