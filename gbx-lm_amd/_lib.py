@@ -295,7 +295,7 @@ def check(rc: int) -> None:
 # --------------------------------------------------------------------------- libgbx_mixers.so (include/gbx_mixers.h)
 _MSO = os.path.join(_CSRC, "libgbx_mixers.so")
 _mlib = None
-GBXM_BF16, GBXM_F32 = 1, 2
+GBXM_BF16, GBXM_F32, GBXM_F16 = 1, 2, 3
 
 
 class WindowAttnArgs(ctypes.Structure):
@@ -441,6 +441,8 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_glu.argtypes = [p, i64, p, i64, p, i64, i64, i32, i32, f32, f32, i32, p]
         L.gbxm_route_sigmoid_groups.argtypes = [p, p, p, p, i64, i32, i32, i32, i32, i32, f32, p]
         L.gbxm_expert_glu_act.argtypes = [p, p, p, p, p, i64, i32, i32, i32, i32, i32, i32, f32, p, sz, p]
+        L.gbxm_log_softmax_workspace.argtypes, L.gbxm_log_softmax_workspace.restype = [i64, i32], sz
+        L.gbxm_log_softmax.argtypes = [p, p, i64, i32, i32, p, sz, p]
         L.gbxm_packed_experts_workspace.argtypes, L.gbxm_packed_experts_workspace.restype = [i64, i32, i32], sz
         L.gbxm_packed_experts.argtypes = [ctypes.POINTER(PackedExpertsArgs), p]
         L.gbxm_expert_ff.argtypes = [ctypes.POINTER(ExpertArgs), p]

@@ -213,6 +213,7 @@ class BatchScheduler:
         """Generate for several prompts at once: one ragged prompt step, then one token per live sequence and step.  A sequence that
         samples a stop token (or reaches ``max_tokens``) leaves the batch and frees its slot; the others go on.  ``sampler`` maps
         log-probabilities [n, vocab] to token ids [n] (default: greedy), as in ``generate_step``."""
+        from .mixer_ops import log_probabilities
         sampler = sampler or (lambda lp: torch.argmax(lp, dim=-1))
         stop = set(stop_tokens)
         ids = [object() for _ in prompts]
@@ -221,7 +222,7 @@ class BatchScheduler:
         feed = {i: list(prompts[i]) for i in live}
         while live:
             logits = self.step([(ids[i], feed[i]) for i in live])
-            logprobs = logits - torch.logsumexp(logits, dim=-1, keepdim=True)
+            logprobs = log_probabilities(logits)
             toks = sampler(logprobs).reshape(-1).tolist()
             nxt = []
             for i, t in zip(live, toks):

@@ -1,6 +1,7 @@
 // Row kernels of ragged steps: embedding, segment norms, the branch-norm residual update, the last norm, the router and the
 // append to the window rings.  One workgroup per row; statistics in fp32 with a fixed summation order, so a row's result does
 // not depend on which other rows share the step.
+#include <type_traits>
 #include "mixers_common.h"
 
 namespace gbxm {
@@ -29,6 +30,161 @@ __global__ __launch_bounds__(NT) void embed_kernel(const T* __restrict__ table, 
     x[t * width + c] = v;
     if (h) h[t * h_row + c] = from_f32<T>(v);
   }
+}
+
+// Logits -> log-probabilities: out = x - lse, lse = log sum exp x in fp32, rounded to the row's type before the subtraction.  A workgroup of 16
+// waves per row; a row's first 128 KB stay in registers between the three passes (maximum, sum, result), what lies beyond is read again
+// from the L2 that the first pass filled.  Rows with an infinite maximum are summed unshifted, so that they come out as the definition has it.
+// A few long rows are bound by the vector instructions of the few CUs that hold them (one row of 128 256 bf16 logits: 22 us): slices of a row are
+// then workgroups of their own that leave (maximum, sum) in the first of two launches and write their slice in the second.
+// Replaces torch's logsumexp and subtraction, some ten launches: 1 x 32 000 fp32 40 -> 7 us, 32 x 32 000 fp32 40 -> 8, 1 x 128 256 bf16 62 -> 12.
+constexpr int LSM_NT = 1024, LSM_VR = 8;
+
+template <typename T> __device__ __forceinline__ float lsm_get(const uint4& v, int j) {
+  const unsigned w[4] = {v.x, v.y, v.z, v.w};
+  if constexpr (sizeof(T) == 4) return __uint_as_float(w[j]);
+  else {
+    const unsigned short h = static_cast<unsigned short>(w[j >> 1] >> (16 * (j & 1)));
+    if constexpr (std::is_same<T, _Float16>::value) return static_cast<float>(__builtin_bit_cast(_Float16, h));
+    else return to_f32(static_cast<bf16_t>(h));
+  }
+}
+// (a plain cast: rounds to nearest even and keeps NaN and infinities)
+template <typename T> __device__ __forceinline__ unsigned short lsm_bits(float f) {
+  if constexpr (std::is_same<T, _Float16>::value) return __builtin_bit_cast(unsigned short, static_cast<_Float16>(f));
+  else return __builtin_bit_cast(unsigned short, static_cast<__bf16>(f));
+}
+template <typename T> __device__ __forceinline__ float lsm_round(float f) {
+  if constexpr (sizeof(T) == 4) return f;
+  else {
+    const unsigned short h = lsm_bits<T>(f);
+    if constexpr (std::is_same<T, _Float16>::value) return static_cast<float>(__builtin_bit_cast(_Float16, h));
+    else return to_f32(static_cast<bf16_t>(h));
+  }
+}
+
+constexpr int LSM_SLICE = 8192;                              // logits per workgroup of the sliced form
+
+// (maximum, sum of exponentials against it or against 0 where it is infinite) of one slice
+template <typename T>
+__global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n) {
+  __shared__ float red[4];
+  const T* row = x + static_cast<int64_t>(blockIdx.y) * n;
+  const int lo = blockIdx.x * LSM_SLICE, hi = min(lo + LSM_SLICE, n);
+  float v[LSM_SLICE / 256], m = -INFINITY, s = 0.f;
+#pragma unroll
+  for (int i = 0; i < LSM_SLICE / 256; ++i) {
+    const int k = lo + threadIdx.x + i * 256;
+    v[i] = k < hi ? static_cast<float>(row[k]) : -INFINITY;
+    m = fmaxf(m, v[i]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float shift = isinf(m) ? 0.f : m;
+#pragma unroll
+  for (int i = 0; i < LSM_SLICE / 256; ++i) s += lo + static_cast<int>(threadIdx.x) + i * 256 < hi ? expf(v[i] - shift) : 0.f;
+  s = block_sum<4>(s, red);
+  if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = float2{m, s};
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, T* __restrict__ out, int n) {
+  const float2* p = part + blockIdx.y * gridDim.x;
+  float m = -INFINITY, s = 0.f;
+  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) m = fmaxf(m, p[i].x);
+  const float shift = isinf(m) ? 0.f : m;
+  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) s += p[i].y * expf((isinf(p[i].x) ? 0.f : p[i].x) - shift);
+  const float lse = lsm_round<T>(logf(s) + shift);
+  const int lo = blockIdx.x * LSM_SLICE, hi = min(lo + LSM_SLICE, n);
+  const int64_t base = static_cast<int64_t>(blockIdx.y) * n;
+#pragma unroll 8
+  for (int k = lo + threadIdx.x; k < hi; k += 256) out[base + k] = static_cast<T>(static_cast<float>(x[base + k]) - lse);
+}
+
+template <typename T>
+__global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict__ x, T* __restrict__ out, int n, int vec) {
+  constexpr int PER = 16 / sizeof(T), NWV = LSM_NT / 64;
+  __shared__ float red[NWV];
+  const T* row = x + static_cast<int64_t>(blockIdx.x) * n;
+  T* orow = out + static_cast<int64_t>(blockIdx.x) * n;
+  const int nv = vec ? n / PER : 0;                          // whole 16-byte pieces; the rest (all of it where rows are not aligned) one by one
+  const uint4* rv = reinterpret_cast<const uint4*>(row);
+  const int tid = threadIdx.x;
+  uint4 v[LSM_VR];
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < LSM_VR; ++i) {
+    const int k = tid + i * LSM_NT;
+    if (k < nv) {
+      v[i] = rv[k];
+#pragma unroll
+      for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(v[i], j));
+    }
+  }
+  for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) {
+    const uint4 u = rv[k];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(u, j));
+  }
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) m = fmaxf(m, static_cast<float>(row[k]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((tid & 63) == 0) red[tid >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NWV; ++i) m = fmaxf(m, red[i]);
+  if (isinf(m)) m = 0.f;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < LSM_VR; ++i)
+    if (tid + i * LSM_NT < nv) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(v[i], j) - m);
+    }
+  for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) {
+    const uint4 u = rv[k];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(u, j) - m);
+  }
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) s += expf(static_cast<float>(row[k]) - m);
+  s = block_sum<NWV>(s, red);
+  const float lse = lsm_round<T>(logf(s) + m);
+  auto put = [&](int k, const uint4& u) {
+    uint4 r;
+    unsigned* w = &r.x;
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = __float_as_uint(lsm_get<T>(u, j) - lse);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        w[j] = static_cast<unsigned>(lsm_bits<T>(lsm_get<T>(u, 2 * j) - lse)) | (static_cast<unsigned>(lsm_bits<T>(lsm_get<T>(u, 2 * j + 1) - lse)) << 16);
+    }
+    reinterpret_cast<uint4*>(orow)[k] = r;
+  };
+#pragma unroll
+  for (int i = 0; i < LSM_VR; ++i)
+    if (tid + i * LSM_NT < nv) put(tid + i * LSM_NT, v[i]);
+  for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) put(k, rv[k]);
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) orow[k] = static_cast<T>(static_cast<float>(row[k]) - lse);
+}
+
+template <typename T>
+void launch_log_softmax(const void* x, void* out, int64_t rows, int n, float* part, hipStream_t s) {
+  constexpr int PER = 16 / sizeof(T);
+  const T* xt = static_cast<const T*>(x);
+  T* ot = static_cast<T*>(out);
+  if (part) {
+    const dim3 grid((n + LSM_SLICE - 1) / LSM_SLICE, static_cast<unsigned>(rows));
+    log_softmax_slice_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<float2*>(part), n);
+    log_softmax_write_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<const float2*>(part), ot, n);
+    return;
+  }
+  const int vec = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0 && (rows == 1 || n % PER == 0);
+  log_softmax_kernel<T><<<static_cast<unsigned>(rows), LSM_NT, 0, s>>>(xt, ot, n, vec);
 }
 
 template <typename T>
@@ -206,6 +362,24 @@ int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   GBXM_DISPATCH(act, (embed_kernel<T><<<dim3(T_), NT, 0, s>>>(static_cast<const T*>(table), tokens, x, static_cast<T*>(h), h_row, width, scale)));
   return after_launch("embed_scaled");
+}
+
+extern "C" size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n) {
+  // few rows (at sixteen and more the one-launch form keeps as many CUs busy as this one does at its least) that are long
+  return rows > 0 && rows < 16 && n >= 4 * LSM_SLICE + 1 ? static_cast<size_t>(rows) * ((n + LSM_SLICE - 1) / LSM_SLICE) * 8 : 0;
+}
+
+extern "C" int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream) {
+  if (rows < 0 || n <= 0 || (type != GBXM_BF16 && type != GBXM_F32 && type != GBXM_F16) || rows > 0x7fffffff) return fail(GBXM_ERR_INVALID, "log_softmax: bad argument");
+  if (rows == 0) return GBXM_OK;
+  const size_t need = gbxm_log_softmax_workspace(rows, n);
+  if (!x || !out || (need && (!ws || ws_bytes < need || reinterpret_cast<uintptr_t>(ws) % 8))) return fail(GBXM_ERR_INVALID, "log_softmax: null pointer or workspace");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* part = need ? static_cast<float*>(ws) : nullptr;
+  if (type == GBXM_F32) launch_log_softmax<float>(x, out, rows, n, part, s);
+  else if (type == GBXM_BF16) launch_log_softmax<__bf16>(x, out, rows, n, part, s);
+  else launch_log_softmax<_Float16>(x, out, rows, n, part, s);
+  return after_launch("log_softmax");
 }
 
 int gbxm_segment_rmsnorm(void* rows, int64_t T_, int64_t row_stride, int32_t n0, int32_t n1, const float* w0, const float* w1, float eps,

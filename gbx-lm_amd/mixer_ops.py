@@ -107,6 +107,25 @@ _GLU = {"silu": 1, "clamped_swish": 2, "gelu_tanh": 3, "sigmoid": 4}
 _EXPERT = {"silu": 1, "clamped_swish": 2, "relu2": 16}
 
 
+_LSM = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32, torch.float16: _lib.GBXM_F16}
+
+
+def log_probabilities(logits: torch.Tensor) -> torch.Tensor:
+    """``logits - logsumexp(logits)`` over the last axis, the logarithm formed in fp32 and rounded to the logits' dtype: one launch on the
+    GPU (two for a few long rows), torch elsewhere."""
+    if not logits.is_cuda or logits.dtype not in _LSM or not logits.numel():
+        return logits - torch.logsumexp(logits.float(), dim=-1, keepdim=True).to(logits.dtype)
+    x = logits.contiguous()
+    n = x.shape[-1]
+    out = torch.empty_like(x)
+    L, rows = _lib.mixers(), x.numel() // n
+    need = L.gbxm_log_softmax_workspace(rows, n)
+    ws = torch.empty((need,), dtype=torch.uint8, device=x.device) if need else None
+    _lib.check_mixers(L.gbxm_log_softmax(x.data_ptr(), out.data_ptr(), rows, n, _LSM[x.dtype], None if ws is None else ws.data_ptr(), need,
+                                         _stream(x.device)))
+    return out
+
+
 def expert_glu(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, idx: torch.Tensor, activation: str = "silu",
                limit: float = 0.0, scale: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The chosen experts' outputs [T, top, K]; ``activation`` "relu2": experts without a gate (``gate_up`` [E, F, K] is up alone);

@@ -344,7 +344,8 @@ def generate_step(prompt: torch.Tensor, model: nn.Module, *, max_tokens: int = 2
             from . import ops                                     # logsumexp, subtraction and argmax in two small launches
             logprobs, y = ops.logprobs_argmax(logits)
             return y.reshape(-1), logprobs.squeeze(0), prompt_hidden_states
-        logprobs = logits - torch.logsumexp(logits.float(), dim=-1, keepdim=True).to(logits.dtype)
+        from .mixer_ops import log_probabilities
+        logprobs = log_probabilities(logits)                      # (one launch on the GPU)
         y = sampler(logprobs)
         return y.reshape(-1), logprobs.squeeze(0), prompt_hidden_states
 

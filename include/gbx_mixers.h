@@ -18,6 +18,7 @@ extern "C" {
 #define GBXM_ERR_UNSUPPORTED 3
 #define GBXM_BF16 1
 #define GBXM_F32 2
+#define GBXM_F16 3              /* where a function says so */
 
 int gbxm_version(void);
 const char* gbxm_last_error(void);
@@ -26,6 +27,9 @@ const char* gbxm_last_error(void);
  * no image is written). */
 int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* h, int64_t h_row, int64_t T, int32_t width, float scale,
                       int32_t act, void* stream);
+/* out[r] = x[r] - lse(x[r]), lse = log sum exp over the row's n values in fp32, rounded to the rows' type (`type`: also GBXM_F16). */
+size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n);
+int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream);
 /* In place: rows[t][0:n0] and rows[t][n0:n0+n1] each RMS-normalised over the whole segment (fp32 statistics), times w0 / w1. */
 int gbxm_segment_rmsnorm(void* rows, int64_t T, int64_t row_stride, int32_t n0, int32_t n1, const float* w0, const float* w1,
                          float eps, int32_t act, void* stream);

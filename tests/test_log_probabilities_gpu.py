@@ -1,0 +1,40 @@
+"""Log-probabilities in one launch (csrc/mixers_ops.hip: log_softmax_kernel): rows shorter than a wave, around the registers a workgroup keeps
+(8 pieces of 16 bytes a thread), far beyond them, off the 16-byte grid; masked, infinite and undefined logits.  Reference: float64.  The
+logarithm is an fp32 sum of n terms (n 2^-24 relative, so as much absolute in its logarithm, plus its own last place) rounded once to the
+rows' type; the difference is rounded once more."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+LAST = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+@pytest.mark.parametrize("dt", list(LAST))
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 7), (2, 8), (5, 1000), (2, 32767), (32, 32000), (2, 32800), (1, 65536), (1, 65537), (1, 128256), (3, 151936)])
+def test_rows(dt, rows, n):
+    from gbx_lm_amd.mixer_ops import log_probabilities
+    x = (torch.randn((rows, n), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n)) * 3).to(dt)
+    got, want = log_probabilities(x), x.double() - torch.logsumexp(x.double(), -1, keepdim=True)
+    assert got.dtype == dt and got.shape == x.shape
+    lse = torch.logsumexp(x.double(), -1, keepdim=True).abs()
+    room = LAST[dt] * (lse + want.abs()) + n * 2.0 ** -24 + 2.0 ** -22 * (1 + lse)
+    assert bool(((got.double() - want).abs() <= room).all())
+    off = torch.empty(rows * n + 1, dtype=dt, device="cuda")[1:].view(rows, n).copy_(x)            # rows off the 16-byte grid
+    assert bool(((log_probabilities(off).double() - want).abs() <= room).all())
+
+
+@pytest.mark.parametrize("n", [500, 40000])
+@pytest.mark.parametrize("dt", list(LAST))
+def test_masked_and_undefined_logits(dt, n):
+    from gbx_lm_amd.mixer_ops import log_probabilities
+    x = torch.randn((5, n), device="cuda").to(dt)
+    x[0, 100:] = float("-inf")
+    x[1] = float("-inf")
+    x[2, 7] = float("inf")
+    x[3, 9] = float("nan")
+    x[4] = torch.finfo(dt).min
+    got = log_probabilities(x)
+    want = x - torch.logsumexp(x.float(), -1, keepdim=True).to(dt)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    ok = torch.isfinite(want)
+    assert bool(((got - want).abs()[ok].float() <= 2 * LAST[dt] * (1 + want.abs()[ok].float())).all())
