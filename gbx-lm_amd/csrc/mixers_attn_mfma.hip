@@ -1,15 +1,17 @@
 // Matrix-core kernel of gated sliding-window attention for bf16 prompt portions (mechanism: mixers_attn.hip).
 //
-// One workgroup = 4 waves = one tile of up to 128 query rows of one (sequence, head); a wave owns 32 queries.  Key / value tiles
-// of 32 positions go global -> registers (one tile ahead) -> LDS once per workgroup (ring rows for positions before the step, projection rows inside it; rows
+// One workgroup = one tile of up to 128 query rows of one (sequence, head), a wave owns 32 of them; two groups of four waves take every other
+// key tile.  Key / value tiles of 64 positions go global -> registers (one tile ahead) -> LDS once per group (ring rows for positions before the step, projection rows inside it; rows
 // past the tile's last query are zero-filled so that a zero gate never meets a stale NaN).  Both products are computed swapped so
 // that a lane owns ONE query and the gate arithmetic is lane-local:
 //   S^T[key, q] = mfma(K rows, Q rows)      lane (q = lane % 32) holds 16 keys of the tile, the other 16 are in lane ^ 32
 //   O^T[d, q]  += mfma(V^T rows, G^T)       the gate operand of k-step t is the lane's own g[8t .. 8t+7]; V^T comes out of LDS by
 //                                            transposed reads in the same key order
 // No softmax: gates of different keys are independent, O^T just accumulates -- no running maximum, no rescale, no final division.
-// The fp32 part per score (soft cap, log distance penalty, sigmoid: five transcendentals) outweighs the MFMAs: the kernel is bound
-// by the quarter-rate transcendental pipe, not by the matrix cores.  Gates are rounded to bf16 for the value product.
+// The fp32 part per score (four transcendentals, see `exponent`) costs more than the products: the kernel is bound by vector
+// instructions, and by the tiles that start last -- late tiles of all heads come first.  Gates are rounded to bf16 for the value product.
+// Measured, 32 / 4 heads of 128: prompts of 2 047 + 1 100 + 333 + 1 tokens 339 -> 141 us; one of 4 000 tokens 343 (4 096 before: 1 105); 16 heads of 64, 900
+// tokens, one group of waves per tile 43, two 30.
 #include "mixers_mfma.h"
 
 namespace gbxm {
@@ -30,20 +32,34 @@ struct TileArgs {
   float scale, softcap;
 };
 
+// Two groups of four waves take every other key tile of the same queries (their sums meet in LDS at the end): a tile late in a long prompt
+// is a chain of key tiles that the rest of the launch would otherwise wait for.  Heads too large for two waves per SIMD keep one group.
+template <int DK, int DV> struct WindowShape {
+  static constexpr int GROUPS = DK + DV > 256 ? 1 : 2;
+  static constexpr int KT = DK + DV > 256 ? 32 : 64;        // keys per tile (larger heads: 64 would cost the second wave per SIMD)
+  static constexpr int KROW = DK * 2 + 16;                  // +16 B: conflict-free 16-byte fragment reads
+  static constexpr int VROW = DV * 2 + 64;                  // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
+  static constexpr int BYTES = KT * (KROW + VROW) + 1024;   // one group's key and value tile, and its 256 exponents by distance
+  static constexpr int JOIN = GROUPS > 1 ? 4 * (DV / 32) * 16 * 64 * 4 : 0;
+  static constexpr int LDS = GROUPS * BYTES > JOIN ? GROUPS * BYTES : JOIN;
+};
+
 template <int DK, int DV>
-__global__ __launch_bounds__(256) void window_tile_kernel(const TileArgs a) {
-  constexpr int KT = 32;
-  constexpr int KROW = DK * 2 + 16;          // +16 B: conflict-free 16-byte fragment reads
-  constexpr int VROW = DV * 2 + 64;          // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
+__global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS)) void window_tile_kernel(const TileArgs a) {
+  typedef WindowShape<DK, DV> Shape;
+  constexpr int KT = Shape::KT, KROW = Shape::KROW, VROW = Shape::VROW, GROUPS = Shape::GROUPS, STEP = GROUPS * KT;
   constexpr int KS = DK / 16, DT = DV / 32;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[KT * KROW + KT * VROW];
+  extern __shared__ __attribute__((aligned(16))) unsigned char all_lds[];
+  const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  unsigned char* lds = all_lds + group * Shape::BYTES;
   unsigned char* kl = lds;
   unsigned char* vl = lds + KT * KROW;
+  float* dist_tab = reinterpret_cast<float*>(vl + KT * VROW);      // entry distance & 255
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hb = lane >> 5;
-  const int b = a.tiles[2 * blockIdx.x], tq = a.tiles[2 * blockIdx.x + 1];
-  const int head = blockIdx.y, kvh = head / (a.H / a.G);
+  const int tile = (gridDim.x - 1 - blockIdx.x) / a.H;      // (of all heads) late tiles, which see the most keys, start first
+  const int b = a.tiles[2 * tile], tq = a.tiles[2 * tile + 1];
+  const int head = blockIdx.x % a.H, kvh = head / (a.H / a.G);
   const int slot = a.seq[4 * b], pos0 = a.seq[4 * b + 1], n = a.seq[4 * b + 2], row0 = a.seq[4 * b + 3];
   const int W = a.window;
   const int qn = min(a.q_tile, n - tq);                     // queries of this tile
@@ -65,8 +81,14 @@ __global__ __launch_bounds__(256) void window_tile_kernel(const TileArgs a) {
   const int jfirst = max(0, pos0 + tq - W + 1), jlast = pos0 + tq + qn - 1;
   const bool wave_live = wave * 32 < qn;
   const int wq0 = pos0 + tq + wave * 32, wq1 = min(wq0 + 31, jlast);   // positions of this wave's queries
-  const float dm = a.dmul[head], dr = a.drate[head], gb = a.gbias[head];
-  const float cap = a.softcap, inv_cap = cap > 0.f ? 1.f / cap : 0.f, scale = a.scale;
+  // gate = 1 / (1 + 2^z),  z = -log2e (s + gb) + dm log2(1 + dr dist),  s = cap tanh(x / cap) = cap - 2 cap / (1 + 2^(x 2 log2e / cap)): four
+  // transcendentals a score.  What of z depends on the distance alone comes from a table that moves on with the key tile (the queries and keys
+  // of a tile span 127 + KT distances, the ring holds 256); distances outside the window stand there as infinity, which
+  // makes the gate zero without a test per score.
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float dm = a.dmul[head], dr = a.drate[head], cap = a.softcap;
+  const float zc = -LOG2E * (a.gbias[head] + cap), z2 = 2.f * LOG2E * cap, xs = cap > 0.f ? a.scale * 2.f * LOG2E / cap : -LOG2E * a.scale;
+  auto exponent = [&](int d) { return d >= 0 && d < W ? fmaf(dm, __log2f(1.f + dr * static_cast<float>(d)), zc) : INFINITY; };
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
@@ -91,9 +113,17 @@ __global__ __launch_bounds__(256) void window_tile_kernel(const TileArgs a) {
       if (p < KT * (DV / 8) && j <= jlast) vr[i] = *reinterpret_cast<const u32x4*>(src(a.vc, nkv_v, a.nq + a.nk, j) + kvh * DV + c * 8);
     }
   };
-  fetch(jfirst);
-  for (int jt = jfirst; jt <= jlast; jt += KT) {
+  const int j1 = jfirst + group * KT, tiles = (jlast - jfirst + STEP) / STEP;      // (every group runs as many rounds: the barriers are common)
+  if (j1 <= jlast) fetch(j1);
+  const int d1 = pos0 + tq - j1;                              // distance of the tile's first query from the group's first key
+  if (tid < 127 + KT) dist_tab[(d1 + 127 - tid) & 255] = exponent(d1 + 127 - tid);
+  for (int round = 0; round < tiles; ++round) {
+    const int jt = j1 + round * STEP;
     __syncthreads();                                          // the previous tile has been consumed
+    if (tid < STEP) {                                         // the distances that the tile brings in
+      const int d = pos0 + tq - jt - KT + 1 + tid;
+      dist_tab[d & 255] = exponent(d);
+    }
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
       const int p = tid + 256 * i;
@@ -105,37 +135,83 @@ __global__ __launch_bounds__(256) void window_tile_kernel(const TileArgs a) {
       if (p < KT * (DV / 8)) *reinterpret_cast<u32x4*>(vl + (p / (DV / 8)) * VROW + (p % (DV / 8)) * 16) = vr[i];
     }
     __syncthreads();
-    if (jt + KT <= jlast) fetch(jt + KT);                     // the next tile travels while this one is computed
+    if (jt + STEP <= jlast) fetch(jt + STEP);                 // the next tile travels while this one is computed
     if (!wave_live || jt > wq1 || jt + KT - 1 < wq0 - W + 1) continue;      // wave-uniform: no key of the tile is seen by this wave
 
-    f32x16 st = f32x16{0};
+    auto scores = [&](int h) {
+      f32x16 st = f32x16{0};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) st = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + ks * 32), qf[ks], st);
-    float g[16];
+      for (int ks = 0; ks < KS; ++ks) st = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + h * 32 * KROW + ks * 32), qf[ks], st);
+      return st;
+    };
+    auto gates = [&](int h, const f32x16& st, u32x4 (&gf)[2]) {
+      const int j0 = jt + 32 * h, dq = qpos - j0 - 4 * hb;
+      float g[16], t[16];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int dist = qpos - (jt + 8 * (e >> 2) + 4 * hb + (e & 3));
-      float s = st[e] * scale;
-      if (cap > 0.f) s = cap * tanh_<true>(s * inv_cap);
-      s -= dm * __logf(1.f + dr * static_cast<float>(max(dist, 0)));
-      const float v = sigmoid_<true>(s + gb);
-      g[e] = (qvalid && dist >= 0 && dist < W) ? v : 0.f;
+      for (int e = 0; e < 16; ++e) {
+        t[e] = dist_tab[(dq - 8 * (e >> 2) - (e & 3)) & 255];
+        const float z = cap > 0.f ? fmaf(z2, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(st[e] * xs)), t[e]) : fmaf(st[e], xs, t[e]);
+        g[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(z));
+      }
+      if (j0 + 31 > wq0 || wq1 - j0 >= W) {                     // (wave-uniform) keys outside: zero also where the score is no number
+#pragma unroll
+        for (int e = 0; e < 16; ++e) g[e] = t[e] == INFINITY ? 0.f : g[e];
+      }
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+        gf[tt] = u32x4{pack2(g[8 * tt], g[8 * tt + 1]), pack2(g[8 * tt + 2], g[8 * tt + 3]), pack2(g[8 * tt + 4], g[8 * tt + 5]),
+                       pack2(g[8 * tt + 6], g[8 * tt + 7])};
+    };
+    auto values = [&](int h, const u32x4 (&gf)[2]) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          const u32x2 v0 = lds_read_tr(vbase + (32 * h + 16 * tt) * VROW + dt * 64);
+          const u32x2 v1 = lds_read_tr(vbase + (32 * h + 16 * tt + 8) * VROW + dt * 64);
+          o[dt] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[dt]);
+        }
+    };
+    auto half = [&](int h) {
+      const int j0 = jt + 32 * h;
+      if (j0 > wq1 || j0 + 31 < wq0 - W + 1) return;           // (wave-uniform)
+      u32x4 gf[2];
+      gates(h, scores(h), gf);
+      values(h, gf);
+    };
+    if constexpr (KT == 64) {
+      if (jt + 32 <= wq1 && jt + 31 >= wq0 - W + 1) {           // both halves are seen: one half's matrix products under the other's gates
+        const f32x16 s0 = scores(0), s1 = scores(1);
+        u32x4 g0[2], g1[2];
+        gates(0, s0, g0);
+        values(0, g0);
+        gates(1, s1, g1);
+        values(1, g1);
+        continue;
+      }
+      half(0);
+      half(1);
+    } else {
+      half(0);
     }
-    u32x4 gf[2];
+  }
+
+  if constexpr (GROUPS > 1) {
+    float* join = reinterpret_cast<float*>(all_lds) + wave * (DT * 16 * 64) + lane;
+    __syncthreads();
+    if (group == 1) {
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-      gf[tt] = u32x4{pack2(g[8 * tt], g[8 * tt + 1]), pack2(g[8 * tt + 2], g[8 * tt + 3]), pack2(g[8 * tt + 4], g[8 * tt + 5]),
-                     pack2(g[8 * tt + 6], g[8 * tt + 7])};
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) join[(dt * 16 + e) * 64] = o[dt][e];
+    }
+    __syncthreads();
+    if (group == 1) return;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const u32x2 v0 = lds_read_tr(vbase + (16 * tt) * VROW + dt * 64);
-        const u32x2 v1 = lds_read_tr(vbase + (16 * tt + 8) * VROW + dt * 64);
-        o[dt] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[dt]);
-      }
+      for (int e = 0; e < 16; ++e) o[dt][e] += join[(dt * 16 + e) * 64];
   }
-
   if (qvalid) {
     bf16_t* op = a.out + (row0 + tq + qloc) * (static_cast<int64_t>(a.H) * DV) + head * DV;
 #pragma unroll
@@ -150,7 +226,14 @@ __global__ __launch_bounds__(256) void window_tile_kernel(const TileArgs a) {
 
 template <int DK, int DV>
 int launch(const TileArgs& t, int n_tiles, int H, hipStream_t s) {
-  window_tile_kernel<DK, DV><<<dim3(n_tiles, H), 256, 0, s>>>(t);
+  typedef WindowShape<DK, DV> Shape;
+  static OncePerDevice once;
+  if (once.pending()) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_tile_kernel<DK, DV>), hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS);
+    if (e != hipSuccess) return hip_fail(e, "window_attention (tiles)");
+    once.done();
+  }
+  window_tile_kernel<DK, DV><<<static_cast<unsigned>(H) * n_tiles, 256 * Shape::GROUPS, Shape::LDS, s>>>(t);
   return after_launch("window_attention (tiles)");
 }
 
@@ -165,7 +248,7 @@ bool window_tiles_shape(int dk, int dv) {
 
 int launch_window_tiles(const gbxm_window_attn_args& a, hipStream_t s) {
   if (!window_tiles_shape(a.dk, a.dv)) return GBXM_ERR_UNSUPPORTED;
-  if (a.q_tile != 128 || a.H > 65535 || a.row_stride % 8 || (reinterpret_cast<uintptr_t>(a.qkv) | reinterpret_cast<uintptr_t>(a.kcache) |
+  if (a.q_tile != 128 || static_cast<int64_t>(a.H) * a.n_tiles > 0x7fffffff || a.row_stride % 8 || (reinterpret_cast<uintptr_t>(a.qkv) | reinterpret_cast<uintptr_t>(a.kcache) |
                                                              reinterpret_cast<uintptr_t>(a.vcache) | reinterpret_cast<uintptr_t>(a.out)) % 16)
     return GBXM_ERR_UNSUPPORTED;
   TileArgs t{static_cast<const bf16_t*>(a.qkv), static_cast<const bf16_t*>(a.kcache), static_cast<const bf16_t*>(a.vcache), a.seq, a.tiles,
