@@ -1,13 +1,18 @@
 // Matrix-core kernel of softmax attention with a sink for bf16 prompt portions (mechanism and key order: mixers_sink.hip).
 //
-// One workgroup = 4 waves = one tile of up to 128 query rows of one (sequence, head); a wave owns 32 queries.  Key / value tiles
-// of 32 visible positions go global -> registers (one tile ahead) -> LDS once per workgroup.  Both products are computed swapped,
+// One workgroup = tiles of up to 128 query rows of one (sequence, head); a wave owns 32 queries, and one or two groups of four waves share a
+// tile's keys (SinkShape).  Key / value tiles of 64 (large heads: 32) visible positions go global -> registers (one tile ahead) -> LDS once per
+// group.  Both products are computed swapped,
 //   S^T[key, q] = mfma(K rows, Q rows),    O^T[d, q] += mfma(V^T rows, P^T),
 // so that a lane owns ONE query: lane (q = lane % 32, half = lane / 32) holds 16 of the tile's 32 scores of its query, the other 16
-// are in lane ^ 32.  The running maximum is shared by the two lanes of a query (one cross-lane exchange per tile), each keeps its
+// are in lane ^ 32 (and as many of each further 32 keys).  The running maximum is shared by the two lanes of a query (one cross-lane exchange per tile), each keeps its
 // own part of the denominator (joined once at the end), and both rescale their accumulators (different channels of the same
 // query) by the same factor.  The sink starts the running maximum and counts once in the denominator.  Weights are rounded to bf16
 // for the value product; the denominator sums them in fp32.
+//
+// Bound by vector instructions (one exponential, four others a score) and, in short prompts, by how few tiles there are: two groups halve the
+// chain of key tiles behind the last query tile.  Measured, 16 heads, us: <128, 128> 1 501 + 700 + 65 rows 144 -> 45, 4 000 rows 235 -> 130, 8 192 rows
+// 513 -> 469; <192, 128> 4 000 rows 289 -> 187, 8 192 rows 648 -> 658; <64, 64> 3 000 + 500 rows 134 -> 59.
 //
 // Head sizes are run-time numbers (multiples of 8) inside a compiled capacity <DK, DV>: channels beyond them are staged as zeros.
 #include <algorithm>
@@ -52,19 +57,31 @@ __device__ __forceinline__ u32x2 out4(const SinkTileArgs& a, int64_t row, int he
   return u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
 }
 
-template <int DK, int DV>
-__device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile, unsigned char* lds) {
-  constexpr int KT = 32;
-  constexpr int KROW = DK * 2 + 16;          // +16 B: conflict-free 16-byte fragment reads
-  constexpr int VROW = DV * 2 + 64;          // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
-  constexpr int KS = DK / 16, DT = DV / 32;
-  unsigned char* kl = lds;
-  unsigned char* vl = lds + KT * KROW;
+// With two GROUPS of four waves each takes every other key tile of the same queries, with a maximum and denominator of its own; the halves
+// meet in LDS at the end.
+template <int DK, int DV, int GROUPS_> struct SinkShape {
+  static constexpr int GROUPS = GROUPS_;
+  static constexpr int KT = DK + DV > 256 ? 32 : 64;         // keys per tile (larger heads: 64 would cost the second wave per SIMD)
+  static constexpr int KROW = DK * 2 + 16;                   // +16 B: conflict-free 16-byte fragment reads
+  static constexpr int VROW = DV * 2 + 64;                   // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
+  static constexpr int BYTES = KT * (KROW + VROW);
+  static constexpr int JOIN = GROUPS > 1 ? 4 * (DV / 32 * 16 + 2) * 64 * 4 : 0;
+  static constexpr int LDS = GROUPS * BYTES > JOIN ? GROUPS * BYTES : JOIN;
+  static constexpr int WAVES = DK + DV <= 320 ? 2 : 1;       // per SIMD
+};
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <int DK, int DV, int GROUPS_>
+__device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile, const int head, unsigned char* all_lds) {
+  typedef SinkShape<DK, DV, GROUPS_> Shape;
+  constexpr int KT = Shape::KT, KROW = Shape::KROW, VROW = Shape::VROW, GROUPS = Shape::GROUPS, STEP = GROUPS * KT, NH = KT / 32;
+  constexpr int KS = DK / 16, DT = DV / 32;
+  const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  unsigned char* kl = all_lds + group * Shape::BYTES;
+  unsigned char* vl = kl + KT * KROW;
+
   const int r = lane & 31, hb = lane >> 5;
   const int b = a.tiles[2 * tile], tq = a.tiles[2 * tile + 1];
-  const int head = blockIdx.y, kvh = head / (a.H / a.G);
+  const int kvh = head / (a.H / a.G);
   const int slot = a.seq[4 * b], pos0 = a.seq[4 * b + 1], n = a.seq[4 * b + 2], row0 = a.seq[4 * b + 3];
   const int qn = min(a.q_tile, n - tq);                     // queries of this tile
   const int qloc = wave * 32 + r;
@@ -96,8 +113,8 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float scale2 = (a.head_scale ? a.scale * a.head_scale[head] : a.scale) * LOG2E;
-  float m = a.sink ? a.sink[head] * LOG2E : -INFINITY;
-  float l = (a.sink && hb == 0) ? 1.f : 0.f;                            // the sink counts once per query
+  float m = a.sink && group == 0 ? a.sink[head] * LOG2E : -INFINITY;
+  float l = (a.sink && group == 0 && hb == 0) ? 1.f : 0.f;              // the sink counts once per query
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
@@ -126,8 +143,10 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
       if (p < KT * (DV / 8) && iv < total && c * 8 < a.dv) vr[i] = *reinterpret_cast<const u32x4*>(vrow(pos_of(iv)) + c * 8);
     }
   };
-  fetch(0);
-  for (int it = 0; it < total; it += KT) {
+  const int i1 = group * KT, rounds = (total + STEP - 1) / STEP;        // (every group runs as many rounds: the barriers are common)
+  if (i1 < total) fetch(i1);
+  for (int round = 0; round < rounds; ++round) {
+    const int it = i1 + round * STEP;
     __syncthreads();                                          // the previous tile has been consumed
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
@@ -140,31 +159,49 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
       if (p < KT * (DV / 8)) *reinterpret_cast<u32x4*>(vl + (p / (DV / 8)) * VROW + (p % (DV / 8)) * 16) = vr[i];
     }
     __syncthreads();
-    if (it + KT < total) fetch(it + KT);                      // the next tile travels while this one is computed
+    if (it + STEP < total) fetch(it + STEP);                  // the next tile travels while this one is computed
     // wave-uniform: no key of the tile is seen by a query of this wave
+    if (!wave_live || it >= total) continue;
     const int jmin = pos_of(it), jmax = pos_of(min(it + KT, total) - 1);
-    if (!wave_live || jmin > wq1 || (jmax < wlo0 && jmin >= a.keep)) continue;
+    if (jmin > wq1 || (jmax < wlo0 && jmin >= a.keep)) continue;
 
-    f32x16 st = f32x16{0};
+    f32x16 st[NH];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) st = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + ks * 32), qf[ks], st);
+    for (int h = 0; h < NH; ++h) {
+      st[h] = f32x16{0};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) st[h] = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + h * 32 * KROW + ks * 32), qf[ks], st[h]);
+    }
     // scores in units of ln 2 (the exponentials below are base 2).  Inside the mask -- every key of the tile before every query of the
-    // wave, inside every window -- nothing is tested per score.
+    // wave, inside every window -- nothing is tested per score, the scale meets the maximum once and the rest inside the exponent.
     const bool inside = it + KT <= total && jmax <= wq0 && (jmin >= wlo1 || jmax < a.keep);
-    float s[16];
-    float mx = -INFINITY;
+    float mx;
     if (inside) {
+      float e0 = st[0][0];
+      if (scale2 >= 0.f) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) { s[e] = st[e] * scale2; mx = fmaxf(mx, s[e]); }
-    } else {
+        for (int h = 0; h < NH; ++h)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int iv = it + 8 * (e >> 2) + 4 * hb + (e & 3);
-        const int j = pos_of(iv);
-        const bool seen = qvalid && iv < total && j <= qpos && (j >= qlo || j < a.keep);
-        s[e] = seen ? st[e] * scale2 : -INFINITY;
-        mx = fmaxf(mx, s[e]);
+          for (int e = 0; e < 16; ++e) e0 = fmaxf(e0, st[h][e]);
+      } else {
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) e0 = fminf(e0, st[h][e]);
       }
+      mx = e0 * scale2;
+    } else {
+      mx = -INFINITY;
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int iv = it + 32 * h + 8 * (e >> 2) + 4 * hb + (e & 3);
+          const int j = pos_of(iv);
+          const bool seen = qvalid && iv < total && j <= qpos && (j >= qlo || j < a.keep);
+          st[h][e] = seen ? st[h][e] * scale2 : -INFINITY;
+          mx = fmaxf(mx, st[h][e]);
+        }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                   // the other half of the query's scores
     const float m_new = fmaxf(m, mx);
@@ -173,8 +210,11 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
     const bool moved = m_new != m;
     m = m_new;
     float ps = 0.f;
+    const float f2 = inside ? scale2 : 1.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) { s[e] = __builtin_amdgcn_exp2f(s[e] - m_ref); ps += s[e]; }
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) { st[h][e] = __builtin_amdgcn_exp2f(fmaf(st[h][e], f2, -m_ref)); ps += st[h][e]; }
     l = l * alpha + ps;
     if (__any(moved)) {                                       // wave-uniform: the maximum of no query of the wave has moved -> alpha is 1
 #pragma unroll
@@ -182,21 +222,45 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
     }
-    u32x4 gf[2];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-      gf[tt] = u32x4{pack2(s[8 * tt], s[8 * tt + 1]), pack2(s[8 * tt + 2], s[8 * tt + 3]), pack2(s[8 * tt + 4], s[8 * tt + 5]),
-                     pack2(s[8 * tt + 6], s[8 * tt + 7])};
+    for (int h = 0; h < NH; ++h) {
+      u32x4 gf[2];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+        gf[tt] = u32x4{pack2(st[h][8 * tt], st[h][8 * tt + 1]), pack2(st[h][8 * tt + 2], st[h][8 * tt + 3]), pack2(st[h][8 * tt + 4], st[h][8 * tt + 5]),
+                       pack2(st[h][8 * tt + 6], st[h][8 * tt + 7])};
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          const u32x2 v0 = lds_read_tr(vbase + (32 * h + 16 * tt) * VROW + dt * 64);
+          const u32x2 v1 = lds_read_tr(vbase + (32 * h + 16 * tt + 8) * VROW + dt * 64);
+          o[dt] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[dt]);
+        }
+    }
+  }
+
+  if constexpr (GROUPS > 1) {
+    float* join = reinterpret_cast<float*>(all_lds) + wave * ((DT * 16 + 2) * 64) + lane;
+    __syncthreads();
+    if (group == 1) {
+      join[0] = m;
+      join[64] = l;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) join[(2 + dt * 16 + e) * 64] = o[dt][e];
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = join[0], mj = fmaxf(m, m1), mr = mj == -INFINITY ? 0.f : mj;
+    const float f0 = __builtin_amdgcn_exp2f(m - mr), f1 = __builtin_amdgcn_exp2f(m1 - mr);
+    l = l * f0 + join[64] * f1;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const u32x2 v0 = lds_read_tr(vbase + (16 * tt) * VROW + dt * 64);
-        const u32x2 v1 = lds_read_tr(vbase + (16 * tt + 8) * VROW + dt * 64);
-        o[dt] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[dt]);
-      }
+      for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * f0 + join[(2 + dt * 16 + e) * 64] * f1;
   }
-
   l += __shfl_xor(l, 32, 64);
   if (qvalid) {
     const int64_t row = row0 + tq + qloc;
@@ -422,20 +486,44 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
   return launch_sink_reduce(a, splits, s);
 }
 
-// A workgroup takes two query tiles, one from each end of the step's list: in a long causal prompt a late tile (many keys) and an
-// early one (few), so that workgroups carry about the same work however they are spread over the chip.
-template <int DK, int DV>
-__global__ __launch_bounds__(256, (DK + DV <= 320 ? 2 : 1)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[32 * (DK * 2 + 16) + 32 * (DV * 2 + 64)];
-  const int first = n_tiles - 1 - blockIdx.x, second = blockIdx.x;
-  sink_tile<DK, DV>(a, first, lds);
-  if (second != first) sink_tile<DK, DV>(a, second, lds);
+// One group: a workgroup takes two query tiles, one from each end of the step's list -- in a long causal prompt a late tile (many keys) and an
+// early one (few) -- so that workgroups carry about the same work however they are spread over the chip.  Two groups: a tile each, of all
+// heads the late ones first.
+template <int DK, int DV, int GROUPS>
+__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  if constexpr (GROUPS == 1) {
+    const int pairs = (n_tiles + 1) / 2, second = blockIdx.x % pairs, first = n_tiles - 1 - second, head = blockIdx.x / pairs;
+    sink_tile<DK, DV, 1>(a, first, head, lds);
+    if (second != first) sink_tile<DK, DV, 1>(a, second, head, lds);
+  } else {
+    sink_tile<DK, DV, 2>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
+  }
 }
 
+template <int DK, int DV, int GROUPS>
+int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(t.H) * (GROUPS == 1 ? (n_tiles + 1) / 2 : n_tiles);
+  constexpr int bytes = SinkShape<DK, DV, GROUPS>::LDS;
+  static OncePerDevice once;
+  if (once.pending()) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return hip_fail(e, "sink_attention (tiles)");
+    once.done();
+  }
+  sink_tile_kernel<DK, DV, GROUPS><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles);
+  return after_launch("sink_attention (tiles)");
+}
+
+// Tiles times heads up to which two groups share a tile.  Measured, one group against two, us, 16 heads: 12 + 6 + 1 tiles of <128, 128> 112 | 44; one prompt of
+// 32 tiles <192, 128> 282 | 187; 47 tiles 434 | 390; three of 20 334 | 250; 64 tiles 658 | 680, <128, 128> 469 | 466, <64, 64> 286 | 305.
+constexpr unsigned TWO_GROUPS = 960;
 template <int DK, int DV>
 int launch(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
-  sink_tile_kernel<DK, DV><<<dim3((n_tiles + 1) / 2, t.H), 256, 0, s>>>(t, n_tiles);
-  return after_launch("sink_attention (tiles)");
+  if constexpr (DK + DV <= 320) {
+    if (static_cast<unsigned>(t.H) * n_tiles <= TWO_GROUPS) return launch_groups<DK, DV, 2>(t, n_tiles, s);
+  }
+  return launch_groups<DK, DV, 1>(t, n_tiles, s);
 }
 
 constexpr int CAPS[][2] = {{32, 32}, {64, 64}, {64, 128}, {96, 96}, {128, 128}, {192, 128}, {256, 256}};
@@ -469,7 +557,7 @@ static SinkTileArgs tile_args(const gbxm_sink_attn_args& a) {
 }
 
 int launch_sink_tiles(const gbxm_sink_attn_args& a, hipStream_t s) {
-  if (!sink_tiles_shape(a.dk, a.dv) || a.q_tile != 128 || a.H > 65535 || !tile_operands(a)) return GBXM_ERR_UNSUPPORTED;
+  if (!sink_tiles_shape(a.dk, a.dv) || a.q_tile != 128 || static_cast<int64_t>(a.H) * a.n_tiles > 0x7fffffff || !tile_operands(a)) return GBXM_ERR_UNSUPPORTED;
   const SinkTileArgs t = tile_args(a);
 #define GBXM_TILE(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch<DK_, DV_>(t, a.n_tiles, s)
   GBXM_TILE(32, 32); GBXM_TILE(64, 64); GBXM_TILE(64, 128); GBXM_TILE(96, 96); GBXM_TILE(128, 128); GBXM_TILE(192, 128); GBXM_TILE(256, 256);

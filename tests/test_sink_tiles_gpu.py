@@ -1,0 +1,41 @@
+"""Softmax attention of prompt portions (csrc/mixers_sink_mfma.hip) on both sides of the rule that gives a query tile one or two groups of waves,
+at lengths around 32, 64 and 128 keys, with windows that end inside a tile, sinks, and head factors of either sign and zero.  Reference:
+float64 from the same bf16 rows.  Tolerance: weights are rounded to bf16 for the value product, 2^-8 of each, independent of each other; the
+result is rounded once: 2^-8 (|y| + the root of the sum of squared terms), 3 x for the extremes; 2^-16 of the terms' absolute sum for the
+fp32 scores and exponentials (scores of up to 2^5)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+FEW = [1, 33, 64, 65, 129, 300]
+MANY = [1 + (37 * i) % 170 for i in range(140)]
+
+
+@pytest.mark.parametrize("lens", [FEW, MANY], ids=["two-groups", "one-group"])
+@pytest.mark.parametrize("dk,dv", [(32, 32), (128, 128), (192, 128), (72, 40)])
+@pytest.mark.parametrize("window", [None, 1, 65])
+def test_portions(lens, dk, dv, window):
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.batching import StepBatch
+    gen = torch.Generator(device=DEV).manual_seed(dk + len(lens))
+    H, G, T = 8, 2, sum(lens)
+    assert (len(lens) > 100) == (sum((n + 127) // 128 for n in lens) * H > 960)
+    batch = StepBatch.build(list(range(len(lens))), [0] * len(lens), lens, DEV)
+    q, k, v = (torch.randn((T, n, d), device=DEV, generator=gen).to(torch.bfloat16) for n, d in ((H, dk), (G, dk), (G, dv)))
+    sink = torch.randn(H, device=DEV, generator=gen)
+    factor = torch.tensor([1.0, -1.0, 0.5, 0.0, 1.3, 2.0, -0.7, 1.0], device=DEV)
+    got = M.sink_attention(q, k, v, None, batch, dk ** -0.5, window, 0, sink, head_scale=factor).double().view(T, H, dv)
+    r0 = 0
+    for n in lens:
+        i = torch.arange(n, device=DEV)
+        hidden = (i[None] > i[:, None]) | ((i[:, None] - i[None] >= window) if window else False)
+        for h in range(H):
+            qq, kk, vv = (t[r0:r0 + n].double() for t in (q[:, h], k[:, h // 4], v[:, h // 4]))
+            s = (qq @ kk.t() * (dk ** -0.5 * factor[h].double())).masked_fill(hidden, float("-inf"))
+            den = torch.logaddexp(torch.logsumexp(s, -1, keepdim=True), sink[h].double())
+            p = torch.exp(s - den)
+            want, spread, total = p @ vv, (p ** 2 @ vv ** 2).sqrt(), p @ vv.abs()
+            err = (got[r0:r0 + n, h] - want).abs()
+            assert bool((err <= 3 * 2.0 ** -8 * (want.abs() + spread) + 2.0 ** -16 * total + 1e-6).all()), (n, h, float(err.max()))
+        r0 += n
