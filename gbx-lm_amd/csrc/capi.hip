@@ -114,8 +114,7 @@ int gbx_qlinear_forward_ws(const void* x, const uint32_t* qweight, const void* s
     const size_t img = (static_cast<size_t>(N) * K * 2 + 255) & ~static_cast<size_t>(255);
     const size_t part = gbx::gemm_dense_workspace_bytes(static_cast<int>(M), N, K);
     if (part && workspace_bytes >= img + part) dense_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + img);
-    const long long tiles = ((M + 255) / 256) * ((N + 255) / 256);
-    if (!dense_part && M < gbx::GBX_DENSE_MIN_M && tiles < 176) use_dense = false;
+    if (!dense_part && !gbx::dense_fills_chip(M, N)) use_dense = false;
   }
   if (!force_generic && M > 1 && M <= 64 && (K % 128) == 0 && K >= 512) {
     // a sufficient, 16-byte aligned workspace lets the batched-decode kernel split k across workgroups

@@ -61,16 +61,22 @@ hipError_t launch_qgemm_dense_swiglu(const void* x, const uint32_t* gq, const vo
 constexpr int GBX_DENSE_MIN_M = 4096;
 // Prompt-sized calls with caller scratch: dequantise once + the 256 x 256 dense GEMM wherever its tiles fill the chip --
 // always from 4096 rows, from 1024 rows when the 256 x 256 tiles make at least ~0.7 of a round over the 256 CUs (measured,
-// 4 bits: M 3072 x N 4096: 161 -> 96 us, M 1024 x N 14336: 172 -> 96, M 2048 x N 14336: 268 -> 190; below that the fused tiles
-// with their finer shapes / k split win, e.g. M 2048 x N 4096: 89 vs 96)
+// 4 bits: M 3072 x N 4096: 161 -> 96 us, M 1024 x N 14336: 172 -> 96, M 2048 x N 14336: 268 -> 190) or the fused path's own tiles,
+// 256 rows x 128 outputs, no longer fit one: its second round costs as much as its first, at every K (us, fused | dequantise + dense, 4 bits:
+// M 3001 x N 3072, 288 fused and 144 dense tiles: K 128 27 | 15, K 1024 56 | 34, K 4096 160 | 89, K 8192 313 | 171; M 1500 x N 5632, 264 and
+// 132: 27 | 16, 57 | 37, 161 | 95).  Within one round the fused tiles win (M 1024 x N 7168, 224 and 112: K 512 23 | 30), and where the outputs
+// do not divide into the dense GEMM's 8-byte stores (M 2817 x N 2561: K 2048 51 | 68).
 // ... and, with its k range split over workgroups (gemm_dense_ksplit, fp32 slices + a summing launch), the few-tile shapes of a
 // 1024..4095-row chunk too (M 1024 x N 4096: 83 -> 45 us, K 14336: 256 -> 104)
 int gemm_dense_ksplit(int M, int N, int K);
+inline bool dense_fills_chip(long long M, int N) {
+  const long long rows = (M + 255) / 256;
+  return M >= GBX_DENSE_MIN_M || rows * ((N + 255) / 256) >= 176 || (N % 4 == 0 && rows * ((N + 127) / 128) > 256);
+}
 inline bool dense_path_wanted(long long M, int N, int K) {
   if ((K % 128) != 0) return false;
-  if (M >= GBX_DENSE_MIN_M) return true;
   if (M < 1024) return false;
-  return ((M + 255) / 256) * ((N + 255) / 256) >= 176 || (N % 4 == 0 && gemm_dense_ksplit(static_cast<int>(M), N, K) > 1);
+  return dense_fills_chip(M, N) || (N % 4 == 0 && gemm_dense_ksplit(static_cast<int>(M), N, K) > 1);
 }
 hipError_t launch_rope_kv_write(const void* k, const void* v, void* kcache, void* vcache, const float* inv_freq, long long pos0,
                                 long long B, int H, int L, int D, long long ksb, long long ksh, long long ksl, long long vsb,
