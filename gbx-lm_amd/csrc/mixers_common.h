@@ -65,6 +65,43 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// The same over a workgroup of blockDim.x threads (whole waves, at most 16 of them); `red` is 16 floats of LDS that no earlier call used.
+__device__ __forceinline__ float row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float s = 0.f;
+  for (int i = 0; i < static_cast<int>(blockDim.x >> 6); ++i) s += red[i];
+  return s;
+}
+
+// Row kernels that give every thread one group of four neighbouring channels (rows of up to 4 * 1024): every operand of a row is in flight
+// at once, where a loop over channels whose stores may alias its loads pays a trip to memory per pass.  Threads of a workgroup for `width`
+// channels; 0: the row is too wide or not in groups of four.
+inline int row_threads(int width) { return width % 4 == 0 && width <= 4096 ? (width / 4 + 63) / 64 * 64 : 0; }
+template <typename... P>
+inline bool all_aligned(size_t bytes, const P*... p) { return ((reinterpret_cast<uintptr_t>(p) | ...) & (bytes - 1)) == 0; }
+
+// z = a row of a sublayer's output, or sum_k mix[k] (candidate row k), at channels c .. c + 3; eight candidates in flight at a time.
+template <typename T>
+__device__ __forceinline__ void candidate_sum(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c, float* z) {
+  if (!mix) { Lanes<T, 4>::load(y + c, z); return; }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) z[i] = 0.f;
+  for (int k0 = 0; k0 < top; k0 += 8) {
+    float u[8][4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) Lanes<T, 4>::load(y + static_cast<int64_t>(min(k0 + k, top - 1)) * width + c, u[k]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k0 + k < top) {
+        const float m = mix[k0 + k];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[i] += m * u[k][i];
+      }
+  }
+}
+
 // Transcendentals: exact library forms for fp32 models, hardware approximations (a few ulp) where activations are bf16.
 template <bool FAST> __device__ __forceinline__ float exp_(float x) { if constexpr (FAST) return __expf(x); else return expf(x); }
 template <bool FAST> __device__ __forceinline__ float sigmoid_(float x) {

@@ -1,0 +1,97 @@
+"""Row kernels that hold a row in one group of four channels per thread (csrc/mixers_common.h: row_threads): one group, a wave's end, ragged waves, the
+widest row, the widths on either side that stay with the looping kernels, candidates beside the eight in flight, a base that is not aligned.
+Reference: the torch path in float64 sums; tolerances: a few fp32 roundings of sums of positive terms, results rounded to the activation type."""
+import pytest
+import torch
+
+from gbx_lm_amd.batching import StepBatch
+from gbx_lm_amd.models import residual as R
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ROW = {torch.float32: 2e-6, torch.bfloat16: 2.0 ** -8}
+WIDTHS = (4, 6, 252, 256, 260, 2048, 4092, 4096, 4100)
+
+
+def near(got, want, dt):
+    tol = ROW[dt]
+    return bool(((got.cpu().double() - want).abs() <= tol * want.abs() + 16 * 2.0 ** -24 * want.abs().amax(-1, keepdim=True)).all())
+
+
+def shifted(x, n):
+    """The same values at an address n elements past an allocation's start."""
+    buf = torch.empty(x.numel() + n, dtype=x.dtype, device=DEV)
+    buf[n:] = x.reshape(-1).to(DEV)
+    return buf[n:].view(x.shape)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", WIDTHS)
+@pytest.mark.parametrize("s,top,off", [(4, 8, 0), (1, 1, 0), (8, 9, 0), (3, 2, 1)])
+def test_streams(width, dt, s, top, off):
+    g = torch.Generator().manual_seed(width + s)
+    X, y = torch.randn((3, s, width), generator=g), torch.randn((3, top, width) if top > 1 else (3, width), generator=g).to(dt)
+    y_mix = torch.rand((3, top), generator=g) if top > 1 else None
+    mix, write, read = torch.randn((s, s), generator=g), torch.randn(s, generator=g), torch.rand(s, generator=g) + 0.1
+    norm = R.StreamLayerNorm(width, 1e-2)
+    norm.weight, norm.bias = torch.rand(width, generator=g) + 0.5, torch.randn(width, generator=g)
+    z = y.double() if top == 1 else (y.double() * y_mix.double().unsqueeze(-1)).sum(1)
+    Xn = torch.einsum("ij,tiw->tjw", mix.double(), X.double()) + write.double()[None, :, None] * z[:, None]
+    bound = torch.einsum("ij,tiw->tjw", mix.double().abs(), X.double().abs()) + write.double().abs()[None, :, None] * (
+        y.double().abs() if top == 1 else (y.double().abs() * y_mix.double().unsqueeze(-1)).sum(1))[:, None]
+    u, room = (Xn * read.double()[None, :, None]).sum(1), (bound * read.double()[None, :, None]).sum(1)
+    sd = (u - u.mean(-1, keepdim=True)).pow(2).mean(-1, keepdim=True).add(norm.eps).sqrt()
+    want = (u - u.mean(-1, keepdim=True)) / sd * norm.weight.double() + norm.bias.double()
+    dev = lambda t: None if t is None else t.to(DEV)
+    nd = R.StreamLayerNorm(width, 1e-2)
+    nd.weight, nd.bias = norm.weight.to(DEV), norm.bias.to(DEV)
+    Xd = shifted(X, off)
+    h = R.hyper_step_(Xd, shifted(y, off), dev(y_mix), dev(mix), dev(write), dev(read), nd, dt)
+    terms = (s + top + 4) * 2.0 ** -24
+    assert bool(((Xd.cpu().double() - Xn).abs() <= terms * bound).all())
+    err = (2 * terms * room.amax(-1, keepdim=True) / sd * norm.weight.double() + ROW[dt] * want.abs() + 2.0 ** -20) * (1 + want.abs())
+    assert bool(((h.cpu().double() - want).abs() <= err).all())
+    total = R.hyper_step_(shifted(X, off), shifted(y, off), dev(y_mix), dev(mix), dev(write), None, None, dt)
+    assert bool(((total.cpu().double() - Xn.sum(1)).abs() <= 2 * terms * bound.sum(1)).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", WIDTHS)
+@pytest.mark.parametrize("top,extra,off", [(1, False, 0), (8, True, 0), (9, False, 0), (2, True, 1)])
+def test_branch_norm(width, dt, top, extra, off):
+    g = torch.Generator().manual_seed(width + top)
+    x, y = torch.randn((3, width), generator=g), torch.rand((3, top, width) if top > 1 else (3, width), generator=g).to(dt) + 0.5
+    mix, ex = (torch.rand((3, top), generator=g) if top > 1 else None), (torch.rand((3, width), generator=g).to(dt) if extra else None)
+    w, nw = torch.rand(width, generator=g) + 0.5, torch.rand(width, generator=g) + 0.5
+    unit = lambda v: v / v.pow(2).mean(-1, keepdim=True).add(1e-5).sqrt()
+    z = y.double() if top == 1 else (y.double() * mix.double().unsqueeze(-1)).sum(1)
+    z = z + ex.double() if extra else z
+    new = x.double() + unit(z) * w.double()
+    xd = shifted(x, off)
+    dev = lambda t: None if t is None else t.to(DEV)
+    h = R.branch_norm_add_norm_(xd, shifted(y, off), dev(mix), dev(ex), w.to(DEV), 1e-5, nw.to(DEV), dt)
+    assert near(xd, new, torch.float32) and near(h, unit(new) * nw.double(), dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", WIDTHS)
+def test_shift(width, dt):
+    """Two sequences over two steps: the slot's row is the norm that the next row would have computed, bit for bit."""
+    from gbx_lm_amd.models.cache import SequenceSlots, SlotRowCache
+    g = torch.Generator().manual_seed(width)
+    x, w, shift = torch.randn((9, width), generator=g) + 0.5, torch.rand(width, generator=g) + 0.5, torch.rand(width, generator=g)
+    n = x.double() / x.double().pow(2).mean(-1, keepdim=True).add(1e-5).sqrt() * w.double()
+    prev = torch.cat([torch.zeros(1, width, dtype=torch.float64), n[:5], torch.zeros(1, width, dtype=torch.float64), n[6:8]])
+    want = n + (prev - n) * shift.double()
+    slots = SequenceSlots(2)
+    slots.length[0] = slots.length[1] = 0
+    cache = SlotRowCache(width, "f32", slots)
+    cache.reserve(dt, DEV)
+    cache.rows.fill_(7.0)
+    run = lambda rows, batch: R.norm_token_shift(rows.to(DEV), w.to(DEV), 1e-5, shift.to(DEV), cache, batch, dt)
+    whole = run(x, StepBatch.build([0, 1], [0, 0], [6, 3], DEV))
+    kept = cache.rows.clone()
+    assert near(whole, want, dt) and near(kept[:2], torch.stack([n[5], n[8]]), torch.float32)
+    parts = [run(torch.cat([x[:2], x[6:7]]), StepBatch.build([0, 1], [0, 0], [2, 1], DEV)), run(torch.cat([x[2:6], x[7:]]), StepBatch.build([0, 1], [2, 1], [4, 2], DEV))]
+    again = torch.cat([parts[0][:2], parts[1][:4], parts[0][2:], parts[1][4:]])
+    assert torch.equal(again, whole) and torch.equal(cache.rows[:2], kept[:2])
