@@ -82,6 +82,23 @@ inline int row_threads(int width) { return width % 4 == 0 && width <= 4096 ? (wi
 template <typename... P>
 inline bool all_aligned(size_t bytes, const P*... p) { return ((reinterpret_cast<uintptr_t>(p) | ...) & (bytes - 1)) == 0; }
 
+// Candidates in front of candidate e of value x among 4 n4 values: larger ones, and equal ones of a lower index.  Every candidate's rank is
+// taken at once, where rounds of arg-max wait for one another.
+__device__ __forceinline__ int rank_of(const float* v, int n4, int e, float x) {
+  int rank = 0;
+#pragma unroll 8
+  for (int j = 0; j < n4; ++j) {
+    const float4 u = *reinterpret_cast<const float4*>(v + 4 * j);
+    const float w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) rank += (w[k] > x || (w[k] == x && 4 * j + k < e)) ? 1 : 0;
+  }
+  return rank;
+}
+// Experts up to which a router's choice goes by rank (every expert reads all scores; beyond, the rounds' work grows slower): sigmoid router of
+// 1 row x 32 experts 7.9 -> 5.4 us, of 2266 x 128 16.0 -> 13.6, softmax of 32 rows x 128 experts 11.7 -> 9.6.
+constexpr int RANK_EXPERTS = 512;
+
 // z = a row of a sublayer's output, or sum_k mix[k] (candidate row k), at channels c .. c + 3; eight candidates in flight at a time.
 template <typename T>
 __device__ __forceinline__ void candidate_sum(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c, float* z) {

@@ -325,6 +325,64 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   if (renorm && threadIdx.x < top) weight[t * top + threadIdx.x] /= chosen_sum;
 }
 
+// The same by rank (E <= RANK_EXPERTS): probabilities and their order as above, no round waits for another.
+__global__ __launch_bounds__(NT) void route_topk_rank_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int E,
+                                                            int top, int renorm) {
+  __shared__ __attribute__((aligned(16))) float pl[RANK_EXPERTS];
+  __shared__ float sel[NT];
+  __shared__ float red[NW], mxs[NW];
+  const int64_t t = blockIdx.x;
+  constexpr int PER = RANK_EXPERTS / NT;
+  float v[PER];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = threadIdx.x + i * NT;
+    v[i] = e < E ? logits[t * E + e] : -INFINITY;
+    mx = fmaxf(mx, v[i]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if ((threadIdx.x & 63) == 0) mxs[threadIdx.x >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) mx = fmaxf(mx, mxs[i]);
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
+    v[i] = live ? expf(v[i] - mx) : 0.f;
+    sum += v[i];
+  }
+  sum = block_sum<NW>(sum, red);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
+    v[i] = live ? v[i] / sum : -1.f;
+    if (!(v[i] == v[i])) v[i] = -1.f;            // (not a number: behind every probability)
+    pl[threadIdx.x + i * NT] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = threadIdx.x + i * NT;
+    if (e < E) {
+      const int rank = rank_of(pl, (E + 3) / 4, e, v[i]);
+      if (rank < top) {
+        idx[t * top + rank] = e;
+        if (renorm) sel[rank] = v[i]; else weight[t * top + rank] = v[i];
+      }
+    }
+  }
+  if (!renorm) return;
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < top) {
+    float chosen = 0.f;
+    for (int k = 0; k < top; ++k) chosen += sel[k];
+    weight[t * top + threadIdx.x] = sel[threadIdx.x] / chosen;
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(NT) void window_append_kernel(const T* __restrict__ qkv, int64_t stride, int nq, int nk, int nv, T* __restrict__ kc,
                                                           T* __restrict__ vc, const int* __restrict__ seq, const int* __restrict__ tok, int window) {
@@ -418,7 +476,8 @@ int gbxm_route_topk(const float* logits, int32_t* idx, float* weight, int64_t T_
   if (top > NT) return fail(GBXM_ERR_UNSUPPORTED, "route_topk: top > %d", NT);
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
+  if (E <= RANK_EXPERTS) route_topk_rank_kernel<<<dim3(T_), NT, 0, s>>>(logits, idx, weight, E, top, renorm);
+  else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
   return after_launch("route_topk");
 }
 

@@ -136,17 +136,6 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
   auto at = [&](int e) { const float v = lr[e]; return v == v ? v : -INFINITY; };
   for (int e = tid; e < (E + 3) / 4 * 4; e += nth) cl[e] = e < E ? at(e) : -INFINITY;
   __syncthreads();
-  auto rank_of = [&](const float* v, int n4, int e, float x) {
-    int rank = 0;
-#pragma unroll 8
-    for (int j = 0; j < n4; ++j) {
-      const float4 u = *reinterpret_cast<const float4*>(v + 4 * j);
-      const float w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) rank += (w[k] > x || (w[k] == x && 4 * j + k < e)) ? 1 : 0;
-    }
-    return rank;
-  };
   if (sigmoid) {                                       // (its order is the logits' order)
     for (int e = tid; e < E; e += nth) {
       const int rank = rank_of(cl, (E + 3) / 4, e, cl[e]);
