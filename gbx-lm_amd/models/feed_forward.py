@@ -13,6 +13,8 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .projection import project
+
 ACTIVATIONS = ("relu2", "gelu_tanh")
 
 
@@ -42,7 +44,7 @@ class DenseFeedForward(nn.Module):
             p.requires_grad_(False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(activate_(F.linear(h, self.up.weight), self.activation), self.down.weight)
+        return project(activate_(project(h, self.up.weight), self.activation), self.down.weight)
 
 
 GLU_KINDS = ("silu", "clamped_swish", "gelu_tanh", "sigmoid")
@@ -103,4 +105,4 @@ class GatedDenseFeedForward(nn.Module):
             p.requires_grad_(False)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(glu_(F.linear(h, self.gate_up.weight, self.gate_up.bias), self.kind), self.down.weight, self.down.bias)
+        return project(glu_(project(h, self.gate_up.weight, self.gate_up.bias), self.kind), self.down.weight, self.down.bias)

@@ -25,10 +25,10 @@ import math
 from typing import Optional
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .cache import SlotStateCache
+from .projection import project
 from .recurrent_mixers import conv_tail_update
 
 
@@ -124,10 +124,10 @@ class GatedLRUBlock(nn.Module):
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
         c = self.lru_width
-        xy = F.linear(h, self.inp.weight, self.inp.bias)
+        xy = project(h, self.inp.weight, self.inp.bias)
         cache.reserve(xy.dtype, xy.device)
         u = causal_conv_rows(xy[:, :c], self.conv, self.conv_bias, cache, batch)
         if self.taps > 1:
             conv_tail_update(xy, c, cache, batch)
         logits = block_gate_logits(u, self.gates, self.gates_bias, self._gates_f32_t() if (u.is_cuda and u.shape[0] > 16) else None)
-        return F.linear(gated_lru_scan(u, logits, self.lam_sp, xy[:, c:], self.rate, cache, batch), self.o.weight)
+        return project(gated_lru_scan(u, logits, self.lam_sp, xy[:, c:], self.rate, cache, batch), self.o.weight)

@@ -21,12 +21,12 @@ from dataclasses import dataclass
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from ..batching import StepBatch
 from .base import BaseModelArgs
 from .feed_forward import glu_
+from .projection import project
 from .recurrent_mixers import Retention, StateSpaceDual
 from .residual import StreamRMSNorm, layer_update_
 from .sink_attention import ChunkedAttention
@@ -93,7 +93,7 @@ class Layer(nn.Module):
         """``h`` = this layer's norm of the fp32 stream ``x``.  Updates ``x`` in place (and leaves its image in ``image``); returns the next
         run's norm of it if ``next_norm`` is given."""
         t, n, ff = h.shape[0], self.mixer.ctx_width, self.shared_ff
-        y = F.linear(h, self.inp.weight)
+        y = project(h, self.inp.weight)
         full = n % 8 == 0 and ff % 8 == 0                             # no empty channels between the parts
         rows = (torch.empty if full else torch.zeros)((t, self.o.in_features), dtype=h.dtype, device=h.device)
         self.mixer.mix(y[:, :self.mixer.in_rows], batch, cache, rows[:, :n])
@@ -102,7 +102,7 @@ class Layer(nn.Module):
             cand, w = self.routed(h)
         if ff:
             glu_(y[:, self.mixer.in_rows:self.mixer.in_rows + 2 * ff], "silu", row_scale=w[:, self.routed.top], out=rows[:, self.off_ff:self.off_ff + ff])
-        return layer_update_(x, F.linear(rows, self.o.weight), cand, w, next_norm, image)
+        return layer_update_(x, project(rows, self.o.weight), cand, w, next_norm, image)
 
 
 class LeripelModel(nn.Module):
@@ -152,7 +152,7 @@ class Model(RaggedStepModel):
             if enters:
                 if n == 0:
                     pair[:, :width].copy_(pair[:, width:])
-                h = layer_update_(x, F.linear(pair, self.model.loop_in.weight), None, None, layer.norm1, replace=True)
+                h = layer_update_(x, project(pair, self.model.loop_in.weight), None, None, layer.norm1, replace=True)
             elif n == 0:
                 h = layer.norm1(x, dt)
             after = runs[n + 1] if n + 1 < len(runs) else None

@@ -19,6 +19,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .base import BaseModelArgs, cache_offset, create_attention_mask, scaled_dot_product_attention, swiglu
+from .projection import RowLinear
 from .qllama import RMSNorm
 from .quantized_linear_gba import QuantizedLinear
 from .rope_utils import RoPE, YarnRoPE, yarn_get_mscale
@@ -222,7 +223,7 @@ class Model(nn.Module):
         self.args = config
         self.model_type = config.model_type
         self.model = DeepseekV3Model(config)
-        self.lm_head = nn.Linear(config.hidden_size, config.vocab_size, bias=False)
+        self.lm_head = RowLinear(config.hidden_size, config.vocab_size, bias=False)
         self.lm_head.weight.requires_grad_(False)
 
     def forward(self, inputs, cache=None, mask=None, hidden_states: bool = False):

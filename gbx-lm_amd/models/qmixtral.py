@@ -17,6 +17,7 @@ from torch import nn
 from .. import ops
 from . import qllama
 from .base import BaseModelArgs, create_attention_mask
+from .projection import RowLinear
 from .switch_layers import SwitchGLU
 
 
@@ -111,7 +112,7 @@ class Model(nn.Module):
         self.args = args
         self.model_type = args.model_type
         self.model = MixtralModel(args)
-        self.lm_head = nn.Linear(args.hidden_size, args.vocab_size, bias=False)
+        self.lm_head = RowLinear(args.hidden_size, args.vocab_size, bias=False)
         self.lm_head.weight.requires_grad_(False)
 
     def forward(self, inputs, mask=None, cache=None, hidden_states: bool = False):

@@ -17,6 +17,7 @@ from torch import nn
 
 from .base import (BaseModelArgs, cache_offset, create_attention_mask, rope_keys_and_update_cache, scaled_dot_product_attention,
                    swiglu)
+from .projection import RowLinear
 from .qllama import RMSNorm
 from .quantized_linear_gba import QuantizedLinear
 from .rope_utils import RoPE, SuScaledRotaryEmbedding
@@ -143,7 +144,7 @@ class Model(nn.Module):
         self.args = args
         self.model_type = args.model_type
         self.model = Phi3Model(args)
-        self.lm_head = nn.Linear(args.hidden_size, args.vocab_size, bias=False)
+        self.lm_head = RowLinear(args.hidden_size, args.vocab_size, bias=False)
         self.lm_head.weight.requires_grad_(False)
 
     def forward(self, inputs, mask=None, cache=None, hidden_states: bool = False):

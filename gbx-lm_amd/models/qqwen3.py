@@ -11,10 +11,10 @@ from dataclasses import dataclass
 from typing import Any, Dict, List, Optional, Union
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .base import BaseModelArgs, create_attention_mask
+from .projection import project
 from .qllama import RMSNorm
 from .qqwen3_moe import MLP, Attention as _QKNormAttention
 
@@ -93,7 +93,7 @@ class Model(nn.Module):
 
     def forward(self, inputs, mask=None, cache=None, hidden_states: bool = False):
         out = self.model(inputs, mask, cache)
-        logits = F.linear(out, self.head_weight())
+        logits = project(out, self.head_weight())
         return (logits, out) if hidden_states else logits
 
     def sanitize(self, weights: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
@@ -110,7 +110,7 @@ class Model(nn.Module):
         """``self(inputs, cache=cache)[:, -1, :]`` (gbx_lm/utils.py:291-294) with the output head applied to the last
         position only -- at a 4096-token prompt the full head is 2 x 4096 x vocab x hidden flops of discarded work."""
         hidden = self.model(inputs, None, cache)
-        return F.linear(hidden[:, -1:, :], self.head_weight())[:, -1, :]
+        return project(hidden[:, -1:, :], self.head_weight())[:, -1, :]
 
     def decode_step(self, y: torch.Tensor, prompt_cache) -> torch.Tensor:
         """Single-token fast path: the hand-fused five-launch block of the Llama graph when the checkpoint qualifies (the

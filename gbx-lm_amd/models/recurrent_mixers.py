@@ -37,6 +37,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .cache import SlotStateCache
+from .projection import project
 
 GATE_SILU, GATE_SIGMOID = 1, 2
 
@@ -268,7 +269,7 @@ class _RecurrentMixer(nn.Module):
         if self.taps > 1:
             conv_tail_update(y, 2 * lay.nq + lay.nv, cache, batch)
         o = decayed_state_scan(r, lay, cache, batch, self.delta)
-        return F.linear(head_norm_gate(o, gate, self.out_norm, 1 if self.norm_heads_together else lay.heads, self.eps, self.gate_kind), self.o.weight)
+        return project(head_norm_gate(o, gate, self.out_norm, 1 if self.norm_heads_together else lay.heads, self.eps, self.gate_kind), self.o.weight)
 
 
 class GatedLinearAttention(_RecurrentMixer):
@@ -292,8 +293,8 @@ class GatedLinearAttention(_RecurrentMixer):
             p.requires_grad_(False)
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
-        y = F.linear(h, self.inp.weight)
-        a = F.linear(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight)
+        y = project(h, self.inp.weight)
+        a = project(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight)
         return self._mix(y, a, y[:, self.off_gate:self.off_gate + self.layout.nv], batch, cache)
 
 
@@ -323,7 +324,7 @@ class LightningAttention(_RecurrentMixer):
             p.requires_grad_(False)
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
-        y = F.linear(h, self.inp.weight)
+        y = project(h, self.inp.weight)
         return self._mix(y, None, y[:, self.off_gate:self.off_gate + self.layout.nv], batch, cache)
 
 
@@ -367,9 +368,9 @@ class ChannelDeltaRule(_RecurrentMixer):
         return w
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
-        y = F.linear(h, self.inp.weight)
-        a = F.linear(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight)
-        gate = F.linear(y[:, self.off_g1:self.off_g1 + self.gate_rank], self.g2.weight)
+        y = project(h, self.inp.weight)
+        a = project(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight)
+        gate = project(y[:, self.off_g1:self.off_g1 + self.gate_rank], self.g2.weight)
         return self._mix(y, a, gate, batch, cache)
 
 
@@ -404,7 +405,7 @@ class Retention(nn.Module):
         return head_norm_gate(o, y[:, self.off_gate:self.off_gate + self.ctx_width], None, self.heads, self.eps, GATE_SILU, out)
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
-        return F.linear(self.mix(F.linear(h, self.inp.weight), batch, cache), self.o.weight)
+        return project(self.mix(project(h, self.inp.weight), batch, cache), self.o.weight)
 
 
 class StateSpaceDual(nn.Module):
@@ -446,4 +447,4 @@ class StateSpaceDual(nn.Module):
         return gate_group_norm(o, y[:, :self.inner], self.out_norm, self.norm_groups, self.eps, out)
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
-        return F.linear(self.mix(F.linear(h, self.inp.weight), batch, cache), self.o.weight)
+        return project(self.mix(project(h, self.inp.weight), batch, cache), self.o.weight)

@@ -35,10 +35,10 @@ from dataclasses import dataclass
 from typing import List, Optional
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .cache import SharedLatentRows, SlotKVCache
+from .projection import project
 from .rope_utils import rotary_table
 
 NORM_NONE, NORM_UNIT, NORM_WEIGHT = 0, 1, 2
@@ -214,7 +214,7 @@ class RotatedValueWindowAttention(nn.Module):
 
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
         t = h.shape[0]
-        qkv = F.linear(h, self.qkv.weight)
+        qkv = project(h, self.qkv.weight)
         pos = batch.tok[:, 1]
         rotate_norm_heads_(qkv, pos, [
             HeadSegment(0, self.heads, self.dim, 0, self.rot_dims, self.freq, self.rot_mult, norm=NORM_UNIT),
@@ -226,7 +226,7 @@ class RotatedValueWindowAttention(nn.Module):
                           v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, self.keep_first, self.sink)
         rotate_norm_heads_(ctx, pos, [HeadSegment(0, self.heads, self.vdim, 0, self.vdim, self.vfreq, sign=-1.0)], self.eps)
         cache_append(cache, k_rows, v_rows, batch)
-        return F.linear(ctx, self.o.weight)
+        return project(ctx, self.o.weight)
 
 
 class GatedSinkWindowAttention(nn.Module):
@@ -272,7 +272,7 @@ class GatedSinkWindowAttention(nn.Module):
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
         from .feed_forward import gate_mul
         t = h.shape[0]
-        y = F.linear(h, self.inp.weight, self.inp.bias)
+        y = project(h, self.inp.weight, self.inp.bias)
         pos = batch.tok[:, 1]
         rotate_norm_heads_(y, pos, [
             HeadSegment(0, self.heads, self.dim, 0, self.rot_dims, self.freq, self.rot_mult, norm=NORM_WEIGHT, weight=self.q_norm, norm_first=True),
@@ -283,7 +283,7 @@ class GatedSinkWindowAttention(nn.Module):
         ctx = sink_attend(y[:, :self.nq].view(t, self.heads, self.dim), k_rows.view(t, self.kv_heads, self.dim),
                           v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, 0, self.sink)
         cache_append(cache, k_rows, v_rows, batch)
-        return F.linear(gate_mul(y[:, self.off_gate:self.off_gate + self.ng], ctx, "sigmoid"), self.o.weight, self.o.bias)
+        return project(gate_mul(y[:, self.off_gate:self.off_gate + self.ng], ctx, "sigmoid"), self.o.weight, self.o.bias)
 
 
 class ChunkedAttention(nn.Module):
@@ -333,7 +333,7 @@ class ChunkedAttention(nn.Module):
         return ctx
 
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
-        return F.linear(self.mix(F.linear(h, self.inp.weight), batch, cache), self.o.weight)
+        return project(self.mix(project(h, self.inp.weight), batch, cache), self.o.weight)
 
 
 class SharedKeyValueAttention(nn.Module):
@@ -376,7 +376,7 @@ class SharedKeyValueAttention(nn.Module):
 
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
         d, r = self.dim, self.rot_dims
-        y = F.linear(h, self.inp.weight)
+        y = project(h, self.inp.weight)
         if r:
             rotate_norm_heads_(y, batch.tok[:, 1], [HeadSegment(0, self.heads, d, d - r, r, self.freq),
                                                     HeadSegment(self.off_k, self.kv_heads, self.head_row, d, r, self.freq)], 0.0)
@@ -385,7 +385,7 @@ class SharedKeyValueAttention(nn.Module):
         heads = rows.unflatten(1, (self.kv_heads, self.head_row))
         ctx = sink_attend(y[:, :self.nq].unflatten(1, (self.heads, d)), heads[:, :, r:], heads[:, :, :d], cache, batch, self.scale, None, 0, self.sink)
         cache_append(cache, rows, None, batch)
-        return F.linear(ctx, self.o.weight)
+        return project(ctx, self.o.weight)
 
 
 class LatentAttention(nn.Module):
@@ -458,7 +458,7 @@ class LatentAttention(nn.Module):
 
     def forward(self, h: torch.Tensor, batch, cache) -> torch.Tensor:
         t, hd, d, r, dv, rank = h.shape[0], self.heads, self.dim, self.rot_dim, self.vdim, self.kv_rank
-        y = F.linear(h, self.inp.weight)
+        y = project(h, self.inp.weight)
         pos = batch.tok[:, 1]
         turn = HeadSegment(0, hd, self.dk, d, r, self.freq, self.rot_mult, interleaved=self.interleaved) if r else None
         if self.q_rank is not None:
@@ -472,7 +472,7 @@ class LatentAttention(nn.Module):
         if segments:
             rotate_norm_heads_(y, pos, segments, self.eps)
         if self.q_rank is not None:                                                # (these queries are turned further down)
-            q = F.linear(y[:, :self.n_first], self.uq.weight).view(t, hd, self.dk)
+            q = project(y[:, :self.n_first], self.uq.weight).view(t, hd, self.dk)
         else:
             q, turn = y[:, :self.nq].view(t, hd, self.dk), None
         gate = y[:, self.off_gate:self.off_gate + self.n_gate] if self.gated else None
@@ -486,7 +486,7 @@ class LatentAttention(nn.Module):
                 raise RuntimeError("the mixer that owns the latent rows has not run in this step")
         if not any(batch.pos0) and not batch.decode_only:           # (one-token steps always take the form below: a captured step
                                                                     # is replayed at later positions)
-            kv = F.linear(latent[:, :rank], self.up.weight)
+            kv = project(latent[:, :rank], self.up.weight)
             keys = kv[:, :self.nq].view(t, hd, self.dk)
             if r:
                 keys[:, :, d:] = latent[:, None, rank:]
@@ -502,4 +502,4 @@ class LatentAttention(nn.Module):
         if self.own_latent:
             cache_append(cache, latent, None, batch)
             cache.step_rows = latent                                # for mixers that attend over these rows later in the step
-        return F.linear(ctx, self.o.weight)
+        return project(ctx, self.o.weight)

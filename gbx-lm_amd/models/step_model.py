@@ -11,11 +11,11 @@ from __future__ import annotations
 from typing import Any, Dict, List, Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from ..batching import StepBatch
 from .cache import SequenceSlots
+from .projection import project
 
 
 def loop_runs(n_layers: int, loop: Optional[Dict[str, int]]) -> List[Tuple[int, bool]]:
@@ -66,7 +66,7 @@ class RaggedStepModel(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         """Last norm and output head on rows of the stream."""
         w = self.lm_head.weight
-        return F.linear(self.model.norm(x, w.dtype), w)
+        return project(self.model.norm(x, w.dtype), w)
 
     def _run(self, inputs: torch.Tensor, cache):
         b, l = inputs.shape

@@ -18,13 +18,13 @@ from dataclasses import dataclass
 from typing import Any, Dict, List, Optional
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from ..batching import StepBatch
 from .base import BaseModelArgs
 from .cache import SequenceSlots
 from .feed_forward import GatedDenseFeedForward
+from .projection import project
 from .recurrent_mixers import ChannelDeltaRule, GatedLinearAttention
 from .residual import StreamLayerNorm, hyper_step_
 from .sink_attention import LatentAttention
@@ -168,7 +168,7 @@ class Model(RaggedStepModel):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         """Last norm, output head and the logit scale (applied in fp32) on rows of the summed stream."""
         w = self.lm_head.weight
-        return F.linear(self.model.norm(x, w.dtype), w).float() * self.logit_scale
+        return project(self.model.norm(x, w.dtype), w).float() * self.logit_scale
 
     @staticmethod
     def shapes_from(weights: Dict[str, torch.Tensor], config: Dict[str, Any]) -> Dict[int, Dict[str, int]]:

@@ -19,10 +19,10 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from .cache import WindowKVCache
+from .projection import project
 
 
 def segment_rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -81,7 +81,7 @@ class GatedWindowAttention(nn.Module):
 
     def forward(self, h: torch.Tensor, batch, cache: WindowKVCache) -> torch.Tensor:
         """h [T, width] (the step's rows back to back) -> [T, width]; the step's keys / values are in ``cache`` afterwards."""
-        qkv = F.linear(h, self.qkv.weight)
+        qkv = project(h, self.qkv.weight)
         cache.reserve(qkv[:, self.nq:self.nq + self.nk], qkv[:, self.nq + self.nk:])
         if h.is_cuda:
             from .. import mixer_ops as M
@@ -101,4 +101,4 @@ class GatedWindowAttention(nn.Module):
             for slot, pos0, n in zip(batch.slot, batch.pos0, batch.n_new):       # append only after every query has attended
                 cache.append_rows(k[r0:r0 + n], v[r0:r0 + n], slot, pos0)
                 r0 += n
-        return F.linear(ctx, self.o.weight)
+        return project(ctx, self.o.weight)

@@ -1,0 +1,49 @@
+"""Products of few rows (csrc/mixers_rows.hip) against float64: one row to the last row of each tile, contractions of one block to the last one of every
+wave count, outputs that end inside a tile or fill several rounds of workgroups, rows with a stride, a bias; and what stays with the library.
+Tolerance: K fp32 additions of the terms' magnitudes in the worst case, one rounding to bf16."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def case(t, n, k, bias, pad, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rnd = lambda *s: torch.randn(s, device=DEV, generator=g).bfloat16()
+    x = rnd(t, k + pad)[:, pad // 2 // 8 * 8:][:, :k]
+    return x, rnd(n, k) * 0.05, (rnd(n) if bias else None)
+
+
+@pytest.mark.parametrize("t", [1, 2, 15, 16, 17, 31, 32])
+@pytest.mark.parametrize("n,k,bias,pad", [(1, 64, False, 0), (15, 448, True, 0), (17, 512, False, 16), (2048, 576, False, 8), (4100, 1024, True, 0),
+                                          (33, 1088, False, 0), (8193, 2048, False, 64), (16, 2112, True, 0), (4113, 4096, False, 0)])
+def test_rows(t, n, k, bias, pad):
+    from gbx_lm_amd import mixer_ops as M
+    x, w, b = case(t, n, k, bias, pad, t + n + k)
+    y = M.linear_rows(x, w, b)
+    if t > 16 and k > 2048:
+        assert y is None
+        return
+    want, room = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    if bias:
+        want, room = want + b.double(), room + b.double().abs()
+    assert y.shape == (t, n) and bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (k + 1) * 2.0 ** -24 * room).all())
+    if t > 1:                                                  # a row's bits do not depend on the rows beside it
+        assert torch.equal(M.linear_rows(x[:1], w, b), y[:1])
+
+
+def test_what_stays_with_the_library():
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.models.projection import project
+    x, w, b = case(4, 48, 256, True, 0, 3)
+    for xx, ww, bb in ((x[:0], w, b), (x.float(), w.float(), b.float()), (x[:, :40], w[:, :40].contiguous(), b), (x.half(), w.half(), b.half()),
+                       (x.t().contiguous().t(), w, b), (x, w.t().contiguous().t(), b), (x.expand(4, 4, 256).reshape(16, 256)[:1].expand(3, 256), w, b),
+                       (torch.cat([x] * 9), w, b), (torch.cat([x] * 17, 1), torch.cat([w] * 17, 1), b)):
+        assert M.linear_rows(xx, ww, bb) is None
+        assert torch.equal(project(xx, ww, bb), F.linear(xx, ww, bb))
+    y = project(x.view(2, 2, 256), w, b)
+    assert y.shape == (2, 2, 48) and torch.equal(y.view(4, 48), M.linear_rows(x, w, b))
+    wg = w.clone().requires_grad_(True)
+    assert project(x, wg, b).requires_grad and not project(x, wg.detach(), b).requires_grad
