@@ -112,16 +112,22 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 
 // NW waves per workgroup = 4 NW columns of one (sequence, head).  The operands of CH tokens (q | k | decay padded to 16 R channels, the
-// workgroup's value columns, beta) are staged in LDS, shared by the waves, two buffers: the next chunk is fetched into registers before
-// the current one is computed and parked in the other buffer afterwards, one barrier per chunk.  Lane ks of a 16-lane row owns the key
-// channels ks, ks + 16, ...: LDS reads and the state's loads and stores are contiguous over the row.
-template <int R, bool DELTA, int NW>
+// workgroup's value columns; the betas beside them) are staged in LDS, shared by the waves, two buffers: the next chunk is fetched into registers
+// before the current one is computed and parked in the other buffer afterwards, one barrier per chunk.  Lane ks of a 16-lane row owns the key
+// channels 4 ks .. 4 ks + 3, and those 64, 128, ... further on: LDS reads, and the state's loads and stores, are 16-byte accesses that are
+// contiguous over the row.  Bound by issue slots (a long prompt leaves one or two waves a SIMD, each token costs a wave 4 R multiply-adds and what
+// feeds them), so operands are read four at a time: V = 4 floats per staging access where sizes, strides and addresses allow, else 1.
+// (4-byte accesses and operands read where they are used -> now, us: rows of 1501 + 700 + 65 tokens, 8 heads of 128 x 256 393 -> 253, delta rule over 32
+// of 128 x 128 507 -> 351; 32 prompts of 8 to 163 tokens 273 -> 144; one token of 32 sequences, 67 MB of state 30.1 -> 15.1.)
+template <int R, bool DELTA, int NW, int V>
 __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __restrict__ r, int64_t r_stride, float* __restrict__ state,
                                                             float* __restrict__ out, const int* __restrict__ seq, int H, int G, int dk, int dv) {
-  constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL + 1, NTH = 64 * NW;
+  static_assert(R % 4 == 0, "four neighbouring channels per access");
+  constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL, NTH = 64 * NW, Q = R / 4;
   constexpr int CH = NW == 1 ? (R <= 4 ? 4 : 2) : (R <= 4 ? 32 : (R <= 8 ? 16 : 8)) * NW / 4;     // one-wave workgroups serve steps of few rows
-  constexpr int PF = (CH * ROW + NTH - 1) / NTH;
-  __shared__ float buf[2][CH * ROW];
+  constexpr int SLOTS = CH * ROW / V, PF = (SLOTS + NTH - 1) / NTH;
+  __shared__ __attribute__((aligned(16))) float buf[2][CH * ROW];
+  __shared__ float betas[2][CH];
   const int b = blockIdx.z, h = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ks = lane & 15;
   const int col0 = blockIdx.x * NCOL, lcol = wave * 4 + (lane >> 4), col = col0 + lcol;
@@ -130,55 +136,61 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
   const int colc = col_ok ? col : dv - 1;
   const int nq = G * dk, nv = H * dv;
   const int g = h / (H / G);
-  float* sp = state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk + min(ks, dk - 1);     // (a lane past the last channel holds zeros)
+  float* sp = state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;     // (channels past the last one hold zeros)
   // every load below is issued unconditionally from an address inside the buffers (what it must not deliver is replaced afterwards):
   // loads under a branch wait for one another, and a chunk's fetch then costs the sum of their latencies
   float S[R];
 #pragma unroll
-  for (int i = 0; i < R; ++i) S[i] = sp[ks + 16 * i < dk ? 16 * i : 0];
+  for (int i = 0; i < Q; ++i) {
+    const int c = 4 * ks + 64 * i;
+    if constexpr (V == 4) {
+      Lanes<float, 4>::load(sp + min(c, dk - 4), S + 4 * i);
+    } else {
 #pragma unroll
-  for (int i = 0; i < R; ++i) S[i] = (pos0 > 0 && ks + 16 * i < dk) ? S[i] : 0.f;
+      for (int j = 0; j < 4; ++j) S[4 * i + j] = sp[min(c + j, dk - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S[4 * i + j] = (pos0 > 0 && c + j < dk) ? S[4 * i + j] : 0.f;
+  }
   const float* base = r + static_cast<int64_t>(row0) * r_stride;
   const int oq = g * dk, ok = nq + g * dk, ov = 2 * nq + h * dv, og = 2 * nq + nv + h * dk, ob = 2 * nq + nv + H * dk + h;
-  float pf[PF];
+  float pf[PF][V], pb = 0.f;
   int offs[PF], tts[PF];                    // where slot i of this thread's share of a chunk comes from: token of the chunk, offset in its row
-  unsigned loaded = 0;                      // bit i: pf[i] is an operand (else the slot's neutral value: 1 for a decay, 0 elsewhere)
+  unsigned loaded = 0, decays = 0;          // bit i: pf[i] is an operand (else the slot's neutral value: 1 for a decay, 0 elsewhere)
+  static_assert(PF <= 32, "a bit per slot");
 #pragma unroll
   for (int i = 0; i < PF; ++i) {
-    const int idx = min(static_cast<int>(threadIdx.x) + i * NTH, CH * ROW - 1);
-    const int tt = idx / ROW, j = idx - tt * ROW;
+    const int idx = min(static_cast<int>(threadIdx.x) + i * NTH, SLOTS - 1);
+    const int tt = idx / (ROW / V), j = (idx - tt * (ROW / V)) * V;
     const int seg = j < DKP ? 0 : (j < 2 * DKP ? 1 : (j < 3 * DKP ? 2 : 3));
-    const int jj = j - seg * DKP;                                     // segment 3: the value columns, then beta
-    const bool is_beta = seg == 3 && jj == NCOL;
+    const int jj = j - seg * DKP;                                     // segment 3: the value columns
     const int first = seg == 0 ? oq : (seg == 1 ? ok : (seg == 2 ? og : ov + col0));
-    const int count = seg < 3 ? dk : min(dv - col0, NCOL);
-    const bool valid = is_beta ? DELTA : jj < count;
-    offs[i] = valid ? (is_beta ? ob : first + jj) : oq;
+    const bool valid = jj < (seg < 3 ? dk : min(dv - col0, NCOL));
+    offs[i] = valid ? first + jj : oq;
     tts[i] = tt;
     loaded |= static_cast<unsigned>(valid) << i;
+    decays |= static_cast<unsigned>(seg == 2) << i;
   }
   auto fetch = [&](int t0) {
     const float* cb = base + static_cast<int64_t>(t0) * r_stride;
-    if (t0 + CH <= n) {
+    const int last = min(CH, n - t0) - 1;   // the sequence's last chunk: rows past its end are read as its last row (and never used)
 #pragma unroll
-      for (int i = 0; i < PF; ++i) pf[i] = cb[static_cast<int64_t>(tts[i]) * r_stride + offs[i]];
-    } else {                                // the sequence's last chunk: rows past its end are read as its last row (and never used)
-      const int last = n - 1 - t0;
-#pragma unroll
-      for (int i = 0; i < PF; ++i) pf[i] = cb[static_cast<int64_t>(min(tts[i], last)) * r_stride + offs[i]];
-    }
+    for (int i = 0; i < PF; ++i) Lanes<float, V>::load(cb + static_cast<int64_t>(min(tts[i], last)) * r_stride + offs[i], pf[i]);
+    if (DELTA) pb = cb[static_cast<int64_t>(min(static_cast<int>(threadIdx.x), last)) * r_stride + ob];
   };
-  auto park = [&](float* dst) {
+  auto park = [&](int which) {
 #pragma unroll
     for (int i = 0; i < PF; ++i) {
       const int idx = threadIdx.x + i * NTH;
-      const int j = idx % ROW;
-      const float neutral = ((j >= 2 * DKP && j < 3 * DKP) || j == ROW - 1) ? 1.f : 0.f;
-      if (idx < CH * ROW) dst[idx] = ((loaded >> i) & 1u) ? pf[i] : neutral;
+      const float neutral = (decays >> i) & 1u ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < V; ++j) pf[i][j] = ((loaded >> i) & 1u) ? pf[i][j] : neutral;
+      if (idx < SLOTS) Lanes<float, V>::store(buf[which] + idx * V, pf[i]);
     }
+    if (DELTA && static_cast<int>(threadIdx.x) < CH) betas[which][threadIdx.x] = pb;
   };
   fetch(0);
-  park(buf[0]);
+  park(0);
   __syncthreads();
   float* op = out + static_cast<int64_t>(row0) * nv + h * dv + colc;
   int which = 0;
@@ -187,36 +199,67 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
     if (more) fetch(t0 + CH);
     const float* cur = buf[which];
     const int cn = min(CH, n - t0);
-#pragma unroll 2
-    for (int tt = 0; tt < cn; ++tt) {
-      const float* row = cur + tt * ROW;
-      float q[R], k[R];
+    struct Token { float q[R], k[R], d[R], v, beta; };
+    auto read = [&](int tt, Token& x) {
+      const float* at = cur + tt * ROW + 4 * ks;
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        q[i] = row[ks + 16 * i];
-        k[i] = row[DKP + ks + 16 * i];
-        S[i] *= row[2 * DKP + ks + 16 * i];
+      for (int i = 0; i < Q; ++i) {
+        Lanes<float, 4>::load(at + 64 * i, x.q + 4 * i);
+        Lanes<float, 4>::load(at + DKP + 64 * i, x.k + 4 * i);
+        Lanes<float, 4>::load(at + 2 * DKP + 64 * i, x.d + 4 * i);
       }
-      float u = row[3 * DKP + lcol];
+      x.v = cur[tt * ROW + 3 * DKP + lcol];
+      if (DELTA) x.beta = betas[which][tt];
+    };
+    auto step = [&](int tt, const Token& x) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) S[i] *= x.d[i];
+      float u = x.v;
       if constexpr (DELTA) {
-        float dot = 0.f;
+        float dot[2] = {0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < R; ++i) dot += k[i] * S[i];
-        u = row[3 * DKP + NCOL] * (u - row16_sum(dot));
+        for (int i = 0; i < R; ++i) dot[i & 1] += x.k[i] * S[i];
+        u = x.beta * (u - row16_sum(dot[0] + dot[1]));
       }
-      float o = 0.f;
+      float o[2] = {0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < R; ++i) { S[i] += k[i] * u; o += q[i] * S[i]; }
-      o = row16_sum(o);
-      if (ks == 0 && col_ok) op[static_cast<int64_t>(t0 + tt) * nv] = o;
+      for (int i = 0; i < R; ++i) { S[i] += x.k[i] * u; o[i & 1] += x.q[i] * S[i]; }
+      const float sum = row16_sum(o[0] + o[1]);
+      if (ks == 0 && col_ok) op[static_cast<int64_t>(t0 + tt) * nv] = sum;
+    };
+    Token x;
+    if constexpr (NW > 1) {                  // a token's operands are read while the one before it is computed
+      Token y;
+      read(0, x);
+      int tt = 0;
+      for (; tt + 1 < cn; tt += 2) {
+        read(tt + 1, y);
+        step(tt, x);
+        read(min(tt + 2, cn - 1), x);
+        step(tt + 1, y);
+      }
+      if (tt < cn) step(tt, x);
+    } else {                                 // few tokens, many sequences: the registers serve occupancy
+      for (int tt = 0; tt < cn; ++tt) {
+        read(tt, x);
+        step(tt, x);
+      }
     }
-    if (more) park(buf[which ^ 1]);
+    if (more) park(which ^ 1);
     __syncthreads();
   }
   if (col_ok) {
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-      if (ks + 16 * i < dk) sp[16 * i] = S[i];
+    for (int i = 0; i < Q; ++i) {
+      const int c = 4 * ks + 64 * i;
+      if constexpr (V == 4) {
+        if (c < dk) Lanes<float, 4>::store(sp + c, S + 4 * i);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < dk) sp[c + j] = S[4 * i + j];
+      }
+    }
   }
 }
 
@@ -245,12 +288,13 @@ template <bool DELTA, int NW>
 int launch_scan(int R, int B, hipStream_t s, const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int H, int G, int dk,
                 int dv) {
   const dim3 grid((dv + 4 * NW - 1) / (4 * NW), H, B);
-#define GBXM_SCAN(N) state_scan_kernel<N, DELTA, NW><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv)
-  if (R <= 1) GBXM_SCAN(1);
-  else if (R <= 2) GBXM_SCAN(2);
-  else if (R <= 3) GBXM_SCAN(3);
-  else if (R <= 4) GBXM_SCAN(4);
-  else if (R <= 6) GBXM_SCAN(6);
+  const bool vec = dk % 4 == 0 && dv % 4 == 0 && r_stride % 4 == 0 && all_aligned(16, r, state);
+#define GBXM_SCAN(N)                                                                                                    \
+  do {                                                                                                                  \
+    if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);   \
+    else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);       \
+  } while (0)
+  if (R <= 4) GBXM_SCAN(4);
   else if (R <= 8) GBXM_SCAN(8);
   else if (R <= 12) GBXM_SCAN(12);
   else GBXM_SCAN(16);
