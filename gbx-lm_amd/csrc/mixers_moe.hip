@@ -3,9 +3,9 @@
 // factor meets the fp32 sums of its first products.
 //
 //   * row kernels -- weight-bandwidth bound: the kernels of decode steps, of fp32 models and of shapes the grouped kernel does not
-//     take.  Two launches so that even ONE row spreads over the chip: expert_up_rows (a workgroup = one (row, choice) pair x 8 hidden
-//     channels, a wave per channel pair gate / up, lanes across the contraction with 16-byte loads, fp32 sums in a fixed order)
-//     leaves the hidden row in the workspace, expert_down_rows (a pair x 16 output channels) consumes it.
+//     take.  Two launches so that even ONE row spreads over the chip: the first (a workgroup = one (row, choice) pair x some hidden
+//     channels, lanes across the contraction, fp32 sums in a fixed order) leaves the hidden row in the workspace, the second (a pair x 16
+//     output channels) consumes it.  expert_up_vec / expert_down_vec where rows are whole 16-byte vectors, else expert_up_rows / _down_rows.
 //   * grouped matrix-core products for bf16 prompt portions (rows sorted by expert on the device, no host round trip).
 #include "mixers_common.h"
 
@@ -16,34 +16,94 @@ constexpr int NT = 256, NW = NT / 64;
 constexpr int FC = 8;             // hidden channels per workgroup of expert_up_rows
 constexpr int KC = 16;            // output channels per workgroup of expert_down_rows
 
-// sum_k w[k] * x[k] over this lane's share of n elements; x in LDS (fp32).  VEC: n is a multiple of the 16-byte vector.
-template <typename T, bool VEC>
-__device__ __forceinline__ float lane_dot(const T* __restrict__ w, const float* __restrict__ x, int n, int lane) {
-  float acc = 0.f;
-  if constexpr (VEC) {
-    constexpr int PER = 16 / sizeof(T);
-    for (int k = lane * PER; k < n; k += 64 * PER) {
-      const uint4 raw = *reinterpret_cast<const uint4*>(w + k);
-      if constexpr (sizeof(T) == 2) {
-        const unsigned u[4] = {raw.x, raw.y, raw.z, raw.w};
+// The vector form.  Four rows of weights per wave, 16 lanes a row: a row's whole sum is four cross-lane adds, the four rows' at once, and the row that
+// they meet is read as it is, from the first cache: nothing is staged and no barrier stands before the weights.  UN steps of 16 lanes x 16 bytes are in
+// flight per matrix.  Bound by the weights' way from memory (16 pairs of 768 x 2048) or one trip to it (4 pairs of 512 x 1024).
+// (Rows staged in LDS, one wave per channel -> now, us: 16 pairs, 768 x 2048, first and second product 17.4 + 17.9 -> 13.1 + 12.3 (4.1 TB/s); 4 gated
+// pairs, 512 x 1024, 7.2 + 5.3 -> 5.9 + 3.8.)
+constexpr int UN = 4;
+
+// s0 = sum_k w0[k] x[k], s1 = sum_k w1[k] x[k] (PAIR), every lane of the 16 gets them; n a multiple of the vector
+template <typename T, bool PAIR>
+__device__ __forceinline__ void rows_dot(const T* __restrict__ w0, const T* __restrict__ w1, const T* __restrict__ x, int n, int l16, float& s0, float& s1) {
+  constexpr int PER = 16 / sizeof(T), STEP = 16 * PER;
+  float a0[2] = {0.f, 0.f}, a1[2] = {0.f, 0.f};
+  for (int k0 = 0; k0 < n; k0 += UN * STEP) {
+    uint4 u[UN], v[UN], y[UN];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc += __uint_as_float(u[i] << 16) * x[k + 2 * i];
-          acc += __uint_as_float(u[i] & 0xFFFF0000u) * x[k + 2 * i + 1];
+    for (int i = 0; i < UN; ++i) {
+      const int k = min(k0 + i * STEP + l16 * PER, n - PER);
+      u[i] = *reinterpret_cast<const uint4*>(w0 + k);
+      if (PAIR) v[i] = *reinterpret_cast<const uint4*>(w1 + k);
+      y[i] = *reinterpret_cast<const uint4*>(x + k);
+    }
+#pragma unroll
+    for (int i = 0; i < UN; ++i) {
+      if (k0 + i * STEP + l16 * PER < n) {
+        const unsigned uu[4] = {u[i].x, u[i].y, u[i].z, u[i].w}, yy[4] = {y[i].x, y[i].y, y[i].z, y[i].w};
+        const unsigned vv[4] = {PAIR ? v[i].x : 0, PAIR ? v[i].y : 0, PAIR ? v[i].z : 0, PAIR ? v[i].w : 0};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (sizeof(T) == 2) {
+            const float lo = __uint_as_float(yy[j] << 16), hi = __uint_as_float(yy[j] & 0xFFFF0000u);
+            a0[0] += __uint_as_float(uu[j] << 16) * lo;
+            a0[1] += __uint_as_float(uu[j] & 0xFFFF0000u) * hi;
+            if (PAIR) {
+              a1[0] += __uint_as_float(vv[j] << 16) * lo;
+              a1[1] += __uint_as_float(vv[j] & 0xFFFF0000u) * hi;
+            }
+          } else {
+            a0[j & 1] += __uint_as_float(uu[j]) * __uint_as_float(yy[j]);
+            if (PAIR) a1[j & 1] += __uint_as_float(vv[j]) * __uint_as_float(yy[j]);
+          }
         }
-      } else {
-        acc += __uint_as_float(raw.x) * x[k] + __uint_as_float(raw.y) * x[k + 1] + __uint_as_float(raw.z) * x[k + 2] + __uint_as_float(raw.w) * x[k + 3];
       }
     }
-  } else {
-    for (int k = lane; k < n; k += 64) acc += to_f32(w[k]) * x[k];
   }
+  s0 = row16_sum(a0[0] + a0[1]);
+  if (PAIR) s1 = row16_sum(a1[0] + a1[1]);
+}
+
+constexpr int VC = 4 * NW;        // channels per workgroup of the vector form
+
+template <typename T, bool FAST, bool GATED>
+__global__ __launch_bounds__(NT) void expert_up_vec(const T* __restrict__ h, const T* __restrict__ first, const int* __restrict__ idx,
+                                                   const float* __restrict__ scale, T* __restrict__ act, int K, int F, int top, int kind, float limit) {
+  const int64_t pair = blockIdx.x;
+  const int lane = threadIdx.x & 63, f = blockIdx.y * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), fc = min(f, F - 1);
+  const T* w = first + (static_cast<int64_t>(idx[pair]) * (GATED ? 2 : 1) * F + fc) * K;
+  float a, u;
+  rows_dot<T, GATED>(w, w + static_cast<int64_t>(F) * K, h + (pair / top) * K, K, lane & 15, a, u);
+  const float sc = scale ? scale[pair] : 1.f;
+  if ((lane & 15) == 0 && f < F) {
+    if constexpr (GATED) a = glu_act<FAST>(sc * a, sc * u, kind, limit, 1.702f);
+    else { a = fmaxf(sc * a, 0.f); a *= a; }
+    act[pair * F + f] = from_f32<T>(a);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(NT) void expert_down_vec(const T* __restrict__ act, const T* __restrict__ down, const int* __restrict__ idx, T* __restrict__ y,
+                                                     int K, int F) {
+  const int64_t pair = blockIdx.x;
+  const int lane = threadIdx.x & 63, c = blockIdx.y * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), cc = min(c, K - 1);
+  float a, unused;
+  const T* w = down + (static_cast<int64_t>(idx[pair]) * K + cc) * F;
+  rows_dot<T, false>(w, w, act + pair * F, F, lane & 15, a, unused);
+  if ((lane & 15) == 0 && c < K) y[pair * K + c] = from_f32<T>(a);
+}
+
+// sum_k w[k] * x[k] over this lane's share of n elements; x in LDS (fp32)
+template <typename T>
+__device__ __forceinline__ float lane_dot(const T* __restrict__ w, const float* __restrict__ x, int n, int lane) {
+  float acc = 0.f;
+  for (int k = lane; k < n; k += 64) acc += to_f32(w[k]) * x[k];
   return acc;
 }
 
 // GATED: first = gate rows over up rows, a wave takes one hidden channel at a time; else first = up rows, a wave takes its two channels of
 // the workgroup's FC = 2 NW together.
-template <typename T, bool FAST, bool VEC, bool GATED>
+template <typename T, bool FAST, bool GATED>
 __global__ __launch_bounds__(NT) void expert_up_rows(const T* __restrict__ h, const T* __restrict__ first, const int* __restrict__ idx,
                                                     const float* __restrict__ scale, T* __restrict__ act, int K, int F, int top, int kind, float limit) {
   static_assert(FC == 2 * NW, "two hidden channels per wave");
@@ -59,8 +119,8 @@ __global__ __launch_bounds__(NT) void expert_up_rows(const T* __restrict__ h, co
   if constexpr (!GATED) {
     const int fa = blockIdx.y * FC + wave, fb = fa + NW;
     if (fa >= F) return;
-    float a = lane_dot<T, VEC>(wg + static_cast<int64_t>(fa) * K, hl, K, lane);
-    float b = lane_dot<T, VEC>(wg + static_cast<int64_t>(min(fb, F - 1)) * K, hl, K, lane);
+    float a = lane_dot<T>(wg + static_cast<int64_t>(fa) * K, hl, K, lane);
+    float b = lane_dot<T>(wg + static_cast<int64_t>(min(fb, F - 1)) * K, hl, K, lane);
     a = fmaxf(sc * wave_sum(a), 0.f);
     b = fmaxf(sc * wave_sum(b), 0.f);
     if (lane == 0) {
@@ -72,13 +132,13 @@ __global__ __launch_bounds__(NT) void expert_up_rows(const T* __restrict__ h, co
   const T* wu = wg + static_cast<int64_t>(F) * K;
   const int f_end = min(F, (static_cast<int>(blockIdx.y) + 1) * FC);
   for (int f = blockIdx.y * FC + wave; f < f_end; f += NW) {
-    const float ag = sc * wave_sum(lane_dot<T, VEC>(wg + static_cast<int64_t>(f) * K, hl, K, lane));
-    const float au = sc * wave_sum(lane_dot<T, VEC>(wu + static_cast<int64_t>(f) * K, hl, K, lane));
+    const float ag = sc * wave_sum(lane_dot<T>(wg + static_cast<int64_t>(f) * K, hl, K, lane));
+    const float au = sc * wave_sum(lane_dot<T>(wu + static_cast<int64_t>(f) * K, hl, K, lane));
     if (lane == 0) act[pair * F + f] = from_f32<T>(glu_act<FAST>(ag, au, kind, limit, 1.702f));
   }
 }
 
-template <typename T, bool VEC>
+template <typename T>
 __global__ __launch_bounds__(NT) void expert_down_rows(const T* __restrict__ act, const T* __restrict__ down, const int* __restrict__ idx,
                                                       T* __restrict__ y, int K, int F) {
   extern __shared__ float al[];                     // the hidden row [F]
@@ -90,28 +150,35 @@ __global__ __launch_bounds__(NT) void expert_down_rows(const T* __restrict__ act
   const T* wd = down + static_cast<int64_t>(e) * K * F;
   const int c_end = min(K, (static_cast<int>(blockIdx.y) + 1) * KC);
   for (int c = blockIdx.y * KC + wave; c < c_end; c += NW) {
-    const float acc = wave_sum(lane_dot<T, VEC>(wd + static_cast<int64_t>(c) * F, al, F, lane));
+    const float acc = wave_sum(lane_dot<T>(wd + static_cast<int64_t>(c) * F, al, F, lane));
     if (lane == 0) y[pair * K + c] = from_f32<T>(acc);
   }
 }
 
-template <typename T, bool FAST, bool VEC, bool GATED>
+template <typename T, bool FAST, bool GATED>
 int launch_rows(const gbxm_expert_args& a, hipStream_t s) {
+  constexpr int PER = 16 / sizeof(T);
+  const bool vec = a.K % PER == 0 && a.F % PER == 0 &&
+                   all_aligned(16, static_cast<const T*>(a.first), static_cast<const T*>(a.down), static_cast<const T*>(a.h), static_cast<const T*>(a.ws));
   const int64_t P = a.T * a.top;
-  const dim3 gu(P, (a.F + FC - 1) / FC), gd(P, (a.K + KC - 1) / KC);
+  const dim3 gu(P, (a.F + (vec ? VC : FC) - 1) / (vec ? VC : FC)), gd(P, (a.K + KC - 1) / KC);
+  static_assert(VC == KC, "one grid for both forms of the second product");
   T* act = static_cast<T*>(a.ws);
-  expert_up_rows<T, FAST, VEC, GATED><<<gu, NT, a.K * sizeof(float), s>>>(static_cast<const T*>(a.h), static_cast<const T*>(a.first), a.idx, a.scale, act, a.K,
-                                                                         a.F, a.top, a.kind, a.limit);
-  expert_down_rows<T, VEC><<<gd, NT, a.F * sizeof(float), s>>>(act, static_cast<const T*>(a.down), a.idx, static_cast<T*>(a.y), a.K, a.F);
+  const T *h = static_cast<const T*>(a.h), *first = static_cast<const T*>(a.first), *down = static_cast<const T*>(a.down);
+  T* y = static_cast<T*>(a.y);
+  if (vec) {
+    expert_up_vec<T, FAST, GATED><<<gu, NT, 0, s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit);
+    expert_down_vec<T><<<gd, NT, 0, s>>>(act, down, a.idx, y, a.K, a.F);
+  } else {
+    expert_up_rows<T, FAST, GATED><<<gu, NT, a.K * sizeof(float), s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit);
+    expert_down_rows<T><<<gd, NT, a.F * sizeof(float), s>>>(act, down, a.idx, y, a.K, a.F);
+  }
   return after_launch("expert_ff (rows)");
 }
 
 template <typename T, bool FAST>
 int launch_rows(const gbxm_expert_args& a, hipStream_t s) {
-  constexpr int PER = 16 / sizeof(T);
-  const bool vec = a.K % PER == 0 && a.F % PER == 0 && (reinterpret_cast<uintptr_t>(a.first) | reinterpret_cast<uintptr_t>(a.down)) % 16 == 0;
-  if (a.kind == GBXM_EXPERT_RELU2) return vec ? launch_rows<T, FAST, true, false>(a, s) : launch_rows<T, FAST, false, false>(a, s);
-  return vec ? launch_rows<T, FAST, true, true>(a, s) : launch_rows<T, FAST, false, true>(a, s);
+  return a.kind == GBXM_EXPERT_RELU2 ? launch_rows<T, FAST, false>(a, s) : launch_rows<T, FAST, true>(a, s);
 }
 
 }  // namespace
