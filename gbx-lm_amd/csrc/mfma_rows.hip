@@ -1,0 +1,191 @@
+// Quantised products of 2 to 32 rows outside the group-128 batch kernel: groups of 32 and 64, and contractions that are no multiple of 1024.
+//   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
+// A workgroup takes 16 NT outputs, its waves share out the chunks of 128 of K; packed words, scales and the rows' image go straight to the registers of
+// the lane that feeds them to the matrix cores (packed_fields.h), one chunk ahead of the one being multiplied; sum_k x comes from the matrix cores too
+// (a product with ones, shared by the wave's outputs), and the waves' sums meet in LDS.  No weight is expanded or rounded to the activation type.
+// Bound by the latency of a wave's two or three chunks and by the rows' way through the first cache (27 rows: five bytes of rows for each byte of
+// weights).  Measured against the dequantising kernel that took these (us, weights cold): 3 bits,
+// group 64: 27 rows of 8192 x 3072 21.0 -> 14.0, 2 rows 20.9 -> 9.9, 8 rows of 4096 x 4096 14.9 -> 8.6, 32 of 14336 x 4096 39.2 -> 35.3; 4 bits, group 32:
+// 8 rows of 4096 x 11008 38.5 -> 20.4.
+#include "packed_fields.h"
+
+namespace gbx {
+namespace {
+
+constexpr int RW = 8;                      // waves
+
+template <int BITS, int GRP, bool BF16, int MT, int NT>
+__global__ __launch_bounds__(64 * RW) void qgemm_rows_kernel(MfmaArgs args) {
+  typedef Packed<BITS, GRP, BF16, NT> P;
+  constexpr int NF = P::NF, SPG = P::SPG;
+  __shared__ float part[RW][MT * NT * 256];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, fr = lane & 15, f = lane >> 4;
+  // the matrix: one, or one of up to three that share the rows, tiled one after another
+  const uint32_t* qw = args.qweight;
+  const unsigned short *sc = args.scales, *ze = args.zeros, *bias = args.bias;
+  unsigned short* y = args.y;
+  int N = args.nseg > 1 ? args.n_seg[0] : args.N, tile = blockIdx.x;
+  for (int g = 1; g < args.nseg && tile >= (N + 16 * NT - 1) / (16 * NT); ++g) {
+    tile -= (N + 16 * NT - 1) / (16 * NT);
+    qw = args.qweight_x[g - 1]; sc = args.scales_x[g - 1]; ze = args.zeros_x[g - 1]; bias = args.bias_x[g - 1]; y = args.y_x[g - 1];
+    N = args.n_seg[g];
+  }
+  const unsigned short* x = args.x;
+  const int M = args.M, K = args.K;
+  const int n0 = tile * (16 * NT), chunks = K >> 7, words = (K >> 5) * BITS, groups = K / GRP;
+  const unsigned short* xp[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xp[i] = x + static_cast<int64_t>(min(16 * i + fr, M - 1)) * K;
+  struct Chunk { P w; packed_x4 x[MT][4]; };
+  auto load = [&](int c, Chunk& k) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int64_t n = min(n0 + 16 * j + fr, N - 1);
+      k.w.load(j, qw + n * words + c * P::WPC, f);
+      k.w.load_affine(j, sc + n * groups + c * NF, ze + n * groups + c * NF);
+    }
+    // the octet of step t: 4 f + t of 16 (groups of 128), 2 f + t % 2 of the group's eight (64), f of its four (32)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const unsigned short* p = xp[i] + c * 128;
+        if constexpr (BITS == 2 && GRP == 32) {            // half of the word's 16: values 4 (f % 2) .. + 3 and the 4 that lie 8 further on
+          const packed_x2 lo = *reinterpret_cast<const packed_x2*>(p + 32 * t + 16 * (f >> 1) + 4 * (f & 1));
+          const packed_x2 hi = *reinterpret_cast<const packed_x2*>(p + 32 * t + 16 * (f >> 1) + 4 * (f & 1) + 8);
+          k.x[i][t] = packed_x4{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          const int o = GRP == 128 ? 4 * f + t : GRP == 64 ? (t >> 1) * 8 + 2 * f + (t & 1) : 4 * t + f;
+          k.x[i][t] = *reinterpret_cast<const packed_x4*>(p + 8 * o);
+        }
+      }
+  };
+  // the rows in the order in which fields leave a word
+  auto arrange = [&](Chunk& k) {
+    constexpr unsigned LO = 0x05040100u, HI = 0x07060302u;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if constexpr (BITS == 4 || (BITS == 2 && GRP == 32)) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const packed_x4 v = k.x[i][t];
+          k.x[i][t] = packed_x4{__builtin_amdgcn_perm(v.z, v.x, LO), __builtin_amdgcn_perm(v.z, v.x, HI), __builtin_amdgcn_perm(v.w, v.y, LO),
+                                __builtin_amdgcn_perm(v.w, v.y, HI)};
+        }
+      } else if constexpr (BITS == 2) {                    // two steps share a word
+#pragma unroll
+        for (int t = 0; t < 4; t += 2) {
+          const packed_x4 l = k.x[i][t], h = k.x[i][t + 1];
+          k.x[i][t] = packed_x4{__builtin_amdgcn_perm(h.x, l.x, LO), __builtin_amdgcn_perm(h.x, l.x, HI), __builtin_amdgcn_perm(h.y, l.y, LO),
+                                __builtin_amdgcn_perm(h.y, l.y, HI)};
+          k.x[i][t + 1] = packed_x4{__builtin_amdgcn_perm(h.z, l.z, LO), __builtin_amdgcn_perm(h.z, l.z, HI), __builtin_amdgcn_perm(h.w, l.w, LO),
+                                    __builtin_amdgcn_perm(h.w, l.w, HI)};
+        }
+      }
+    }
+  };
+  constexpr unsigned ONE = BF16 ? 0x3F803F80u : 0x3C003C00u;
+  const packed_x4 ones{ONE, ONE, ONE, ONE};
+  f32x4v acc[NT][MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[j][i] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](Chunk& k) {
+    arrange(k);
+#pragma unroll
+    for (int g = 0; g < NF; ++g) {
+      f32x4v xs[MT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        xs[i] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < SPG; ++t) xs[i] = mfma16<BF16>(k.x[i][g * SPG + t], ones, xs[i]);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float s = act_to_f32<BF16>(k.w.sc[j][g]), zc = act_to_f32<BF16>(k.w.ze[j][g]) - P::C * s;
+        packed_x4 op[SPG];
+#pragma unroll
+        for (int t = 0; t < SPG; ++t) op[t] = k.w.operand(j, g * SPG + t, f);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          f32x4v d{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int t = 0; t < SPG; ++t) d = mfma16<BF16>(k.x[i][g * SPG + t], op[t], d);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[j][i][v] = fmaf(s, d[v], fmaf(zc, xs[i][v], acc[j][i][v]));
+        }
+      }
+    }
+  };
+  if (wave < chunks) {
+    Chunk a, b;
+    load(wave, a);
+    for (int c = wave; c < chunks; c += 2 * RW) {
+      if (c + RW < chunks) load(c + RW, b);
+      compute(a);
+      if (c + RW < chunks) {
+        if (c + 2 * RW < chunks) load(c + 2 * RW, a);
+        compute(b);
+      }
+    }
+  }
+  // a lane holds rows 4 f + v of output fr
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[wave][(i * 16 + 4 * f + v) * (16 * NT) + 16 * j + fr] = acc[j][i][v];
+  __syncthreads();
+  for (int i = threadIdx.x; i < MT * NT * 256; i += 64 * RW) {
+    const int n = n0 + i % (16 * NT), m = i / (16 * NT);
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < RW; ++v) s += part[v][i];
+    if (n < N && m < M) {
+      unsigned short r = f32_to_act<BF16>(s);                              // (a bias is a second rounding)
+      if (bias) r = f32_to_act<BF16>(act_to_f32<BF16>(r) + act_to_f32<BF16>(bias[n]));
+      y[static_cast<int64_t>(m) * N + n] = r;
+    }
+  }
+}
+
+template <int BITS, int GRP, int MT>
+hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
+#define GBX_QROWS(NT)                                                                               \
+  do {                                                                                              \
+    int grid = 0;                                                                                   \
+    for (int g = 0; g < (a.nseg > 1 ? a.nseg : 1); ++g) grid += ((a.nseg > 1 ? a.n_seg[g] : a.N) + 16 * NT - 1) / (16 * NT); \
+    if (bf16) qgemm_rows_kernel<BITS, GRP, true, MT, NT><<<grid, 64 * RW, 0, s>>>(a);               \
+    else qgemm_rows_kernel<BITS, GRP, false, MT, NT><<<grid, 64 * RW, 0, s>>>(a);                   \
+  } while (0)
+  // 32 outputs a workgroup share the rows' image where that still leaves a workgroup for every CU (3 bits, group 64, 27 rows, 16 | 32 outputs, us:
+  // 4096 x 4096 12.8 | 17.1, 8192 x 3072 19.2 | 13.9)
+  if (a.N > 4096) GBX_QROWS(2);
+  else GBX_QROWS(1);
+#undef GBX_QROWS
+  return hipGetLastError();
+}
+
+template <int BITS, int GRP>
+hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
+  return a.M <= 16 ? launch_rows<BITS, GRP, 1>(a, bf16, s) : launch_rows<BITS, GRP, 2>(a, bf16, s);
+}
+
+template <int BITS>
+hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
+  return a.log2g == 7 ? launch_rows<BITS, 128>(a, bf16, s) : a.log2g == 6 ? launch_rows<BITS, 64>(a, bf16, s) : launch_rows<BITS, 32>(a, bf16, s);
+}
+
+}  // namespace
+
+hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
+  uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
+  for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
+  if (a.swiglu || a.M < 2 || a.M > 32 || a.K % 128 || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
+  return bits == 2 ? launch_rows<2>(a, bf16, s) : bits == 3 ? launch_rows<3>(a, bf16, s) : bits == 4 ? launch_rows<4>(a, bf16, s) : hipErrorInvalidValue;
+}
+
+}  // namespace gbx

@@ -285,6 +285,10 @@ hipError_t launch_qgemm_skinny_multi(const void* x, int nseg, const uint32_t* co
     const hipError_t e = launch_batch_rows(a, bits, bf16, s);
     if (e != hipErrorInvalidValue) return e;        // segment rows the wide workgroups cannot tile: split-K kernel
   }
+  if (a.M <= 32) {                // (33 to 64 rows are too many for the rows kernel's registers: 4096 x 11008, 3 bits, group 64, 48 rows 42.6 us here, 45.5 there)
+    const hipError_t e = launch_qgemm_rows(a, bits, bf16, s);
+    if (e != hipErrorInvalidValue) return e;
+  }
   switch (bits) {
     case 2: return launch_skinny_bits<2>(a, bf16, s);
     case 3: return launch_skinny_bits<3>(a, bf16, s);
@@ -329,6 +333,10 @@ hipError_t launch_qgemm_skinny(const void* x, const uint32_t* qw, const void* sc
   if (use_batch_kernel(a, bits)) {
     const hipError_t e = launch_batch_rows(a, bits, bf16, s);
     if (e != hipErrorInvalidValue) return e;        // segment rows the wide workgroups cannot tile: split-K kernel
+  }
+  if (a.M <= 32) {                // (33 to 64 rows are too many for the rows kernel's registers: 4096 x 11008, 3 bits, group 64, 48 rows 42.6 us here, 45.5 there)
+    const hipError_t e = launch_qgemm_rows(a, bits, bf16, s);
+    if (e != hipErrorInvalidValue) return e;
   }
   switch (bits) {
     case 2: return launch_skinny_bits<2>(a, bf16, s);

@@ -17,11 +17,13 @@
 //   3 600 pairs, 128 experts, 3 bits, group 128: 2 x 768 x 2048 gated  78 (2.0 TB/s of packed weights), 2048 x 768  43
 //   32 experts of 768 x 2048, 280 | 1 800 | 8 000 pairs: 3 bits 32 | 49 | 79, 4 bits 37 | 53 | 90 -- before 2 454 | 2 455 | 2 777
 // and the relative error against 64 bits at 1 800 pairs 1.66e-3 (bf16) and 2.1e-4 (fp16), before 2.16e-3 and 2.7e-4.
-#include "mfma_common.h"
 #include "mixers_mfma.h"
+#include "packed_fields.h"
 
 namespace gbxm {
 namespace {
+
+using gbx::Packed;
 
 constexpr int PT = 64;                 // pairs per tile at most
 constexpr int PLDS = 4 * PT * 144;     // LDS bytes: two chunks of activations (2 x 64 x 256) and xsum, then four output tiles of 64 rows x 144
@@ -35,98 +37,6 @@ struct PackedArgs {
   const int *offsets, *sorted, *tile_tab;
   unsigned short* y;                   // [pairs][N]
   int N, K, E, x_div, cols;
-};
-
-template <int BITS, int GRP, bool BF16>
-struct Packed {
-  static constexpr int NF = 128 / GRP;                     // groups per chunk
-  static constexpr int SPG = 4 / NF;                       // product steps per group
-  static constexpr int WPC = 4 * BITS;                     // packed words per row and chunk
-  static constexpr int RAW = BITS == 4 ? 4 : BITS == 3 ? (GRP == 128 ? 3 : GRP == 64 ? 4 : 8) : (GRP == 32 ? 4 : 2);
-  static constexpr unsigned MAGIC = BF16 ? 0x43004300u : 0x64006400u;
-  static constexpr float C = BF16 ? 128.f : 1024.f;
-  static constexpr unsigned MASK = BITS == 2 ? 0x00030003u : BITS == 3 ? 0x00070007u : 0x000F000Fu;
-
-  unsigned raw[4][RAW];                                    // per row tile: the lane's packed words of the chunk
-  unsigned short sc[4][NF], ze[4][NF];
-
-  // octet of step t and lane quarter f: f owns GRP / 4 neighbours of every group
-  static __device__ __forceinline__ int step_of(int o) { return GRP == 128 ? (o & 3) : GRP == 64 ? (o >> 3) * 2 + (o & 1) : o >> 2; }
-  static __device__ __forceinline__ int quarter_of(int o) { return GRP == 128 ? o >> 2 : GRP == 64 ? (o & 7) >> 1 : o & 3; }
-
-  __device__ __forceinline__ void load(int i, const uint32_t* p, int f) {      // p: the chunk's words of the row
-    if constexpr (BITS == 4 && GRP == 128) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(p + 4 * f);
-      raw[i][0] = v.x; raw[i][1] = v.y; raw[i][2] = v.z; raw[i][3] = v.w;
-    } else if constexpr (BITS == 4 && GRP == 64) {
-      const u32x2 a = *reinterpret_cast<const u32x2*>(p + 2 * f), b = *reinterpret_cast<const u32x2*>(p + 8 + 2 * f);
-      raw[i][0] = a.x; raw[i][1] = a.y; raw[i][2] = b.x; raw[i][3] = b.y;
-    } else if constexpr (BITS == 4) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) raw[i][t] = p[4 * t + f];
-    } else if constexpr (BITS == 2 && GRP == 128) {
-      const u32x2 a = *reinterpret_cast<const u32x2*>(p + 2 * f);
-      raw[i][0] = a.x; raw[i][1] = a.y;
-    } else if constexpr (BITS == 2 && GRP == 64) {
-      raw[i][0] = p[f]; raw[i][1] = p[4 + f];
-    } else if constexpr (BITS == 2) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) raw[i][t] = p[2 * t + (f >> 1)];
-    } else if constexpr (GRP == 128) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) raw[i][q] = p[3 * f + q];
-    } else if constexpr (GRP == 64) {                      // 48 bits from bit 48 f (+ 192): words 3 f / 2 and the next
-      const int a = (3 * f) >> 1;
-      raw[i][0] = p[a]; raw[i][1] = p[a + 1]; raw[i][2] = p[6 + a]; raw[i][3] = p[7 + a];
-    } else {                                               // 24 bits from bit 96 t + 24 f
-      const int a = (3 * f) >> 2, b = min(a + 1, 2);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) { raw[i][2 * t] = p[3 * t + a]; raw[i][2 * t + 1] = p[3 * t + b]; }
-    }
-  }
-  __device__ __forceinline__ void load_affine(int i, const unsigned short* sp, const unsigned short* zp) {
-    if constexpr (NF == 1) {
-      sc[i][0] = *sp; ze[i][0] = *zp;
-    } else if constexpr (NF == 2) {
-      const unsigned a = *reinterpret_cast<const unsigned*>(sp), b = *reinterpret_cast<const unsigned*>(zp);
-      sc[i][0] = a & 0xFFFF; sc[i][1] = a >> 16; ze[i][0] = b & 0xFFFF; ze[i][1] = b >> 16;
-    } else {
-      const u32x2 a = *reinterpret_cast<const u32x2*>(sp), b = *reinterpret_cast<const u32x2*>(zp);
-      sc[i][0] = a.x & 0xFFFF; sc[i][1] = a.x >> 16; sc[i][2] = a.y & 0xFFFF; sc[i][3] = a.y >> 16;
-      ze[i][0] = b.x & 0xFFFF; ze[i][1] = b.x >> 16; ze[i][2] = b.y & 0xFFFF; ze[i][3] = b.y >> 16;
-    }
-  }
-  // the eight operands C + q of step t (compile-time) of row tile i, in the order of the stored activations
-  __device__ __forceinline__ u32x4 operand(int i, int t, int f) const {
-    u32x4 r;
-    if constexpr (BITS == 4) {
-      const unsigned w = raw[i][t];
-      r.x = (w & MASK) | MAGIC; r.y = ((w >> 4) & MASK) | MAGIC; r.z = ((w >> 8) & MASK) | MAGIC; r.w = ((w >> 12) & MASK) | MAGIC;
-    } else if constexpr (BITS == 2) {
-      const unsigned w = GRP == 32 ? raw[i][t] >> (8 * (f & 1)) : raw[i][t >> 1] >> (8 * (t & 1));
-      r.x = (w & MASK) | MAGIC; r.y = ((w >> 2) & MASK) | MAGIC; r.z = ((w >> 4) & MASK) | MAGIC; r.w = ((w >> 6) & MASK) | MAGIC;
-    } else {
-      unsigned w;                                          // the octet's 24 bits from bit 0
-      if constexpr (GRP == 128) {
-        const int b0 = 24 * t, a = b0 >> 5;
-        w = (b0 & 31) == 0 ? raw[i][a] : __builtin_amdgcn_alignbit(raw[i][a + 1 < 3 ? a + 1 : 2], raw[i][a], b0 & 31);
-      } else if constexpr (GRP == 64) {
-        const unsigned lo = raw[i][2 * (t >> 1)], hi = raw[i][2 * (t >> 1) + 1];
-        const int sh = 16 * (f & 1);                       // (48 f mod 32)
-        w = (t & 1) == 0 ? __builtin_amdgcn_alignbit(hi, lo, sh) : sh ? hi >> 8 : __builtin_amdgcn_alignbit(hi, lo, 24);
-      } else {
-        w = __builtin_amdgcn_alignbit(raw[i][2 * t + 1], raw[i][2 * t], (24 * f) & 31);
-      }
-      unsigned v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const unsigned q = (w >> (6 * j)) & 0x3F;
-        v[j] = ((q | (q << 13)) & MASK) | MAGIC;
-      }
-      r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
-    }
-    return r;
-  }
 };
 
 template <bool BF16> __device__ __forceinline__ float pair_sum(unsigned v, float acc) {

@@ -1,0 +1,55 @@
+"""Quantised products of 2 to 32 rows outside the group-128 batch kernel (csrc/mfma_rows.hip): every width of field and group, one row tile and two, their
+edges, contractions that leave waves without a chunk or with unequal numbers, outputs that end inside a workgroup, both output tilings, a bias, and
+scales that are not aligned to a chunk's (the dequantising kernel).  Reference: float64; tolerance: the result's rounding (two with a bias; the
+dequantising kernel rounds every weight too) and fp32 sums of K terms as large as C + q = 143 (bf16) or 1039 (fp16)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def run(m, n, k, bits, g, dt, bias, shift, seed):
+    from gbx_lm_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    qw = torch.randint(-2**31, 2**31, (n, k // 32 * bits), device=DEV, generator=gen, dtype=torch.int64).to(torch.int32).view(torch.uint32)
+    top = (1 << bits) - 1
+    s = (torch.rand((n, k // g), device=DEV, generator=gen) + 0.5) * (0.1 / top)
+    z = (-s * top / 2 + torch.randn(s.shape, device=DEV, generator=gen) * 0.2 * s).to(dt)
+    s = s.to(dt)
+    if shift:                                                   # an address one element past the allocation's
+        s, z = (torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape) for t in (s, z))
+    x = torch.randn((m, k), device=DEV, generator=gen).to(dt)
+    b = torch.randn(n, device=DEV, generator=gen).to(dt) if bias else None
+    w = ops.unpack(qw, bits).double() * s.double().repeat_interleave(g, 1) + z.double().repeat_interleave(g, 1)
+    want = x.double() @ w.t() + (b.double() if bias else 0.0)
+    y = ops.quantized_matmul(x, qw, s, z, group_size=g, bits=bits, bias=b)
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    terms = x.double().abs() @ (s.double().repeat_interleave(g, 1) * (144 if dt == torch.bfloat16 else 1040)).t()
+    room = 2 * eps * (want.abs() + (b.double().abs() if bias else 0.0)) + 2.0 ** -22 * terms
+    if shift:
+        room = room + 4 * eps * (x.double() ** 2 @ (w ** 2).t()).sqrt()
+    assert bool(((y.double() - want).abs() <= room).all())
+    return x, qw, s, z, b, y
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (2, 128), (3, 32), (3, 64), (3, 128), (4, 32), (4, 64), (4, 128)])
+@pytest.mark.parametrize("m,n,k,bias", [(2, 16, 512, False), (16, 33, 896, True), (17, 17, 1152, False), (27, 4097, 640, True), (32, 4112, 2176, False), (31, 100, 3200, False)])
+def test_fields_groups_and_edges(dt, bits, g, m, n, k, bias):
+    run(m, n, k, bits, g, dt, bias, False, m + n + k + bits + g)
+
+
+@pytest.mark.parametrize("bits,g", [(3, 32), (3, 64), (4, 32), (4, 64)])
+def test_whole_kilochannels_and_unaligned_scales(bits, g):
+    for m in (2, 15, 32):
+        run(m, 5000, 1024, bits, g, torch.bfloat16, m == 15, False, m)
+        run(m, 72, 3072, bits, g, torch.float16, m == 15, False, m)
+        run(m, 72, 1024, bits, g, torch.bfloat16, False, True, m)
+
+
+def test_a_row_does_not_depend_on_the_others():
+    from gbx_lm_amd import ops
+    x, qw, s, z, b, y = run(32, 4100, 1152, 3, 64, torch.bfloat16, False, False, 5)
+    for rows in (slice(0, 2), slice(3, 19), slice(1, 18)):
+        assert torch.equal(ops.quantized_matmul(x[rows].contiguous(), qw, s, z, group_size=64, bits=3), y[rows])
