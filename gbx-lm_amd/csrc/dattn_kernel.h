@@ -1108,8 +1108,8 @@ __global__ __launch_bounds__(DA_NT) void dattn_kernel(const DattnArgs a) {
       }
     } else {
     // ---- cached positions [0, pos): 16 lanes per position, online softmax per lane group (attn_decode_kernel, 16-wave form)
-    // Packed fp32 arithmetic (v_pk_fma_f32: two lanes of work per issue slot -- this sweep is vector-ALU bound once the K / V rows
-    // sit in registers) and a two-pass softmax over the prefetched rounds: all scores first, ONE running-maximum update, then the
+    // Pairs of fp32 channels (this sweep is vector-ALU bound once the K / V rows sit in registers; the pairs issue as two plain fp32
+    // instructions, packed ones are off in the build) and a two-pass softmax over the prefetched rounds: all scores first, ONE running-maximum update, then the
     // exponentials and the value sums without a per-position rescale.
     DA_STAMP(12);
     typedef float f32x2 __attribute__((ext_vector_type(2)));

@@ -42,7 +42,7 @@ inline const EnvSwitch* env_table(int* n) {
       {"GBX_BATCH_KSPLIT_MINK", 8192, "batch GEMM: smallest K that is split across workgroups (tuning aid)"},
       {"GBX_DENSE_SKINNY", 1, "dense GEMM at M <= 32 (the head of a decode batch): the row-streaming kernel (0: the 256 x 256 tile) (A/B)"},
       {"GBX_BATCH_ROWS", 0, "batch GEMM: force the activation rows staged per pass (tuning aid)"},
-      {"GBX_NO_BATCH_KERNEL", 0, "1: 2 <= M <= 32 on the split-K dequantising kernel instead of the no-dequant batch GEMM (diagnostic)"},
+      {"GBX_NO_BATCH_KERNEL", 0, "1: 2 <= M <= 32 on the general no-dequant kernel (33 to 64 rows: the split-K dequantising one) instead of the batch GEMM (diagnostic)"},
       {"GBX_PREFILL_TILE", 0, "prefill GEMM: force the tile (11 / 12 / 13) (tuning aid)"},
       {"GBX_DENSE_NO_8PHASE", 0, "1: the register-staged round-1 tile on dequantised weights instead of the 8-phase dense GEMM (A/B)"},
       {"GBX_P2P_SPIN_LOG2", 26, "one-shot P2P all-reduce: log2 of the polls of one granule before a launch gives up and raises its error word (test hook: a small value makes the time-out path reachable in a test)"},
