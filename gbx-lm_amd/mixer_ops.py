@@ -17,7 +17,8 @@ _DT = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32}
 
 
 def _stream(device) -> int:
-    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
+    index = (device if type(device) is torch.device else torch.device(device)).index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _act(t: torch.Tensor, name: str) -> int:

@@ -19,7 +19,8 @@ _DT = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16, torch.float32
 
 def _stream_ptr(device) -> int:
     """hipStream_t of the device's current stream (the raw handle: building a Stream object around it costs 2 us a launch)."""
-    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
+    index = (device if type(device) is torch.device else torch.device(device)).index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _require_cuda(t: torch.Tensor, name: str) -> None:
