@@ -1,5 +1,5 @@
 """Quantised products of 2 to 32 rows outside the group-128 batch kernel (csrc/mfma_rows.hip): every width of field and group, one row tile and two, their
-edges, contractions that leave waves without a chunk or with unequal numbers, outputs that end inside a workgroup, both output tilings, a bias, and
+edges, contractions that give waves one chunk each or unequal numbers, outputs that end inside a workgroup, both output tilings, a bias, and
 scales that are not aligned to a chunk's (the dequantising kernel).  Reference: float64; tolerance: the result's rounding (two with a bias; the
 dequantising kernel rounds every weight too) and fp32 sums of K terms as large as C + q = 143 (bf16) or 1039 (fp16)."""
 import pytest
@@ -35,7 +35,7 @@ def run(m, n, k, bits, g, dt, bias, shift, seed):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (2, 128), (3, 32), (3, 64), (3, 128), (4, 32), (4, 64), (4, 128)])
-@pytest.mark.parametrize("m,n,k,bias", [(2, 16, 512, False), (16, 33, 896, True), (17, 17, 1152, False), (27, 4097, 640, True), (32, 4112, 2176, False), (31, 100, 3200, False)])
+@pytest.mark.parametrize("m,n,k,bias", [(2, 16, 1024, False), (16, 33, 1280, True), (17, 17, 1152, False), (27, 4097, 1408, True), (32, 4112, 2176, False), (31, 100, 3200, False)])
 def test_fields_groups_and_edges(dt, bits, g, m, n, k, bias):
     run(m, n, k, bits, g, dt, bias, False, m + n + k + bits + g)
 
