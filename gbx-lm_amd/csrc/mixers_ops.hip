@@ -96,7 +96,9 @@ __global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restr
   float m = -INFINITY, s = 0.f;
   for (int i = 0; i < static_cast<int>(gridDim.x); ++i) m = fmaxf(m, p[i].x);
   const float shift = isinf(m) ? 0.f : m;
-  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) s += p[i].y * expf((isinf(p[i].x) ? 0.f : p[i].x) - shift);
+  // (an infinite maximum: the slice's sum is 0, infinite or no number against any shift -- the shift's own exponential may be infinite, and 0 times that is
+  // no number)
+  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) s += isinf(p[i].x) ? p[i].y : p[i].y * expf(p[i].x - shift);
   const float lse = lsm_round<T>(logf(s) + shift);
   const int lo = blockIdx.x * LSM_SLICE, hi = min(lo + LSM_SLICE, n);
   const int64_t base = static_cast<int64_t>(blockIdx.y) * n;

@@ -38,3 +38,22 @@ def test_masked_and_undefined_logits(dt, n):
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
     ok = torch.isfinite(want)
     assert bool(((got - want).abs()[ok].float() <= 2 * LAST[dt] * (1 + want.abs()[ok].float())).all())
+
+
+@pytest.mark.parametrize("dt", list(LAST))
+def test_slices_without_a_candidate(dt):
+    """A few long rows are summed slice by slice: slices in which every logit is masked add nothing, however low the row's maximum lies."""
+    from gbx_lm_amd.mixer_ops import log_probabilities
+    x = torch.full((4, 40000), float("-inf"), device="cuda", dtype=dt)
+    x[0, :100] = -200
+    x[1, 39990:] = -30000
+    x[2, 20000] = 300
+    x[3, :100], x[3, 30000] = -200, float("nan")
+    got = log_probabilities(x)
+    lse = torch.logsumexp(x.double(), -1, keepdim=True)
+    want = x.double() - lse
+    assert torch.isnan(got[3]).all()
+    for r in range(3):
+        ok = torch.isfinite(x[r])
+        assert (got[r][~ok] == float("-inf")).all()
+        assert bool(((got[r].double() - want[r]).abs()[ok] <= LAST[dt] * (lse[r].abs() + want[r].abs()[ok]) + 2.0 ** -22 * (1 + lse[r].abs())).all())
