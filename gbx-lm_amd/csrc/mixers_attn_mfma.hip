@@ -86,7 +86,7 @@ __global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS)) void window_ti
   // of a tile span 127 + KT distances, the ring holds 256); distances outside the window stand there as infinity, which
   // makes the gate zero without a test per score.
   constexpr float LOG2E = 1.4426950408889634f;
-  const float dm = a.dmul[head], dr = a.drate[head], cap = a.softcap;
+  const float dm = a.dmul[head], dr = a.drate[head], cap = fmaxf(a.softcap, 0.f);      // (zero or below: no cap)
   const float zc = -LOG2E * (a.gbias[head] + cap), z2 = 2.f * LOG2E * cap, xs = cap > 0.f ? a.scale * 2.f * LOG2E / cap : -LOG2E * a.scale;
   auto exponent = [&](int d) { return d >= 0 && d < W ? fmaf(dm, __log2f(1.f + dr * static_cast<float>(d)), zc) : INFINITY; };
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;

@@ -46,3 +46,21 @@ def test_portions(dk, dv, cap, window):
             err = (got[r0:r0 + n, h] - want).abs()
             assert bool((err <= 3 * 2.0 ** -8 * (want.abs() + spread) + 2.0 ** -18 * total + 1e-6).all()), (n, p, h, float(err.max()))
         r0 += n
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (192, 128)])
+def test_a_soft_cap_below_zero_is_none(dk, dv):
+    """In prompt portions as in steps of single tokens: the same bits as without one."""
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.batching import StepBatch
+    gen = torch.Generator(device=DEV).manual_seed(dk)
+    H, G, W, n_new, pos0 = 4, 2, 100, [1, 140, 1, 33], [30, 0, 7, 64]
+    batch = StepBatch.build(list(range(4)), pos0, n_new, DEV)
+    qkv = torch.randn((sum(n_new), H * dk + G * (dk + dv)), device=DEV, generator=gen).to(torch.bfloat16)
+    kc, vc = (torch.randn((4, W, G * d), device=DEV, generator=gen).to(torch.bfloat16) for d in (dk, dv))
+    vec = lambda: torch.rand(H, device=DEV, generator=gen)
+    m = SimpleNamespace(window=W, nk=G * dk, nv=G * dv, heads=H, kv_heads=G, dim=dk, vdim=dv, dist_mul=vec(), dist_rate=vec(), gate_bias=vec() - 0.5,
+                        scale=dk ** -0.5, softcap=0.0)
+    want = M.window_attention(qkv, kc, vc, batch, m)
+    m.softcap = -3.0
+    assert torch.equal(M.window_attention(qkv, kc, vc, batch, m), want)
