@@ -2,7 +2,8 @@
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
 // A workgroup takes 16 NT outputs, its waves share out the chunks of 128 of K; packed words, scales and the rows' image go straight to the registers of
 // the lane that feeds them to the matrix cores (packed_fields.h), one chunk ahead of the one being multiplied; sum_k x comes from the matrix cores too
-// (a product with ones, shared by the wave's outputs), and the waves' sums meet in LDS.  No weight is expanded or rounded to the activation type.
+// (a product with ones, shared by the wave's outputs), and the waves' sums meet in LDS.  No weight is expanded or rounded to the activation type; only an
+// output whose sum is not finite is taken again, weight by weight (expanded_dot): infinite activations give what their products with the weights give.
 // Bound by the latency of a wave's two or three chunks and by the rows' way through the first cache (27 rows: five bytes of rows for each byte of
 // weights).  Measured against the dequantising kernel that took these (us, weights cold): 3 bits,
 // group 64: 27 rows of 8192 x 3072 21.0 -> 14.0, 2 rows 20.9 -> 9.9, 8 rows of 4096 x 4096 14.9 -> 8.6, 32 of 14336 x 4096 39.2 -> 35.3; 4 bits, group 32:
@@ -139,16 +140,31 @@ __global__ __launch_bounds__(64 * RW) void qgemm_rows_kernel(MfmaArgs args) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) part[wave][(i * 16 + 4 * f + v) * (16 * NT) + 16 * j + fr] = acc[j][i][v];
   __syncthreads();
-  for (int i = threadIdx.x; i < MT * NT * 256; i += 64 * RW) {
-    const int n = n0 + i % (16 * NT), m = i / (16 * NT);
+  auto put = [&](int n, int m, float v) {
+    unsigned short r = f32_to_act<BF16>(v);                                // (a bias is a second rounding)
+    if (bias) r = f32_to_act<BF16>(act_to_f32<BF16>(r) + act_to_f32<BF16>(bias[n]));
+    y[static_cast<int64_t>(m) * N + n] = r;
+  };
+  auto sum = [&](int i) {
     float s = 0.f;
 #pragma unroll
     for (int v = 0; v < RW; ++v) s += part[v][i];
-    if (n < N && m < M) {
-      unsigned short r = f32_to_act<BF16>(s);                              // (a bias is a second rounding)
-      if (bias) r = f32_to_act<BF16>(act_to_f32<BF16>(r) + act_to_f32<BF16>(bias[n]));
-      y[static_cast<int64_t>(m) * N + n] = r;
-    }
+    return s;
+  };
+  bool finite = true;
+  for (int i = threadIdx.x; i < MT * NT * 256; i += 64 * RW) {
+    const int n = n0 + i % (16 * NT), m = i / (16 * NT);
+    const float s = sum(i);
+    finite &= __builtin_isfinite(s);
+    if (n < N && m < M) put(n, m, s);
+  }
+  if (finite) return;
+#pragma unroll 1
+  for (int i = threadIdx.x; i < MT * NT * 256; i += 64 * RW) {
+    const int n = n0 + i % (16 * NT), m = i / (16 * NT);
+    if (n < N && m < M && !__builtin_isfinite(sum(i)))
+      put(n, m, expanded_dot<BITS, GRP, BF16>(x + static_cast<int64_t>(m) * K, qw + static_cast<int64_t>(n) * words, sc + static_cast<int64_t>(n) * groups,
+                                              ze + static_cast<int64_t>(n) * groups, K));
   }
 }
 

@@ -102,4 +102,23 @@ struct Packed {
   }
 };
 
+// sum_k x[k] (s q + z), weights rounded to the activation type as the dequantising kernels have them: for the sums that the form above leaves without a
+// finite number.  An infinite activation meets C + q and -C s as infinity minus infinity where its product with the weight is an infinity; one near the
+// largest of its type overflows in C + q alone.  One output a thread; a sum that is no number is final.
+template <int BITS, int GRP, bool BF16>
+__device__ __forceinline__ float expanded_dot(const unsigned short* __restrict__ x, const uint32_t* __restrict__ w, const unsigned short* __restrict__ s,
+                                              const unsigned short* __restrict__ z, int K) {
+  float acc = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K && acc == acc; k += 32) {
+    const float sf = act_to_f32<BF16>(s[k / GRP]), zf = act_to_f32<BF16>(z[k / GRP]);
+#pragma unroll 8
+    for (int j = k; j < k + 32; ++j) {
+      const float v = act_to_f32<BF16>(f32_to_act<BF16>(fmaf(sf, static_cast<float>(field_of_row<BITS>(w, j)), zf)));
+      acc = fmaf(act_to_f32<BF16>(x[j]), v, acc);
+    }
+  }
+  return acc;
+}
+
 }  // namespace gbx

@@ -53,3 +53,49 @@ def test_a_row_does_not_depend_on_the_others():
     x, qw, s, z, b, y = run(32, 4100, 1152, 3, 64, torch.bfloat16, False, False, 5)
     for rows in (slice(0, 2), slice(3, 19), slice(1, 18)):
         assert torch.equal(ops.quantized_matmul(x[rows].contiguous(), qw, s, z, group_size=64, bits=3), y[rows])
+
+
+def extremes(dt, m, k, seed):
+    """Rows with infinities (of one sign, in one group, of both signs), one that is not a number, and one so large that its products with C + q leave
+    fp32 where those with the weights do not (bf16), beside ordinary rows."""
+    x = torch.randn((m, k), device=DEV, generator=torch.Generator(device=DEV).manual_seed(seed)).to(dt)
+    x[0, 3], x[1, k - 1], x[2, 5], x[2, 6], x[3, 70], x[4, 9], x[4, k - 7] = [float("inf"), float("-inf"), float("inf"), float("inf"), float("nan"),
+                                                                              float("inf"), float("-inf")]
+    x[5, 100] = 3e36 if dt == torch.bfloat16 else 60000.0
+    return x
+
+
+def same_numbers(y, want, eps, room):
+    """Infinities and NaN where the reference has them, the rest within the tolerance."""
+    y, most = y.double(), 3.3e38 if eps > 2.0 ** -10 else 65504.0
+    want = torch.where(want.abs() > most, want.sign() * float("inf"), want)
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(y[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
+    assert bool(((y - want).abs() <= eps * want.abs() + room)[finite].all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (3, 32), (3, 64), (3, 128), (4, 32), (4, 64), (4, 128)])
+def test_infinite_undefined_and_huge_activations(dt, bits, g):
+    """An infinity times the weight, not infinity minus infinity.  Tolerance: the roundings of the result and, where a row is huge, of its weights; fp32 sums
+    of K terms as large as C + q."""
+    from gbx_lm_amd import ops
+    n, k = 100, 1152
+    gen = torch.Generator(device=DEV).manual_seed(bits * g)
+    qw = torch.randint(-2**31, 2**31, (n, k // 32 * bits), device=DEV, generator=gen, dtype=torch.int64).to(torch.int32).view(torch.uint32)
+    s = ((torch.rand((n, k // g), device=DEV, generator=gen) + 0.5) * 0.03).to(dt)
+    z = (-s.float() * ((1 << bits) - 1) / 2 * 0.9).to(dt)
+    w = ops.unpack(qw, bits).double() * s.double().repeat_interleave(g, 1) + z.double().repeat_interleave(g, 1)
+    for m in (8, 20):
+        x = extremes(dt, m, k, m)
+        y = ops.quantized_matmul(x, qw, s, z, group_size=g, bits=bits)
+        eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+        room = 2.0 ** -22 * (x.double().nan_to_num(0, 0, 0).abs() @ (s.double().repeat_interleave(g, 1) * (144 if dt == torch.bfloat16 else 1040)).t())
+        room[5] *= dt != torch.bfloat16                             # (there: every weight rounded, the terms as they are)
+        same_numbers(y, torch.stack([row @ w.t() if torch.isfinite(row).all() else ieee(row, w) for row in x.double()]), 3 * eps, room + 2.0 ** -10)
+
+
+def ieee(row, w):
+    """sum_k row[k] w[n, k] with infinities and NaN as they are (a matrix product may order its sums, which decides nothing here)."""
+    odd = ~torch.isfinite(row)
+    return (row[odd][None] * w[:, odd]).sum(1)
