@@ -6,7 +6,8 @@
 // (gated: 128 rows of each matrix), a wave 64 of them.  Weights are never expanded: a field ORed under the exponent of 128.0 (bf16) or
 // 1024.0 (fp16) IS the number C + q, a shift and an and-or make two operands of a product, and the affine map meets the fp32 sums of a group:
 //   acc[m, n] += s[n, g] t[m, n] + (z[n, g] - C s[n, g]) xsum[m, g],   t = sum_k x (C + q),   xsum = sum_k x.
-// No weight is rounded to the activation type, so the error is that of the fp32 sums and of the one rounding of the result.
+// No weight is rounded to the activation type, so the error is that of the fp32 sums and of the one rounding of the result.  Infinite activations, for
+// which this form has infinity minus infinity, are seen in the sums, and their outputs taken again weight by weight (expanded_dot).
 // The contraction runs in chunks of 128.  Inside a chunk the order of k is free as long as both operands agree: step t of lane quarter f
 // multiplies octet o(t, f) of the row -- the one that lets a lane read its packed words of a group in one piece -- and the activations are
 // stored in that order, in the pair order in which fields leave a word ((j, j + 8) of 16 fields of 2 bits, (j, j + 4) of 8 of 4 bits).
@@ -180,6 +181,18 @@ __device__ __forceinline__ void packed_tile(const PackedArgs& a, unsigned char* 
   // a lane holds pairs 4 f + v of channel fr: through LDS of the wave's own, then rows of 64 (gated: 32) channels in 16-byte pieces
   constexpr int OC = GATED ? 32 : 64, OROW = 144;
   unsigned char* ot = lds + wave * (PT * OROW);
+  // the roundings of the separate operations
+  auto result = [&](float c, float up, float b) {
+    unsigned short r = gbx::f32_to_act<BF16>(c);
+    if constexpr (GATED) {
+      const float g = gbx::act_to_f32<BF16>(r), u = gbx::act_to_f32<BF16>(gbx::f32_to_act<BF16>(up));
+      r = gbx::f32_to_act<BF16>(gbx::act_to_f32<BF16>(gbx::f32_to_act<BF16>(g / (1.f + __expf(-g)))) * u);
+    } else if (a.bias) {
+      r = gbx::f32_to_act<BF16>(gbx::act_to_f32<BF16>(r) + b);
+    }
+    return r;
+  };
+  float odd = 0.f;                                                      // (0 times what is no finite number is no number)
 #pragma unroll
   for (int j = 0; j < (GATED ? 2 : 4); ++j) {
     const float b = !GATED && a.bias ? gbx::act_to_f32<BF16>(a.bias[static_cast<int64_t>(e) * N + min(c0 + j * 16 + fr, N - 1)]) : 0.f;
@@ -187,18 +200,28 @@ __device__ __forceinline__ void packed_tile(const PackedArgs& a, unsigned char* 
     for (int i = 0; i < NR; ++i)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        unsigned short r = gbx::f32_to_act<BF16>(acc[j][i][v]);
-        if constexpr (GATED) {
-          const float g = gbx::act_to_f32<BF16>(r), u = gbx::act_to_f32<BF16>(gbx::f32_to_act<BF16>(acc[j + 2][i][v]));
-          r = gbx::f32_to_act<BF16>(gbx::act_to_f32<BF16>(gbx::f32_to_act<BF16>(g / (1.f + __expf(-g)))) * u);
-        } else if (a.bias) {
-          r = gbx::f32_to_act<BF16>(gbx::act_to_f32<BF16>(r) + b);
-        }
-        *reinterpret_cast<unsigned short*>(ot + (i * 16 + 4 * f + v) * OROW + (j * 16 + fr) * 2) = r;
+        const float c = acc[j][i][v], u = GATED ? acc[j + 2][i][v] : 0.f;
+        odd = fmaf(c, 0.f, fmaf(u, 0.f, odd));
+        *reinterpret_cast<unsigned short*>(ot + (i * 16 + 4 * f + v) * OROW + (j * 16 + fr) * 2) = result(c, u, b);
       }
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  auto visible = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+  visible();
+  if (__any(odd != 0.f)) {                                              // infinite activations: those outputs again, weight by weight
+#pragma unroll 1
+    for (int p = lane; p < 16 * NR * OC; p += 64) {
+      const int row = p / OC, ch = c0 + p % OC;
+      unsigned short* at = reinterpret_cast<unsigned short*>(ot + row * OROW + p % OC * 2);
+      constexpr unsigned short MOST = BF16 ? 0x7F80 : 0x7C00;
+      if (lo + row >= hi || ch >= N || (*at & MOST) != MOST) continue;
+      const unsigned short* x = a.x + static_cast<int64_t>(a.sorted[lo + row] / a.x_div) * K;
+      float c[2] = {0.f, 0.f};
+      for (int m = 0; m < (GATED ? 2 : 1); ++m)
+        c[m] = gbx::expanded_dot<BITS, GRP, BF16>(x, a.w[m] + ew + ch * words, a.s[m] + eg + ch * groups, a.z[m] + eg + ch * groups, K);
+      *at = result(c[0], c[1], !GATED && a.bias ? gbx::act_to_f32<BF16>(a.bias[static_cast<int64_t>(e) * N + ch]) : 0.f);
+    }
+    visible();
+  }
   constexpr int PPR = OC / 8;                                           // 16-byte pieces per row
   const bool whole = c0 + OC <= N && N % 8 == 0;
 #pragma unroll

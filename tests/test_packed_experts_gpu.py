@@ -112,3 +112,37 @@ def test_replays_in_a_graph(oracle):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, run())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,g", [(2, 64), (3, 32), (3, 128), (4, 32), (4, 128)])
+def test_infinite_and_undefined_activations(oracle, bits, g, dt):
+    """An infinity times the weight, not infinity minus infinity; rows beside it keep their bits.  Tiles of every height, and the gated form."""
+    from gbx_lm_amd import ops
+    from gbx_lm_amd.models.switch_layers import QuantizedSwitchLinear
+    E, N, K = len(COUNTS), 200, 384
+    qw, s, z, w, _ = make(oracle, E, N, K, bits, g, dt, seed=bits)
+    idx = indices(3).to(DEV)
+    P = idx.numel()
+    x = torch.randn((P, 1, 1, K), device=DEV).to(dt)
+    plain = ops.gather_quantized_matmul(x, qw, s, z, idx[:, None], group_size=g, bits=bits).view(P, N)
+    odd = torch.arange(0, P, 3, device=DEV)
+    x.view(P, K)[odd, odd % K] = torch.tensor([float("inf"), float("-inf")], device=DEV, dtype=dt)[odd % 2]
+    x.view(P, K)[odd[::7], 17] = float("nan")
+    got = ops.gather_quantized_matmul(x, qw, s, z, idx[:, None], group_size=g, bits=bits).view(P, N)
+    sign = torch.where(odd % 2 == 0, 1.0, -1.0).double()[:, None] * w[idx[odd], :, odd % K].sign()
+    want = sign * float("inf")
+    want[::7] = float("nan")
+    assert bool((torch.isnan(got[odd]) == torch.isnan(want)).all()) and torch.equal(got[odd].double().nan_to_num(0, 1, -1), want.nan_to_num(0, 1, -1))
+    rest = torch.ones(P, dtype=torch.bool, device=DEV)
+    rest[odd] = False
+    assert torch.equal(got[rest], plain[rest])
+    if dt == torch.bfloat16:
+        up = make(oracle, E, N, K, bits, g, dt, seed=bits + 9)[:3]
+        mods = []
+        for t in ((qw, s, z), up):
+            m = QuantizedSwitchLinear(K, N, E, bias=False, group_size=g, bits=bits)
+            m._buffers["qweight"], m._buffers["scales"], m._buffers["zeros"] = t
+            mods.append(m)
+        a, b = ops.gather_swiglu(x, mods[0], mods[1], idx[:, None]), ops.swiglu(mods[0](x, idx[:, None]), mods[1](x, idx[:, None]))
+        assert torch.equal(a.float().nan_to_num(7e9, 8e9, -8e9), b.float().nan_to_num(7e9, 8e9, -8e9))
