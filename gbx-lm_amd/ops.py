@@ -18,8 +18,13 @@ _DT = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16, torch.float32
 
 
 def _stream_ptr(device) -> int:
-    """hipStream_t of the device's current stream (the raw handle: building a Stream object around it costs 2 us a launch)."""
-    index = (device if type(device) is torch.device else torch.device(device)).index
+    """hipStream_t of the device's current stream (the raw handle: building a Stream object around it costs 2 us a launch).  Other devices than the GPU
+    raise, as in ``torch.cuda.current_stream``: a launch must not see a host tensor's address."""
+    if type(device) is not torch.device:
+        device = torch.device(device)
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
+    index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 

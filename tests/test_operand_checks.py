@@ -1,0 +1,43 @@
+"""Operands that a kernel cannot take are met before any launch: the call raises, or goes the way on which torch or the general path
+refuses it.  Tensors that say they live on the device stand in for such a device's and every launch is a failure, so nothing here runs a kernel."""
+import pytest
+import torch
+
+from gbx_lm_amd import _lib, mixer_ops as M, ops
+
+
+class _NoLaunch:
+    """A library whose size queries answer and whose launches fail the test."""
+
+    def __getattr__(self, name):
+        if name.endswith(("_workspace", "_workspace_bytes")):
+            return lambda *a: 1 << 20
+
+        def launch(*a):
+            raise AssertionError(f"{name} was reached")
+        return launch
+
+
+@pytest.fixture
+def no_launch(monkeypatch):
+    lib = _NoLaunch()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(_lib, "mixers", lambda: lib)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda device: 0)
+    monkeypatch.setattr(M, "_stream", lambda device: 0)
+
+
+def bf16(*shape):
+    return torch.randn(*shape).bfloat16()
+
+
+def test_only_devices_have_streams(monkeypatch):
+    """A host tensor that reaches a launch is refused there, as torch's own lookup of a current stream refuses it."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 7, raising=False)
+    for name in ("cpu", torch.device("cpu"), torch.device("meta")):
+        for lookup in (ops._stream_ptr, M._stream):
+            with pytest.raises(ValueError, match="cuda device"):
+                lookup(name)
+    for name in ("cuda:0", "cuda", torch.device("cuda", 1)):
+        assert ops._stream_ptr(name) == M._stream(name) == 7
