@@ -97,13 +97,15 @@ def stream_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, act_dtype: torc
 def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``x @ w.T (+ bias)`` of few bf16 rows [T, K] as one launch, or None for what the kernel does not take (it wins over the vendor library's
     product up to 16 rows of 4096 channels and 32 of 2048: csrc/mixers_rows.hip; longer contractions are the library's, 2048 x 8192: 12.6 us both)."""
-    t, k = x.shape
-    stride = x.stride(0)
-    if (t > 32 or k % 64 or k > (2048 if t > 16 else 4096) or t == 0 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.stride(1) != 1
-            or stride % 8 or stride < k or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16 or w.shape[1] != k or w.device != x.device
-            or (bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_contiguous()))):
+    if x.dim() != 2 or w.dim() != 2:
         return None
-    n = w.shape[0]
+    (t, k), n, stride = x.shape, w.shape[0], x.stride(0)
+    if (t > 32 or k % 64 or k > (2048 if t > 16 else 4096) or not (t and k and 0 < n <= 1 << 26) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
+            or x.stride(1) != 1 or stride % 8 or stride < k or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16 or w.shape[1] != k
+            or w.device != x.device):
+        return None
+    if bias is not None and (bias.shape != (n,) or bias.device != x.device or bias.dtype != torch.bfloat16 or not bias.is_contiguous()):
+        return None
     y = torch.empty((t, n), dtype=torch.bfloat16, device=x.device)
     _lib.check_mixers(_lib.mixers().gbxm_linear_rows(x.data_ptr(), stride, w.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), n, t, n,
                                                     k, _stream(x.device)))

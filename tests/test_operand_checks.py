@@ -41,3 +41,15 @@ def test_only_devices_have_streams(monkeypatch):
                 lookup(name)
     for name in ("cuda:0", "cuda", torch.device("cuda", 1)):
         assert ops._stream_ptr(name) == M._stream(name) == 7
+
+
+@pytest.mark.parametrize("bias", [bf16(47), bf16(49), bf16(1), bf16(48, 1), torch.empty(48, dtype=torch.bfloat16, device="meta")],
+                         ids=["short", "long", "one", "column", "other device"])
+def test_row_products_leave_other_biases_to_torch(no_launch, bias):
+    """A bias that is not one value per output on the rows' device."""
+    assert M.linear_rows(bf16(4, 256), bf16(48, 256), bias) is None
+
+
+@pytest.mark.parametrize("x,w", [((4, 256), (0, 256)), ((4, 0), (48, 0)), ((4, 256), (256,)), ((2, 4, 256), (48, 256)), ((256,), (48, 256)), ((4, 256), (2, 48, 256))])
+def test_row_products_leave_other_shapes_to_torch(no_launch, x, w):
+    assert M.linear_rows(bf16(*x), bf16(*w), None) is None
