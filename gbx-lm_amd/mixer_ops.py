@@ -121,8 +121,12 @@ def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
     17.4 -> 5.0)."""
     act = _act(h, "h")
     _f32(router, "router")
+    if h.dim() != 2 or router.dim() != 2:
+        raise ValueError("rows [T, W] and a router [experts, W]")
+    if router.device != h.device:
+        raise RuntimeError(f"rows on {h.device}, router on {router.device}")
     t, rows = h.shape[0], router.shape[0]
-    if t > ROUTER_ROWS or h.shape[1] != router.shape[1]:
+    if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1]:
         return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
     h = h.contiguous()
     logits = torch.empty((t, rows), dtype=torch.float32, device=h.device)

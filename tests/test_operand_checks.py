@@ -53,3 +53,26 @@ def test_row_products_leave_other_biases_to_torch(no_launch, bias):
 @pytest.mark.parametrize("x,w", [((4, 256), (0, 256)), ((4, 0), (48, 0)), ((4, 256), (256,)), ((2, 4, 256), (48, 256)), ((256,), (48, 256)), ((4, 256), (2, 48, 256))])
 def test_row_products_leave_other_shapes_to_torch(no_launch, x, w):
     assert M.linear_rows(bf16(*x), bf16(*w), None) is None
+
+
+class OnDevice(torch.Tensor):
+    """A host tensor that says it is the GPU's (results of operations on it say so too)."""
+    is_cuda = property(lambda self: True)
+
+
+def dev(t):
+    return t.as_subclass(OnDevice)
+
+
+ROUTERS = [lambda h, r: M.route_topk(h, r, 2), lambda h, r: M.route_sigmoid_groups(h, r, torch.zeros(8), 2, None, False, 1.0),
+           lambda h, r: M.route_groups(h, r, 8, 2, None)]
+
+
+@pytest.mark.parametrize("route", ROUTERS, ids=["softmax", "sigmoid", "groups"])
+def test_routers_on_other_devices_and_rows_of_other_ranks_raise(no_launch, route):
+    router = torch.randn(8, 64)
+    with pytest.raises((RuntimeError, ValueError)):
+        route(dev(torch.randn(4, 64)), router.to("meta"))
+    for h in (torch.randn(64), torch.randn(4, 64, 64), torch.randn(4, 32)):
+        with pytest.raises((RuntimeError, ValueError, IndexError)):
+            route(dev(h), router)
