@@ -15,6 +15,7 @@ import torch
 from . import _lib, env
 
 _DT = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16, torch.float32: _lib.GBX_F32}
+_ACT16 = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16}              # what activations of a product may be
 
 
 def _stream_ptr(device) -> int:
@@ -412,7 +413,8 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     x: [..., 1, 1, K] or [..., k, 1, K]; rhs_indices: [..., k] -> [..., k, 1, N].  Few (token, slot) pairs run the
     expert-indexed decode GEMV in ONE launch; many pairs are bucketed by expert on the device and run as tiles of the matrix cores
     (``_packed_experts``); what neither takes is grouped on the host (one batched GEMM per expert present).  The reference's
-    ``sorted_indices`` hint needs no special handling."""
+    ``sorted_indices`` hint needs no special handling.  An index that names no expert is not looked for on the host, which would have to wait for the
+    device: among many pairs its row is NaN, among few the nearest expert's."""
     if not transpose:
         raise NotImplementedError("gather_quantized_matmul supports transpose=True only (the reference's only use)")
     for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases"), (rhs_indices, "rhs_indices")):
@@ -470,9 +472,22 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
 
 def _packed_experts(xr: torch.Tensor, first, second, bias, idx: torch.Tensor, x_div: int, E: int, N: int, K: int, bits: int, group_size: int):
     """Rows [pairs, N] of the chosen experts' products over many (token, slot) pairs (gbxm_packed_experts): ``first`` = (qweight, scales,
-    zeros) [E, ...]; with ``second`` alike, silu(first) * second.  None where the launch does not serve the shapes."""
-    L = _lib.mixers()
+    zeros) [E, ...]; with ``second`` alike, silu(first) * second.  None where the launch does not serve the operands (the caller's other path
+    takes or refuses them)."""
     pairs = idx.numel()
+    if xr.dtype not in _ACT16 or not idx.is_cuda or idx.dtype not in (torch.int32, torch.int64) or xr.shape[0] * x_div != pairs or K % 128 or bits not in (2, 3, 4):
+        return None
+    words, groups = (E, N, K * bits // 32), (E, N, K // group_size)
+    for q, s, z in (first, second or first):
+        if not (q is not None and s is not None and z is not None and q.is_cuda and s.is_cuda and z.is_cuda and q.dtype in (torch.uint32, torch.int32)
+                and s.dtype == z.dtype == xr.dtype and q.shape == words and s.shape == z.shape == groups and q.is_contiguous() and s.is_contiguous()
+                and z.is_contiguous()):
+            return None
+    if bias is not None:
+        if not bias.is_cuda or bias.dtype != xr.dtype or bias.shape != (E, N):
+            return None
+        bias = bias.contiguous()
+    L = _lib.mixers()
     nbytes = L.gbxm_packed_experts_workspace(pairs, K, E)
     if not nbytes:
         return None
@@ -496,12 +511,10 @@ def gather_swiglu(x: torch.Tensor, gate, up, rhs_indices: torch.Tensor):
     K, N, k = x.shape[-1], gate.output_dims, rhs_indices.shape[-1]
     pairs = rhs_indices.numel()
     max_k = 512 * (64 if gate.bits == 2 else 32)
-    if (x.is_cuda and x.dtype in _DT and (pairs > 64 or K > max_k) and pairs and x.shape[-2] == 1 and x.shape[-3] in (1, k)
-            and (gate.bits, gate.group_size, gate.output_dims, gate.input_dims) == (up.bits, up.group_size, up.output_dims, up.input_dims)
-            and gate.num_experts == up.num_experts and gate.input_dims == K
-            and getattr(gate, "bias", None) is None and getattr(up, "bias", None) is None
-            and gate.scales.dtype == x.dtype and up.scales.dtype == x.dtype and gate.zeros.dtype == x.dtype and up.zeros.dtype == x.dtype
-            and all(t.is_contiguous() for m in (gate, up) for t in (m.qweight, m.scales, m.zeros))):
+    if (x.is_cuda and x.dtype in _ACT16 and (pairs > 64 or K > max_k) and pairs and x.dim() >= 3 and x.shape[-2] == 1 and x.shape[-3] in (1, k)
+            and x.shape[:-3] == rhs_indices.shape[:-1] and (gate.bits, gate.group_size, gate.output_dims, gate.input_dims, gate.num_experts)
+            == (up.bits, up.group_size, up.output_dims, up.input_dims, up.num_experts) and gate.input_dims == K
+            and getattr(gate, "bias", None) is None and getattr(up, "bias", None) is None):
         y = _packed_experts(x.reshape(-1, K).contiguous(), (gate.qweight, gate.scales, gate.zeros), (up.qweight, up.scales, up.zeros), None,
                             rhs_indices.reshape(-1), k if x.shape[-3] == 1 else 1, gate.num_experts, N, K, gate.bits, gate.group_size)
         return None if y is None else y.reshape(*rhs_indices.shape[:-1], k, 1, N)

@@ -76,3 +76,57 @@ def test_routers_on_other_devices_and_rows_of_other_ranks_raise(no_launch, route
     for h in (torch.randn(64), torch.randn(4, 64, 64), torch.randn(4, 32)):
         with pytest.raises((RuntimeError, ValueError, IndexError)):
             route(dev(h), router)
+
+
+def experts(e=6, n=64, k=256, g=64, bits=4, dt=torch.bfloat16):
+    from gbx_lm_amd.models.switch_layers import QuantizedSwitchLinear
+    m = QuantizedSwitchLinear(k, n, e, bias=False, group_size=g, bits=bits)
+    qw = torch.zeros((e, n, k // 32 * bits), dtype=torch.int32)
+    m._buffers["qweight"], m._buffers["scales"], m._buffers["zeros"] = dev(qw), dev(torch.ones(e, n, k // g).to(dt)), dev(torch.zeros(e, n, k // g).to(dt))
+    return m
+
+
+def changed(m, **buffers):
+    for name, t in buffers.items():
+        m._buffers[name] = dev(t)
+    return m
+
+
+X, IDX = (100, 1, 1, 256), (torch.arange(100) % 6).to(torch.int32)[:, None]
+GATED = {
+    "rows in 32 bits": lambda: (dev(torch.randn(X)), experts(dt=torch.float32), IDX),
+    "other leading sizes": lambda: (dev(bf16(90, 1, 1, 256)), experts(), IDX),
+    "one row for all": lambda: (dev(bf16(1, 1, 1, 256)), experts(), IDX),
+    "leading sizes in another order": lambda: (dev(bf16(50, 2, 1, 1, 256)), experts(), IDX.view(2, 50, 1)),
+    "too few experts": lambda: (dev(bf16(*X)), changed(experts(), qweight=torch.zeros(5, 64, 32, dtype=torch.int32)), IDX),
+    "too few outputs": lambda: (dev(bf16(*X)), changed(experts(), qweight=torch.zeros(6, 60, 32, dtype=torch.int32)), IDX),
+    "too few groups": lambda: (dev(bf16(*X)), changed(experts(), scales=bf16(6, 64, 2)), IDX),
+    "zeros of another shape": lambda: (dev(bf16(*X)), changed(experts(), zeros=bf16(6, 64, 2)), IDX),
+    "words of another type": lambda: (dev(bf16(*X)), changed(experts(), qweight=torch.zeros(6, 64, 32)), IDX),
+    "indices that are no integers": lambda: (dev(bf16(*X)), experts(), IDX.float()),
+    "indices on the host": lambda: (dev(bf16(*X)), experts(), IDX),
+    "weights on the host": lambda: (dev(bf16(*X)), experts(), IDX),
+}
+
+
+@pytest.mark.parametrize("name", list(GATED))
+def test_gated_experts_leave_what_they_cannot_take_to_the_separate_products(no_launch, name):
+    x, m, idx = GATED[name]()
+    if name == "weights on the host":
+        m._buffers["scales"] = m.scales.as_subclass(torch.Tensor)
+    assert ops.gather_swiglu(x, m, m, idx if name == "indices on the host" else dev(idx)) is None
+
+
+def test_gated_experts_of_fitting_operands_reach_the_launch(no_launch):
+    with pytest.raises(AssertionError, match="gbxm_packed_experts was reached"):
+        ops.gather_swiglu(dev(bf16(*X)), experts(), experts(), dev(IDX))
+
+
+@pytest.mark.parametrize("name", ["too few groups", "zeros of another shape", "words of another type", "short bias", "wide bias", "bias on the host", "indices that are no integers"])
+def test_experts_of_many_pairs_leave_what_they_cannot_take_to_one_expert_at_a_time(no_launch, monkeypatch, name):
+    """... whose products refuse it."""
+    x, m, idx = GATED[name]() if name in GATED else (dev(bf16(*X)), experts(), IDX)
+    bias = {"short bias": dev(bf16(6, 32)), "wide bias": dev(bf16(6, 65)), "bias on the host": bf16(6, 64)}.get(name)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    with pytest.raises((ValueError, RuntimeError, TypeError, IndexError)):
+        ops.gather_quantized_matmul(x, m.qweight, m.scales, m.zeros, dev(idx), group_size=64, bits=4, bias=bias)

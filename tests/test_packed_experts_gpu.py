@@ -146,3 +146,31 @@ def test_infinite_and_undefined_activations(oracle, bits, g, dt):
             mods.append(m)
         a, b = ops.gather_swiglu(x, mods[0], mods[1], idx[:, None]), ops.swiglu(mods[0](x, idx[:, None]), mods[1](x, idx[:, None]))
         assert torch.equal(a.float().nan_to_num(7e9, 8e9, -8e9), b.float().nan_to_num(7e9, 8e9, -8e9))
+
+
+def test_a_bias_in_another_order_is_read_in_its_own(oracle):
+    from gbx_lm_amd import ops
+    E, N, K = 5, 72, 128
+    qw, s, z, _, _ = make(oracle, E, N, K, 4, 64, torch.bfloat16, 9)
+    idx = (torch.arange(100, device=DEV) % E)[:, None]
+    x, bias = torch.randn((100, 1, 1, K), device=DEV).to(torch.bfloat16), torch.randn((E, N), device=DEV).to(torch.bfloat16)
+    run = lambda b: ops.gather_quantized_matmul(x, qw, s, z, idx, group_size=64, bits=4, bias=b)
+    assert torch.equal(run(bias.t().contiguous().t()), run(bias))
+
+
+def test_rows_in_32_bits_are_refused(oracle):
+    """The launch reads 16-bit rows: anything else raises, as one matrix at a time does."""
+    from gbx_lm_amd import ops
+    from gbx_lm_amd.models.switch_layers import QuantizedSwitchLinear
+    E, N, K = 6, 64, 256
+    mods = []
+    for seed in (1, 2):
+        qw, s, z, _, _ = make(oracle, E, N, K, 4, 64, torch.float32, seed)
+        m = QuantizedSwitchLinear(K, N, E, bias=False, group_size=64, bits=4)
+        m._buffers["qweight"], m._buffers["scales"], m._buffers["zeros"] = qw, s, z
+        mods.append(m)
+    idx = (torch.arange(100, device=DEV) % E)[:, None].to(torch.int32)
+    x = torch.randn((100, 1, 1, K), device=DEV)
+    assert ops.gather_swiglu(x, mods[0], mods[1], idx) is None
+    with pytest.raises(ValueError):
+        mods[0](x, idx)
