@@ -197,7 +197,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases")):
             _require_cuda(t, nm)
     dt = x.dtype
-    act = _DT.get(dt)
+    act = _ACT16.get(dt)
     if act is None:
         raise ValueError(f"activations must be float16 or bfloat16, got {dt}")
     if w.dtype not in (torch.uint32, torch.int32):

@@ -130,3 +130,13 @@ def test_experts_of_many_pairs_leave_what_they_cannot_take_to_one_expert_at_a_ti
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     with pytest.raises((ValueError, RuntimeError, TypeError, IndexError)):
         ops.gather_quantized_matmul(x, m.qweight, m.scales, m.zeros, dev(idx), group_size=64, bits=4, bias=bias)
+
+
+@pytest.mark.parametrize("rows", [1, 300, 1024])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64, torch.int32])
+def test_activations_of_a_packed_product_are_16_bits(no_launch, monkeypatch, rows, dt):
+    """... and nothing is converted or allocated for others."""
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: pytest.fail("allocated"))
+    w, s = dev(torch.zeros(64, 32, dtype=torch.int32)), dev(torch.ones(64, 4).bfloat16())
+    with pytest.raises(ValueError, match="float16 or bfloat16"):
+        ops.quantized_matmul(dev(torch.ones(rows, 256, dtype=dt)), w, s, s, group_size=64, bits=4)
