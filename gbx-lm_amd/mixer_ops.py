@@ -155,10 +155,11 @@ _LSM = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32, torch.floa
 
 
 def log_probabilities(logits: torch.Tensor) -> torch.Tensor:
-    """``logits - logsumexp(logits)`` over the last axis, the logarithm formed in fp32 and rounded to the logits' dtype: one launch on the
-    GPU (two for a few long rows), torch elsewhere."""
+    """``logits - logsumexp(logits)`` over the last axis, the logarithm formed in fp32 (fp64 for fp64) and rounded to the logits' dtype: one launch
+    on the GPU (two for a few long rows), torch elsewhere."""
     if not logits.is_cuda or logits.dtype not in _LSM or not logits.numel():
-        return logits - torch.logsumexp(logits.float(), dim=-1, keepdim=True).to(logits.dtype)
+        wide = logits if logits.dtype == torch.float64 else logits.float()
+        return logits - torch.logsumexp(wide, dim=-1, keepdim=True).to(logits.dtype)
     x = logits.contiguous()
     n = x.shape[-1]
     out = torch.empty_like(x)

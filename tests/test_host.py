@@ -375,3 +375,10 @@ def test_graph_capture_runs_without_the_garbage_collector(monkeypatch):
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+def test_log_probabilities_of_64_bit_logits_stay_in_64_bits():
+    import torch
+    from gbx_lm_amd.mixer_ops import log_probabilities
+    x = torch.randn(3, 1000, dtype=torch.float64) * 5
+    assert torch.equal(log_probabilities(x), x - torch.logsumexp(x, -1, keepdim=True))
