@@ -10,6 +10,7 @@ import ctypes
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -24,6 +25,19 @@ def _stream(device) -> int:
         raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def outside_torch(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether nothing in torch is to see an operation on ``tensors``, so that a launch may stand in for it: plain tensors, no gradient or forward-mode
+    tangent wanted, no trace being recorded, no transform, dispatch mode or autocast active."""
+    if torch.compiler.is_compiling():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)):
+            return False
+    return (forward_ad._current_level < 0 and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch._C._is_any_autocast_enabled())
 
 
 def _act(t: torch.Tensor, name: str) -> int:
@@ -157,7 +171,7 @@ _LSM = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32, torch.floa
 def log_probabilities(logits: torch.Tensor) -> torch.Tensor:
     """``logits - logsumexp(logits)`` over the last axis, the logarithm formed in fp32 (fp64 for fp64) and rounded to the logits' dtype: one launch
     on the GPU (two for a few long rows), torch elsewhere."""
-    if not logits.is_cuda or logits.dtype not in _LSM or not logits.numel():
+    if not (logits.is_cuda and logits.dtype in _LSM and logits.numel() and outside_torch(logits)):
         wide = logits if logits.dtype == torch.float64 else logits.float()
         return logits - torch.logsumexp(wide, dim=-1, keepdim=True).to(logits.dtype)
     x = logits.contiguous()

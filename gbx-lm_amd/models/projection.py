@@ -1,5 +1,5 @@
 """``x @ w.T (+ bias)`` with unquantised weights: a decode step's few rows on the HIP kernel that streams the weights once, everything else (prompts,
-fp32, long contractions, tensors that gradients are wanted for) on ``F.linear``."""
+fp32, long contractions, whatever torch is to see for gradients, transforms, traces or autocast) on ``F.linear``."""
 from __future__ import annotations
 
 from typing import Optional
@@ -8,10 +8,11 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .. import mixer_ops as M
+
 
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    if x.is_cuda and x.numel() <= 32 * x.shape[-1] and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
-        from .. import mixer_ops as M
+    if isinstance(x, torch.Tensor) and x.is_cuda and 0 < x.numel() <= 32 * x.shape[-1] and M.outside_torch(x, w, bias):
         y = M.linear_rows(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), w, bias)
         if y is not None:
             return y if x.dim() == 2 else y.view(*x.shape[:-1], w.shape[0])

@@ -47,3 +47,35 @@ def test_what_stays_with_the_library():
     assert y.shape == (2, 2, 48) and torch.equal(y.view(4, 48), M.linear_rows(x, w, b))
     wg = w.clone().requires_grad_(True)
     assert project(x, wg, b).requires_grad and not project(x, wg.detach(), b).requires_grad
+
+
+def test_what_torch_does_around_a_product_stays():
+    """Gradients of a bias alone, forward-mode tangents, vmap, autocast, symbolic and recorded traces, dispatch modes: the rows then go through torch."""
+    import torch.autograd.forward_ad as fw
+    from torch.utils.flop_counter import FlopCounterMode
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.models.projection import RowLinear, project
+    x, w, b = case(4, 48, 256, True, 0, 3)
+    bg = b.clone().requires_grad_(True)
+    project(x, w, bg).float().sum().backward()
+    assert torch.equal(bg.grad, torch.full_like(b, 4.0))
+    with torch.no_grad(), fw.dual_level():
+        t = torch.ones_like(x)
+        assert torch.equal(fw.unpack_dual(project(fw.make_dual(x, t), w, b)).tangent, F.linear(t, w))
+    xs = torch.stack([x, x + 1])
+    with torch.no_grad():
+        assert torch.equal(torch.func.vmap(lambda v: project(v, w, b))(xs), torch.func.vmap(lambda v: F.linear(v, w, b))(xs))
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert project(x, w, b).dtype == torch.float16
+        with FlopCounterMode(display=False) as flops:
+            project(x, w, b)
+        assert flops.get_total_flops() == 2 * 4 * 48 * 256
+        layer = RowLinear(256, 48, device=DEV, dtype=torch.bfloat16)
+        traced = torch.jit.trace(layer, (x,))
+        assert torch.equal(traced(x + 1), F.linear(x + 1, layer.weight, layer.bias))
+        symbolic = torch.fx.symbolic_trace(layer)
+        assert torch.equal(symbolic(x), F.linear(x, layer.weight, layer.bias))
+        compiled = torch.compile(lambda v: project(v, w, b) * 2, backend="eager", fullgraph=True)
+        assert torch.equal(compiled(x), F.linear(x, w, b) * 2)
+        assert torch.equal(project(x[:, :0], w[:, :0], b), F.linear(x[:, :0], w[:, :0], b))
+        assert not torch.equal(project(x, w, b), torch.zeros_like(project(x, w, b))) and torch.equal(project(x, w, b), M.linear_rows(x, w, b))

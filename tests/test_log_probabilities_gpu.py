@@ -57,3 +57,19 @@ def test_slices_without_a_candidate(dt):
         ok = torch.isfinite(x[r])
         assert (got[r][~ok] == float("-inf")).all()
         assert bool(((got[r].double() - want[r]).abs()[ok] <= LAST[dt] * (lse[r].abs() + want[r].abs()[ok]) + 2.0 ** -22 * (1 + lse[r].abs())).all())
+
+
+def test_what_torch_does_around_the_rows_stays():
+    """Gradients, forward-mode tangents and vmap of the logits: torch's operations."""
+    import torch.autograd.forward_ad as fw
+    from gbx_lm_amd.mixer_ops import log_probabilities
+    x = torch.randn((3, 500), device="cuda")
+    g = x.clone().requires_grad_(True)
+    log_probabilities(g)[:, 0].sum().backward()
+    want = -torch.softmax(x, -1)
+    want[:, 0] += 1
+    assert torch.allclose(g.grad, want, atol=1e-6)
+    with torch.no_grad(), fw.dual_level():
+        t = torch.ones_like(x)
+        assert fw.unpack_dual(log_probabilities(fw.make_dual(x, t))).tangent.abs().max() < 1e-5
+    assert torch.allclose(torch.func.vmap(log_probabilities)(x[None].expand(2, 3, 500))[1], log_probabilities(x), atol=1e-5)
