@@ -28,6 +28,12 @@ template <typename T> struct Lanes<T, 1> {
   static __device__ __forceinline__ void load(const T* p, float* v) { v[0] = to_f32(*p); }
   static __device__ __forceinline__ void store(T* p, const float* v) { *p = from_f32<T>(v[0]); }
 };
+template <> struct Lanes<float, 2> {
+  static __device__ __forceinline__ void load(const float* p, float* v) {
+    const float2 f = *reinterpret_cast<const float2*>(p);
+    v[0] = f.x; v[1] = f.y;
+  }
+};
 template <> struct Lanes<float, 4> {
   static __device__ __forceinline__ void load(const float* p, float* v) {
     const float4 f = *reinterpret_cast<const float4*>(p);

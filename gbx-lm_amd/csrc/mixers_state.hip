@@ -105,16 +105,19 @@ __global__ __launch_bounds__(NT) void conv_tail_kernel(const T* __restrict__ y, 
 // NW waves per workgroup = 4 NW columns of one (sequence, head).  The operands of CH tokens (q | k | decay padded to 16 R channels, the
 // workgroup's value columns; the betas beside them) are staged in LDS, shared by the waves, two buffers: the next chunk is fetched into registers
 // before the current one is computed and parked in the other buffer afterwards, one barrier per chunk.  Lane ks of a 16-lane row owns the key
-// channels 4 ks .. 4 ks + 3, and those 64, 128, ... further on: LDS reads, and the state's loads and stores, are 16-byte accesses that are
-// contiguous over the row.  Bound by issue slots (a long prompt leaves one or two waves a SIMD, each token costs a wave 4 R multiply-adds and what
+// channels 4 ks .. 4 ks + 3, and those 64, 128, ... further on (R a multiple of 4; heads of up to 16, 32 or 96 channels: 1, 2 or 2 neighbours): LDS reads,
+// and the state's loads and stores, are 16-byte accesses that are contiguous over the row.  Bound by issue slots (a long prompt leaves one or two waves a SIMD, each token costs a wave 4 R multiply-adds and what
 // feeds them), so operands are read four at a time: V = 4 floats per staging access where sizes, strides and addresses allow, else 1.
 // (4-byte accesses and operands read where they are used -> now, us: rows of 1501 + 700 + 65 tokens, 8 heads of 128 x 256 393 -> 253, delta rule over 32
 // of 128 x 128 507 -> 351; 32 prompts of 8 to 163 tokens 273 -> 144; one token of 32 sequences, 67 MB of state 30.1 -> 15.1.)
+// Heads of few channels have forms of their own, which stage and multiply no more than there is (16 heads, 32 prompts of 40 tokens, every lane four
+// channels | this: 16 x 64 25.3 | 15.6, 32 x 128 45.3 | 29.5, 16 x 50 element by element 44.4 | 17.7); 48 channels are the four-channel form's (R = 3 at
+// one channel a lane 51.6, 28.4 here), 66 to 96 only where sizes are not in groups of four (94 x 64 59.4 | 43.1; 96 x 96 in groups of four 50).
 template <int R, bool DELTA, int NW, int V>
 __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __restrict__ r, int64_t r_stride, float* __restrict__ state,
                                                             float* __restrict__ out, const int* __restrict__ seq, int H, int G, int dk, int dv) {
-  static_assert(R % 4 == 0, "four neighbouring channels per access");
-  constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL, NTH = 64 * NW, Q = R / 4;
+  constexpr int C = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;                 // neighbouring channels of a lane
+  constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL, NTH = 64 * NW, Q = R / C;
   constexpr int CH = NW == 1 ? (R <= 4 ? 4 : 2) : (R <= 4 ? 32 : (R <= 8 ? 16 : 8)) * NW / 4;     // one-wave workgroups serve steps of few rows
   constexpr int SLOTS = CH * ROW / V, PF = (SLOTS + NTH - 1) / NTH;
   __shared__ __attribute__((aligned(16))) float buf[2][CH * ROW];
@@ -133,15 +136,15 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
   float S[R];
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
-    const int c = 4 * ks + 64 * i;
-    if constexpr (V == 4) {
+    const int c = C * ks + 16 * C * i;
+    if constexpr (V == 4 && C == 4) {
       Lanes<float, 4>::load(sp + min(c, dk - 4), S + 4 * i);
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) S[4 * i + j] = sp[min(c + j, dk - 1)];
+      for (int j = 0; j < C; ++j) S[C * i + j] = sp[min(c + j, dk - 1)];
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) S[4 * i + j] = (pos0 > 0 && c + j < dk) ? S[4 * i + j] : 0.f;
+    for (int j = 0; j < C; ++j) S[C * i + j] = (pos0 > 0 && c + j < dk) ? S[C * i + j] : 0.f;
   }
   const float* base = r + static_cast<int64_t>(row0) * r_stride;
   const int oq = g * dk, ok = nq + g * dk, ov = 2 * nq + h * dv, og = 2 * nq + nv + h * dk, ob = 2 * nq + nv + H * dk + h;
@@ -192,12 +195,12 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
     const int cn = min(CH, n - t0);
     struct Token { float q[R], k[R], d[R], v, beta; };
     auto read = [&](int tt, Token& x) {
-      const float* at = cur + tt * ROW + 4 * ks;
+      const float* at = cur + tt * ROW + C * ks;
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        Lanes<float, 4>::load(at + 64 * i, x.q + 4 * i);
-        Lanes<float, 4>::load(at + DKP + 64 * i, x.k + 4 * i);
-        Lanes<float, 4>::load(at + 2 * DKP + 64 * i, x.d + 4 * i);
+        Lanes<float, C>::load(at + 16 * C * i, x.q + C * i);
+        Lanes<float, C>::load(at + DKP + 16 * C * i, x.k + C * i);
+        Lanes<float, C>::load(at + 2 * DKP + 16 * C * i, x.d + C * i);
       }
       x.v = cur[tt * ROW + 3 * DKP + lcol];
       if (DELTA) x.beta = betas[which][tt];
@@ -242,13 +245,13 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
   if (col_ok) {
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-      const int c = 4 * ks + 64 * i;
-      if constexpr (V == 4) {
+      const int c = C * ks + 16 * C * i;
+      if constexpr (V == 4 && C == 4) {
         if (c < dk) Lanes<float, 4>::store(sp + c, S + 4 * i);
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (c + j < dk) sp[c + j] = S[4 * i + j];
+        for (int j = 0; j < C; ++j)
+          if (c + j < dk) sp[c + j] = S[C * i + j];
       }
     }
   }
@@ -285,7 +288,10 @@ int launch_scan(int R, int B, hipStream_t s, const float* r, int64_t r_stride, f
     if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);   \
     else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);       \
   } while (0)
-  if (R <= 4) GBXM_SCAN(4);
+  if (R <= 1) GBXM_SCAN(1);
+  else if (R <= 2) GBXM_SCAN(2);
+  else if (R <= 4) GBXM_SCAN(4);
+  else if (R <= 6 && !vec) state_scan_kernel<6, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);
   else if (R <= 8) GBXM_SCAN(8);
   else if (R <= 12) GBXM_SCAN(12);
   else GBXM_SCAN(16);

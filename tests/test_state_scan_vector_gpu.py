@@ -16,6 +16,18 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("dk,dv,H", [(4, 4, 4), (60, 20, 4), (64, 16, 2), (68, 12, 4), (128, 36, 4), (132, 8, 4), (192, 4, 4), (196, 4, 3), (256, 20, 4), (62, 20, 4), (64, 18, 4)])
 @pytest.mark.parametrize("counts", [(33, 15), (1, 2), (7, 8)])
 def test_scan(dk, dv, H, counts, delta):
+    scan(dk, dv, H, counts, delta)
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("dk,dv,H", [(1, 3, 2), (4, 20, 4), (15, 4, 3), (16, 36, 4), (17, 5, 3), (20, 8, 4), (31, 18, 4), (32, 16, 4), (33, 4, 3), (66, 18, 4), (95, 7, 3), (96, 6, 4), (97, 4, 3)])
+@pytest.mark.parametrize("counts", [(33, 15), (1, 2)])
+def test_heads_of_few_channels(dk, dv, H, counts, delta):
+    """Lanes of one, two and four channels: the first and last sizes of each."""
+    scan(dk, dv, H, counts, delta)
+
+
+def scan(dk, dv, H, counts, delta):
     G, g = 1, torch.Generator().manual_seed(dk + dv + counts[0])
     lay = RM.RecurrentLayout(H, G, dk, dv, 0, G * dk, 2 * G * dk, 2 * G * dk + H * dv if delta else -1)
     T = sum(counts)
