@@ -8,6 +8,8 @@
 //   * B operand: lane (n = l&31, h = l>>5) dequantises 8 consecutive k of weight row n from its own packed words.
 //   * A operand: lane (m = l&31, h) loads its 8 consecutive k of activation row m straight from global memory (x is
 //     at most 64 rows: L2-resident), one chunk ahead in registers.
+// What still runs here: 33 to 64 rows outside the wide projections, and of 2 to 32 rows those that mfma_rows.hip leaves -- contractions of 512 to 896, and
+// groups of 32 or 64 whose scales or zeros are not aligned to a chunk's.
 // Replaces mx.quantized_matmul for x of shape [B, 1, K] with 2 <= B <= 64 (gbx_lm/models/quantized_linear_gba.py:195-203).
 #include "mfma_common.h"
 #include "gbx_env.h"
@@ -227,9 +229,11 @@ static hipError_t launch_skinny_mt(const MfmaArgs& a, bool bf16, hipStream_t s) 
   // 8-way K split (a wave holds its whole K range in one window at K = 4096), 4-way for short rows
   const int nchunks = a.K / KC;
   // wide scale/zero loads need every window to start at an even chunk (4-byte aligned pair of 16-bit values)
-  const bool g128 = a.log2g == 7 && (nchunks % 16) == 0;
-  if (nchunks >= 32) return g128 ? launch_skinny_cfg<BITS, TN, MT, 8, true>(a, bf16, s) : launch_skinny_cfg<BITS, TN, MT, 8, false>(a, bf16, s);
-  return g128 ? launch_skinny_cfg<BITS, TN, MT, 4, true>(a, bf16, s) : launch_skinny_cfg<BITS, TN, MT, 4, false>(a, bf16, s);
+  if constexpr (MT * TN > 32) {
+    if (a.log2g == 7 && nchunks % 16 == 0)
+      return nchunks >= 32 ? launch_skinny_cfg<BITS, TN, MT, 8, true>(a, bf16, s) : launch_skinny_cfg<BITS, TN, MT, 4, true>(a, bf16, s);
+  }
+  return nchunks >= 32 ? launch_skinny_cfg<BITS, TN, MT, 8, false>(a, bf16, s) : launch_skinny_cfg<BITS, TN, MT, 4, false>(a, bf16, s);
 }
 
 template <int BITS>
