@@ -299,11 +299,14 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   float sum = 0.f;
   for (int e = threadIdx.x; e < E; e += NT) { const float p = expf(lg[e] - mx); lg[e] = p; sum += p; }
   sum = block_sum<NW>(sum, red);
-  for (int e = threadIdx.x; e < E; e += NT) lg[e] = lg[e] / sum;
+  for (int e = threadIdx.x; e < E; e += NT) {
+    const float p = lg[e] / sum;
+    lg[e] = p == p ? p : -1.f;                                 // (not a number: behind every probability, but still an expert)
+  }
   __syncthreads();
   float chosen_sum = 0.f;
   for (int s = 0; s < top; ++s) {
-    float bv = -1.f;
+    float bv = -1.5f;                                          // (-2: taken)
     int bi = 0x7fffffff;
     for (int e = threadIdx.x; e < E; e += NT)
       if (lg[e] > bv) { bv = lg[e]; bi = e; }                  // ascending e per thread: the first of equals stays

@@ -217,16 +217,17 @@ __global__ __launch_bounds__(64) void route_sigmoid_groups_kernel(const float* _
   const int lane = threadIdx.x;
   for (int e = lane; e < E; e += 64) {
     const float s = 1.f / (1.f + expf(-logits[t * E + e]));
+    const float c = s + correction[e];
     sl[e] = s;
-    cl[e] = s + correction[e];
+    cl[e] = c == c ? c : -INFINITY;
   }
   __syncthreads();
-  // arg-max over n values of `v` (ties: the lower index); every lane gets the result
+  // arg-max over n values of `v` (ties: the lower index; not a number: taken); every lane gets the result
   auto arg_max = [&](const float* v, int n) {
     float bv = -INFINITY;
     int bi = 0x7fffffff;
     for (int e = lane; e < n; e += 64)
-      if (v[e] > bv || bi == 0x7fffffff) { bv = v[e]; bi = e; }          // ascending e per lane: the first of equals stays
+      if (v[e] > bv || (bi == 0x7fffffff && v[e] == v[e])) { bv = v[e]; bi = e; }          // ascending e per lane: the first of equals stays
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const float ov = __shfl_xor(bv, o, 64);
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(64) void route_sigmoid_groups_kernel(const float* _
     const int e = arg_max(cl, E);
     __syncthreads();
     chosen += sl[e];
-    if (lane == 0) { idx[t * top + k] = e; weight[t * top + k] = sl[e]; cl[e] = -INFINITY; }
+    if (lane == 0) { idx[t * top + k] = e; weight[t * top + k] = sl[e]; cl[e] = NAN; }
     __syncthreads();
   }
   const float mul = renorm ? scale / (chosen + 1e-20f) : scale;

@@ -67,3 +67,51 @@ def test_grouped_sigmoid_choice(e, top, groups, t, dt, renorm):
         assert all(abs(c[a].item() - c[b].item()) < 1e-6 or c[a] == c[b] for a, b in zip(got.tolist(), want))
         sw = s[got] * 1.5 / (s[got].sum() + 1e-20 if renorm else 1.0)
         assert float(((w[r].cpu().double() - sw).abs() / sw).max()) < 32 * 2.0 ** -24
+
+
+def odd_rows(e):
+    """Logit rows with numbers missing here and there or throughout, infinities of both signs, one candidate alone, all equal."""
+    rows = torch.randn((8, e), generator=torch.Generator().manual_seed(e))
+    rows[0, ::3], rows[1], rows[2, e // 2], rows[3], rows[4, e - 1] = float("nan"), float("nan"), float("inf"), float("-inf"), float("-inf")
+    rows[5], rows[5, e - 2], rows[6] = float("-inf"), 1.0, 0.25
+    return rows
+
+
+def choose(rows, top, groups=None, correction=None):
+    from gbx_lm_amd import _lib
+    t, e = rows.shape
+    logits, idx, w = rows.to(DEV).contiguous(), torch.full((t, top), -1, dtype=torch.int32, device=DEV), torch.empty((t, top), device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    if correction is None:
+        _lib.check_mixers(_lib.mixers().gbxm_route_topk(logits.data_ptr(), idx.data_ptr(), w.data_ptr(), t, e, top, 0, stream))
+    else:
+        count, keep = groups or (0, 0)
+        c = correction.to(DEV)
+        _lib.check_mixers(_lib.mixers().gbxm_route_sigmoid_groups(logits.data_ptr(), c.data_ptr(), idx.data_ptr(), w.data_ptr(), t, e, top, count, keep, 0, 1.0,
+                                                                  stream))
+    return idx.cpu(), w.cpu()
+
+
+@pytest.mark.parametrize("e,top", [(8, 8), (32, 2), (33, 2), (128, 8), (129, 8), (256, 16), (257, 3), (520, 8)])
+def test_softmax_choice_of_odd_logits(e, top):
+    """Always ``top`` different experts; a row without probabilities (a logit that is no number or +inf, none finite) gives the first ones."""
+    rows = odd_rows(e)
+    idx, _ = choose(rows, top)
+    p = torch.softmax(rows.double(), -1)
+    for r in range(len(rows)):
+        assert idx[r].tolist() == [i for _, i in sorted((-v if v == v else 1.0, i) for i, v in enumerate(p[r].tolist()))[:top]]
+
+
+@pytest.mark.parametrize("e,top,groups", [(8, 8, None), (22, 2, None), (24, 2, None), (88, 8, None), (89, 8, None), (128, 8, (8, 4)), (136, 8, (8, 4)), (256, 8, (8, 4)),
+                                          (256, 8, None), (520, 8, None)])
+def test_sigmoid_choice_of_odd_logits(e, top, groups):
+    """Always ``top`` different experts, those whose score is no number after all others (in groups: an order of its own, checked for being one)."""
+    rows, correction = odd_rows(e), torch.zeros(e)
+    idx, _ = choose(rows, top, groups, correction)
+    assert all(len(set(r)) == top and min(r) >= 0 and max(r) < e for r in idx.tolist())
+    if groups is None:
+        c = 1.0 / (1.0 + torch.exp(-rows))
+        for r in (0, 1, 2, 3, 4, 5, 6):
+            key = sorted((-v if v == v else 1.0, i) for i, v in enumerate(c[r].tolist()))
+            got = [c[r, i].item() for i in idx[r].tolist()]
+            assert all(a != a if v > 0 else abs(a + v) < 1e-6 for a, (v, _) in zip(got, key))
