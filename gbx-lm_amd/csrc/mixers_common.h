@@ -110,9 +110,14 @@ __device__ __forceinline__ int rank_of(const float* v, int n4, int e, float x) {
   }
   return rank;
 }
-// Experts up to which a router's choice goes by rank (every expert reads all scores; beyond, the rounds' work grows slower): sigmoid router of
-// 1 row x 32 experts 7.9 -> 5.4 us, of 2266 x 128 16.0 -> 13.6, softmax of 32 rows x 128 experts 11.7 -> 9.6.
-constexpr int RANK_EXPERTS = 512;
+// Where a router's choice goes by rank: every expert reads all scores, E / 16 steps of a wave, where each of the `rounds` of arg-max (one per choice and per
+// kept group) is a chain of its own; `per_round` steps cost what one of them does.  Measured, rounds | rank, us: softmax, top 8, 1 row: 64 experts
+// 9.7 | 5.2, 128 9.6 | 8.1, 256 9.5 | 14.1, 512 10.3 | 49; 4000 rows: 64 29.6 | 11.5, 128 30.0 | 20.8, 256 30.6 | 47; top 2, 1 row: 64 4.1 | 5.2.
+// Sigmoid, top 8, 1 row: 64 6.8 | 5.1, 128 7.4 | 7.9, 256 8.6 | 14.1; in 8 groups of which 4 stay 64 10.4 | 5.9, 128 11.9 | 9.0, 256 14.9 | 15.6, 4000 rows
+// 64 15.4 | 8.1, 128 17.0 | 17.5, 160 18.1 | 29.4; top 2 in groups 64 6.5 | 5.9, 96 7.2 | 7.5.
+constexpr int RANK_EXPERTS = 256;
+inline bool choice_by_rank(int E, int rounds, int per_round) { return E <= RANK_EXPERTS && E <= per_round * rounds; }
+constexpr int RANK_PER_SOFTMAX_ROUND = 16, RANK_PER_SIGMOID_ROUND = 11;
 
 // z = a row of a sublayer's output, or sum_k mix[k] (candidate row k), at channels c .. c + 3; eight candidates in flight at a time.
 template <typename T>

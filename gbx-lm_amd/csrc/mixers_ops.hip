@@ -330,7 +330,7 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   if (renorm && threadIdx.x < top) weight[t * top + threadIdx.x] /= chosen_sum;
 }
 
-// The same by rank (E <= RANK_EXPERTS): probabilities and their order as above, no round waits for another.
+// The same by rank (choice_by_rank): probabilities and their order as above, no round waits for another.
 __global__ __launch_bounds__(NT) void route_topk_rank_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int E,
                                                             int top, int renorm) {
   __shared__ __attribute__((aligned(16))) float pl[RANK_EXPERTS];
@@ -481,7 +481,7 @@ int gbxm_route_topk(const float* logits, int32_t* idx, float* weight, int64_t T_
   if (top > NT) return fail(GBXM_ERR_UNSUPPORTED, "route_topk: top > %d", NT);
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (E <= RANK_EXPERTS) route_topk_rank_kernel<<<dim3(T_), NT, 0, s>>>(logits, idx, weight, E, top, renorm);
+  if (choice_by_rank(E, top, RANK_PER_SOFTMAX_ROUND)) route_topk_rank_kernel<<<dim3(T_), NT, 0, s>>>(logits, idx, weight, E, top, renorm);
   else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
   return after_launch("route_topk");
 }

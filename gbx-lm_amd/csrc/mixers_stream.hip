@@ -222,17 +222,17 @@ __global__ __launch_bounds__(64) void route_sigmoid_groups_kernel(const float* _
     cl[e] = c == c ? c : -INFINITY;
   }
   __syncthreads();
-  // arg-max over n values of `v` (ties: the lower index; not a number: taken); every lane gets the result
+  // arg-max over the n values of `v` above -inf (ties: the lower index), 0x7fffffff if there is none; every lane gets the result
   auto arg_max = [&](const float* v, int n) {
     float bv = -INFINITY;
     int bi = 0x7fffffff;
     for (int e = lane; e < n; e += 64)
-      if (v[e] > bv || (bi == 0x7fffffff && v[e] == v[e])) { bv = v[e]; bi = e; }          // ascending e per lane: the first of equals stays
+      if (v[e] > bv) { bv = v[e]; bi = e; }                              // ascending e per lane: the first of equals stays
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const float ov = __shfl_xor(bv, o, 64);
       const int oi = __shfl_xor(bi, o, 64);
-      if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
+      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
     }
     return bi;
   };
@@ -250,26 +250,27 @@ __global__ __launch_bounds__(64) void route_sigmoid_groups_kernel(const float* _
     for (int k = 0; k < keep_groups; ++k) {
       const int g = arg_max(gl, n_groups);
       __syncthreads();
-      if (lane == 0) gl[g] = -INFINITY;            // taken: -inf marks a kept group from here on (scores are finite)
+      if (lane == 0 && g < n_groups) gl[g] = -INFINITY;            // taken: -inf marks a kept group from here on (scores are finite)
       __syncthreads();
     }
     for (int e = lane; e < E; e += 64)
       if (gl[e / size] != -INFINITY) cl[e] = -INFINITY;
-    __syncthreads();
   }
+  for (int e = lane; e < E; e += 64) cl[e] = fmaxf(cl[e], -3.402823466e38f);      // (-inf: taken from here on)
+  __syncthreads();
   float chosen = 0.f;
   for (int k = 0; k < top; ++k) {
     const int e = arg_max(cl, E);
     __syncthreads();
     chosen += sl[e];
-    if (lane == 0) { idx[t * top + k] = e; weight[t * top + k] = sl[e]; cl[e] = NAN; }
+    if (lane == 0) { idx[t * top + k] = e; weight[t * top + k] = sl[e]; cl[e] = -INFINITY; }
     __syncthreads();
   }
   const float mul = renorm ? scale / (chosen + 1e-20f) : scale;
   for (int k = lane; k < top; k += 64) weight[t * top + k] = sl[idx[t * top + k]] * mul;
 }
 
-// The same by rank (E <= RANK_EXPERTS): scores, groups and their order as above.  A group with fewer than two experts that can be chosen scores
+// The same by rank (choice_by_rank): scores, groups and their order as above.  A group with fewer than two experts that can be chosen scores
 // -inf and is never struck out, here as there.
 __global__ __launch_bounds__(NT) void route_sigmoid_rank_kernel(const float* __restrict__ logits, const float* __restrict__ correction,
                                                                int* __restrict__ idx, float* __restrict__ weight, int E, int top, int n_groups,
@@ -400,7 +401,7 @@ int gbxm_route_sigmoid_groups(const float* logits, const float* correction, int3
   if (E > 4096) return fail(GBXM_ERR_UNSUPPORTED, "route_sigmoid_groups: more than 4096 experts");
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (E <= RANK_EXPERTS)
+  if (choice_by_rank(E, top + (n_groups > 0 ? keep_groups : 0), RANK_PER_SIGMOID_ROUND))
     route_sigmoid_rank_kernel<<<dim3(T_), min((E + 63) / 64 * 64, NT), 0, s>>>(logits, correction, idx, weight, E, top, n_groups, keep_groups, renorm, scale);
   else
     route_sigmoid_groups_kernel<<<dim3(T_), 64, (2 * E + (n_groups > 0 ? n_groups : 1)) * sizeof(float), s>>>(logits, correction, idx, weight, E, top,
