@@ -126,7 +126,10 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) 
     return y
 
 
-ROUTER_ROWS = 32          # rows up to which a router's logits are one launch on the rows as they are
+# Rows up to which a router's logits are one launch on the rows as they are -- every (row, expert) reads its router row again, so a router that the
+# XCDs' caches do not hold (8 MB) takes it for few products only.  Library with its widened copy | launch, us: 32 rows x 256 x 4096 15.0 | 10.4, x 256 x 7168
+# 21.9 | 16.8, x 1024 x 1024 10.3 | 11.2; 8 MB: 4 x 1024 x 2048 10.2 | 4.6, 8 rows 10.3 | 12.2, 32 rows 11.1 | 19.5; 32 x 1024 x 4096 15.0 | 35.8.
+ROUTER_ROWS, ROUTER_HELD, ROUTER_FEW = 32, 1 << 21, 1 << 23
 
 
 def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
@@ -140,7 +143,7 @@ def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
     if router.device != h.device:
         raise RuntimeError(f"rows on {h.device}, router on {router.device}")
     t, rows = h.shape[0], router.shape[0]
-    if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1]:
+    if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1] or (router.numel() >= ROUTER_HELD and t * router.numel() > ROUTER_FEW):
         return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
     h = h.contiguous()
     logits = torch.empty((t, rows), dtype=torch.float32, device=h.device)

@@ -115,3 +115,14 @@ def test_sigmoid_choice_of_odd_logits(e, top, groups):
             key = sorted((-v if v == v else 1.0, i) for i, v in enumerate(c[r].tolist()))
             got = [c[r, i].item() for i in idx[r].tolist()]
             assert all(a != a if v > 0 else abs(a + v) < 1e-6 for a, (v, _) in zip(got, key))
+
+
+@pytest.mark.parametrize("t,e,k", [(4, 1024, 2048), (5, 1024, 2048), (32, 1023, 2048), (32, 1024, 2048), (1, 1025, 8190), (33, 64, 100)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_logits_on_both_sides_of_the_rule(t, e, k, dt):
+    """K fp32 additions of the terms' magnitudes."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator(device=DEV).manual_seed(t + e)
+    h, router = torch.randn((t, k), device=DEV, generator=g).to(dt), torch.randn((e, k), device=DEV, generator=g)
+    want, room = h.double() @ router.double().t(), h.double().abs() @ router.double().abs().t()
+    assert bool(((M._router_logits(h, router).double() - want).abs() <= k * 2.0 ** -24 * room).all())
