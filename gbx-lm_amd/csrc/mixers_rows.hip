@@ -3,7 +3,7 @@
 // Bound by the weights' way from memory (below a few MB, by one trip to it; at 17 to 32 rows by the rows' image through the first cache).  Every
 // weight is read once, straight into the registers of the lane that feeds it to the matrix cores: lane l holds output l % 16, channels
 // 8 (l / 16) .. + 7 and the 8 that lie 32 further on, of blocks of 64 channels that the waves of a workgroup share out, so one load reads 64
-// neighbouring bytes of each output.  All of a tile's blocks (at most UNROLL a wave) are in flight before its first product, the next tile's while the
+// neighbouring bytes of each output.  All of a tile's blocks (at most four a wave) are in flight before its first product, the next tile's while the
 // waves' sums meet in LDS, and the rows' image stays in registers from tile to tile.  A row's result does not depend on the other rows of the step.
 // Measured against the library's product (us, weights cold, N x K): 1 row 1024 x 1024 5.8 -> 3.2, 2048 x 2048 11.1 -> 4.8, 2048 x 4096 14.6 -> 7.3,
 // 16384 x 2048 17.5 -> 13.6, 151936 x 2048 204 -> 112 (5.5 TB/s); 16 rows 5120 x 2048 12.2 -> 8.0; 32 rows 2048 x 2048 11.2 -> 7.6.
@@ -12,10 +12,10 @@
 namespace gbxm {
 namespace {
 
-constexpr int BK = 64, UNROLL = 4;
+constexpr int BK = 64;
 
-// Workgroups walk over tiles of 16 outputs (grid <= their number).  MT: tiles of 16 rows.  K <= BK UNROLL WAVES.
-template <int MT, int WAVES>
+// Workgroups walk over tiles of 16 outputs (grid <= their number).  MT: tiles of 16 rows.  UNROLL: blocks a wave at most, K <= BK UNROLL WAVES.
+template <int MT, int WAVES, int UNROLL>
 __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(const bf16_t* __restrict__ x, int64_t x_stride, const bf16_t* __restrict__ w,
                                                                 const bf16_t* __restrict__ bias, bf16_t* __restrict__ y, int64_t y_stride, int T, int N,
                                                                 int K) {
@@ -72,14 +72,16 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_kernel(const bf16_t* _
   }
 }
 
-// Waves: as many as give each of them at most UNROLL blocks of K; workgroups: what the chip holds at a time (8 waves a CU measured best, the 16-wave
-// form needs 16), so that long outputs stream.
-template <int WAVES>
+// Waves: as many as give each of them at most four blocks of K; workgroups: what the chip holds at a time (8 waves a CU measured best, the 16-wave
+// form needs 16), so that long outputs stream.  A form holds as many blocks a wave as there are (with four for all of them the missing ones were the
+// last one's again, requests that nothing hides in long outputs; library | four | as many as there are, us: 1 row of 151936 x 64 12.2 | 19.9 | 9.1, 50304 x 2560
+// 48.6 | 53.5 | 45.3, 16 rows of it 49.4 | 57.1 | 51.3, 32 rows of 50304 x 1152 24.8 | 38.6 | 32.0).
+template <int WAVES, int UNROLL>
 void launch_rows(hipStream_t s, const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int64_t y_stride, int T, int N, int K) {
   const int grid = min((N + 15) / 16, 256 * (WAVES < 8 ? 8 / WAVES : 1));
-#define GBXM_ROWS(MT)                                                                                                                               \
-  linear_rows_kernel<MT, WAVES><<<grid, 64 * WAVES, 0, s>>>(static_cast<const bf16_t*>(x), x_stride, static_cast<const bf16_t*>(w),                   \
-                                                            static_cast<const bf16_t*>(bias), static_cast<bf16_t*>(y), y_stride, T, N, K)
+#define GBXM_ROWS(MT)                                                                                                                                \
+  linear_rows_kernel<MT, WAVES, UNROLL><<<grid, 64 * WAVES, 0, s>>>(static_cast<const bf16_t*>(x), x_stride, static_cast<const bf16_t*>(w),           \
+                                                                    static_cast<const bf16_t*>(bias), static_cast<bf16_t*>(y), y_stride, T, N, K)
   if constexpr (WAVES <= 8) {
     if (T > 16) { GBXM_ROWS(2); return; }
   }
@@ -101,9 +103,17 @@ extern "C" int gbxm_linear_rows(const void* x, int64_t x_stride, const void* w, 
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int T = static_cast<int>(T_);
-  if (K <= 512) launch_rows<2>(s, x, x_stride, w, bias, y, y_stride, T, N, K);
-  else if (K <= 1024) launch_rows<4>(s, x, x_stride, w, bias, y, y_stride, T, N, K);
-  else if (K <= 2048) launch_rows<8>(s, x, x_stride, w, bias, y, y_stride, T, N, K);
-  else launch_rows<16>(s, x, x_stride, w, bias, y, y_stride, T, N, K);
+#define GBXM_FORM(WAVES, UNROLL) if (K <= BK * WAVES * UNROLL) launch_rows<WAVES, UNROLL>(s, x, x_stride, w, bias, y, y_stride, T, N, K)
+  GBXM_FORM(2, 1);
+  else GBXM_FORM(2, 2);
+  else GBXM_FORM(2, 3);
+  else GBXM_FORM(2, 4);
+  else GBXM_FORM(4, 3);
+  else GBXM_FORM(4, 4);
+  else GBXM_FORM(8, 3);
+  else GBXM_FORM(8, 4);
+  else GBXM_FORM(16, 3);
+  else GBXM_FORM(16, 4);
+#undef GBXM_FORM
   return after_launch("linear_rows");
 }

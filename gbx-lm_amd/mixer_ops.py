@@ -108,13 +108,20 @@ def stream_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, act_dtype: torc
     return out
 
 
+def rows_win(t: int, n: int, k: int) -> bool:
+    """Where ``linear_rows`` is the faster product (library | launch, us: 16 rows of 4096 x 4096 15.8 | 10.6, 32 of 4096 x 2048 10.8 | 8.0; longer contractions
+    are the library's, 2048 x 8192: 12.6 both).  Above 16 rows a tile's fixed part shows in long outputs of contractions that fill no whole form: 32 rows of
+    50304 x 1152 24.8 | 32.0, x 1792 35.5 | 44.0, 151936 x 1792 114.6 | 122.5, but x 1024 22.4 | 23.4, x 2048 53.8 | 44.8 and 16384 x 1536 18.5 | 14.3."""
+    return k <= 4096 if t <= 16 else t <= 32 and k <= 2048 and (k <= 1024 or k == 2048 or n < 32768)
+
+
 def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """``x @ w.T (+ bias)`` of few bf16 rows [T, K] as one launch, or None for what the kernel does not take (it wins over the vendor library's
-    product up to 16 rows of 4096 channels and 32 of 2048: csrc/mixers_rows.hip; longer contractions are the library's, 2048 x 8192: 12.6 us both)."""
+    """``x @ w.T (+ bias)`` of few bf16 rows [T, K] as one launch, or None for what the kernel does not take or the vendor library is
+    faster at (``rows_win``)."""
     if x.dim() != 2 or w.dim() != 2:
         return None
     (t, k), n, stride = x.shape, w.shape[0], x.stride(0)
-    if (t > 32 or k % 64 or k > (2048 if t > 16 else 4096) or not (t and k and 0 < n <= 1 << 26) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
+    if (not rows_win(t, n, k) or k % 64 or not (t and k and 0 < n <= 1 << 26) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
             or x.stride(1) != 1 or stride % 8 or stride < k or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16 or w.shape[1] != k
             or w.device != x.device):
         return None

@@ -12,7 +12,8 @@ from .. import mixer_ops as M
 
 
 def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    if isinstance(x, torch.Tensor) and x.is_cuda and 0 < x.numel() <= 32 * x.shape[-1] and M.outside_torch(x, w, bias):
+    if isinstance(x, torch.Tensor) and x.is_cuda and 0 < x.numel() <= 32 * x.shape[-1] and M.rows_win(x.numel() // x.shape[-1], w.shape[0], x.shape[-1]) \
+            and M.outside_torch(x, w, bias):
         y = M.linear_rows(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]), w, bias)
         if y is not None:
             return y if x.dim() == 2 else y.view(*x.shape[:-1], w.shape[0])

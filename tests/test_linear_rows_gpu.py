@@ -79,3 +79,26 @@ def test_what_torch_does_around_a_product_stays():
         assert torch.equal(compiled(x), F.linear(x, w, b) * 2)
         assert torch.equal(project(x[:, :0], w[:, :0], b), F.linear(x[:, :0], w[:, :0], b))
         assert not torch.equal(project(x, w, b), torch.zeros_like(project(x, w, b))) and torch.equal(project(x, w, b), M.linear_rows(x, w, b))
+
+
+@pytest.mark.parametrize("t,n,k,taken", [(16, 40000, 4096, True), (17, 32768, 1088, False), (17, 32767, 1088, True), (32, 32768, 1984, False), (32, 40000, 2048, True),
+                                         (32, 40000, 1024, True), (32, 16, 2112, False), (33, 16, 64, False)])
+def test_the_rule(t, n, k, taken):
+    from gbx_lm_amd import mixer_ops as M
+    x, w, _ = case(t, n, k, False, 0, t)
+    y = M.linear_rows(x, w, None)
+    assert (y is not None) == taken == M.rows_win(t, n, k)
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 704, 768, 832, 1472, 1536, 1600, 2944, 3072, 3136])
+@pytest.mark.parametrize("t", [1, 32])
+def test_blocks_of_every_form(t, k):
+    """The last contraction of each number of blocks a wave, and those beside it."""
+    from gbx_lm_amd import mixer_ops as M
+    x, w, b = case(t, 300, k, True, 0, k)
+    y = M.linear_rows(x, w, b)
+    if y is None:
+        assert t > 16 and k > 2048
+        return
+    want, room = x.double() @ w.double().t() + b.double(), x.double().abs() @ w.double().abs().t() + b.double().abs()
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + (k + 1) * 2.0 ** -24 * room).all())
