@@ -412,9 +412,9 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
 
     x: [..., 1, 1, K] or [..., k, 1, K]; rhs_indices: [..., k] -> [..., k, 1, N].  Few (token, slot) pairs run the
     expert-indexed decode GEMV in ONE launch; many pairs are bucketed by expert on the device and run as tiles of the matrix cores
-    (``_packed_experts``); what neither takes is grouped on the host (one batched GEMM per expert present).  The reference's
+    (``_packed_experts``); what neither takes, and thousands of pairs per large expert, is grouped on the host (one batched GEMM per expert present).  The reference's
     ``sorted_indices`` hint needs no special handling.  An index that names no expert is not looked for on the host, which would have to wait for the
-    device: among many pairs its row is NaN, among few the nearest expert's."""
+    device: among many pairs its row is NaN, among few the nearest expert's (among so many that the host groups them, it raises)."""
     if not transpose:
         raise NotImplementedError("gather_quantized_matmul supports transpose=True only (the reference's only use)")
     for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases"), (rhs_indices, "rhs_indices")):
@@ -470,12 +470,19 @@ def gather_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tens
     return y.reshape(*lead, k, 1, N)
 
 
+# Multiply-adds per expert from which one expert at a time is the faster way: its dense GEMM on dequantised weights makes up for the host's grouping and a
+# dozen launches (some 110 us an expert), which the packed tiles' vector work per group does not allow.  One at a time | packed, us, 8 experts: 4 bits, group 128,
+# 4096 x 14336, 1000 pairs each 2543 | 1904, 2000 2656 | 3363; 3 bits, group 64, 14336 x 4096, 500 1489 | 1349, 1000 2110 | 2576, 4096 x 4096, 2000 1418 | 1191,
+# 3000 1584 | 1768; 4 bits, group 32, 4096 x 4096, 1500 1771 | 1251, 2000 1429 | 1639.
+_EXPERT_WORK = {128: 85_000_000_000, 64: 50_000_000_000, 32: 30_000_000_000}
+
+
 def _packed_experts(xr: torch.Tensor, first, second, bias, idx: torch.Tensor, x_div: int, E: int, N: int, K: int, bits: int, group_size: int):
     """Rows [pairs, N] of the chosen experts' products over many (token, slot) pairs (gbxm_packed_experts): ``first`` = (qweight, scales,
     zeros) [E, ...]; with ``second`` alike, silu(first) * second.  None where the launch does not serve the operands (the caller's other path
     takes or refuses them)."""
     pairs = idx.numel()
-    if xr.dtype not in _ACT16 or not idx.is_cuda or idx.dtype not in (torch.int32, torch.int64) or xr.shape[0] * x_div != pairs or K % 128 or bits not in (2, 3, 4):
+    if group_size not in _EXPERT_WORK or xr.dtype not in _ACT16 or not idx.is_cuda or idx.dtype not in (torch.int32, torch.int64) or xr.shape[0] * x_div != pairs or K % 128 or bits not in (2, 3, 4):
         return None
     words, groups = (E, N, K * bits // 32), (E, N, K // group_size)
     for q, s, z in (first, second or first):
@@ -487,6 +494,8 @@ def _packed_experts(xr: torch.Tensor, first, second, bias, idx: torch.Tensor, x_
         if not bias.is_cuda or bias.dtype != xr.dtype or bias.shape != (E, N):
             return None
         bias = bias.contiguous()
+    if pairs * N * K >= E * _EXPERT_WORK[group_size] and not torch.cuda.is_current_stream_capturing():      # (the host cannot group inside a capture)
+        return None
     L = _lib.mixers()
     nbytes = L.gbxm_packed_experts_workspace(pairs, K, E)
     if not nbytes:

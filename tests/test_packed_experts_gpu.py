@@ -174,3 +174,28 @@ def test_rows_in_32_bits_are_refused(oracle):
     assert ops.gather_swiglu(x, mods[0], mods[1], idx) is None
     with pytest.raises(ValueError):
         mods[0](x, idx)
+
+
+@pytest.mark.parametrize("bits,g", [(3, 32), (2, 64), (4, 128)])
+def test_thousands_of_pairs_per_expert_go_one_expert_at_a_time(oracle, monkeypatch, bits, g):
+    """Both sides of the rule, and a capture beyond it.  Tolerance: every weight rounded (2^-8 of it) on the way of the general path, fp32 sums, one rounding."""
+    from gbx_lm_amd import graphs, ops
+    E, N, K = 2, 136, 256
+    qw, s, z, w, mag = make(oracle, E, N, K, bits, g, torch.bfloat16, 5)
+    P = 3000
+    x, idx = torch.randn((P, 1, 1, K), device=DEV).to(torch.bfloat16), torch.randint(0, E, (P, 1), device=DEV)
+    want, calls, real = rows(x.view(P, K).double(), w, idx.view(-1)), [], ops.quantized_matmul
+    room = 2.0 ** -7 * want.abs() + 4 * 2.0 ** -8 * rows(x.view(P, K).double() ** 2, w ** 2, idx.view(-1)).sqrt() + K * 2.0 ** -24 * rows(x.view(P, K).double().abs(), mag, idx.view(-1))
+    monkeypatch.setattr(ops, "quantized_matmul", lambda *a, **k: calls.append(1) or real(*a, **k))
+    run = lambda: ops.gather_quantized_matmul(x, qw, s, z, idx, group_size=g, bits=bits).view(P, N)
+    for line, n in ((P * N * K // E + 1, 0), (P * N * K // E, E)):
+        monkeypatch.setitem(ops._EXPERT_WORK, g, line)
+        del calls[:]
+        assert bool(((run().double() - want).abs() <= room).all()) and len(calls) == n
+    del calls[:]
+    graph = torch.cuda.CUDAGraph()
+    with graphs.capture(graph):
+        y = run()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert not calls and bool(((y.double() - want).abs() <= room).all())
