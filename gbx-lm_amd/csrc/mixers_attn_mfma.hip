@@ -42,10 +42,11 @@ template <int DK, int DV> struct WindowShape {
   static constexpr int BYTES = KT * (KROW + VROW) + 1024;   // one group's key and value tile, and its 256 exponents by distance
   static constexpr int JOIN = GROUPS > 1 ? 4 * (DV / 32) * 16 * 64 * 4 : 0;
   static constexpr int LDS = GROUPS * BYTES > JOIN ? GROUPS * BYTES : JOIN;
+  static constexpr int WAVES = DK + DV <= 320 ? 2 : 1;      // per SIMD: left to itself <192, 128> takes the registers of both
 };
 
 template <int DK, int DV>
-__global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS)) void window_tile_kernel(const TileArgs a) {
+__global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS), (WindowShape<DK, DV>::WAVES)) void window_tile_kernel(const TileArgs a) {
   typedef WindowShape<DK, DV> Shape;
   constexpr int KT = Shape::KT, KROW = Shape::KROW, VROW = Shape::VROW, GROUPS = Shape::GROUPS, STEP = GROUPS * KT;
   constexpr int KS = DK / 16, DT = DV / 32;
