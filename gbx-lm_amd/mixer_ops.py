@@ -13,18 +13,9 @@ import torch
 from torch.autograd import forward_ad
 
 from . import _lib
+from .ops import _stream_ptr as _stream
 
 _DT = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32}
-
-
-def _stream(device) -> int:
-    """The raw handle of the device's current stream; other devices than the GPU raise, as in ``torch.cuda.current_stream``."""
-    if type(device) is not torch.device:
-        device = torch.device(device)
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def outside_torch(*tensors: Optional[torch.Tensor]) -> bool:

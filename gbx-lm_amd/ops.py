@@ -18,15 +18,19 @@ _DT = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16, torch.float32
 _ACT16 = {torch.float16: _lib.GBX_F16, torch.bfloat16: _lib.GBX_BF16}              # what activations of a product may be
 
 
+_GPUS = {torch.device("cuda", i): i for i in range(64)}          # (one look-up instead of asking a device for its type, which costs 0.24 us)
+
+
 def _stream_ptr(device) -> int:
     """hipStream_t of the device's current stream (the raw handle: building a Stream object around it costs 2 us a launch).  Other devices than the GPU
     raise, as in ``torch.cuda.current_stream``: a launch must not see a host tensor's address."""
-    if type(device) is not torch.device:
+    index = _GPUS.get(device)
+    if index is None:
         device = torch.device(device)
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _require_cuda(t: torch.Tensor, name: str) -> None:
