@@ -1,7 +1,7 @@
 // Matrix-core kernel of gated sliding-window attention for bf16 prompt portions (mechanism: mixers_attn.hip).
 //
-// One workgroup = one tile of up to 128 query rows of one (sequence, head), a wave owns 32 of them; two groups of four waves take every other
-// key tile.  Key / value tiles of 64 positions go global -> registers (one tile ahead) -> LDS once per group (ring rows for positions before the step, projection rows inside it; rows
+// One workgroup = one tile of up to 128 query rows of one (sequence, head), a wave owns 32 of them; one group of four waves, or two that take every
+// other key tile.  Key / value tiles of 32 (two groups: 64) positions go global -> registers (one tile ahead) -> LDS once per group (ring rows for positions before the step, projection rows inside it; rows
 // past the tile's last query are zero-filled so that a zero gate never meets a stale NaN).  Both products are computed swapped so
 // that a lane owns ONE query and the gate arithmetic is lane-local:
 //   S^T[key, q] = mfma(K rows, Q rows)      lane (q = lane % 32) holds 16 keys of the tile, the other 16 are in lane ^ 32
@@ -10,8 +10,7 @@
 // No softmax: gates of different keys are independent, O^T just accumulates -- no running maximum, no rescale, no final division.
 // The fp32 part per score (four transcendentals, see `exponent`) costs more than the products: the kernel is bound by vector
 // instructions, and by the tiles that start last -- late tiles of all heads come first.  Gates are rounded to bf16 for the value product.
-// Measured, 32 / 4 heads of 128: prompts of 2 047 + 1 100 + 333 + 1 tokens 339 -> 141 us; one of 4 000 tokens 343 (4 096 before: 1 105); 16 heads of 64, 900
-// tokens, one group of waves per tile 43, two 30.
+// Measured against five transcendentals a score and one group for all: see `launch`.
 #include "mixers_mfma.h"
 
 namespace gbxm {
@@ -33,10 +32,9 @@ struct TileArgs {
 };
 
 // Two groups of four waves take every other key tile of the same queries (their sums meet in LDS at the end): a tile late in a long prompt
-// is a chain of key tiles that the rest of the launch would otherwise wait for.  Heads too large for two waves per SIMD keep one group.
-template <int DK, int DV> struct WindowShape {
-  static constexpr int GROUPS = DK + DV > 256 ? 1 : 2;
-  static constexpr int KT = DK + DV > 256 ? 32 : 64;        // keys per tile (larger heads: 64 would cost the second wave per SIMD)
+// is a chain of key tiles that the rest of the launch would otherwise wait for.  `launch` chooses.
+template <int DK, int DV, int GROUPS_, int KT_> struct WindowShape {
+  static constexpr int GROUPS = GROUPS_, KT = KT_;          // KT: keys per tile
   static constexpr int KROW = DK * 2 + 16;                  // +16 B: conflict-free 16-byte fragment reads
   static constexpr int VROW = DV * 2 + 64;                  // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
   static constexpr int BYTES = KT * (KROW + VROW) + 1024;   // one group's key and value tile, and its 256 exponents by distance
@@ -45,10 +43,10 @@ template <int DK, int DV> struct WindowShape {
   static constexpr int WAVES = DK + DV <= 320 ? 2 : 1;      // per SIMD: left to itself <192, 128> takes the registers of both
 };
 
-template <int DK, int DV>
-__global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS), (WindowShape<DK, DV>::WAVES)) void window_tile_kernel(const TileArgs a) {
-  typedef WindowShape<DK, DV> Shape;
-  constexpr int KT = Shape::KT, KROW = Shape::KROW, VROW = Shape::VROW, GROUPS = Shape::GROUPS, STEP = GROUPS * KT;
+template <int DK, int DV, int GROUPS, int KT>
+__global__ __launch_bounds__((256 * GROUPS), (WindowShape<DK, DV, GROUPS, KT>::WAVES)) void window_tile_kernel(const TileArgs a) {
+  typedef WindowShape<DK, DV, GROUPS, KT> Shape;
+  constexpr int KROW = Shape::KROW, VROW = Shape::VROW, STEP = GROUPS * KT;
   constexpr int KS = DK / 16, DT = DV / 32;
   extern __shared__ __attribute__((aligned(16))) unsigned char all_lds[];
   const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
@@ -225,17 +223,32 @@ __global__ __launch_bounds__((256 * WindowShape<DK, DV>::GROUPS), (WindowShape<D
   }
 }
 
-template <int DK, int DV>
-int launch(const TileArgs& t, int n_tiles, int H, hipStream_t s) {
-  typedef WindowShape<DK, DV> Shape;
+template <int DK, int DV, int GROUPS, int KT>
+int launch_shape(const TileArgs& t, int n_tiles, hipStream_t s) {
+  constexpr int bytes = WindowShape<DK, DV, GROUPS, KT>::LDS;
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_tile_kernel<DK, DV>), hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_tile_kernel<DK, DV, GROUPS, KT>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hip_fail(e, "window_attention (tiles)");
     once.done();
   }
-  window_tile_kernel<DK, DV><<<static_cast<unsigned>(H) * n_tiles, 256 * Shape::GROUPS, Shape::LDS, s>>>(t);
+  window_tile_kernel<DK, DV, GROUPS, KT><<<static_cast<unsigned>(t.H) * n_tiles, 256 * GROUPS, bytes, s>>>(t);
   return after_launch("window_attention (tiles)");
+}
+
+// Two groups of waves a tile, 64 keys each, while every CU then has at most one tile (a CU holds one such workgroup and two of one group), and for some more
+// tiles where they are long: they shorten the chain of key tiles behind the last queries.  Otherwise one group and 32 keys.  One | two, us, tiles x heads:
+//   32 heads of 128: 256, 1 000 rows 65 | 40; 352, 1 300 rows 82 | 49; 576, 2 200 rows 137 | 109; 1 024: 4 000 rows 256 | 295, with a window of 64 41 | 59,
+//   64 rows x 32 18 | 32; 2 048, 20 rows x 64 13 | 40 (five transcendentals, one group before both: 86, 129, 248, 783, 51, 21, 19);
+//   16 heads of 64: 384, 3 000 rows with a window of 1 024 60 | 60, without 144 | 80; 512: 2 000 rows x 2 109 | 68, 500 rows x 8 33 | 35, 64 rows x 32 7 | 11.
+// The line: tiles x heads up to 3 / 8 of the keys that a row can see, and up to 768.
+template <int DK, int DV>
+int launch(const TileArgs& t, int n_tiles, int longest, hipStream_t s) {
+  if constexpr (DK + DV <= 256) {                            // (larger heads: 64 keys or a second group would cost the second wave per SIMD)
+    const int64_t n = static_cast<int64_t>(t.H) * n_tiles, keys = longest > 0 && longest < t.window ? longest : t.window;
+    if (n <= 256 || (n <= 768 && 8 * n <= 3 * keys)) return launch_shape<DK, DV, 2, 64>(t, n_tiles, s);
+  }
+  return launch_shape<DK, DV, 1, 32>(t, n_tiles, s);
 }
 
 }  // namespace
@@ -255,7 +268,7 @@ int launch_window_tiles(const gbxm_window_attn_args& a, hipStream_t s) {
   TileArgs t{static_cast<const bf16_t*>(a.qkv), static_cast<const bf16_t*>(a.kcache), static_cast<const bf16_t*>(a.vcache), a.seq, a.tiles,
              static_cast<bf16_t*>(a.out), a.dist_mul, a.dist_rate, a.gate_bias, a.row_stride, a.q_tile, a.H, a.G, a.window, a.H * a.dk,
              a.G * a.dk, a.scale, a.softcap};
-#define GBXM_TILE(DK_, DV_) if (a.dk == DK_ && a.dv == DV_) return launch<DK_, DV_>(t, a.n_tiles, a.H, s)
+#define GBXM_TILE(DK_, DV_) if (a.dk == DK_ && a.dv == DV_) return launch<DK_, DV_>(t, a.n_tiles, a.longest, s)
   GBXM_TILE(64, 64); GBXM_TILE(96, 64); GBXM_TILE(128, 64); GBXM_TILE(64, 128); GBXM_TILE(128, 128); GBXM_TILE(192, 128); GBXM_TILE(256, 256);
   GBXM_TILE(96, 96); GBXM_TILE(64, 32); GBXM_TILE(32, 32); GBXM_TILE(32, 64);
 #undef GBXM_TILE

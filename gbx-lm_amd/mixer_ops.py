@@ -233,7 +233,8 @@ def window_attention(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
                             _f32(m.dist_mul, "dist_mul").data_ptr(), _f32(m.dist_rate, "dist_rate").data_ptr(),
                             _f32(m.gate_bias, "gate_bias").data_ptr(), batch.total, len(batch.slot),
                             0 if batch.tiles is None else batch.tiles.shape[0], batch.q_tile, m.heads, m.kv_heads, m.dim, m.vdim, m.window,
-                            m.scale, m.softcap, int(batch.decode_only), act, None if partial is None else partial.data_ptr(), splits)
+                            m.scale, m.softcap, int(batch.decode_only), act, None if partial is None else partial.data_ptr(), splits,
+                            max(p + n for p, n in zip(batch.pos0, batch.n_new)))
     _lib.check_mixers(_lib.mixers().gbxm_window_attention(ctypes.byref(a), _stream(qkv.device)))
     return out
 

@@ -16,12 +16,22 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("cap", [0.0, 5.0])
 @pytest.mark.parametrize("window", [1, 63, 64, 65, 129, 300])
 def test_portions(dk, dv, cap, window):
+    portions([1, 31, 33, 64, 65, 127, 129, 191, 257, 320], [0, 7, 0, 64, 200, 0, 33, 0, 130, 0], dk, dv, cap, window)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (32, 64)])
+@pytest.mark.parametrize("cap,window", [(0.0, 33), (5.0, 300)])
+def test_more_tiles_than_compute_units(dk, dv, cap, window):
+    """One group of waves a tile, tiles of 32 keys: edges of both, beside prompts of a few rows with and without history."""
+    portions([1, 31, 32, 33, 63, 65, 129, 257] + [1 + (11 * i) % 40 for i in range(60)], [0, 7, 33, 0, 64, 300, 31, 0] + [(5 * i) % 47 for i in range(60)],
+             dk, dv, cap, window)
+
+
+def portions(n_new, pos0, dk, dv, cap, window):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
     gen = torch.Generator(device=DEV).manual_seed(window + dk)
     H, G = 4, 2
-    n_new = [1, 31, 33, 64, 65, 127, 129, 191, 257, 320]
-    pos0 = [0, 7, 0, 64, 200, 0, 33, 0, 130, 0]
     T = sum(n_new)
     batch = StepBatch.build(list(range(len(n_new))), pos0, n_new, DEV)
     qkv = torch.randn((T, H * dk + G * (dk + dv)), device=DEV, generator=gen).to(torch.bfloat16)
