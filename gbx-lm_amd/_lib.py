@@ -329,7 +329,8 @@ class SinkAttnArgs(ctypes.Structure):
                 ("H", ctypes.c_int32), ("G", ctypes.c_int32), ("dk", ctypes.c_int32), ("dv", ctypes.c_int32),
                 ("window", ctypes.c_int32), ("keep", ctypes.c_int32), ("ring", ctypes.c_int32), ("scale", ctypes.c_float),
                 ("decode_only", ctypes.c_int32), ("act", ctypes.c_int32), ("partial", ctypes.c_void_p), ("partial_splits", ctypes.c_int32),
-                ("chunk", ctypes.c_int32), ("head_scale", ctypes.c_void_p), ("out_row", ctypes.c_int64), ("gate_channels", ctypes.c_int32)]
+                ("chunk", ctypes.c_int32), ("head_scale", ctypes.c_void_p), ("out_row", ctypes.c_int64), ("gate_channels", ctypes.c_int32),
+                ("longest", ctypes.c_int32)]
 
 
 class HeadProjectArgs(ctypes.Structure):

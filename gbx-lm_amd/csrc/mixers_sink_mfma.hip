@@ -1,7 +1,7 @@
 // Matrix-core kernel of softmax attention with a sink for bf16 prompt portions (mechanism and key order: mixers_sink.hip).
 //
 // One workgroup = tiles of up to 128 query rows of one (sequence, head); a wave owns 32 queries, and one or two groups of four waves share a
-// tile's keys (SinkShape).  Key / value tiles of 64 (large heads: 32) visible positions go global -> registers (one tile ahead) -> LDS once per
+// tile's keys (SinkShape).  Key / value tiles of 64 (large heads and short sequences: 32) visible positions go global -> registers (one tile ahead) -> LDS once per
 // group.  Both products are computed swapped,
 //   S^T[key, q] = mfma(K rows, Q rows),    O^T[d, q] += mfma(V^T rows, P^T),
 // so that a lane owns ONE query: lane (q = lane % 32, half = lane / 32) holds 16 of the tile's 32 scores of its query, the other 16
@@ -59,9 +59,8 @@ __device__ __forceinline__ u32x2 out4(const SinkTileArgs& a, int64_t row, int he
 
 // With two GROUPS of four waves each takes every other key tile of the same queries, with a maximum and denominator of its own; the halves
 // meet in LDS at the end.
-template <int DK, int DV, int GROUPS_> struct SinkShape {
-  static constexpr int GROUPS = GROUPS_;
-  static constexpr int KT = DK + DV > 256 ? 32 : 64;         // keys per tile (larger heads: 64 would cost the second wave per SIMD)
+template <int DK, int DV, int GROUPS_, int KT_> struct SinkShape {
+  static constexpr int GROUPS = GROUPS_, KT = KT_;           // KT: keys per tile
   static constexpr int KROW = DK * 2 + 16;                   // +16 B: conflict-free 16-byte fragment reads
   static constexpr int VROW = DV * 2 + 64;                   // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
   static constexpr int BYTES = KT * (KROW + VROW);
@@ -70,10 +69,10 @@ template <int DK, int DV, int GROUPS_> struct SinkShape {
   static constexpr int WAVES = DK + DV <= 320 ? 2 : 1;       // per SIMD
 };
 
-template <int DK, int DV, int GROUPS_>
+template <int DK, int DV, int GROUPS, int KT>
 __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile, const int head, unsigned char* all_lds) {
-  typedef SinkShape<DK, DV, GROUPS_> Shape;
-  constexpr int KT = Shape::KT, KROW = Shape::KROW, VROW = Shape::VROW, GROUPS = Shape::GROUPS, STEP = GROUPS * KT, NH = KT / 32;
+  typedef SinkShape<DK, DV, GROUPS, KT> Shape;
+  constexpr int KROW = Shape::KROW, VROW = Shape::VROW, STEP = GROUPS * KT, NH = KT / 32;
   constexpr int KS = DK / 16, DT = DV / 32;
   const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   unsigned char* kl = all_lds + group * Shape::BYTES;
@@ -487,43 +486,51 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
 }
 
 // One group: a workgroup takes two query tiles, one from each end of the step's list -- in a long causal prompt a late tile (many keys) and an
-// early one (few) -- so that workgroups carry about the same work however they are spread over the chip.  Two groups: a tile each, of all
-// heads the late ones first.
-template <int DK, int DV, int GROUPS>
-__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
+// early one (few) -- so that workgroups carry about the same work however they are spread over the chip; or (not `paired`) one.  Two groups: a
+// tile each, of all heads the late ones first.
+template <int DK, int DV, int GROUPS, int KT>
+__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles, const bool paired) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   if constexpr (GROUPS == 1) {
-    const int pairs = (n_tiles + 1) / 2, second = blockIdx.x % pairs, first = n_tiles - 1 - second, head = blockIdx.x / pairs;
-    sink_tile<DK, DV, 1>(a, first, head, lds);
-    if (second != first) sink_tile<DK, DV, 1>(a, second, head, lds);
+    const int per_head = paired ? (n_tiles + 1) / 2 : n_tiles, second = blockIdx.x % per_head, first = paired ? n_tiles - 1 - second : second;
+    const int head = blockIdx.x / per_head;
+    sink_tile<DK, DV, 1, KT>(a, first, head, lds);
+    if (second != first) sink_tile<DK, DV, 1, KT>(a, second, head, lds);
   } else {
-    sink_tile<DK, DV, 2>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
+    sink_tile<DK, DV, 2, KT>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
   }
 }
 
-template <int DK, int DV, int GROUPS>
-int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
-  const unsigned grid = static_cast<unsigned>(t.H) * (GROUPS == 1 ? (n_tiles + 1) / 2 : n_tiles);
-  constexpr int bytes = SinkShape<DK, DV, GROUPS>::LDS;
+template <int DK, int DV, int GROUPS, int KT>
+int launch_groups(const SinkTileArgs& t, int n_tiles, bool paired, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(t.H) * (paired ? (n_tiles + 1) / 2 : n_tiles);
+  constexpr int bytes = SinkShape<DK, DV, GROUPS, KT>::LDS;
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hip_fail(e, "sink_attention (tiles)");
     once.done();
   }
-  sink_tile_kernel<DK, DV, GROUPS><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles);
+  sink_tile_kernel<DK, DV, GROUPS, KT><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles, paired);
   return after_launch("sink_attention (tiles)");
 }
 
 // Tiles times heads up to which two groups share a tile.  Measured, one group against two, us, 16 heads: 12 + 6 + 1 tiles of <128, 128> 112 | 44; one prompt of
 // 32 tiles <192, 128> 282 | 187; 47 tiles 434 | 390; three of 20 334 | 250; 64 tiles 658 | 680, <128, 128> 469 | 466, <64, 64> 286 | 305.
+// Sequences of a tile's keys and less have no chain to share and nothing to balance: one group, 32 keys, a tile per workgroup.  The form that the line above gives |
+// this, us: 16 heads of <128, 128>, 20 rows 8.1 | 6.3, 20 rows x 16 8.4 | 6.5, x 64 14.6 | 11.9, 64 rows x 32 17.0 | 10.5 (32 heads: 18.6 | 19.9); <64, 128>, 100 rows x 200
+// 86 | 66; <96, 96> 86 | 68, but 128 rows x 64 30 | 32.5 and <128, 128>, 100 rows x 200 98 | 102.
 constexpr unsigned TWO_GROUPS = 960;
 template <int DK, int DV>
-int launch(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
+int launch(const SinkTileArgs& t, int n_tiles, int longest, hipStream_t s) {
+  constexpr int KT = DK + DV > 256 ? 32 : 64;                // (larger heads: 64 would cost the second wave per SIMD)
+  const int64_t n = static_cast<int64_t>(t.H) * n_tiles;
+  if (longest > 0 && (longest <= (n <= TWO_GROUPS ? 64 : 48) || (DK + DV < 256 && longest <= 128 && n > 1536)))
+    return launch_groups<DK, DV, 1, 32>(t, n_tiles, false, s);
   if constexpr (DK + DV <= 320) {
-    if (static_cast<unsigned>(t.H) * n_tiles <= TWO_GROUPS) return launch_groups<DK, DV, 2>(t, n_tiles, s);
+    if (n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT>(t, n_tiles, false, s);
   }
-  return launch_groups<DK, DV, 1>(t, n_tiles, s);
+  return launch_groups<DK, DV, 1, KT>(t, n_tiles, true, s);
 }
 
 constexpr int CAPS[][2] = {{32, 32}, {64, 64}, {64, 128}, {96, 96}, {128, 128}, {192, 128}, {256, 256}};
@@ -559,7 +566,7 @@ static SinkTileArgs tile_args(const gbxm_sink_attn_args& a) {
 int launch_sink_tiles(const gbxm_sink_attn_args& a, hipStream_t s) {
   if (!sink_tiles_shape(a.dk, a.dv) || a.q_tile != 128 || static_cast<int64_t>(a.H) * a.n_tiles > 0x7fffffff || !tile_operands(a)) return GBXM_ERR_UNSUPPORTED;
   const SinkTileArgs t = tile_args(a);
-#define GBXM_TILE(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch<DK_, DV_>(t, a.n_tiles, s)
+#define GBXM_TILE(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch<DK_, DV_>(t, a.n_tiles, a.longest, s)
   GBXM_TILE(32, 32); GBXM_TILE(64, 64); GBXM_TILE(64, 128); GBXM_TILE(96, 96); GBXM_TILE(128, 128); GBXM_TILE(192, 128); GBXM_TILE(256, 256);
 #undef GBXM_TILE
   return GBXM_ERR_UNSUPPORTED;

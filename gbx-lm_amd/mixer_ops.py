@@ -399,7 +399,7 @@ def sink_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, ca
     a.T, a.B, a.n_tiles, a.q_tile = t, len(batch.slot), 0 if batch.tiles is None else batch.tiles.shape[0], batch.q_tile
     a.H, a.G, a.dk, a.dv = heads, groups, dk, dv
     a.window, a.scale = (0 if window is None else int(window)), float(scale)
-    a.decode_only, a.act = int(batch.decode_only), act
+    a.decode_only, a.act, a.longest = int(batch.decode_only), act, longest
     partial = None
     if t * groups < 256 and t <= 64:                            # few rows: room for key-split partial sums
         # keys of the longest row; launches that are being captured are replayed for longer sequences: size for the table then

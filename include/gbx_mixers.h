@@ -156,6 +156,7 @@ typedef struct {
   const float* head_scale;      /* [H], or null */
   int64_t out_row;              /* elements between output rows (0: H*dv) */
   int32_t gate_channels;        /* the gate is a number per channel of the concatenated heads */
+  int32_t longest;              /* positions of the step's longest sequence, its new ones included; 0: unknown.  Chooses among forms of the prompt kernel */
 } gbxm_sink_attn_args;
 int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream);
 int gbxm_sink_attention_tiled(int32_t dk, int32_t dv, int32_t act, int32_t decode_only);

@@ -16,11 +16,24 @@ MANY = [1 + (37 * i) % 170 for i in range(140)]
 @pytest.mark.parametrize("dk,dv", [(32, 32), (128, 128), (192, 128), (72, 40)])
 @pytest.mark.parametrize("window", [None, 1, 65])
 def test_portions(lens, dk, dv, window):
+    assert (len(lens) > 100) == (sum((n + 127) // 128 for n in lens) * 8 > 960)
+    portions(lens, dk, dv, window)
+
+
+@pytest.mark.parametrize("lens", [[7], [1, 31, 32, 33, 64], [48 - (7 * i) % 48 for i in range(130)], [128 - (37 * i) % 128 for i in range(200)]],
+                         ids=["one", "few up to 64", "many up to 48", "many up to 128"])
+@pytest.mark.parametrize("dk,dv", [(32, 32), (128, 128), (72, 40)])
+@pytest.mark.parametrize("window", [None, 33])
+def test_sequences_of_a_tile_and_less(lens, dk, dv, window):
+    """The form for short sequences and, of the last list, heads on either side of its rule."""
+    portions(lens, dk, dv, window)
+
+
+def portions(lens, dk, dv, window):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
     gen = torch.Generator(device=DEV).manual_seed(dk + len(lens))
     H, G, T = 8, 2, sum(lens)
-    assert (len(lens) > 100) == (sum((n + 127) // 128 for n in lens) * H > 960)
     batch = StepBatch.build(list(range(len(lens))), [0] * len(lens), lens, DEV)
     q, k, v = (torch.randn((T, n, d), device=DEV, generator=gen).to(torch.bfloat16) for n, d in ((H, dk), (G, dk), (G, dv)))
     sink = torch.randn(H, device=DEV, generator=gen)
