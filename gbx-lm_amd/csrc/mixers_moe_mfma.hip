@@ -267,17 +267,32 @@ __global__ __launch_bounds__(512) void expert_group_kernel(const GroupArgs a) {
 // rows and their gated activation.  N output channels, C contraction; both multiples of 32.
 enum { SKINNY_DOWN = 0, SKINNY_UP = 1, SKINNY_GATED = 2 };
 
+// A workgroup's row tile and column block, cut from the tiles that exist, and those first: workgroups without work in between put two with work on
+// one CU and leave another idle.  The row tiles of one expert, which read the same weights, are neighbours on one XCD.  Few tiles: the XCDs share out all
+// units, column block by column block; from 48 tiles on each takes a run of tiles, which loses less to its remainder than to the strides between
+// experts.  (Runs cut from the grid | units | runs, us: 8 experts of 3 x 4096 x 2048, 256 pairs 198 | 128 | 174; 64 of 3 x 2048 x 2048, 256 pairs 304 | 341 | 302.)
+struct SkinnyUnit { int tile, col; };
+__device__ __forceinline__ SkinnyUnit skinny_unit(int tiles, int cols) {
+  if (tiles < 48) {
+    const int u = xcd_unit(tiles * cols);
+    return u < 0 ? SkinnyUnit{-1, 0} : SkinnyUnit{u % tiles, u / tiles};
+  }
+  const int per = (tiles + 7) / 8, j = blockIdx.x >> 3, tile = (blockIdx.x & 7) * per + j % per, col = j / per;
+  return col < cols && tile < tiles ? SkinnyUnit{tile, col} : SkinnyUnit{-1, 0};
+}
+
 template <int FORM>
 __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __restrict__ in, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
                                                            const int* __restrict__ sorted, const int* __restrict__ tile_tab, const float* __restrict__ scale,
                                                            bf16_t* __restrict__ out, int N, int C, int E, int top, int kind, float limit) {
   constexpr bool TWO = FORM == SKINNY_GATED;
-  const int bt = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;   // a contiguous run of row tiles per XCD (gridDim.x is a multiple of 8)
-  const int e = tile_tab[2 * bt];
-  if (e < 0 || e >= E) return;
+  const SkinnyUnit u = skinny_unit(offsets[E + 2], (N + 127) / 128);
+  if (u.tile < 0) return;
+  const int bt = u.tile, e = tile_tab[2 * bt];
+  if (e >= E) return;
   const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, hb = lane >> 5;
-  const int c0 = blockIdx.y * 128 + wave * 32;
+  const int c0 = u.col * 128 + wave * 32;
   if (c0 >= N) return;
   const int row = min(lo + r, hi - 1), pair = sorted[row];
   constexpr int PARTS = TWO ? 3 : 2;                                     // weights (twice), activations
@@ -376,7 +391,14 @@ constexpr int64_t MIN_PAIRS = 64;         // below this the weight-streaming row
 // 128 experts of 3 x 2048 x 768  231 | 248 | 297 | 459  against 235 | 243 | 243 | 277;  64 of 2 x 2048 x 2048  230 | 237 | 277 | 448  against
 // 254 | 256 | 258 | 276;  32 of 3 x 1024 x 512  31 | 30 | 33 | 42  against 29 | 29 | 30 | 35.
 constexpr int64_t SKINNY_PAIRS = 8;
-int rows_of(int64_t P, int E) { return P <= SKINNY_PAIRS * E ? RS : GR; }
+// ... and, where the grouped form's first product has at most half a chip of workgroups, each of them a chain over the whole contraction, up to 64.  Skinny |
+// grouped, us: without a gate, 16 experts of 2 x 1024 x 512, 4 | 32 | 64 pairs per expert 21 | 23 | 26 against 27 | 30 | 35; 8 of 2 x 4096 x 2048, 16 | 32 | 64
+// 71 | 90 | 113 against 106 | 108 | 119, 128 172 against 136; gated, 4 of 3 x 512 x 2048, 64 pairs 33 against 43.
+constexpr int64_t SKINNY_PAIRS_FEW = 64, FEW_GROUPS = 128;
+int rows_of(int64_t P, int E, int F, bool gated) {
+  const int64_t groups = (P / GR + E) * (gated ? (F + 127) / 128 : (F + 255) / 256);
+  return P <= (groups <= FEW_GROUPS ? SKINNY_PAIRS_FEW : SKINNY_PAIRS) * E ? RS : GR;
+}
 
 
 }  // namespace
@@ -402,7 +424,7 @@ int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBucke
 size_t expert_grouped_workspace(int64_t T, int K, int F, int E, int top) {
   const int64_t P = T * top;
   if (P < MIN_PAIRS || K % 32 || F % 32 || E > 4096 || P > 0x3fffffff) return 0;
-  return expert_buckets_bytes(P, rows_of(P, E), E) + align16(sizeof(bf16_t) * P * F);
+  return expert_buckets_bytes(P, RS, E) + align16(sizeof(bf16_t) * P * F);      // (the form with more tiles)
 }
 
 int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
@@ -430,14 +452,17 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
     return GBXM_ERR_UNSUPPORTED;
   const int P = static_cast<int>(a.T * top);
   ExpertBuckets k;
-  int rc = expert_buckets(a.idx, P, rows_of(P, E), E, a.ws, &k, s);
+  const bool gated = a.kind != GBXM_EXPERT_RELU2;
+  const int rows = rows_of(P, E, F, gated);
+  int rc = expert_buckets(a.idx, P, rows, E, a.ws, &k, s);
   if (rc != GBXM_OK) return rc;
   const int *offsets = k.offsets, *sorted = k.sorted, *tile_tab = k.tile_tab, tiles = k.tiles;
-  bf16_t* act = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(a.ws) + expert_buckets_bytes(P, rows_of(P, E), E));
+  bf16_t* act = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(a.ws) + expert_buckets_bytes(P, RS, E));
   const bf16_t* h = static_cast<const bf16_t*>(a.h);
   const bf16_t* first = static_cast<const bf16_t*>(a.first);
-  if (rows_of(P, E) == RS) {
-    const dim3 up(tiles, (F + 127) / 128), dn(tiles, (K + 127) / 128);
+  if (rows == RS) {
+    const auto grid = [&](int n) { return static_cast<unsigned>((static_cast<int64_t>(tiles) * ((n + 127) / 128) + 7) / 8 * 8); };
+    const unsigned up = grid(F), dn = grid(K);
     if (a.kind == GBXM_EXPERT_RELU2)
       expert_skinny_kernel<SKINNY_UP><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
     else
@@ -446,7 +471,6 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
                                                          static_cast<bf16_t*>(a.y), K, F, E, top, a.kind, a.limit);
     return after_launch("expert_ff (skinny groups)");
   }
-  const bool gated = a.kind != GBXM_EXPERT_RELU2;
   GroupArgs g{h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, gated ? (F + 127) / 128 : (F + 255) / 256, a.limit};
   rc = !gated ? launch_group<EXPERT_UP>(g, tiles, s) : a.kind == GBXM_GLU_SILU ? launch_group<EXPERT_SILU>(g, tiles, s) : launch_group<EXPERT_CLAMPED>(g, tiles, s);
   if (rc != GBXM_OK) return rc;

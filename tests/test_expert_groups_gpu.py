@@ -40,14 +40,26 @@ def reference(h, first, down, idx, kind, limit, scale):
 @pytest.mark.parametrize("kind", ["silu", "clamped_swish", "relu2"])
 @pytest.mark.parametrize("width,ff", [(32, 32), (64, 96), (96, 160), (288, 64), (160, 352)])
 def test_tiles_of_every_height(kind, width, ff):
+    tiles(COUNTS, kind, width, ff)
+
+
+@pytest.mark.parametrize("kind", ["silu", "clamped_swish", "relu2"])
+@pytest.mark.parametrize("width,ff", [(32, 32), (160, 288), (288, 96)])
+@pytest.mark.parametrize("counts", [[0, 1, 31, 32, 33, 63, 64, 65, 97, 128], [64], [(13 * i) % 41 for i in range(60)]], ids=["units", "one expert", "runs"])
+def test_skinny_tiles(kind, width, ff, counts):
+    """Few workgroups in the grouped form: tiles of 32 pairs, both ways of sharing them out among the XCDs."""
+    tiles(counts, kind, width, ff)
+
+
+def tiles(counts, kind, width, ff):
     from gbx_lm_amd import mixer_ops as M
     gen = torch.Generator(device="cuda").manual_seed(width + ff)
-    E, T = len(COUNTS), sum(COUNTS)
+    E, T = len(counts), sum(counts)
     rnd = lambda *s: torch.randn(s, device="cuda", generator=gen)
     h = rnd(T, width).to(torch.bfloat16)
     first = (rnd(E, ff * (1 if kind == "relu2" else 2), width) * width ** -0.5).to(torch.bfloat16)
     down = (rnd(E, width, ff) * ff ** -0.5).to(torch.bfloat16)
-    idx = torch.cat([torch.full((n,), e) for e, n in enumerate(COUNTS)])[torch.randperm(T, generator=torch.Generator().manual_seed(1))]
+    idx = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=torch.Generator().manual_seed(1))]
     idx = idx.to(torch.int32).to("cuda")[:, None].contiguous()
     for scale in (None, torch.rand((T, 1), device="cuda", generator=gen) + 0.5):
         got = M.expert_glu(h, first, down, idx, kind, 1.5, scale).double()
