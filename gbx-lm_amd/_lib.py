@@ -306,7 +306,8 @@ class WindowAttnArgs(ctypes.Structure):
                 ("T", ctypes.c_int64), ("B", ctypes.c_int32), ("n_tiles", ctypes.c_int32), ("q_tile", ctypes.c_int32),
                 ("H", ctypes.c_int32), ("G", ctypes.c_int32), ("dk", ctypes.c_int32), ("dv", ctypes.c_int32), ("window", ctypes.c_int32),
                 ("scale", ctypes.c_float), ("softcap", ctypes.c_float), ("decode_only", ctypes.c_int32), ("act", ctypes.c_int32),
-                ("partial", ctypes.c_void_p), ("partial_splits", ctypes.c_int32), ("longest", ctypes.c_int32)]
+                ("partial", ctypes.c_void_p), ("partial_splits", ctypes.c_int32),
+                ("most_keys", ctypes.c_int32), ("tile_keys", ctypes.c_int64)]
 
 
 class HeadSegment(ctypes.Structure):

@@ -11,7 +11,7 @@ descriptor tables built here once per step (one host-to-device copy).
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
@@ -30,10 +30,19 @@ class StepBatch:
     tok: torch.Tensor               # int32 [T, 2]: sequence of the step a row belongs to, its position
     q_tile: int = 0                 # query rows per tile of ``tiles``
     tiles: Optional[torch.Tensor] = None   # int32 [n_tiles, 2]: sequence of the step, first row of the tile inside it
+    keys_of: Dict[int, Tuple[int, int]] = field(default_factory=dict, repr=False, compare=False)       # ``tile_keys``: the same for every layer of the step
 
     @property
     def decode_only(self) -> bool:
         return all(n == 1 for n in self.n_new)
+
+    def tile_keys(self, window: int) -> Tuple[int, int]:
+        """Keys that a tile's rows see together under ``window``: the most of any tile, and their sum over the tiles."""
+        if window not in self.keys_of:
+            q = self.q_tile
+            keys = [min(p + min(t + q, n), window + min(q, n - t) - 1) for p, n in zip(self.pos0, self.n_new) for t in range(0, n, q)] if q else [0]
+            self.keys_of[window] = max(keys), sum(keys)
+        return self.keys_of[window]
 
     @staticmethod
     def build(slot: Sequence[int], pos0: Sequence[int], n_new: Sequence[int], device, q_tile: int = 128) -> "StepBatch":

@@ -11,6 +11,7 @@
 // The fp32 part per score (four transcendentals, see `exponent`) costs more than the products: the kernel is bound by vector
 // instructions, and by the tiles that start last -- late tiles of all heads come first.  Gates are rounded to bf16 for the value product.
 // Measured against five transcendentals a score and one group for all: see `launch`.
+#include <algorithm>
 #include "mixers_mfma.h"
 
 namespace gbxm {
@@ -236,17 +237,20 @@ int launch_shape(const TileArgs& t, int n_tiles, hipStream_t s) {
   return after_launch("window_attention (tiles)");
 }
 
-// Two groups of waves a tile, 64 keys each, while every CU then has at most one tile (a CU holds one such workgroup and two of one group), and for some more
-// tiles where they are long: they shorten the chain of key tiles behind the last queries.  Otherwise one group and 32 keys.  One | two, us, tiles x heads:
-//   32 heads of 128: 256, 1 000 rows 65 | 40; 352, 1 300 rows 82 | 49; 576, 2 200 rows 137 | 109; 1 024: 4 000 rows 256 | 295, with a window of 64 41 | 59,
-//   64 rows x 32 18 | 32; 2 048, 20 rows x 64 13 | 40 (five transcendentals, one group before both: 86, 129, 248, 783, 51, 21, 19);
-//   16 heads of 64: 384, 3 000 rows with a window of 1 024 60 | 60, without 144 | 80; 512: 2 000 rows x 2 109 | 68, 500 rows x 8 33 | 35, 64 rows x 32 7 | 11.
-// The line: tiles x heads up to 3 / 8 of the keys that a row can see, and up to 768.
+// Two groups of waves a tile, 64 keys each, shorten the chain of a long tile; one group and 32 keys leave a CU room for two tiles.  Either form takes as
+// long as its longest tile or as all of them on the tiles that fit at a time (256 | 512), in units of a key that one group multiplies, with what a tile
+// costs beside its keys as 140 | 175 of them.  One | two, us (in brackets: one group, five transcendentals a score, before both):
+//   32 heads of 128: 1 000 rows 65 | 40 (86), 1 300 82 | 49 (129), 2 200 137 | 109 (248), 4 000 256 | 295 (783), with a window of 64 41 | 59 (51); 2 047 + 1 100 + 333 +
+//   1 rows 145 | 138 (339); 64 rows x 32 18 | 32 (21); 20 rows x 64 13 | 40 (19); 20 rows x 30 beside 2 000 126 | 101;
+//   16 heads of 64: 4 000 rows 193 | 122 (351), with a window of 1 024 71 | 71 (112); 2 000 rows x 2 109 | 68 (182); 500 rows x 8 33 | 35 (53); 33 rows 5.7 | 6.1 (6.4).
 template <int DK, int DV>
-int launch(const TileArgs& t, int n_tiles, int longest, hipStream_t s) {
+int launch(const TileArgs& t, int n_tiles, int64_t most, int64_t sum, hipStream_t s) {
   if constexpr (DK + DV <= 256) {                            // (larger heads: 64 keys or a second group would cost the second wave per SIMD)
-    const int64_t n = static_cast<int64_t>(t.H) * n_tiles, keys = longest > 0 && longest < t.window ? longest : t.window;
-    if (n <= 256 || (n <= 768 && 8 * n <= 3 * keys)) return launch_shape<DK, DV, 2, 64>(t, n_tiles, s);
+    constexpr int64_t ONE = 140, TWO = 175;
+    if (most <= 0 || sum <= 0) { most = t.window; sum = n_tiles * most; }
+    const int64_t n = static_cast<int64_t>(t.H) * n_tiles, keys = sum * t.H;
+    const int64_t one = std::max(most + ONE, (keys + n * ONE) / 512), two = std::max(most / 2 + TWO, (keys / 2 + n * TWO) / 256);
+    if (two < one) return launch_shape<DK, DV, 2, 64>(t, n_tiles, s);
   }
   return launch_shape<DK, DV, 1, 32>(t, n_tiles, s);
 }
@@ -268,7 +272,7 @@ int launch_window_tiles(const gbxm_window_attn_args& a, hipStream_t s) {
   TileArgs t{static_cast<const bf16_t*>(a.qkv), static_cast<const bf16_t*>(a.kcache), static_cast<const bf16_t*>(a.vcache), a.seq, a.tiles,
              static_cast<bf16_t*>(a.out), a.dist_mul, a.dist_rate, a.gate_bias, a.row_stride, a.q_tile, a.H, a.G, a.window, a.H * a.dk,
              a.G * a.dk, a.scale, a.softcap};
-#define GBXM_TILE(DK_, DV_) if (a.dk == DK_ && a.dv == DV_) return launch<DK_, DV_>(t, a.n_tiles, a.longest, s)
+#define GBXM_TILE(DK_, DV_) if (a.dk == DK_ && a.dv == DV_) return launch<DK_, DV_>(t, a.n_tiles, a.most_keys, a.tile_keys, s)
   GBXM_TILE(64, 64); GBXM_TILE(96, 64); GBXM_TILE(128, 64); GBXM_TILE(64, 128); GBXM_TILE(128, 128); GBXM_TILE(192, 128); GBXM_TILE(256, 256);
   GBXM_TILE(96, 96); GBXM_TILE(64, 32); GBXM_TILE(32, 32); GBXM_TILE(32, 64);
 #undef GBXM_TILE

@@ -234,7 +234,7 @@ def window_attention(qkv: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tens
                             _f32(m.gate_bias, "gate_bias").data_ptr(), batch.total, len(batch.slot),
                             0 if batch.tiles is None else batch.tiles.shape[0], batch.q_tile, m.heads, m.kv_heads, m.dim, m.vdim, m.window,
                             m.scale, m.softcap, int(batch.decode_only), act, None if partial is None else partial.data_ptr(), splits,
-                            max(p + n for p, n in zip(batch.pos0, batch.n_new)))
+                            *((0, 0) if batch.decode_only else batch.tile_keys(m.window)))
     _lib.check_mixers(_lib.mixers().gbxm_window_attention(ctypes.byref(a), _stream(qkv.device)))
     return out
 

@@ -71,7 +71,8 @@ typedef struct {
   int32_t act;
   void* partial;                /* optional fp32 [partial_splits][T][H*dv]: lets a step of few rows split its keys over workgroups */
   int32_t partial_splits;
-  int32_t longest;              /* positions of the step's longest sequence, its new ones included; 0: unknown.  Chooses among forms of the prompt kernel */
+  int32_t most_keys;            /* keys that the rows of one of `tiles` see together, at most, and */
+  int64_t tile_keys;            /* their sum over `tiles`; 0: unknown.  They choose among forms of the prompt kernel */
 } gbxm_window_attn_args;
 int gbxm_window_attention(const gbxm_window_attn_args* a, void* stream);
 /* 1 if a step of this kind runs on the matrix-core tile kernel, 0 if on the row kernel (tests and benchmarks name the kernel). */

@@ -382,3 +382,15 @@ def test_log_probabilities_of_64_bit_logits_stay_in_64_bits():
     from gbx_lm_amd.mixer_ops import log_probabilities
     x = torch.randn(3, 1000, dtype=torch.float64) * 5
     assert torch.equal(log_probabilities(x), x - torch.logsumexp(x, -1, keepdim=True))
+
+
+def test_keys_of_a_steps_tiles():
+    from gbx_lm_amd.batching import StepBatch
+    for lens, pos, window in (([2047, 1100, 333, 1], [0] * 4, 4096), ([4000], [0], 64), ([300, 128, 129], [5, 0, 700], 64), ([20, 5, 1], [900, 3, 63], 64), ([7], [0], 1)):
+        keys = []
+        for p, n in zip(pos, lens):
+            for t in range(0, n, 128):
+                last = p + min(t + 128, n) - 1
+                keys.append(last - max(0, p + t - window + 1) + 1)
+        batch = StepBatch.build(list(range(len(lens))), pos, lens, "cpu")
+        assert batch.tile_keys(window) == (max(keys), sum(keys)) == batch.tile_keys(window)

@@ -23,7 +23,7 @@ def test_portions(dk, dv, cap, window):
 @pytest.mark.parametrize("cap,window", [(0.0, 33), (5.0, 300)])
 def test_more_tiles_than_compute_units(dk, dv, cap, window):
     """One group of waves a tile, tiles of 32 keys: edges of both, beside prompts of a few rows with and without history."""
-    portions([1, 31, 32, 33, 63, 65, 129, 257] + [1 + (11 * i) % 40 for i in range(60)], [0, 7, 33, 0, 64, 300, 31, 0] + [(5 * i) % 47 for i in range(60)],
+    portions([1, 31, 32, 33, 63, 65, 129, 257] + [1 + (11 * i) % 40 for i in range(200)], [0, 7, 33, 0, 64, 300, 31, 0] + [(5 * i) % 47 for i in range(200)],
              dk, dv, cap, window)
 
 
