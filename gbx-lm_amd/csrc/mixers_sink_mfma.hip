@@ -486,32 +486,31 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
 }
 
 // One group: a workgroup takes two query tiles, one from each end of the step's list -- in a long causal prompt a late tile (many keys) and an
-// early one (few) -- so that workgroups carry about the same work however they are spread over the chip; or (not `paired`) one.  Two groups: a
+// early one (few) -- so that workgroups carry about the same work however they are spread over the chip; or (not PAIRED) one.  Two groups: a
 // tile each, of all heads the late ones first.
-template <int DK, int DV, int GROUPS, int KT>
-__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles, const bool paired) {
+template <int DK, int DV, int GROUPS, int KT, bool PAIRED>
+__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  if constexpr (GROUPS == 1) {
-    const int per_head = paired ? (n_tiles + 1) / 2 : n_tiles, second = blockIdx.x % per_head, first = paired ? n_tiles - 1 - second : second;
-    const int head = blockIdx.x / per_head;
-    sink_tile<DK, DV, 1, KT>(a, first, head, lds);
-    if (second != first) sink_tile<DK, DV, 1, KT>(a, second, head, lds);
+  if constexpr (PAIRED) {
+    const int pairs = (n_tiles + 1) / 2, second = blockIdx.x % pairs, first = n_tiles - 1 - second, head = blockIdx.x / pairs;
+    sink_tile<DK, DV, GROUPS, KT>(a, first, head, lds);
+    if (second != first) sink_tile<DK, DV, GROUPS, KT>(a, second, head, lds);
   } else {
-    sink_tile<DK, DV, 2, KT>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
+    sink_tile<DK, DV, GROUPS, KT>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
   }
 }
 
-template <int DK, int DV, int GROUPS, int KT>
-int launch_groups(const SinkTileArgs& t, int n_tiles, bool paired, hipStream_t s) {
-  const unsigned grid = static_cast<unsigned>(t.H) * (paired ? (n_tiles + 1) / 2 : n_tiles);
+template <int DK, int DV, int GROUPS, int KT, bool PAIRED>
+int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(t.H) * (PAIRED ? (n_tiles + 1) / 2 : n_tiles);
   constexpr int bytes = SinkShape<DK, DV, GROUPS, KT>::LDS;
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT, PAIRED>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hip_fail(e, "sink_attention (tiles)");
     once.done();
   }
-  sink_tile_kernel<DK, DV, GROUPS, KT><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles, paired);
+  sink_tile_kernel<DK, DV, GROUPS, KT, PAIRED><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles);
   return after_launch("sink_attention (tiles)");
 }
 
@@ -519,18 +518,20 @@ int launch_groups(const SinkTileArgs& t, int n_tiles, bool paired, hipStream_t s
 // 32 tiles <192, 128> 282 | 187; 47 tiles 434 | 390; three of 20 334 | 250; 64 tiles 658 | 680, <128, 128> 469 | 466, <64, 64> 286 | 305.
 // Sequences of a tile's keys and less have no chain to share and nothing to balance: one group, 32 keys, a tile per workgroup.  The form that the line above gives |
 // this, us: 16 heads of <128, 128>, 20 rows 8.1 | 6.3, 20 rows x 16 8.4 | 6.5, x 64 14.6 | 11.9, 64 rows x 32 17.0 | 10.5 (32 heads: 18.6 | 19.9); <64, 128>, 100 rows x 200
-// 86 | 66; <96, 96> 86 | 68, but 128 rows x 64 30 | 32.5 and <128, 128>, 100 rows x 200 98 | 102.
+// 86 | 66; <96, 96> 86 | 68, but 128 rows x 64 30 | 32.5 and <128, 128>, 100 rows x 200 98 | 102, 40 rows x 200 95 | 100.  Large heads share tiles of 32 keys as it is: <192, 128>, 64 rows 8.7 | 9.5, x 16 9.5 |
+// 10.2, x 32 17.7 | 13.2, 20 rows 7.2 | 6.6.
 constexpr unsigned TWO_GROUPS = 960;
 template <int DK, int DV>
 int launch(const SinkTileArgs& t, int n_tiles, int longest, hipStream_t s) {
   constexpr int KT = DK + DV > 256 ? 32 : 64;                // (larger heads: 64 would cost the second wave per SIMD)
   const int64_t n = static_cast<int64_t>(t.H) * n_tiles;
-  if (longest > 0 && (longest <= (n <= TWO_GROUPS ? 64 : 48) || (DK + DV < 256 && longest <= 128 && n > 1536)))
-    return launch_groups<DK, DV, 1, 32>(t, n_tiles, false, s);
+  const int short_keys = n > TWO_GROUPS ? (DK + DV < 256 ? 48 : 32) : n <= 256 && KT == 32 ? 32 : 64;
+  if (longest > 0 && (longest <= short_keys || (DK + DV < 256 && longest <= 128 && n > 1536)))
+    return launch_groups<DK, DV, 1, 32, false>(t, n_tiles, s);
   if constexpr (DK + DV <= 320) {
-    if (n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT>(t, n_tiles, false, s);
+    if (n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT, false>(t, n_tiles, s);
   }
-  return launch_groups<DK, DV, 1, KT>(t, n_tiles, true, s);
+  return launch_groups<DK, DV, 1, KT, true>(t, n_tiles, s);
 }
 
 constexpr int CAPS[][2] = {{32, 32}, {64, 64}, {64, 128}, {96, 96}, {128, 128}, {192, 128}, {256, 256}};
