@@ -41,6 +41,8 @@
 //     launch alone ~25 us): with 2 steps per workgroup the ramp / drain of the staging pipeline outweighs the bytes saved.
 // In-kernel stamps of this kernel (compute waves, 4096-value rows = 4 steps): a step is ~8k cycles of which the MFMAs are
 // ~2.5k; ISSUING the next step's 6 weight loads takes 3-5k (they queue behind the loaders' 64 requests in the in-order path).
+// Vector instructions do not bound it either: with the group's product started from -C xsum and z xsum of two groups by one fp32 matrix instruction, 68 of a
+// step's 138 multiply-adds were gone and the times the same (28672 x 4096, 2 bits, 32 rows 17.5 | 17.4, 14336 x 4096 13.4 | 13.5, 4096 x 4096, 4 bits 10.0 | 10.2).
 // -DBX_STAMPS: diagnostic build with s_memtime phase stamps (scratch/stamps_batch.py).
 #include "mfma_common.h"
 #include "gbx_env.h"
