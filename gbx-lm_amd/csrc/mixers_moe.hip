@@ -66,11 +66,24 @@ __device__ __forceinline__ void rows_dot(const T* __restrict__ w0, const T* __re
 
 constexpr int VC = 4 * NW;        // channels per workgroup of the vector form
 
-template <typename T, bool FAST, bool GATED>
+// A workgroup's pair and block of VC channels, from a grid of pairs x blocks, or (RUNS) from one dimension of workgroups, which go round-robin over the 8
+// XCDs -- each gets a run of units, blocks one after another and all pairs of a block together, so that the pairs of one expert read its rows from one L2.
+struct PairUnit { int64_t pair; int block; };
+template <bool RUNS> __device__ __forceinline__ PairUnit pair_unit(unsigned pairs, int blocks) {
+  if constexpr (!RUNS) return {blockIdx.x, static_cast<int>(blockIdx.y)};
+  const unsigned units = pairs * blocks, per = (units + 7) / 8, j = blockIdx.x >> 3, u = (blockIdx.x & 7) * per + j;
+  if (j >= per || u >= units) return {0, -1};
+  return {u % pairs, static_cast<int>(u / pairs)};
+}
+
+template <typename T, bool FAST, bool GATED, bool RUNS>
 __global__ __launch_bounds__(NT) void expert_up_vec(const T* __restrict__ h, const T* __restrict__ first, const int* __restrict__ idx,
-                                                   const float* __restrict__ scale, T* __restrict__ act, int K, int F, int top, int kind, float limit) {
-  const int64_t pair = blockIdx.x;
-  const int lane = threadIdx.x & 63, f = blockIdx.y * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), fc = min(f, F - 1);
+                                                   const float* __restrict__ scale, T* __restrict__ act, int K, int F, int top, int kind, float limit,
+                                                   unsigned pairs) {
+  const PairUnit at = pair_unit<RUNS>(pairs, (F + VC - 1) / VC);
+  if (at.block < 0) return;
+  const int64_t pair = at.pair;
+  const int lane = threadIdx.x & 63, f = at.block * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), fc = min(f, F - 1);
   const T* w = first + (static_cast<int64_t>(idx[pair]) * (GATED ? 2 : 1) * F + fc) * K;
   float a, u;
   rows_dot<T, GATED>(w, w + static_cast<int64_t>(F) * K, h + (pair / top) * K, K, lane & 15, a, u);
@@ -82,11 +95,13 @@ __global__ __launch_bounds__(NT) void expert_up_vec(const T* __restrict__ h, con
   }
 }
 
-template <typename T>
+template <typename T, bool RUNS>
 __global__ __launch_bounds__(NT) void expert_down_vec(const T* __restrict__ act, const T* __restrict__ down, const int* __restrict__ idx, T* __restrict__ y,
-                                                     int K, int F) {
-  const int64_t pair = blockIdx.x;
-  const int lane = threadIdx.x & 63, c = blockIdx.y * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), cc = min(c, K - 1);
+                                                     int K, int F, unsigned pairs) {
+  const PairUnit at = pair_unit<RUNS>(pairs, (K + VC - 1) / VC);
+  if (at.block < 0) return;
+  const int64_t pair = at.pair;
+  const int lane = threadIdx.x & 63, c = at.block * VC + 4 * (threadIdx.x >> 6) + (lane >> 4), cc = min(c, K - 1);
   float a, unused;
   const T* w = down + (static_cast<int64_t>(idx[pair]) * K + cc) * F;
   rows_dot<T, false>(w, w, act + pair * F, F, lane & 15, a, unused);
@@ -155,6 +170,11 @@ __global__ __launch_bounds__(NT) void expert_down_rows(const T* __restrict__ act
   }
 }
 
+// Where enough pairs meet in an expert for the runs of `pair_unit` to pay.  Grid of pairs x blocks | runs, us: fp32, 8 experts of 3 x 4096 x 2048, 16 pairs 233 | 166, 128
+// 1 061 | 698 (an earlier form 945); 128 of 3 x 2048 x 768, 64 pairs 191 | 168, 512 1 170 | 1 060, but 16 49 | 51; 64 of 2 x 2048 x 2048, 16 pairs 89 | 99, 32 180 | 171; bf16, 16 of
+// 3 x 1024 x 512, 8 pairs 6.6 | 8.2, 16 12.9 | 9.0, 48 26 | 15; 4 of 3 x 512 x 2048, 4 pairs 9.7 | 9.0, 8 14.3 | 10.2; 64 of 3 x 1024 x 256, 16 pairs 7.1 | 7.6, 32 12.7 | 10.5.
+bool pairs_share(int64_t P, int E) { return P >= 2 * static_cast<int64_t>(E) || (P >= 16 && 2 * P >= E); }
+
 template <typename T, bool FAST, bool GATED>
 int launch_rows(const gbxm_expert_args& a, hipStream_t s) {
   constexpr int PER = 16 / sizeof(T);
@@ -167,8 +187,15 @@ int launch_rows(const gbxm_expert_args& a, hipStream_t s) {
   const T *h = static_cast<const T*>(a.h), *first = static_cast<const T*>(a.first), *down = static_cast<const T*>(a.down);
   T* y = static_cast<T*>(a.y);
   if (vec) {
-    expert_up_vec<T, FAST, GATED><<<gu, NT, 0, s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit);
-    expert_down_vec<T><<<gd, NT, 0, s>>>(act, down, a.idx, y, a.K, a.F);
+    const auto grid = [](const dim3& g) { return dim3((g.x * g.y + 7) / 8 * 8); };
+    if (pairs_share(P, a.E) && P * gu.y < 0x7ffffff0 && P * gd.y < 0x7ffffff0) {
+      const unsigned pairs = static_cast<unsigned>(P);
+      expert_up_vec<T, FAST, GATED, true><<<grid(gu), NT, 0, s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit, pairs);
+      expert_down_vec<T, true><<<grid(gd), NT, 0, s>>>(act, down, a.idx, y, a.K, a.F, pairs);
+    } else {
+      expert_up_vec<T, FAST, GATED, false><<<gu, NT, 0, s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit, 0);
+      expert_down_vec<T, false><<<gd, NT, 0, s>>>(act, down, a.idx, y, a.K, a.F, 0);
+    }
   } else {
     expert_up_rows<T, FAST, GATED><<<gu, NT, a.K * sizeof(float), s>>>(h, first, a.idx, a.scale, act, a.K, a.F, a.top, a.kind, a.limit);
     expert_down_rows<T><<<gd, NT, a.F * sizeof(float), s>>>(act, down, a.idx, y, a.K, a.F);

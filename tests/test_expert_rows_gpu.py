@@ -13,13 +13,27 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("k,f,off", [(8, 8, 0), (120, 16, 0), (128, 136, 0), (136, 24, 0), (512, 520, 0), (520, 504, 0), (2048, 768, 0), (12, 40, 0), (20, 7, 0), (128, 64, 1)])
 @pytest.mark.parametrize("kind,scaled", [("silu", False), ("clamped_swish", True), ("relu2", True)])
 def test_rows(dt, k, f, off, kind, scaled):
+    rows(dt, k, f, off, kind, scaled, torch.tensor([[4, 0], [2, 4], [1, 2]], dtype=torch.int32, device=DEV), 5)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,f", [(8, 8), (136, 24), (264, 520)])
+@pytest.mark.parametrize("t,e", [(8, 5), (9, 32), (15, 3), (1, 1)])
+def test_runs_of_pairs(dt, k, f, t, e):
+    """Pairs that share experts, blocks of channels in runs: both terms of the rule, units on and off the eighth."""
+    top = min(2, e)
+    idx = torch.stack([(torch.arange(top) * 7 + 5 * i + i // 3) % e for i in range(t)]).to(torch.int32).to(DEV)
+    for kind in ("silu", "relu2"):
+        rows(dt, k, f, 0, kind, False, idx, e)
+
+
+def rows(dt, k, f, off, kind, scaled, idx, e):
     from gbx_lm_amd import mixer_ops as M
-    t, top, e = 3, 2, 5
+    t, top = idx.shape
     g = torch.Generator(device=DEV).manual_seed(k + f)
     rnd = lambda *s: torch.randn(s, device=DEV, generator=g).to(dt)
     h = torch.empty(t * k + off, dtype=dt, device=DEV)[off:].view(t, k).copy_(rnd(t, k))
     first, down = rnd(e, f * (1 if kind == "relu2" else 2), k) * k ** -0.5, rnd(e, k, f) * f ** -0.5
-    idx = torch.tensor([[4, 0], [2, 4], [1, 2]], dtype=torch.int32, device=DEV)
     scale = torch.rand((t, top), device=DEV, generator=g) + 0.5 if scaled else None
     got = M.expert_glu(h, first, down, idx, kind, 1.5, scale).double()
     eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -22
