@@ -47,7 +47,7 @@ struct MfmaArgs {
 // mfma_batch.hip: 2 <= M <= 32, 2/4 bits, group 128 (no-dequant matrix-core kernel); false -> use the split-K kernel
 bool qgemm_batch_supported(int M, int K, int bits, int log2g);
 hipError_t launch_qgemm_batch(const MfmaArgs& a, int bits, bool bf16, hipStream_t s);
-// mfma_rows.hip: 2 <= M <= 32, K >= 1024 (a chunk of 128 for each of a workgroup's eight waves), any bits and group, no dequantising;
+// mfma_rows.hip, mfma_slab_impl.h: 2 <= M <= 32, K >= 1024 (a chunk of 128 for each of a workgroup's eight waves), any bits and group, no dequantising;
 // hipErrorInvalidValue for less, and for scales or zeros that are not aligned to a chunk's
 hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t s);
 // second launch of a k-split GEMM: y = round(sum of the fp32 slices ws[slices][M][N]) (+ bias as a second rounding)

@@ -1,13 +1,13 @@
-// Quantised products of 2 to 32 rows outside the group-128 batch kernel: groups of 32 and 64, and contractions that are no multiple of 1024.
+// Quantised products of 2 to 32 rows over contractions whose rows do not fit the registers (beyond 4096, not in slices; shorter ones: mfma_slab_impl.h), outside the group-128
+// batch kernel.
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
 // A workgroup takes 16 NT outputs, its waves share out the chunks of 128 of K; packed words, scales and the rows' image go straight to the registers of
 // the lane that feeds them to the matrix cores (packed_fields.h), one chunk ahead of the one being multiplied; sum_k x comes from the matrix cores too
 // (a product with ones, shared by the wave's outputs), and the waves' sums meet in LDS.  No weight is expanded or rounded to the activation type; only an
 // output whose sum is not finite is taken again, weight by weight (expanded_dot): infinite activations give what their products with the weights give.
 // Bound by the latency of a wave's two or three chunks and by the rows' way through the first cache (27 rows: five bytes of rows for each byte of
-// weights).  Measured against the dequantising kernel that took these (us, weights cold): 3 bits,
-// group 64: 27 rows of 8192 x 3072 21.0 -> 14.0, 2 rows 20.9 -> 9.9, 8 rows of 4096 x 4096 14.9 -> 8.6, 32 of 14336 x 4096 39.2 -> 35.3; 4 bits, group 32:
-// 8 rows of 4096 x 11008 38.5 -> 20.4.
+// weights).  Measured against the dequantising kernel that took these (us, weights cold): 4 bits, group 32: 8 rows of 4096 x 11008 38.5 -> 20.4.
+#include "mfma_slab.h"
 #include "packed_fields.h"
 
 namespace gbx {
@@ -203,6 +203,7 @@ hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t
   uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
   for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
   if (a.swiglu || a.M < 2 || a.M > 32 || a.K % 128 || a.K < 128 * RW || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
+  if (const hipError_t e = launch_qgemm_slab(a, bits, bf16, s); e != hipErrorInvalidValue) return e;
   return bits == 2 ? launch_rows<2>(a, bf16, s) : bits == 3 ? launch_rows<3>(a, bf16, s) : bits == 4 ? launch_rows<4>(a, bf16, s) : hipErrorInvalidValue;
 }
 

@@ -57,6 +57,57 @@ struct Packed {
       for (int t = 0; t < 4; ++t) { raw[i][2 * t] = p[3 * t + a]; raw[i][2 * t + 1] = p[3 * t + b]; }
     }
   }
+  // the same words through a buffer: `at` the first byte of the lane's row plus lane_byte(f), `chunk` the chunk's first byte in the row (uniform)
+  static __device__ __forceinline__ int lane_byte(int f) {
+    return BITS == 4 ? (GRP == 128 ? 16 : GRP == 64 ? 8 : 4) * f
+         : BITS == 2 ? (GRP == 128 ? 8 * f : GRP == 64 ? 4 * f : 4 * (f >> 1))
+                     : (GRP == 128 ? 12 * f : GRP == 64 ? 4 * ((3 * f) >> 1) : 4 * ((3 * f) >> 2));
+  }
+  __device__ __forceinline__ void load_buffer(int i, __amdgpu_buffer_rsrc_t r, int at, int chunk) {
+    auto one = [&](int byte) { return __builtin_amdgcn_raw_buffer_load_b32(r, at + byte, chunk, 0); };
+    auto two = [&](int byte, int q) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, at + byte, chunk, 0);
+      raw[i][q] = v[0]; raw[i][q + 1] = v[1];
+    };
+    if constexpr (BITS == 4 && GRP == 128) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, at, chunk, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) raw[i][q] = v[q];
+    } else if constexpr (BITS == 4 && GRP == 64) {
+      two(0, 0); two(32, 2);
+    } else if constexpr (BITS == 4) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) raw[i][t] = one(16 * t);
+    } else if constexpr (BITS == 2 && GRP == 128) {
+      two(0, 0);
+    } else if constexpr (BITS == 2 && GRP == 64) {
+      raw[i][0] = one(0); raw[i][1] = one(16);
+    } else if constexpr (BITS == 2) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) raw[i][t] = one(8 * t);
+    } else if constexpr (GRP == 128) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, at, chunk, 0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) raw[i][q] = v[q];
+    } else if constexpr (GRP == 64) {
+      two(0, 0); two(24, 2);
+    } else {                                               // (quarter 3 ends with its first word: the second is the next row's, and nothing of it is used)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) two(12 * t, 2 * t);
+    }
+  }
+  __device__ __forceinline__ void load_affine_buffer(int i, __amdgpu_buffer_rsrc_t rs, __amdgpu_buffer_rsrc_t rz, int at, int first) {
+    if constexpr (NF == 1) {
+      sc[i][0] = __builtin_amdgcn_raw_buffer_load_b16(rs, at, first, 0); ze[i][0] = __builtin_amdgcn_raw_buffer_load_b16(rz, at, first, 0);
+    } else if constexpr (NF == 2) {
+      const unsigned a = __builtin_amdgcn_raw_buffer_load_b32(rs, at, first, 0), b = __builtin_amdgcn_raw_buffer_load_b32(rz, at, first, 0);
+      sc[i][0] = a & 0xFFFF; sc[i][1] = a >> 16; ze[i][0] = b & 0xFFFF; ze[i][1] = b >> 16;
+    } else {
+      const auto a = __builtin_amdgcn_raw_buffer_load_b64(rs, at, first, 0), b = __builtin_amdgcn_raw_buffer_load_b64(rz, at, first, 0);
+      sc[i][0] = a[0] & 0xFFFF; sc[i][1] = a[0] >> 16; sc[i][2] = a[1] & 0xFFFF; sc[i][3] = a[1] >> 16;
+      ze[i][0] = b[0] & 0xFFFF; ze[i][1] = b[0] >> 16; ze[i][2] = b[1] & 0xFFFF; ze[i][3] = b[1] >> 16;
+    }
+  }
   __device__ __forceinline__ void load_affine(int i, const unsigned short* sp, const unsigned short* zp) {
     if constexpr (NF == 1) {
       sc[i][0] = *sp; ze[i][0] = *zp;
@@ -69,15 +120,16 @@ struct Packed {
       ze[i][0] = b.x & 0xFFFF; ze[i][1] = b.x >> 16; ze[i][2] = b.y & 0xFFFF; ze[i][3] = b.y >> 16;
     }
   }
-  // the eight operands C + q of step t (compile-time) of row tile i, in the order of the stored activations
-  __device__ __forceinline__ packed_x4 operand(int i, int t, int f) const {
+  // the eight operands C + q of step t (compile-time) of row tile i, in the order of the stored activations.  `mask` and `magic`: MASK and MAGIC, from a
+  // caller that holds them in registers (one v_and_or_b32 a dword takes no literal: from constants the compiler makes two instructions)
+  __device__ __forceinline__ packed_x4 operand(int i, int t, int f, unsigned mask = MASK, unsigned magic = MAGIC) const {
     packed_x4 r;
     if constexpr (BITS == 4) {
       const unsigned w = raw[i][t];
-      r.x = (w & MASK) | MAGIC; r.y = ((w >> 4) & MASK) | MAGIC; r.z = ((w >> 8) & MASK) | MAGIC; r.w = ((w >> 12) & MASK) | MAGIC;
+      r.x = (w & mask) | magic; r.y = ((w >> 4) & mask) | magic; r.z = ((w >> 8) & mask) | magic; r.w = ((w >> 12) & mask) | magic;
     } else if constexpr (BITS == 2) {
       const unsigned w = GRP == 32 ? raw[i][t] >> (8 * (f & 1)) : raw[i][t >> 1] >> (8 * (t & 1));
-      r.x = (w & MASK) | MAGIC; r.y = ((w >> 2) & MASK) | MAGIC; r.z = ((w >> 4) & MASK) | MAGIC; r.w = ((w >> 6) & MASK) | MAGIC;
+      r.x = (w & mask) | magic; r.y = ((w >> 2) & mask) | magic; r.z = ((w >> 4) & mask) | magic; r.w = ((w >> 6) & mask) | magic;
     } else {
       unsigned w;                                          // the octet's 24 bits from bit 0
       if constexpr (GRP == 128) {
@@ -94,7 +146,7 @@ struct Packed {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const unsigned q = (w >> (6 * j)) & 0x3F;
-        v[j] = ((q | (q << 13)) & MASK) | MAGIC;
+        v[j] = ((q | (q << 13)) & mask) | magic;
       }
       r.x = v[0]; r.y = v[1]; r.z = v[2]; r.w = v[3];
     }
