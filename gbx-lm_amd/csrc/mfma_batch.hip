@@ -621,13 +621,10 @@ static hipError_t launch_batch_bits(const MfmaArgs& a0, bool bf16, hipStream_t s
   MfmaArgs a = a0;
   a.ksplit = (a.ws && a.log2g == 7) ? batch_ksplit(a.N, a.K, a.nseg, a.partials_only != 0) : 1;
   if (a.ksplit <= 1) a.ws = nullptr;
-  // Steps of batched decoding (slices summed by their reader, gate and up) keep this kernel: a stack of layers carries every changed rounding on from step to step, and
+  // Steps of batched decoding (slices of the contraction, gate and up) keep this kernel: a stack of layers carries every changed rounding on from step to step, and
   // the other kernel gains little there (here | there, us, 32 rows, 2 bits: 6144 x 4096 9.6 | 8.6, 4096 x 4096 7.2 | 6.9, 4096 x 14336 13.8 | 14.1, gate and up of
   // 14336 x 4096 20.4 | 20.6).
-  if (const hipError_t e = a.swiglu || a.partials_only ? hipErrorInvalidValue : launch_qgemm_slab(a, BITS, bf16, s); e != hipErrorInvalidValue) {
-    if (e != hipSuccess || !a.ws) return e;
-    return launch_splitk_finish(a.ws, a.bias, a.y, a.ksplit, a.M, a.N, bf16, s);
-  }
+  if (const hipError_t e = a.swiglu || a.ws ? hipErrorInvalidValue : launch_qgemm_slab(a, BITS, bf16, s); e != hipErrorInvalidValue) return e;
   if (a.ws) {                                       // 128-row workgroups x ksplit slices, then the summing launch
     // (few tiles even after the split -- o_proj: 32 x 4 -- : 64-row workgroups put one on every CU)
     const bool narrow = a.partials_only && ((a.N + 127) / 128) * a.ksplit <= 128 && a.N % 64 == 0;
@@ -681,8 +678,7 @@ bool qgemm_batch_supported(int M, int K, int bits, int log2g) {
 hipError_t launch_qgemm_slab(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
   uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
   for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
-  const int slices = a.ws ? a.ksplit : 1;
-  if (a.swiglu || a.M < 2 || a.M > 32 || a.K % 128 || a.K < 1024 || (a.K / 128) % slices || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
+  if (a.swiglu || a.ws || a.M < 2 || a.M > 32 || a.K % 128 || a.K < 1024 || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
   return bits == 2 ? launch_slab_bits<2>(a, bf16, s) : bits == 3 ? launch_slab_bits<3>(a, bf16, s) : bits == 4 ? launch_slab_bits<4>(a, bf16, s) : hipErrorInvalidValue;
 }
 

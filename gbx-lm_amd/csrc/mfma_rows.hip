@@ -1,4 +1,4 @@
-// Quantised products of 2 to 32 rows over contractions whose rows do not fit the registers (beyond 4096, not in slices; shorter ones: mfma_slab_impl.h), outside the group-128
+// Quantised products of 2 to 32 rows over contractions whose rows do not fit the registers (beyond 4096; shorter ones: mfma_slab_impl.h), outside the group-128
 // batch kernel.
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
 // A workgroup takes 16 NT outputs, its waves share out the chunks of 128 of K; packed words, scales and the rows' image go straight to the registers of

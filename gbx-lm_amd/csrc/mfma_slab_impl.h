@@ -1,7 +1,7 @@
 // Quantised products of 2 to 32 rows: the rows stay in registers, the packed weights stream past them.
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
-// A workgroup owns the whole contraction, or one slice of it, for up to 8 (16 rows of x: 16) tiles of 16 outputs.  Each of its eight waves owns CW
-// neighbouring chunks of 128 of that range: it brings its part of the rows into registers once (LDS-DMA in row order, then fragments), and walks the tiles with
+// A workgroup owns the whole contraction (up to 4096) for up to 8 (16 rows of x: 16) tiles of 16 outputs.  Each of its eight waves owns CW
+// neighbouring chunks of 128 of it: it brings its part of the rows into registers once (LDS-DMA in row order, then fragments), and walks the tiles with
 // weights requested up to three tiles ahead.  Waves share nothing until the end, where their sums meet in LDS: one barrier per workgroup.
 //   * fields go to the matrix cores as the numbers C + q (packed_fields.h); sum_k x per group comes from a product with ones at the start;
 //   * lane quarter f loads scale and zero of chunk f of the wave: the scales reach the other quarters by one exchange a chunk, and the zeros' part
@@ -14,7 +14,7 @@
 // Bound by its start -- arguments, code, then the rows: 256 KB of them a CU (32 x 4096) take 3 us -- and by the field and scale arithmetic of a tile.  Measured (us, weights
 // cold; before: mfma_rows.hip, and mfma_batch.hip where groups are of 128 and K a multiple of 1024): 27 rows of 8192 x 3072, 3 bits, group 64
 // 14.3 -> 10.0; 32 rows of 14336 x 4096, 4 bits, group 32 49 -> 18.5; 32 of 16384 x 2048, 3 bits, group 32 34 -> 14.3; group 128: 16 of 11008 x 4096, 3 bits 18.9 -> 10.8;
-// 2 of 4096 x 4096, 4 bits 9.2 -> 6.7; 17, 2 bits 10.0 -> 7.6; 32 of 4096 x 14336, 2 bits, in seven slices 17.8 -> 16.6; q, k and v of 4096 x 4096, 32 rows 11.6 -> 9.1.
+// 2 of 4096 x 4096, 4 bits 9.2 -> 6.7; 17, 2 bits 10.0 -> 7.6; q, k and v of 4096 x 4096, 32 rows 11.6 -> 9.1.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -34,9 +34,8 @@ struct SlabArgs {
   const uint32_t* qw[3];
   const unsigned short *sc[3], *ze[3], *bias[3];
   unsigned short* y[3];
-  float* ws;
   int N[3], block0[3];                     // rows of a matrix, first workgroup of it
-  int M, K, cps, tpb;                      // cps: chunks of a slice; tpb: tiles of a workgroup
+  int M, K, tpb;                           // tpb: tiles of a workgroup
 };
 
 // s_waitcnt: at most n vector memory accesses outstanding
@@ -62,11 +61,11 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char slab_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, f = lane >> 4;
   unsigned char* mine = slab_lds + wave * SLAB_BYTES;
-  const int K = a.K, words = (K >> 5) * BITS, groups = K / GRP, c_slice = blockIdx.y * a.cps;
-  const int c0 = c_slice + wave * CW, own = a.cps - wave * CW;         // the wave's first chunk, and how many there are from it on
+  const int K = a.K, words = (K >> 5) * BITS, groups = K / GRP, chunks = K >> 7;
+  const int c0 = wave * CW, own = chunks - c0;                         // the wave's first chunk, and how many there are from it on
   // (every argument is asked for at once: one trip to memory instead of one per use)
   asm volatile("" ::"s"(a.qw[0]), "s"(a.qw[1]), "s"(a.qw[2]), "s"(a.sc[0]), "s"(a.sc[1]), "s"(a.sc[2]), "s"(a.ze[0]), "s"(a.ze[1]), "s"(a.ze[2]), "s"(a.x), "s"(a.N[0]), "s"(a.N[1]), "s"(a.N[2]),
-               "s"(a.block0[1]), "s"(a.block0[2]), "s"(a.M), "s"(a.K), "s"(a.cps), "s"(a.tpb));
+               "s"(a.block0[1]), "s"(a.block0[2]), "s"(a.M), "s"(a.K), "s"(a.tpb));
   const int seg = (blockIdx.x >= a.block0[1]) + (blockIdx.x >= a.block0[2]);
   const int N = pick(seg, a.N[0], a.N[1], a.N[2]), tile0 = (blockIdx.x - pick(seg, a.block0[0], a.block0[1], a.block0[2])) * a.tpb, nt = min(a.tpb, ((N + 15) >> 4) - tile0);
 
@@ -237,7 +236,6 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   unsigned short* y = a.y[seg];
   auto write = [&](int n, int m, float r) {
     const size_t at = static_cast<size_t>(m) * N + n;
-    if (a.ws) { a.ws[static_cast<size_t>(blockIdx.y) * a.M * N + at] = r; return; }
     unsigned short o = f32_to_act<BF16>(r);
     if (bias) o = f32_to_act<BF16>(act_to_f32<BF16>(o) + act_to_f32<BF16>(bias[n]));       // (a second rounding)
     y[at] = o;
@@ -255,7 +253,6 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   }
   if (finite) return;
   // (the places that this thread has written: nobody else's results change)
-  const int64_t k0 = static_cast<int64_t>(c_slice) * 128;
 #pragma unroll 1
   for (int q = 0; tid + (q >> 2) * 64 * SLAB_WAVES < places; ++q) {
     const int p = tid + (q >> 2) * 64 * SLAB_WAVES, v = q & 3, m = (p >> 6) % MT * 16 + 4 * f + v;
@@ -264,8 +261,7 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
     float r = 0.f;
     for (int w = 0; w < SLAB_WAVES; ++w) r += *reinterpret_cast<const float*>(slab_lds + w * SLAB_BYTES + p * 16 + v * 4);
     if (!__builtin_isfinite(r))
-      write(n, m, expanded_dot<BITS, GRP, BF16>(a.x + static_cast<int64_t>(m) * K + k0, a.qw[seg] + n * words + c_slice * P::WPC, a.sc[seg] + n * groups + c_slice * NF,
-                                                a.ze[seg] + n * groups + c_slice * NF, a.cps * 128));
+      write(n, m, expanded_dot<BITS, GRP, BF16>(a.x + static_cast<int64_t>(m) * K, a.qw[seg] + n * words, a.sc[seg] + n * groups, a.ze[seg] + n * groups, K));
   }
 }
 
@@ -283,23 +279,22 @@ hipError_t launch_slab_shape(const MfmaArgs& a, hipStream_t s) {
     done.done();
   }
   SlabArgs t{a.x, {a.qweight, a.qweight_x[0], a.qweight_x[1]}, {a.scales, a.scales_x[0], a.scales_x[1]}, {a.zeros, a.zeros_x[0], a.zeros_x[1]},
-             {a.bias, a.bias_x[0], a.bias_x[1]}, {a.y, a.y_x[0], a.y_x[1]}, a.ws, {a.N, 0, 0}, {0, 0x7FFFFFFF, 0x7FFFFFFF}, a.M, a.K, 0, 0};
-  const int slices = a.ws ? a.ksplit : 1, most = SLAB_BYTES / (MT * 1024);
-  t.cps = a.K / 128 / slices;
+             {a.bias, a.bias_x[0], a.bias_x[1]}, {a.y, a.y_x[0], a.y_x[1]}, {a.N, 0, 0}, {0, 0x7FFFFFFF, 0x7FFFFFFF}, a.M, a.K, 0};
+  constexpr int most = SLAB_BYTES / (MT * 1024);
   // a workgroup fills a CU: as many tiles a workgroup as spread them evenly over as few rounds of 256 as their sums' place in LDS allows
   int tiles = 0;
   for (int g = 0; g < std::max(a.nseg, 1); ++g) {
     if (a.nseg > 1) t.N[g] = a.n_seg[g];
     tiles += (t.N[g] + 15) / 16;
   }
-  const int rounds = (tiles * slices + 256 * most - 1) / (256 * most), wide = std::max(256 * rounds / slices, 1);
-  t.tpb = std::clamp((tiles + wide - 1) / wide, 1, most);
+  const int rounds = (tiles + 256 * most - 1) / (256 * most);
+  t.tpb = (tiles + 256 * rounds - 1) / (256 * rounds);
   int blocks = 0;
   for (int g = 0; g < std::max(a.nseg, 1); ++g) {
     t.block0[g] = blocks;
     blocks += ((t.N[g] + 15) / 16 + t.tpb - 1) / t.tpb;
   }
-  qgemm_slab_kernel<BITS, GRP, BF16, MT, CW><<<dim3(blocks, slices), 64 * SLAB_WAVES, SLAB_LDS, s>>>(t);
+  qgemm_slab_kernel<BITS, GRP, BF16, MT, CW><<<blocks, 64 * SLAB_WAVES, SLAB_LDS, s>>>(t);
   return hipGetLastError();
 }
 
@@ -310,8 +305,7 @@ hipError_t launch_slab_type(const MfmaArgs& a, bool bf16, hipStream_t s) {
 
 template <int BITS, int GRP, int MT>
 hipError_t launch_slab_chunks(const MfmaArgs& a, bool bf16, hipStream_t s) {
-  const int cps = a.ws ? a.K / 128 / a.ksplit : a.K / 128;
-  switch ((cps + SLAB_WAVES - 1) / SLAB_WAVES) {
+  switch ((a.K / 128 + SLAB_WAVES - 1) / SLAB_WAVES) {
     case 1: return launch_slab_type<BITS, GRP, MT, 1>(a, bf16, s);
     case 2: return launch_slab_type<BITS, GRP, MT, 2>(a, bf16, s);
     case 3: return launch_slab_type<BITS, GRP, MT, 3>(a, bf16, s);
