@@ -675,20 +675,25 @@ static int split_heads(int batch, int n_heads, int rep, int capacity) {
   return (capacity <= 1536 && batch * n_heads <= 64) ? 1 : 2;
 }
 
-int attn_splits(int batch, int n_heads, int n_kv, int capacity) {
+// One sequence on the grouped kernel (query / key norms): its kv heads are few workgroups (4 kv heads of 8 query heads: 8, 16.3 us a launch at context 500), so that its
+// context is split from the shortest cache on, 32 positions a slice.  Whole | split, 24 tokens of 6 such layers, ms: context 130 13.45 | 13.22,
+// 330 13.77 | 13.45, 620 14.6 | 13.5, 920 15.6 (slices of 128) | 13.5.  Batches keep the rule below: their sequences are workgroups, and a stack of layers
+// would carry every changed rounding on.
+int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
   const int rep = n_heads / n_kv;
   static const int force_r = gbx::env_switch("GBX_ATTN_SPLIT_R");   // tuning aid
   const int R = force_r ? force_r : split_heads(batch, n_heads, rep, capacity);
   const int wgs = n_kv * (rep / R) * batch;
   static const int min_cap = gbx::env_switch("GBX_ATTN_SPLIT_MIN");   // tuning aid
-  if (capacity < min_cap) return 1;                    // short caches: the un-split kernels win (649 vs 774 tok/s at context 128)
   static const int div = gbx::env_switch("GBX_ATTN_SPLIT_DIV");     // tuning aid
-  int s = std::min(std::min(512 / std::max(wgs, 1), capacity / div), 32);
+  const bool one = grouped && batch == 1 && n_kv <= 4 && capacity <= 1536;
+  if (capacity < (one ? 64 : min_cap)) return 1;       // short caches: the un-split kernels win (649 vs 774 tok/s at context 128)
+  int s = std::min(std::min(512 / std::max(wgs, 1), capacity / (one ? 32 : div)), 32);
   return s < 2 ? 1 : s;
 }
 
 size_t attn_workspace_bytes(int batch, int n_heads, int n_kv, int head_dim, int capacity) {
-  const int s = attn_splits(batch, n_heads, n_kv, capacity);
+  const int s = attn_splits(batch, n_heads, n_kv, capacity, true);       // (never fewer than without the norms)
   return s > 1 ? static_cast<size_t>(batch) * n_heads * s * (head_dim + 2) * sizeof(float) : 0;
 }
 
@@ -707,7 +712,7 @@ hipError_t launch_attn_decode(const void* q, const void* k, const void* v, void*
   a.stamps = stamp_region();
 #endif
   const int rep = n_heads / n_kv;
-  const int splits = ws ? attn_splits(batch, n_heads, n_kv, capacity) : 1;
+  const int splits = ws ? attn_splits(batch, n_heads, n_kv, capacity, q_norm_w || q_bias || qkv_ws) : 1;
   if (splits > 1) a.ws = ws;
   if (qkv_ws) {
     a.qkv_ws = qkv_ws; a.qkv_slices = qkv_slices;

@@ -121,7 +121,7 @@ hipError_t launch_attn_decode(const void* q, const void* k, const void* v, void*
                               const void* q_norm_w = nullptr, const void* k_norm_w = nullptr, float norm_eps = 0.f,
                               const void* q_bias = nullptr, const void* k_bias = nullptr, const void* v_bias = nullptr,
                               float* ws = nullptr, const float* qkv_ws = nullptr, int qkv_slices = 0);
-int attn_splits(int batch, int n_heads, int n_kv, int capacity);
+int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped);
 // p2p_allreduce.hip: one-shot push all-reduce of a short 16-bit vector over peer-mapped inboxes
 hipError_t launch_p2p_allreduce(void* x, int n, int rank, int world, void* const* inbox, int cap, void* state, bool bf16, hipStream_t s);
 // attn_oproj.hip: attention + o_proj slices of one decode token in one launch (short caches)

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(NT) void embed_kernel(const T* __restrict__ table, 
 // from the L2 that the first pass filled.  Rows with an infinite maximum are summed unshifted, so that they come out as the definition has it.
 // A few long rows are bound by the vector instructions of the few CUs that hold them (one row of 128 256 bf16 logits: 22 us): slices of a row are
 // then workgroups of their own that leave (maximum, sum) in the first of two launches and write their slice in the second.
-// Replaces torch's logsumexp and subtraction, some ten launches: 1 x 32 000 fp32 40 -> 7 us, 32 x 32 000 fp32 40 -> 8, 1 x 128 256 bf16 62 -> 12.
+// Replaces torch's logsumexp and subtraction, some ten launches: 1 x 32 000 fp32 40 -> 5.5 us, 32 x 32 000 fp32 40 -> 8, 1 x 128 256 bf16 62 -> 5.6.
 constexpr int LSM_NT = 1024, LSM_VR = 8;
 
 template <typename T> __device__ __forceinline__ float lsm_get(const uint4& v, int j) {
@@ -63,47 +63,82 @@ template <typename T> __device__ __forceinline__ float lsm_round(float f) {
   }
 }
 
-constexpr int LSM_SLICE = 8192;                              // logits per workgroup of the sliced form
+// Few long rows: 8 logits a thread, as many workgroups as that makes, whose (maximum, sum) pairs the second launch puts together.  Slices of 8192 in loads of one
+// logit left 19 workgroups with 32 round trips' worth of requests each: 1 x 151 936 bf16 12.4 -> 5.6 us, 8 x 128 256 12.1 -> 6.2, and 1 x 32 000 fp32 7.1 (one workgroup) -> 5.5; 20 000 5.4 in one launch, 5.5 in two.
+constexpr int LSM_SLICE = 2048;
+
+template <typename T>
+__device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int n, int vec, float* v) {
+  if (vec) {                                                  // (n is a multiple of 8: all of them are in the row, or none)
+    constexpr int PER = 16 / sizeof(T);
+    uint4 u[8 / PER];
+#pragma unroll
+    for (int i = 0; i < 8 / PER; ++i) u[i] = *reinterpret_cast<const uint4*>(row + min(k, n - 8) + i * PER);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = k < n ? lsm_get<T>(u[j / PER], j % PER) : -INFINITY;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = k + j < n ? static_cast<float>(row[k + j]) : -INFINITY;
+  }
+}
 
 // (maximum, sum of exponentials against it or against 0 where it is infinite) of one slice
 template <typename T>
-__global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n) {
-  __shared__ float red[4];
-  const T* row = x + static_cast<int64_t>(blockIdx.y) * n;
-  const int lo = blockIdx.x * LSM_SLICE, hi = min(lo + LSM_SLICE, n);
-  float v[LSM_SLICE / 256], m = -INFINITY, s = 0.f;
+__global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n, int vec) {
+  __shared__ float top[4], red[4];
+  const int k = blockIdx.x * LSM_SLICE + threadIdx.x * 8;
+  float v[8], m = -INFINITY, s = 0.f;
+  lsm_load8(x + static_cast<int64_t>(blockIdx.y) * n, k, n, vec, v);
 #pragma unroll
-  for (int i = 0; i < LSM_SLICE / 256; ++i) {
-    const int k = lo + threadIdx.x + i * 256;
-    v[i] = k < hi ? static_cast<float>(row[k]) : -INFINITY;
-    m = fmaxf(m, v[i]);
-  }
+  for (int j = 0; j < 8; ++j) m = fmaxf(m, v[j]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
   __syncthreads();
-  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  m = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
   const float shift = isinf(m) ? 0.f : m;
 #pragma unroll
-  for (int i = 0; i < LSM_SLICE / 256; ++i) s += lo + static_cast<int>(threadIdx.x) + i * 256 < hi ? expf(v[i] - shift) : 0.f;
+  for (int j = 0; j < 8; ++j) s += k + j < n ? expf(v[j] - shift) : 0.f;
   s = block_sum<4>(s, red);
   if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = float2{m, s};
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, T* __restrict__ out, int n) {
+__global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, T* __restrict__ out, int n, int vec) {
+  __shared__ float top[4], red[4];
   const float2* p = part + blockIdx.y * gridDim.x;
-  float m = -INFINITY, s = 0.f;
-  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) m = fmaxf(m, p[i].x);
+  const int parts = gridDim.x, k = blockIdx.x * LSM_SLICE + threadIdx.x * 8;
+  const int64_t base = static_cast<int64_t>(blockIdx.y) * n;
+  float v[8], m = -INFINITY, s = 0.f;
+  lsm_load8(x + base, k, n, vec, v);
+  for (int i = threadIdx.x; i < parts; i += 256) m = fmaxf(m, p[i].x);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
   const float shift = isinf(m) ? 0.f : m;
   // (an infinite maximum: the slice's sum is 0, infinite or no number against any shift -- the shift's own exponential may be infinite, and 0 times that is
   // no number)
-  for (int i = 0; i < static_cast<int>(gridDim.x); ++i) s += isinf(p[i].x) ? p[i].y : p[i].y * expf(p[i].x - shift);
-  const float lse = lsm_round<T>(logf(s) + shift);
-  const int lo = blockIdx.x * LSM_SLICE, hi = min(lo + LSM_SLICE, n);
-  const int64_t base = static_cast<int64_t>(blockIdx.y) * n;
-#pragma unroll 8
-  for (int k = lo + threadIdx.x; k < hi; k += 256) out[base + k] = static_cast<T>(static_cast<float>(x[base + k]) - lse);
+  for (int i = threadIdx.x; i < parts; i += 256) s += isinf(p[i].x) ? p[i].y : p[i].y * expf(p[i].x - shift);
+  const float lse = lsm_round<T>(logf(block_sum<4>(s, red)) + shift);
+  if (vec) {
+    if (k >= n) return;
+    if constexpr (sizeof(T) == 4) {
+      float* o = reinterpret_cast<float*>(out) + base + k;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<float4*>(o + 4 * i) = float4{v[4 * i] - lse, v[4 * i + 1] - lse, v[4 * i + 2] - lse, v[4 * i + 3] - lse};
+    } else {
+      unsigned w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = static_cast<unsigned>(lsm_bits<T>(v[2 * j] - lse)) | (static_cast<unsigned>(lsm_bits<T>(v[2 * j + 1] - lse)) << 16);
+      *reinterpret_cast<uint4*>(out + base + k) = uint4{w[0], w[1], w[2], w[3]};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k + j < n) out[base + k + j] = static_cast<T>(v[j] - lse);
+  }
 }
 
 template <typename T>
@@ -179,13 +214,15 @@ void launch_log_softmax(const void* x, void* out, int64_t rows, int n, float* pa
   constexpr int PER = 16 / sizeof(T);
   const T* xt = static_cast<const T*>(x);
   T* ot = static_cast<T*>(out);
+  const bool aligned = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   if (part) {
     const dim3 grid((n + LSM_SLICE - 1) / LSM_SLICE, static_cast<unsigned>(rows));
-    log_softmax_slice_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<float2*>(part), n);
-    log_softmax_write_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<const float2*>(part), ot, n);
+    const int vec = aligned && n % 8 == 0;
+    log_softmax_slice_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<float2*>(part), n, vec);
+    log_softmax_write_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<const float2*>(part), ot, n, vec);
     return;
   }
-  const int vec = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0 && (rows == 1 || n % PER == 0);
+  const int vec = aligned && (rows == 1 || n % PER == 0);
   log_softmax_kernel<T><<<static_cast<unsigned>(rows), LSM_NT, 0, s>>>(xt, ot, n, vec);
 }
 
@@ -428,8 +465,8 @@ int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* 
 }
 
 extern "C" size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n) {
-  // few rows (at sixteen and more the one-launch form keeps as many CUs busy as this one does at its least) that are long
-  return rows > 0 && rows < 16 && n >= 4 * LSM_SLICE + 1 ? static_cast<size_t>(rows) * ((n + LSM_SLICE - 1) / LSM_SLICE) * 8 : 0;
+  // few rows that are long: sixteen and more keep that many CUs busy in the one-launch form, shorter ones are done there before a second launch would start
+  return rows > 0 && rows < 16 && n > 12 * LSM_SLICE ? static_cast<size_t>(rows) * ((n + LSM_SLICE - 1) / LSM_SLICE) * 8 : 0;
 }
 
 extern "C" int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream) {
