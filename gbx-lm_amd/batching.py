@@ -76,7 +76,15 @@ class _DecodeGraph:
         self.words = b + 2 * b + b + b
         self.static = torch.zeros((self.words,), dtype=torch.int64, device=dev)
         self.pinned = [torch.zeros((self.words,), dtype=torch.int64, pin_memory=True) for _ in range(2)]
-        self.copied = [None, None]
+        self.views = []                                  # per host buffer: tokens, and the places of the positions; the rest never changes
+        for host in self.pinned:
+            a64 = host.numpy()
+            a32 = a64.view("int32")
+            seq, tok, tiles = a32[2 * b:6 * b].reshape(b, 4), a32[6 * b:8 * b].reshape(b, 2), a32[8 * b:10 * b].reshape(b, 2)
+            seq[:, 0], seq[:, 2], seq[:, 3] = slots, 1, range(b)
+            tok[:, 0] = tiles[:, 0] = range(b)
+            self.views.append((a64[:b], seq[:, 1], tok[:, 1]))
+        self.copied = [torch.cuda.Event() for _ in range(2)]           # (an event that was never recorded has passed)
         self.turn = 0
         i32 = self.static.view(torch.int32)
         self.tokens = self.static[:b]
@@ -88,17 +96,11 @@ class _DecodeGraph:
     def fill(self, tokens: Sequence[int], pos0: Sequence[int]) -> None:
         k = self.turn % 2
         self.turn += 1
-        if self.copied[k] is not None:
-            self.copied[k].synchronize()                 # the copy that last read this host buffer has run
-        host = self.pinned[k]
-        b = len(self.slots)
-        host[:b] = torch.tensor(tokens, dtype=torch.int64)
-        i32 = host.view(torch.int32)
-        i32[2 * b:6 * b] = torch.tensor([v for i, (s, p) in enumerate(zip(self.slots, pos0)) for v in (s, p, 1, i)], dtype=torch.int32)
-        i32[6 * b:8 * b] = torch.tensor([v for i, p in enumerate(pos0) for v in (i, p)], dtype=torch.int32)
-        i32[8 * b:10 * b] = torch.tensor([v for i in range(b) for v in (i, 0)], dtype=torch.int32)
-        self.static.copy_(host, non_blocking=True)
-        self.copied[k] = torch.cuda.Event()
+        self.copied[k].synchronize()                     # the copy that last read this host buffer has run
+        words, seq_pos, tok_pos = self.views[k]
+        words[:] = tokens
+        seq_pos[:] = tok_pos[:] = pos0
+        self.static.copy_(self.pinned[k], non_blocking=True)
         self.copied[k].record(torch.cuda.current_stream(self.static.device))
         self.batch.pos0 = list(pos0)
 
@@ -143,6 +145,10 @@ class BatchScheduler:
         """``entries``: (sequence id, next tokens); an id not seen before starts a sequence at position 0.  ``want[i]``: places among
         entry i's tokens whose logits are returned (default: the last one), in the order of entries and places.  Returns fp32
         [wanted, vocab]."""
+        return self._step(entries, want)
+
+    def _step(self, entries, want=None, keep: bool = True) -> torch.Tensor:
+        """``keep`` False: the caller is done with the logits before the next step, whose replay may overwrite them."""
         if not entries:
             return torch.empty((0, 0))
         new_tokens = sum(len(t) for _, t in entries)
@@ -167,7 +173,7 @@ class BatchScheduler:
                 if not rows:
                     return torch.empty((0, self.model.args.vocab), dtype=torch.float32, device=self.device)
                 if len(rows) == len(slot):
-                    return logits.float() if logits.dtype != torch.float32 else logits.clone()      # (the graph's buffer is overwritten by the next replay)
+                    return logits.float() if logits.dtype != torch.float32 else logits.clone() if keep else logits      # (the graph's buffer is overwritten by the next replay)
                 return logits.index_select(0, torch.tensor(rows, dtype=torch.long, device=self.device)).float()
         batch = StepBatch.build(slot, pos0, n_new, self.device)
         tokens = torch.tensor([t for _, ts in entries for t in ts], dtype=torch.long)
@@ -230,8 +236,7 @@ class BatchScheduler:
         live = list(range(len(prompts)))
         feed = {i: list(prompts[i]) for i in live}
         while live:
-            logits = self.step([(ids[i], feed[i]) for i in live])
-            logprobs = log_probabilities(logits)
+            logprobs = log_probabilities(self._step([(ids[i], feed[i]) for i in live], keep=False))      # (a tensor of its own)
             toks = sampler(logprobs).reshape(-1).tolist()
             nxt = []
             for i, t in zip(live, toks):
