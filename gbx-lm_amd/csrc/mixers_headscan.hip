@@ -75,6 +75,66 @@ __global__ __launch_bounds__(NT) void ssm_prepare_kernel(gbxm_ssm_prepare_args p
   }
 }
 
+// Portions, four taps: a thread takes four neighbouring channels of R neighbouring rows of the step, reads every input once and not once per tap, and its taps once.
+// The sums run as above.  Measured, us: 8 192 rows of 4 352 channels 94 -> 45, 2 777 of 6 144 54 -> 29.
+template <typename T, bool FAST, int R>
+__global__ __launch_bounds__(NT) void ssm_prepare_rows_kernel(gbxm_ssm_prepare_args p) {
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * R;
+  const int n = static_cast<int>(min(static_cast<int64_t>(R), p.T - t0)), C = p.C;
+  const T* __restrict__ y = static_cast<const T*>(p.y);
+  const int c = (blockIdx.y * NT + threadIdx.x) * 4;
+  if (c < C) {
+    const T* __restrict__ x0 = y + p.off_x + c;
+    T* __restrict__ out = static_cast<T*>(p.out) + t0 * C + c;
+    float x[R][4], w[4][4], h[3][4], bias[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < R; ++i) Lanes<T, 4>::load(x0 + (t0 + min(i, n - 1)) * p.y_stride, x[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) Lanes<T, 4>::load(static_cast<const T*>(p.conv) + static_cast<int64_t>(j) * C + c, w[j]);
+    if (p.bias) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) bias[k] = p.bias[c + k];
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (i >= n) break;
+      const int b = p.tok[2 * (t0 + i)], pos = p.tok[2 * (t0 + i) + 1], pos0 = p.seq[4 * b + 1];
+      if (i == 0 || pos == pos0) {                           // the three inputs before this row: of the step, of the slot, or none
+        const int64_t row0 = p.seq[4 * b + 3];
+        const T* tail = static_cast<const T*>(p.tail) + static_cast<int64_t>(p.seq[4 * b]) * 3 * C + c;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const int src = pos - 3 + j;
+          Lanes<T, 4>::load(src >= pos0 ? x0 + (row0 + (src - pos0)) * p.y_stride : tail + static_cast<int64_t>(max(src - pos0 + 3, 0)) * C, h[j]);
+          if (src < 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) h[j][k] = 0.f;
+          }
+        }
+      }
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float acc = bias[k] + w[0][k] * h[0][k];
+        acc += w[1][k] * h[1][k];
+        acc += w[2][k] * h[2][k];
+        acc += w[3][k] * x[i][k];
+        v[k] = acc * sigmoid_<FAST>(acc);
+        h[0][k] = h[1][k]; h[1][k] = h[2][k]; h[2][k] = x[i][k];
+      }
+      Lanes<T, 4>::store(out + static_cast<int64_t>(i) * C, v);
+    }
+  }
+  if (blockIdx.y == gridDim.y - 1)
+    for (int i = threadIdx.x; i < n * p.H; i += NT) {
+      const int64_t t = t0 + i / p.H;
+      const int hd = i % p.H;
+      const float z = to_f32(y[t * p.y_stride + p.off_dt + hd]) + p.dt_bias[hd], u = z > 20.f ? z : log1pf(expf(z));
+      p.dt_out[t * 2 * p.H + hd] = -p.rate[hd] * u;
+      p.dt_out[t * 2 * p.H + p.H + hd] = u;
+    }
+}
+
 // Sum over the 16 lanes of a row; every lane of the row gets the same bits.
 __device__ __forceinline__ float row16_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
@@ -311,11 +371,56 @@ __global__ __launch_bounds__(NTH) void gate_group_norm_kernel(const float* __res
   for (int c = threadIdx.x + GR * NTH; c < size; c += NTH) y[c] = from_f32<T>(value(c) * r * w[first + c]);
 }
 
+// The same in groups of four channels, parts of up to 4 NTH V channels.  Measured, us: 8 192 rows of 4 096 in one part 70 -> 40, in eight 82 -> 64.
+template <typename T, bool FAST, int NTH, int V>
+__global__ __launch_bounds__(NTH) void gate_group_norm_vec_kernel(const float* __restrict__ o, const T* __restrict__ z, int64_t z_stride, const float* __restrict__ w,
+                                                                 T* __restrict__ out, int64_t out_stride, int groups, int size, float eps) {
+  __shared__ float red[NTH / 64];
+  const int64_t t = blockIdx.x;
+  const int first = blockIdx.y * size;
+  const float* x = o + t * groups * size + first;
+  const T* zr = z + t * z_stride + first;
+  float v[V][4], g[V][4], m[V][4], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = min((static_cast<int>(threadIdx.x) + i * NTH) * 4, size - 4);
+    Lanes<float, 4>::load(x + c, v[i]);
+    Lanes<T, 4>::load(zr + c, g[i]);
+    Lanes<float, 4>::load(w + first + c, m[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const bool in = (static_cast<int>(threadIdx.x) + i * NTH) * 4 < size;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[i][k] *= g[i][k] * sigmoid_<FAST>(g[i][k]);
+      ss += in ? v[i][k] * v[i][k] : 0.f;
+    }
+  }
+  ss = block_sum<NTH / 64>(ss, red);
+  const float r = 1.f / sqrtf(ss / size + eps);
+  T* y = out + t * out_stride + first;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = (static_cast<int>(threadIdx.x) + i * NTH) * 4;
+    if (c >= size) break;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[i][k] = v[i][k] * r * m[i][k];
+    Lanes<T, 4>::store(y + c, v[i]);
+  }
+}
+
 template <typename T, bool FAST>
 int launch_gate_norm(const float* o, const void* z, int64_t zs, const float* w, void* out, int64_t os, int64_t T_, int groups, int size, float eps, hipStream_t s) {
   const dim3 grid(T_, groups);
   const T* zp = static_cast<const T*>(z);
   T* op = static_cast<T*>(out);
+  if (size % 4 == 0 && size <= 4096 && zs % 4 == 0 && os % 4 == 0 && all_aligned(4 * sizeof(T), zp, static_cast<const T*>(op)) && all_aligned(16, o, w)) {
+    if (size <= 256) gate_group_norm_vec_kernel<T, FAST, 64, 1><<<grid, 64, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
+    else if (size <= 1024) gate_group_norm_vec_kernel<T, FAST, 128, 2><<<grid, 128, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
+    else gate_group_norm_vec_kernel<T, FAST, 256, 4><<<grid, 256, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
+    return after_launch("gate_group_norm");
+  }
   if (size <= 256) gate_group_norm_kernel<T, FAST, 64><<<grid, 64, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
   else if (size <= 1024) gate_group_norm_kernel<T, FAST, 128><<<grid, 128, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
   else gate_group_norm_kernel<T, FAST, 256><<<grid, 256, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
@@ -348,6 +453,12 @@ int gbxm_ssm_prepare(const gbxm_ssm_prepare_args* a, void* stream) {
   const bool vec = a->C % 4 == 0 && a->off_x % 4 == 0 && a->y_stride % 4 == 0 && aligned(a->y, vb) && aligned(a->conv, vb) && aligned(a->out, vb) &&
                    (a->taps == 1 || aligned(a->tail, vb));
   const int64_t work = (a->C / (vec ? 4 : 1) + NT - 1) / NT;              // workgroups a row can feed
+  if (vec && a->taps == 4 && !a->move_tail && a->T * work >= 8 * 1024 && work <= 65535) {
+    const dim3 tiles((a->T + 7) / 8, static_cast<unsigned>(work));
+    if (a->act == GBXM_BF16) ssm_prepare_rows_kernel<bf16_t, true, 8><<<tiles, NT, 0, s>>>(*a);
+    else ssm_prepare_rows_kernel<float, false, 8><<<tiles, NT, 0, s>>>(*a);
+    return after_launch("ssm_prepare (rows)");
+  }
   const unsigned splits = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(work, (2048 + a->T - 1) / a->T)));
   const dim3 grid(a->T, splits);
   if (a->act == GBXM_BF16) {
