@@ -419,6 +419,7 @@ def mixers() -> ctypes.CDLL:
         i64, i32, p, f32, sz = ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p, ctypes.c_float, ctypes.c_size_t
         L.gbxm_version.restype = ctypes.c_int
         L.gbxm_last_error.restype = ctypes.c_char_p
+        L.gbxm_step_tables.argtypes = [p, p, p, p, i32, i32, i32, i32, p]
         L.gbxm_embed_scaled.argtypes = [p, p, p, p, i64, i64, i32, f32, i32, p]
         L.gbxm_segment_rmsnorm.argtypes = [p, i64, i64, i32, i32, p, p, f32, i32, p]
         L.gbxm_residual_norm_add.argtypes = [p, p, p, p, p, i64, i32, i32, f32, f32, i32, p]

@@ -11,6 +11,7 @@ descriptor tables built here once per step (one host-to-device copy).
 """
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass, field
 from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
 
@@ -46,21 +47,30 @@ class StepBatch:
 
     @staticmethod
     def build(slot: Sequence[int], pos0: Sequence[int], n_new: Sequence[int], device, q_tile: int = 128) -> "StepBatch":
-        rows, seq, tok, tiles = 0, [], [], []
-        for b, (s, p, n) in enumerate(zip(slot, pos0, n_new)):
+        rows, seq, tile0, n_tiles = 0, [], [], 0
+        for s, p, n in zip(slot, pos0, n_new):
             if n <= 0:
                 raise ValueError("a sequence of a step brings at least one token")
-            seq.append((s, p, n, rows))
-            tok.extend((b, p + i) for i in range(n))
-            tiles.extend((b, t) for t in range(0, n, q_tile))
+            seq += (s, p, n, rows)
+            tile0.append(n_tiles)
             rows += n
-        packed = torch.tensor([v for r in seq for v in r] + [v for r in tok for v in r] + [v for r in tiles for v in r],
-                              dtype=torch.int32)
-        if torch.device(device).type == "cuda":
-            packed = packed.pin_memory().to(device, non_blocking=True)
-        nb, nt = len(seq), len(tok)
-        return StepBatch(list(slot), list(pos0), list(n_new), rows, packed[:4 * nb].view(nb, 4),
-                         packed[4 * nb:4 * nb + 2 * nt].view(nt, 2), q_tile, packed[4 * nb + 2 * nt:].view(-1, 2))
+            n_tiles += -(-n // q_tile)
+        nb, dev = len(tile0), torch.device(device)
+        head = torch.tensor(seq + tile0, dtype=torch.int32)
+        if dev.type == "cuda":                          # the tables of rows and tiles are written on the device
+            head = head.pin_memory().to(dev, non_blocking=True)
+            tables = torch.empty((2 * (rows + n_tiles),), dtype=torch.int32, device=dev)
+            tok, tiles = tables[:2 * rows].view(rows, 2), tables[2 * rows:].view(n_tiles, 2)
+            if nb:
+                from . import _lib, ops
+                _lib.check_mixers(_lib.mixers().gbxm_step_tables(head.data_ptr(), head.data_ptr() + 16 * nb, tok.data_ptr(), tiles.data_ptr(), nb, rows, n_tiles, q_tile,
+                                                                 ops._stream_ptr(tables.device)))
+        else:
+            firsts, counts = head[:4 * nb].view(nb, 4), torch.tensor([-(-n // q_tile) for n in n_new], dtype=torch.long)
+            b, t = (torch.repeat_interleave(torch.arange(nb, dtype=torch.int32), c) for c in (firsts[:, 2].long(), counts))
+            tok = torch.stack([b, firsts[b.long(), 1] + torch.arange(rows, dtype=torch.int32) - firsts[b.long(), 3]], 1)
+            tiles = torch.stack([t, (torch.arange(n_tiles, dtype=torch.int32) - head[4 * nb:][t.long()]) * q_tile], 1)
+        return StepBatch(list(slot), list(pos0), list(n_new), rows, head[:4 * nb].view(nb, 4), tok, q_tile, tiles)
 
 
 class _DecodeGraph:
@@ -176,7 +186,13 @@ class BatchScheduler:
                     return logits.float() if logits.dtype != torch.float32 else logits.clone() if keep else logits      # (the graph's buffer is overwritten by the next replay)
                 return logits.index_select(0, torch.tensor(rows, dtype=torch.long, device=self.device)).float()
         batch = StepBatch.build(slot, pos0, n_new, self.device)
-        tokens = torch.tensor([t for _, ts in entries for t in ts], dtype=torch.long)
+        try:
+            flat = array("q")
+            for _, ts in entries:
+                flat.extend(ts)
+            tokens = torch.frombuffer(flat, dtype=torch.long)
+        except TypeError:                               # not whole numbers: torch's conversion
+            tokens = torch.tensor([t for _, ts in entries for t in ts], dtype=torch.long)
         if self.device.type == "cuda":
             tokens = tokens.pin_memory().to(self.device, non_blocking=True)
         hidden = self.model.forward_tokens(tokens, batch, self.caches)
