@@ -2,7 +2,7 @@
 // prefill path (mfma_gemm.hip: launch_qgemm_dense).  The weights arrive already dequantised to the activation dtype
 // (gbx_dequantize arithmetic: fields -> fp32, w = s*q + z, one rounding), so this is a plain 16-bit GEMM and the kernel can
 // spend everything on keeping the matrix pipe fed:
-//   * workgroup tile 256 x 256, K tiles of 64, 8 waves as 2 (M) x 4 (N), a wave owns 128 x 64 = 8 x 4 accumulators of
+//   * workgroup tile 256 x 256 (or 192 in either direction: gemm_dense_shape), K tiles of 64, 8 waves as 2 (M) x 4 (N), a wave owns 128 x 64 = 8 x 4 accumulators of
 //     v_mfma_f32_16x16x32 (128 VGPRs) -- the 256^2 "8-phase" structure of cdna_hip_programming.md section 5;
 //   * both operands go HBM/L2 -> LDS by LDS-DMA (`buffer_load_dwordx4 ... lds`, no VGPR staging, no ds_write pass), four
 //     16 KB half-tiles per K tile (A rows 0-127 / 128-255, B rows 0-127 / 128-255), two K tiles of LDS (128 KB);
@@ -25,11 +25,9 @@ namespace gbx {
 
 namespace {
 
-constexpr int DT = 256;            // tile edge (M and N)
+constexpr int DT = 256;            // tile edge (M and N) of the widest shape
 constexpr int DK = 64;             // K tile
-constexpr int HALF = 128 * DK * 2; // bytes of one half-tile (128 rows x 64 k)
-constexpr int TILE_LDS = 4 * HALF; // A-lo | A-hi | B-lo | B-hi
-constexpr int DENSE_LDS = 8 * 128 * 144;   // 2 K tiles (131072 B) during the loop; 8 wave-private 128 x 144 B output tiles in the epilogue
+constexpr int HALF = 128 * DK * 2; // bytes of 128 rows x 64 k
 
 #define DLDSP(p) ((__attribute__((address_space(3))) void*)(p))
 __device__ __forceinline__ constexpr int wc_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
@@ -48,8 +46,20 @@ struct DenseArgs2 {
   int ksplit;
 };
 
-template <bool BF16>
+// Tiles of 32 RT x 64 CT: a wave owns 16 RT rows and 16 CT columns; of an operand with 192 rows a tile (RT = 6, CT = 3) the second request is 64 rows.
+template <int RT, int CT> struct DenseShape {
+  static constexpr int TM = 32 * RT, TN = 64 * CT;
+  static constexpr int B0 = TM * DK * 2;             // LDS: TM rows of x | TN rows of w
+  static constexpr int TILE_LDS = (TM + TN) * DK * 2;
+  static constexpr int EROW = 32 * CT + 16;          // epilogue: a wave's own 16 RT x 16 CT outputs
+  static constexpr int LDS = 2 * TILE_LDS > 8 * 16 * RT * EROW ? 2 * TILE_LDS : 8 * 16 * RT * EROW;
+  static constexpr int A2 = RT == 8 ? 2 : 1, B2 = CT == 4 ? 2 : 1;                // requests of a thread for rows 128 on
+};
+
+template <bool BF16, int RT, int CT>
 __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
+  typedef DenseShape<RT, CT> Shape;
+  constexpr int TM = Shape::TM, TN = Shape::TN, TILE_LDS = Shape::TILE_LDS, A2 = Shape::A2, B2 = Shape::B2, RH = RT / 2, C0 = 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -59,12 +69,12 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
   const int nk = K / DK / ksplit;                    // K tiles of this workgroup's slice
 
   // XCD-aware tile order (as mfma_gemm.hip): every XCD walks a contiguous run of (tile, k slice) units, M-tile major
-  const int tiles_n = (N + DT - 1) / DT, tiles_m = (M + DT - 1) / DT, tiles = tiles_m * tiles_n * ksplit;
+  const int tiles_n = (N + TN - 1) / TN, tiles_m = (M + TM - 1) / TM, tiles = tiles_m * tiles_n * ksplit;
   const int per_xcd = (tiles + 7) / 8;
   const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (unit >= tiles) return;
   const int tile = unit / ksplit, kslice = unit % ksplit;
-  const int m0 = (tile / tiles_n) * DT, n0 = (tile % tiles_n) * DT;
+  const int m0 = (tile / tiles_n) * TM, n0 = (tile % tiles_n) * TN;
   const int kbase = kslice * nk * (DK * 2);          // byte offset of the slice inside a row
 
   // ---- DMA side: piece p = tid + 512 i (i = 0, 1) of a half-tile = (row p >> 3, 16-byte column p & 7); LDS linear, the
@@ -85,53 +95,53 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
   // half-tile h (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) of K tile kt -> LDS buffer kt & 1
   auto stage = [&](int kt, int h) {
     const int ktc = min(kt, nk - 1);                 // past the end: re-request the last tile (keeps the vmcnt arithmetic uniform)
-    unsigned char* dst = lds + (kt & 1) * TILE_LDS + h * HALF + dma_lds;
+    unsigned char* dst = lds + (kt & 1) * TILE_LDS + (h < 2 ? 0 : Shape::B0) + (h & 1) * HALF + dma_lds;
     const int koff = kbase + ktc * (DK * 2);
     if (h < 2) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, DLDSP(dst), 16, voa[h][0], koff, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, DLDSP(dst + 8192), 16, voa[h][1], koff, 0, 0);
+      if (h == 0 || A2 == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, DLDSP(dst + 8192), 16, voa[h][1], koff, 0, 0);
     } else {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, DLDSP(dst), 16, vob[h - 2][0], koff, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, DLDSP(dst + 8192), 16, vob[h - 2][1], koff, 0, 0);
+      if (h == 2 || B2 == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, DLDSP(dst + 8192), 16, vob[h - 2][1], koff, 0, 0);
     }
   };
 
   // ---- fragment side: lane = (row l & 15, k block l >> 4) of a 16 x 32 operand; swizzled column
   const int fr = lane & 15, fk = lane >> 4;
   const int sw = (fr >> 1) & 7;
-  const int fa_off = wr * HALF + fr * 128;                          // + rt * 2048 + ((ks * 4 + fk) ^ sw) * 16
-  const int fb_off = (2 + (wcn >> 1)) * HALF + ((wcn & 1) * 64 + fr) * 128;
+  const int fa_off = (wr * 16 * RT + fr) * 128;                     // + rt * 2048 + ((ks * 4 + fk) ^ sw) * 16
+  const int fb_off = Shape::B0 + (wcn * 16 * CT + fr) * 128;
   const int c0 = (fk ^ sw) * 16, c1 = ((4 + fk) ^ sw) * 16;         // k-step 0 / 1 column bytes
-  u32x4 fa[8][2], fb[4][2];
-  auto read_a = [&](const unsigned char* buf, int half) {           // row tiles 4 half .. 4 half + 3
+  u32x4 fa[RT][2], fb[CT][2];
+  auto read_a = [&](const unsigned char* buf, int half) {           // one half of the row tiles
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      fa[half * 4 + rt][0] = *reinterpret_cast<const u32x4*>(buf + fa_off + (half * 4 + rt) * 2048 + c0);
-      fa[half * 4 + rt][1] = *reinterpret_cast<const u32x4*>(buf + fa_off + (half * 4 + rt) * 2048 + c1);
+    for (int rt = half * RH; rt < (half + 1) * RH; ++rt) {
+      fa[rt][0] = *reinterpret_cast<const u32x4*>(buf + fa_off + rt * 2048 + c0);
+      fa[rt][1] = *reinterpret_cast<const u32x4*>(buf + fa_off + rt * 2048 + c1);
     }
   };
-  auto read_b = [&](const unsigned char* buf, int half) {           // column tiles 2 half, 2 half + 1
+  auto read_b = [&](const unsigned char* buf, int half) {           // column tiles 0 and 1, or the rest
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      fb[half * 2 + ct][0] = *reinterpret_cast<const u32x4*>(buf + fb_off + (half * 2 + ct) * 2048 + c0);
-      fb[half * 2 + ct][1] = *reinterpret_cast<const u32x4*>(buf + fb_off + (half * 2 + ct) * 2048 + c1);
+    for (int ct = half * C0; ct < (half ? CT : C0); ++ct) {
+      fb[ct][0] = *reinterpret_cast<const u32x4*>(buf + fb_off + ct * 2048 + c0);
+      fb[ct][1] = *reinterpret_cast<const u32x4*>(buf + fb_off + ct * 2048 + c1);
     }
   };
-  f32x4v acc[8][4];
+  f32x4v acc[RT][CT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4v{0};
+    for (int j = 0; j < CT; ++j) acc[i][j] = f32x4v{0};
   auto quadrant = [&](int ah, int bh) {
 #ifndef DENSE_NOPRIO
     __builtin_amdgcn_s_setprio(1);
 #endif
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = ah * RH; rt < (ah + 1) * RH; ++rt)
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct) {
-        acc[ah * 4 + rt][bh * 2 + ct] = mfma16<BF16>(fa[ah * 4 + rt][0], fb[bh * 2 + ct][0], acc[ah * 4 + rt][bh * 2 + ct]);
-        acc[ah * 4 + rt][bh * 2 + ct] = mfma16<BF16>(fa[ah * 4 + rt][1], fb[bh * 2 + ct][1], acc[ah * 4 + rt][bh * 2 + ct]);
+      for (int ct = bh * C0; ct < (bh ? CT : C0); ++ct) {
+        acc[rt][ct] = mfma16<BF16>(fa[rt][0], fb[ct][0], acc[rt][ct]);
+        acc[rt][ct] = mfma16<BF16>(fa[rt][1], fb[ct][1], acc[rt][ct]);
       }
 #ifndef DENSE_NOPRIO
     __builtin_amdgcn_s_setprio(0);
@@ -143,7 +153,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
   for (int h = 0; h < 4; ++h) stage(0, h);
   stage(1, 0);
   stage(1, 1);
-  __builtin_amdgcn_s_waitcnt(wc_vm(4));              // K tile 0 has landed (this wave's share); tile 1's two may fly
+  __builtin_amdgcn_s_waitcnt(wc_vm(2 + A2));         // K tile 0 has landed (this wave's share); tile 1's two may fly
   bar();
   if (wr == 1) bar();                                // the second wave group runs one barrier interval behind the first
 
@@ -171,9 +181,9 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
     bar();
     quadrant(1, 1);
     bar();
-    // phase 4: quadrant (A1, B0); request half-tile 1 of K tile t+2; K tile t+1 must have landed: all but the 4 youngest DMAs
+    // phase 4: quadrant (A1, B0); request half-tile 1 of K tile t+2; K tile t+1 must have landed: all but the youngest DMAs, tile t+2's of x
     stage(t + 2, 1);
-    __builtin_amdgcn_s_waitcnt(wc_vm(4));
+    __builtin_amdgcn_s_waitcnt(wc_vm(2 + A2));
     bar();
     quadrant(1, 0);
     bar();
@@ -186,7 +196,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
   // lane in 32-byte segments (measured: ~30 us per workgroup, a quarter of the K = 4096 tile).  The wave's 128 x 64 tile
   // goes through its own LDS region instead (rows of 128 B + 16 B pad) and leaves as 16-byte row-contiguous stores.
   bar();                                             // every wave is past its last fragment read / DMA wait: LDS is free
-  if (ksplit > 1) {
+  if constexpr (RT == 8 && CT == 4) if (ksplit > 1) {
     // fp32 partial tile of this k slice, through the wave's own LDS region in two passes of 64 rows (rows of 256 B + 16 B pad)
     // so that it leaves as 16-byte row-contiguous stores
     constexpr int PROW = 64 * 4 + 16;
@@ -224,15 +234,15 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
     }
     return;
   }
-  constexpr int EROW = 144;
-  unsigned char* et = lds + wave * (128 * EROW);
-  const int nb = n0 + wcn * 64, mb = m0 + wr * 128;
+  constexpr int EROW = Shape::EROW;
+  unsigned char* et = lds + wave * (16 * RT * EROW);
+  const int nb = n0 + wcn * 16 * CT, mb = m0 + wr * 16 * RT;
 #pragma unroll
-  for (int ct = 0; ct < 4; ++ct) {
+  for (int ct = 0; ct < CT; ++ct) {
     const int n = min(nb + ct * 16 + fr, N - 1);
     const float b = a.bias ? act_to_f32<BF16>(a.bias[n]) : 0.f;
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {                  // C/D layout of the 16x16 tile: row = 4 (lane >> 4) + e, column = lane & 15
         float v = acc[rt][ct][e];
@@ -241,18 +251,18 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
       }
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);                // the wave's own LDS writes (no other wave touches this region)
-  if (a.swiglu) {
+  if constexpr (CT == 4) if (a.swiglu) {
     // Tile columns 0-127 are gate rows j, columns 128-255 the up rows of the SAME j (waves wcn and wcn + 2 of one wave row):
     // y[m, n0 / 2 + j] = round(round(silu(gate)) * up) on the already rounded GEMM outputs -- the reference's op-by-op
     // roundings (qllama.py:115), what gbx_swiglu computes from the two tensors this epilogue never writes.
     bar();
     const int NO = N >> 1;
-    const unsigned char* gt = lds + (wr * 4 + (wcn & 1)) * (128 * EROW);
-    const unsigned char* ut = lds + (wr * 4 + 2 + (wcn & 1)) * (128 * EROW);
+    const unsigned char* gt = lds + (wr * 4 + (wcn & 1)) * (16 * RT * EROW);
+    const unsigned char* ut = lds + (wr * 4 + 2 + (wcn & 1)) * (16 * RT * EROW);
     const int ob = (n0 >> 1) + (wcn & 1) * 64;       // output column of this wave's piece 0
 #pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int p = it * 64 + lane, row = (wcn >> 1) * 64 + (p >> 3), c = p & 7;
+    for (int it = 0; it < RT; ++it) {
+      const int p = it * 64 + lane, row = (wcn >> 1) * (8 * RT) + (p >> 3), c = p & 7;
       const int m = mb + row;
       if (m >= M) continue;
       const u32x4 gv = *reinterpret_cast<const u32x4*>(gt + row * EROW + c * 16);
@@ -271,10 +281,10 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
     }
     return;
   }
-  const bool full_n = (nb + 64 <= N) && (N % 8 == 0);
+  const bool full_n = (nb + 16 * CT <= N) && (N % 8 == 0);
 #pragma unroll
-  for (int it = 0; it < 16; ++it) {
-    const int p = it * 64 + lane, row = p >> 3, c = p & 7;       // 16-byte piece c of row `row`
+  for (int it = 0; it < RT * CT / 2; ++it) {
+    const int p = it * 64 + lane, row = p / (2 * CT), c = p % (2 * CT);       // 16-byte piece c of row `row`
     const int m = mb + row;
     if (m >= M) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(et + row * EROW + c * 16);
@@ -400,6 +410,42 @@ __global__ __launch_bounds__(NWV * 64) void dense_batch_kernel(const DenseArgs2 
   }
 }
 
+template <int RT, int CT>
+hipError_t launch_dense_tiles(const DenseArgs2& a, bool bf16, hipStream_t s) {
+  typedef DenseShape<RT, CT> Shape;
+  static DeviceOnce once;
+  if (once.pending()) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<true, RT, CT>), hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS);
+    if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<false, RT, CT>), hipFuncAttributeMaxDynamicSharedMemorySize, Shape::LDS);
+    if (e != hipSuccess) return e;
+    once.done();
+  }
+  const int tiles = ((a.N + Shape::TN - 1) / Shape::TN) * ((a.M + Shape::TM - 1) / Shape::TM) * (a.part ? a.ksplit : 1);
+  dim3 grid(8 * ((tiles + 7) / 8)), block(512);
+  if (bf16) hipLaunchKernelGGL((gemm_dense_kernel<true, RT, CT>), grid, block, Shape::LDS, s, a);
+  else hipLaunchKernelGGL((gemm_dense_kernel<false, RT, CT>), grid, block, Shape::LDS, s, a);
+  return hipGetLastError();
+}
+
+// Tile of an unsplit product: the shape whose rounds of 256 workgroups take least.  Cost of a full round against 256 x 256, and of a last round of n workgroups:
+// 0.62 + 0.38 n / 256 of a full one (what is alone on the chip runs faster).  Every output sums its products in the same order in all four.  Measured, us, 256 x 256 | 256 x 192 |
+// 192 x 256 | 192 x 192: 3001 x 3072, K 3072 69 | 60 | 60 | 55, K 8192 173 | 160 | 161 | 152; 3001 x 5120, K 3072 82 | 115 | 109 | 110; 6000 x 4096, K 4096 171 | 214 |
+// 158 | 191; 6000 x 3072, K 8192 315 | 267 | 270 | 249; 2048 x 6144, K 4096 90 | 84 | 136 | 123; 2500 x 28672, K 4096 488 | 512 | 561 | 607.
+int gemm_dense_shape(int M, int N, bool swiglu) {
+  constexpr float cost[4] = {1.f, 0.8f, 0.8f, 0.66f};                    // 256 x 256, 256 x 192, 192 x 256, 192 x 192
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    if (swiglu && (i & 1)) continue;                                     // (gate and up meet in tiles of 256 columns)
+    const int tm = i & 2 ? 192 : 256, tn = i & 1 ? 192 : 256;
+    const long long tiles = static_cast<long long>((N + tn - 1) / tn) * ((M + tm - 1) / tm), rest = tiles % 256;
+    const float t = cost[i] * (tiles / 256 + (rest ? 0.62f + 0.38f * rest / 256 : 0.f));
+    if (i == 0 || t < least) { best = i; least = i == 0 ? 0.97f * t : t; }  // (what gains less than three in a hundred is not sure to gain)
+  }
+  return best;
+}
+
 template <int NWV>
 hipError_t launch_dense_batch_w(const DenseArgs2& a, bool bf16, hipStream_t s) {
   constexpr int LDSB = skinny_lds(NWV);
@@ -453,21 +499,11 @@ hipError_t launch_gemm_dense(const void* x, const void* w, const void* bias, voi
     return launch_dense_batch(a, bf16, s);
   }
   const int ksplit = (part && !swiglu && N % 4 == 0) ? gemm_dense_ksplit(M, N, K) : 1;
-  static DeviceOnce once;
-  if (once.pending()) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, DENSE_LDS);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, DENSE_LDS);
-    if (e != hipSuccess) return e;
-    once.done();
-  }
   DenseArgs2 a{static_cast<const unsigned short*>(x), static_cast<const unsigned short*>(w), static_cast<const unsigned short*>(bias),
                static_cast<unsigned short*>(y), M, N, K, swiglu ? 1 : 0, ksplit > 1 ? part : nullptr, ksplit};
-  const int tiles = ((N + DT - 1) / DT) * ((M + DT - 1) / DT) * ksplit;
-  dim3 grid(8 * ((tiles + 7) / 8)), block(512);
-  if (bf16) hipLaunchKernelGGL((gemm_dense_kernel<true>), grid, block, DENSE_LDS, s, a);
-  else hipLaunchKernelGGL((gemm_dense_kernel<false>), grid, block, DENSE_LDS, s, a);
-  hipError_t e = hipGetLastError();
+  const int shape = ksplit > 1 ? 0 : gemm_dense_shape(M, N, swiglu);
+  const hipError_t e = shape == 0 ? launch_dense_tiles<8, 4>(a, bf16, s) : shape == 1 ? launch_dense_tiles<8, 3>(a, bf16, s)
+                     : shape == 2 ? launch_dense_tiles<6, 4>(a, bf16, s) : launch_dense_tiles<6, 3>(a, bf16, s);
   if (e != hipSuccess || ksplit <= 1) return e;
   return launch_splitk_finish(part, static_cast<const unsigned short*>(bias), static_cast<unsigned short*>(y), ksplit, M, N, bf16, s);
 }
