@@ -14,11 +14,15 @@
 // a barrier apart, so that one group multiplies while the other reads fragments and issues requests.  Stages of 64 elements, because a row
 // piece is then a whole 128-byte line: 256 x 128 tiles with stages of 32 elements and two workgroups per CU spent their time on twice the L2
 // requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
-// Measured (us, first + second products with the sort; before: 128-pair tiles, weight fragments straight from the matrices):
-//   27 848 pairs, 128 experts, 2048 x 768 gated:  1 027 -> 479 (548 TFLOP/s, 2.5 TB/s of weights)
-//   18 128 pairs of the same:                       794 -> 327 (3.7 TB/s)
-//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 856 -> 424
-//    8 192 pairs,   8 experts, 4096 x 2048 gated:   975 -> 472 (873 TFLOP/s)
+// Measured (us, first + second products with the sort; 128-pair tiles and weight fragments straight from the matrices -> 256-pair tiles -> results by rows):
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  1 027 -> 480 -> 462 (570 TFLOP/s, 2.6 TB/s of weights)
+//   18 128 pairs of the same:                       794 -> 357 -> 331 (3.7 TB/s)
+//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 856 -> 422 -> 398; a factor of the weights' way from memory (one expert's for all: 269) and of the results'
+//   (kept back: 324), which tiles of one round write at the same time
+//    8 192 pairs,   8 experts, 4096 x 2048 gated:   975 -> 457 -> 444 (930 TFLOP/s)
+// The table keeps a lower tile beside its expert's others.  By falling height, so that the last round is short, tiles read their weights anew: 256 pairs an
+// expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  Requests of a whole stage ahead, or its lines ordered into L2
+// before, gain nothing.
 // The grid is sized for the worst case sum_e ceil(n_e / 256) <= P / 256 + E; surplus workgroups leave at once.
 // Steps with few pairs per expert (a batch that decodes) stream weights and little else: expert_skinny_kernel takes tiles of 32 pairs, a
 // wave per 32 output channels and no barrier.  A wave moves its own rows -- eight lanes to a row's 128 bytes, so an access touches eight
@@ -110,8 +114,7 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wc = wave & 3;
   const int fr = lane & 15, fk = lane >> 4;
   const int N = a.N, C = a.C, n = (C + 63) >> 6;
-  const int r0 = GATED ? col * 128 : col * 256;                         // the tile's and the wave's first output channel
-  const int c0 = r0 + wc * (GATED ? 32 : 64);
+  const int r0 = GATED ? col * 128 : col * 256;                         // the tile's first output channel
   int* ids = reinterpret_cast<int*>(lds + 2 * GSTAGE);
   float* factor = reinterpret_cast<float*>(ids + GR);
   if (tid < 32 * NR) {
@@ -226,15 +229,15 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
   }
   if (wr == 0) bar();                                                   // the groups' barrier counts match again
   __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(0));                         // no LDS-DMA outlives the workgroup
+  bar();                                                                // every wave is past its last fragment: the stages' LDS is free
+  // The tile's results meet in LDS (16-byte column c of row r at place c ^ (r & 15): neither side meets a bank twice) and leave as whole rows of it
+  constexpr int OPC = GATED ? 16 : 32;                                  // 16-byte columns of a row
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
-    const int at = wr * 16 * NR + i * 16 + fr, row = lo + at;
-    if (row >= hi) continue;
+    const int at = wr * 16 * NR + i * 16 + fr;
     const float sc = factor[at];
-    bf16_t* op = a.out + static_cast<int64_t>(FORM == EXPERT_DOWN ? ids[at] : row) * N + c0 + 4 * fk;
 #pragma unroll
     for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-      if (c0 + j * 16 >= N) break;                                      // (N is a multiple of 32)
       float v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -242,8 +245,19 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
         else if constexpr (FORM == EXPERT_UP) { const float z = fmaxf(sc * acc[i][j][q], 0.f); v[q] = z * z; }
         else v[q] = glu_act<true>(sc * acc[i][j][q], sc * acc[i][j + 2][q], FORM == EXPERT_SILU ? GBXM_GLU_SILU : GBXM_GLU_CLAMPED_SWISH, a.limit, 1.702f);
       }
-      *reinterpret_cast<u32x2*>(op + j * 16) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
+      *reinterpret_cast<u32x2*>(lds + (at * OPC + ((wc * (GATED ? 4 : 8) + j * 2 + (fk >> 1)) ^ fr)) * 16 + (fk & 1) * 8) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
     }
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  bar();
+  const int oc = tid & (OPC - 1), rows = min(hi - lo, 32 * NR);
+  if (r0 + oc * 8 >= N) return;                                         // (N is a multiple of 32)
+#pragma unroll
+  for (int i = 0; i < NR * OPC / 16; ++i) {
+    const int at = i * (512 / OPC) + tid / OPC;
+    if (at >= rows) break;
+    *reinterpret_cast<u32x4*>(a.out + static_cast<int64_t>(FORM == EXPERT_DOWN ? ids[at] : lo + at) * N + r0 + oc * 8) =
+        *reinterpret_cast<const u32x4*>(lds + (at * OPC + (oc ^ (at & 15))) * 16);
   }
 }
 
