@@ -82,3 +82,12 @@ def test_choices_share_rows_across_tiles():
     got = M.expert_glu(h, first, down, idx, "silu", 0.0, None).double()
     want, spread = reference(h, first, down, idx, "silu", 0.0, None)
     assert bool(((got - want).abs() <= 2.0 ** -8 * (want.abs() + spread) * 3 + 1e-6).all())
+
+
+@pytest.mark.parametrize("experts,pairs", [(8, 32768), (8, 32769), (5, 70000), (300, 40000)])
+def test_more_pairs_than_the_sort_keeps(experts, pairs):
+    """The pairs beyond those whose places the sort holds in registers; uneven experts."""
+    w = torch.arange(1, experts + 1, dtype=torch.float64)
+    counts = (w / w.sum() * pairs).long().tolist()
+    counts[-1] += pairs - sum(counts)
+    tiles(counts, "relu2", 32, 32)
