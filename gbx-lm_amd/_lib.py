@@ -468,6 +468,7 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_gate_group_norm.argtypes = [p, p, i64, p, p, i64, i64, i32, i32, f32, i32, p]
         L.gbxm_layer_update.argtypes = [ctypes.POINTER(LayerUpdateArgs), p]
         L.gbxm_router_rows.argtypes = [p, p, p, i64, i32, i32, i32, p]
+        L.gbxm_router_tiles.argtypes = [p, p, p, i64, i32, i32, p]
         L.gbxm_linear_rows.argtypes = [p, i64, p, p, p, i64, i64, i32, i32, p]
         L.gbxm_route_groups.argtypes = [p, i64, p, p, i64, i64, i32, i32, i32, i32, i32, i32, p]
         _mlib = L

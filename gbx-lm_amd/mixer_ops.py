@@ -128,11 +128,15 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) 
 # XCDs' caches do not hold (8 MB) takes it for few products only.  Library with its widened copy | launch, us: 32 rows x 256 x 4096 15.0 | 10.4, x 256 x 7168
 # 21.9 | 16.8, x 1024 x 1024 10.3 | 11.2; 8 MB: 4 x 1024 x 2048 10.2 | 4.6, 8 rows 10.3 | 12.2, 32 rows 11.1 | 19.5; 32 x 1024 x 4096 15.0 | 35.8.
 ROUTER_ROWS, ROUTER_HELD, ROUTER_FEW = 32, 1 << 21, 1 << 23
+# Prompt-sized steps whose bf16 rows the matrix cores take as they are (csrc/mixers_router.hip).  Widened copy and library | this, us, rows x experts x channels:
+# 3481 x 128 x 2048 47.5 | 26.6, 8192 x 64 x 2048 40.3 | 26.5, 8192 x 32 x 1024 25.5 | 12.2, 700 x 256 x 2048 19.4 | 18.1, 16384 x 128 x 2048 99 | 96; outside the rule
+# 300 x 128 x 2048 12.8 | 17.3, 2000 x 256 x 7168 77 | 80, 8192 x 256 x 4096 167 | 181.
+TILE_ROWS, TILE_EXPERTS, TILE_CHANNELS, TILE_LOGITS = 512, 256, 2048, 1 << 21
 
 
 def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
     """fp32 product of the rows (their bf16 image widened, when activations are bf16) with the fp32 router: few rows one HIP launch, prompt-sized
-    steps a widened copy and the vendor library's GEMM (1 row x 32 experts of 1024: 11.7 -> 2.3 us, 32 rows x 128 of 2048:
+    steps another or, by the rules above, a widened copy and the vendor library's GEMM (1 row x 32 experts of 1024: 11.7 -> 2.3 us, 32 rows x 128 of 2048:
     17.4 -> 5.0)."""
     act = _act(h, "h")
     _f32(router, "router")
@@ -142,7 +146,15 @@ def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
         raise RuntimeError(f"rows on {h.device}, router on {router.device}")
     t, rows = h.shape[0], router.shape[0]
     if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1] or (router.numel() >= ROUTER_HELD and t * router.numel() > ROUTER_FEW):
-        return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
+        k = h.shape[1]
+        if h.dtype == torch.float32 or k != router.shape[1] or k % 8 or not 0 < k <= TILE_CHANNELS or rows > TILE_EXPERTS or not TILE_ROWS <= t <= TILE_LOGITS // rows:
+            return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
+        h = h.contiguous()
+        if (h.data_ptr() | router.data_ptr()) % 16:
+            return torch.matmul(h.float(), router.t())
+        logits = torch.empty((t, rows), dtype=torch.float32, device=h.device)
+        _lib.check_mixers(_lib.mixers().gbxm_router_tiles(h.data_ptr(), router.data_ptr(), logits.data_ptr(), t, k, rows, _stream(h.device)))
+        return logits
     h = h.contiguous()
     logits = torch.empty((t, rows), dtype=torch.float32, device=h.device)
     _lib.check_mixers(_lib.mixers().gbxm_router_rows(h.data_ptr(), router.data_ptr(), logits.data_ptr(), t, h.shape[1], rows, act, _stream(h.device)))

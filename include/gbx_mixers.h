@@ -380,6 +380,8 @@ typedef struct {
 int gbxm_layer_update(const gbxm_layer_update_args* a, void* stream);
 /* logits[t][e] = sum_k h[t][k] router[e][k] in fp32, for few rows. */
 int gbxm_router_rows(const void* h, const float* router, float* logits, int64_t T, int32_t K, int32_t E, int32_t act, void* stream);
+/* The same for any number of bf16 rows: K a multiple of 8, operands 16-byte aligned, E K < 2^29. */
+int gbxm_router_tiles(const void* h, const float* router, float* logits, int64_t T, int32_t K, int32_t E, void* stream);
 /* y[t][n] = sum_k x[t][k] w[n][k] (+ bias[n]): bf16 in and out, fp32 sums, T <= 16 rows of K <= 4096 or T <= 32 of K <= 2048, K a multiple of 64;
  * x rows (x_stride elements apart, a multiple of 8) and w [N][K] 16-byte aligned. */
 int gbxm_linear_rows(const void* x, int64_t x_stride, const void* w, const void* bias, void* y, int64_t y_stride, int64_t T, int32_t N, int32_t K,

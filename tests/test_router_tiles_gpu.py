@@ -1,0 +1,28 @@
+"""Router logits of prompt-sized steps on the matrix cores (csrc/mixers_router.hip) at the edges of their tiles: rows and experts off the grid of 16, each
+of the two widths, channels off the block of 32 and fewer blocks than waves, rows that lie apart.  Reference: float64; tolerance: K fp32 roundings of the
+terms' magnitudes.  An infinity stays in its row and an infinity."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("t,k,e", [(512, 8, 1), (513, 40, 5), (540, 256, 32), (600, 264, 33), (700, 1024, 63), (1030, 520, 128), (2050, 2048, 129), (2100, 2040, 256), (5000, 288, 64)])
+@pytest.mark.parametrize("apart", [False, True])
+def test_logits(t, k, e, apart):
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator(device=DEV).manual_seed(t + e)
+    h = torch.randn((t, k + 8 * apart), device=DEV, generator=g).to(torch.bfloat16)[:, :k]
+    router = torch.randn((e, k), device=DEV, generator=g)
+    got = M._router_logits(h, router)
+    want, terms = h.double() @ router.double().t(), h.double().abs() @ router.double().abs().t()
+    assert got.shape == want.shape and got.dtype == torch.float32
+    assert bool(((got.double() - want).abs() <= k * 2.0 ** -24 * terms).all())
+    h = h.clone()
+    h[t // 2, k - 1], h[3, 0] = torch.inf, torch.nan
+    bad = M._router_logits(h, router)
+    rows = torch.ones(t, dtype=torch.bool)
+    rows[[3, t // 2]] = False
+    want = h.float() @ router.t()
+    assert bool(torch.isnan(bad[3]).all()) and torch.equal(bad[t // 2], want[t // 2]) and torch.equal(bad[rows], got[rows])
