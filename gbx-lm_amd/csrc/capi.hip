@@ -407,6 +407,11 @@ size_t gbx_attn_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv_hea
   return gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity);
 }
 
+int32_t gbx_attn_splits(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t capacity, int32_t normed) {
+  if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || capacity <= 0) return 1;
+  return gbx::attn_splits(batch, n_heads, n_kv_heads, capacity, normed != 0);
+}
+
 int gbx_attn_decode_ws(const void* q, const void* k, const void* v, void* kcache, void* vcache, const float* inv_freq,
                        const int64_t* pos, void* out, int32_t batch, int32_t n_heads, int32_t n_kv_heads,
                        int32_t head_dim, int32_t capacity, float rope_scale, float sm_scale, int32_t traditional,

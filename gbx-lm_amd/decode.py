@@ -403,8 +403,12 @@ class FusedDecodeRunner(DecodeRunner):
             self.all_keys = torch.zeros((64 * model.tp_world,), dtype=torch.int64, device=dev)
             self.logits_full = torch.zeros((1, self.tp_vocab[2]), dtype=dt, device=dev)
         from . import _lib as _l
-        need = _l.lib().gbx_attn_workspace_bytes(1, a0.n_heads, a0.n_kv_heads, a0.head_dim, caches[0].capacity)
-        self.attn_ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None   # context split of long caches
+        shape = (1, a0.n_heads, a0.n_kv_heads)
+        normed = any(getattr(b.self_attn, "q_norm", None) is not None or b.self_attn.q_proj.bias is not None for b in model.model.layers)
+        need = _l.lib().gbx_attn_workspace_bytes(*shape, a0.head_dim, caches[0].capacity)
+        split = _l.lib().gbx_attn_splits(*shape, caches[0].capacity, int(normed)) > 1          # the attention launch of its own splits the context
+        self.attn_ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need and split else None
+        self.long_cache = _l.lib().gbx_attn_splits(*shape, caches[0].capacity, 0) > 1          # too long for one workgroup per head's whole context
         self.chain = False                  # True while capturing / replaying the on-device greedy chain
         self.graph_chain = None
         # Short caches (no context split): attention + o_proj as ONE launch whose partial sums land in a fixed-point
@@ -413,7 +417,7 @@ class FusedDecodeRunner(DecodeRunner):
         # hand-off costs what the removed boundary cost (profiles/r03_chain_floor.txt: 750-753 vs 750-762 tok/s).
         import os
         self.acc = torch.zeros((D + a0.n_kv_heads * ops.ATTN_OPROJ_HANDOFF_WORDS,), dtype=torch.int64, device=dev)   # o_proj sums | hand-off words
-        self.fuse_ao = (env.flag("GBX_FUSE_AO") and not tp and self.attn_ws is None and
+        self.fuse_ao = (env.flag("GBX_FUSE_AO") and not tp and not self.long_cache and
                         all(getattr(b.self_attn, "q_norm", None) is None and b.self_attn.q_proj.bias is None and
                             ops.attn_oproj_supported(b.self_attn.n_heads, b.self_attn.n_kv_heads, b.self_attn.head_dim, b.self_attn.o_proj) and
                             b.mlp.gate_proj.group_size >= 64 and
@@ -427,7 +431,7 @@ class FusedDecodeRunner(DecodeRunner):
         # A model whose hand-offs timed out once (decode_fallback) stays on the five-launch block; so does a device that fails the
         # layout check (partition mode, CU mask, a dispatcher that does not deal workgroups round-robin over the XCDs).
         self.use_dattn = (env.flag("GBX_DATTN") and not tp and not self.fuse_ao and env.flag("GBX_DGEMV") and env.flag("GBX_QKV_CAT") and
-                          (self.attn_ws is None or a0.n_heads // a0.n_kv_heads in (3, 4)) and
+                          (not self.long_cache or a0.n_heads // a0.n_kv_heads in (3, 4)) and
                           not getattr(model, "_fused_handoff_disabled", False) and ops.xcd_layout_ok(dev))
         self.use_dmlp = self.use_dattn and env.flag("GBX_DMLP")
         # Round 6: the whole 2-bit block as ONE launch (gbx_dblock_forward) while the context is short enough for the head's own workgroup

@@ -546,6 +546,8 @@ int gbx_attn_decode_normed(const void* q, const void* k, const void* v, void* kc
  * sequence) are split over several workgroups (flash-decoding) and a second launch merges their (max, sum, numerator)
  * partials -- the per-head kernel reads a 2048-token context with 32 workgroups. */
 size_t gbx_attn_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t capacity);
+/* Slices that such a launch splits the context into (1: it does not); normed: with query / key norms or biases, which split one short sequence too. */
+int32_t gbx_attn_splits(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t capacity, int32_t normed);
 int gbx_attn_decode_ws(const void* q, const void* k, const void* v, void* kcache, void* vcache, const float* inv_freq,
                        const int64_t* pos, void* out, int32_t batch, int32_t n_heads, int32_t n_kv_heads,
                        int32_t head_dim, int32_t capacity, float rope_scale, float sm_scale, int32_t traditional,

@@ -45,3 +45,20 @@ def test_log_probabilities_around_the_second_launch(dt, rows, n):
     assert torch.equal(torch.isfinite(got), seen)
     room = last * (lse.abs() + want.abs()) + n * 2.0 ** -24 + 2.0 ** -22 * (1 + lse.abs())
     assert bool(((got.double() - want).abs() <= room)[seen].all())
+
+
+@pytest.mark.parametrize("kv,heads", [(1, 8), (2, 8), (4, 8), (4, 16)])
+def test_short_caches_keep_the_fused_block(kv, heads):
+    """What the attention launch of its own does with a short cache does not take the block's fused launch away: only a long one does."""
+    from gbx_lm_amd import synthetic as S
+    from gbx_lm_amd.decode import FusedDecodeRunner
+    from gbx_lm_amd.models.cache import KVCache
+    cfg = dict(S.TINY, hidden_size=1024, intermediate_size=2048, num_attention_heads=heads, num_key_value_heads=kv, num_hidden_layers=1)
+    model = S.build_model(cfg, S.make_strategy("S22", 1, 128), device=DEV, seed=3)
+    at = model.model.layers[0].self_attn
+    for capacity, long in ((256, False), (8192, True)):
+        c = KVCache(step=capacity)
+        like = torch.empty((1, at.n_kv_heads, 1, at.head_dim), dtype=torch.bfloat16, device=DEV)
+        c.reserve(1, like, like)
+        r = FusedDecodeRunner(model, [c], use_graph=False)
+        assert r.long_cache == long and (r.attn_ws is None) == (not long)
