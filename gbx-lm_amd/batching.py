@@ -108,7 +108,10 @@ class _DecodeGraph:
         self.turn += 1
         self.copied[k].synchronize()                     # the copy that last read this host buffer has run
         words, seq_pos, tok_pos = self.views[k]
-        words[:] = tokens
+        try:
+            words[:] = array("q", tokens)                # (as in an eager step: device tensors by their value)
+        except TypeError:                                # not whole numbers: torch's conversion
+            words[:] = torch.tensor(tokens, dtype=torch.long).numpy()
         seq_pos[:] = tok_pos[:] = pos0
         self.static.copy_(self.pinned[k], non_blocking=True)
         self.copied[k].record(torch.cuda.current_stream(self.static.device))

@@ -1,0 +1,30 @@
+"""What a step of the slot scheduler takes (batching.py): tokens of every kind that torch's conversion takes, in eager steps and in replayed ones alike."""
+import pytest
+import torch
+
+import revitar_oracle as O
+from gbx_lm_amd.batching import BatchScheduler
+from gbx_lm_amd.utils import load_model
+
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+CONFIG = O.make_config([O.attention_layer(4, 2, 32, 32, window=16, mlp=O.moe(4, 2, 32))], vocab=50, width=64)
+
+
+@pytest.fixture(scope="module")
+def path(tmp_path_factory):
+    return O.save_checkpoint(str(tmp_path_factory.mktemp("steps")), CONFIG, O.make_weights(CONFIG, 1))
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("form", ["device tensors", "host tensors", "floats", "numpy"])
+def test_decode_steps_take_what_their_first_ones_take(path, device, form):
+    """The third step of a set of slots is the first that a graph replays."""
+    import numpy as np
+    model = load_model(path, device=device, dtype=torch.float32)[0]
+    made = {"device tensors": lambda t: torch.tensor(t, device=device), "host tensors": torch.tensor, "floats": float, "numpy": np.int32}[form]
+    plain, other = BatchScheduler(model), BatchScheduler(model)
+    for i in range(6):
+        tokens = [(7 * i + j) % 50 for j in range(2)]
+        a = plain.step([(j, [t]) for j, t in enumerate(tokens)])
+        b = other.step([(j, [made(t)]) for j, t in enumerate(tokens)])
+        assert torch.equal(a, b)
