@@ -28,3 +28,26 @@ def test_decode_steps_take_what_their_first_ones_take(path, device, form):
         a = plain.step([(j, [t]) for j, t in enumerate(tokens)])
         b = other.step([(j, [made(t)]) for j, t in enumerate(tokens)])
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("put", ["subclass", "object", "class"])
+def test_generate_goes_through_a_step_put_in_its_place(path, device, put, monkeypatch):
+    """A subclass's, an object's or the class's own replaced step sees every step, and its logits last as long as it keeps them."""
+    model = load_model(path, device=device, dtype=torch.float32)[0]
+    prompts, seen = [[3, 1, 4], [1, 5]], []
+    want = BatchScheduler(model).generate(prompts, max_tokens=7)
+    step = BatchScheduler.step
+
+    def watched(self, entries, want=None):
+        logits = step(self, entries, want)
+        seen.append((logits, logits.clone()))
+        return logits
+
+    eng = type("Watched", (BatchScheduler,), {"step": watched})(model) if put == "subclass" else BatchScheduler(model)
+    if put == "object":
+        eng.step = lambda entries, want=None: watched(eng, entries, want)
+    elif put == "class":
+        monkeypatch.setattr(BatchScheduler, "step", watched)
+    assert eng.generate(prompts, max_tokens=7) == want
+    assert len(seen) == 7 and all(torch.equal(a, b) for a, b in seen)
