@@ -13,6 +13,7 @@ from __future__ import annotations
 
 from array import array
 from dataclasses import dataclass, field
+from operator import index
 from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
@@ -47,10 +48,14 @@ class StepBatch:
 
     @staticmethod
     def build(slot: Sequence[int], pos0: Sequence[int], n_new: Sequence[int], device, q_tile: int = 128) -> "StepBatch":
+        if q_tile < 1:
+            raise ValueError("a query tile holds at least one row")
         rows, seq, tile0, n_tiles = 0, [], [], 0
-        for s, p, n in zip(slot, pos0, n_new):
+        for s, p, n in zip(slot, pos0, map(index, n_new)):
             if n <= 0:
                 raise ValueError("a sequence of a step brings at least one token")
+            if p + n > 1 << 31:
+                raise RuntimeError("a position does not fit the tables' 32 bits")
             seq += (s, p, n, rows)
             tile0.append(n_tiles)
             rows += n

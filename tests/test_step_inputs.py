@@ -51,3 +51,12 @@ def test_generate_goes_through_a_step_put_in_its_place(path, device, put, monkey
         monkeypatch.setattr(BatchScheduler, "step", watched)
     assert eng.generate(prompts, max_tokens=7) == want
     assert len(seen) == 7 and all(torch.equal(a, b) for a, b in seen)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("pos0,n_new,q_tile,error", [([0], [2.0], 128, TypeError), ([0], [3], 0, ValueError), ([2 ** 31 - 2], [3], 128, RuntimeError)])
+def test_tables_of_impossible_steps_are_refused(device, pos0, n_new, q_tile, error):
+    """Rows that are no whole number, tiles without a row, positions past the tables' 32 bits."""
+    from gbx_lm_amd.batching import StepBatch
+    with pytest.raises(error):
+        StepBatch.build([1], pos0, n_new, device, q_tile)
