@@ -59,3 +59,15 @@ def test_several_matrices_in_a_launch():
         for l, y in zip(ls, ops.quantized_matmul_multi(x, ls)):
             want, terms = exact(x, l)
             assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -22 * terms).all())
+
+
+@pytest.mark.parametrize("m", [33, 34, 49, 64])
+@pytest.mark.parametrize("n,k,bits,g", [(24576, 1024, 2, 128), (24592, 2048, 4, 128), (24600, 1024, 2, 32)])
+def test_a_row_does_not_depend_on_its_place(m, n, k, bits, g):
+    """More than 32 rows of a wide product go in two launches: the last row comes out as it does among the first."""
+    from gbx_lm_amd import ops
+    l, x = layer(n, k, bits, g, torch.bfloat16, n), rows(m, k, torch.bfloat16, m)
+    y = ops.quantized_matmul(x, l.qweight, l.scales, l.zeros, group_size=g, bits=bits)
+    want, terms = exact(x, l)
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -22 * terms).all())
+    assert torch.equal(ops.quantized_matmul(x[m - 32:].contiguous(), l.qweight, l.scales, l.zeros, group_size=g, bits=bits), y[m - 32:])
