@@ -7,7 +7,9 @@
 // experts (32 where that leaves half the chip idle).  Its eight waves share out the channels: lane l of a block of 32 holds expert (and row) l % 16, channels
 // 4 (l / 16) .. + 3 of each half, so a load reads 64 neighbouring bytes of an expert; the next block's operands load under the products.  The waves' sums meet
 // in LDS in a fixed order: a row's logits do not depend on the other rows.
-// Logits that are not finite are summed again in fp32: an infinity has no rest, and infinity times a rest of zero is no number.
+// Logits that are not finite are summed again in fp32, on the matrix cores, by the workgroup that meets one: an infinity has no rest, and infinity times a rest
+// of zero is no number.  A thread's own sum of K terms for each of them took 1 905 us where all of 3481 rows x 128 experts x 2048 are odd and 586 where one row is; 51
+// and 49 here.
 // Widened copy and library | this, us: 3481 rows x 128 experts x 2048 47.5 | 26.6, 8192 x 64 x 2048 40.3 | 26.5, 8192 x 32 x 1024 25.5 | 12.2 (error against 64 bits
 // 8.1e-7 | 1.8e-7 of the logits' norm); the rule is where the rows are (mixer_ops.py: TILE_ROWS).
 #include "mixers_mfma.h"
@@ -23,6 +25,7 @@ template <int NT>
 __global__ __launch_bounds__(64 * RW) void router_tile_kernel(const bf16_t* __restrict__ h, const float* __restrict__ router, float* __restrict__ logits,
                                                             int T, int K, int E) {
   __shared__ __attribute__((aligned(16))) float part[RW][32][16 * NT];
+  __shared__ int met;                                                   // a logit that is not finite (written before the sums' barrier, read after the next one)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fk = lane >> 4;
   const int t0 = blockIdx.x * 32, e0 = blockIdx.y * 16 * NT, steps = (K + 31) / 32;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(h + static_cast<int64_t>(t0) * K), 0, 0x7FFFFFFF, 0x00020000);
@@ -81,23 +84,51 @@ __global__ __launch_bounds__(64 * RW) void router_tile_kernel(const bf16_t* __re
     __builtin_amdgcn_sched_barrier(0);
   }
   constexpr int SW = 4 * NT - 1 < 15 ? 4 * NT - 1 : 15;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4v*>(&part[wave][16 * i + fr][((4 * j + fk) ^ (fr & SW)) * 4]) = acc[i][j];
-  __syncthreads();
   const int row = tid / (4 * NT), q = tid % (4 * NT), t = t0 + row, e = e0 + 4 * q;
-  if (row >= 32 || t >= T || e >= E) return;
-  f32x4v sum = f32x4v{0};
+  const bool live = row < 32 && t < T && e < E;
+  auto meet = [&]() {                                                   // the waves' sums of this thread's four logits
 #pragma unroll
-  for (int w = 0; w < RW; ++w) sum += *reinterpret_cast<const f32x4v*>(&part[w][row][(q ^ (row & SW)) * 4]);
-  float v[4] = {sum.x, sum.y, sum.z, sum.w};
-  for (int i = 0; i < 4 && e + i < E; ++i)
-    if (!(fabsf(v[i]) < INFINITY)) {
-      float z = 0.f;
-      for (int k = 0; k < K; ++k) z = fmaf(to_f32(h[static_cast<int64_t>(t) * K + k]), router[static_cast<int64_t>(e + i) * K + k], z);
-      v[i] = z;
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4v*>(&part[wave][16 * i + fr][((4 * j + fk) ^ (fr & SW)) * 4]) = acc[i][j];
+    __syncthreads();
+    f32x4v sum = f32x4v{0};
+    if (live) {
+#pragma unroll
+      for (int w = 0; w < RW; ++w) sum += *reinterpret_cast<const f32x4v*>(&part[w][row][(q ^ (row & SW)) * 4]);
     }
+    return sum;
+  };
+  if (tid == 0) met = 0;
+  f32x4v v = meet();
+  bool odd = false;
+  for (int i = 0; i < 4 && e + i < E; ++i) odd |= !(fabsf(v[i]) < INFINITY);
+  if (live && odd) met = 1;
+  __syncthreads();
+  if (met) {                                                            // (the whole workgroup, past its last read of the sums)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = f32x4v{0};
+#pragma unroll 1
+    for (int s = wave; s < steps; s += RW) {
+      load(b0, s);
+#pragma unroll
+      for (int h = 0; h < 8; ++h)                                       // channel h % 4 of the lane's four in half h / 4
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const unsigned pair = b0.x[i][h >> 2][(h & 3) >> 1];
+          const float x = __uint_as_float(h & 1 ? pair & 0xFFFF0000u : pair << 16);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b0.w[j][h >> 2][h & 3]), x, acc[i][j], 0, 0, 0);
+        }
+    }
+    const f32x4v whole = meet();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (!(fabsf(v[i]) < INFINITY)) v[i] = whole[i];
+  }
+  if (!live) return;
   float* out = logits + static_cast<int64_t>(t) * E + e;
   if (E % 4 == 0) *reinterpret_cast<f32x4v*>(out) = f32x4v{v[0], v[1], v[2], v[3]};
   else
