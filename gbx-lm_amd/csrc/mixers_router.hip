@@ -99,40 +99,45 @@ __global__ __launch_bounds__(64 * RW) void router_tile_kernel(const bf16_t* __re
     }
     return sum;
   };
+  auto leave = [&](const f32x4v& v) {
+    float* out = logits + static_cast<int64_t>(t) * E + e;
+    if (E % 4 == 0) *reinterpret_cast<f32x4v*>(out) = v;
+    else
+      for (int i = 0; i < 4 && e + i < E; ++i) out[i] = v[i];
+  };
   if (tid == 0) met = 0;
   f32x4v v = meet();
-  bool odd = false;
-  for (int i = 0; i < 4 && e + i < E; ++i) odd |= !(fabsf(v[i]) < INFINITY);
-  if (live && odd) met = 1;
-  __syncthreads();
-  if (met) {                                                            // (the whole workgroup, past its last read of the sums)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[i][j] = f32x4v{0};
-#pragma unroll 1
-    for (int s = wave; s < steps; s += RW) {
-      load(b0, s);
-#pragma unroll
-      for (int h = 0; h < 8; ++h)                                       // channel h % 4 of the lane's four in half h / 4
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const unsigned pair = b0.x[i][h >> 2][(h & 3) >> 1];
-          const float x = __uint_as_float(h & 1 ? pair & 0xFFFF0000u : pair << 16);
-#pragma unroll
-          for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b0.w[j][h >> 2][h & 3]), x, acc[i][j], 0, 0, 0);
-        }
-    }
-    const f32x4v whole = meet();
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (!(fabsf(v[i]) < INFINITY)) v[i] = whole[i];
+  if (live) {
+    bool odd = false;
+    for (int i = 0; i < 4 && e + i < E; ++i) odd |= !(fabsf(v[i]) < INFINITY);
+    if (odd) met = 1;
+    leave(v);
   }
+  __syncthreads();
+  if (!met) return;                                                     // (the whole workgroup, past its last read of the sums)
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4v{0};
+#pragma unroll 1
+  for (int s = wave; s < steps; s += RW) {
+    load(b0, s);
+#pragma unroll
+    for (int h = 0; h < 8; ++h)                                         // channel h % 4 of the lane's four in half h / 4
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const unsigned pair = b0.x[i][h >> 2][(h & 3) >> 1];
+        const float x = __uint_as_float(h & 1 ? pair & 0xFFFF0000u : pair << 16);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b0.w[j][h >> 2][h & 3]), x, acc[i][j], 0, 0, 0);
+      }
+  }
+  const f32x4v whole = meet();
   if (!live) return;
-  float* out = logits + static_cast<int64_t>(t) * E + e;
-  if (E % 4 == 0) *reinterpret_cast<f32x4v*>(out) = f32x4v{v[0], v[1], v[2], v[3]};
-  else
-    for (int i = 0; i < 4 && e + i < E; ++i) out[i] = v[i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (!(fabsf(v[i]) < INFINITY)) v[i] = whole[i];
+  leave(v);
 }
 
 }  // namespace
