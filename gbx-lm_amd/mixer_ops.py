@@ -147,7 +147,7 @@ def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
     t, rows = h.shape[0], router.shape[0]
     if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1] or (router.numel() >= ROUTER_HELD and t * router.numel() > ROUTER_FEW):
         k = h.shape[1]
-        if h.dtype == torch.float32 or k != router.shape[1] or k % 8 or not 0 < k <= TILE_CHANNELS or rows > TILE_EXPERTS or not TILE_ROWS <= t <= TILE_LOGITS // rows:
+        if h.dtype == torch.float32 or k != router.shape[1] or k % 8 or not 0 < k <= TILE_CHANNELS or not 0 < rows <= TILE_EXPERTS or not TILE_ROWS <= t <= TILE_LOGITS // rows:
             return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
         h = h.contiguous()
         if (h.data_ptr() | router.data_ptr()) % 16:

@@ -51,3 +51,11 @@ def test_odd_numbers(t, k, e):
     got, x = M._router_logits(h, router), h[:, k // 2].float()
     assert torch.equal(got[:, :e - 1], plain[:, :e - 1])
     assert torch.equal(got[x != 0, e - 1], x[x != 0].sign() * torch.inf) and bool(torch.isnan(got[x == 0, e - 1]).all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_a_router_without_experts(dt):
+    """Nothing to choose from: no logits, as of any product."""
+    from gbx_lm_amd import mixer_ops as M
+    got = M._router_logits(torch.ones((600, 64), device=DEV, dtype=dt), torch.ones((0, 64), device=DEV))
+    assert got.shape == (600, 0) and got.dtype == torch.float32
