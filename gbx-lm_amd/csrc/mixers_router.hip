@@ -4,14 +4,14 @@
 // numbers is exact in fp32: three bf16 products a weight round less than one fp32 product does, at five times the rate of the fp32 instruction (which took
 // 38 us for the first line below, the library beside its widened copy 47).
 // Bound by the splitting, 5.5 instructions a weight and workgroup, with the router's way through the first cache beside it; a workgroup takes 32 rows x 64
-// experts (32 where that leaves half the chip idle).  Its eight waves share out the channels: lane l of a block of 32 holds expert (and row) l % 16, channels
+// experts (32 where those are one round of the CUs).  Its eight waves share out the channels: lane l of a block of 32 holds expert (and row) l % 16, channels
 // 4 (l / 16) .. + 3 of each half, so a load reads 64 neighbouring bytes of an expert; the next block's operands load under the products.  The waves' sums meet
 // in LDS in a fixed order: a row's logits do not depend on the other rows.
 // Logits that are not finite are summed again in fp32, on the matrix cores, by the workgroup that meets one: an infinity has no rest, and infinity times a rest
 // of zero is no number.  A thread's own sum of K terms for each of them took 1 905 us where all of 3481 rows x 128 experts x 2048 are odd and 586 where one row is; 51
 // and 49 here.
-// Widened copy and library | this, us: 3481 rows x 128 experts x 2048 47.5 | 26.6, 8192 x 64 x 2048 40.3 | 26.5, 8192 x 32 x 1024 25.5 | 12.2 (error against 64 bits
-// 8.1e-7 | 1.8e-7 of the logits' norm); the rule is where the rows are (mixer_ops.py: TILE_ROWS).
+// Widened copy and library | this, us: 3481 rows x 128 experts x 2048 46.2 | 25.6, 8192 x 64 x 2048 38.5 | 25.7, 8192 x 32 x 1024 24.8 | 10.6 (error against 64 bits
+// 8.1e-7 | 1.8e-7 of the logits' norm); the rule is where the rows are (mixer_ops.py: router_tiles_win).
 #include "mixers_mfma.h"
 
 namespace gbxm {
@@ -152,7 +152,9 @@ extern "C" int gbxm_router_tiles(const void* h, const float* router, float* logi
     return fail(GBXM_ERR_UNSUPPORTED, "router_tiles: channels in multiples of 8, operands 16-byte aligned, a router under 2 GB");
   if (T == 0) return GBXM_OK;
   const int64_t rows = (T + 31) / 32;
-  const bool wide = rows * ((E + 63) / 64) >= 128;
+  // 32 experts a workgroup where those fill one round of the CUs at most, else 64, whose rounds are half as many (us, 32 | 64: 2047 rows x 128 x 2048 17.6 | 24.6,
+  // 1024 x 256 x 2048 17.5 | 24.6, 2500 x 128 x 2048 31.6 | 24.7, 4500 x 64 x 2048 31.7 | 25.0); a router of no more is not the wider one's (12000 x 32 x 2048 31.8 | 37.2)
+  const bool wide = E > 32 && rows * ((E + 31) / 32) > 256;
   const dim3 grid(static_cast<unsigned>(rows), static_cast<unsigned>(wide ? (E + 63) / 64 : (E + 31) / 32));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (wide) router_tile_kernel<4><<<grid, 64 * RW, 0, s>>>(static_cast<const bf16_t*>(h), router, logits, static_cast<int>(T), K, E);

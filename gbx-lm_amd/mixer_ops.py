@@ -128,10 +128,17 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) 
 # XCDs' caches do not hold (8 MB) takes it for few products only.  Library with its widened copy | launch, us: 32 rows x 256 x 4096 15.0 | 10.4, x 256 x 7168
 # 21.9 | 16.8, x 1024 x 1024 10.3 | 11.2; 8 MB: 4 x 1024 x 2048 10.2 | 4.6, 8 rows 10.3 | 12.2, 32 rows 11.1 | 19.5; 32 x 1024 x 4096 15.0 | 35.8.
 ROUTER_ROWS, ROUTER_HELD, ROUTER_FEW = 32, 1 << 21, 1 << 23
-# Prompt-sized steps whose bf16 rows the matrix cores take as they are (csrc/mixers_router.hip).  Widened copy and library | this, us, rows x experts x channels:
-# 3481 x 128 x 2048 47.5 | 26.6, 8192 x 64 x 2048 40.3 | 26.5, 8192 x 32 x 1024 25.5 | 12.2, 700 x 256 x 2048 19.4 | 18.1, 16384 x 128 x 2048 99 | 96; outside the rule
-# 300 x 128 x 2048 12.8 | 17.3, 2000 x 256 x 7168 77 | 80, 8192 x 256 x 4096 167 | 181.
-TILE_ROWS, TILE_EXPERTS, TILE_CHANNELS, TILE_LOGITS = 512, 256, 2048, 1 << 21
+TILE_EXPERTS, TILE_CHANNELS, TILE_LOGITS = 256, 2048, 3 << 19
+
+
+def router_tiles_win(t: int, e: int, k: int) -> bool:
+    """Prompt-sized steps whose bf16 rows the matrix cores take as they are (csrc/mixers_router.hip), by whole rounds of the CUs: one is 17 us at 2048
+    channels, which the library beats for few rows and meets again where rounds end badly.  Widened copy and library | this, us, rows x experts x channels:
+    512 x 128 x 1024 11.4 | 10.2, x 1152 10.0 | 11.3, x 2048 13.3 | 17.4; 1024 x 64 x 2048 15.6 | 17.2, 1536 x 64 x 2048 21.4 | 17.4, x 32 18.3 | 17.1, 1024 x 64 x 1536
+    12.9 | 13.7, 1280 18.0 | 13.7; 3481 x 128 x 2048 46.2 | 25.6, 8192 x 64 x 2048 38.5 | 25.7, x 32 x 1024 24.8 | 10.6; more experts 2047 x 256 x 2048 30.8 | 25.2,
+    2500 44.1 | 47.8, 8192 81.3 | 94.2, 4500 x 200 x 1536 40.2 | 42.8; 16000 x 128 x 2048 91.1 | 94.3, 12000 83.7 | 71.2, 8192 x 256 x 1024 50.0 | 52.8."""
+    return (0 < e <= TILE_EXPERTS and 0 < k <= TILE_CHANNELS and k % 8 == 0 and t >= (512 if k <= 1024 else 3 * k // 4) and t * e <= TILE_LOGITS
+            and (e <= 128 or k <= 1024 or t <= 2048))
 
 
 def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
@@ -147,7 +154,7 @@ def _router_logits(h: torch.Tensor, router: torch.Tensor) -> torch.Tensor:
     t, rows = h.shape[0], router.shape[0]
     if t > ROUTER_ROWS or h.shape[1] != router.shape[1] or not h.shape[1] or (router.numel() >= ROUTER_HELD and t * router.numel() > ROUTER_FEW):
         k = h.shape[1]
-        if h.dtype == torch.float32 or k != router.shape[1] or k % 8 or not 0 < k <= TILE_CHANNELS or not 0 < rows <= TILE_EXPERTS or not TILE_ROWS <= t <= TILE_LOGITS // rows:
+        if h.dtype == torch.float32 or k != router.shape[1] or not router_tiles_win(t, rows, k):
             return torch.matmul(h if h.dtype == torch.float32 else h.float(), router.t())
         h = h.contiguous()
         if (h.data_ptr() | router.data_ptr()) % 16:
