@@ -62,3 +62,21 @@ def test_short_caches_keep_the_fused_block(kv, heads):
         c.reserve(1, like, like)
         r = FusedDecodeRunner(model, [c], use_graph=False)
         assert r.long_cache == long and (r.attn_ws is None) == (not long)
+
+
+@pytest.mark.parametrize("normed,cap", [(False, 256), (False, 768), (False, 4096), (True, 512)])
+def test_scratch_only_where_the_context_is_split(normed, cap):
+    """A launch that reads its context in one piece is given none."""
+    from gbx_lm_amd import _lib, ops
+    from gbx_lm_amd.models.rope_utils import RoPE
+    nh, nkv, hd = 32, 4, 128
+    q, k, v = (torch.randn((1, n * hd), device=DEV).to(torch.bfloat16) for n in (nh, nkv, nkv))
+    kc, vc = (torch.zeros((1, nkv, cap, hd), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    w = torch.ones(hd, dtype=torch.bfloat16, device=DEV) if normed else None
+    inv, p, out = RoPE(hd, traditional=False, base=10000.0).inv_freq.to(DEV), torch.tensor([9], device=DEV), torch.zeros((1, nh * hd), dtype=torch.bfloat16, device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.attn_decode_batched(q, k, v, kc, vc, inv, p, out, nh, nkv, hd, 1.0, hd ** -0.5, False, w, w, 1e-6)
+    split = _lib.lib().gbx_attn_splits(1, nh, nkv, cap, int(normed)) > 1
+    assert split == (normed or cap == 4096) and (torch.cuda.max_memory_allocated() > before) == split
