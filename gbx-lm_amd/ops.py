@@ -1204,6 +1204,14 @@ def attn_oproj_decode(q, k, v, kcache, vcache, inv_freq, pos, o_proj, acc, n_hea
                                                 _stream_ptr(q.device)))
 
 
+def _attn_scratch(b: int, n_heads: int, n_kv: int, head_dim: int, cap: int, grouped: bool, device) -> Optional[torch.Tensor]:
+    """Scratch for the slices of a launch that splits its context (flash-decoding), none for one that does not."""
+    L = _lib.lib()
+    if L.gbx_attn_splits(b, n_heads, n_kv, cap, int(grouped)) <= 1:
+        return None
+    return torch.empty((L.gbx_attn_workspace_bytes(b, n_heads, n_kv, head_dim, cap),), dtype=torch.uint8, device=device)
+
+
 def attn_decode_batched(q, k, v, kcache, vcache, inv_freq, pos, out, n_heads: int, n_kv: int, head_dim: int,
                         rope_scale: float, sm_scale: float, traditional: bool, q_norm_w=None, k_norm_w=None,
                         norm_eps: float = 0.0, q_bias=None, k_bias=None, v_bias=None, workspace=None) -> None:
@@ -1211,9 +1219,8 @@ def attn_decode_batched(q, k, v, kcache, vcache, inv_freq, pos, out, n_heads: in
     caches [B, n_kv, capacity, hd] (gbx_attn_decode_batched: RoPE + cache append + softmax(q k^T) v in one launch)."""
     _require_cuda(q, "q")
     b, cap = kcache.shape[0], kcache.shape[2]
-    if workspace is None:                               # long caches: scratch for the context split (flash-decoding)
-        need = _lib.lib().gbx_attn_workspace_bytes(b, n_heads, n_kv, head_dim, cap)
-        workspace = torch.empty((need,), dtype=torch.uint8, device=q.device) if need else None
+    if workspace is None:
+        workspace = _attn_scratch(b, n_heads, n_kv, head_dim, cap, q_norm_w is not None or q_bias is not None, q.device)
     _lib.check(_lib.lib().gbx_attn_decode_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), kcache.data_ptr(), vcache.data_ptr(),
                                              inv_freq.data_ptr(), pos.data_ptr(), out.data_ptr(), b, n_heads, n_kv, head_dim,
                                                  cap, float(rope_scale), float(sm_scale), int(bool(traditional)),
@@ -1235,8 +1242,7 @@ def attn_decode_slices(qkv_ws: torch.Tensor, slices: int, kcache, vcache, inv_fr
     b, cap = kcache.shape[0], kcache.shape[2]
     assert qkv_ws.dtype == torch.float32 and qkv_ws.numel() >= slices * b * (n_heads + 2 * n_kv) * head_dim
     if workspace is None:
-        need = _lib.lib().gbx_attn_workspace_bytes(b, n_heads, n_kv, head_dim, cap)
-        workspace = torch.empty((need,), dtype=torch.uint8, device=out.device) if need else None
+        workspace = _attn_scratch(b, n_heads, n_kv, head_dim, cap, True, out.device)
     _lib.check(_lib.lib().gbx_attn_decode_slices(qkv_ws.data_ptr(), int(slices), kcache.data_ptr(), vcache.data_ptr(), inv_freq.data_ptr(),
                                                  pos.data_ptr(), out.data_ptr(), b, n_heads, n_kv, head_dim, cap, float(rope_scale),
                                                  float(sm_scale), int(bool(traditional)),
