@@ -675,10 +675,15 @@ static int split_heads(int batch, int n_heads, int rep, int capacity) {
   return (capacity <= 1536 && batch * n_heads <= 64) ? 1 : 2;
 }
 
-// One sequence on the grouped kernel (query / key norms): its kv heads are few workgroups (4 kv heads of 8 query heads: 8, 16.3 us a launch at context 500), so that its
-// context is split from the shortest cache on, 32 positions a slice.  Whole | split, 24 tokens of 6 such layers, ms: context 130 13.45 | 13.22,
-// 330 13.77 | 13.45, 620 14.6 | 13.5, 920 15.6 (slices of 128) | 13.5.  Batches keep the rule below: their sequences are workgroups, and a stack of layers
-// would carry every changed rounding on.
+// One sequence on the grouped kernel (query / key norms) whose unsplit workgroups would take three or four query heads each: caches of 256 to 1023 positions
+// split their context into eight slices, which is what the rule of the longer ones comes to at 1024 and leaves no step there.  A launch's slices are the
+// context's at that time, rounded up to 64 positions (heads of 128; 128 for 64).  Whole | eight slices, us a launch (cold caches), context 1, 63, 130, last:
+//   heads of 128, 32 on 4 kv heads: cache of 256 7.9 7.9 9.8 11.7 | 7.2 7.4 7.4 8.1, 512 7.9 7.9 9.8 15.8 | 7.0 7.5 7.6 9.0, 768 7.9 8.0 9.8 19.4 | 7.0 7.4 7.5 9.7
+//   32 on 8: 512 7.9 7.9 9.9 15.8 | 7.0 7.4 7.6 9.0;  64 on 8: 512 8.0 8.0 9.9 16.0 | 7.8 8.0 8.2 10.1;  heads of 64, 8 on 2: 512 7.0 7.0 8.1 10.4 | 7.0 7.5 7.5 7.6
+//   24 on 4 (three a workgroup): 256 7.0 7.1 8.9 10.0 | 7.0 7.5 7.5 7.6, 512 7.1 7.1 8.9 13.9 | 7.0 7.4 7.4 8.6;  heads of 64: 512 6.6 6.7 7.4 9.5 | 7.2 7.5 7.6 7.7
+// Fewer heads a workgroup are as many workgroups already (16 on 8: 256 5.6 5.6 7.1 7.8 | 6.9 7.3 7.3 7.5; 7 on 1: 4.9 4.9 5.9 6.5 | 7.1 7.6 7.6 7.8).  From 1024 on,
+// context 512 and last, slices of 128 | 64 | 32 positions: 16 on 4 8.1 9.1 | 7.9 8.8 | 9.1 9.5, 32 on 4 8.9 10.1 | 9.1 10.1 | 9.1 10.1, 24 on 4 8.6 9.5 | 9.4 9.9 | 9.9 10.4.
+// Batches keep the rule of the longer caches: their sequences are workgroups.
 int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
   const int rep = n_heads / n_kv;
   static const int force_r = gbx::env_switch("GBX_ATTN_SPLIT_R");   // tuning aid
@@ -686,9 +691,9 @@ int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
   const int wgs = n_kv * (rep / R) * batch;
   static const int min_cap = gbx::env_switch("GBX_ATTN_SPLIT_MIN");   // tuning aid
   static const int div = gbx::env_switch("GBX_ATTN_SPLIT_DIV");     // tuning aid
-  const bool one = grouped && batch == 1 && n_kv <= 4 && capacity <= 1536;
-  if (capacity < (one ? 64 : min_cap)) return 1;       // short caches: the un-split kernels win (649 vs 774 tok/s at context 128)
-  int s = std::min(std::min(512 / std::max(wgs, 1), capacity / (one ? 32 : div)), 32);
+  const bool one = grouped && batch == 1 && (rep % 4 == 0 || rep % 3 == 0) && capacity >= min_cap / 4;
+  if (capacity < min_cap && !one) return 1;            // short caches: the un-split kernels win (649 vs 774 tok/s at context 128)
+  const int s = std::min(std::min(512 / std::max(wgs, 1), capacity < min_cap ? 8 : capacity / div), 32);
   return s < 2 ? 1 : s;
 }
 

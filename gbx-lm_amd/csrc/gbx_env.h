@@ -36,7 +36,7 @@ inline const EnvSwitch* env_table(int* n) {
       {"GBX_ATTN_WIDE", 1, "decode attention at head_dim 128: 16 waves per head with the in-wave state merge (0: 4 waves) (A/B)"},
       {"GBX_ATTN_GQA_WIDE", 1, "batched decode attention (head_dim 128, 4 query heads per kv head, unsplit context): 8 waves per workgroup (0: 4) (A/B)"},
       {"GBX_ATTN_SPLIT_R", 0, "decode attention: force the context split (tuning aid)"},
-      {"GBX_ATTN_SPLIT_MIN", 1024, "decode attention: smallest cache capacity that is split over workgroups (tuning aid)"},
+      {"GBX_ATTN_SPLIT_MIN", 1024, "decode attention: smallest cache capacity that is split over workgroups; a quarter of it for one sequence with query / key norms (tuning aid)"},
       {"GBX_ATTN_SPLIT_DIV", 128, "decode attention: cached positions per split (tuning aid)"},
       {"GBX_ATTN_GROUPED", 0, "1: the grouped-query decode attention kernel at batch 1 too (tuning aid)"},
       {"GBX_BATCH_KSPLIT_MINK", 8192, "batch GEMM: smallest K that is split across workgroups (tuning aid)"},
