@@ -67,6 +67,11 @@ template <typename T> __device__ __forceinline__ float lsm_round(float f) {
 // logit left 19 workgroups with 32 round trips' worth of requests each: 1 x 151 936 bf16 12.4 -> 5.6 us, 8 x 128 256 12.1 -> 6.2, and 1 x 32 000 fp32 7.1 (one workgroup) -> 5.5; 20 000 5.4 in one launch, 5.5 in two.
 constexpr int LSM_SLICE = 2048;
 
+// A thread's logits are k + j `step`: neighbours where 16-byte accesses reach them and in 16 bits, whose eight are 16 bytes anyway; 32-bit ones off that grid lie
+// beside those of the neighbouring threads (neighbours | beside, us: 1 x 24 577 7.9 | 6.4, 15 x 50 257 10.5 | 7.4, 15 x 151 935 19.4 | 9.3; 1 x 24 577 bf16 6.9 | 7.1).
+template <typename T> __device__ __forceinline__ int lsm_step(int vec) { return vec || sizeof(T) == 2 ? 1 : 256; }
+template <typename T> __device__ __forceinline__ int lsm_first(int vec) { return blockIdx.x * LSM_SLICE + threadIdx.x * (lsm_step<T>(vec) == 1 ? 8 : 1); }
+
 template <typename T>
 __device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int n, int vec, float* v) {
   if (vec) {                                                  // (n is a multiple of 8: all of them are in the row, or none)
@@ -77,8 +82,9 @@ __device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int 
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = k < n ? lsm_get<T>(u[j / PER], j % PER) : -INFINITY;
   } else {
+    const int step = lsm_step<T>(0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = k + j < n ? static_cast<float>(row[k + j]) : -INFINITY;
+    for (int j = 0; j < 8; ++j) v[j] = k + j * step < n ? static_cast<float>(row[k + j * step]) : -INFINITY;
   }
 }
 
@@ -86,7 +92,7 @@ __device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int 
 template <typename T>
 __global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n, int vec) {
   __shared__ float top[4], red[4];
-  const int k = blockIdx.x * LSM_SLICE + threadIdx.x * 8;
+  const int k = lsm_first<T>(vec), step = lsm_step<T>(vec);
   float v[8], m = -INFINITY, s = 0.f;
   lsm_load8(x + static_cast<int64_t>(blockIdx.y) * n, k, n, vec, v);
 #pragma unroll
@@ -98,7 +104,7 @@ __global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restr
   m = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
   const float shift = isinf(m) ? 0.f : m;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) s += k + j < n ? expf(v[j] - shift) : 0.f;
+  for (int j = 0; j < 8; ++j) s += k + j * step < n ? expf(v[j] - shift) : 0.f;
   s = block_sum<4>(s, red);
   if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = float2{m, s};
 }
@@ -107,7 +113,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, T* __restrict__ out, int n, int vec) {
   __shared__ float top[4], red[4];
   const float2* p = part + blockIdx.y * gridDim.x;
-  const int parts = gridDim.x, k = blockIdx.x * LSM_SLICE + threadIdx.x * 8;
+  const int parts = gridDim.x, k = lsm_first<T>(vec);
   const int64_t base = static_cast<int64_t>(blockIdx.y) * n;
   float v[8], m = -INFINITY, s = 0.f;
   lsm_load8(x + base, k, n, vec, v);
@@ -137,7 +143,7 @@ __global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restr
   } else {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (k + j < n) out[base + k + j] = static_cast<T>(v[j] - lse);
+      if (k + j * lsm_step<T>(0) < n) out[base + k + j * lsm_step<T>(0)] = static_cast<T>(v[j] - lse);
   }
 }
 
@@ -496,8 +502,9 @@ extern "C" int gbxm_step_tables(const int32_t* seq, const int32_t* tile0, int32_
 }
 
 extern "C" size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n) {
-  // few rows that are long: sixteen and more keep that many CUs busy in the one-launch form, shorter ones are done there before a second launch would start
-  return rows > 0 && rows < 16 && n > 12 * LSM_SLICE ? static_cast<size_t>(rows) * ((n + LSM_SLICE - 1) / LSM_SLICE) * 8 : 0;
+  // few rows that are long: sixteen and more keep that many CUs busy in the one-launch form, shorter ones are done there before a second launch would start; one row
+  // off the grid of eight takes wide accesses there and none in slices (one launch | two, us, bf16: 24 577 6.2 | 6.9, 28 001 6.7 | 7.0, 30 001 6.9 both, 32 769 9.9 | 6.9)
+  return rows > 0 && rows < 16 && n > (rows == 1 && n % 8 ? 14 : 12) * LSM_SLICE ? static_cast<size_t>(rows) * ((n + LSM_SLICE - 1) / LSM_SLICE) * 8 : 0;
 }
 
 extern "C" int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream) {

@@ -75,7 +75,7 @@ def test_split_context_against_a_batch_of_the_same_sequence_twice(hd, nh, nkv, c
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,n", [(1, 24576), (1, 24577), (15, 24584), (16, 24584), (2, 26623)])
+@pytest.mark.parametrize("rows,n", [(1, 24576), (1, 24577), (15, 24584), (16, 24584), (2, 26623), (1, 28672), (1, 28673), (3, 50257)])
 def test_log_probabilities_around_the_second_launch(dt, rows, n):
     """The logarithm: an fp32 sum of n terms rounded to the rows' type; the difference is rounded once more."""
     from gbx_lm_amd.mixer_ops import log_probabilities
