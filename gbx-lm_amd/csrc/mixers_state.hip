@@ -177,12 +177,14 @@ __global__ __launch_bounds__(NT) void recurrent_prep_rows_kernel(gbxm_recurrent_
       out[(i / p.H) * p.out_stride + C + nd + i % p.H] = sigmoid_<false>(to_f32(y[(t0 + i / p.H) * p.y_stride + p.off_beta + i % p.H]));
 }
 
-// What that kernel takes: heads of 4, 8, .. 256 channels, everything in groups of four on the grid of their loads, four taps or no convolution.
+// What that kernel takes: heads of 4, 8, .. 256 channels, everything in groups of four on the grid of their loads, four taps or no convolution.  Without one, rows
+// of few numbers leave most of its lanes idle (one number a lane | this, us: 500 rows of 128 numbers 4.4 | 5.1, 8 192 16.0 | 29; of 256 4.4 | 4.9, 8 192 16.2 | 16.3,
+// 16 000 30.8 | 21.5; of 512 4.6 | 3.9, 8 192 20.3 | 16.9).
 template <typename T>
 bool prep_rows_shape(const gbxm_recurrent_prep_args& a) {
   const int C = 2 * a.G * a.dk + a.H * a.dv;
   if (a.dk < 4 || a.dk > 256 || (a.dk & (a.dk - 1)) || a.H * a.dv % 4 || a.off_q % 4 || a.off_k % 4 || a.off_v % 4 || a.y_stride % 4 || a.out_stride % 4 || (a.conv && a.taps != 4) ||
-      (a.a && a.a_stride % 4))
+      (a.a && a.a_stride % 4) || (!a.conv && C + a.H * a.dk < 256))
     return false;
   const T* none = nullptr;
   return all_aligned(4 * sizeof(T), static_cast<const T*>(a.y), a.a ? static_cast<const T*>(a.a) : none, a.conv ? static_cast<const T*>(a.conv) : none,
@@ -426,7 +428,8 @@ void launch_head_norm_gate(const float* o, const void* gate, int64_t gate_stride
   const T* g = static_cast<const T*>(gate);
   T* y = static_cast<T*>(out);
   const int64_t blocks = (static_cast<int64_t>(H) * dv / 4 + NT - 1) / NT;
-  if (dv >= 4 && dv <= 256 && !(dv & (dv - 1)) && gate_stride % 4 == 0 && out_row % 4 == 0 && all_aligned(4 * sizeof(T), g, static_cast<const T*>(y)) && all_aligned(16, o) &&
+  // (rows of less than 32 channels are a few lanes of a workgroup: 1 000 rows of one head of 16 2.6 us | 3.4)
+  if (H * dv >= 32 && dv >= 4 && dv <= 256 && !(dv & (dv - 1)) && gate_stride % 4 == 0 && out_row % 4 == 0 && all_aligned(4 * sizeof(T), g, static_cast<const T*>(y)) && all_aligned(16, o) &&
       blocks <= 65535)
     head_norm_gate_vec_kernel<T, false><<<dim3(T_, static_cast<unsigned>(blocks)), NT, 0, s>>>(o, g, gate_stride, w, y, out_row, H * dv, dv, eps, kind);
   else
