@@ -1,6 +1,7 @@
-"""Quantised products of 2 to 32 rows outside the group-128 batch kernel (csrc/mfma_rows.hip): every width of field and group, one row tile and two, their
-edges, contractions that give waves one chunk each or unequal numbers, outputs that end inside a workgroup, both output tilings, a bias, and
-scales that are not aligned to a chunk's (the dequantising kernel).  Reference: float64; tolerance: the result's rounding (two with a bias; the
+"""Quantised products of 2 to 32 rows: every width of field and group, one row tile and two, their edges, contractions that give waves one chunk each or
+unequal numbers, outputs that end inside a workgroup, a bias, and scales that are not aligned to a chunk's (the dequantising kernel).  Contractions of 1024 to
+4096 run in the kernel that keeps the rows in registers (csrc/mfma_slab_impl.h), or, for few rows off the grid of 1024, in csrc/mfma_rows.hip; longer ones there
+(both output tilings: up to and beyond 4096 outputs) or, in groups of 128 on that grid, in csrc/mfma_batch.hip.  Reference: float64; tolerance: the result's rounding (two with a bias; the
 dequantising kernel rounds every weight too) and fp32 sums of K terms as large as C + q = 143 (bf16) or 1039 (fp16)."""
 import pytest
 import torch
@@ -40,6 +41,22 @@ def test_fields_groups_and_edges(dt, bits, g, m, n, k, bias):
     run(m, n, k, bits, g, dt, bias, False, m + n + k + bits + g)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (2, 128), (3, 32), (3, 64), (3, 128), (4, 32), (4, 64), (4, 128)])
+@pytest.mark.parametrize("m,n,k,bias", [(2, 4097, 4224, True), (16, 33, 11008, False), (17, 4096, 4224, False), (32, 4112, 11008, True), (9, 100, 4352, True), (3, 70, 1152, True)])
+def test_rows_that_stay_in_memory(dt, bits, g, m, n, k, bias):
+    """Contractions beyond 4096 that are no multiple of 1024, and few rows of a short one."""
+    run(m, n, k, bits, g, dt, bias, False, m + n + k + bits + g)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (2, 128), (3, 128), (4, 128)])
+@pytest.mark.parametrize("m,n,bias", [(32, 24584, False), (7, 12300, True), (16, 5130, False), (2, 1000, True), (33, 24576, False)])
+def test_unsplit_workgroups_of_the_batch_kernel(dt, bits, g, m, n, bias):
+    """Its 128, 64, 32 and 16 output rows a workgroup (64 for 128 in groups of 32 and 64), outputs that end inside one, and 33 rows in two launches."""
+    run(m, n, 5120, bits, g, dt, bias, False, m + n + bits + g)
+
+
 @pytest.mark.parametrize("bits,g", [(3, 32), (3, 64), (4, 32), (4, 64)])
 def test_whole_kilochannels_and_unaligned_scales(bits, g):
     for m in (2, 15, 32):
@@ -76,17 +93,18 @@ def same_numbers(y, want, eps, room):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits,g", [(2, 32), (2, 64), (3, 32), (3, 64), (3, 128), (4, 32), (4, 64), (4, 128)])
-def test_infinite_undefined_and_huge_activations(dt, bits, g):
+@pytest.mark.parametrize("k", [1152, 2176, 4224])                   # in registers and, of up to 12 and 6 rows, not; beyond them
+def test_infinite_undefined_and_huge_activations(dt, bits, g, k):
     """An infinity times the weight, not infinity minus infinity.  Tolerance: the roundings of the result and, where a row is huge, of its weights; fp32 sums
     of K terms as large as C + q."""
     from gbx_lm_amd import ops
-    n, k = 100, 1152
+    n = 100
     gen = torch.Generator(device=DEV).manual_seed(bits * g)
     qw = torch.randint(-2**31, 2**31, (n, k // 32 * bits), device=DEV, generator=gen, dtype=torch.int64).to(torch.int32).view(torch.uint32)
     s = ((torch.rand((n, k // g), device=DEV, generator=gen) + 0.5) * 0.03).to(dt)
     z = (-s.float() * ((1 << bits) - 1) / 2 * 0.9).to(dt)
     w = ops.unpack(qw, bits).double() * s.double().repeat_interleave(g, 1) + z.double().repeat_interleave(g, 1)
-    for m in (8, 20):
+    for m in (6, 8, 20):
         x = extremes(dt, m, k, m)
         y = ops.quantized_matmul(x, qw, s, z, group_size=g, bits=bits)
         eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11

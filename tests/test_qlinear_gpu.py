@@ -209,9 +209,9 @@ def test_skinny_mfma_tiles(ops, oracle, c_oracle, bits, g, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(32, 24576, 1024), (7, 12288, 2048), (16, 6144, 3072), (2, 4096, 4096), (32, 1000, 1024),
                                    (25, 4096, 14336), (33, 24576, 1024), (64, 28672, 1024)])
 def test_batch_kernel_no_dequant(ops, oracle, c_oracle, bits, dt, m, n, k):
-    """2 <= M <= 32, group 128: integer fields straight to the matrix cores, affine map per group on the accumulators
-    (mfma_batch.hip) -- every workgroup shape (128 / 64 / 32 / 16 rows), 1..14 steps, ragged N and M, both activation
-    dtypes, bias as a second rounding."""
+    """2 <= M <= 32, group 128: integer fields straight to the matrix cores, affine map per group on the accumulators, ragged N and M,
+    both activation dtypes, bias as a second rounding.  K up to 4096 runs in mfma_slab_impl.h, 14336 split in mfma_batch.hip (its unsplit
+    workgroups: test_qgemm_rows_gpu.py)."""
     d = oracle.synth_layer(n, k, bits, 128, seed=m + bits + n % 13, m=m, act_dtype=dt, bias=(n == 6144))
     x = d["x"].clone()
     x[0, 5] = 90.0                       # an outlier: the per-group offset term (C * xsum) must cancel exactly enough
@@ -226,8 +226,8 @@ def test_batch_kernel_no_dequant(ops, oracle, c_oracle, bits, dt, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(32, 24576, 1024), (9, 12288, 2048), (16, 6144, 3072), (5, 4096, 4096), (32, 1000, 1024),
                                    (20, 4096, 14336)])
 def test_batch_kernel_small_groups(ops, oracle, c_oracle, g, m, n, k):
-    """2-bit weights with groups of 64 / 32 on the no-dequant kernel: the k assignment is interleaved so that every MFMA
-    step stays inside one group, 2 / 4 affine flushes per chunk; every workgroup shape, ragged N."""
+    """2-bit weights with groups of 64 / 32 on the no-dequant kernels: the k assignment is interleaved so that every MFMA
+    step stays inside one group, 2 / 4 affine flushes per chunk; ragged N.  K = 14336 runs in mfma_batch.hip, the rest in mfma_slab_impl.h."""
     for dt in ("bf16", "f16"):
         d = oracle.synth_layer(n, k, 2, g, seed=m + g + n % 11, m=m, act_dtype=dt)
         x = d["x"].clone()

@@ -1,5 +1,5 @@
-"""Rows of recurrent mixers in groups of four channels (csrc/mixers_state.hip, mixers_headscan.hip): preparation with and without a convolution, eight rows a thread
-and one, sequences that start, go on or end inside a thread's rows, a slot used before, and both norms, against the forms for any layout (the same
+"""Rows of recurrent mixers in groups of four channels (csrc/mixers_state.hip, mixers_headscan.hip): preparation with and without a convolution, one row a thread and
+eight, sequences that start, go on or end inside a thread's rows, a slot used before, and both norms, against the forms for any layout (the same
 tensors one element off the grid of their loads).  Tolerance: sums of up to 4096 squares in another order, 2^-20 in fp32, and one rounding to bf16."""
 import pytest
 import torch
@@ -28,9 +28,21 @@ def step(lens, first):
 @pytest.mark.parametrize("lens,first", [([5], [0]), ([1, 1, 1], [4, 0, 9]), ([700, 3, 1, 501], [0, 2, 0, 1]), ([1100, 1], [7, 3])])
 @pytest.mark.parametrize("conv,unit,G,H,dk,dv", [(True, True, 2, 4, 64, 32), (False, False, 4, 4, 256, 64), (True, False, 3, 3, 4, 8), (False, True, 1, 2, 128, 260)])
 def test_recurrent_prepare(dt, lens, first, conv, unit, G, H, dk, dv):
+    prepare(dt, lens, first, conv, unit, G, H, dk, dv)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens,first", [([700, 3, 1, 2, 501], [0, 2, 1, 0, 5]), ([1] * 9 + [850], [i % 5 for i in range(10)]), ([901, 8, 1, 8, 5], [3, 0, 4, 1, 2])])
+@pytest.mark.parametrize("conv,unit,G,H,dk,dv", [(True, True, 16, 32, 128, 128), (False, False, 16, 32, 128, 128), (True, False, 40, 40, 64, 64)])
+def test_recurrent_prepare_eight_rows_a_thread(dt, lens, first, conv, unit, G, H, dk, dv):
+    """Enough rows and channels for that form: sequences that start, go on and end inside a thread's eight, and a last thread of fewer."""
+    cols = -(-(2 * G * dk + H * dv + H * dk) // 1024)
+    assert sum(lens) * cols >= 8192 and sum(lens) % 8
+    prepare(dt, lens, first, conv, unit, G, H, dk, dv)
+
+
+def prepare(dt, lens, first, conv, unit, G, H, dk, dv):
     T, nq, nv = sum(lens), G * dk, H * dv
-    if T * (2 * nq + nv) > 4_000_000:
-        pytest.skip("more of the same")
     batch, slots = step(lens, first)
     lay = RM.RecurrentLayout(H, G, dk, dv, 0, nq, 2 * nq, 2 * nq + nv)
     gen = torch.Generator(device=DEV).manual_seed(T + dk)
