@@ -674,14 +674,6 @@ bool qgemm_batch_supported(int M, int K, int bits, int log2g) {
   return M >= 1 && M <= 32 && bits >= 2 && bits <= 4 && (log2g == 7 || (bits == 2 && (log2g == 6 || log2g == 5))) && K % 1024 == 0;
 }
 
-// (contractions under 1024: as launch_qgemm_rows; one row: what is left of 33, by the kernel of the other 32)
-hipError_t launch_qgemm_slab(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
-  uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
-  for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
-  if (a.swiglu || a.ws || a.M < 1 || a.M > 32 || a.K % 128 || a.K < 1024 || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
-  return bits == 2 ? launch_slab_bits<2>(a, bf16, s) : bits == 3 ? launch_slab_bits<3>(a, bf16, s) : bits == 4 ? launch_slab_bits<4>(a, bf16, s) : hipErrorInvalidValue;
-}
-
 hipError_t launch_qgemm_batch(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
   return bits == 2 ? launch_batch_bits<2>(a, bf16, s) : bits == 3 ? launch_batch_bits<3>(a, bf16, s) : launch_batch_bits<4>(a, bf16, s);
 }

@@ -61,29 +61,9 @@ __global__ __launch_bounds__(64 * RW) void qgemm_rows_kernel(MfmaArgs args) {
         }
       }
   };
-  // the rows in the order in which fields leave a word
   auto arrange = [&](Chunk& k) {
-    constexpr unsigned LO = 0x05040100u, HI = 0x07060302u;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      if constexpr (BITS == 4 || (BITS == 2 && GRP == 32)) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const packed_x4 v = k.x[i][t];
-          k.x[i][t] = packed_x4{__builtin_amdgcn_perm(v.z, v.x, LO), __builtin_amdgcn_perm(v.z, v.x, HI), __builtin_amdgcn_perm(v.w, v.y, LO),
-                                __builtin_amdgcn_perm(v.w, v.y, HI)};
-        }
-      } else if constexpr (BITS == 2) {                    // two steps share a word
-#pragma unroll
-        for (int t = 0; t < 4; t += 2) {
-          const packed_x4 l = k.x[i][t], h = k.x[i][t + 1];
-          k.x[i][t] = packed_x4{__builtin_amdgcn_perm(h.x, l.x, LO), __builtin_amdgcn_perm(h.x, l.x, HI), __builtin_amdgcn_perm(h.y, l.y, LO),
-                                __builtin_amdgcn_perm(h.y, l.y, HI)};
-          k.x[i][t + 1] = packed_x4{__builtin_amdgcn_perm(h.z, l.z, LO), __builtin_amdgcn_perm(h.z, l.z, HI), __builtin_amdgcn_perm(h.w, l.w, LO),
-                                    __builtin_amdgcn_perm(h.w, l.w, HI)};
-        }
-      }
-    }
+    for (int i = 0; i < MT; ++i) packed_order<BITS, GRP>(k.x[i]);
   };
   constexpr unsigned ONE = BF16 ? 0x3F803F80u : 0x3C003C00u;
   const packed_x4 ones{ONE, ONE, ONE, ONE};
@@ -196,6 +176,14 @@ hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
 }
 
 }  // namespace
+
+// (contractions under 1024: see below; one row: what is left of 33, by the kernel of the other 32)
+hipError_t launch_qgemm_slab(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
+  uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
+  for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
+  if (a.swiglu || a.ws || a.M < 1 || a.M > 32 || a.K % 128 || a.K < 1024 || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
+  return bits == 2 ? launch_slab_bits<2>(a, bf16, s) : bits == 3 ? launch_slab_bits<3>(a, bf16, s) : bits == 4 ? launch_slab_bits<4>(a, bf16, s) : hipErrorInvalidValue;
+}
 
 // Contractions under 1024 stay with the dequantising kernel although it is the slower one (16 rows of 4096 x 512, 4 bits, group 128: 5.7 us there, 3.2
 // here): models that small are held to recorded token histories, and their results keep their bits.

@@ -47,7 +47,9 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void each(F&&
   if constexpr (I < N) { fn(std::integral_constant<int, I>{}); each<N, I + 1>(fn); }
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_buffer(const void* p, int64_t first, int64_t end) {      // reads from `end` bytes on give zero
+// Reads from `end` bytes on give zero and make no access.  gfx950 takes the scalar offset into that check, and one that is past the end by itself reads nothing (lanes
+// of 64 bytes over 4096, scalar offsets 0, 1024, 4032, 4096 and 65 536: 64, 48, 1, 0 and 0 of them read; over 0 bytes none, from registers and to LDS alike).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_buffer(const void* p, int64_t first, int64_t end) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p)) + first, 0, static_cast<int>(end - first < 0x7FFFFFFF ? end - first : 0x7FFFFFFF), 0x00020000);
 }
 
@@ -135,30 +137,13 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
     unsigned mask = P::MASK, magic = P::MAGIC;
     asm("" : "+s"(mask));
     asm("" : "+v"(magic));
-    constexpr unsigned ONE = BF16 ? 0x3F803F80u : 0x3C003C00u, LO = 0x05040100u, HI = 0x07060302u;
+    constexpr unsigned ONE = BF16 ? 0x3F803F80u : 0x3C003C00u;
     const packed_x4 ones{ONE, ONE, ONE, ONE};
 #pragma unroll
     for (int j = 0; j < CW; ++j)
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
-        // the order in which fields leave a word
-        if constexpr (BITS == 4 || (BITS == 2 && GRP == 32)) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const packed_x4 v = x[j][i][t];
-            x[j][i][t] = packed_x4{__builtin_amdgcn_perm(v.z, v.x, LO), __builtin_amdgcn_perm(v.z, v.x, HI), __builtin_amdgcn_perm(v.w, v.y, LO),
-                                   __builtin_amdgcn_perm(v.w, v.y, HI)};
-          }
-        } else if constexpr (BITS == 2) {                  // two steps share a word
-#pragma unroll
-          for (int t = 0; t < 4; t += 2) {
-            const packed_x4 l = x[j][i][t], h = x[j][i][t + 1];
-            x[j][i][t] = packed_x4{__builtin_amdgcn_perm(h.x, l.x, LO), __builtin_amdgcn_perm(h.x, l.x, HI), __builtin_amdgcn_perm(h.y, l.y, LO),
-                                   __builtin_amdgcn_perm(h.y, l.y, HI)};
-            x[j][i][t + 1] = packed_x4{__builtin_amdgcn_perm(h.z, l.z, LO), __builtin_amdgcn_perm(h.z, l.z, HI), __builtin_amdgcn_perm(h.w, l.w, LO),
-                                       __builtin_amdgcn_perm(h.w, l.w, HI)};
-          }
-        }
+        packed_order<BITS, GRP>(x[j][i]);
 #pragma unroll
         for (int g = 0; g < NF; ++g) {
           f32x4v d{0.f, 0.f, 0.f, 0.f};

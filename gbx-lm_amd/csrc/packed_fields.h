@@ -10,6 +10,26 @@ namespace gbx {
 typedef unsigned packed_x2 __attribute__((ext_vector_type(2)));
 typedef unsigned packed_x4 __attribute__((ext_vector_type(4)));
 
+// A lane's four octets of a chunk of activations in the order in which fields leave a word.
+template <int BITS, int GRP>
+__device__ __forceinline__ void packed_order(packed_x4 (&x)[4]) {
+  constexpr unsigned LO = 0x05040100u, HI = 0x07060302u;
+  if constexpr (BITS == 4 || (BITS == 2 && GRP == 32)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const packed_x4 v = x[t];
+      x[t] = packed_x4{__builtin_amdgcn_perm(v.z, v.x, LO), __builtin_amdgcn_perm(v.z, v.x, HI), __builtin_amdgcn_perm(v.w, v.y, LO), __builtin_amdgcn_perm(v.w, v.y, HI)};
+    }
+  } else if constexpr (BITS == 2) {                        // two steps share a word
+#pragma unroll
+    for (int t = 0; t < 4; t += 2) {
+      const packed_x4 l = x[t], h = x[t + 1];
+      x[t] = packed_x4{__builtin_amdgcn_perm(h.x, l.x, LO), __builtin_amdgcn_perm(h.x, l.x, HI), __builtin_amdgcn_perm(h.y, l.y, LO), __builtin_amdgcn_perm(h.y, l.y, HI)};
+      x[t + 1] = packed_x4{__builtin_amdgcn_perm(h.z, l.z, LO), __builtin_amdgcn_perm(h.z, l.z, HI), __builtin_amdgcn_perm(h.w, l.w, LO), __builtin_amdgcn_perm(h.w, l.w, HI)};
+    }
+  }
+}
+
 template <int BITS, int GRP, bool BF16, int TILES = 4>
 struct Packed {
   static constexpr int NF = 128 / GRP;                     // groups per chunk
