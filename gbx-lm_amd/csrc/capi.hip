@@ -403,13 +403,9 @@ int gbx_attn_decode_normed(const void* q, const void* k, const void* v, void* kc
 }
 
 size_t gbx_attn_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t capacity) {
-  if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || capacity <= 0 || (head_dim != 64 && head_dim != 128)) return 0;
-  return gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity);
-}
-
-int32_t gbx_attn_splits(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t capacity, int32_t normed) {
-  if (batch <= 0 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || capacity <= 0) return 1;
-  return gbx::attn_splits(batch, n_heads, n_kv_heads, capacity, normed != 0);
+  const bool normed = batch < 0;
+  if (batch == 0 || batch == INT32_MIN || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || capacity <= 0 || (head_dim != 64 && head_dim != 128)) return 0;
+  return gbx::attn_workspace_bytes(normed ? -batch : batch, n_heads, n_kv_heads, head_dim, capacity, normed);
 }
 
 int gbx_attn_decode_ws(const void* q, const void* k, const void* v, void* kcache, void* vcache, const float* inv_freq,
@@ -431,7 +427,7 @@ int gbx_attn_decode_ws(const void* q, const void* k, const void* v, void* kcache
   if (!aligned(kcache, 16) || !aligned(vcache, 16)) return fail(GBX_ERR_INVALID, "KV cache must be 16-byte aligned");
   float* ws = nullptr;                              // enough caller scratch: long contexts are split over workgroups
   {
-    const size_t need = gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity);
+    const size_t need = gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity, q_norm_weight || q_bias);
     if (workspace && need && workspace_bytes >= need && aligned(workspace, 16)) ws = static_cast<float*>(workspace);
   }
   hipError_t e = gbx::launch_attn_decode(q, k, v, kcache, vcache, inv_freq, reinterpret_cast<const long long*>(pos), out,
@@ -459,7 +455,7 @@ int gbx_attn_decode_slices(const float* qkv_slices_ws, int32_t slices, void* kca
   if (!aligned(kcache, 16) || !aligned(vcache, 16) || !aligned(qkv_slices_ws, 4)) return fail(GBX_ERR_INVALID, "misaligned pointer");
   float* ws = nullptr;
   {
-    const size_t need = gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity);
+    const size_t need = gbx::attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim, capacity, true);
     if (workspace && need && workspace_bytes >= need && aligned(workspace, 16)) ws = static_cast<float*>(workspace);
   }
   hipError_t e = gbx::launch_attn_decode(nullptr, nullptr, nullptr, kcache, vcache, inv_freq, reinterpret_cast<const long long*>(pos), out,

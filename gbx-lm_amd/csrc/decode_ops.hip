@@ -684,7 +684,7 @@ static int split_heads(int batch, int n_heads, int rep, int capacity) {
 // Fewer heads a workgroup are as many workgroups already (16 on 8: 256 5.6 5.6 7.1 7.8 | 6.9 7.3 7.3 7.5; 7 on 1: 4.9 4.9 5.9 6.5 | 7.1 7.6 7.6 7.8).  From 1024 on,
 // context 512 and last, slices of 128 | 64 | 32 positions: 16 on 4 8.1 9.1 | 7.9 8.8 | 9.1 9.5, 32 on 4 8.9 10.1 | 9.1 10.1 | 9.1 10.1, 24 on 4 8.6 9.5 | 9.4 9.9 | 9.9 10.4.
 // Batches keep the rule of the longer caches: their sequences are workgroups.
-int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
+static int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
   const int rep = n_heads / n_kv;
   static const int force_r = gbx::env_switch("GBX_ATTN_SPLIT_R");   // tuning aid
   const int R = force_r ? force_r : split_heads(batch, n_heads, rep, capacity);
@@ -697,8 +697,8 @@ int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped) {
   return s < 2 ? 1 : s;
 }
 
-size_t attn_workspace_bytes(int batch, int n_heads, int n_kv, int head_dim, int capacity) {
-  const int s = attn_splits(batch, n_heads, n_kv, capacity, true);       // (never fewer than without the norms)
+size_t attn_workspace_bytes(int batch, int n_heads, int n_kv, int head_dim, int capacity, bool grouped) {
+  const int s = attn_splits(batch, n_heads, n_kv, capacity, grouped);
   return s > 1 ? static_cast<size_t>(batch) * n_heads * s * (head_dim + 2) * sizeof(float) : 0;
 }
 

@@ -121,7 +121,6 @@ hipError_t launch_attn_decode(const void* q, const void* k, const void* v, void*
                               const void* q_norm_w = nullptr, const void* k_norm_w = nullptr, float norm_eps = 0.f,
                               const void* q_bias = nullptr, const void* k_bias = nullptr, const void* v_bias = nullptr,
                               float* ws = nullptr, const float* qkv_ws = nullptr, int qkv_slices = 0);
-int attn_splits(int batch, int n_heads, int n_kv, int capacity, bool grouped);
 // p2p_allreduce.hip: one-shot push all-reduce of a short 16-bit vector over peer-mapped inboxes
 hipError_t launch_p2p_allreduce(void* x, int n, int rank, int world, void* const* inbox, int cap, void* state, bool bf16, hipStream_t s);
 // attn_oproj.hip: attention + o_proj slices of one decode token in one launch (short caches)
@@ -130,7 +129,7 @@ hipError_t launch_attn_oproj(const void* q, const void* k, const void* v, void* 
                              const long long* pos, const uint32_t* qweight, const void* scales, const void* zeros, long long* acc,
                              int n_heads, int n_kv, int head_dim, int capacity, int D, int bits, int log2g, float rope_scale,
                              float sm_scale, int traditional, bool bf16, hipStream_t s);
-size_t attn_workspace_bytes(int batch, int n_heads, int n_kv, int head_dim, int capacity);
+size_t attn_workspace_bytes(int batch, int n_heads, int n_kv, int head_dim, int capacity, bool grouped);
 hipError_t launch_dense_gemv(const void* x, const void* w, void* y, const void* norm_w, float eps, int N, int K, void* best,
                              bool bf16, hipStream_t s, int index_offset = 0);
 hipError_t launch_embed_next(void* best, void* tok_io, void* pos, const void* table, void* h, int D, int vocab, int mode,

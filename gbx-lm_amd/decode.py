@@ -403,12 +403,11 @@ class FusedDecodeRunner(DecodeRunner):
             self.all_keys = torch.zeros((64 * model.tp_world,), dtype=torch.int64, device=dev)
             self.logits_full = torch.zeros((1, self.tp_vocab[2]), dtype=dt, device=dev)
         from . import _lib as _l
-        shape = (1, a0.n_heads, a0.n_kv_heads)
+        shape = (a0.n_heads, a0.n_kv_heads, a0.head_dim, caches[0].capacity)
         normed = any(getattr(b.self_attn, "q_norm", None) is not None or b.self_attn.q_proj.bias is not None for b in model.model.layers)
-        need = _l.lib().gbx_attn_workspace_bytes(*shape, a0.head_dim, caches[0].capacity)
-        split = _l.lib().gbx_attn_splits(*shape, caches[0].capacity, int(normed)) > 1          # the attention launch of its own splits the context
-        self.attn_ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need and split else None
-        self.long_cache = _l.lib().gbx_attn_splits(*shape, caches[0].capacity, 0) > 1          # too long for one workgroup per head's whole context
+        need = _l.lib().gbx_attn_workspace_bytes(-1 if normed else 1, *shape)                  # the attention launch of its own splits the context
+        self.attn_ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need else None
+        self.long_cache = _l.lib().gbx_attn_workspace_bytes(1, *shape) > 0                     # too long for one workgroup per head's whole context
         self.chain = False                  # True while capturing / replaying the on-device greedy chain
         self.graph_chain = None
         # Short caches (no context split): attention + o_proj as ONE launch whose partial sums land in a fixed-point

@@ -1206,10 +1206,8 @@ def attn_oproj_decode(q, k, v, kcache, vcache, inv_freq, pos, o_proj, acc, n_hea
 
 def _attn_scratch(b: int, n_heads: int, n_kv: int, head_dim: int, cap: int, grouped: bool, device) -> Optional[torch.Tensor]:
     """Scratch for the slices of a launch that splits its context (flash-decoding), none for one that does not."""
-    L = _lib.lib()
-    if L.gbx_attn_splits(b, n_heads, n_kv, cap, int(grouped)) <= 1:
-        return None
-    return torch.empty((L.gbx_attn_workspace_bytes(b, n_heads, n_kv, head_dim, cap),), dtype=torch.uint8, device=device)
+    need = _lib.lib().gbx_attn_workspace_bytes(-b if grouped else b, n_heads, n_kv, head_dim, cap)
+    return torch.empty((need,), dtype=torch.uint8, device=device) if need else None
 
 
 def attn_decode_batched(q, k, v, kcache, vcache, inv_freq, pos, out, n_heads: int, n_kv: int, head_dim: int,

@@ -542,12 +542,11 @@ int gbx_attn_decode_normed(const void* q, const void* k, const void* v, void* kc
                            const void* k_bias, const void* v_bias, int32_t act_dtype, void* hip_stream);
 
 /* gbx_attn_decode_normed with caller-owned scratch of gbx_attn_workspace_bytes(batch, n_heads, n_kv_heads, head_dim,
- * capacity) bytes (16-byte aligned; 0 = no use for it, whatever the launch; gbx_attn_splits says it for one launch): once the cache is long the cached positions of a (kv group,
+ * capacity) bytes (16-byte aligned; 0 = no use for it): once the cache is long the cached positions of a (kv group,
  * sequence) are split over several workgroups (flash-decoding) and a second launch merges their (max, sum, numerator)
- * partials -- the per-head kernel reads a 2048-token context with 32 workgroups. */
+ * partials -- the per-head kernel reads a 2048-token context with 32 workgroups.  Launches with query / key norms or biases, and those of
+ * gbx_attn_decode_slices, split one sequence's shorter caches too: for them the size is that of `batch` with a minus sign. */
 size_t gbx_attn_workspace_bytes(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t capacity);
-/* Slices that such a launch splits the context into (1: it does not); normed: with query / key norms or biases, which split one sequence from 256 positions on. */
-int32_t gbx_attn_splits(int32_t batch, int32_t n_heads, int32_t n_kv_heads, int32_t capacity, int32_t normed);
 int gbx_attn_decode_ws(const void* q, const void* k, const void* v, void* kcache, void* vcache, const float* inv_freq,
                        const int64_t* pos, void* out, int32_t batch, int32_t n_heads, int32_t n_kv_heads,
                        int32_t head_dim, int32_t capacity, float rope_scale, float sm_scale, int32_t traditional,

@@ -37,7 +37,7 @@ def test_split_context_against_float64(hd, nh, nkv, cap):
     from gbx_lm_amd import _lib
     rep = nh // nkv
     expect = cap >= 1024 or (cap >= 256 and (rep % 4 == 0 or rep % 3 == 0))
-    assert (_lib.lib().gbx_attn_splits(1, nh, nkv, cap, 1) > 1) == expect
+    assert (_lib.lib().gbx_attn_workspace_bytes(-1, nh, nkv, hd, cap) > 0) == expect and (_lib.lib().gbx_attn_workspace_bytes(1, nh, nkv, hd, cap) > 0) == (cap >= 1024)
     q, k, v, kc, vc, qw, kw, inv = operands(hd, nh, nkv, cap)
 
     def turned(x, w, pos):
@@ -65,7 +65,7 @@ def test_split_context_against_float64(hd, nh, nkv, cap):
 def test_split_context_against_a_batch_of_the_same_sequence_twice(hd, nh, nkv, cap):
     """Batches are not split at these sizes.  The two sums run over the same products in another order (fp32), their result is rounded once."""
     from gbx_lm_amd import _lib
-    assert _lib.lib().gbx_attn_splits(1, nh, nkv, cap, 1) > 1 and _lib.lib().gbx_attn_splits(2, nh, nkv, cap, 1) == 1
+    assert _lib.lib().gbx_attn_workspace_bytes(-1, nh, nkv, hd, cap) > 0 and _lib.lib().gbx_attn_workspace_bytes(-2, nh, nkv, hd, cap) == 0
     q, k, v, kc, vc, qw, kw, inv = operands(hd, nh, nkv, cap)
     for pos in (0, 1, 15, 31, 32, 47, 63, cap - 1):
         (one, k1, v1), (two, k2, v2) = (attend(q, k, v, kc, vc, qw, kw, inv, pos, nh, nkv, hd, b) for b in (1, 2))
@@ -120,5 +120,5 @@ def test_scratch_only_where_the_context_is_split(normed, cap):
     torch.cuda.reset_peak_memory_stats()
     before = torch.cuda.memory_allocated()
     ops.attn_decode_batched(q, k, v, kc, vc, inv, p, out, nh, nkv, hd, 1.0, hd ** -0.5, False, w, w, 1e-6)
-    split = _lib.lib().gbx_attn_splits(1, nh, nkv, cap, int(normed)) > 1
+    split = _lib.lib().gbx_attn_workspace_bytes(-1 if normed else 1, nh, nkv, hd, cap) > 0
     assert split == (normed and cap >= 256 or cap == 4096) and (torch.cuda.max_memory_allocated() > before) == split
