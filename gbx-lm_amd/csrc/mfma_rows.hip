@@ -1,5 +1,5 @@
-// Quantised products of 2 to 32 rows over contractions whose rows do not fit the registers (beyond 4096; shorter ones: mfma_slab_impl.h), outside the group-128
-// batch kernel.
+// Quantised products of 2 to 32 rows over contractions whose rows do not fit the registers (beyond 4096; shorter ones: mfma_slab_impl.h, except for few rows off the
+// grid of 1024), outside the batch kernel.
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
 // A workgroup takes 16 NT outputs, its waves share out the chunks of 128 of K; packed words, scales and the rows' image go straight to the registers of
 // the lane that feeds them to the matrix cores (packed_fields.h), one chunk ahead of the one being multiplied; sum_k x comes from the matrix cores too
@@ -157,8 +157,9 @@ hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
     if (bf16) qgemm_rows_kernel<BITS, GRP, true, MT, NT><<<grid, 64 * RW, 0, s>>>(a);               \
     else qgemm_rows_kernel<BITS, GRP, false, MT, NT><<<grid, 64 * RW, 0, s>>>(a);                   \
   } while (0)
-  // 32 outputs a workgroup share the rows' image where that still leaves a workgroup for every CU (3 bits, group 64, 27 rows, 16 | 32 outputs, us:
-  // 4096 x 4096 12.8 | 17.1, 8192 x 3072 19.2 | 13.9)
+  // 32 outputs a workgroup share the rows' image where that still leaves a workgroup for every CU (16 | 32 outputs, us, 2, 8 and 27 rows: 3 bits, group 64, 4096 x 4224
+  // 6.3 7.0 10.6 | 8.8 9.3 12.8, 4112 x 4224 8.7 10.1 18.6 | 8.8 9.4 12.9, 8192 x 11008 21.1 24.8 43.8 | 19.5 21.4 30.1; 4 bits, group 32, 4096 x 11008 17.8 20.2 31.1 | 28.7
+  // 31.6 53.3, 4112 x 11008 30.3 35.8 58.0 | 28.6 31.7 53.4)
   if (a.N > 4096) GBX_QROWS(2);
   else GBX_QROWS(1);
 #undef GBX_QROWS

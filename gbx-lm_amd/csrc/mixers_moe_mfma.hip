@@ -14,12 +14,13 @@
 // a barrier apart, so that one group multiplies while the other reads fragments and issues requests.  Stages of 64 elements, because a row
 // piece is then a whole 128-byte line: 256 x 128 tiles with stages of 32 elements and two workgroups per CU spent their time on twice the L2
 // requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
-// Measured (us, first + second products with the sort; 128-pair tiles and weight fragments straight from the matrices -> 256-pair tiles -> results by rows):
-//   27 848 pairs, 128 experts, 2048 x 768 gated:  1 027 -> 480 -> 462 (570 TFLOP/s, 2.6 TB/s of weights)
-//   18 128 pairs of the same:                       794 -> 357 -> 331 (3.7 TB/s)
-//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 856 -> 422 -> 398; a factor of the weights' way from memory (one expert's for all: 269) and of the results'
-//   (kept back: 324), which tiles of one round write at the same time
-//    8 192 pairs,   8 experts, 4096 x 2048 gated:   975 -> 457 -> 444 (930 TFLOP/s)
+// Measured (us, first + second products with the sort; 256-pair tiles with results from the registers -> results by rows, in turn on one card, uniform choices, the least of
+// four places of the weights in memory, which move these times by up to a tenth):
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (620 TFLOP/s, 2.9 TB/s of weights)
+//   18 128 pairs of the same:                       340 -> 326 (3.7 TB/s)
+//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 437 -> 422; a factor of the weights' way from memory (one expert's for all: 150 less) and of the results' (kept back:
+//   75 less), which tiles of one round write at the same time
+//    8 192 pairs,   8 experts, 4096 x 2048 gated:   461 -> 457 (900 TFLOP/s)
 // The table keeps a lower tile beside its expert's others.  By falling height, so that the last round is short, tiles read their weights anew: 256 pairs an
 // expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  Requests of a whole stage ahead, or its lines ordered into L2
 // before, gain nothing.
