@@ -21,6 +21,11 @@ import torch
 from . import env, graphs
 
 
+# Rows up to which the host writes a step's tables entry by entry: the device's kernel starts behind a copy of its own (us a table, host's time / until it is there, host |
+# device: 1 row 17 / 20 | 22 / 35, 64 rows 24 / 27 | 23 / 34, 200 38 / 42 | 23 / 35, 8 192 1 009 / 1 023 | 23 / 35; 32 sequences of one row 39 / 42 | 30 / 42).
+HOST_ROWS = 64
+
+
 @dataclass
 class StepBatch:
     """One step's layout.  Host lists (one item per sequence of the step) and their device images."""
@@ -61,21 +66,21 @@ class StepBatch:
             rows += n
             n_tiles += -(-n // q_tile)
         nb, dev = len(tile0), torch.device(device)
-        head = torch.tensor(seq + tile0, dtype=torch.int32)
-        if dev.type == "cuda":                          # the tables of rows and tiles are written on the device
-            head = head.pin_memory().to(dev, non_blocking=True)
+        if dev.type == "cuda" and rows > HOST_ROWS:
+            from . import _lib, ops
+            head = torch.tensor(seq + tile0, dtype=torch.int32).pin_memory().to(dev, non_blocking=True)
             tables = torch.empty((2 * (rows + n_tiles),), dtype=torch.int32, device=dev)
             tok, tiles = tables[:2 * rows].view(rows, 2), tables[2 * rows:].view(n_tiles, 2)
-            if nb:
-                from . import _lib, ops
-                _lib.check_mixers(_lib.mixers().gbxm_step_tables(head.data_ptr(), head.data_ptr() + 16 * nb, tok.data_ptr(), tiles.data_ptr(), nb, rows, n_tiles, q_tile,
-                                                                 ops._stream_ptr(tables.device)))
-        else:
-            firsts, counts = head[:4 * nb].view(nb, 4), torch.tensor([-(-n // q_tile) for n in n_new], dtype=torch.long)
-            b, t = (torch.repeat_interleave(torch.arange(nb, dtype=torch.int32), c) for c in (firsts[:, 2].long(), counts))
-            tok = torch.stack([b, firsts[b.long(), 1] + torch.arange(rows, dtype=torch.int32) - firsts[b.long(), 3]], 1)
-            tiles = torch.stack([t, (torch.arange(n_tiles, dtype=torch.int32) - head[4 * nb:][t.long()]) * q_tile], 1)
-        return StepBatch(list(slot), list(pos0), list(n_new), rows, head[:4 * nb].view(nb, 4), tok, q_tile, tiles)
+            _lib.check_mixers(_lib.mixers().gbxm_step_tables(head.data_ptr(), head.data_ptr() + 16 * nb, tok.data_ptr(), tiles.data_ptr(), nb, rows, n_tiles, q_tile,
+                                                             ops._stream_ptr(tables.device)))
+            return StepBatch(list(slot), list(pos0), list(n_new), rows, head[:4 * nb].view(nb, 4), tok, q_tile, tiles)
+        tok = [v for b, (p, n) in enumerate(zip(pos0, n_new)) for i in range(n) for v in (b, p + i)]
+        tiles = [v for b, n in enumerate(n_new) for t in range(0, n, q_tile) for v in (b, t)]
+        packed = torch.tensor(seq + tok + tiles, dtype=torch.int32)
+        if dev.type == "cuda":
+            packed = packed.pin_memory().to(dev, non_blocking=True)
+        return StepBatch(list(slot), list(pos0), list(n_new), rows, packed[:4 * nb].view(nb, 4), packed[4 * nb:4 * nb + 2 * rows].view(rows, 2), q_tile,
+                         packed[4 * nb + 2 * rows:].view(n_tiles, 2))
 
 
 class _DecodeGraph:

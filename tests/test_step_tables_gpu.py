@@ -1,11 +1,11 @@
-"""The tables of a step's rows and query tiles, written on the device (csrc/mixers_ops.hip: step_tables_kernel): whole numbers, equal to those made entry by entry."""
+"""The tables of a step's rows and query tiles, beyond 64 rows written on the device (csrc/mixers_ops.hip: step_tables_kernel): whole numbers, equal to those made entry by entry."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("lens,q_tile", [([1], 128), ([128, 129, 127, 1], 128), ([1] * 300, 128), ([7, 8192, 1, 256, 255], 128), ([5, 64, 65], 32), ([3, 1, 2], 1)])
+@pytest.mark.parametrize("lens,q_tile", [([1], 128), ([128, 129, 127, 1], 128), ([1] * 300, 128), ([7, 8192, 1, 256, 255], 128), ([5, 64, 65], 32), ([3, 1, 2], 1), ([64], 32), ([65], 32), ([1] * 64, 128), ([1] * 65, 128)])
 def test_rows_and_tiles(lens, q_tile):
     from gbx_lm_amd.batching import StepBatch
     first = [(i * 37) % 11 for i in range(len(lens))]
