@@ -23,11 +23,11 @@ extern "C" {
 int gbxm_version(void);
 const char* gbxm_last_error(void);
 
-/* x[t] = table[token[t]] * scale (fp32 stream) and its image h in the activation dtype (rows h_row elements apart; h may be null:
- * no image is written). */
 /* Tables of a step from its sequences: seq [B][4] (slot, first position, rows, first row of the step), tile0 [B] first query tile of each; every sequence has a row.
  * tok [T][2] <- (sequence, position) of every row; tiles [n_tiles][2] <- (sequence, first row of the tile inside it).  8-byte aligned. */
 int gbxm_step_tables(const int32_t* seq, const int32_t* tile0, int32_t* tok, int32_t* tiles, int32_t B, int32_t T, int32_t n_tiles, int32_t q_tile, void* stream);
+/* x[t] = table[token[t]] * scale (fp32 stream) and its image h in the activation dtype (rows h_row elements apart; h may be null:
+ * no image is written). */
 int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* h, int64_t h_row, int64_t T, int32_t width, float scale,
                       int32_t act, void* stream);
 /* out[r] = x[r] - lse(x[r]), lse = log sum exp over the row's n values in fp32, rounded to the rows' type (`type`: also GBXM_F16). */
