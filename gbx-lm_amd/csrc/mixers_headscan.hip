@@ -371,7 +371,8 @@ __global__ __launch_bounds__(NTH) void gate_group_norm_kernel(const float* __res
   for (int c = threadIdx.x + GR * NTH; c < size; c += NTH) y[c] = from_f32<T>(value(c) * r * w[first + c]);
 }
 
-// The same in groups of four channels, parts of up to 4 NTH V channels.  Measured, us: 8 192 rows of 4 096 in one part 70 -> 40, in eight 82 -> 64.
+// The same in groups of four channels, parts of up to 4 NTH V channels; V is what the part needs (8 192 rows of 1 280 in one part with V = 4 26 us, 2 17; one number a lane 22).
+// Measured, us: 8 192 rows of 4 096 in one part 70 -> 40, in eight 82 -> 64; 1 600 of 2 048 7.8 -> 6.2.
 template <typename T, bool FAST, int NTH, int V>
 __global__ __launch_bounds__(NTH) void gate_group_norm_vec_kernel(const float* __restrict__ o, const T* __restrict__ z, int64_t z_stride, const float* __restrict__ w,
                                                                  T* __restrict__ out, int64_t out_stride, int groups, int size, float eps) {
@@ -416,9 +417,17 @@ int launch_gate_norm(const float* o, const void* z, int64_t zs, const float* w, 
   const T* zp = static_cast<const T*>(z);
   T* op = static_cast<T*>(out);
   if (size % 4 == 0 && size <= 4096 && zs % 4 == 0 && os % 4 == 0 && all_aligned(4 * sizeof(T), zp, static_cast<const T*>(op)) && all_aligned(16, o, w)) {
-    if (size <= 256) gate_group_norm_vec_kernel<T, FAST, 64, 1><<<grid, 64, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
-    else if (size <= 1024) gate_group_norm_vec_kernel<T, FAST, 128, 2><<<grid, 128, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
-    else gate_group_norm_vec_kernel<T, FAST, 256, 4><<<grid, 256, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
+    const auto go = [&](auto nth, auto v) {
+      gate_group_norm_vec_kernel<T, FAST, nth.value, v.value><<<grid, nth.value, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);
+    };
+    typedef std::integral_constant<int, 1> one; typedef std::integral_constant<int, 2> two; typedef std::integral_constant<int, 3> three; typedef std::integral_constant<int, 4> four;
+    typedef std::integral_constant<int, 64> w1; typedef std::integral_constant<int, 128> w2; typedef std::integral_constant<int, 256> w4;
+    if (size <= 256) go(w1{}, one{});
+    else if (size <= 512) go(w2{}, one{});
+    else if (size <= 1024) go(w2{}, two{});
+    else if (size <= 2048) go(w4{}, two{});
+    else if (size <= 3072) go(w4{}, three{});
+    else go(w4{}, four{});
     return after_launch("gate_group_norm");
   }
   if (size <= 256) gate_group_norm_kernel<T, FAST, 64><<<grid, 64, 0, s>>>(o, zp, zs, w, op, os, groups, size, eps);

@@ -98,7 +98,7 @@ def test_norms(dt):
         o, gate = torch.randn((rows, heads * dv), device=DEV, generator=gen), torch.randn((rows, heads * dv), device=DEV, generator=gen).to(dt)
         w = torch.rand(dv, device=DEV, generator=gen) if weighted else None
         same(M.head_norm_gate(o, gate, w, heads, 1e-5, 1 if kind == "silu" else 2), M.head_norm_gate(o, off(gate), w, heads, 1e-5, 1 if kind == "silu" else 2))
-    for rows, groups, size in ((1, 1, 4), (9, 3, 252), (5, 8, 512), (6, 1, 1024), (4, 2, 2056), (3, 1, 4096)):
+    for rows, groups, size in ((1, 1, 4), (9, 3, 252), (5, 2, 260), (5, 8, 512), (3, 3, 516), (6, 1, 1024), (4, 2, 1028), (2, 1, 2048), (4, 2, 2056), (3, 1, 3072), (2, 2, 3076), (3, 1, 4096)):
         o, gate = torch.randn((rows, groups * size), device=DEV, generator=gen), torch.randn((rows, groups * size), device=DEV, generator=gen).to(dt)
         w = torch.rand(groups * size, device=DEV, generator=gen)
         same(M.gate_group_norm(o, gate, w, groups, 1e-5), M.gate_group_norm(o, off(gate), w, groups, 1e-5))
