@@ -186,19 +186,28 @@ hipError_t launch_qgemm_slab(const MfmaArgs& a, int bits, bool bf16, hipStream_t
   return bits == 2 ? launch_slab_bits<2>(a, bf16, s) : bits == 3 ? launch_slab_bits<3>(a, bf16, s) : bits == 4 ? launch_slab_bits<4>(a, bf16, s) : hipErrorInvalidValue;
 }
 
+// Contractions off the grid of eight chunks leave some of the register-resident kernel's waves without work and give the others as much as a longer one would, while
+// here every wave starts on one: few rows whose outputs fit one round stay here.  2-bit groups of 32, whose fields cost more to take apart here, do not; 3-bit ones stay with
+// more rows too where two row tiles of four chunks leave the registers no room for two tiles of weights.  Here | there, us, 4096 outputs, 2, 8, 16, 17 and 32 rows: x 1152, 4
+// bits, group 64 3.8 4.1 4.5 4.8 5.5 | 4.4 4.5 4.6 5.2 5.3, 3 bits, group 128 3.5 3.8 4.1 4.5 5.2 | 4.0 4.0 4.1 4.7 4.8; x 1408, 3 bits 3.6 3.9 4.3 4.8 5.5 | 4.2 4.2 4.4 4.9
+// 5.1; x 1536 4.5 4.9 5.4 5.7 6.6 | 4.5 4.6 4.7 5.3 5.5 and 3.7 4.0 4.5 4.9 5.8 | 4.2 4.2 4.3 4.9 5.0; x 3200 5.4 6.0 .. | 6.3 6.4 .. and 5.0 5.4 .. | 5.5 5.5 ..; 2 bits, group
+// 32, x 1152 4.7 5.1 5.9 6.8 8.1 | 4.7 4.7 4.8 5.5 5.6; 11008 outputs, x 1152 7.1 7.5 .. | 5.9 6.0 ..; there in parts of here, 3, 6, 12, 16, 17 and 32 rows: 3 bits, group 32,
+// x 1152 1.18 1.18 1.16 1.09 1.04 0.97, x 1664 1.09 1.08 1.05 1.00 0.97 0.87, x 2560 0.85 0.83 0.78 0.77 0.69 0.63, x 3200 0.95 0.93 0.90 0.89 1.28 1.18; 4 bits, group 32,
+// x 1152 1.08 1.05 0.99 0.96 1.01 0.92.
+static bool rows_start_evenly(const MfmaArgs& a, int bits) {
+  const int chunks = a.K >> 7;
+  if (chunks % RW == 0 || a.N > 4096) return false;
+  if (a.log2g == 5) return bits == 3 ? (chunks < 12 ? a.M <= 16 : chunks < 16 ? a.M <= 6 : chunks > 24 && a.M > 16) : bits == 4 && chunks < 12 && a.M <= 6;
+  return a.M <= (chunks < 12 ? (bits == 3 ? 16 : 12) : 6);
+}
+
 // Contractions under 1024 stay with the dequantising kernel although it is the slower one (16 rows of 4096 x 512, 4 bits, group 128: 5.7 us there, 3.2
 // here): models that small are held to recorded token histories, and their results keep their bits.
 hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
   uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
   for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
   if (a.swiglu || a.M < 2 || a.M > 32 || a.K % 128 || a.K < 128 * RW || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
-  // Contractions off the grid of eight chunks leave some of the register-resident kernel's waves without work and give the others as much as a longer one would, while
-  // here every wave starts on one: few rows (12 of up to eleven chunks, 6 of more) whose outputs fit one round stay here, groups of 32 excepted, whose fields cost more to take apart.  Here | there, us,
-  // 4096 outputs, 2, 8, 16, 17 and 32 rows: x 1152, 4 bits, group 64 3.8 4.1 4.5 4.8 5.5 | 4.4 4.5 4.6 5.2 5.3, 3 bits, group 128 3.5 3.8 4.1 4.5 5.2 | 4.0 4.0 4.1 4.7 4.8;
-  // x 1408, 3 bits 3.6 3.9 4.3 4.8 5.5 | 4.2 4.2 4.4 4.9 5.1; x 1536 4.5 4.9 5.4 5.7 6.6 | 4.5 4.6 4.7 5.3 5.5 and 3.7 4.0 4.5 4.9 5.8 | 4.2 4.2 4.3 4.9 5.0; x 3200
-  // 5.4 6.0 .. | 6.3 6.4 .. and 5.0 5.4 .. | 5.5 5.5 ..; 2 bits, group 32, x 1152 4.7 5.1 5.9 6.8 8.1 | 4.7 4.7 4.8 5.5 5.6; 11008 outputs, x 1152 7.1 7.5 .. | 5.9 6.0 ..
-  const int chunks = a.K >> 7;
-  if (!(chunks % RW && a.M <= (chunks < 12 ? 12 : 6) && a.N <= 4096 && a.log2g > 5))
+  if (!rows_start_evenly(a, bits))
     if (const hipError_t e = launch_qgemm_slab(a, bits, bf16, s); e != hipErrorInvalidValue) return e;
   return bits == 2 ? launch_rows<2>(a, bf16, s) : bits == 3 ? launch_rows<3>(a, bf16, s) : bits == 4 ? launch_rows<4>(a, bf16, s) : hipErrorInvalidValue;
 }

@@ -428,8 +428,8 @@ void launch_head_norm_gate(const float* o, const void* gate, int64_t gate_stride
   const T* g = static_cast<const T*>(gate);
   T* y = static_cast<T*>(out);
   const int64_t blocks = (static_cast<int64_t>(H) * dv / 4 + NT - 1) / NT;
-  // (rows of less than 32 channels are a few lanes of a workgroup: 1 000 rows of one head of 16 2.6 us | 3.4)
-  if (H * dv >= 32 && dv >= 4 && dv <= 256 && !(dv & (dv - 1)) && gate_stride % 4 == 0 && out_row % 4 == 0 && all_aligned(4 * sizeof(T), g, static_cast<const T*>(y)) && all_aligned(16, o) &&
+  // (rows of less than 64 channels are a few lanes of a workgroup: 1 000 rows of one head of 16 2.6 us | 3.4, 629 of one of 32 2.5 | 3.2)
+  if (H * dv >= 64 && dv >= 4 && dv <= 256 && !(dv & (dv - 1)) && gate_stride % 4 == 0 && out_row % 4 == 0 && all_aligned(4 * sizeof(T), g, static_cast<const T*>(y)) && all_aligned(16, o) &&
       blocks <= 65535)
     head_norm_gate_vec_kernel<T, false><<<dim3(T_, static_cast<unsigned>(blocks)), NT, 0, s>>>(o, g, gate_stride, w, y, out_row, H * dv, dv, eps, kind);
   else
