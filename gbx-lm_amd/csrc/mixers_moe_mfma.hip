@@ -41,10 +41,11 @@ constexpr int BROW = 128 + 16;  // LDS bytes per activation row of a chunk (+16:
 // in registers; the order then forms in LDS and leaves in whole lines (scattered, a wave's stores take the address unit 64 cycles).  Beyond KEEP
 // pairs a thread the order is written in place, the further pairs count their bucket down from its end.
 // Bound by LDS atomics and trips to memory on one CU.  Two passes of atomics and scattered stores | this, us: 27 848 pairs of 128 experts 24.6 | 9.5, 16 384 of
-// 64 13.5 | 6.5, 256 of 128 4.2 | 4.2, 65 536 of 128 52.5 | 43.7.
-constexpr int KEEP = 32;
+// 64 13.5 | 6.5, 256 of 128 4.2 | 4.2, 65 536 of 128 52.5 | 43.7.  Up to FEW pairs a thread a form of their own: the other's code costs a launch 0.7 us.
+constexpr int KEEP = 32, FEW = 2;         // pairs a thread keeps; few pairs: straight to their places, and no more code than that (it is read cold)
 constexpr int SORT_LDS = (3 * 4097 + 5) * 4 + KEEP * 1024 * 2;           // (E <= 4096)
 
+template <int N>
 __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ idx, int* __restrict__ offsets, int* __restrict__ sorted,
                                                           int* __restrict__ tile_tab, int n_tiles, int rt, int P, int E1) {
   extern __shared__ int sm[];                 // counts [E1] | starts [E1 + 1] | first tile [E1] | tiles | the order, 16 bits a pair
@@ -52,23 +53,26 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   int* start = sm + E1;
   int* first = start + E1 + 1;
   unsigned short* order = reinterpret_cast<unsigned short*>(sm + ((3 * E1 + 2 + 3) & ~3));
-  const bool small = P <= KEEP * 1024;
+  constexpr int STEP = N < 8 ? N : 8;
+  const bool small = N > FEW && P <= N * 1024;
   const int tid = threadIdx.x;
   auto bucket = [&](int v) { return static_cast<int>(min(static_cast<unsigned>(v), static_cast<unsigned>(E1 - 1))); };
   for (int e = tid; e < E1; e += 1024) counts[e] = 0;
   __syncthreads();
-  int kept[KEEP], rank[KEEP];
+  int kept[N], rank[N];
 #pragma unroll
-  for (int c = 0; c < KEEP; c += 8)
+  for (int c = 0; c < N; c += STEP)
     if (c * 1024 < P) {
 #pragma unroll
-      for (int j = c; j < c + 8; ++j) kept[j] = bucket(idx[min(j * 1024 + tid, P - 1)]);
+      for (int j = c; j < c + STEP; ++j) kept[j] = bucket(idx[min(j * 1024 + tid, P - 1)]);
 #pragma unroll
-      for (int j = c; j < c + 8; ++j) rank[j] = j * 1024 + tid < P ? atomicAdd(&counts[kept[j]], 1) : 0;
+      for (int j = c; j < c + STEP; ++j) rank[j] = j * 1024 + tid < P ? atomicAdd(&counts[kept[j]], 1) : 0;
     }
   __syncthreads();                             // (every kept pair has its place before a further one is counted: the kept ones come first in their bucket)
-  for (int i = KEEP * 1024 + tid; i < P; i += 1024) atomicAdd(&counts[bucket(idx[i])], 1);
-  __syncthreads();
+  if constexpr (N > FEW) {
+    for (int i = N * 1024 + tid; i < P; i += 1024) atomicAdd(&counts[bucket(idx[i])], 1);
+    __syncthreads();
+  }
   if (tid < 64) {                              // one wave: running sums of pairs and tiles, 64 experts at a time
     int run = 0, tiles = 0;
     for (int e0 = 0; e0 < E1; e0 += 64) {
@@ -96,10 +100,10 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   }
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < KEEP; c += 8)
+  for (int c = 0; c < N; c += STEP)
     if (c * 1024 < P)
 #pragma unroll
-      for (int j = c; j < c + 8; ++j)
+      for (int j = c; j < c + STEP; ++j)
         if (j * 1024 + tid < P) {
           const int at = start[kept[j]] + rank[j];
           if (small) order[at] = j * 1024 + tid;
@@ -110,6 +114,7 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
     for (int t = 0; t < nt; ++t) { tile_tab[2 * (first[e] + t)] = e; tile_tab[2 * (first[e] + t) + 1] = start[e] + t * rt; }
   }
   for (int t = first[E1] + tid; t < n_tiles; t += 1024) tile_tab[2 * t] = -1;
+  if constexpr (N == FEW) return;
   __syncthreads();
   if (small) {                                 // (whole groups of four: expert_buckets_bytes rounds up to them)
     for (int i = tid * 4; i < P; i += 4096) {
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   }
   for (int e = tid; e < E1; e += 1024) counts[e] = start[e + 1];
   __syncthreads();
-  for (int i = KEEP * 1024 + tid; i < P; i += 1024) sorted[atomicSub(&counts[bucket(idx[i])], 1) - 1] = i;
+  for (int i = N * 1024 + tid; i < P; i += 1024) sorted[atomicSub(&counts[bucket(idx[i])], 1) - 1] = i;
 }
 
 // (the gated activations are forms of their own: a tile's epilogue repeats its activation a hundred times over)
@@ -474,12 +479,13 @@ int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBucke
   out->tile_tab = reinterpret_cast<int*>(w);
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_sort_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, SORT_LDS);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_sort_kernel<KEEP>), hipFuncAttributeMaxDynamicSharedMemorySize, SORT_LDS);
     if (e != hipSuccess) return hip_fail(e, "expert buckets");
     once.done();
   }
-  const int lds = ((3 * (E + 1) + 2 + 3) & ~3) * 4 + (P <= KEEP * 1024 ? (P + 3) / 4 * 8 : 0);
-  expert_sort_kernel<<<1, 1024, lds, s>>>(idx, out->offsets, out->sorted, out->tile_tab, out->tiles, rows, P, E + 1);
+  const int counters = ((3 * (E + 1) + 2 + 3) & ~3) * 4;
+  if (P <= FEW * 1024) expert_sort_kernel<FEW><<<1, 1024, counters, s>>>(idx, out->offsets, out->sorted, out->tile_tab, out->tiles, rows, P, E + 1);
+  else expert_sort_kernel<KEEP><<<1, 1024, counters + (P <= KEEP * 1024 ? (P + 3) / 4 * 8 : 0), s>>>(idx, out->offsets, out->sorted, out->tile_tab, out->tiles, rows, P, E + 1);
   return after_launch("expert buckets");
 }
 

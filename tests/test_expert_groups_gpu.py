@@ -84,9 +84,9 @@ def test_choices_share_rows_across_tiles():
     assert bool(((got - want).abs() <= 2.0 ** -8 * (want.abs() + spread) * 3 + 1e-6).all())
 
 
-@pytest.mark.parametrize("experts,pairs", [(8, 32768), (8, 32769), (5, 70000), (300, 40000)])
+@pytest.mark.parametrize("experts,pairs", [(8, 2047), (300, 2048), (8, 2049), (8, 32768), (8, 32769), (5, 70000), (300, 40000)])
 def test_more_pairs_than_the_sort_keeps(experts, pairs):
-    """The pairs beyond those whose places the sort holds in registers; uneven experts."""
+    """Either side of the few pairs that go straight to their places, and the pairs beyond those whose places the sort holds in registers; uneven experts."""
     w = torch.arange(1, experts + 1, dtype=torch.float64)
     counts = (w / w.sum() * pairs).long().tolist()
     counts[-1] += pairs - sum(counts)
