@@ -1,8 +1,9 @@
 // Matrix-core kernel of softmax attention with a sink for bf16 prompt portions (mechanism and key order: mixers_sink.hip).
 //
-// One workgroup = tiles of up to 128 query rows of one (sequence, head); a wave owns 32 queries, and one or two groups of four waves share a
-// tile's keys (SinkShape).  Key / value tiles of 64 (large heads and short sequences: 32) visible positions go global -> registers (one tile ahead) -> LDS once per
-// group.  Both products are computed swapped,
+// One workgroup = a tile of up to 128 query rows of one (sequence, head); a wave owns 32 queries, and one or two groups of four waves share the
+// tile's keys (SinkShape).  Key / value tiles of 64 (large heads and short sequences: 32) visible positions go global -> registers -> LDS once per
+// group, in two buffers: one barrier a tile, two tiles ahead.
+// Both products are computed swapped,
 //   S^T[key, q] = mfma(K rows, Q rows),    O^T[d, q] += mfma(V^T rows, P^T),
 // so that a lane owns ONE query: lane (q = lane % 32, half = lane / 32) holds 16 of the tile's 32 scores of its query, the other 16
 // are in lane ^ 32 (and as many of each further 32 keys).  The running maximum is shared by the two lanes of a query (one cross-lane exchange per tile), each keeps its
@@ -10,9 +11,10 @@
 // query) by the same factor.  The sink starts the running maximum and counts once in the denominator.  Weights are rounded to bf16
 // for the value product; the denominator sums them in fp32.
 //
-// Bound by vector instructions (one exponential, four others a score) and, in short prompts, by how few tiles there are: two groups halve the
-// chain of key tiles behind the last query tile.  Measured, 16 heads, us: <128, 128> 1 501 + 700 + 65 rows 144 -> 45, 4 000 rows 235 -> 130, 8 192 rows
-// 513 -> 469; <192, 128> 4 000 rows 289 -> 187, 8 192 rows 648 -> 658; <64, 64> 3 000 + 500 rows 134 -> 59.
+// Bound by what a wave's own chain leaves idle (of a tile's time the matrix cores work a third, vector instructions a third: one exponential and
+// four others a score) and, in short prompts, by how few tiles there are.  Before (one buffer, every row found by itself, tiles from both ends of
+// a prompt in one workgroup) | now, us: 16 heads of <192, 128>, 8 192 rows 545 | 395, 10 000 rows 1 169 | 620, 2 000 + 777 rows 73 | 58; <128, 128>,
+// 8 192 rows 400 | 302, 4 000 rows 117 | 92, 1 501 + 700 + 65 rows 44 | 35; <64, 64>, 3 000 + 500 rows 54 | 44; 8 heads of <256, 256>, 3 000 rows 324 | 188.
 //
 // Head sizes are run-time numbers (multiples of 8) inside a compiled capacity <DK, DV>: channels beyond them are staged as zeros.
 #include <algorithm>
@@ -59,22 +61,40 @@ __device__ __forceinline__ u32x2 out4(const SinkTileArgs& a, int64_t row, int he
 
 // With two GROUPS of four waves each takes every other key tile of the same queries, with a maximum and denominator of its own; the halves
 // meet in LDS at the end.
-template <int DK, int DV, int GROUPS_, int KT_> struct SinkShape {
-  static constexpr int GROUPS = GROUPS_, KT = KT_;           // KT: keys per tile
+template <int DK, int DV, int GROUPS_, int KT_, int BUFS_> struct SinkShape {
+  static constexpr int GROUPS = GROUPS_, KT = KT_, BUFS = BUFS_;   // KT: keys per tile; two buffers: a tile is read while the next is written
   static constexpr int KROW = DK * 2 + 16;                   // +16 B: conflict-free 16-byte fragment reads
   static constexpr int VROW = DV * 2 + 64;                   // pitch = 16 dwords mod 64: the 4 rows of a transposed block land on disjoint banks
-  static constexpr int BYTES = KT * (KROW + VROW);
+  static constexpr int BUF = KT * (KROW + VROW);             // one tile
+  static constexpr int BYTES = BUFS * BUF;                   // of a group
   static constexpr int JOIN = GROUPS > 1 ? 4 * (DV / 32 * 16 + 2) * 64 * 4 : 0;
   static constexpr int LDS = GROUPS * BYTES > JOIN ? GROUPS * BYTES : JOIN;
-  static constexpr int WAVES = DK + DV <= 320 ? 2 : 1;       // per SIMD
+  static constexpr bool MANY = GROUPS == 1 && BUFS == 1;     // short sequences live on many waves
+  static constexpr int WAVES = DK + DV <= (MANY ? 128 : 64) ? 4 : DK + DV <= 256 && MANY ? 3 : DK + DV <= 320 ? 2 : 1;   // per SIMD
+  // fragments read ahead: a key block's, as far as registers go
+  static constexpr int SLOTS = BUFS == 1 ? 0 : DK <= 192 ? DK / 16 : 8;
 };
 
-template <int DK, int DV, int GROUPS, int KT>
+// How the 256 threads of a group carry the rows of a tile, D channels each, in pieces of 16 bytes: `LANES` neighbouring threads a row, `PER`
+// pieces of it each, `ROWS` rows at a time; or, where a row's pieces do not fall into eights, piece after piece.
+template <int D, int KT> struct RowPieces {
+  static constexpr int C = D / 8, LANES = C % 16 == 0 ? 16 : C % 8 == 0 ? 8 : 4, PER = C / LANES, ROWS = 256 / LANES;
+  static constexpr bool LINEAR = C > 4 && LANES == 4;
+  static constexpr int N = LINEAR ? (KT * C + 255) / 256 : PER * ((KT + ROWS - 1) / ROWS);
+  __device__ static int row(int tid, int i) { return LINEAR ? (tid + 256 * i) / C : tid / LANES + i / PER * ROWS; }
+  __device__ static int piece(int tid, int i) { return LINEAR ? (tid + 256 * i) % C : tid % LANES + i % PER * LANES; }
+  __device__ static bool used(int tid, int i) { return (LINEAR ? KT * C % 256 == 0 : KT % ROWS == 0) || row(tid, i) < KT; }
+};
+
+template <int DK, int DV, int GROUPS, int KT, int BUFS>
 __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile, const int head, unsigned char* all_lds) {
-  typedef SinkShape<DK, DV, GROUPS, KT> Shape;
+  typedef SinkShape<DK, DV, GROUPS, KT, BUFS> Shape;
+  typedef RowPieces<DK, KT> KP;
+  typedef RowPieces<DV, KT> VP;
   constexpr int KROW = Shape::KROW, VROW = Shape::VROW, STEP = GROUPS * KT, NH = KT / 32;
   constexpr int KS = DK / 16, DT = DV / 32;
-  const int group = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char* kl = all_lds + group * Shape::BYTES;
   unsigned char* vl = kl + KT * KROW;
 
@@ -117,59 +137,127 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
+  const bf16_t *kc = a.kc + slot * a.kc_slot + kvh * a.kc_head, *kn = a.kn + kvh * a.k_head;
+  const bf16_t *vc = a.vc + slot * a.vc_slot + kvh * a.vc_head, *vn = a.vn + kvh * a.v_head;
+  auto cached = [&](int j) { return j < a.keep ? j : a.keep + (j - a.keep) % a.ring; };
   auto krow = [&](int j) -> const bf16_t* {
-    if (j < pos0) return a.kc + slot * a.kc_slot + static_cast<int64_t>(j < a.keep ? j : a.keep + (j - a.keep) % a.ring) * a.kc_row + kvh * a.kc_head;
-    return a.kn + static_cast<int64_t>(row0 + (j - pos0)) * a.k_row + kvh * a.k_head;
+    return j < pos0 ? kc + static_cast<int64_t>(cached(j)) * a.kc_row : kn + static_cast<int64_t>(row0 + (j - pos0)) * a.k_row;
   };
   auto vrow = [&](int j) -> const bf16_t* {
-    if (j < pos0) return a.vc + slot * a.vc_slot + static_cast<int64_t>(j < a.keep ? j : a.keep + (j - a.keep) % a.ring) * a.vc_row + kvh * a.vc_head;
-    return a.vn + static_cast<int64_t>(row0 + (j - pos0)) * a.v_row + kvh * a.v_head;
+    return j < pos0 ? vc + static_cast<int64_t>(cached(j)) * a.vc_row : vn + static_cast<int64_t>(row0 + (j - pos0)) * a.v_row;
   };
 
-  constexpr int KP = (KT * (DK / 8) + 255) / 256, VP = (KT * (DV / 8) + 255) / 256;
-  u32x4 kr[KP], vr[VP];
+  u32x4 kr[KP::N], vr[VP::N];
+  // 32 bits of byte offset reach across a tile's rows
+  const bool near = max(max(a.k_row, a.v_row), max(a.kc_row, a.vc_row)) < (1 << 22);
+  // Rows of a whole tile that follow each other in one buffer -- nearly all tiles of long sequences -- come by buffer loads: the tile's place is
+  // scalar, a lane adds a multiple of the stride, and channels beyond the head lie out of range and read as zeros.  Tiles that the end of the
+  // keys, the kept rows, the ring's seam or the first new row cuts find every row by itself (of 16 vector instructions per matrix product the
+  // search for rows was 10).
   auto fetch = [&](int it) {
+    const int j0 = pos_of(it), j1 = j0 + KT;
+    bool whole = BUFS == 2 && near && it + KT <= total && (it >= na || it + KT <= na);
+    int at = row0 + (j0 - pos0);
+    if (whole && j0 < pos0) {
+      at = cached(j0);
+      whole = j1 <= pos0 && (j1 <= a.keep || (j0 >= a.keep && at + KT <= a.keep + a.ring));
+    }
+    if (whole) {
+      const bool old = j0 < pos0;
+      const int ks = static_cast<int>(old ? a.kc_row : a.k_row) * 2, vs = static_cast<int>(old ? a.vc_row : a.v_row) * 2;
+      const bf16_t* kp = (old ? kc : kn) + static_cast<int64_t>(at) * (ks / 2);
+      const bf16_t* vp = (old ? vc : vn) + static_cast<int64_t>(at) * (vs / 2);
+      const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(kp), 0, (KT - 1) * ks + a.dk * 2, 0x00020000);
+      const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vp), 0, (KT - 1) * vs + a.dv * 2, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < KP; ++i) {
-      const int p = tid + 256 * i, row = p / (DK / 8), c = p % (DK / 8), iv = it + row;
-      kr[i] = u32x4{0, 0, 0, 0};
-      if (p < KT * (DK / 8) && iv < total && c * 8 < a.dk) kr[i] = *reinterpret_cast<const u32x4*>(krow(pos_of(iv)) + c * 8);
+      for (int i = 0; i < KP::N; ++i) {
+        const int c = KP::piece(tid, i), off = KP::row(tid, i) * ks + c * 16;
+        kr[i] = __builtin_amdgcn_raw_buffer_load_b128(krs, KP::used(tid, i) && c * 8 < a.dk ? off : 0x7ffffff0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < VP::N; ++i) {
+        const int c = VP::piece(tid, i), off = VP::row(tid, i) * vs + c * 16;
+        vr[i] = __builtin_amdgcn_raw_buffer_load_b128(vrs, VP::used(tid, i) && c * 8 < a.dv ? off : 0x7ffffff0, 0, 0);
+      }
+      return;
     }
 #pragma unroll
-    for (int i = 0; i < VP; ++i) {
-      const int p = tid + 256 * i, row = p / (DV / 8), c = p % (DV / 8), iv = it + row;
+    for (int i = 0; i < KP::N; ++i) {
+      const int iv = it + KP::row(tid, i), c = KP::piece(tid, i);
+      kr[i] = u32x4{0, 0, 0, 0};
+      if (KP::used(tid, i) && iv < total && c * 8 < a.dk) kr[i] = *reinterpret_cast<const u32x4*>(krow(pos_of(iv)) + c * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < VP::N; ++i) {
+      const int iv = it + VP::row(tid, i), c = VP::piece(tid, i);
       vr[i] = u32x4{0, 0, 0, 0};
-      if (p < KT * (DV / 8) && iv < total && c * 8 < a.dv) vr[i] = *reinterpret_cast<const u32x4*>(vrow(pos_of(iv)) + c * 8);
+      if (VP::used(tid, i) && iv < total && c * 8 < a.dv) vr[i] = *reinterpret_cast<const u32x4*>(vrow(pos_of(iv)) + c * 8);
     }
   };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < KP::N; ++i)
+      if (KP::used(tid, i)) *reinterpret_cast<u32x4*>(kl + buf * Shape::BUF + KP::row(tid, i) * KROW + KP::piece(tid, i) * 16) = kr[i];
+#pragma unroll
+    for (int i = 0; i < VP::N; ++i)
+      if (VP::used(tid, i)) *reinterpret_cast<u32x4*>(vl + buf * Shape::BUF + VP::row(tid, i) * VROW + VP::piece(tid, i) * 16) = vr[i];
+  };
+
+  // Two buffers, one barrier a tile: behind it tile t is in buffer t % 2 and tile t + 1 in registers; it is parked in the other buffer, whose
+  // readers have all passed the barrier, and tile t + 2 is asked for.  One buffer: tile t + 1 is asked for while tile t is read.
   const int i1 = group * KT, rounds = (total + STEP - 1) / STEP;        // (every group runs as many rounds: the barriers are common)
   if (i1 < total) fetch(i1);
+  if constexpr (BUFS == 2) {
+    if (i1 < total) stage(0);
+    if (i1 + STEP < total) fetch(i1 + STEP);
+  }
   for (int round = 0; round < rounds; ++round) {
     const int it = i1 + round * STEP;
-    __syncthreads();                                          // the previous tile has been consumed
-#pragma unroll
-    for (int i = 0; i < KP; ++i) {
-      const int p = tid + 256 * i;
-      if (p < KT * (DK / 8)) *reinterpret_cast<u32x4*>(kl + (p / (DK / 8)) * KROW + (p % (DK / 8)) * 16) = kr[i];
-    }
-#pragma unroll
-    for (int i = 0; i < VP; ++i) {
-      const int p = tid + 256 * i;
-      if (p < KT * (DV / 8)) *reinterpret_cast<u32x4*>(vl + (p / (DV / 8)) * VROW + (p % (DV / 8)) * 16) = vr[i];
-    }
     __syncthreads();
-    if (it + STEP < total) fetch(it + STEP);                  // the next tile travels while this one is computed
+    if constexpr (BUFS == 2) {
+      if (it + STEP < total) stage((round + 1) & 1);
+      if (it + 2 * STEP < total) fetch(it + 2 * STEP);
+    } else {
+      if (it < total) stage(0);
+      __syncthreads();
+      if (it + STEP < total) fetch(it + STEP);
+    }
     // wave-uniform: no key of the tile is seen by a query of this wave
     if (!wave_live || it >= total) continue;
     const int jmin = pos_of(it), jmax = pos_of(min(it + KT, total) - 1);
     if (jmin > wq1 || (jmax < wlo0 && jmin >= a.keep)) continue;
 
+    // fragments are read in bulk ahead of the products that take them; a slot is filled again as its product leaves
+    const unsigned char* kb = kbase + (BUFS == 2 ? round & 1 : 0) * Shape::BUF;
+    const unsigned char* vb = vbase + (BUFS == 2 ? round & 1 : 0) * Shape::BUF;
+    constexpr int NK = KS * NH, NV = DT * 2 * NH, SLOTS = Shape::SLOTS, NF = SLOTS < NV ? SLOTS : NV;
+    auto kfrag = [&](int i) { return *reinterpret_cast<const u32x4*>(kb + i / KS * 32 * KROW + i % KS * 32); };
+    auto vfrag = [&](int i) {
+      const int dt = i / (2 * NH), j = i % (2 * NH);
+      const u32x2 v0 = lds_read_tr(vb + 16 * j * VROW + dt * 64);
+      const u32x2 v1 = lds_read_tr(vb + (16 * j + 8) * VROW + dt * 64);
+      return u32x4{v0.x, v0.y, v1.x, v1.y};
+    };
+    u32x4 fr[SLOTS ? SLOTS : 1];
     f32x16 st[NH];
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      st[h] = f32x16{0};
+    for (int h = 0; h < NH; ++h) st[h] = f32x16{0};
+    if constexpr (SLOTS) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) st[h] = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + h * 32 * KROW + ks * 32), qf[ks], st[h]);
+      for (int i = 0; i < SLOTS; ++i) fr[i] = kfrag(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NK; ++i) {
+        st[i / KS] = mfma_bf16(fr[i % SLOTS], qf[i % KS], st[i / KS]);
+        if (i + SLOTS < NK) fr[i % SLOTS] = kfrag(i + SLOTS);
+        if (i % KS == KS - 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < NF; ++i) fr[i] = vfrag(i);           // the first fragments of V^T are read under the exponentials
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NK; ++i) st[i / KS] = mfma_bf16(kfrag(i), qf[i % KS], st[i / KS]);
     }
     // scores in units of ln 2 (the exponentials below are base 2).  Inside the mask -- every key of the tile before every query of the
     // wave, inside every window -- nothing is tested per score, the scale meets the maximum once and the rest inside the exponent.
@@ -203,39 +291,36 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
         }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                   // the other half of the query's scores
-    const float m_new = fmaxf(m, mx);
-    const float m_ref = m_new == -INFINITY ? 0.f : m_new;     // nothing seen yet and no sink: every weight below is 2^-inf = 0
-    const float alpha = __builtin_amdgcn_exp2f(m - m_ref);
-    const bool moved = m_new != m;
-    m = m_new;
-    float ps = 0.f;
-    const float f2 = inside ? scale2 : 1.f;
-#pragma unroll
-    for (int h = 0; h < NH; ++h)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) { st[h][e] = __builtin_amdgcn_exp2f(fmaf(st[h][e], f2, -m_ref)); ps += st[h][e]; }
-    l = l * alpha + ps;
-    if (__any(moved)) {                                       // wave-uniform: the maximum of no query of the wave has moved -> alpha is 1
+    // the sums move to a new maximum only where one grew by more than 2^8 (weights of up to 256 keep as many bits; the factor falls out at the
+    // end).  The first scores always move it; with nothing seen yet and no sink every weight below is 2^-inf = 0
+    if (__any(mx - m > 8.f)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
+      m = m_new;
+      l *= alpha;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
     }
+    const float m_ref = m == -INFINITY ? 0.f : m, f2 = inside ? scale2 : 1.f;
+    float ps = 0.f;
+    u32x4 pf[2 * NH];
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
-      u32x4 gf[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) { st[h][e] = __builtin_amdgcn_exp2f(fmaf(st[h][e], f2, -m_ref)); ps += st[h][e]; }
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
-        gf[tt] = u32x4{pack2(st[h][8 * tt], st[h][8 * tt + 1]), pack2(st[h][8 * tt + 2], st[h][8 * tt + 3]), pack2(st[h][8 * tt + 4], st[h][8 * tt + 5]),
-                       pack2(st[h][8 * tt + 6], st[h][8 * tt + 7])};
+        pf[2 * h + tt] = u32x4{pack2(st[h][8 * tt], st[h][8 * tt + 1]), pack2(st[h][8 * tt + 2], st[h][8 * tt + 3]),
+                               pack2(st[h][8 * tt + 4], st[h][8 * tt + 5]), pack2(st[h][8 * tt + 6], st[h][8 * tt + 7])};
+    }
+    l += ps;
+    if constexpr (SLOTS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-          const u32x2 v0 = lds_read_tr(vbase + (32 * h + 16 * tt) * VROW + dt * 64);
-          const u32x2 v1 = lds_read_tr(vbase + (32 * h + 16 * tt + 8) * VROW + dt * 64);
-          o[dt] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[dt]);
-        }
+    for (int i = 0; i < NV; ++i) {
+      o[i / (2 * NH)] = mfma_bf16(SLOTS ? fr[i % (NF ? NF : 1)] : vfrag(i), pf[i % (2 * NH)], o[i / (2 * NH)]);
+      if (SLOTS && i + NF < NV) fr[i % (NF ? NF : 1)] = vfrag(i + NF);
     }
   }
 
@@ -485,53 +570,51 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
   return launch_sink_reduce(a, splits, s);
 }
 
-// One group: a workgroup takes two query tiles, one from each end of the step's list -- in a long causal prompt a late tile (many keys) and an
-// early one (few) -- so that workgroups carry about the same work however they are spread over the chip; or (not PAIRED) one.  Two groups: a
-// tile each, of all heads the late ones first.
-template <int DK, int DV, int GROUPS, int KT, bool PAIRED>
-__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
+// A workgroup = a query tile of a head; tiles that see many keys, at the end of the step's list, go first.  Heads are the fast index, so that an
+// XCD's workgroups (every eighth) meet in few heads' keys.
+template <int DK, int DV, int GROUPS, int KT, int BUFS>
+__global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT, BUFS>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  if constexpr (PAIRED) {
-    const int pairs = (n_tiles + 1) / 2, second = blockIdx.x % pairs, first = n_tiles - 1 - second, head = blockIdx.x / pairs;
-    sink_tile<DK, DV, GROUPS, KT>(a, first, head, lds);
-    if (second != first) sink_tile<DK, DV, GROUPS, KT>(a, second, head, lds);
-  } else {
-    sink_tile<DK, DV, GROUPS, KT>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
-  }
+  sink_tile<DK, DV, GROUPS, KT, BUFS>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
 }
 
-template <int DK, int DV, int GROUPS, int KT, bool PAIRED>
+template <int DK, int DV, int GROUPS, int KT, int BUFS>
 int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
-  const unsigned grid = static_cast<unsigned>(t.H) * (PAIRED ? (n_tiles + 1) / 2 : n_tiles);
-  constexpr int bytes = SinkShape<DK, DV, GROUPS, KT>::LDS;
+  constexpr int bytes = SinkShape<DK, DV, GROUPS, KT, BUFS>::LDS;
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT, PAIRED>), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT, BUFS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hip_fail(e, "sink_attention (tiles)");
     once.done();
   }
-  sink_tile_kernel<DK, DV, GROUPS, KT, PAIRED><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles);
+  sink_tile_kernel<DK, DV, GROUPS, KT, BUFS><<<static_cast<unsigned>(t.H) * n_tiles, 256 * GROUPS, bytes, s>>>(t, n_tiles);
   return after_launch("sink_attention (tiles)");
 }
 
-// Tiles times heads up to which two groups share a tile.  Measured, one group against two, us, 16 heads: 12 + 6 + 1 tiles of <128, 128> 112 | 44; one prompt of
-// 32 tiles <192, 128> 282 | 187; 47 tiles 434 | 390; three of 20 334 | 250; 64 tiles 658 | 680, <128, 128> 469 | 466, <64, 64> 286 | 305.
-// Sequences of a tile's keys and less have no chain to share and nothing to balance: one group, 32 keys, a tile per workgroup.  The form that the line above gives |
-// this, us: 16 heads of <128, 128>, 20 rows 8.1 | 6.3, 20 rows x 16 8.4 | 6.5, x 64 14.6 | 11.9, 64 rows x 32 17.0 | 10.5 (32 heads: 18.6 | 19.9); <64, 128>, 100 rows x 200
-// 86 | 66; <96, 96> 86 | 68, but 128 rows x 64 30 | 32.5 and <128, 128>, 100 rows x 200 98 | 102, 40 rows x 200 95 | 100.  Large heads share tiles of 32 keys as it is: <192, 128>, 64 rows 8.7 | 9.5, x 16 9.5 |
-// 10.2, x 32 17.7 | 13.2, 20 rows 7.2 | 6.6.
-constexpr unsigned TWO_GROUPS = 960;
+// Which form, by tiles times heads n and the longest sequence's keys (0: unknown, long).  Measured in a replayed graph, us.
+// Up to 64 keys: one group, 32 keys, one buffer, the form with most waves (start-up is all there is: 1 x 20 rows, 16 heads of <128, 128> 6.4 | one
+// group of two buffers 7.8 | two groups 8.5; 64 x 20 rows 10.4 | 16.2 | 30.8); up to 224 also where there is more than a tile a CU: 64 x 200 60 | 70 |
+// 94, <64, 64> 64 x 100 17.7 | 23.9 | 33.4.
+// Two groups halve the chain of key tiles behind the last query tile, at one workgroup a CU.  Two groups | one of two buffers: 4 x 256 rows 13.3 |
+// 14.2, 2 x 500 17.8 | 21.0; small heads of few keys are done before a second buffer pays: two groups of one buffer | of two, <64, 64> 8 x 100 7.9 |
+// 8.6, <32, 32> 16 x 200 8.5 | 9.5.  Beyond a tile a CU only long chains gain: 8 x 500 37.5 | 31.4, 8 x 300 26.6 | 20.1, 4 x 1000 53.5 | 48.9, 2 x 1300
+// 34.8 | 46.9, 2 x 2000 61.9 | 78.2, 4 000 rows 93 | 125, <192, 128> 2 000 + 777 rows 58 | 90; a chip full of tiles has none to wait for: 7 000 rows
+// 251 | 234, 8 192 332 | 301, <192, 128> 8 192 457 | 390, 10 000 669 | 617.
+constexpr int TWO_GROUPS = 960;
 template <int DK, int DV>
 int launch(const SinkTileArgs& t, int n_tiles, int longest, hipStream_t s) {
   constexpr int KT = DK + DV > 256 ? 32 : 64;                // (larger heads: 64 would cost the second wave per SIMD)
   const int64_t n = static_cast<int64_t>(t.H) * n_tiles;
-  const int short_keys = n > TWO_GROUPS ? (DK + DV < 256 ? 48 : 32) : n <= 256 && KT == 32 ? 32 : 64;
-  if (longest > 0 && (longest <= short_keys || (DK + DV < 256 && longest <= 128 && n > 1536)))
-    return launch_groups<DK, DV, 1, 32, false>(t, n_tiles, s);
-  if constexpr (DK + DV <= 320) {
-    if (n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT, false>(t, n_tiles, s);
+  const int keys = longest > 0 ? longest : 1 << 30;
+  if (keys <= 64 || (keys <= 224 && n > (DK + DV > 64 ? 256 : TWO_GROUPS))) return launch_groups<DK, DV, 1, 32, 1>(t, n_tiles, s);
+  if constexpr (DK + DV < 256) {
+    if (keys <= (DK + DV > 64 ? 128 : 256) && n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT, 1>(t, n_tiles, s);
   }
-  return launch_groups<DK, DV, 1, KT, true>(t, n_tiles, s);
+  if constexpr (DK + DV <= 320) {
+    if (n <= 256 || (n <= TWO_GROUPS && keys > 1024)) return launch_groups<DK, DV, 2, KT, 2>(t, n_tiles, s);
+  }
+  return launch_groups<DK, DV, 1, KT, 2>(t, n_tiles, s);
 }
 
 constexpr int CAPS[][2] = {{32, 32}, {64, 64}, {64, 128}, {96, 96}, {128, 128}, {192, 128}, {256, 256}};
