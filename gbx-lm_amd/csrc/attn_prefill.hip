@@ -15,6 +15,9 @@
 //                                            the accumulator column is the lane's query: rescaling by alpha is per lane
 // Online softmax in base 2 (scores scaled by scale * log2 e), fp32 statistics, P rounded to the activation dtype for P V
 // (as every fused attention does), one division at the end.
+// The query heads of a key / value head run on one XCD, whose cache then holds their keys, and every XCD gets query blocks of every length: with the
+// block as the fast index of the grid some XCDs had all the long ones (CUs busy 56 % of the time at 24 blocks).  Before | now, us: 24 heads of 128 on
+// 8, 3001 rows 107 | 83, 32 heads, 1500 rows 45 | 34, 4096 235 | 157, 8192 751 | 570, 8 x 4096 1771 | 1220 (901 TFLOP/s of causal operations).
 // Measured variants (cfg4 shape, TFLOP/s of causal flops): V transposed by 2-byte LDS stores, 1 workgroup / CU 174; transposed
 // reads + 2 workgroups / CU 547; one barrier per tile + bulk fragment reads (this file) 590-611; forced to 1 workgroup / CU 375;
 // S^T of tile t+1 issued before the softmax of tile t 519, softmax per 32-key sub-tile with the other sub-tile's MFMAs issued
@@ -52,8 +55,11 @@ __device__ __forceinline__ u32x2 lds_read_tr(const unsigned char* p) {
       (s16x4 __attribute__((address_space(3)))*)(__attribute__((address_space(3))) unsigned char*)p));
 }
 
-template <bool BF16, int HD>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnArgs a) {
+// GROUPS of four waves share the 128 queries of a workgroup: two take every other key tile each, with a maximum and a sum of their own that meet in LDS
+// at the end.  Workgroups of the last queries, which sweep the most keys, go first; heads are the fast index, the query heads of a key / value
+// head Hkv apart, so that they and every query block of theirs run on the XCD (every eighth workgroup) whose cache holds their keys.
+template <bool BF16, int HD, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, 2) void attn_prefill_kernel(const PrefillAttnArgs a) {
   constexpr int KT = 64;                       // keys per tile
   constexpr int KROW = HD * 2 + 16;            // K tile row bytes (+16: conflict-free 16-byte fragment reads)
   constexpr int VROW = HD * 2 + 64;            // V tile row bytes: pitch = 16 dwords mod 64, the 4 rows of a transposed block
@@ -62,14 +68,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
   constexpr int DT = HD / 32;                  // 32-row tiles of O^T
   constexpr int PPT = KT * HD / 8 / 256;       // 16-byte pieces of a K (or V) tile per thread
   constexpr int KBUF = KT * KROW, VBUF = KT * VROW;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * KBUF + 2 * VBUF];   // K ping | K pong | V ping | V pong
-  unsigned char* kl = lds;
-  unsigned char* vl = lds + 2 * KBUF;
+  constexpr int GBUF = 2 * KBUF + 2 * VBUF;    // of a group: K ping | K pong | V ping | V pong
+  __shared__ __attribute__((aligned(16))) unsigned char lds[GROUPS * GBUF];
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  unsigned char* kl = lds + group * GBUF;
+  unsigned char* vl = kl + 2 * KBUF;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
-  const int head = blockIdx.y, b = blockIdx.z, kvh = head / (a.Hq / a.Hkv);
-  const int qb = (gridDim.x - 1 - blockIdx.x) * 128;                     // longest key sweeps are dispatched first
+  const int row = blockIdx.x % (a.B * a.Hq), b = row / a.Hq, place = row % a.Hq;
+  const int kvh = place % a.Hkv, head = kvh * (a.Hq / a.Hkv) + place / a.Hkv;
+  const int qb = (gridDim.x / (a.B * a.Hq) - 1 - blockIdx.x / (a.B * a.Hq)) * 128;
   const int qi = qb + wave * 32 + r;                                     // this lane's query (both halves of the wave)
   const int L = a.L, S = a.S;
   const unsigned short* kg = a.k + b * a.ks_b + kvh * a.ks_h;
@@ -88,6 +97,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
   // running maximum in RAW score units (the scale is folded into the exponent's fma), partial sum of this lane's 32 keys/tile
   float m_run = -INFINITY, l_run = 0.f;
   const float c = a.scale_log2;
+  auto seen = [](float m) { return GROUPS > 1 && m == -INFINITY ? 0.f : m; };   // (one group: key 0 is visible to every query)
 
   // keys this workgroup needs: 0 .. offset + (last query of the block), at most S
   const int kmax = min(S, a.offset + min(qb + 128, L));
@@ -130,23 +140,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
   // tile t+2 is requested.  LDS fragment reads are issued in bulk ahead of the MFMAs that consume them (the compiler's own
   // order was read-two / wait / multiply, every LDS latency exposed): the K fragments of the second sub-tile refill the
   // registers of the first as its MFMAs retire, the first half of the V^T fragments is requested BEFORE the softmax.
+  // (tiles past the sweep are requested and parked like any other -- zeros past S -- and not multiplied; groups run as many rounds)
   if (ntiles > 0) {
-    load_k(0); load_v(0);
+    load_k(group); load_v(group);
     store_k(0); store_v(0);
-    load_k(1); load_v(1);
+    load_k(group + GROUPS); load_v(group + GROUPS);
   }
-  for (int t = 0; t < ntiles; ++t) {
+  for (int round = 0, t = group; round < (ntiles + GROUPS - 1) / GROUPS; ++round, t += GROUPS) {
     __syncthreads();
-    store_k((t + 1) & 1);
-    store_v((t + 1) & 1);
-    load_k(t + 2);
-    load_v(t + 2);
+    store_k((round + 1) & 1);
+    store_v((round + 1) & 1);
+    load_k(t + 2 * GROUPS);
+    load_v(t + 2 * GROUPS);
+    if (t * KT > min(kmax - 1, a.offset + qb + wave * 32 + 31)) continue;  // wave-uniform: no query of the wave sees a key of the tile
 
     // ---- S^T = K Q^T for the two 32-key sub-tiles
     f32x16 st[2];
     st[0] = f32x16{0};
     st[1] = f32x16{0};
-    const unsigned char* kb = kbase + (t & 1) * KBUF;
+    const unsigned char* kb = kbase + (round & 1) * KBUF;
     u32x4 fr[KS];                                                         // 8 fragments in flight (K, then V^T)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) fr[ks] = *reinterpret_cast<const u32x4*>(kb + ks * 32);
@@ -161,7 +173,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
     for (int ks = 0; ks < KS; ++ks) st[1] = mfma<BF16>(fr[ks], qf[ks], st[1]);
     __builtin_amdgcn_sched_barrier(0);
     // V^T fragments of d-tiles 0 .. DT/2-1 (keys 32u + 16tt + 4h + {0..3} and the same + 8): in flight under the softmax
-    const unsigned char* vb = vbase + (t & 1) * VBUF;
+    const unsigned char* vb = vbase + (round & 1) * VBUF;
     auto vfrag = [&](int dt, int j) {                                     // j = 2u + tt
       const u32x2 v0 = lds_read_tr(vb + ((j >> 1) * 32 + (j & 1) * 16) * VROW + dt * 64);
       const u32x2 v1 = lds_read_tr(vb + ((j >> 1) * 32 + (j & 1) * 16 + 8) * VROW + dt * 64);
@@ -190,7 +202,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
     //      softmax either way, the factor cancels in the final division)
     if (__builtin_amdgcn_ballot_w64((mx - m_run) * c > 8.f) != 0) {
       const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);    // (m_new is finite: key 0 is visible to every query)
+      const float alpha = __builtin_amdgcn_exp2f((m_run - seen(m_new)) * c);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -198,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
     }
-    const float mc = -m_run * c;
+    const float mc = -seen(m_run) * c;
     float ls = 0.f;
     u32x4 pf[4];                                                          // P^T operands: index 2u + tt
 #pragma unroll
@@ -221,6 +233,28 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const PrefillAttnA
     }
   }
 
+  if constexpr (GROUPS > 1) {
+    static_assert(4 * (DT * 16 + 2) * 64 * 4 <= GROUPS * GBUF, "the second group's sums fit the tiles' place");
+    float* join = reinterpret_cast<float*>(lds) + wave * ((DT * 16 + 2) * 64) + lane;
+    __syncthreads();
+    if (group == 1) {
+      join[0] = m_run;
+      join[64] = l_run;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) join[(2 + dt * 16 + e) * 64] = o[dt][e];
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = join[0], mj = fmaxf(m_run, m1);                      // finite: key 0 is group 0's (a second group without a key: -inf, weight 0)
+    const float f0 = __builtin_amdgcn_exp2f((m_run - mj) * c), f1 = __builtin_amdgcn_exp2f((m1 - mj) * c);
+    l_run = l_run * f0 + join[64] * f1;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * f0 + join[(2 + dt * 16 + e) * 64] * f1;
+  }
   // ---- normalise and store: lane (q, h) holds d = 32 dt + (e & 3) + 8 (e >> 2) + 4 h of its query
   const float lt = l_run + __shfl_xor(l_run, 32);
   const float inv = 1.f / lt;
@@ -245,16 +279,22 @@ hipError_t launch_attn_prefill(const void* q, const void* k, const void* v, void
   PrefillAttnArgs a{static_cast<const unsigned short*>(q), static_cast<const unsigned short*>(k), static_cast<const unsigned short*>(v),
                     static_cast<unsigned short*>(out), qs_b, qs_h, qs_l, ks_b, ks_h, vs_b, vs_h, B, Hq, Hkv, L, S, offset,
                     sm_scale * 1.4426950408889634f};
-  dim3 grid((L + 127) / 128, Hq, B), block(256);
-  if (D == 128) {
-    if (bf16) hipLaunchKernelGGL((attn_prefill_kernel<true, 128>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<false, 128>), grid, block, 0, s, a);
-  } else if (D == 64) {
-    if (bf16) hipLaunchKernelGGL((attn_prefill_kernel<true, 64>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<false, 64>), grid, block, 0, s, a);
-  } else {
-    return hipErrorInvalidValue;
-  }
+  const long long n = static_cast<long long>((L + 127) / 128) * Hq * B;
+  if (n > 0x7fffffff) return hipErrorInvalidValue;
+  // Two groups halve the longest chain of key tiles and take a CU; worth it while there are few tiles and the chain is long.  One group | two, us, 32
+  // heads: 512 keys 15.3 both, 1024 26.1 | 23.7, 1500 39.0 | 34.1, 2048 52.9 | 50.7, 4096 157 | 162; 24 heads, 3001 keys (576 tiles) 82.9 | 86.7; one row
+  // behind 1500 32.7 | 24.8, 17 rows behind 300 9.95 | 10.05, 2 x 700 rows (384 tiles) 22.9 | 25.8, 8 x 512 38 | 55
+  const bool two = S > 512 && (n <= 256 || (n <= 512 && S > 1024));
+  const dim3 grid(static_cast<unsigned>(n)), block(two ? 512 : 256);
+#define GBX_ATTN(D_) \
+  if (bf16 && two) hipLaunchKernelGGL((attn_prefill_kernel<true, D_, 2>), grid, block, 0, s, a); \
+  else if (bf16) hipLaunchKernelGGL((attn_prefill_kernel<true, D_, 1>), grid, block, 0, s, a); \
+  else if (two) hipLaunchKernelGGL((attn_prefill_kernel<false, D_, 2>), grid, block, 0, s, a); \
+  else hipLaunchKernelGGL((attn_prefill_kernel<false, D_, 1>), grid, block, 0, s, a)
+  if (D == 128) { GBX_ATTN(128); }
+  else if (D == 64) { GBX_ATTN(64); }
+  else return hipErrorInvalidValue;
+#undef GBX_ATTN
   return hipGetLastError();
 }
 

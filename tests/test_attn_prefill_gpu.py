@@ -53,6 +53,14 @@ def test_shapes(d, dtype):
     _case(1, 8, 2, 260, 40, d, dtype, cache_cap=1024)      # cache with spare capacity: batch / head strides differ from S * D
 
 
+@pytest.mark.parametrize("l,off", [(513, 0), (576, 0), (577, 70), (1, 640), (40, 600), (129, 1023), (1300, 0)])
+def test_two_groups_of_waves(l, off):
+    """Long sweeps of few tiles: every other key tile in a second group of waves -- odd and even numbers of tiles, a last one whose keys some or all
+    queries of a group do not see -- with sequences and heads whose order in the grid is not theirs in memory."""
+    _case(3, 6, 3, l, off, 128, torch.bfloat16)
+    _case(1, 32, 8, l, off, 64, torch.float16)
+
+
 def test_sharp_rows():
     """large logits: one key dominates, the running maximum moves between key tiles"""
     _case(1, 8, 2, 700, 0, 128, torch.bfloat16, amp=6.0)
