@@ -38,6 +38,17 @@ __device__ __forceinline__ u32x2 lds_read_tr(const unsigned char* p) {
 // LDS as the destination of a buffer load
 #define GBXM_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
 
+// How the 256 threads of a group of waves carry the rows of a key or value tile, D channels each, in pieces of 16 bytes: `LANES` neighbouring threads a row, `PER`
+// pieces of it each, `ROWS` rows at a time; or, where a row's pieces do not fall into eights, piece after piece.
+template <int D, int KT> struct RowPieces {
+  static constexpr int C = D / 8, LANES = C % 16 == 0 ? 16 : C % 8 == 0 ? 8 : 4, PER = C / LANES, ROWS = 256 / LANES;
+  static constexpr bool LINEAR = C > 4 && LANES == 4;
+  static constexpr int N = LINEAR ? (KT * C + 255) / 256 : PER * ((KT + ROWS - 1) / ROWS);
+  __device__ static int row(int tid, int i) { return LINEAR ? (tid + 256 * i) / C : tid / LANES + i / PER * ROWS; }
+  __device__ static int piece(int tid, int i) { return LINEAR ? (tid + 256 * i) % C : tid % LANES + i % PER * LANES; }
+  __device__ static bool used(int tid, int i) { return (LINEAR ? KT * C % 256 == 0 : KT % ROWS == 0) || row(tid, i) < KT; }
+};
+
 // Workgroup ids go round-robin over the 8 XCDs, each with an L2 of its own: every XCD gets a contiguous run of units (row tile, column
 // block), so the column blocks of ONE row tile, which read the same activation rows, and the row tiles of one expert, which read the
 // same weights, run on one XCD next to each other.  The runs are cut from the units that exist (the sort counted the tiles), not from

@@ -75,17 +75,6 @@ template <int DK, int DV, int GROUPS_, int KT_, int BUFS_> struct SinkShape {
   static constexpr int SLOTS = BUFS == 1 ? 0 : DK <= 192 ? DK / 16 : 8;
 };
 
-// How the 256 threads of a group carry the rows of a tile, D channels each, in pieces of 16 bytes: `LANES` neighbouring threads a row, `PER`
-// pieces of it each, `ROWS` rows at a time; or, where a row's pieces do not fall into eights, piece after piece.
-template <int D, int KT> struct RowPieces {
-  static constexpr int C = D / 8, LANES = C % 16 == 0 ? 16 : C % 8 == 0 ? 8 : 4, PER = C / LANES, ROWS = 256 / LANES;
-  static constexpr bool LINEAR = C > 4 && LANES == 4;
-  static constexpr int N = LINEAR ? (KT * C + 255) / 256 : PER * ((KT + ROWS - 1) / ROWS);
-  __device__ static int row(int tid, int i) { return LINEAR ? (tid + 256 * i) / C : tid / LANES + i / PER * ROWS; }
-  __device__ static int piece(int tid, int i) { return LINEAR ? (tid + 256 * i) % C : tid % LANES + i % PER * LANES; }
-  __device__ static bool used(int tid, int i) { return (LINEAR ? KT * C % 256 == 0 : KT % ROWS == 0) || row(tid, i) < KT; }
-};
-
 template <int DK, int DV, int GROUPS, int KT, int BUFS>
 __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile, const int head, unsigned char* all_lds) {
   typedef SinkShape<DK, DV, GROUPS, KT, BUFS> Shape;
@@ -570,12 +559,13 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
   return launch_sink_reduce(a, splits, s);
 }
 
-// A workgroup = a query tile of a head; tiles that see many keys, at the end of the step's list, go first.  Heads are the fast index, so that an
-// XCD's workgroups (every eighth) meet in few heads' keys.
+// A workgroup = a query tile of a head; tiles that see many keys, at the end of the step's list, go first.  Heads are the fast index, those of a
+// key / value head G apart, so that an XCD's workgroups (every eighth) meet in few heads' keys.
 template <int DK, int DV, int GROUPS, int KT, int BUFS>
 __global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT, BUFS>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  sink_tile<DK, DV, GROUPS, KT, BUFS>(a, n_tiles - 1 - blockIdx.x / a.H, blockIdx.x % a.H, lds);
+  const int place = blockIdx.x % a.H, head = place % a.G * (a.H / a.G) + place / a.G;
+  sink_tile<DK, DV, GROUPS, KT, BUFS>(a, n_tiles - 1 - blockIdx.x / a.H, head, lds);
 }
 
 template <int DK, int DV, int GROUPS, int KT, int BUFS>

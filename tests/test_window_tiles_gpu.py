@@ -27,6 +27,19 @@ def test_more_tiles_than_compute_units(dk, dv, cap, window):
              dk, dv, cap, window)
 
 
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (192, 128), (96, 96)])
+@pytest.mark.parametrize("cap,window", [(0.0, 300), (5.0, 9)])
+def test_short_sequences_only(dk, dv, cap, window):
+    """Up to 48 keys a tile: one buffer of 32 keys."""
+    portions([1, 31, 32, 33, 40, 7, 17], [0, 0, 0, 0, 8, 41, 31] if window == 300 else [0, 3, 0, 0, 100, 9, 31], dk, dv, cap, window)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 64), (192, 128)])
+def test_long_sequences(dk, dv):
+    """One group of waves, two buffers, whole tiles in the ring and in the step's rows, the ring's seam inside a tile and at its edge."""
+    portions([400, 129, 640, 300, 257, 128, 200, 512], [0, 511, 900, 448, 1024, 512, 64, 700], dk, dv, 5.0, 512)
+
+
 def portions(n_new, pos0, dk, dv, cap, window):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
