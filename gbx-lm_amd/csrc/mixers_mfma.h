@@ -60,9 +60,10 @@ __device__ __forceinline__ int xcd_unit(int units) {
 
 // Pairs (row, choice) bucketed by expert on the device (mixers_moe_mfma.hip): offsets [E + 2] by bucket -- bucket E holds the pairs whose
 // index names no expert -- then the number of row tiles; the pair ids in bucket order; per row tile (of at most `rows` pairs) its bucket
-// and first place in that order (surplus tiles: bucket -1).  `tiles` bounds the tiles on the host.  `ws`: expert_buckets_bytes.
+// and its first and last + 1 place in that order (surplus tiles: bucket -1).  `tiles` bounds the tiles on the host.  `ws`: expert_buckets_bytes.
 struct ExpertBuckets {
-  int *offsets, *sorted, *tile_tab;
+  int *offsets, *sorted;
+  int4* tile_tab;
   int tiles;
 };
 size_t expert_buckets_bytes(int64_t P, int rows, int E);

@@ -9,21 +9,22 @@
 // Products are computed swapped -- C^T[channel, pair] = mfma(weight rows, activation rows) -- so a lane ends up with four consecutive
 // channels of one pair (8-byte stores) and the gate / up pair of a channel sits in the same lane for the activation.
 // What bounds it: a few hundred pairs per expert, so the weights are a stream of their own (1.2 GB at 128 experts of 3 x 2048 x 768: 0.24 ms)
-// beside about as much matrix-core work; both operands therefore go memory -> LDS by DMA, two stages of 64 elements, and a weight row
-// is fetched once per 256 pairs.  Eight waves, a wave 128 pairs x 64 weight rows (16 x 16 x 32 products); four phases a stage, two wave groups
+// beside about as much matrix-core work; both operands therefore go memory -> LDS by DMA, stages of 64 elements, two of activations and three of
+// weights (which come from memory, two stages ahead; with two of either, one ahead: 64 experts of 2 x 2048 x 2048, 16 384 pairs 420 us for 389,
+// 128 of 3 x 2048 x 768, 2 048 pairs 252 for 236, 27 848 415 for 410), and a weight row is fetched once per 256 pairs.  Eight waves, a wave 128 pairs x 64 weight rows (16 x 16 x 32 products); four phases a stage, two wave groups
 // a barrier apart, so that one group multiplies while the other reads fragments and issues requests.  Stages of 64 elements, because a row
 // piece is then a whole 128-byte line: 256 x 128 tiles with stages of 32 elements and two workgroups per CU spent their time on twice the L2
 // requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
 // Measured (us, first + second products with the sort; 256-pair tiles with results from the registers -> results by rows, in turn on one card, uniform choices, the least of
 // four places of the weights in memory, which move these times by up to a tenth):
-//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (620 TFLOP/s, 2.9 TB/s of weights)
-//   18 128 pairs of the same:                       340 -> 326 (3.7 TB/s)
-//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 437 -> 422; a factor of the weights' way from memory (one expert's for all: 150 less) and of the results' (kept back:
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (now 410: 640 TFLOP/s, 2.9 TB/s of weights)
+//   18 128 pairs of the same:                       340 -> 326 (now 315: 3.8 TB/s)
+//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 437 -> 422 (now 389); a factor of the weights' way from memory (one expert's for all: 150 less) and of the results' (kept back:
 //   75 less), which tiles of one round write at the same time
 //    8 192 pairs,   8 experts, 4096 x 2048 gated:   461 -> 457 (900 TFLOP/s)
 // The table keeps a lower tile beside its expert's others.  By falling height, so that the last round is short, tiles read their weights anew: 256 pairs an
-// expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  Requests of a whole stage ahead, or its lines ordered into L2
-// before, gain nothing.
+// expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  A stage's lines ordered into L2 before gain nothing; nor does
+// it matter how many rows a request spans (256 x 128 B, 64 x 512 B or 32 KB in one piece: 4.4 to 4.7 TB/s).
 // The grid is sized for the worst case sum_e ceil(n_e / 256) <= P / 256 + E; surplus workgroups leave at once.
 // Steps with few pairs per expert (a batch that decodes) stream weights and little else: expert_skinny_kernel takes tiles of 32 pairs, a
 // wave per 32 output channels and no barrier.  A wave moves its own rows -- eight lanes to a row's 128 bytes, so an access touches eight
@@ -47,7 +48,7 @@ constexpr int SORT_LDS = (3 * 4097 + 5) * 4 + KEEP * 1024 * 2;           // (E <
 
 template <int N>
 __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ idx, int* __restrict__ offsets, int* __restrict__ sorted,
-                                                          int* __restrict__ tile_tab, int n_tiles, int rt, int P, int E1) {
+                                                          int4* __restrict__ tile_tab, int n_tiles, int rt, int P, int E1) {
   extern __shared__ int sm[];                 // counts [E1] | starts [E1 + 1] | first tile [E1] | tiles | the order, 16 bits a pair
   int* counts = sm;
   int* start = sm + E1;
@@ -111,9 +112,9 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
         }
   for (int e = tid; e < E1; e += 1024) {
     const int nt = (counts[e] + rt - 1) / rt;
-    for (int t = 0; t < nt; ++t) { tile_tab[2 * (first[e] + t)] = e; tile_tab[2 * (first[e] + t) + 1] = start[e] + t * rt; }
+    for (int t = 0; t < nt; ++t) tile_tab[first[e] + t] = int4{e, start[e] + t * rt, start[e] + min(counts[e], (t + 1) * rt), 0};
   }
-  for (int t = first[E1] + tid; t < n_tiles; t += 1024) tile_tab[2 * t] = -1;
+  for (int t = first[E1] + tid; t < n_tiles; t += 1024) tile_tab[t] = int4{-1, 0, 0, 0};
   if constexpr (N == FEW) return;
   __syncthreads();
   if (small) {                                 // (whole groups of four: expert_buckets_bytes rounds up to them)
@@ -139,7 +140,7 @@ struct GroupArgs {
   const bf16_t* w;             // [E][N][C], gated: [E][2 N][C]
   const int* offsets;          // expert_buckets' table
   const int* sorted;
-  const int* tile_tab;
+  const int4* tile_tab;
   const float* scale;
   bf16_t* out;
   int N, C, E, top, cols;
@@ -148,8 +149,9 @@ struct GroupArgs {
 
 constexpr int GR = 256;                      // pairs per row tile at most
 constexpr int GHALF = 128 * 128;             // LDS bytes of a half-tile: 64 elements of 128 rows
-constexpr int GSTAGE = 4 * GHALF;            // activation rows of wave rows 0 | 1, weight rows of wave columns 0, 1 | 2, 3
-constexpr int GLDS = 2 * GSTAGE + GR * 8;    // two stages, then the tile's pair ids and factors
+constexpr int GSTAGE = 2 * GHALF;            // a stage's activation rows of wave rows 0 | 1, or its weight rows of wave columns 0, 1 | 2, 3
+constexpr int GLDS = 5 * GSTAGE;             // two stages of activations, three of weights: all of a CU's LDS
+constexpr int GIDS = 256 * 32 * 16;          // behind the results, at the end: the tile's pair ids and factors
 constexpr int PAST = -16;                    // byte offset (as unsigned) beyond every buffer: such lanes of a buffer load deliver zeros
 
 // One tile of 32 NR pairs x 256 weight rows.  See the head of the file.
@@ -161,14 +163,16 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
   const int fr = lane & 15, fk = lane >> 4;
   const int N = a.N, C = a.C, n = (C + 63) >> 6;
   const int r0 = GATED ? col * 128 : col * 256;                         // the tile's first output channel
-  int* ids = reinterpret_cast<int*>(lds + 2 * GSTAGE);
-  float* factor = reinterpret_cast<float*>(ids + GR);
-  if (tid < 32 * NR) {
-    const int id = a.sorted[min(lo + tid, hi - 1)];
-    ids[tid] = id;
-    factor[tid] = FORM != EXPERT_DOWN && a.scale ? a.scale[id] : 1.f;
-  }
-  __syncthreads();
+  // Start-up is one trip to memory after another (units, tile, rows, operands): the weights, which come from farthest away, are asked for first
+  int ida[2][PA];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const int row = h * 16 * NR + min((tid >> 3) + 64 * i, 16 * NR - 1);
+      ida[h][i] = FORM == EXPERT_DOWN ? min(row, hi - lo - 1) : a.sorted[min(lo + row, hi - 1)];
+    }
+  const int my_id = a.sorted[min(lo + tid, hi - 1)];                    // (of the first 32 NR threads; kept for the end)
   // DMA side: piece p = tid + 512 i of a half-tile is row p / 8, slot p % 8 of its LDS image and holds 16-byte column slot ^ ((row / 2) & 7):
   // every group of 16 lanes that an LDS fragment read serves at a time then meets 16 different bank quads
   const int lcol = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
@@ -183,30 +187,28 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int i = 0; i < PA; ++i) {
-      const int row = h * 16 * NR + min((tid >> 3) + 64 * i, 16 * NR - 1);
-      voa[h][i] = (FORM == EXPERT_DOWN ? min(row, hi - lo - 1) : ids[row] / a.top) * C * 2 + lcol;
-    }
-#pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int b = h * 128 + (tid >> 3) + 64 * i;
       vob[h][i] = min(GATED ? (b >> 6) * 32 + (b & 31) : b, N - 1 - r0) * C * 2 + lcol;
     }
   }
-  auto stage = [&](int t, int h) {                                      // half-tile h (0, 1 activations, 2, 3 weights) of stage t
-    const int tc = min(t, n - 1);                                       // past the end the last one again: every wait counts the same requests
+  // half-tile h of stage t; past the end the last stage again: every wait counts the same requests
+  auto stage_a = [&](int t, int h) {
+    const int tc = min(t, n - 1);
     const bool cut = tc * 64 + 32 == C && lcol >= 64;                   // the second half of a stage that the contraction does not fill
     unsigned char* dst = lds + (t & 1) * GSTAGE + h * GHALF + wave * 1024;
-    if (h < 2) {
 #pragma unroll
-      for (int i = 0; i < PA; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : voa[h][i], tc * 128, 0, 0);
-    } else {
+    for (int i = 0; i < PA; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : voa[h][i], tc * 128, 0, 0);
+  };
+  auto stage_b = [&](int t, int slot, int h) {
+    const int tc = min(t, n - 1);
+    const bool cut = tc * 64 + 32 == C && lcol >= 64;
+    unsigned char* dst = lds + (2 + slot) * GSTAGE + h * GHALF + wave * 1024;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : vob[h - 2][i], tc * 128, 0, 0);
-    }
+    for (int i = 0; i < 2; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : vob[h][i], tc * 128, 0, 0);
   };
   const int sw = (fr >> 1) & 7, k0 = (fk ^ sw) * 16, k1 = ((4 + fk) ^ sw) * 16;
-  const int fa_off = wr * GHALF + fr * 128, fb_off = (2 + (wc >> 1)) * GHALF + ((wc & 1) * 64 + fr) * 128;
+  const int fa_off = wr * GHALF + fr * 128, fb_off = 2 * GSTAGE + (wc >> 1) * GHALF + ((wc & 1) * 64 + fr) * 128;
   u32x4 fa[NR][2], fb[4][2];
   auto read_a = [&](const unsigned char* buf, int half) {
 #pragma unroll
@@ -239,36 +241,48 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
     __builtin_amdgcn_s_setprio(0);
   };
   auto bar = [] { asm volatile("s_barrier" ::: "memory"); };
+  stage_b(0, 0, 0);
+  stage_b(0, 0, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  const float my_factor = FORM != EXPERT_DOWN && a.scale ? a.scale[my_id] : 1.f;
 #pragma unroll
-  for (int h = 0; h < 4; ++h) stage(0, h);
-  stage(1, 0);
-  stage(1, 1);
-  __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(2 * PA));                    // stage 0 has landed (this wave's share), two half-tiles of stage 1 may fly
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < PA; ++i) voa[h][i] = (FORM == EXPERT_DOWN ? ida[h][i] : ida[h][i] / a.top) * C * 2 + lcol;
+  stage_a(0, 0);
+  stage_a(0, 1);
+  stage_b(1, 1, 0);
+  stage_b(1, 1, 1);
+  stage_a(1, 0);
+  stage_a(1, 1);
+  __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(4 + 2 * PA));                // stage 0 has landed (this wave's share), stage 1 may fly
   bar();
   if (wr == 1) bar();                                                   // the second wave group runs one barrier interval behind the first
-  for (int t = 0; t < n; ++t) {
-    const unsigned char* buf = lds + (t & 1) * GSTAGE;
-    read_b(buf, 0);
+  // The weights of stage t + 2 are asked for before stage t is multiplied, into the place of stage t - 1, the activations of t + 2 -- which other
+  // workgroups of the XCD read too -- once stage t is in registers
+  for (int t = 0, now = 0, next = 2; t < n; ++t, next = now, now = now == 2 ? 0 : now + 1) {
+    const unsigned char *abuf = lds + (t & 1) * GSTAGE, *bbuf = lds + now * GSTAGE;
+    read_b(bbuf, 0);
     __builtin_amdgcn_sched_barrier(0);
-    read_a(buf, 0);
-    stage(t + 1, 2);
+    read_a(abuf, 0);
+    stage_b(t + 2, next, 0);
     bar();
     quadrant(0, 0);
     bar();
-    read_b(buf, 1);
+    read_b(bbuf, 1);
     __builtin_amdgcn_sched_barrier(0);
-    read_a(buf, 1);
-    stage(t + 1, 3);
+    read_a(abuf, 1);
+    stage_b(t + 2, next, 1);
     __builtin_amdgcn_s_waitcnt(0xC07F);                                 // lgkmcnt(0): the stage is in registers before the barrier that frees its slots
     bar();
     quadrant(0, 1);
     bar();
-    stage(t + 2, 0);
+    stage_a(t + 2, 0);
     bar();
     quadrant(1, 1);
     bar();
-    stage(t + 2, 1);
-    __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(2 * PA));                  // all of stage t + 1 has landed
+    stage_a(t + 2, 1);
+    __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(4 + 2 * PA));              // all of stage t + 1 has landed
     bar();
     quadrant(1, 0);
     bar();
@@ -276,6 +290,14 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
   if (wr == 0) bar();                                                   // the groups' barrier counts match again
   __builtin_amdgcn_s_waitcnt(lds_and_vmcnt(0));                         // no LDS-DMA outlives the workgroup
   bar();                                                                // every wave is past its last fragment: the stages' LDS is free
+  int* ids = reinterpret_cast<int*>(lds + GIDS);
+  float* factor = reinterpret_cast<float*>(ids + GR);
+  if (tid < 32 * NR) {
+    ids[tid] = my_id;
+    factor[tid] = my_factor;
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  bar();
   // The tile's results meet in LDS (16-byte column c of row r at place c ^ (r & 15): neither side meets a bank twice) and leave as whole rows of it
   constexpr int OPC = GATED ? 16 : 32;                                  // 16-byte columns of a row
 #pragma unroll
@@ -313,7 +335,8 @@ __global__ __launch_bounds__(512) void expert_group_kernel(const GroupArgs a) {
   const int u = xcd_unit(a.offsets[a.E + 2] * a.cols);
   if (u < 0) return;                                                    // (workgroup-uniform, as everything that picks the tile)
   const int bt = u / a.cols, col = u % a.cols;
-  const int e = a.tile_tab[2 * bt], lo = a.tile_tab[2 * bt + 1], hi = min(a.offsets[e + 1], lo + GR);
+  const int4 tab = a.tile_tab[bt];
+  const int e = tab.x, lo = tab.y, hi = tab.z;
   if (e >= a.E) return;                                                 // (pairs without an expert)
   switch ((hi - lo + 63) / 64) {
     case 1: group_tile<FORM, 2>(a, lds, e, lo, hi, col); break;
@@ -343,14 +366,14 @@ __device__ __forceinline__ SkinnyUnit skinny_unit(int tiles, int cols) {
 
 template <int FORM>
 __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __restrict__ in, const bf16_t* __restrict__ w, const int* __restrict__ offsets,
-                                                           const int* __restrict__ sorted, const int* __restrict__ tile_tab, const float* __restrict__ scale,
+                                                           const int* __restrict__ sorted, const int4* __restrict__ tile_tab, const float* __restrict__ scale,
                                                            bf16_t* __restrict__ out, int N, int C, int E, int top, int kind, float limit) {
   constexpr bool TWO = FORM == SKINNY_GATED;
   const SkinnyUnit u = skinny_unit(offsets[E + 2], (N + 127) / 128);
   if (u.tile < 0) return;
-  const int bt = u.tile, e = tile_tab[2 * bt];
+  const int4 tab = tile_tab[u.tile];
+  const int e = tab.x, lo = tab.y, hi = tab.z;
   if (e >= E) return;
-  const int lo = tile_tab[2 * bt + 1], hi = offsets[e + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, hb = lane >> 5;
   const int c0 = u.col * 128 + wave * 32;
   if (c0 >= N) return;
@@ -466,7 +489,7 @@ int rows_of(int64_t P, int E, int F, bool gated) {
 int64_t expert_tiles(int64_t P, int rows, int E) { return (P / rows + E + 1 + 7) / 8 * 8; }
 
 size_t expert_buckets_bytes(int64_t P, int rows, int E) {
-  return align16(sizeof(int) * (E + 3)) + align16(sizeof(int) * P) + align16(sizeof(int) * 2 * expert_tiles(P, rows, E));
+  return align16(sizeof(int) * (E + 3)) + align16(sizeof(int) * P) + align16(sizeof(int4) * expert_tiles(P, rows, E));
 }
 
 int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBuckets* out, hipStream_t s) {
@@ -476,7 +499,7 @@ int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBucke
   w += align16(sizeof(int) * (E + 3));
   out->sorted = reinterpret_cast<int*>(w);
   w += align16(sizeof(int) * P);
-  out->tile_tab = reinterpret_cast<int*>(w);
+  out->tile_tab = reinterpret_cast<int4*>(w);
   static OncePerDevice once;
   if (once.pending()) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_sort_kernel<KEEP>), hipFuncAttributeMaxDynamicSharedMemorySize, SORT_LDS);
@@ -524,7 +547,8 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
   const int rows = rows_of(P, E, F, gated);
   int rc = expert_buckets(a.idx, P, rows, E, a.ws, &k, s);
   if (rc != GBXM_OK) return rc;
-  const int *offsets = k.offsets, *sorted = k.sorted, *tile_tab = k.tile_tab, tiles = k.tiles;
+  const int *offsets = k.offsets, *sorted = k.sorted, tiles = k.tiles;
+  const int4* tile_tab = k.tile_tab;
   bf16_t* act = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(a.ws) + expert_buckets_bytes(P, RS, E));
   const bf16_t* h = static_cast<const bf16_t*>(a.h);
   const bf16_t* first = static_cast<const bf16_t*>(a.first);

@@ -35,7 +35,8 @@ struct PackedArgs {
   const unsigned short* s[2];
   const unsigned short* z[2];
   const unsigned short* bias;          // [E][N] or null
-  const int *offsets, *sorted, *tile_tab;
+  const int *offsets, *sorted;
+  const int4* tile_tab;
   unsigned short* y;                   // [pairs][N]
   int N, K, E, x_div, cols;
 };
@@ -246,7 +247,8 @@ __global__ __launch_bounds__(256, 2) void packed_experts_kernel(const PackedArgs
   const int u = xcd_unit(a.offsets[a.E + 2] * a.cols);
   if (u < 0) return;                                                    // (workgroup-uniform, as everything that picks the tile)
   const int bt = u / a.cols, col = u % a.cols;
-  const int e = a.tile_tab[2 * bt], lo = a.tile_tab[2 * bt + 1], hi = min(a.offsets[e + 1], lo + PT);
+  const int4 tab = a.tile_tab[bt];
+  const int e = tab.x, lo = tab.y, hi = tab.z;
   if (e >= a.E) {                                                       // indices that name no expert: rows that nobody can take for results
     const int cn = min((GATED ? 128 : 256), a.N - col * (GATED ? 128 : 256));
     for (int i = threadIdx.x; i < (hi - lo) * cn; i += 256) a.y[static_cast<int64_t>(a.sorted[lo + i / cn]) * a.N + col * (GATED ? 128 : 256) + i % cn] = 0x7FFF;
