@@ -5,6 +5,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <type_traits>
 #include "gbx_mixers.h"
 
 namespace gbxm {
@@ -97,8 +98,7 @@ inline int row_threads(int width) { return width % 4 == 0 && width <= 4096 ? (wi
 template <typename... P>
 inline bool all_aligned(size_t bytes, const P*... p) { return ((reinterpret_cast<uintptr_t>(p) | ...) & (bytes - 1)) == 0; }
 
-// Candidates in front of candidate e of value x among 4 n4 values: larger ones, and equal ones of a lower index.  Every candidate's rank is
-// taken at once, where rounds of arg-max wait for one another.
+// Candidates in front of candidate e of value x among 4 n4 values: larger ones, and equal ones of a lower index.
 __device__ __forceinline__ int rank_of(const float* v, int n4, int e, float x) {
   int rank = 0;
 #pragma unroll 8
@@ -110,14 +110,55 @@ __device__ __forceinline__ int rank_of(const float* v, int n4, int e, float x) {
   }
   return rank;
 }
-// Where a router's choice goes by rank: every expert reads all scores, E / 16 steps of a wave, where each of the `rounds` of arg-max (one per choice and per
-// kept group) is a chain of its own; `per_round` steps cost what one of them does.  Measured, rounds | rank, us: softmax, top 8, 1 row: 64 experts
-// 9.7 | 5.2, 128 9.6 | 8.1, 256 9.5 | 14.1, 512 10.3 | 49; 4000 rows: 64 29.6 | 11.5, 128 30.0 | 20.8, 256 30.6 | 47; top 2, 1 row: 64 4.1 | 5.2.
-// Sigmoid, top 8, 1 row: 64 6.8 | 5.1, 128 7.4 | 7.9, 256 8.6 | 14.1; in 8 groups of which 4 stay 64 10.4 | 5.9, 128 11.9 | 9.0, 256 14.9 | 15.6, 4000 rows
-// 64 15.4 | 8.1, 128 17.0 | 17.5, 160 18.1 | 29.4; top 2 in groups 64 6.5 | 5.9, 96 7.2 | 7.5.
-constexpr int RANK_EXPERTS = 256;
-inline bool choice_by_rank(int E, int rounds, int per_round) { return E <= RANK_EXPERTS && E <= per_round * rounds; }
-constexpr int RANK_PER_SOFTMAX_ROUND = 16, RANK_PER_SIGMOID_ROUND = 11;
+
+// The largest of a wave's values, the same in every lane: within rows of 16 lanes by DPP, then the four rows' by scalar reads (a number beside
+// values that are none).
+template <typename T, typename Max> __device__ __forceinline__ T wave_most(T x, Max most) {
+  const auto moved = [&](auto dpp) { return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(dpp)::value, 0xf, 0xf, false)); };
+  x = most(x, moved(std::integral_constant<int, 0xB1>{}));           // quad_perm [1,0,3,2]
+  x = most(x, moved(std::integral_constant<int, 0x4E>{}));           // quad_perm [2,3,0,1]
+  x = most(x, moved(std::integral_constant<int, 0x141>{}));          // row_half_mirror
+  x = most(x, moved(std::integral_constant<int, 0x140>{}));          // row_mirror
+  const auto row = [&](int lane) { return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane)); };
+  return most(most(row(0), row(16)), most(row(32), row(48)));
+}
+__device__ __forceinline__ float wave_max(float x) { return wave_most(x, [](float a, float b) { return fmaxf(a, b); }); }
+
+// Floats (numbers and infinities) as unsigned keys of the same order; 0 lies below all of them.
+__device__ __forceinline__ unsigned order_key(float x) {
+  const unsigned b = __float_as_uint(x + 0.f);                       // (-0 is 0)
+  return b ^ (b >> 31 ? 0xFFFFFFFFu : 0x80000000u);
+}
+__device__ __forceinline__ float key_value(unsigned k) { return __uint_as_float(k ^ (k >> 31 ? 0x80000000u : 0xFFFFFFFFu)); }
+
+// Rounds of arg-max over up to 64 PER candidates that one wave holds, candidate 64 i + lane in key[i] (0: none, or taken), of equal ones the
+// lowest first: take(round, candidate, its key), all uniform.  A round is some 40 instructions without a barrier or a trip to LDS.
+// A router's choice with it | every expert counting those in front of it, in LDS, us: softmax, 8 of 128, 1 row 3.5 | 8.9, 3 481 rows
+// 4.9 | 19.8, 8 of 256 6.2 | 27.9, 2 of 16, 1 row 2.7 | 3.8; sigmoid in 8 groups, 2 of 32, 1 row 3.1 | 4.9, 8 of 128, 3 481 rows 6.2 | 17.6; plain sigmoid, 8 of
+// 128, 1 row 3.1 | 8.0, 2 of 64, 8 192 rows 3.6 | 10.0.
+inline bool choice_by_wave(int E, int top) { return E <= 256 && top <= 64; }
+template <int PER, typename Take> __device__ __forceinline__ void wave_choose(unsigned (&key)[PER], int rounds, Take take) {
+  const int lane = threadIdx.x & 63;
+  for (int k = 0; k < rounds; ++k) {
+    unsigned m = key[0];
+#pragma unroll
+    for (int i = 1; i < PER; ++i) m = max(m, key[i]);
+    m = wave_most(m, [](unsigned a, unsigned b) { return max(a, b); });
+    int e = 0;
+#pragma unroll
+    for (int i = PER - 1; i >= 0; --i) {
+      const unsigned long long here = __builtin_amdgcn_ballot_w64(key[i] == m);
+      if (here) e = 64 * i + __builtin_ctzll(here);
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (64 * i + lane == e) key[i] = 0;
+    take(k, e, m);
+  }
+}
+// a wave per row: one a workgroup while rows are few
+inline unsigned choice_threads(int64_t rows) { return rows > 1024 ? 256 : 64; }
+inline unsigned choice_blocks(int64_t rows) { return static_cast<unsigned>(rows > 1024 ? (rows + 3) / 4 : rows); }
 
 // z = a row of a sublayer's output, or sum_k mix[k] (candidate row k), at channels c .. c + 3; eight candidates in flight at a time.
 template <typename T>

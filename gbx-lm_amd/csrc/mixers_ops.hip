@@ -397,62 +397,41 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   if (renorm && threadIdx.x < top) weight[t * top + threadIdx.x] /= chosen_sum;
 }
 
-// The same by rank (choice_by_rank): probabilities and their order as above, no round waits for another.
-__global__ __launch_bounds__(NT) void route_topk_rank_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int E,
-                                                            int top, int renorm) {
-  __shared__ __attribute__((aligned(16))) float pl[RANK_EXPERTS];
-  __shared__ float sel[NT];
-  __shared__ float red[NW], mxs[NW];
-  const int64_t t = blockIdx.x;
-  constexpr int PER = RANK_EXPERTS / NT;
-  float v[PER];
-  float mx = -INFINITY;
+// The same for up to 64 PER experts, a wave per row.
+template <int PER>
+__global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int64_t rows, int E,
+                                                              int top, int renorm) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (t >= rows) return;
+  float v[PER], mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = threadIdx.x + i * NT;
-    v[i] = e < E ? logits[t * E + e] : -INFINITY;
-    mx = fmaxf(mx, v[i]);
-  }
+  for (int i = 0; i < PER; ++i) v[i] = lane + 64 * i < E ? logits[t * E + lane + 64 * i] : -INFINITY;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  if ((threadIdx.x & 63) == 0) mxs[threadIdx.x >> 6] = mx;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NW; ++i) mx = fmaxf(mx, mxs[i]);
+  for (int i = 0; i < PER; ++i) mx = fmaxf(mx, v[i]);
+  mx = wave_max(mx);
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
-    v[i] = live ? expf(v[i] - mx) : 0.f;
-    sum += v[i];
+    v[i] = lane + 64 * i < E ? expf(v[i] - mx) : 0.f;
+    sum += wave_sum(v[i]);
   }
-  sum = block_sum<NW>(sum, red);
+  unsigned key[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
-    v[i] = live ? v[i] / sum : -1.f;
-    if (!(v[i] == v[i])) v[i] = -1.f;            // (not a number: behind every probability)
-    pl[threadIdx.x + i * NT] = v[i];
+    const float p = v[i] / sum;
+    key[i] = lane + 64 * i < E ? order_key(p == p ? p : -1.f) : 0u;      // (not a number: behind every probability, but still an expert)
   }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = threadIdx.x + i * NT;
-    if (e < E) {
-      const int rank = rank_of(pl, (E + 3) / 4, e, v[i]);
-      if (rank < top) {
-        idx[t * top + rank] = e;
-        if (renorm) sel[rank] = v[i]; else weight[t * top + rank] = v[i];
-      }
-    }
-  }
-  if (!renorm) return;
-  __syncthreads();
-  if (static_cast<int>(threadIdx.x) < top) {
-    float chosen = 0.f;
-    for (int k = 0; k < top; ++k) chosen += sel[k];
-    weight[t * top + threadIdx.x] = sel[threadIdx.x] / chosen;
-  }
+  float chosen = 0.f, p = 0.f;                                           // lane k holds choice k
+  int mine = 0;
+  wave_choose(key, top, [&](int k, int e, unsigned m) {
+    const float v = key_value(m);
+    chosen += v;
+    if (lane == k) { mine = e; p = v; }
+  });
+  if (lane >= top) return;
+  idx[t * top + lane] = mine;
+  weight[t * top + lane] = renorm ? p / chosen : p;
 }
 
 template <typename T>
@@ -556,8 +535,12 @@ int gbxm_route_topk(const float* logits, int32_t* idx, float* weight, int64_t T_
   if (top > NT) return fail(GBXM_ERR_UNSUPPORTED, "route_topk: top > %d", NT);
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (choice_by_rank(E, top, RANK_PER_SOFTMAX_ROUND)) route_topk_rank_kernel<<<dim3(T_), NT, 0, s>>>(logits, idx, weight, E, top, renorm);
-  else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
+  if (choice_by_wave(E, top)) {
+    const unsigned blocks = choice_blocks(T_), threads = choice_threads(T_);
+    if (E <= 64) route_topk_wave_kernel<1><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
+    else if (E <= 128) route_topk_wave_kernel<2><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
+    else route_topk_wave_kernel<4><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
+  } else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
   return after_launch("route_topk");
 }
 

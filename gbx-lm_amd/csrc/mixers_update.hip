@@ -121,7 +121,7 @@ __global__ __launch_bounds__(NT) void router_rows_kernel(const T* __restrict__ h
   if (lane == 0) logits[t * E + e] = s;
 }
 
-// One workgroup per row.  The choice runs on the logits (softmax keeps their order) and by RANK: an expert counts the candidates in front
+// One workgroup per row (more than 256 experts or 64 choices; others: route_groups_wave_kernel).  The choice runs on the logits (softmax keeps their order) and by RANK: an expert counts the candidates in front
 // of it -- larger, or equal with a lower index -- so no round waits for another; ranks are a permutation (a logit that is not a number
 // counts as the smallest).  LDS: candidate logits [E, padded to 4 with -inf], group maxima [n_groups, padded], partial sums.
 __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restrict__ logits, int64_t row, int* __restrict__ idx, float* __restrict__ weight,
@@ -131,13 +131,13 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
   float* cl = lds;
   float* gl = lds + (E + 3) / 4 * 4;
   const int64_t t = blockIdx.x;
-  const int nth = blockDim.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const float* lr = logits + t * row;
   auto at = [&](int e) { const float v = lr[e]; return v == v ? v : -INFINITY; };
-  for (int e = tid; e < (E + 3) / 4 * 4; e += nth) cl[e] = e < E ? at(e) : -INFINITY;
+  for (int e = tid; e < (E + 3) / 4 * 4; e += NT) cl[e] = e < E ? at(e) : -INFINITY;
   __syncthreads();
   if (sigmoid) {                                       // (its order is the logits' order)
-    for (int e = tid; e < E; e += nth) {
+    for (int e = tid; e < E; e += NT) {
       const int rank = rank_of(cl, (E + 3) / 4, e, cl[e]);
       if (rank < top) {
         idx[t * top + rank] = e;
@@ -147,27 +147,18 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
     return;
   }
   float mx = -INFINITY;
-  for (int e = tid; e < E; e += nth) mx = fmaxf(mx, cl[e]);
+  for (int e = tid; e < E; e += NT) mx = fmaxf(mx, cl[e]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  if (nth > 64) {
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    for (int i = 0; i < nth / 64; ++i) mx = fmaxf(mx, red[i]);
-    __syncthreads();
-  }
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  for (int i = 0; i < NW; ++i) mx = fmaxf(mx, red[i]);
   float sum = 0.f;
-  for (int e = tid; e < E; e += nth) sum += expf(cl[e] - mx);
-  sum = wave_sum(sum);
-  if (nth > 64) {
-    if ((tid & 63) == 0) red[tid >> 6] = sum;
-    __syncthreads();
-    sum = 0.f;
-    for (int i = 0; i < nth / 64; ++i) sum += red[i];
-  }
+  for (int e = tid; e < E; e += NT) sum += expf(cl[e] - mx);
+  sum = block_sum<NW>(sum, red);
   if (n_groups > 0) {
     const int size = E / n_groups, g4 = (n_groups + 3) / 4;
-    for (int g = tid; g < 4 * g4; g += nth) {
+    for (int g = tid; g < 4 * g4; g += NT) {
       float a = -INFINITY;
       if (g < n_groups)
 #pragma unroll 8
@@ -175,13 +166,13 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
       gl[g] = a;
     }
     __syncthreads();
-    for (int e = tid; e < E; e += nth) {
+    for (int e = tid; e < E; e += NT) {
       const int g = e / size;
       if (rank_of(gl, g4, g, gl[g]) >= keep_groups) cl[e] = -INFINITY;      // (only this thread reads cl[e] until the barrier)
     }
     __syncthreads();
   }
-  for (int e = tid; e < E; e += nth) {
+  for (int e = tid; e < E; e += NT) {
     const float x = cl[e];
     const int rank = rank_of(cl, (E + 3) / 4, e, x);
     if (rank < top) {
@@ -190,6 +181,59 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
     }
   }
   if (gate && tid == 0) weight[t * weight_row + top] = 1.f / (1.f + expf(-lr[E]));
+}
+
+// The same for up to 64 PER experts, a wave per row.
+template <int PER>
+__global__ __launch_bounds__(NT) void route_groups_wave_kernel(const float* __restrict__ logits, int64_t row, int* __restrict__ idx, float* __restrict__ weight,
+                                                              int64_t weight_row, int64_t rows, int E, int top, int n_groups, int keep_groups, int gate, int sigmoid) {
+  __shared__ float all[NW][64 * PER];
+  const int lane = threadIdx.x & 63;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (t >= rows) return;
+  const float* lr = logits + t * row;
+  float x[PER], mx = -INFINITY, sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const float v = lr[min(lane + 64 * i, E - 1)];
+    x[i] = lane + 64 * i < E && v == v ? v : -INFINITY;
+    mx = fmaxf(mx, x[i]);
+  }
+  unsigned key[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) key[i] = lane + 64 * i < E ? order_key(x[i]) : 0u;
+  if (!sigmoid) {
+    mx = wave_max(mx);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sum += wave_sum(lane + 64 * i < E ? expf(x[i] - mx) : 0.f);
+    if (n_groups > 0) {                                                  // (at most 64: a lane each)
+      float* cl = all[threadIdx.x >> 6];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) cl[lane + 64 * i] = x[i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");             // (a wave's LDS accesses run in program order)
+      const int size = E / n_groups;
+      float a = -INFINITY;
+      if (lane < n_groups)
+#pragma unroll 8
+        for (int e = lane * size; e < (lane + 1) * size; ++e) a = fmaxf(a, cl[e]);
+      unsigned long long stays = 0;
+      unsigned group[1] = {lane < n_groups ? order_key(a) : 0u};
+      wave_choose(group, keep_groups, [&](int, int g, unsigned) { stays |= 1ull << g; });
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (lane + 64 * i < E && !(stays >> min((lane + 64 * i) / size, 63) & 1)) key[i] = order_key(-INFINITY);
+    }
+  }
+  float chosen = 0.f;                                                    // lane k holds choice k
+  int mine = 0;
+  wave_choose(key, top, [&](int k, int e, unsigned m) {
+    if (lane == k) { mine = e; chosen = key_value(m); }
+  });
+  if (lane < top) {
+    idx[t * top + lane] = mine;
+    weight[t * weight_row + lane] = sigmoid ? 1.f / (1.f + expf(-chosen)) : expf(chosen - mx) / sum;
+  }
+  if (gate && lane == 0) weight[t * weight_row + top] = 1.f / (1.f + expf(-lr[E]));
 }
 
 bool act_ok(int act) { return act == GBXM_BF16 || act == GBXM_F32; }
@@ -249,9 +293,18 @@ int gbxm_route_groups(const float* logits, int64_t row, int32_t* idx, float* wei
   if (E > 8192) return fail(GBXM_ERR_UNSUPPORTED, "route_groups: more than 8192 experts");
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const size_t lds = ((E + 3) / 4 * 4 + (n_groups + 3) / 4 * 4 + 4) * sizeof(float);
-  route_groups_kernel<<<dim3(T_), E <= 64 ? 64 : (E <= 128 ? 128 : NT), lds, s>>>(logits, row, idx, weight, weight_row, E, top, n_groups, keep_groups, gate,
-                                                                                          sigmoid);
+  if (choice_by_wave(E, top) && n_groups <= 64) {
+    const unsigned blocks = choice_blocks(T_), threads = choice_threads(T_);
+#define GBXM_CHOOSE(PER_) \
+  route_groups_wave_kernel<PER_><<<blocks, threads, 0, s>>>(logits, row, idx, weight, weight_row, T_, E, top, n_groups, keep_groups, gate, sigmoid)
+    if (E <= 64) GBXM_CHOOSE(1);
+    else if (E <= 128) GBXM_CHOOSE(2);
+    else GBXM_CHOOSE(4);
+#undef GBXM_CHOOSE
+  } else {
+    const size_t lds = ((E + 3) / 4 * 4 + (n_groups + 3) / 4 * 4 + 4) * sizeof(float);
+    route_groups_kernel<<<dim3(T_), NT, lds, s>>>(logits, row, idx, weight, weight_row, E, top, n_groups, keep_groups, gate, sigmoid);
+  }
   return after_launch("route_groups");
 }
 

@@ -1,4 +1,4 @@
-"""Router choices by rank (csrc/mixers_common.h: RANK_EXPERTS) against rounds of arg-max on the host: expert counts around a wave, a workgroup and the
+"""Router choices of a wave (csrc/mixers_common.h: wave_choose) and of a workgroup against rounds of arg-max on the host: expert counts around a wave, a workgroup and the
 limit, ties, experts that a correction of -inf takes out, groups, and steps on both sides of the few-row logits.  Rows of a unit matrix make the
 logits exactly the router's entries; weights to a few fp32 roundings."""
 import pytest
@@ -115,6 +115,37 @@ def test_sigmoid_choice_of_odd_logits(e, top, groups):
             key = sorted((-v if v == v else 1.0, i) for i, v in enumerate(c[r].tolist()))
             got = [c[r, i].item() for i in idx[r].tolist()]
             assert all(a != a if v > 0 else abs(a + v) < 1e-6 for a, (v, _) in zip(got, key))
+
+
+CHOICES = [(1, 1, None), (63, 4, (9, 2)), (64, 64, None), (65, 8, None), (128, 8, (8, 4)), (129, 65, None), (192, 6, (64, 40)), (256, 8, (8, 4)), (256, 64, (128, 64)),
+           (260, 8, (4, 2))]
+
+
+@pytest.mark.parametrize("e,top,groups,form", [c + (f,) for c in CHOICES for f in ("softmax", "gate", "sigmoid") if f != "sigmoid" or not c[2]])
+@pytest.mark.parametrize("t", [3, 1030])
+def test_choice_on_logits(e, top, groups, t, form):
+    """Both forms' limits -- 64 experts a register, 256 of them, 64 choices, 64 groups -- with ties, numbers missing and infinities."""
+    from gbx_lm_amd import _lib
+    gate = form == "gate"
+    rows = (torch.randint(-6, 7, (t, e + gate), generator=torch.Generator().manual_seed(e + t)) / 4.0).float()
+    if e > 1:
+        rows[0, : e // 2 : 3], rows[1, e - 1] = float("nan"), float("-inf")
+    x, idx, w = rows.to(DEV).contiguous(), torch.full((t, top), -1, dtype=torch.int32, device=DEV), torch.zeros((t, top + gate), device=DEV)
+    count, keep = groups or (0, 0)
+    _lib.check_mixers(_lib.mixers().gbxm_route_groups(x.data_ptr(), e + gate, idx.data_ptr(), w.data_ptr(), top + gate, t, e, top, count, keep, int(gate), int(form == "sigmoid"),
+                                                     torch.cuda.current_stream().cuda_stream))
+    c = torch.nan_to_num(rows[:, :e], nan=float("-inf"), neginf=float("-inf")).double()
+    p = torch.sigmoid(c) if form == "sigmoid" else torch.softmax(c, -1)
+    if groups:
+        best = torch.sort(c.view(t, count, -1).amax(-1), dim=-1, descending=True, stable=True).indices[:, :keep]
+        kept = torch.zeros((t, count), dtype=torch.bool).scatter_(1, best, True).repeat_interleave(e // count, 1)
+        c = c.masked_fill(~kept, float("-inf"))
+    want = torch.sort(c, dim=-1, descending=True, stable=True).indices[:, :top]
+    assert torch.equal(idx.cpu().long(), want)
+    pw = torch.where(c.gather(1, want) == float("-inf"), 0.0, p.gather(1, want)) if form != "sigmoid" else p.gather(1, want)
+    assert bool(((w.cpu().double()[:, :top] - pw).abs() <= (e / 64 + 24) * 2.0 ** -24 * pw).all())
+    if gate:
+        assert bool(((w.cpu().double()[:, top] - torch.sigmoid(rows[:, e].double())).abs() <= 8 * 2.0 ** -24).all())
 
 
 @pytest.mark.parametrize("t,e,k", [(4, 1024, 2048), (5, 1024, 2048), (32, 1023, 2048), (32, 1024, 2048), (1, 1025, 8190), (33, 64, 100)])
