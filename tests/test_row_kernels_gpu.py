@@ -95,3 +95,47 @@ def test_shift(width, dt):
     parts = [run(torch.cat([x[:2], x[6:7]]), StepBatch.build([0, 1], [0, 0], [2, 1], DEV)), run(torch.cat([x[2:6], x[7:]]), StepBatch.build([0, 1], [2, 1], [4, 2], DEV))]
     again = torch.cat([parts[0][:2], parts[1][:4], parts[0][2:], parts[1][4:]])
     assert torch.equal(again, whole) and torch.equal(cache.rows[:2], kept[:2])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", WIDTHS)
+@pytest.mark.parametrize("top,off", [(1, 0), (8, 0), (9, 0), (2, 1)])
+def test_embedding_and_norms(width, dt, top, off):
+    """Rows embedded (exact but for the scale's rounding), added behind a norm of one branch or of several candidates, normed."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(width + top)
+    table, tok, w = torch.randn((11, width), generator=g).to(dt), torch.tensor([3, 0, 10, 3]), torch.rand(width, generator=g) + 0.5
+    x, h = M.embed_scaled(shifted(table, off), tok.to(DEV), 0.7)
+    want = table[tok].float() * 0.7
+    assert torch.equal(x.cpu(), want) and (h is x or torch.equal(h.cpu(), want.to(dt)))
+    y = torch.rand((4, top, width) if top > 1 else (4, width), generator=g).to(dt) + 0.5
+    mix = torch.rand((4, top), generator=g) if top > 1 else None
+    z = y.double() if top == 1 else (y.double() * mix.double().unsqueeze(-1)).sum(1)
+    new = want.double() + 0.3 * z / z.pow(2).mean(-1, keepdim=True).add(1e-5).sqrt() * w.double()
+    xd = shifted(want, off)
+    h = M.residual_norm_add(xd, shifted(y, off), None if mix is None else mix.to(DEV), w.to(DEV), 1e-5, 0.3, dt)
+    assert near(xd, new, torch.float32) and near(h, new, dt)
+    n = M.stream_rmsnorm(shifted(want, off), w.to(DEV), 1e-5, dt)
+    assert near(n, want.double() / want.double().pow(2).mean(-1, keepdim=True).add(1e-5).sqrt() * w.double(), dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n0,n1,tail,off", [(4096, 512, 512, 0), (256, 256, 0, 0), (260, 4, 8, 0), (2048, 2048, 4, 0), (3840, 260, 0, 0), (6144, 2048, 0, 0), (8192, 512, 0, 0), (6, 4, 2, 0),
+                                            (64, 64, 1, 0), (128, 64, 64, 1)])
+def test_segments_and_window_rows(n0, n1, tail, off, dt):
+    """Two segments of a row normed on their own: one and two groups a thread, the widest that fit, one more, rows off the grid of four; then the rows
+    behind the first segment appended to the rings as they are."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(n0 + n1)
+    rows, w0, w1 = torch.randn((5, n0 + n1 + tail), generator=g).to(dt), torch.rand(n0, generator=g) + 0.5, torch.rand(n1, generator=g) + 0.5
+    d = shifted(rows, off)
+    M.segment_rmsnorm_(d, n0, n1, w0.to(DEV), w1.to(DEV), 1e-5)
+    unit = lambda v: v.double() / v.double().pow(2).mean(-1, keepdim=True).add(1e-5).sqrt()
+    assert near(d[:, :n0], unit(rows[:, :n0]) * w0.double(), dt) and near(d[:, n0:n0 + n1], unit(rows[:, n0:n0 + n1]) * w1.double(), dt)
+    assert torch.equal(d[:, n0 + n1:].cpu(), rows[:, n0 + n1:])
+    if tail:
+        batch = StepBatch.build([1, 0], [0, 2], [3, 2], DEV)
+        kc, vc = (torch.zeros((2, 4, n), dtype=dt, device=DEV) for n in (n1, tail))
+        M.window_append(d, n0, n1, kc, vc, batch, 4)
+        for slot, at, row in ((1, 0, 0), (1, 1, 1), (1, 2, 2), (0, 2, 3), (0, 3, 4)):
+            assert torch.equal(kc[slot, at], d[row, n0:n0 + n1]) and torch.equal(vc[slot, at], d[row, n0 + n1:])
