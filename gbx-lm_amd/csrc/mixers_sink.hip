@@ -212,57 +212,57 @@ __global__ __launch_bounds__(NT) void sink_rows_kernel(const T* __restrict__ q, 
   }
 }
 
-// One workgroup per (row, head): joins the key splits' (sum, maximum, denominator) in split order, adds the sink, applies the gate.
-// Rows of `partial` are partial_width(dv) floats (the sums, padding to a multiple of four, maximum, denominator), so a thread
-// reads four channels at once; the two halves of the workgroup take the even and the odd splits and meet in LDS.
+// Joins the key splits' (sum, maximum, denominator), adds the sink, applies the gate; one workgroup per (row, head, 128 channels).  Rows of `partial`
+// are partial_width(dv) floats (the sums, padding to a multiple of four, maximum, denominator), so a thread reads four channels at once; eight
+// groups of 32 threads take every eighth split, all of it (at most 64) in flight beside the splits' weights -- one trip to memory, where two
+// halves of a workgroup for all channels made eight -- and meet in LDS in a fixed order.
 template <typename T, bool FAST>
 __global__ __launch_bounds__(256) void sink_reduce_kernel(const float* __restrict__ partial, T* __restrict__ out, const float* __restrict__ sink,
                                                          const T* __restrict__ gate, int64_t gate_row, int gate_channels, int64_t T_, int H, int dv,
                                                          int splits, int64_t out_row) {
   __shared__ float wz[64];
   __shared__ float den;
-  __shared__ float4 other[128];
+  __shared__ float4 part[8][32];
   const int64_t t = blockIdx.x;
-  const int head = blockIdx.y, pw = partial_width(dv);
+  const int head = blockIdx.y, pw = partial_width(dv), group = threadIdx.x >> 5, q = threadIdx.x & 31, d = blockIdx.z * 128 + 4 * q;
   const int64_t zs = T_ * H * pw;
   const float* p0 = partial + (t * H + head) * pw;
+  float4 v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {                                          // (channels past dv inside the last four are padding)
+    const int z = group + 8 * i;
+    v[i] = z < splits && d < dv ? *reinterpret_cast<const float4*>(p0 + z * zs + d) : float4{0.f, 0.f, 0.f, 0.f};
+  }
   if (threadIdx.x < 64) {
     const int z = threadIdx.x;
-    const float m = z < splits ? p0[z * zs + pw - 2] : -INFINITY;
-    float top = m;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+    const float m = z < splits ? p0[z * zs + pw - 2] : -INFINITY, lz = z < splits ? p0[z * zs + pw - 1] : 0.f;
+    float top = wave_max(m);
     if (sink) top = fmaxf(top, sink[head]);
     const float w = z < splits ? exp_<FAST>(m - top) : 0.f;
     wz[z] = w;
-    float l = z < splits ? w * p0[z * zs + pw - 1] : 0.f;
-    l = wave_sum(l);
+    const float l = wave_sum(z < splits ? w * lz : 0.f);
     if (z == 0) den = l + (sink ? exp_<FAST>(sink[head] - top) : 0.f);
   }
   __syncthreads();
-  const float f = (gate && !gate_channels ? sigmoid_<FAST>(to_f32(gate[t * gate_row + head])) : 1.f) / den;
-  const int half = threadIdx.x >> 7, q = threadIdx.x & 127;
-  for (int d0 = 0; d0 < dv; d0 += 512) {
-    const int d = d0 + 4 * q;
-    float4 s = float4{0.f, 0.f, 0.f, 0.f};
-    if (d < dv)
-#pragma unroll 4
-      for (int z = half; z < splits; z += 2) {
-        const float4 v = *reinterpret_cast<const float4*>(p0 + z * zs + d);      // (channels past dv inside the last four are padding)
-        const float w = wz[z];
-        s.x += w * v.x; s.y += w * v.y; s.z += w * v.z; s.w += w * v.w;
-      }
-    __syncthreads();
-    if (half) other[q] = s;
-    __syncthreads();
-    if (!half && d < dv) {
-      const float4 u = other[q];
-      const float r[4] = {(s.x + u.x) * f, (s.y + u.y) * f, (s.z + u.z) * f, (s.w + u.w) * f};
-      for (int c = 0; c < 4 && d + c < dv; ++c)
-        out[t * out_row + head * dv + d + c] =
-            from_f32<T>(gate && gate_channels ? r[c] * sigmoid_<FAST>(to_f32(gate[t * gate_row + head * dv + d + c])) : r[c]);
+  float4 s = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (group + 8 * i < splits) {
+      const float w = wz[group + 8 * i];
+      s.x += w * v[i].x; s.y += w * v[i].y; s.z += w * v[i].z; s.w += w * v[i].w;
     }
+  part[group][q] = s;
+  __syncthreads();
+  if (group || d >= dv) return;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) {
+    const float4 u = part[i][q];
+    s.x += u.x; s.y += u.y; s.z += u.z; s.w += u.w;
   }
+  const float f = (gate && !gate_channels ? sigmoid_<FAST>(to_f32(gate[t * gate_row + head])) : 1.f) / den;
+  const float r[4] = {s.x * f, s.y * f, s.z * f, s.w * f};
+  for (int c = 0; c < 4 && d + c < dv; ++c)
+    out[t * out_row + head * dv + d + c] = from_f32<T>(gate && gate_channels ? r[c] * sigmoid_<FAST>(to_f32(gate[t * gate_row + head * dv + d + c])) : r[c]);
 }
 
 template <typename T, bool FAST>
@@ -297,7 +297,7 @@ int launch_rows(const gbxm_sink_attn_args& a, const SinkGeo& g, int rc, int chun
     if (vec) go(sink_rows_kernel<T, FAST, true, NCH_MAX>);
     else go(sink_rows_kernel<T, FAST, false, NCH_MAX>);
   }
-  if (splits > 1) sink_reduce_kernel<T, FAST><<<dim3(a.T, a.H), 256, 0, s>>>(part, out, a.sink, gate, a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits,
+  if (splits > 1) sink_reduce_kernel<T, FAST><<<dim3(a.T, a.H, (a.dv + 127) / 128), 256, 0, s>>>(part, out, a.sink, gate, a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits,
                                                                                        g.out_row);
   return after_launch("sink_attention (rows)");
 }
@@ -684,7 +684,7 @@ int launch_sink_group(const gbxm_sink_attn_args& a, hipStream_t s);     // the s
 bool sink_tiles_shape(int dk, int dv);
 
 int launch_sink_reduce(const gbxm_sink_attn_args& a, int splits, hipStream_t s) {
-  sink_reduce_kernel<bf16_t, true><<<dim3(a.T, a.H), 256, 0, s>>>(static_cast<const float*>(a.partial), static_cast<bf16_t*>(a.out), a.sink,
+  sink_reduce_kernel<bf16_t, true><<<dim3(a.T, a.H, (a.dv + 127) / 128), 256, 0, s>>>(static_cast<const float*>(a.partial), static_cast<bf16_t*>(a.out), a.sink,
                                                                   static_cast<const bf16_t*>(a.gate), a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits,
                                                                   a.out_row > 0 ? a.out_row : static_cast<int64_t>(a.H) * a.dv);
   return after_launch("sink_attention (join of key splits)");

@@ -357,8 +357,10 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
 // owns every fourth 32-channel block of the value product.  No mask besides the end of the key run.  With key splits a workgroup
 // leaves (sum, maximum, denominator) per head for sink_reduce_kernel, else it finishes the row itself.
 // ALIAS: the values are the first dv channels of the key rows (one staged tile serves both products).
-template <int DK, int DV, bool ALIAS>
-__global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, const int* __restrict__ tok, int splits, float* __restrict__ partial) {
+// A launch is one trip to memory and one pass over code that is read cold (1.2 ns a byte): FULL drops the tests of heads smaller than <DK, DV> and of
+// groups of more than 32 heads.
+template <int DK, int DV, bool ALIAS, bool FULL>
+__global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, const int* __restrict__ tok, int R, int splits, float* __restrict__ partial) {
   constexpr int KT = 32;
   constexpr int KROW = DK * 2 + 16;
   constexpr int VROW = ALIAS ? KROW : DV * 2 + 64;
@@ -369,16 +371,17 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
   constexpr bool SPLITK = KS >= 16;
   constexpr int KSW = SPLITK ? (KS + 3) / 4 : KS;
   constexpr int TILE_BYTES = KT * KROW + (ALIAS ? 0 : KT * VROW);
-  __shared__ __attribute__((aligned(16))) unsigned char lds[TILE_BYTES + (SPLITK ? 4 * 16 * 64 * 4 : 0)];
+  constexpr int SROW = 80;                                              // bytes of a lane's 16 partial scores (+16: conflict-free 16-byte accesses)
+  __shared__ __attribute__((aligned(16))) unsigned char lds[TILE_BYTES + (SPLITK ? 4 * 64 * SROW : 0)];
   unsigned char* kl = lds;
   unsigned char* vl = ALIAS ? lds : lds + KT * KROW;
-  float* sred = reinterpret_cast<float*>(lds + TILE_BYTES);            // [4 waves][16][64 lanes]
+  unsigned char* sred = lds + TILE_BYTES;                               // [4 waves][64 lanes][16]
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hb = lane >> 5;
   const int64_t t = blockIdx.x;
-  const int R = a.H / a.G, chunks = (R + 31) / 32;
-  const int kvh = blockIdx.y / chunks, hloc = (blockIdx.y % chunks) * 32 + r;
+  const int chunks = FULL ? 1 : (R + 31) / 32;
+  const int kvh = FULL ? blockIdx.y : blockIdx.y / chunks, hloc = FULL ? r : (blockIdx.y % chunks) * 32 + r;
   const bool hvalid = hloc < R;
   const int head = kvh * R + min(hloc, R - 1);
   const int b = tok[2 * t], pos = tok[2 * t + 1];
@@ -391,7 +394,7 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
 #pragma unroll
     for (int i = 0; i < KSW; ++i) {
       const int c = (ks0 + i) * 16 + hb * 8;
-      qf[i] = (ks0 + i < KS && c < a.dk) ? *reinterpret_cast<const u32x4*>(qp + c) : u32x4{0, 0, 0, 0};
+      qf[i] = (FULL && (!SPLITK || KS % 4 == 0)) || (ks0 + i < KS && c < a.dk) ? *reinterpret_cast<const u32x4*>(qp + c) : u32x4{0, 0, 0, 0};
     }
   }
   f32x16 o[DTW];
@@ -401,15 +404,6 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
   const int lo = first_seen(pos, a.window, a.chunk);
   const int na = min(a.keep, lo);
   const int total = na + (pos - lo + 1);
-  auto pos_of = [&](int iv) { return iv < na ? iv : lo + (iv - na); };
-  auto krow = [&](int j) -> const bf16_t* {
-    if (j < pos0) return a.kc + slot * a.kc_slot + static_cast<int64_t>(j < a.keep ? j : a.keep + (j - a.keep) % a.ring) * a.kc_row + kvh * a.kc_head;
-    return a.kn + static_cast<int64_t>(row0 + (j - pos0)) * a.k_row + kvh * a.k_head;
-  };
-  auto vrow = [&](int j) -> const bf16_t* {
-    if (j < pos0) return a.vc + slot * a.vc_slot + static_cast<int64_t>(j < a.keep ? j : a.keep + (j - a.keep) % a.ring) * a.vc_row + kvh * a.vc_head;
-    return a.vn + static_cast<int64_t>(row0 + (j - pos0)) * a.v_row + kvh * a.v_head;
-  };
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float scale2 = (a.head_scale ? a.scale * a.head_scale[head] : a.scale) * LOG2E;
@@ -419,95 +413,103 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
-  // a key (and value) tile: global -> registers -> LDS; with SPLITK the registers are filled one tile ahead
-  constexpr int KP = (KT * (DK / 8) + 255) / 256, VP = ALIAS ? 1 : (KT * (DV / 8) + 255) / 256;
-  u32x4 kr[KP], vr[VP];
-  auto fetch = [&](int it) {
-#pragma unroll
-    for (int i = 0; i < KP; ++i) {
-      const int p = tid + 256 * i, row = p / (DK / 8), c = p % (DK / 8), iv = it + row;
-      kr[i] = u32x4{0, 0, 0, 0};
-      if (p < KT * (DK / 8) && iv < total && c * 8 < a.dk) kr[i] = *reinterpret_cast<const u32x4*>(krow(pos_of(iv)) + c * 8);
-    }
-    if constexpr (!ALIAS) {
-#pragma unroll
-      for (int i = 0; i < VP; ++i) {
-        const int p = tid + 256 * i, row = p / (DV / 8), c = p % (DV / 8), iv = it + row;
-        vr[i] = u32x4{0, 0, 0, 0};
-        if (p < KT * (DV / 8) && iv < total && c * 8 < a.dv) vr[i] = *reinterpret_cast<const u32x4*>(vrow(pos_of(iv)) + c * 8);
-      }
-    }
+  // A key (and value) tile: global -> registers -> LDS, one tile ahead.  A thread looks each of its rows up once and takes all its pieces of it from there.
+  // The last key's row stands for those behind it, whose weights are zero.
+  typedef RowPieces<DK, KT> KP;
+  typedef RowPieces<ALIAS ? 32 : DV, KT> VP;
+  u32x4 kr[KP::N], vr[VP::N];
+  const bool round = pos >= a.keep + a.ring;                            // the ring has come round
+  auto row_of = [&](const bf16_t* old, int64_t old_row, const bf16_t* fresh, int64_t fresh_row, int iv) -> const bf16_t* {
+    iv = min(iv, total - 1);
+    const int j = iv < na ? iv : lo + (iv - na);
+    return j < pos0 ? old + static_cast<int64_t>(round && j >= a.keep ? a.keep + (j - a.keep) % a.ring : j) * old_row
+                    : fresh + static_cast<int64_t>(j - pos0) * fresh_row;
   };
-  auto stage = [&]() {
+  const bf16_t *kc = a.kc + slot * a.kc_slot + kvh * a.kc_head, *kn = a.kn + row0 * a.k_row + kvh * a.k_head;
+  const bf16_t *vc = a.vc + slot * a.vc_slot + kvh * a.vc_head, *vn = a.vn + row0 * a.v_row + kvh * a.v_head;
+  auto load = [&](auto pieces, u32x4* regs, const bf16_t* old, int64_t old_row, const bf16_t* fresh, int64_t fresh_row, int it, int width) {
+    typedef decltype(pieces) P;
+    const bf16_t* row = nullptr;
 #pragma unroll
-    for (int i = 0; i < KP; ++i) {
-      const int p = tid + 256 * i;
-      if (p < KT * (DK / 8)) *reinterpret_cast<u32x4*>(kl + (p / (DK / 8)) * KROW + (p % (DK / 8)) * 16) = kr[i];
-    }
-    if constexpr (!ALIAS) {
-#pragma unroll
-      for (int i = 0; i < VP; ++i) {
-        const int p = tid + 256 * i;
-        if (p < KT * (DV / 8)) *reinterpret_cast<u32x4*>(vl + (p / (DV / 8)) * VROW + (p % (DV / 8)) * 16) = vr[i];
-      }
+    for (int i = 0; i < P::N; ++i) {
+      if (P::LINEAR || i % P::PER == 0) row = row_of(old, old_row, fresh, fresh_row, it + P::row(tid, i));
+      const int c = P::piece(tid, i);
+      regs[i] = P::used(tid, i) && (FULL || c * 8 < width) ? *reinterpret_cast<const u32x4*>(row + c * 8) : u32x4{0, 0, 0, 0};
     }
   };
 
   const int it0 = static_cast<int>(blockIdx.z) * KT, step = KT * splits;
-  if (SPLITK && it0 < total) fetch(it0);
-  for (int it = it0; it < total; it += step) {
-    if constexpr (!SPLITK) fetch(it);
-    __syncthreads();                                          // the previous tile (and its partial scores) have been consumed
-    stage();
-    __syncthreads();
-    if (SPLITK && it + step < total) fetch(it + step);        // the next tile travels while this one is computed
-    f32x16 st = f32x16{0};
-#pragma unroll
-    for (int i = 0; i < KSW; ++i)
-      if (ks0 + i < KS) st = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + (ks0 + i) * 32), qf[i], st);      // wave-uniform test
-    if constexpr (SPLITK) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sred[(wave * 16 + e) * 64 + lane] = st[e];
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        st[e] = (sred[e * 64 + lane] + sred[(16 + e) * 64 + lane]) + (sred[(32 + e) * 64 + lane] + sred[(48 + e) * 64 + lane]);
+  for (int it = it0;; it += step) {                           // (one loop body: a launch of one tile reads all of its code cold)
+    if (it < total) {
+      load(KP{}, kr, kc, a.kc_row, kn, a.k_row, it, a.dk);
+      if constexpr (!ALIAS) load(VP{}, vr, vc, a.vc_row, vn, a.v_row, it, a.dv);
     }
-    float s[16];
-    float mx = -INFINITY;
+    if (it != it0) {                                          // the tile before is multiplied while this one travels
+      f32x16 st = f32x16{0};
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int iv = it + 8 * (e >> 2) + 4 * hb + (e & 3);
-      s[e] = iv < total ? st[e] * scale2 : -INFINITY;
-      mx = fmaxf(mx, s[e]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                   // finite: a tile holds at least one key
-    const float m_new = fmaxf(m, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-    m = m_new;
-    float ps = 0.f;
+      for (int i = 0; i < KSW; ++i)
+        if (ks0 + i < KS) st = mfma_bf16(*reinterpret_cast<const u32x4*>(kbase + (ks0 + i) * 32), qf[i], st);      // wave-uniform test
+      if constexpr (SPLITK) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) { s[e] = __builtin_amdgcn_exp2f(s[e] - m_new); ps += s[e]; }
-    l = l * alpha + ps;
-    u32x4 gf[2];
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<f32x4v*>(sred + (wave * 64 + lane) * SROW + e * 16) = f32x4v{st[4 * e], st[4 * e + 1], st[4 * e + 2], st[4 * e + 3]};
+        __syncthreads();
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-      gf[tt] = u32x4{pack2(s[8 * tt], s[8 * tt + 1]), pack2(s[8 * tt + 2], s[8 * tt + 3]), pack2(s[8 * tt + 4], s[8 * tt + 5]),
-                     pack2(s[8 * tt + 6], s[8 * tt + 7])};
+        for (int e = 0; e < 4; ++e) {
+          f32x4v p[4];
 #pragma unroll
-    for (int i = 0; i < DTW; ++i) {
-      const int dt = wave + 4 * i;                            // wave-uniform
-      if (dt < DT) {
+          for (int w = 0; w < 4; ++w) p[w] = *reinterpret_cast<const f32x4v*>(sred + (w * 64 + lane) * SROW + e * 16);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+          for (int i = 0; i < 4; ++i) st[4 * e + i] = (p[0][i] + p[1][i]) + (p[2][i] + p[3][i]);
+        }
+      }
+      const int first = it - step + 4 * hb;
+      float s[16];
+      float mx = -INFINITY;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-          const u32x2 v0 = lds_read_tr(vbase + (16 * tt) * VROW + dt * 64);
-          const u32x2 v1 = lds_read_tr(vbase + (16 * tt + 8) * VROW + dt * 64);
-          o[i] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[i]);
+      for (int e = 0; e < 16; ++e) {
+        s[e] = first + 8 * (e >> 2) + (e & 3) < total ? st[e] * scale2 : -INFINITY;
+        mx = fmaxf(mx, s[e]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                 // finite: a tile holds at least one key
+      const float m_new = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      float ps = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) { s[e] = __builtin_amdgcn_exp2f(s[e] - m_new); ps += s[e]; }
+      l = l * alpha + ps;
+      u32x4 gf[2];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+        gf[tt] = u32x4{pack2(s[8 * tt], s[8 * tt + 1]), pack2(s[8 * tt + 2], s[8 * tt + 3]), pack2(s[8 * tt + 4], s[8 * tt + 5]),
+                       pack2(s[8 * tt + 6], s[8 * tt + 7])};
+#pragma unroll
+      for (int i = 0; i < DTW; ++i) {
+        const int dt = wave + 4 * i;                          // wave-uniform
+        if (DT % 4 == 0 || dt < DT) {
+          if (it != it0 + step)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+#pragma unroll
+          for (int tt = 0; tt < 2; ++tt) {
+            const u32x2 v0 = lds_read_tr(vbase + (16 * tt) * VROW + dt * 64);
+            const u32x2 v1 = lds_read_tr(vbase + (16 * tt + 8) * VROW + dt * 64);
+            o[i] = mfma_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, gf[tt], o[i]);
+          }
         }
       }
     }
+    if (it >= total) break;
+    __syncthreads();                                          // the tile before (and its partial scores) has been consumed
+#pragma unroll
+    for (int i = 0; i < KP::N; ++i)
+      if (KP::used(tid, i)) *reinterpret_cast<u32x4*>(kl + KP::row(tid, i) * KROW + KP::piece(tid, i) * 16) = kr[i];
+    if constexpr (!ALIAS) {
+#pragma unroll
+      for (int i = 0; i < VP::N; ++i)
+        if (VP::used(tid, i)) *reinterpret_cast<u32x4*>(vl + VP::row(tid, i) * VROW + VP::piece(tid, i) * 16) = vr[i];
+    }
+    __syncthreads();
   }
 
   l += __shfl_xor(l, 32, 64);
@@ -518,11 +520,11 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
 #pragma unroll
     for (int i = 0; i < DTW; ++i) {
       const int dt = wave + 4 * i;
-      if (dt < DT)
+      if (DT % 4 == 0 || dt < DT)
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
           const int d = dt * 32 + 8 * q4 + 4 * hb;
-          if (d < a.dv) *reinterpret_cast<float4*>(prow + d) = float4{o[i][4 * q4], o[i][4 * q4 + 1], o[i][4 * q4 + 2], o[i][4 * q4 + 3]};
+          if (FULL || d < a.dv) *reinterpret_cast<float4*>(prow + d) = float4{o[i][4 * q4], o[i][4 * q4 + 1], o[i][4 * q4 + 2], o[i][4 * q4 + 3]};
         }
     }
     if (wave == 0 && hb == 0) { prow[pw - 2] = m / LOG2E; prow[pw - 1] = l; }
@@ -553,7 +555,9 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
     splits = static_cast<int>(std::min<int64_t>(std::min<int64_t>(512 / groups, 64), a.partial_splits));
     if (splits < 2) splits = 1;
   }
-  sink_group_kernel<DK, DV, ALIAS><<<dim3(a.T, a.G * chunks, splits), 256, 0, s>>>(t, a.tok, splits, static_cast<float*>(a.partial));
+  const dim3 grid(a.T, a.G * chunks, splits);
+  if (a.dk == DK && a.dv == DV && R <= 32) sink_group_kernel<DK, DV, ALIAS, true><<<grid, 256, 0, s>>>(t, a.tok, R, splits, static_cast<float*>(a.partial));
+  else sink_group_kernel<DK, DV, ALIAS, false><<<grid, 256, 0, s>>>(t, a.tok, R, splits, static_cast<float*>(a.partial));
   const int rc = after_launch("sink_attention (grouped rows)");
   if (rc != GBXM_OK || splits == 1) return rc;
   return launch_sink_reduce(a, splits, s);

@@ -59,37 +59,57 @@ def portions(lens, dk, dv, window):
 def test_portions_behind_a_history(window, keep, dk, dv, H):
     """Key tiles that lie whole in the table or in the step's rows, and those that the kept rows, the ring's seam or the first new row cuts; rows
     further apart than a head.  The last shape takes the form of one group."""
+    behind([0, 1, 64, 130, 515, 1000], [300, 129, 64, 200, 33, 140], window, keep, dk, dv, H, 2)
+
+
+@pytest.mark.parametrize("window,keep", [(None, 0), (200, 5), (33, 0)])
+@pytest.mark.parametrize("dk,dv,H,G,values", [(64, 64, 8, 2, True), (128, 128, 16, 4, True), (128, 104, 16, 4, True), (96, 96, 40, 1, True), (256, 256, 8, 2, True), (576, 512, 16, 1, False),
+                                              (560, 512, 16, 1, False), (320, 256, 8, 1, False), (96, 96, 36, 1, False)])
+@pytest.mark.parametrize("rows", [1, 7, 300])
+def test_single_rows_behind_a_history(window, keep, dk, dv, H, G, values, rows):
+    """One row a sequence: heads that fill their capacity and heads that do not, groups of more than 32, values of their own and values that are the
+    keys', key tiles shared out over many workgroups and one workgroup for all."""
+    first = [(37 * i * i + 11 * i) % (700 if rows < 300 else 90) for i in range(rows)]
+    first[0] = 650 if rows < 300 else 89
+    behind(first, [1] * rows, window, keep, dk, dv, H, G, values)
+
+
+def behind(first, lens, window, keep, dk, dv, H, G, values=True):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
     from gbx_lm_amd.models.cache import SequenceSlots, SlotKVCache
     gen = torch.Generator(device=DEV).manual_seed(dk + dv + H)
-    first, lens, G = [0, 1, 64, 130, 515, 1000], [300, 129, 64, 200, 33, 140], 2
     T, n = sum(lens), len(lens)
 
     def rows(count, heads, d):
         return torch.randn((count, heads * d + 24), device=DEV, generator=gen).to(torch.bfloat16)[:, 8:8 + heads * d].view(count, heads, d)
 
-    cache = SlotKVCache(G * dk, G * dv, window, keep, SequenceSlots(n))
+    cache = SlotKVCache(G * dk, G * dv if values else 0, window, keep, SequenceSlots(n))
     cache.reserve(max(f + c for f, c in zip(first, lens)), torch.bfloat16, torch.device(DEV))
-    past = [(rows(f, G, dk), rows(f, G, dv)) for f in first]
-    for b, (k, v) in enumerate(past):
-        for p in range(k.shape[0]):                            # (later positions of a ring take the places of earlier ones)
-            at = p if p < cache.keep else cache.keep + (p - cache.keep) % cache.ring
-            cache.keys[b, at], cache.values[b, at] = k[p].reshape(-1), v[p].reshape(-1)
+    past = []
+    for b, f in enumerate(first):
+        k = rows(f, G, dk)
+        past.append((k, rows(f, G, dv) if values else k[..., :dv]))
+        p = torch.arange(f, device=DEV)
+        p = p[(p < cache.keep) | (p >= f - cache.ring)]            # (later positions of a ring take the places of earlier ones)
+        at = cache.row_of(p)
+        cache.keys[b, at] = k[p].reshape(-1, G * dk)
+        if values:
+            cache.values[b, at] = past[b][1][p].reshape(-1, G * dv)
     batch = StepBatch.build(list(range(n)), first, lens, DEV)
-    q, k, v = rows(T, H, dk), rows(T, G, dk), rows(T, G, dv)
+    q, k = rows(T, H, dk), rows(T, G, dk)
+    v = rows(T, G, dv) if values else k[..., :dv]
     sink = torch.randn(H, device=DEV, generator=gen)
     got = M.sink_attention(q, k, v, cache, batch, dk ** -0.5, window, keep, sink).double().view(T, H, dv)
     r0 = 0
     for b, (f, c) in enumerate(zip(first, lens)):
         i, j = torch.arange(f, f + c, device=DEV)[:, None], torch.arange(f + c, device=DEV)[None]
         hidden = (j > i) | ((i - j >= window) & (j >= keep) if window else torch.zeros_like(j, dtype=torch.bool))
-        for h in range(H):
-            g = h // (H // G)
-            kk, vv = (torch.cat([old[:, g], new[r0:r0 + c, g]]).double() for old, new in zip(past[b], (k, v)))
-            s = (q[r0:r0 + c, h].double() @ kk.t() * dk ** -0.5).masked_fill(hidden, float("-inf"))
-            p = torch.exp(s - torch.logaddexp(torch.logsumexp(s, -1, keepdim=True), sink[h].double()))
-            want, spread, total = p @ vv, (p ** 2 @ vv ** 2).sqrt(), p @ vv.abs()
-            err = (got[r0:r0 + c, h] - want).abs()
-            assert bool((err <= 3 * 2.0 ** -8 * (want.abs() + spread) + 2.0 ** -16 * total + 1e-6).all()), (b, h, float(err.max()))
+        kk, vv = (torch.cat([old, new[r0:r0 + c]]).double().repeat_interleave(H // G, 1).transpose(0, 1) for old, new in zip(past[b], (k, v)))
+        s = torch.matmul(q[r0:r0 + c].double().transpose(0, 1), kk.transpose(1, 2).contiguous()) * dk ** -0.5
+        s = s.masked_fill(hidden, float("-inf"))
+        p = torch.exp(s - torch.logaddexp(torch.logsumexp(s, -1, keepdim=True), sink.double()[:, None, None]))
+        want, spread, total = (x.transpose(0, 1) for x in (torch.matmul(p, vv.contiguous()), torch.matmul(p ** 2, vv.contiguous() ** 2).sqrt(), torch.matmul(p, vv.contiguous().abs())))
+        err = (got[r0:r0 + c] - want).abs()
+        assert bool((err <= 3 * 2.0 ** -8 * (want.abs() + spread) + 2.0 ** -16 * total + 1e-6).all()), (b, float(err.max()))
         r0 += c
