@@ -139,3 +139,66 @@ def test_segments_and_window_rows(n0, n1, tail, off, dt):
         M.window_append(d, n0, n1, kc, vc, batch, 4)
         for slot, at, row in ((1, 0, 0), (1, 1, 1), (1, 2, 2), (0, 2, 3), (0, 3, 4)):
             assert torch.equal(kc[slot, at], d[row, n0:n0 + n1]) and torch.equal(vc[slot, at], d[row, n0 + n1:])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", WIDTHS)
+@pytest.mark.parametrize("branch,top,mixed,extra,replace,normed,off", [(True, 0, False, False, False, True, 0), (False, 8, True, False, False, True, 0), (True, 9, True, True, True, False, 0),
+                                                                         (False, 1, False, True, False, True, 0), (True, 2, True, False, False, True, 1)])
+def test_layer_update(width, dt, branch, top, mixed, extra, replace, normed, off):
+    """Every part of the sum alone and together, the stream replaced or added to, with and without the next norm; an image at a stride of its own."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(width + top)
+    x, w = torch.randn((3, width), generator=g), torch.rand(width, generator=g) + 0.5
+    b = torch.randn((3, width), generator=g).to(dt) if branch else None
+    cand = torch.randn((3, top, width), generator=g).to(dt) if top else None
+    mix = torch.rand((3, top + 1), generator=g) if mixed else None
+    ex = torch.randn((3, width), generator=g).to(dt) if extra else None
+    parts = [p.double() for p in (None if replace else x, b, ex) if p is not None]
+    if top:
+        parts += [cand[:, k].double() * (mix[:, k:k + 1].double() if mixed else 1.0) for k in range(top)]
+    want, room = sum(parts), sum(p.abs() for p in parts)
+    dev = lambda t: None if t is None else shifted(t, off)
+    xd, image = shifted(x, off), torch.zeros((3, width + 8), dtype=dt, device=DEV)
+    h = M.layer_update_(xd, dev(b), dev(cand), None if mix is None else mix.to(DEV), w.to(DEV) if normed else None, 1e-5, image[:, :width], replace, dev(ex))
+    assert bool(((xd.cpu().double() - want).abs() <= (top + 4) * 2.0 ** -24 * room).all())
+    assert torch.equal(image[:, :width], xd.to(dt)) and float(image[:, width:].abs().max()) == 0.0
+    if normed:
+        unit = xd.cpu().double() / xd.cpu().double().pow(2).mean(-1, keepdim=True).add(1e-5).sqrt() * w.double()
+        assert near(h, unit, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,heads,n_in,n_out,tail", [(1, 1, 1, 8, 0), (2, 16, 128, 512, 64), (2, 16, 512, 128, 0), (3, 5, 100, 72, 8), (1, 8, 64, 1032, 0), (15, 17, 33, 40, 2), (16, 16, 128, 72, 8)])
+def test_a_matrix_per_head(rows, heads, n_in, n_out, tail, dt):
+    """Few rows times heads cut into runs of outputs -- a last run that is not full, inputs off the grid of a workgroup -- and one more, uncut; the tail as it is."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(n_in + n_out)
+    x, w = torch.randn((rows, heads, n_in + tail), generator=g).to(dt), torch.randn((heads, n_in, n_out), generator=g).to(dt)
+    gate = torch.randn((rows, heads * n_out), generator=g).to(dt) if not tail else None
+    got = M.head_project(x.to(DEV), w.to(DEV), tail, gate=None if gate is None else gate.to(DEV)).cpu().double()
+    z, room = (torch.matmul(a.transpose(0, 1), b).transpose(0, 1) for a, b in ((x[..., :n_in].double(), w.double()), (x[..., :n_in].double().abs(), w.double().abs())))
+    f = torch.sigmoid(gate.double()).view(rows, heads, n_out) if gate is not None else 1.0
+    assert bool(((got[..., :n_out] - z * f).abs() <= (ROW[dt] if dt == torch.bfloat16 else 2.0 ** -20) * (z * f).abs() + (n_in + 8) * 2.0 ** -24 * room).all())
+    assert torch.equal(got[..., n_out:], x[..., n_in:].double())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,v,off", [(8, 4, 0), (576, 0, 0), (6, 4, 0), (8, 6, 0), (8, 8, 1), (1028, 512, 0)])
+@pytest.mark.parametrize("window,keep", [(None, 0), (5, 3)])
+def test_rows_appended_to_slots(k, v, off, dt, window, keep):
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.models.cache import SequenceSlots, SlotKVCache
+    g = torch.Generator().manual_seed(k + v)
+    cache = SlotKVCache(k, v, window, keep, SequenceSlots(2), first_capacity=16)
+    cache.reserve(16, dt, torch.device(DEV))
+    batch = StepBatch.build([1, 0], [2, 9], [11, 1], DEV)
+    kr, vr = torch.randn((12, k), generator=g).to(dt), torch.randn((12, v), generator=g).to(dt) if v else None
+    M.slot_append(cache, shifted(kr, off), None if vr is None else shifted(vr, off), batch)
+    rows = {}
+    for r, (slot, pos) in enumerate([(1, 2 + i) for i in range(11)] + [(0, 9)]):
+        rows[(slot, pos if pos < cache.keep else cache.keep + (pos - cache.keep) % cache.ring)] = r
+    for (slot, at), r in rows.items():
+        assert torch.equal(cache.keys[slot, at].cpu(), kr[r])
+        if v:
+            assert torch.equal(cache.values[slot, at].cpu(), vr[r])
