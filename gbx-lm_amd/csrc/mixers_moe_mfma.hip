@@ -17,14 +17,19 @@
 // requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
 // Measured (us, first + second products with the sort; 256-pair tiles with results from the registers -> results by rows, in turn on one card, uniform choices, the least of
 // four places of the weights in memory, which move these times by up to a tenth):
-//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (now 410: 640 TFLOP/s, 2.9 TB/s of weights)
-//   18 128 pairs of the same:                       340 -> 326 (now 315: 3.8 TB/s)
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (now 406: 650 TFLOP/s, 3.0 TB/s of weights)
+//   18 128 pairs of the same:                       340 -> 326 (now 306: 3.9 TB/s)
 //   16 384 pairs,  64 experts, 2048 x 2048, no gate: 437 -> 422 (now 389); a factor of the weights' way from memory (one expert's for all: 150 less) and of the results' (kept back:
 //   75 less), which tiles of one round write at the same time
 //    8 192 pairs,   8 experts, 4096 x 2048 gated:   461 -> 457 (900 TFLOP/s)
 // The table keeps a lower tile beside its expert's others.  By falling height, so that the last round is short, tiles read their weights anew: 256 pairs an
 // expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  A stage's lines ordered into L2 before gain nothing; nor does
 // it matter how many rows a request spans (256 x 128 B, 64 x 512 B or 32 KB in one piece: 4.4 to 4.7 TB/s).
+// An expert's tiles walk the contraction from a stage of their own (expert % stages, so that a pair's sums do not depend on the step's other pairs): rows of
+// a power of two of bytes put a column of every row on the same memory channels, and workgroups that started together stayed there together.  All from the
+// first stage | this, us: 64 experts of 2 x 2048 x 2048, 2 000 pairs 259 | 200 (5.4 TB/s), 64 of 3 x 2048 x 1024, 6 000 pairs 208 | 178, 128 of 3 x 2048 x
+// 768, 2 048 pairs 237 | 228, 18 128 318 | 306; offsets by column
+// block as well lose the activation rows that its workgroups share in L2 (8 experts of 3 x 4096 x 2048, 8 192 pairs 449 | 446 | 479 by both).
 // The grid is sized for the worst case sum_e ceil(n_e / 256) <= P / 256 + E; surplus workgroups leave at once.
 // Steps with few pairs per expert (a batch that decodes) stream weights and little else: expert_skinny_kernel takes tiles of 32 pairs, a
 // wave per 32 output channels and no barrier.  A wave moves its own rows -- eight lanes to a row's 128 bytes, so an access touches eight
@@ -36,7 +41,10 @@ namespace gbxm {
 namespace {
 
 constexpr int RS = 32;          // pairs per tile of the skinny form
-constexpr int BROW = 128 + 16;  // LDS bytes per activation row of a chunk (+16: conflict-free 16-byte fragment reads)
+// LDS bytes per row of a chunk; 16-byte column c of row r lies at c ^ ((r / 2) & 7), which meets no bank twice in the 16 lanes of a fragment read and lets
+// three gated workgroups share a CU (rows of 144 bytes: two)
+constexpr int BROW = 128;
+__device__ __forceinline__ int chunk_at(int r, int c) { return r * BROW + ((c ^ (r >> 1)) & 7) * 16; }
 
 // One workgroup; E1 = E + 1 buckets, the last for indices that name no expert.  A pair's place in its bucket is what the counting atomic returns, kept
 // in registers; the order then forms in LDS and leaves in whole lines (scattered, a wave's stores take the address unit 64 cycles).  Beyond KEEP
@@ -156,7 +164,7 @@ constexpr int PAST = -16;                    // byte offset (as unsigned) beyond
 
 // One tile of 32 NR pairs x 256 weight rows.  See the head of the file.
 template <int FORM, int NR>
-__device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* lds, int e, int lo, int hi, int col) {
+__device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* lds, int e, int lo, int hi, int col, int turn) {
   constexpr bool GATED = FORM == EXPERT_SILU || FORM == EXPERT_CLAMPED;
   constexpr int PA = (NR + 3) / 4;                                      // 16-byte activation pieces per thread and half-tile
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wc = wave & 3;
@@ -192,16 +200,17 @@ __device__ __forceinline__ void group_tile(const GroupArgs& a, unsigned char* ld
       vob[h][i] = min(GATED ? (b >> 6) * 32 + (b & 31) : b, N - 1 - r0) * C * 2 + lcol;
     }
   }
+  auto stage_of = [&](int t) { t = min(t, n - 1) + turn; return t < n ? t : t - n; };
   // half-tile h of stage t; past the end the last stage again: every wait counts the same requests
   auto stage_a = [&](int t, int h) {
-    const int tc = min(t, n - 1);
+    const int tc = stage_of(t);
     const bool cut = tc * 64 + 32 == C && lcol >= 64;                   // the second half of a stage that the contraction does not fill
     unsigned char* dst = lds + (t & 1) * GSTAGE + h * GHALF + wave * 1024;
 #pragma unroll
     for (int i = 0; i < PA; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, GBXM_LDSP(dst + i * 8192), 16, cut ? PAST : voa[h][i], tc * 128, 0, 0);
   };
   auto stage_b = [&](int t, int slot, int h) {
-    const int tc = min(t, n - 1);
+    const int tc = stage_of(t);
     const bool cut = tc * 64 + 32 == C && lcol >= 64;
     unsigned char* dst = lds + (2 + slot) * GSTAGE + h * GHALF + wave * 1024;
 #pragma unroll
@@ -338,11 +347,12 @@ __global__ __launch_bounds__(512) void expert_group_kernel(const GroupArgs a) {
   const int4 tab = a.tile_tab[bt];
   const int e = tab.x, lo = tab.y, hi = tab.z;
   if (e >= a.E) return;                                                 // (pairs without an expert)
+  const int turn = e % ((a.C + 63) >> 6);
   switch ((hi - lo + 63) / 64) {
-    case 1: group_tile<FORM, 2>(a, lds, e, lo, hi, col); break;
-    case 2: group_tile<FORM, 4>(a, lds, e, lo, hi, col); break;
-    case 3: group_tile<FORM, 6>(a, lds, e, lo, hi, col); break;
-    default: group_tile<FORM, 8>(a, lds, e, lo, hi, col); break;
+    case 1: group_tile<FORM, 2>(a, lds, e, lo, hi, col, turn); break;
+    case 2: group_tile<FORM, 4>(a, lds, e, lo, hi, col, turn); break;
+    case 3: group_tile<FORM, 6>(a, lds, e, lo, hi, col, turn); break;
+    default: group_tile<FORM, 8>(a, lds, e, lo, hi, col, turn); break;
   }
 }
 
@@ -374,7 +384,7 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
   const int4 tab = tile_tab[u.tile];
   const int e = tab.x, lo = tab.y, hi = tab.z;
   if (e >= E) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, hb = lane >> 5;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, hb = lane >> 5;
   const int c0 = u.col * 128 + wave * 32;
   if (c0 >= N) return;
   const int row = min(lo + r, hi - 1), pair = sorted[row];
@@ -383,23 +393,27 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
   unsigned char* mine = lds[wave][0];
   // this lane's pieces of a chunk: rows lane / 8 + 8 i, 16 bytes at column piece lane % 8 (a 32-element tail has four column pieces)
   const int mrow = lane >> 3, col = lane & 7;
-  const bf16_t* wp = w + (static_cast<int64_t>(e) * (TWO ? 2 : 1) * N + c0 + mrow) * C + col * 8;
-  const int64_t up = static_cast<int64_t>(N) * C;
-  const bf16_t* xp[4];
+  // (buffer loads: a lane's place is fixed, the chunk is scalar; the down product's rows are neighbours, the others lie within 2 GB)
+  const bf16_t *w0 = w + (static_cast<int64_t>(e) * (TWO ? 2 : 1) * N + c0) * C, *x0 = FORM == SKINNY_DOWN ? in + static_cast<int64_t>(lo) * C : in;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w0), 0, 0x7FFFFFFF, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w0 + static_cast<int64_t>(N) * C), 0, 0x7FFFFFFF, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(x0), 0, 0x7FFFFFFF, 0x00020000);
+  const int wo = (mrow * C + col * 8) * 2;
+  int xo[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int p = min(lo + mrow + 8 * i, hi - 1);
-    xp[i] = in + static_cast<int64_t>(FORM == SKINNY_DOWN ? p : sorted[p] / top) * C + col * 8;
+    xo[i] = ((FORM == SKINNY_DOWN ? p - lo : sorted[p] / top) * C + col * 8) * 2;
   }
   f32x16 acc = f32x16{0}, acc2 = f32x16{0};
   struct Pieces { u32x4 v[PARTS][4]; };
   auto load = [&](Pieces& f, int k0, int cols) {
-    const int k = col < cols ? k0 : k0 - 32;                            // (a piece past the tail repeats one inside it; nobody reads it)
+    const int back = col < cols ? 0 : 64;                               // (a piece past the tail repeats one inside it; nobody reads it)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      f.v[0][i] = *reinterpret_cast<const u32x4*>(wp + static_cast<int64_t>(8 * i) * C + k);
-      if constexpr (TWO) f.v[1][i] = *reinterpret_cast<const u32x4*>(wp + up + static_cast<int64_t>(8 * i) * C + k);
-      f.v[PARTS - 1][i] = *reinterpret_cast<const u32x4*>(xp[i] + k);
+      f.v[0][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo - back, (8 * i * C + k0) * 2, 0));
+      if constexpr (TWO) f.v[1][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, wo - back, (8 * i * C + k0) * 2, 0));
+      f.v[PARTS - 1][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i] - back, k0 * 2, 0));
     }
   };
   auto mul = [&](const Pieces& f, auto steps_c) {
@@ -408,12 +422,12 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
 #pragma unroll                                                          //  no barrier among waves, only the compiler must keep the order)
     for (int q = 0; q < PARTS; ++q)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(mine + q * (RS * BROW) + (mrow + 8 * i) * BROW + col * 16) = f.v[q][i];
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(mine + q * (RS * BROW) + chunk_at(mrow + 8 * i, col)) = f.v[q][i];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < S; ++i) {
-      const unsigned char* p = mine + r * BROW + (hb * S + i) * 16;
+      const unsigned char* p = mine + chunk_at(r, hb * S + i);
       const u32x4 x = *reinterpret_cast<const u32x4*>(p + (PARTS - 1) * (RS * BROW));
       acc = mfma_bf16(*reinterpret_cast<const u32x4*>(p), x, acc);
       if constexpr (TWO) acc2 = mfma_bf16(*reinterpret_cast<const u32x4*>(p + RS * BROW), x, acc2);
@@ -425,11 +439,14 @@ __global__ __launch_bounds__(256) void expert_skinny_kernel(const bf16_t* __rest
   const int full = C / 64;
   if (full) {
     Pieces f0, f1;
-    load(f0, 0, 8);
+    // (column blocks of experts start the contraction at chunks of their own, as the tiles above)
+    const int turn = (u.col + e * 5) & ((1 << (31 - __builtin_clz(full))) - 1);
+    const auto chunk = [&](int i) { i = min(i, full - 1) + turn; return (i < full ? i : i - full) * 64; };
+    load(f0, chunk(0), 8);
     for (int i = 0; i < full; i += 2) {                                 // (the loads past the end repeat the last chunk)
-      load(f1, min(i + 1, full - 1) * 64, 8);
+      load(f1, chunk(i + 1), 8);
       mul(f0, whole);
-      load(f0, min(i + 2, full - 1) * 64, 8);
+      load(f0, chunk(i + 2), 8);
       if (i + 1 < full) mul(f1, whole);
     }
   }
@@ -471,12 +488,12 @@ int launch_group(const GroupArgs& g, int tiles, hipStream_t s) {
 size_t align16(size_t n) { return (n + 15) & ~static_cast<size_t>(15); }
 constexpr int64_t MIN_PAIRS = 64;         // below this the weight-streaming row kernels read less
 // Pairs per expert (on average) up to which the skinny form is taken.  Measured at 4 | 8 | 16 | 64 pairs per expert, skinny against grouped, us:
-// 128 experts of 3 x 2048 x 768  231 | 248 | 297 | 459  against 235 | 243 | 243 | 277;  64 of 2 x 2048 x 2048  230 | 237 | 277 | 448  against
-// 254 | 256 | 258 | 276;  32 of 3 x 1024 x 512  31 | 30 | 33 | 42  against 29 | 29 | 30 | 35.
+// 128 experts of 3 x 2048 x 768  215 | 223 | 235 | 389  against 220 | 219 | 223 | 255;  64 of 2 x 2048 x 2048  187 | 196 | 211 | 374  against
+// 191 | 194 | 199 | 218;  32 of 3 x 1024 x 512  28 | 28 | 28 | 41  against 29 | 29 | 29 | 36.
 constexpr int64_t SKINNY_PAIRS = 8;
 // ... and, where the grouped form's first product has at most half a chip of workgroups, each of them a chain over the whole contraction, up to 64.  Skinny |
-// grouped, us: without a gate, 16 experts of 2 x 1024 x 512, 4 | 32 | 64 pairs per expert 21 | 23 | 26 against 27 | 30 | 35; 8 of 2 x 4096 x 2048, 16 | 32 | 64
-// 71 | 90 | 113 against 106 | 108 | 119, 128 172 against 136; gated, 4 of 3 x 512 x 2048, 64 pairs 33 against 43.
+// grouped, us: without a gate, 16 experts of 2 x 1024 x 512, 4 | 32 | 64 pairs per expert 18 | 20 | 23 against 26 | 28 | 32; 8 of 2 x 4096 x 2048, 16 | 32 | 64
+// 58 | 76 | 111 against 79 | 81 | 96; gated, 4 of 3 x 512 x 2048, 32 | 64 | 128 pairs 26 | 27 | 32 against 37 | 46 | 56.
 constexpr int64_t SKINNY_PAIRS_FEW = 64, FEW_GROUPS = 128;
 int rows_of(int64_t P, int E, int F, bool gated) {
   const int64_t groups = (P / GR + E) * (gated ? (F + 127) / 128 : (F + 255) / 256);
@@ -555,10 +572,8 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
   if (rows == RS) {
     const auto grid = [&](int n) { return static_cast<unsigned>((static_cast<int64_t>(tiles) * ((n + 127) / 128) + 7) / 8 * 8); };
     const unsigned up = grid(F), dn = grid(K);
-    if (a.kind == GBXM_EXPERT_RELU2)
-      expert_skinny_kernel<SKINNY_UP><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
-    else
-      expert_skinny_kernel<SKINNY_GATED><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
+    if (gated) expert_skinny_kernel<SKINNY_GATED><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
+    else expert_skinny_kernel<SKINNY_UP><<<up, 256, 0, s>>>(h, first, offsets, sorted, tile_tab, a.scale, act, F, K, E, top, a.kind, a.limit);
     expert_skinny_kernel<SKINNY_DOWN><<<dn, 256, 0, s>>>(act, static_cast<const bf16_t*>(a.down), offsets, sorted, tile_tab, nullptr,
                                                          static_cast<bf16_t*>(a.y), K, F, E, top, a.kind, a.limit);
     return after_launch("expert_ff (skinny groups)");

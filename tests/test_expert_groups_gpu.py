@@ -91,3 +91,20 @@ def test_more_pairs_than_the_sort_keeps(experts, pairs):
     counts = (w / w.sum() * pairs).long().tolist()
     counts[-1] += pairs - sum(counts)
     tiles(counts, "relu2", 32, 32)
+
+
+@pytest.mark.parametrize("rows,top", [(40, 2), (700, 2)], ids=["skinny", "grouped"])
+@pytest.mark.parametrize("width,ff", [(1056, 736), (512, 1056)])
+def test_a_pair_does_not_depend_on_its_neighbours(rows, top, width, ff):
+    """Experts start the contraction at places of their own, over whole and odd numbers of chunks: the same bits for a row wherever it stands in the step."""
+    from gbx_lm_amd import mixer_ops as M
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    experts = 9
+    first = (torch.randn(experts, 2 * ff, width, generator=gen, device="cuda") / width ** 0.5).bfloat16()
+    down = (torch.randn(experts, width, ff, generator=gen, device="cuda") / ff ** 0.5).bfloat16()
+    h = torch.randn(rows, width, generator=gen, device="cuda").bfloat16()
+    idx = torch.rand(rows, experts, generator=gen, device="cuda").topk(top, -1).indices.to(torch.int32).contiguous()
+    got = M.expert_glu(h, first, down, idx, "silu", 1.5, None)
+    turned = torch.randperm(rows, generator=gen, device="cuda")
+    again = M.expert_glu(h[turned].contiguous(), first, down, idx[turned].contiguous(), "silu", 1.5, None)
+    assert torch.equal(got.reshape(rows, -1)[turned], again.reshape(rows, -1))
