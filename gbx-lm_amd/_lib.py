@@ -452,6 +452,8 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_recurrent_prepare.argtypes = [ctypes.POINTER(RecurrentPrepArgs), p]
         L.gbxm_conv_tail_update.argtypes = [p, i64, p, p, i32, i32, i32, i32, p]
         L.gbxm_state_scan.argtypes = [p, i64, p, p, p, i32, i64, i32, i32, i32, i32, i32, p]
+        L.gbxm_state_scan_ws.argtypes = [p, i64, p, p, p, i32, i64, i32, i32, i32, i32, i32, p, sz, p]
+        L.gbxm_state_scan_workspace.argtypes, L.gbxm_state_scan_workspace.restype = [i32, i64, i64, i32, i32, i32], sz
         L.gbxm_head_norm_gate.argtypes = [p, p, i64, p, p, i64, i64, i32, i32, f32, i32, i32, p]
         L.gbxm_embed_hashed_pair.argtypes = [p, p, p, p, p, p, p, i64, i32, i64, i64, i64, i32, p]
         L.gbxm_norm_token_shift.argtypes = [p, p, p, p, p, p, p, i64, i32, f32, i32, p]

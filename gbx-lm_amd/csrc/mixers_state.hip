@@ -3,14 +3,14 @@
 //   recurrent_prep_kernel   short causal convolution + silu on q | k | v, unit q / k heads (a wave per head), q scale, the decay
 //                           exp(-rate_h softplus(sign (a + bias))) and beta = sigmoid(b), all in fp32, into one fp32 row.
 //   conv_tail_kernel        the last taps-1 convolution inputs of every sequence into its slot.
-//   state_scan_kernel<R>    the scan.  The columns of a head's state (one per value channel) never meet: a wave takes four columns, 16
+//   state_scan_kernel<R>    the scan token by token (longer portions go by chunks: mixers_state_mfma.hip).  The columns of a head's state (one per value channel) never meet: a wave takes four columns, 16
 //                           lanes per column, a lane holds R key channels of its column in registers; per token the two dot products
 //                           over key channels are R multiply-adds and four cross-lane adds inside a 16-lane row (all 16 lanes end
 //                           with the same bits).  Operands come through LDS in chunks of tokens, the next chunk fetched while the
 //                           current one is computed.  Sums run in a fixed order: a sequence's result does not depend on what else is
 //                           in the step, nor on how many columns a workgroup takes.
 //   head_norm_gate_kernel   per-head RMS norm of the read-out, weight and gate, one wave per (row, head).
-#include "mixers_common.h"
+#include "mixers_mfma.h"
 
 namespace gbxm {
 namespace {
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(NT) void conv_tail_kernel(const T* __restrict__ y, 
 // one channel a lane 51.6, 28.4 here), 66 to 96 only where sizes are not in groups of four (94 x 64 59.4 | 43.1; 96 x 96 in groups of four 50).
 template <int R, bool DELTA, int NW, int V>
 __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __restrict__ r, int64_t r_stride, float* __restrict__ state,
-                                                            float* __restrict__ out, const int* __restrict__ seq, int H, int G, int dk, int dv) {
+                                                            float* __restrict__ out, const int* __restrict__ seq, int H, int G, int dk, int dv, StateChunks made) {
   constexpr int C = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;                 // neighbouring channels of a lane
   constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL, NTH = 64 * NW, Q = R / C;
   constexpr int CH = NW == 1 ? (R <= 4 ? 4 : 2) : (R <= 4 ? 32 : (R <= 8 ? 16 : 8)) * NW / 4;     // one-wave workgroups serve steps of few rows
@@ -243,6 +243,7 @@ __global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __rest
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ks = lane & 15;
   const int col0 = blockIdx.x * NCOL, lcol = wave * 4 + (lane >> 4), col = col0 + lcol;
   const int slot = seq[4 * b], pos0 = seq[4 * b + 1], n = seq[4 * b + 2], row0 = seq[4 * b + 3];
+  if (made.flags && state_by_chunks(n, made.flags + static_cast<int64_t>(h) * made.places + row0 / 16 + b, (n + 15) / 16)) return;
   const bool col_ok = col < dv;
   const int colc = col_ok ? col : dv - 1;
   const int nq = G * dk, nv = H * dv;
@@ -438,18 +439,18 @@ void launch_head_norm_gate(const float* o, const void* gate, int64_t gate_stride
 
 template <bool DELTA, int NW>
 int launch_scan(int R, int B, hipStream_t s, const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int H, int G, int dk,
-                int dv) {
+                int dv, StateChunks made) {
   const dim3 grid((dv + 4 * NW - 1) / (4 * NW), H, B);
   const bool vec = dk % 4 == 0 && dv % 4 == 0 && r_stride % 4 == 0 && all_aligned(16, r, state);
 #define GBXM_SCAN(N)                                                                                                    \
   do {                                                                                                                  \
-    if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);   \
-    else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);       \
+    if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);   \
+    else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);       \
   } while (0)
   if (R <= 1) GBXM_SCAN(1);
   else if (R <= 2) GBXM_SCAN(2);
   else if (R <= 4) GBXM_SCAN(4);
-  else if (R <= 6 && !vec) state_scan_kernel<6, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv);
+  else if (R <= 6 && !vec) state_scan_kernel<6, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);
   else if (R <= 8) GBXM_SCAN(8);
   else if (R <= 12) GBXM_SCAN(12);
   else GBXM_SCAN(16);
@@ -509,8 +510,17 @@ int gbxm_conv_tail_update(const void* y, int64_t y_stride, void* tail, const int
   return after_launch("conv_tail_update");
 }
 
+size_t gbxm_state_scan_workspace(int32_t B, int64_t T_, int64_t longest, int32_t H, int32_t dk, int32_t dv) {
+  return longest < STATE_CHUNKS_FROM || B < 1 || T_ < longest || H < 1 ? 0 : state_chunks_workspace(T_, B, H, dk, dv);
+}
+
 int gbxm_state_scan(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T_, int32_t H, int32_t G,
                     int32_t dk, int32_t dv, int32_t delta, void* stream) {
+  return gbxm_state_scan_ws(r, r_stride, state, out, seq, B, T_, H, G, dk, dv, delta, nullptr, 0, stream);
+}
+
+int gbxm_state_scan_ws(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T_, int32_t H, int32_t G,
+                       int32_t dk, int32_t dv, int32_t delta, void* ws, size_t ws_bytes, void* stream) {
   if (!r || !state || !out || !seq || B < 0 || H < 1 || G < 1 || H % G || dk < 1 || dv < 1 ||
       r_stride < 2 * G * dk + H * dv + H * dk + (delta ? H : 0))
     return fail(GBXM_ERR_INVALID, "state_scan: bad argument");
@@ -519,13 +529,19 @@ int gbxm_state_scan(const float* r, int64_t r_stride, float* state, float* out, 
   if (B > 65535 || H > 65535) return fail(GBXM_ERR_UNSUPPORTED, "state_scan: grid");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int R = (dk + 15) / 16;
+  StateChunks made{nullptr, 0};
+  const size_t need = ws ? state_chunks_workspace(T_, B, H, dk, dv) : 0;
+  if (need && ws_bytes >= need && r_stride % 4 == 0 && r_stride <= (1 << 22) && all_aligned(16, r, static_cast<const float*>(ws), state)) {
+    const int rc = launch_state_chunks(r, r_stride, state, out, seq, B, T_, H, G, dk, dv, delta, ws, s, &made);
+    if (rc != GBXM_OK) return rc;
+  }
   // long rows (prompts): 16 columns per workgroup share the staged operands; a few rows per sequence: 4 columns, four times the
   // workgroups for the state's traffic.  A column's arithmetic is the same in both.
   if (T_ >= 8 * static_cast<int64_t>(B))
-    return delta ? launch_scan<true, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv)
-                 : launch_scan<false, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv);
-  return delta ? launch_scan<true, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv)
-               : launch_scan<false, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv);
+    return delta ? launch_scan<true, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made)
+                 : launch_scan<false, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made);
+  return delta ? launch_scan<true, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made)
+               : launch_scan<false, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made);
 }
 
 int gbxm_head_norm_gate(const float* o, const void* gate, int64_t gate_stride, const float* w, void* out, int64_t out_row, int64_t T_, int32_t H, int32_t dv,

@@ -559,8 +559,13 @@ def decayed_state_scan(r: torch.Tensor, lay, cache, batch, delta: bool) -> torch
     if state is None or state.dtype != torch.float32 or tuple(state.shape[1:]) != (lay.heads, lay.dv, lay.dk) or state.shape[0] <= max(batch.slot) or not state.is_contiguous():
         raise ValueError("decayed_state_scan: the cache's states do not fit the mixer or the step's slots")
     out = torch.empty((batch.total, lay.nv), dtype=torch.float32, device=r.device)
-    _lib.check_mixers(_lib.mixers().gbxm_state_scan(r.data_ptr(), r.stride(0), state.data_ptr(), out.data_ptr(), batch.seq.data_ptr(), len(batch.slot),
-                                                   batch.total, lay.heads, lay.groups, lay.dk, lay.dv, int(bool(delta)), _stream(r.device)))
+    L = _lib.mixers()
+    longest = max(batch.n_new, default=0)
+    nbytes = L.gbxm_state_scan_workspace(len(batch.slot), batch.total, longest, lay.heads, lay.dk, lay.dv) if longest > 1 else 0
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=r.device) if nbytes else None
+    _lib.check_mixers(L.gbxm_state_scan_ws(r.data_ptr(), r.stride(0), state.data_ptr(), out.data_ptr(), batch.seq.data_ptr(), len(batch.slot), batch.total,
+                                           lay.heads, lay.groups, lay.dk, lay.dv, int(bool(delta)), None if ws is None else ws.data_ptr(), nbytes,
+                                           _stream(r.device)))
     return out
 
 

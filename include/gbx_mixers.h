@@ -263,6 +263,12 @@ int gbxm_conv_tail_update(const void* y, int64_t y_stride, void* tail, const int
  * S <- S + k u^T; o = S^T q.  T: rows of the step (chooses the workgroup shape).  dk <= 256. */
 int gbxm_state_scan(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T, int32_t H, int32_t G,
                     int32_t dk, int32_t dv, int32_t delta, void* stream);
+/* The same with a workspace of gbxm_state_scan_workspace bytes (16-byte aligned; longest: rows of the step's longest sequence; 0: not a step for it): sequences of
+ * 128 rows and more then run in chunks of 16 rows on the matrix cores (fp32 products and sums in another order).  `seq` lists the sequences in the order of their
+ * rows.  No or too small a workspace: as gbxm_state_scan. */
+size_t gbxm_state_scan_workspace(int32_t B, int64_t T, int64_t longest, int32_t H, int32_t dk, int32_t dv);
+int gbxm_state_scan_ws(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T, int32_t H, int32_t G,
+                       int32_t dk, int32_t dv, int32_t delta, void* ws, size_t ws_bytes, void* stream);
 /* out[t][h][c] = o[t][h][c] / sqrt(mean_c o^2 + eps) * w[c] * gate(g[t][h][c]); gate kind 1 silu, 2 sigmoid; o fp32, g / out activation dtype;
  * w null: no weight. */
 int gbxm_head_norm_gate(const float* o, const void* gate, int64_t gate_stride, const float* w, void* out, int64_t out_row, int64_t T, int32_t H,

@@ -1,0 +1,81 @@
+"""Prompt portions of the decayed states by chunks of 16 tokens (csrc/mixers_state_mfma.hip): sequences on either side of the fewest rows that go that way, whole chunks
+and remainders, key channels in and off the 64s, value channels off the 16s, rows that are not in groups of four (three heads: token by token), fresh and carried states, decays down to zero, and numbers that the chunks leave to the
+token-by-token form (infinities, NaN, decays above one, numbers whose products might not stay finite).  Reference: float64 token by token; tolerance: fp32 sums
+over the key channels, the chunk's tokens and the tokens that a decay keeps, relative to the sums of absolute values."""
+import pytest
+import torch
+
+from gbx_lm_amd.batching import StepBatch
+from gbx_lm_amd.models import recurrent_mixers as RM
+from gbx_lm_amd.models.cache import SequenceSlots, SlotStateCache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def step(dk, dv, H, G, counts, delta, low, spoil=None):
+    g = torch.Generator().manual_seed(dk + dv + counts[0])
+    lay = RM.RecurrentLayout(H, G, dk, dv, 0, G * dk, 2 * G * dk, 2 * G * dk + H * dv if delta else -1)
+    T, B = sum(counts), len(counts)
+    q = torch.randn((T, G * dk), generator=g)
+    k = torch.nn.functional.normalize(torch.randn((T, G, dk), generator=g), dim=-1).view(T, G * dk)
+    v, d = torch.randn((T, H * dv), generator=g), torch.rand((T, H * dk), generator=g) * (1 - low) + low
+    if low == 0:
+        d[torch.rand(d.shape, generator=g) < 0.05] = 0.0
+    beta = torch.rand((T, H), generator=g)
+    if spoil:
+        spoil(q, k, v, d, beta)
+    r = torch.cat([q, k, v, d] + ([beta] if delta else []), 1)
+    cache = SlotStateCache(H, dk, dv, 0, 0, SequenceSlots(B))
+    cache.reserve(torch.float32, DEV)
+    start = torch.randn(cache.state.shape, generator=g)
+    cache.state.copy_(start)
+    slots, pos = [B - 1 - i for i in range(B)], [0 if i % 2 else 5 for i in range(B)]
+    out = RM.decayed_state_scan(r.to(DEV), lay, cache, StepBatch.build(slots, pos, list(counts), DEV), delta).cpu().double().view(T, H, dv)
+    rep, r0 = H // G, 0
+    for slot, pos0, n in zip(slots, pos, counts):
+        S = start[slot].double().clone() if pos0 else torch.zeros_like(start[slot].double())          # [H, dv, dk]
+        want, room = [], 1.0
+        for t in range(r0, r0 + n):
+            kt, qt = (x[t].double().view(G, 1, dk).repeat_interleave(rep, 0) for x in (k, q))
+            S = S * d[t].double().view(H, 1, dk)
+            u = v[t].double().view(H, dv)
+            if delta:
+                u = beta[t].double().view(H, 1) * (u - (S * kt).sum(-1))
+            S = S + u.unsqueeze(-1) * kt
+            want.append((S * qt).sum(-1))
+            room = max(room, float((S.abs() * qt.abs()).sum(-1).nan_to_num(0, 0, 0).amax()))
+        yield out[r0:r0 + n], torch.stack(want), room, cache.state[slot].cpu().double(), S
+        r0 += n
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("dk,dv,H,G", [(64, 16, 4, 2), (128, 36, 4, 2), (100, 18, 4, 1), (192, 20, 4, 1), (256, 16, 4, 4), (128, 17, 4, 4), (128, 16, 3, 1)])
+@pytest.mark.parametrize("counts,low", [((127, 128, 1, 129), 0.5), ((144, 40, 177), 0.9), ((200,), 0.0)])
+def test_chunks(dk, dv, H, G, counts, low, delta):
+    for out, want, room, state, S in step(dk, dv, H, G, counts, delta, low):
+        bound = (dk + 60) * 2.0 ** -24 * 4
+        assert float((out - want).abs().max()) < bound * room
+        assert float((state - S).abs().max()) < bound * max(float(S.abs().max()), 1.0)
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["nan value", "inf value", "nan key", "growing decay", "large key"])
+def test_left_to_the_tokens(what, delta):
+    """Each token before the odd number stays exact, and what the token-by-token form gives is not finite in the same places."""
+    def spoil(q, k, v, d, beta):
+        if what == "nan value":
+            v[37, 3] = float("nan")
+        elif what == "inf value":
+            v[37, 3] = float("inf")
+        elif what == "nan key":
+            k[37, 70] = float("nan")
+        elif what == "growing decay":
+            d[37, 5] = 1.5
+        else:
+            k[37, 5] = 1e13
+    for out, want, room, state, S in step(128, 32, 4, 1, (144, 130), delta, 0.5, spoil):
+        assert torch.equal(out.isfinite(), want.isfinite())
+        if what in ("growing decay",):
+            assert float((out - want).abs().max()) < 200 * 2.0 ** -24 * 4 * room
+        assert float((out[:37] - want[:37]).abs().max()) < 200 * 2.0 ** -24 * 4 * 100
