@@ -202,3 +202,17 @@ def test_rows_appended_to_slots(k, v, off, dt, window, keep):
         assert torch.equal(cache.keys[slot, at].cpu(), kr[r])
         if v:
             assert torch.equal(cache.values[slot, at].cpu(), vr[r])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dv,heads,off", [(256, 1, 0), (260, 3, 0), (1024, 1, 0), (1028, 2, 0), (2044, 1, 0), (2052, 1, 0), (4096, 1, 0), (4100, 1, 0), (2046, 1, 0), (2048, 1, 1)])
+@pytest.mark.parametrize("kind,weighed", [(1, True), (2, False)])
+def test_norm_of_heads_of_many_channels(dv, heads, off, dt, kind, weighed):
+    """fp32 sums of dv squares: at most (dv / 1024 + 10) roundings each way, halved by the root; the product rounds four times more."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(dv)
+    o, gate, w = torch.randn((7, heads * dv), generator=g) * 3, torch.randn((7, heads * dv), generator=g).to(dt), torch.rand(dv, generator=g)
+    got = M.head_norm_gate(o.to(DEV), shifted(gate, off), w.to(DEV) if weighed else None, heads, 1e-6, kind).cpu().double()
+    x, z = o.double().view(7, heads, dv), gate.double().view(7, heads, dv)
+    want = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * (w.double() if weighed else 1.0) * torch.sigmoid(z) * (z if kind == 1 else 1.0)
+    assert bool(((got - want.view(got.shape)).abs() <= (ROW[dt] if dt == torch.bfloat16 else 2.0 ** -20) * want.view(got.shape).abs() + 1e-30).all())
