@@ -64,7 +64,7 @@ def test_portions_behind_a_history(window, keep, dk, dv, H):
 
 @pytest.mark.parametrize("window,keep", [(None, 0), (200, 5), (33, 0)])
 @pytest.mark.parametrize("dk,dv,H,G,values", [(64, 64, 8, 2, True), (128, 128, 16, 4, True), (128, 104, 16, 4, True), (96, 96, 40, 1, True), (256, 256, 8, 2, True), (576, 512, 16, 1, False),
-                                              (560, 512, 16, 1, False), (320, 256, 8, 1, False), (96, 96, 36, 1, False)])
+                                              (512, 512, 16, 1, False), (256, 256, 8, 1, False), (560, 512, 16, 1, False), (320, 256, 8, 1, False), (96, 96, 36, 1, False)])
 @pytest.mark.parametrize("rows", [1, 7, 300])
 def test_single_rows_behind_a_history(window, keep, dk, dv, H, G, values, rows):
     """One row a sequence: heads that fill their capacity and heads that do not, groups of more than 32, values of their own and values that are the
