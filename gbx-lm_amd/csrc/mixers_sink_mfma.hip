@@ -414,7 +414,8 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
   // A key (and value) tile: global -> registers -> LDS, one tile ahead.  A thread looks each of its rows up once and takes all its pieces of it from there.
-  // The last key's row stands for those behind it, whose weights are zero.
+  // The last key's row is read in place of those behind it; values behind it go to LDS as zeros, so that a weight of zero
+  // meets no infinity (an infinite channel of a row that is key and value is no number in either case).
   typedef RowPieces<DK, KT> KP;
   typedef RowPieces<ALIAS ? 32 : DV, KT> VP;
   u32x4 kr[KP::N], vr[VP::N];
@@ -507,7 +508,8 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
     if constexpr (!ALIAS) {
 #pragma unroll
       for (int i = 0; i < VP::N; ++i)
-        if (VP::used(tid, i)) *reinterpret_cast<u32x4*>(vl + VP::row(tid, i) * VROW + VP::piece(tid, i) * 16) = vr[i];
+        if (VP::used(tid, i))
+          *reinterpret_cast<u32x4*>(vl + VP::row(tid, i) * VROW + VP::piece(tid, i) * 16) = it + VP::row(tid, i) < total ? vr[i] : u32x4{0, 0, 0, 0};
     }
     __syncthreads();
   }

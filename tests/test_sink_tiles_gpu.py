@@ -74,6 +74,26 @@ def test_single_rows_behind_a_history(window, keep, dk, dv, H, G, values, rows):
     behind(first, [1] * rows, window, keep, dk, dv, H, G, values)
 
 
+@pytest.mark.parametrize("dk,dv,H,G", [(64, 64, 8, 2), (128, 104, 16, 4), (128, 128, 16, 4), (256, 256, 8, 2)])
+@pytest.mark.parametrize("first", [[0], [40, 3, 31], [700] + [32 * i + 5 for i in range(20)]])
+def test_an_infinite_value_of_the_newest_row(dk, dv, H, G, first):
+    """The last tile of keys is not full: what lies behind the newest row adds nothing to its infinity."""
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.batching import StepBatch
+    from gbx_lm_amd.models.cache import SequenceSlots, SlotKVCache
+    gen, n = torch.Generator(device=DEV).manual_seed(dk + len(first)), len(first)
+    cache = SlotKVCache(G * dk, G * dv, None, 0, SequenceSlots(n))
+    cache.reserve(max(first) + 1, torch.bfloat16, torch.device(DEV))
+    cache.keys.normal_(generator=gen)
+    cache.values.normal_(generator=gen)
+    q, k, v = (torch.randn((n, h, d), device=DEV, generator=gen).to(torch.bfloat16) for h, d in ((H, dk), (G, dk), (G, dv)))
+    v[:, :, 3], v[:, :, dv - 2] = float("inf"), float("-inf")
+    got = M.sink_attention(q, k, v, cache, StepBatch.build(list(range(n)), first, [1] * n, DEV), dk ** -0.5, None, 0, None).float().view(n, H, dv)
+    assert bool((got[..., 3] == float("inf")).all()) and bool((got[..., dv - 2] == float("-inf")).all())
+    got[..., 3] = got[..., dv - 2] = 0
+    assert bool(got.isfinite().all())
+
+
 def behind(first, lens, window, keep, dk, dv, H, G, values=True):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
