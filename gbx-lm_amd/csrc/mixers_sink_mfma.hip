@@ -8,7 +8,7 @@
 // so that a lane owns ONE query: lane (q = lane % 32, half = lane / 32) holds 16 of the tile's 32 scores of its query, the other 16
 // are in lane ^ 32 (and as many of each further 32 keys).  The running maximum is shared by the two lanes of a query (one cross-lane exchange per tile), each keeps its
 // own part of the denominator (joined once at the end), and both rescale their accumulators (different channels of the same
-// query) by the same factor.  The sink starts the running maximum and counts once in the denominator.  Weights are rounded to bf16
+// query) by the same factor.  The sink starts the running maximum and counts once in the denominator.  Weights, at most 1, are rounded to bf16
 // for the value product; the denominator sums them in fp32.
 //
 // Bound by what a wave's own chain leaves idle (of a tile's time the matrix cores work a third, vector instructions a third: one exponential and
@@ -121,8 +121,10 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float scale2 = (a.head_scale ? a.scale * a.head_scale[head] : a.scale) * LOG2E;
-  float m = a.sink && group == 0 ? a.sink[head] * LOG2E : -INFINITY;
-  float l = (a.sink && group == 0 && hb == 0) ? 1.f : 0.f;              // the sink counts once per query
+  // what the weights are measured from: the largest score when it last moved, and 8 more, so that no weight exceeds 1 until a score is 2^8 times that one
+  constexpr float ROOM = 8.f;
+  float m = a.sink && group == 0 ? a.sink[head] * LOG2E + ROOM : -INFINITY;
+  float l = (a.sink && group == 0 && hb == 0) ? 1.f / (1 << static_cast<int>(ROOM)) : 0.f;      // the sink counts once per query
   const unsigned char* vbase = vl + (4 * hb + ((lane >> 2) & 3)) * VROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const unsigned char* kbase = kl + r * KROW + hb * 16;
 
@@ -280,10 +282,11 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
         }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                   // the other half of the query's scores
-    // the sums move to a new maximum only where one grew by more than 2^8 (weights of up to 256 keep as many bits; the factor falls out at the
-    // end).  The first scores always move it; with nothing seen yet and no sink every weight below is 2^-inf = 0
-    if (__any(mx - m > 8.f)) {
-      const float m_new = fmaxf(m, mx);
+    // the sums move to a new maximum only where a weight would exceed 1 (weights of 2^-8 keep as many bits, the factor falls out at the end; weights
+    // above 1 would take sums of values near the end of the range past it).  The first scores always move it; with nothing seen yet and no sink every
+    // weight below is 2^-inf = 0
+    if (__any(mx > m)) {
+      const float m_new = fmaxf(m, mx + ROOM);
       const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
       m = m_new;
       l *= alpha;

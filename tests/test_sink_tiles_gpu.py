@@ -94,6 +94,30 @@ def test_an_infinite_value_of_the_newest_row(dk, dv, H, G, first):
     assert bool(got.isfinite().all())
 
 
+@pytest.mark.parametrize("lens,dk,dv,H", [([130], 64, 64, 8), ([300], 128, 128, 2), ([300], 192, 128, 2), ([300] * 8, 64, 64, 32), ([300] * 8, 128, 128, 32), ([300], 256, 256, 2),
+                                          ([300] * 3, 96, 96, 4)])
+@pytest.mark.parametrize("sink", [False, True])
+def test_values_near_the_end_of_the_range(lens, dk, dv, H, sink):
+    """A key of a later tile outweighs those before it by 2^4.3 .. 2^7.9: its value of 2e38 stays finite.  Weights round to bf16 (2^-8), the result
+    once more."""
+    from gbx_lm_amd import mixer_ops as M
+    from gbx_lm_amd.batching import StepBatch
+    T = sum(lens)
+    for score in (3.0, 4.85, 5.5):
+        q, k, v = (torch.zeros((T, H, d), device=DEV, dtype=torch.bfloat16) for d in (dk, dk, dv))
+        q[..., 0] = 1.0
+        rows = [sum(lens[:b]) + 128 for b in range(len(lens))]
+        k[rows, :, 0], v[rows] = score, 2e38
+        score = float(k[rows[0], 0, 0])
+        got = M.sink_attention(q, k, v, None, StepBatch.build(list(range(len(lens))), [0] * len(lens), lens, DEV), 1.0, None, 0,
+                               torch.zeros(H, device=DEV) if sink else None).double().view(T, H, dv)
+        for r, n in zip(rows, lens):
+            i = torch.arange(128, n, device=DEV, dtype=torch.float64)
+            e = torch.exp(torch.tensor(score, dtype=torch.float64, device=DEV))
+            want = (float(v[r, 0, 0]) * e / (i + sink + e))[:, None, None]
+            assert bool(((got[r:r + n - 128] - want).abs() <= 2.0 ** -6 * want).all()), (score, n)
+
+
 def behind(first, lens, window, keep, dk, dv, H, G, values=True):
     from gbx_lm_amd import mixer_ops as M
     from gbx_lm_amd.batching import StepBatch
