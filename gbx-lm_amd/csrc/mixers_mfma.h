@@ -69,22 +69,14 @@ struct ExpertBuckets {
 size_t expert_buckets_bytes(int64_t P, int rows, int E);
 int expert_buckets(const int* idx, int P, int rows, int E, void* ws, ExpertBuckets* out, hipStream_t s);
 
-// Prompt portions of the decayed matrix states by chunks (mixers_state_mfma.hip): sequences of at least STATE_CHUNKS_FROM rows whose numbers pass the check of
-// their chunks (`flags` [H][places], 0: passed); all others go token by token.  A workgroup asks with all its threads.  One sequence of 70 | 100 | 128 | 200 rows,
-// token by token against chunks, us: delta rule, 8 heads of 64 x 128 14 | 18 | 22 | 33 against 20 | 22 | 22 | 26; 32 of 128 x 128 20 | 26 | 33 | 49 against 23 | 25 | 26 | 34.
-// A rule of the sequence alone, so that its sums do not depend on what else is in the step; a step whose longest sequence is just above it pays for both ways
-// (8, 17, 64, 100 and 130 rows of 16 heads 31 | 45).
+// Steps with sequences of STATE_CHUNKS_FROM rows and more through the decayed matrix states (mixers_state_mfma.hip).  Workspace 0: not a step for it.
+// left->flags: what the launches did, and left the rest of (null: nothing is left).
+// One sequence of 70 | 100 | 128 | 200 rows, token by token against chunks, us: delta rule, 8 heads of 64 x 128 14 | 18 | 22 | 33 against 19 | 21 | 19 | 24; 32 of 128 x 128
+// 20 | 26 | 34 | 50 against 22 | 24 | 23 | 32.
 constexpr int STATE_CHUNKS_FROM = 128;
-constexpr float STATE_MOST = 1099511627776.f;     // 2^40: sums of products of such numbers stay finite
-struct StateChunks { const int* flags; int places; };
-__device__ __forceinline__ bool state_by_chunks(int n, const int* flags, int chunks) {
-  if (n < STATE_CHUNKS_FROM) return false;
-  int bad = 0;
-  for (int i = threadIdx.x; i < chunks; i += blockDim.x) bad |= flags[i];
-  return !__syncthreads_or(bad);
-}
+struct StateArgs;
+struct StateChunks;
 size_t state_chunks_workspace(int64_t T, int64_t B, int H, int dk, int dv);
-int launch_state_chunks(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int B, int64_t T, int H, int G, int dk, int dv, bool delta,
-                        void* ws, hipStream_t s, StateChunks* made);
+int launch_state_chunks(const StateArgs& a, int64_t T, bool delta, void* ws, hipStream_t s, StateChunks* left);
 
 }  // namespace gbxm

@@ -3,7 +3,7 @@
 //   recurrent_prep_kernel   short causal convolution + silu on q | k | v, unit q / k heads (a wave per head), q scale, the decay
 //                           exp(-rate_h softplus(sign (a + bias))) and beta = sigmoid(b), all in fp32, into one fp32 row.
 //   conv_tail_kernel        the last taps-1 convolution inputs of every sequence into its slot.
-//   state_scan_kernel<R>    the scan token by token (longer portions go by chunks: mixers_state_mfma.hip).  The columns of a head's state (one per value channel) never meet: a wave takes four columns, 16
+//   state_scan_kernel<R>    the scan token by token (mixers_state_scan.h; steps with longer portions: mixers_state_mfma.hip).  The columns of a head's state (one per value channel) never meet: a wave takes four columns, 16
 //                           lanes per column, a lane holds R key channels of its column in registers; per token the two dot products
 //                           over key channels are R multiply-adds and four cross-lane adds inside a 16-lane row (all 16 lanes end
 //                           with the same bits).  Operands come through LDS in chunks of tokens, the next chunk fetched while the
@@ -11,6 +11,7 @@
 //                           in the step, nor on how many columns a workgroup takes.
 //   head_norm_gate_kernel   per-head RMS norm of the read-out, weight and gate, one wave per (row, head).
 #include "mixers_mfma.h"
+#include "mixers_state_scan.h"
 
 namespace gbxm {
 namespace {
@@ -219,160 +220,12 @@ __global__ __launch_bounds__(NT) void conv_tail_kernel(const T* __restrict__ y, 
   }
 }
 
-// NW waves per workgroup = 4 NW columns of one (sequence, head).  The operands of CH tokens (q | k | decay padded to 16 R channels, the
-// workgroup's value columns; the betas beside them) are staged in LDS, shared by the waves, two buffers: the next chunk is fetched into registers
-// before the current one is computed and parked in the other buffer afterwards, one barrier per chunk.  Lane ks of a 16-lane row owns the key
-// channels 4 ks .. 4 ks + 3, and those 64, 128, ... further on (R a multiple of 4; heads of up to 16, 32 or 96 channels: 1, 2 or 2 neighbours): LDS reads,
-// and the state's loads and stores, are 16-byte accesses that are contiguous over the row.  Bound by issue slots (a long prompt leaves one or two waves a SIMD, each token costs a wave 4 R multiply-adds and what
-// feeds them), so operands are read four at a time: V = 4 floats per staging access where sizes, strides and addresses allow, else 1.
-// (4-byte accesses and operands read where they are used -> now, us: rows of 1501 + 700 + 65 tokens, 8 heads of 128 x 256 393 -> 253, delta rule over 32
-// of 128 x 128 507 -> 351; 32 prompts of 8 to 163 tokens 273 -> 144; one token of 32 sequences, 67 MB of state 30.1 -> 15.1.)
-// Heads of few channels have forms of their own, which stage and multiply no more than there is (16 heads, 32 prompts of 40 tokens, every lane four
-// channels | this: 16 x 64 25.3 | 15.6, 32 x 128 45.3 | 29.5, 16 x 50 element by element 44.4 | 17.7); 48 channels are the four-channel form's (R = 3 at
-// one channel a lane 51.6, 28.4 here), 66 to 96 only where sizes are not in groups of four (94 x 64 59.4 | 43.1; 96 x 96 in groups of four 50).
 template <int R, bool DELTA, int NW, int V>
-__global__ __launch_bounds__(64 * NW) void state_scan_kernel(const float* __restrict__ r, int64_t r_stride, float* __restrict__ state,
-                                                            float* __restrict__ out, const int* __restrict__ seq, int H, int G, int dk, int dv, StateChunks made) {
-  constexpr int C = R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;                 // neighbouring channels of a lane
-  constexpr int DKP = 16 * R, NCOL = 4 * NW, ROW = 3 * DKP + NCOL, NTH = 64 * NW, Q = R / C;
-  constexpr int CH = NW == 1 ? (R <= 4 ? 4 : 2) : (R <= 4 ? 32 : (R <= 8 ? 16 : 8)) * NW / 4;     // one-wave workgroups serve steps of few rows
-  constexpr int SLOTS = CH * ROW / V, PF = (SLOTS + NTH - 1) / NTH;
-  __shared__ __attribute__((aligned(16))) float buf[2][CH * ROW];
-  __shared__ float betas[2][CH];
-  const int b = blockIdx.z, h = blockIdx.y;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ks = lane & 15;
-  const int col0 = blockIdx.x * NCOL, lcol = wave * 4 + (lane >> 4), col = col0 + lcol;
-  const int slot = seq[4 * b], pos0 = seq[4 * b + 1], n = seq[4 * b + 2], row0 = seq[4 * b + 3];
-  if (made.flags && state_by_chunks(n, made.flags + static_cast<int64_t>(h) * made.places + row0 / 16 + b, (n + 15) / 16)) return;
-  const bool col_ok = col < dv;
-  const int colc = col_ok ? col : dv - 1;
-  const int nq = G * dk, nv = H * dv;
-  const int g = h / (H / G);
-  float* sp = state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;     // (channels past the last one hold zeros)
-  // every load below is issued unconditionally from an address inside the buffers (what it must not deliver is replaced afterwards):
-  // loads under a branch wait for one another, and a chunk's fetch then costs the sum of their latencies
-  float S[R];
-#pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const int c = C * ks + 16 * C * i;
-    if constexpr (V == 4 && C == 4) {
-      Lanes<float, 4>::load(sp + min(c, dk - 4), S + 4 * i);
-    } else {
-#pragma unroll
-      for (int j = 0; j < C; ++j) S[C * i + j] = sp[min(c + j, dk - 1)];
-    }
-#pragma unroll
-    for (int j = 0; j < C; ++j) S[C * i + j] = (pos0 > 0 && c + j < dk) ? S[C * i + j] : 0.f;
-  }
-  const float* base = r + static_cast<int64_t>(row0) * r_stride;
-  const int oq = g * dk, ok = nq + g * dk, ov = 2 * nq + h * dv, og = 2 * nq + nv + h * dk, ob = 2 * nq + nv + H * dk + h;
-  float pf[PF][V], pb = 0.f;
-  int offs[PF], tts[PF];                    // where slot i of this thread's share of a chunk comes from: token of the chunk, offset in its row
-  unsigned loaded = 0, decays = 0;          // bit i: pf[i] is an operand (else the slot's neutral value: 1 for a decay, 0 elsewhere)
-  static_assert(PF <= 32, "a bit per slot");
-#pragma unroll
-  for (int i = 0; i < PF; ++i) {
-    const int idx = min(static_cast<int>(threadIdx.x) + i * NTH, SLOTS - 1);
-    const int tt = idx / (ROW / V), j = (idx - tt * (ROW / V)) * V;
-    const int seg = j < DKP ? 0 : (j < 2 * DKP ? 1 : (j < 3 * DKP ? 2 : 3));
-    const int jj = j - seg * DKP;                                     // segment 3: the value columns
-    const int first = seg == 0 ? oq : (seg == 1 ? ok : (seg == 2 ? og : ov + col0));
-    const bool valid = jj < (seg < 3 ? dk : min(dv - col0, NCOL));
-    offs[i] = valid ? first + jj : oq;
-    tts[i] = tt;
-    loaded |= static_cast<unsigned>(valid) << i;
-    decays |= static_cast<unsigned>(seg == 2) << i;
-  }
-  auto fetch = [&](int t0) {
-    const float* cb = base + static_cast<int64_t>(t0) * r_stride;
-    const int last = min(CH, n - t0) - 1;   // the sequence's last chunk: rows past its end are read as its last row (and never used)
-#pragma unroll
-    for (int i = 0; i < PF; ++i) Lanes<float, V>::load(cb + static_cast<int64_t>(min(tts[i], last)) * r_stride + offs[i], pf[i]);
-    if (DELTA) pb = cb[static_cast<int64_t>(min(static_cast<int>(threadIdx.x), last)) * r_stride + ob];
-  };
-  auto park = [&](int which) {
-#pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      const int idx = threadIdx.x + i * NTH;
-      const float neutral = (decays >> i) & 1u ? 1.f : 0.f;
-#pragma unroll
-      for (int j = 0; j < V; ++j) pf[i][j] = ((loaded >> i) & 1u) ? pf[i][j] : neutral;
-      if (idx < SLOTS) Lanes<float, V>::store(buf[which] + idx * V, pf[i]);
-    }
-    if (DELTA && static_cast<int>(threadIdx.x) < CH) betas[which][threadIdx.x] = pb;
-  };
-  fetch(0);
-  park(0);
-  __syncthreads();
-  float* op = out + static_cast<int64_t>(row0) * nv + h * dv + colc;
-  int which = 0;
-  for (int t0 = 0; t0 < n; t0 += CH, which ^= 1) {
-    const bool more = t0 + CH < n;
-    if (more) fetch(t0 + CH);
-    const float* cur = buf[which];
-    const int cn = min(CH, n - t0);
-    struct Token { float q[R], k[R], d[R], v, beta; };
-    auto read = [&](int tt, Token& x) {
-      const float* at = cur + tt * ROW + C * ks;
-#pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        Lanes<float, C>::load(at + 16 * C * i, x.q + C * i);
-        Lanes<float, C>::load(at + DKP + 16 * C * i, x.k + C * i);
-        Lanes<float, C>::load(at + 2 * DKP + 16 * C * i, x.d + C * i);
-      }
-      x.v = cur[tt * ROW + 3 * DKP + lcol];
-      if (DELTA) x.beta = betas[which][tt];
-    };
-    auto step = [&](int tt, const Token& x) {
-#pragma unroll
-      for (int i = 0; i < R; ++i) S[i] *= x.d[i];
-      float u = x.v;
-      if constexpr (DELTA) {
-        float dot[2] = {0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < R; ++i) dot[i & 1] += x.k[i] * S[i];
-        u = x.beta * (u - row16_sum(dot[0] + dot[1]));
-      }
-      float o[2] = {0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < R; ++i) { S[i] += x.k[i] * u; o[i & 1] += x.q[i] * S[i]; }
-      const float sum = row16_sum(o[0] + o[1]);
-      if (ks == 0 && col_ok) op[static_cast<int64_t>(t0 + tt) * nv] = sum;
-    };
-    Token x;
-    if constexpr (NW > 1) {                  // a token's operands are read while the one before it is computed
-      Token y;
-      read(0, x);
-      int tt = 0;
-      for (; tt + 1 < cn; tt += 2) {
-        read(tt + 1, y);
-        step(tt, x);
-        read(min(tt + 2, cn - 1), x);
-        step(tt + 1, y);
-      }
-      if (tt < cn) step(tt, x);
-    } else {                                 // few tokens, many sequences: the registers serve occupancy
-      for (int tt = 0; tt < cn; ++tt) {
-        read(tt, x);
-        step(tt, x);
-      }
-    }
-    if (more) park(which ^ 1);
-    __syncthreads();
-  }
-  if (col_ok) {
-#pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const int c = C * ks + 16 * C * i;
-      if constexpr (V == 4 && C == 4) {
-        if (c < dk) Lanes<float, 4>::store(sp + c, S + 4 * i);
-      } else {
-#pragma unroll
-        for (int j = 0; j < C; ++j)
-          if (c + j < dk) sp[c + j] = S[C * i + j];
-      }
-    }
-  }
+__global__ __launch_bounds__(64 * NW) void state_scan_kernel(const StateArgs a, const StateChunks made) {
+  __shared__ __attribute__((aligned(16))) float lds[ScanShape<R, NW, scan_tokens(R, NW)>::FLOATS];
+  const int b = blockIdx.z;
+  if (made.flags && state_by_chunks(made, b, blockIdx.y, a.seq[4 * b + 2], a.seq[4 * b + 3])) return;
+  scan_columns<R, DELTA, NW, V>(a, b, blockIdx.y, blockIdx.x * 4 * NW, lds);
 }
 
 template <typename T, bool FAST>
@@ -484,19 +337,18 @@ void launch_head_norm_gate(const float* o, const void* gate, int64_t gate_stride
 }
 
 template <bool DELTA, int NW>
-int launch_scan(int R, int B, hipStream_t s, const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int H, int G, int dk,
-                int dv, StateChunks made) {
-  const dim3 grid((dv + 4 * NW - 1) / (4 * NW), H, B);
-  const bool vec = dk % 4 == 0 && dv % 4 == 0 && r_stride % 4 == 0 && all_aligned(16, r, state);
-#define GBXM_SCAN(N)                                                                                                    \
-  do {                                                                                                                  \
-    if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);   \
-    else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);       \
+int launch_scan(const StateArgs& a, const StateChunks& made, bool vec, hipStream_t s) {
+  const int R = (a.dk + 15) / 16;
+  const dim3 grid((a.dv + 4 * NW - 1) / (4 * NW), a.H, a.B);
+#define GBXM_SCAN(N)                                                        \
+  do {                                                                      \
+    if (vec) state_scan_kernel<N, DELTA, NW, 4><<<grid, 64 * NW, 0, s>>>(a, made); \
+    else state_scan_kernel<N, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(a, made);     \
   } while (0)
   if (R <= 1) GBXM_SCAN(1);
   else if (R <= 2) GBXM_SCAN(2);
   else if (R <= 4) GBXM_SCAN(4);
-  else if (R <= 6 && !vec) state_scan_kernel<6, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(r, r_stride, state, out, seq, H, G, dk, dv, made);
+  else if (R <= 6 && !vec) state_scan_kernel<6, DELTA, NW, 1><<<grid, 64 * NW, 0, s>>>(a, made);
   else if (R <= 8) GBXM_SCAN(8);
   else if (R <= 12) GBXM_SCAN(12);
   else GBXM_SCAN(16);
@@ -574,20 +426,18 @@ int gbxm_state_scan_ws(const float* r, int64_t r_stride, float* state, float* ou
   if (B == 0) return GBXM_OK;
   if (B > 65535 || H > 65535) return fail(GBXM_ERR_UNSUPPORTED, "state_scan: grid");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int R = (dk + 15) / 16;
+  const StateArgs a{r, r_stride, state, out, seq, B, H, G, dk, dv};
+  const bool vec = dk % 4 == 0 && dv % 4 == 0 && r_stride % 4 == 0 && all_aligned(16, r, state);
+  const size_t need = ws && vec ? state_chunks_workspace(T_, B, H, dk, dv) : 0;
   StateChunks made{nullptr, 0};
-  const size_t need = ws ? state_chunks_workspace(T_, B, H, dk, dv) : 0;
-  if (need && ws_bytes >= need && r_stride % 4 == 0 && r_stride <= (1 << 22) && all_aligned(16, r, static_cast<const float*>(ws), state)) {
-    const int rc = launch_state_chunks(r, r_stride, state, out, seq, B, T_, H, G, dk, dv, delta, ws, s, &made);
-    if (rc != GBXM_OK) return rc;
+  if (need && ws_bytes >= need && r_stride <= (1 << 22) && all_aligned(16, static_cast<const char*>(ws))) {
+    const int rc = launch_state_chunks(a, T_, delta, ws, s, &made);
+    if (rc != GBXM_OK || !made.flags) return rc;
   }
   // long rows (prompts): 16 columns per workgroup share the staged operands; a few rows per sequence: 4 columns, four times the
   // workgroups for the state's traffic.  A column's arithmetic is the same in both.
-  if (T_ >= 8 * static_cast<int64_t>(B))
-    return delta ? launch_scan<true, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made)
-                 : launch_scan<false, 4>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made);
-  return delta ? launch_scan<true, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made)
-               : launch_scan<false, 1>(R, B, s, r, r_stride, state, out, seq, H, G, dk, dv, made);
+  if (T_ >= 8 * static_cast<int64_t>(B)) return delta ? launch_scan<true, 4>(a, made, vec, s) : launch_scan<false, 4>(a, made, vec, s);
+  return delta ? launch_scan<true, 1>(a, made, vec, s) : launch_scan<false, 1>(a, made, vec, s);
 }
 
 int gbxm_head_norm_gate(const float* o, const void* gate, int64_t gate_stride, const float* w, void* out, int64_t out_row, int64_t T_, int32_t H, int32_t dv,

@@ -14,18 +14,23 @@
 //
 // Token by token a wave of four columns spends 8 instructions a channel and waits for two sums over lanes a token (590 cycles a token and more).  A chunk here is
 // 2 600 cycles, of which the matrix cores are busy 930: it is a chain of waits (LDS, two barriers, dependent products), not bound by a unit.  Tried: carrying and
-// multiplying in the same four waves (3 080 cycles), loads four chunks ahead (no change), pairs of channels a lane (8 % slower).  Measured, all kernels of a call,
-// token by token | chunks, us: 1 501 + 700 + 65 rows, delta rule, 32 heads of 128 x 128 332 | 194, 8 of 128 x 256 without it 242 | 110; 6 000 rows of the former 1 297 | 544;
-// 32 sequences of 8 .. 163 rows, delta rule, 32 of 128 x 128 302 | 292, 16 without it 142 | 132.  Error against 64 bits, relative, 1e-8, over rows that models prepare:
+// multiplying in the same four waves (3 080 cycles), loads four chunks ahead (no change), pairs of channels a lane (8 % slower).  Shorter sequences of the step go token by
+// token in the same launch (TOGETHER), in chunks of few tokens, which keep the kernel's registers at two workgroups a CU (16 tokens: 8 registers spilled).
+// Measured, all kernels of a call, token by token | chunks, us: 1 501 + 700 + 65 rows, delta rule, 32 heads of 128 x 128 325 | 182, 8 of 128 x 256 without it 243 | 99;
+// 130 + 100 + 64 + 17 + 8 rows, delta rule, 32 heads 52 | 54, 16 heads 40 | 39; 32 sequences of 8 .. 163 rows 305 | 300 and 176 | 178, 8 heads of 128 x 256 without it 141 | 134;
+// one sequence of 128 | 200 rows, 32 heads 34 | 23 and 50 | 32.  The first kernel's 6 us are lost where a sequence that just goes by chunks meets one that just does not: 127 + 128
+// rows, 16 heads 34 | 42.  Error against 64 bits, relative, 1e-8, over rows that models prepare:
 // delta rule 19.4 | 16.2, without it 42.8 | 38.0 (decays 0.92 .. 0.9998 a token and channel), 8.1 | 7.7 (one decay a head).
 #include <type_traits>
 #include "mixers_mfma.h"
+#include "mixers_state_scan.h"
 
 namespace gbxm {
 namespace {
 
-constexpr int CT = 16;                       // tokens of a chunk
+constexpr int CT = STATE_CHUNK;
 constexpr int PAIR = 2 * CT * CT;            // numbers per (chunk, head): M, B
+constexpr float STATE_MOST = 1099511627776.f;     // 2^40: sums of products of such numbers stay finite
 
 __device__ __forceinline__ f32x4v mfma_f32(float a, float b, const f32x4v& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -38,8 +43,6 @@ __device__ __forceinline__ f32x4v load4(__amdgpu_buffer_rsrc_t r, int at) { retu
 __device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, int at, float x) { __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, at, 0, 0); }
 __device__ __forceinline__ constexpr unsigned bits(float x) { return __builtin_bit_cast(unsigned, x) & 0x7FFFFFFFu; }
 constexpr int PAST = 0x7FFFFFF0;             // an offset beyond every buffer
-// Places of the chunks: sequence b's first one is row0 / 16 + b, which leaves room for its part of a chunk
-__device__ __forceinline__ int first_chunk(int row0, int b) { return row0 / CT + b; }
 
 // grid (chunk places, heads): wave w takes the tokens j = 4 w .. 4 w + 3, a 16-lane row each; lane ks of it the channels 4 ks .. 4 ks + 3 and those 64 further on.
 template <int TPW, bool DELTA>
@@ -135,7 +138,9 @@ __global__ __launch_bounds__(256) void state_pairs_kernel(const float* __restric
 template <int TPW, bool DELTA> struct ChunkLds {
   static constexpr int CP = 64 * TPW, LD = CP + 4, LT = CT + 4;
   static constexpr int Q = 0, K = Q + CT * LD, KT = K + (DELTA ? CT * LD : 0), P = KT + CP * LT, SIZE = P + CP;
-  static constexpr int OUT = 2 * SIZE, RED = OUT + 2 * 4 * 256, BYTES = (RED + (DELTA ? 4 * 256 : 0)) * 4;   // the waves' parts of O (twice) and of (K P) S
+  static constexpr int OUT = 2 * SIZE, RED = OUT + 2 * 4 * 256, END = RED + (DELTA ? 4 * 256 : 0);   // the waves' parts of O (twice) and of (K P) S
+  static constexpr int TOKENS = TPW == 1 ? 16 : 8;                      // of a chunk of the sequences that go token by token: few, so that registers and LDS stay the chunks'
+  static constexpr int SCAN = ScanShape<4 * TPW, 4, TOKENS>::FLOATS, BYTES = (END > SCAN ? END : SCAN) * 4;
 };
 
 // Loads that fly across a barrier: only LDS has to be settled
@@ -146,23 +151,27 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 template <int TPW, bool DELTA>
-__global__ __launch_bounds__(512) void state_chunk_kernel(const float* __restrict__ r, int64_t r_stride, float* __restrict__ state, float* __restrict__ out,
-                                                         const int* __restrict__ seq, const float* __restrict__ pairs, const int* __restrict__ flags, int places,
-                                                         int B_, int H, int G, int dk, int dv) {
+__global__ __launch_bounds__(512, (TPW <= 2 ? 4 : 2)) void state_chunk_kernel(const StateArgs a, const float* __restrict__ pairs, const StateChunks made, int together) {
   typedef ChunkLds<TPW, DELTA> L;
   constexpr int CP = L::CP, LD = L::LD, LT = L::LT, CI = (CP + 127) / 128;
   extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int64_t r_stride = a.r_stride;
+  const int H = a.H, G = a.G, dk = a.dk, dv = a.dv;
+  const int* seq = a.seq;
   // the column blocks of one (sequence, head) read the same operands: neighbours on one XCD
   const int cols = (dv + 15) / 16, unit = blockIdx.x >> 3, which = unit / cols * 8 + (blockIdx.x & 7);
-  if (which >= B_ * H) return;
+  if (which >= a.B * H) return;
   const int b = which / H, h = which % H;
   const int slot = seq[4 * b], pos0 = seq[4 * b + 1], n = seq[4 * b + 2], row0 = seq[4 * b + 3];
   const int tid = threadIdx.x, lane = tid & 63, part = __builtin_amdgcn_readfirstlane(tid >> 6), wave = part & 3, fr = lane & 15, g4 = 4 * (lane >> 4);
   const int place0 = first_chunk(row0, b), chunks = (n + CT - 1) / CT;
-  if (!state_by_chunks(n, flags + static_cast<int64_t>(h) * places + place0, chunks)) return;
+  if (!state_by_chunks(made, b, h, n, row0)) {                          // token by token: half of the waves
+    if (together && tid < 256) scan_columns<4 * TPW, DELTA, 4, 4, L::TOKENS>(a, b, h, unit % cols * 16, lds);
+    return;
+  }
   const int col = unit % cols * 16 + fr, colc = min(col, dv - 1);
   const int g = h / (H / G), nq = G * dk, nv = H * dv;
-  const float* base = r + static_cast<int64_t>(row0) * r_stride;
+  const float* base = a.r + static_cast<int64_t>(row0) * r_stride;
   // a wave takes 32 channels (of every 128), its halves eight tokens each; what the other half's decays multiply to comes across the wave
   const int late = lane >> 5, ch = 32 * wave + (lane & 31), rs = static_cast<int>(r_stride) * 4;
   const float *bq = base + g * dk, *bk = bq + nq, *bd = base + 2 * nq + nv + h * dk, *bv = base + 2 * nq + h * dv;
@@ -231,7 +240,7 @@ __global__ __launch_bounds__(512) void state_chunk_kernel(const float* __restric
     const int ocol = unit % cols * 16 + (tid >> 2 & 15), ato = ocol < dv ? ((4 * wave + (tid & 3)) * nv + ocol) * 4 : PAST;
     auto put = [&](int c) {
       const float* o = lds + L::OUT + (c & 1) * (4 * 256) + (tid & 255);
-      store1(rows_of(out + static_cast<int64_t>(row0 + c * CT) * nv + h * dv, tokens(c) * nv * 4), ato, (o[0] + o[256]) + (o[512] + o[768]));
+      store1(rows_of(a.out + static_cast<int64_t>(row0 + c * CT) * nv + h * dv, tokens(c) * nv * 4), ato, (o[0] + o[256]) + (o[512] + o[768]));
     };
     auto carry = [&](int c, Raw& f) {                                   // `f` holds chunk c + 1, whose buffer nobody reads since the last barrier
       if (c > 0) put(c - 1);
@@ -253,7 +262,7 @@ __global__ __launch_bounds__(512) void state_chunk_kernel(const float* __restric
     return;
   }
   // and four multiply
-  float* sp = state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;
+  float* sp = a.state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;
   f32x4v S[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
@@ -341,10 +350,15 @@ __global__ __launch_bounds__(512) void state_chunk_kernel(const float* __restric
 
 int64_t chunk_places(int64_t T, int64_t B) { return T / CT + B; }
 size_t flag_bytes(int64_t places, int H) { return (static_cast<size_t>(places) * H * sizeof(int) + 15) & ~static_cast<size_t>(15); }
+int64_t chunk_units(const StateArgs& a) { return (static_cast<int64_t>(a.B) * a.H + 7) / 8 * 8 * ((a.dv + 15) / 16); }
+// Column blocks of a step up to which the chunks' launch also takes what goes token by token: the two need not wait for one another, but such a workgroup works
+// with half of its waves, two a CU.  Above, the chip is full many times over either way, and the token kernel's own launch has three workgroups a CU.  One launch |
+// two, us: delta rule, heads of 128 x 128, 16 heads 130 + 100 + 64 + 17 + 8 rows 39 | 57, 16 sequences (2 048 blocks) 99 | 99, 24 136 | 132, 32 heads, 16 sequences 171 | 161,
+// 32 328 | 299; without it, 32 sequences (4 096 blocks) of 16 heads 135 | 143, of 8 heads of 128 x 256 134 | 135.
+constexpr int64_t TOGETHER_DELTA = 2048, TOGETHER = 4096;
 
 template <int TPW, bool DELTA>
-int launch(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int B, int places, int H, int G, int dk, int dv, int* flags,
-           float* pairs, hipStream_t s) {
+int launch(const StateArgs& a, const StateChunks& made, int* flags, float* pairs, bool together, hipStream_t s) {
   constexpr int BYTES = ChunkLds<TPW, DELTA>::BYTES;
   static OncePerDevice once;
   if (once.pending()) {
@@ -352,9 +366,8 @@ int launch(const float* r, int64_t r_stride, float* state, float* out, const int
     if (e != hipSuccess) return hip_fail(e, "state_scan");
     once.done();
   }
-  state_pairs_kernel<TPW, DELTA><<<dim3(places, H), 256, 0, s>>>(r, r_stride, pairs, flags, seq, B, H, G, dk, dv);
-  const int64_t units = (static_cast<int64_t>(B) * H + 7) / 8 * 8 * ((dv + 15) / 16);
-  state_chunk_kernel<TPW, DELTA><<<static_cast<unsigned>(units), 512, BYTES, s>>>(r, r_stride, state, out, seq, pairs, flags, places, B, H, G, dk, dv);
+  state_pairs_kernel<TPW, DELTA><<<dim3(made.places, a.H), 256, 0, s>>>(a.r, a.r_stride, pairs, flags, a.seq, a.B, a.H, a.G, a.dk, a.dv);
+  state_chunk_kernel<TPW, DELTA><<<static_cast<unsigned>(chunk_units(a)), 512, BYTES, s>>>(a, pairs, made, together);
   return after_launch("state_scan (chunks)");
 }
 
@@ -362,19 +375,18 @@ int launch(const float* r, int64_t r_stride, float* state, float* out, const int
 
 size_t state_chunks_workspace(int64_t T, int64_t B, int H, int dk, int dv) {
   const int64_t places = chunk_places(T, B);
-  if (dk % 4 || dk < 64 || dk > 256 || dv < 16 || H * dv % 4 || H > 65535 || B < 1 || places > (1 << 24) || B * H * ((dv + 15) / 16) > (1 << 26)) return 0;
+  if (dk % 4 || dk < 64 || dk > 256 || dv < 16 || dv % 4 || H > 65535 || B < 1 || places > (1 << 24) || B * H * ((dv + 15) / 16) > (1 << 26)) return 0;
   return flag_bytes(places, H) + static_cast<size_t>(places) * H * PAIR * sizeof(float);
 }
 
-int launch_state_chunks(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int B, int64_t T, int H, int G, int dk, int dv, bool delta,
-                        void* ws, hipStream_t s, StateChunks* made) {
-  const int places = static_cast<int>(chunk_places(T, B));
+int launch_state_chunks(const StateArgs& a, int64_t T, bool delta, void* ws, hipStream_t s, StateChunks* left) {
   int* flags = static_cast<int*>(ws);
-  float* pairs = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + flag_bytes(places, H));
-  *made = StateChunks{flags, places};
-#define GBXM_CHUNKS(N)                                                                                                                                            \
-  (delta ? launch<N, true>(r, r_stride, state, out, seq, B, places, H, G, dk, dv, flags, pairs, s) : launch<N, false>(r, r_stride, state, out, seq, B, places, H, G, dk, dv, flags, pairs, s))
-  switch ((dk + 63) / 64) {
+  const StateChunks made{flags, static_cast<int>(chunk_places(T, a.B))};
+  float* pairs = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + flag_bytes(made.places, a.H));
+  const bool together = chunk_units(a) <= (delta ? TOGETHER_DELTA : TOGETHER);
+  *left = together ? StateChunks{nullptr, 0} : made;
+#define GBXM_CHUNKS(N) (delta ? launch<N, true>(a, made, flags, pairs, together, s) : launch<N, false>(a, made, flags, pairs, together, s))
+  switch ((a.dk + 63) / 64) {
     case 1: return GBXM_CHUNKS(1);
     case 2: return GBXM_CHUNKS(2);
     case 3: return GBXM_CHUNKS(3);

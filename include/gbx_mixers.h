@@ -264,7 +264,8 @@ int gbxm_conv_tail_update(const void* y, int64_t y_stride, void* tail, const int
 int gbxm_state_scan(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T, int32_t H, int32_t G,
                     int32_t dk, int32_t dv, int32_t delta, void* stream);
 /* The same with a workspace of gbxm_state_scan_workspace bytes (16-byte aligned; longest: rows of the step's longest sequence; 0: not a step for it): sequences of
- * 128 rows and more then run in chunks of 16 rows on the matrix cores (fp32 products and sums in another order).  `seq` lists the sequences in the order of their
+ * 128 rows and more then run in chunks of 16 rows on the matrix cores (fp32 products and sums in another order) where dk (64 .. 256), dv and the rows' stride
+ * are multiples of 4 and rows and states 16-byte aligned.  `seq` lists the sequences in the order of their
  * rows.  No or too small a workspace: as gbxm_state_scan. */
 size_t gbxm_state_scan_workspace(int32_t B, int64_t T, int64_t longest, int32_t H, int32_t dk, int32_t dv);
 int gbxm_state_scan_ws(const float* r, int64_t r_stride, float* state, float* out, const int32_t* seq, int32_t B, int64_t T, int32_t H, int32_t G,

@@ -1,5 +1,5 @@
 """Prompt portions of the decayed states by chunks of 16 tokens (csrc/mixers_state_mfma.hip): sequences on either side of the fewest rows that go that way, whole chunks
-and remainders, key channels in and off the 64s, value channels off the 16s, rows that are not in groups of four (three heads: token by token), fresh and carried states, decays down to zero, and numbers that the chunks leave to the
+and remainders, key channels in and off the 64s, value channels off the 16s, rows or value channels that are not in groups of four (token by token), fresh and carried states, decays down to zero, and numbers that the chunks leave to the
 token-by-token form (infinities, NaN, decays above one, numbers whose products might not stay finite).  Reference: float64 token by token; tolerance: fp32 sums
 over the key channels, the chunk's tokens and the tokens that a decay keeps, relative to the sums of absolute values."""
 import pytest
@@ -79,3 +79,27 @@ def test_left_to_the_tokens(what, delta):
         if what in ("growing decay",):
             assert float((out - want).abs().max()) < 200 * 2.0 ** -24 * 4 * room
         assert float((out[:37] - want[:37]).abs().max()) < 200 * 2.0 ** -24 * 4 * 100
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("dk,dv,H,short,long", [(128, 36, 4, [127, 1, 64], [130]), (64, 16, 16, [3] * 299, [128]), (192, 16, 4, [40, 9], [128, 200]), (256, 32, 4, [33], [144])])
+def test_the_others_of_the_step(dk, dv, H, short, long, delta):
+    """Short sequences give the same bits beside long ones as without them: in the chunks' launch (few column blocks) and in one of their own."""
+    g = torch.Generator().manual_seed(dk + dv)
+    lay = RM.RecurrentLayout(H, H, dk, dv, 0, H * dk, 2 * H * dk, 2 * H * dk + H * dv if delta else -1)
+    counts = short[:1] + long + short[1:]
+    rows = [torch.rand((n, 3 * H * dk + H * dv + (H if delta else 0)), generator=g) * 0.9 / dk ** 0.25 for n in counts]
+    start = torch.randn((len(counts), H, dv, dk), generator=g)
+
+    def scan(which):
+        cache = SlotStateCache(H, dk, dv, 0, 0, SequenceSlots(len(counts)))
+        cache.reserve(torch.float32, DEV)
+        cache.state.copy_(start)
+        batch = StepBatch.build(which, [0 if i % 2 else 5 for i in which], [counts[i] for i in which], DEV)
+        out = RM.decayed_state_scan(torch.cat([rows[i] for i in which]).to(DEV), lay, cache, batch, delta)
+        return dict(zip(which, out.split([counts[i] for i in which]))), cache.state
+
+    few = [i for i, n in enumerate(counts) if n < 128]
+    (whole, state), (alone, kept) = scan(list(range(len(counts)))), scan(few)
+    for i in few:
+        assert torch.equal(whole[i], alone[i]) and torch.equal(state[i], kept[i])
