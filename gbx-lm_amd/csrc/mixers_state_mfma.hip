@@ -1,4 +1,4 @@
-// The decayed matrix states of mixers_state.hip for prompt portions: 16 tokens at a time on the matrix cores, in fp32 throughout.
+// The decayed matrix states of mixers_state.hip for prompt portions: 16 tokens at a time on the matrix cores, in fp32 (products of decays in fp64).
 //
 // With P_i = d_1 .. d_i the decays of a chunk up to token i (per key channel) and S the state before it,
 //   A[i][j] = sum_c k_i k_j d_{j+1} .. d_i  (j < i),   B[i][j] = sum_c q_i k_j d_{j+1} .. d_i  (j <= i),   M = (1 + diag(beta) A)^-1 diag(beta)
@@ -30,7 +30,8 @@ namespace {
 
 constexpr int CT = STATE_CHUNK;
 constexpr int PAIR = 2 * CT * CT;            // numbers per (chunk, head): M, B
-constexpr float STATE_MOST = 1099511627776.f;     // 2^40: sums of products of such numbers stay finite
+// 2^40: what the first kernel lets pass; it only looks at its own operands, and a chain whose sums leave the range all the same is seen at its end
+constexpr float STATE_MOST = 1099511627776.f;
 
 __device__ __forceinline__ f32x4v mfma_f32(float a, float b, const f32x4v& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -235,12 +236,19 @@ __global__ __launch_bounds__(512, (TPW <= 2 ? 4 : 2)) void state_chunk_kernel(co
       to[L::P + cc] = static_cast<float>(whole * other);                                    // (both halves write the same bits)
     }
   };
+  float* sp = a.state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;
+  f32x4v S[TPW];
+  bool wild = false;                                                    // an infinity or NaN came up ...
+  __shared__ int any_wild;                                              // ... in some thread
+  if (tid == 0) any_wild = 0;
   if (part >= 4) {                                                      // four waves carry: operands in, read-outs out
     // O of a chunk is summed and written during the next one, a number per thread
     const int ocol = unit % cols * 16 + (tid >> 2 & 15), ato = ocol < dv ? ((4 * wave + (tid & 3)) * nv + ocol) * 4 : PAST;
     auto put = [&](int c) {
       const float* o = lds + L::OUT + (c & 1) * (4 * 256) + (tid & 255);
-      store1(rows_of(a.out + static_cast<int64_t>(row0 + c * CT) * nv + h * dv, tokens(c) * nv * 4), ato, (o[0] + o[256]) + (o[512] + o[768]));
+      const float x = (o[0] + o[256]) + (o[512] + o[768]);
+      wild |= !(fabsf(x) < INFINITY);
+      store1(rows_of(a.out + static_cast<int64_t>(row0 + c * CT) * nv + h * dv, tokens(c) * nv * 4), ato, x);
     };
     auto carry = [&](int c, Raw& f) {                                   // `f` holds chunk c + 1, whose buffer nobody reads since the last barrier
       if (c > 0) put(c - 1);
@@ -259,88 +267,99 @@ __global__ __launch_bounds__(512, (TPW <= 2 ? 4 : 2)) void state_chunk_kernel(co
       carry(c + 1, even);
     }
     put((chunks - 1) | 1);
-    return;
-  }
-  // and four multiply
-  float* sp = a.state + ((static_cast<int64_t>(slot) * H + h) * dv + colc) * dk;
-  f32x4v S[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int c = 16 * (wave * TPW + t) + g4;
-    const f32x4v v = *reinterpret_cast<const f32x4v*>(sp + min(c, dk - 4));
-    S[t] = pos0 > 0 && c < dk ? v : f32x4v{0};
-  }
-  // M and B of a chunk by lanes as left operands (row lane % 16, contraction index 4 (lane / 16) + i), V as the accumulators lie
-  struct Small { f32x4v m, v; float b; } now, then;
-  const float* pairs0 = pairs + (static_cast<int64_t>(place0) * H + h) * PAIR;
-  const int atm = (fr * CT + g4) * 4;
-  int atv[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    atv[i] = (g4 + i) * rs + colc * 4;
-  }
-  auto fetch_small = [&](int c, Small& s) {
-    const __amdgpu_buffer_rsrc_t rp = rows_of(pairs0 + static_cast<int64_t>(c) * H * PAIR, PAIR * 4);
-    if constexpr (DELTA) s.m = load4(rp, atm);
-    s.b = load1(rp, atm + CT * CT * 4 + wave * 4);                      // B U is shared out by steps of the contraction
-    const __amdgpu_buffer_rsrc_t rv = rows_of(bv + static_cast<int64_t>(c) * CT * r_stride, min(CT, n - c * CT) * rs);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s.v[i] = load1(rv, atv[i]);
-  };
-  auto chunk = [&](int c, const Small& now, Small& next) {              // (products are interleaved so that neighbours do not wait for one another)
-    const float* cur = lds + (c & 1) * L::SIZE;
-    f32x4v u = now.v, y = now.v, o[TPW], z[TPW], q[TPW], k[TPW], p[TPW];
-    f32x4v* red = reinterpret_cast<f32x4v*>(lds + L::RED);
-    fetch_small(min(c + 1, chunks - 1), next);
-    const int rows = fr * LD + 16 * wave * TPW + g4;
+  } else {                                                              // and four multiply
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
-      if constexpr (DELTA) k[t] = *reinterpret_cast<const f32x4v*>(cur + L::K + rows + 16 * t);
-      q[t] = *reinterpret_cast<const f32x4v*>(cur + L::Q + rows + 16 * t);
-      o[t] = z[t] = f32x4v{0};
+      const int c = 16 * (wave * TPW + t) + g4;
+      const f32x4v v = *reinterpret_cast<const f32x4v*>(sp + min(c, dk - 4));
+      S[t] = pos0 > 0 && c < dk ? v : f32x4v{0};
     }
-    if constexpr (DELTA) {
+    // M and B of a chunk by lanes as left operands (row lane % 16, contraction index 4 (lane / 16) + i), V as the accumulators lie
+    struct Small { f32x4v m, v; float b; } now, then;
+    const float* pairs0 = pairs + (static_cast<int64_t>(place0) * H + h) * PAIR;
+    const int atm = (fr * CT + g4) * 4;
+    int atv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      atv[i] = (g4 + i) * rs + colc * 4;
+    }
+    auto fetch_small = [&](int c, Small& s) {
+      const __amdgpu_buffer_rsrc_t rp = rows_of(pairs0 + static_cast<int64_t>(c) * H * PAIR, PAIR * 4);
+      if constexpr (DELTA) s.m = load4(rp, atm);
+      s.b = load1(rp, atm + CT * CT * 4 + wave * 4);                      // B U is shared out by steps of the contraction
+      const __amdgpu_buffer_rsrc_t rv = rows_of(bv + static_cast<int64_t>(c) * CT * r_stride, min(CT, n - c * CT) * rs);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s.v[i] = load1(rv, atv[i]);
+    };
+    auto chunk = [&](int c, const Small& now, Small& next) {              // (products are interleaved so that neighbours do not wait for one another)
+      const float* cur = lds + (c & 1) * L::SIZE;
+      f32x4v u = now.v, y = now.v, o[TPW], z[TPW], q[TPW], k[TPW], p[TPW];
+      f32x4v* red = reinterpret_cast<f32x4v*>(lds + L::RED);
+      fetch_small(min(c + 1, chunks - 1), next);
+      const int rows = fr * LD + 16 * wave * TPW + g4;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        if constexpr (DELTA) k[t] = *reinterpret_cast<const f32x4v*>(cur + L::K + rows + 16 * t);
+        q[t] = *reinterpret_cast<const f32x4v*>(cur + L::Q + rows + 16 * t);
+        o[t] = z[t] = f32x4v{0};
+      }
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < TPW; ++t) z[t] = mfma_f32(k[t][i], S[t][i], z[t]);
+#pragma unroll
+        for (int t = 1; t < TPW; ++t) z[0] += z[t];
+        red[wave * 64 + lane] = z[0];
+        lds_barrier();
+        y -= (red[lane] + red[64 + lane]) + (red[128 + lane] + red[192 + lane]);
+        u = f32x4v{0};
+      }
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        k[t] = *reinterpret_cast<const f32x4v*>(cur + L::KT + (16 * (wave * TPW + t) + fr) * LT + g4);
+        p[t] = *reinterpret_cast<const f32x4v*>(cur + L::P + 16 * (wave * TPW + t) + g4);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) o[t] = mfma_f32(q[t][i], S[t][i], o[t]);
+        if constexpr (DELTA) u = mfma_f32(now.m[i], y[i], u);
+      }
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) S[t] *= p[t];
+      o[0] = mfma_f32(now.b, wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3], o[0]);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < TPW; ++t) z[t] = mfma_f32(k[t][i], S[t][i], z[t]);
+        for (int t = 0; t < TPW; ++t) S[t] = mfma_f32(k[t][i], u[i], S[t]);
 #pragma unroll
-      for (int t = 1; t < TPW; ++t) z[0] += z[t];
-      red[wave * 64 + lane] = z[0];
+      for (int t = 1; t < TPW; ++t) o[0] += o[t];
+      *reinterpret_cast<f32x4v*>(lds + L::OUT + (c & 1) * (4 * 256) + wave * 256 + lane * 4) = o[0];
       lds_barrier();
-      y -= (red[lane] + red[64 + lane]) + (red[128 + lane] + red[192 + lane]);
-      u = f32x4v{0};
-    }
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      k[t] = *reinterpret_cast<const f32x4v*>(cur + L::KT + (16 * (wave * TPW + t) + fr) * LT + g4);
-      p[t] = *reinterpret_cast<const f32x4v*>(cur + L::P + 16 * (wave * TPW + t) + g4);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int t = 0; t < TPW; ++t) o[t] = mfma_f32(q[t][i], S[t][i], o[t]);
-      if constexpr (DELTA) u = mfma_f32(now.m[i], y[i], u);
-    }
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) S[t] *= p[t];
-    o[0] = mfma_f32(now.b, wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3], o[0]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int t = 0; t < TPW; ++t) S[t] = mfma_f32(k[t][i], u[i], S[t]);
-#pragma unroll
-    for (int t = 1; t < TPW; ++t) o[0] += o[t];
-    *reinterpret_cast<f32x4v*>(lds + L::OUT + (c & 1) * (4 * 256) + wave * 256 + lane * 4) = o[0];
+    };
+    fetch_small(0, now);
     lds_barrier();
-  };
-  fetch_small(0, now);
-  lds_barrier();
-  for (int c = 0; c < chunks; c += 2) {
-    chunk(c, now, then);
-    chunk(c + 1, then, now);
+    for (int c = 0; c < chunks; c += 2) {
+      chunk(c, now, then);
+      chunk(c + 1, then, now);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wild |= !(fabsf(S[t][i]) < INFINITY);
   }
-  if (col >= dv) return;
+  // What an infinity of the carried state, or sums that left the range, make of a chunk's other tokens (zeros of the factors between them times
+  // infinity) is not what they make token by token: such columns start again, from the state as it was.
+  if (wild) any_wild = 1;
+  lds_barrier();
+  if (any_wild) {
+    __threadfence();                                                    // this wave's results are behind those that come
+    __syncthreads();
+    if (tid < 256) scan_columns<4 * TPW, DELTA, 4, 4, L::TOKENS>(a, b, h, unit % cols * 16, lds);
+    return;
+  }
+  if (part >= 4 || col >= dv) return;
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
     const int c = 16 * (wave * TPW + t) + g4;

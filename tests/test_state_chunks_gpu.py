@@ -103,3 +103,42 @@ def test_the_others_of_the_step(dk, dv, H, short, long, delta):
     (whole, state), (alone, kept) = scan(list(range(len(counts)))), scan(few)
     for i in few:
         assert torch.equal(whole[i], alone[i]) and torch.equal(state[i], kept[i])
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["inf state", "nan state", "sums beyond the range"])
+def test_carried_states_that_are_not_numbers(what, delta):
+    """A state with an infinity behind a chunk's decays, and sums of finite numbers that leave the range inside one: as token by token, to the bit;
+    other columns as ever."""
+    H, dk, dv, n = 4, 128, 48, 150
+    g = torch.Generator().manual_seed(3)
+    lay = RM.RecurrentLayout(H, H, dk, dv, 0, H * dk, 2 * H * dk, 2 * H * dk + H * dv if delta else -1)
+    r = torch.rand((n, 3 * H * dk + H * dv + (H if delta else 0)), generator=g) * 0.9
+    r[:, :2 * H * dk] /= dk ** 0.5
+    start = torch.randn((1, H, dv, dk), generator=g)
+    if what == "sums beyond the range":
+        r[:, 2 * H * dk + H * dv:3 * H * dk + H * dv] = 1.0
+        start[0, 1, 20] = 2e38
+        r[n // 2:, H * dk + dk:H * dk + 2 * dk] = 1e6
+        r[n // 2:, 2 * H * dk + dv:2 * H * dk + 2 * dv] = 1e12
+    else:
+        start[0, 1, 20, 5] = float("inf" if what == "inf state" else "nan")
+        r[:, 2 * H * dk + H * dv + dk:2 * H * dk + H * dv + 2 * dk] = 1e-6             # decays whose product over a chunk is zero in 32 bits
+
+    from gbx_lm_amd import _lib
+    L, got = _lib.mixers(), []
+    seq = torch.tensor([[0, 7, n, 0]], dtype=torch.int32, device=DEV)
+    rd = r.to(DEV)
+    for nbytes in (L.gbxm_state_scan_workspace(1, n, n, H, dk, dv), 0):
+        state, out, ws = start.to(DEV).clone(), torch.empty((n, H * dv), device=DEV), torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=DEV)
+        _lib.check_mixers(L.gbxm_state_scan_ws(rd.data_ptr(), rd.stride(0), state.data_ptr(), out.data_ptr(), seq.data_ptr(), 1, n, H, H, dk, dv, int(delta),
+                                               ws.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream))
+        got.append((out.cpu(), state.cpu()))
+    (out, state), (out1, state1) = got
+    assert not bool(state1[0, 1, 20].isfinite().all()) or not bool(out1.isfinite().all())
+    wild, heads = torch.arange(dv) // 16 == 1, torch.arange(H) != 1                    # the column block that goes again; heads whose sums are ordinary
+    assert torch.equal(out.view(n, H, dv)[:, 1, wild].nan_to_num(7.0), out1.view(n, H, dv)[:, 1, wild].nan_to_num(7.0))
+    assert torch.equal(state[0, 1, wild].nan_to_num(7.0), state1[0, 1, wild].nan_to_num(7.0))
+    assert torch.equal(out.isnan(), out1.isnan()) and torch.equal(state.isnan(), state1.isnan())
+    assert float((out - out1).view(n, H, dv)[:, heads].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
+    assert float((state - state1)[0, heads].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
