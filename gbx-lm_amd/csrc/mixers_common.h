@@ -133,10 +133,6 @@ __device__ __forceinline__ float key_value(unsigned k) { return __uint_as_float(
 
 // Rounds of arg-max over up to 64 PER candidates that one wave holds, candidate 64 i + lane in key[i] (0: none, or taken), of equal ones the
 // lowest first: take(round, candidate, its key), all uniform.  A round is some 40 instructions without a barrier or a trip to LDS.
-// A router's choice with it | every expert counting those in front of it, in LDS, us: softmax, 8 of 128, 1 row 3.5 | 8.9, 3 481 rows
-// 4.9 | 19.8, 8 of 256 6.2 | 27.9, 2 of 16, 1 row 2.7 | 3.8; sigmoid in 8 groups, 2 of 32, 1 row 3.1 | 4.9, 8 of 128, 3 481 rows 6.2 | 17.6; plain sigmoid, 8 of
-// 128, 1 row 3.1 | 8.0, 2 of 64, 8 192 rows 3.6 | 10.0.
-inline bool choice_by_wave(int E, int top) { return E <= 256 && top <= 64; }
 template <int PER, typename Take> __device__ __forceinline__ void wave_choose(unsigned (&key)[PER], int rounds, Take take) {
   const int lane = threadIdx.x & 63;
   for (int k = 0; k < rounds; ++k) {
@@ -156,6 +152,22 @@ template <int PER, typename Take> __device__ __forceinline__ void wave_choose(un
     take(k, e, m);
   }
 }
+// Which form a router's choice takes: rounds of a wave, or by rank, where every expert counts those in front of it in LDS, whatever their number.  The line is each
+// kernel's own (`most` choices; the softmax kernel's ranks cost more: it takes probabilities in 256 threads), a row's form does not depend on the other rows.  Rank | wave, us,
+// 1 row / 3 481 rows.  Softmax: 8 of 16 3.4 | 2.8 / 6.6 | 4.1, 16 of 16 3.5 | 3.5 / 6.7 | 5.4; 28 of 32 4.4 | 4.6 / 8.6 | 7.4; 8 of 64 5.6 | 2.8 / 11.4 | 4.1, 36 of 64 5.9 | 5.3 / 11.8 |
+// 8.6, 52 of 64 6.0 | 6.8 / 12.0 | 11.2, 64 of 64 5.9 | 7.9 / 11.8 | 13.2; 8 of 128 8.5 | 3.1 / 19.8 | 4.7, 64 of 128 9.0 | 9.8 / 20.2 | 15.9; 64 of 256 15.1 | 13.2 / 43.5 | 21.6.
+// Sigmoid: 12 of 16 2.9 | 3.3 / 4.2 | 4.6; 12 of 32 3.7 | 3.3 / 5.0 | 4.6, 20 of 32 3.7 | 4.1 / 5.1 | 6.0; 28 of 64 5.2 | 5.0 / 7.1 | 7.3, 36 of 64 5.3 | 5.9 / 7.2 | 8.7; 36 of 128 8.3 | 6.8 /
+// 16.0 | 10.3, 52 of 128 8.4 | 9.0 / 16.3 | 13.6; 64 of 256 14.6 | 13.8 / 42.9 | 21.2; softmax over the logits' order: 28 of 64 5.3 | 4.7 / 7.3 | 7.2, 36 of 64 5.4 | 5.4 / 7.3 | 8.5, 52 of 128
+// 8.6 | 8.3 / 16.4 | 13.1.  Sigmoid, groups kept of all + choices of experts: 4 of 8 + 8 of 128 9.0 | 3.8 / 17.4 | 6.0, 32 of 64 + 8 of 128 11.5 | 6.0 / 22.8 | 9.3, 16 of 32 + 16 of 64
+// 7.0 | 5.2 / 9.5 | 8.0, 40 of 64 + 40 of 64 8.5 | 9.7 / 11.8 | 15.6.  A lane holds a choice and a group: 64 of either at most.
+constexpr int most_of_softmax(int E) { return 6 + 5 * E / 8; }
+constexpr int most_of_logits(int E) { return 4 + 3 * E / 8; }
+inline bool choice_by_wave(int E, int top, int most, int groups = 0, int keep = 0) {
+  return E <= 256 && top <= 64 && groups <= 64 && top <= most && (groups == 0 || top + keep <= 16 + E / 2);
+}
+// Beyond that few choices with many groups remain, whose rounds of arg-max (per choice and kept group) a workgroup makes in about the time of 11 experts' ranks.
+constexpr int RANK_EXPERTS = 256;
+inline bool choice_by_rank(int E, int rounds) { return E <= RANK_EXPERTS && E <= 11 * rounds; }
 // a wave per row: one a workgroup while rows are few
 inline unsigned choice_threads(int64_t rows) { return rows > 1024 ? 256 : 64; }
 inline unsigned choice_blocks(int64_t rows) { return static_cast<unsigned>(rows > 1024 ? (rows + 3) / 4 : rows); }

@@ -504,6 +504,64 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   if (renorm && threadIdx.x < top) weight[t * top + threadIdx.x] /= chosen_sum;
 }
 
+// The same by rank: probabilities and their order as above, no round waits for another.
+__global__ __launch_bounds__(NT) void route_topk_rank_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int E,
+                                                            int top, int renorm) {
+  __shared__ __attribute__((aligned(16))) float pl[RANK_EXPERTS];
+  __shared__ float sel[NT];
+  __shared__ float red[NW], mxs[NW];
+  const int64_t t = blockIdx.x;
+  constexpr int PER = RANK_EXPERTS / NT;
+  float v[PER];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = threadIdx.x + i * NT;
+    v[i] = e < E ? logits[t * E + e] : -INFINITY;
+    mx = fmaxf(mx, v[i]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if ((threadIdx.x & 63) == 0) mxs[threadIdx.x >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) mx = fmaxf(mx, mxs[i]);
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
+    v[i] = live ? expf(v[i] - mx) : 0.f;
+    sum += v[i];
+  }
+  sum = block_sum<NW>(sum, red);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const bool live = static_cast<int>(threadIdx.x) + i * NT < E;
+    v[i] = live ? v[i] / sum : -1.f;
+    if (!(v[i] == v[i])) v[i] = -1.f;            // (not a number: behind every probability)
+    pl[threadIdx.x + i * NT] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = threadIdx.x + i * NT;
+    if (e < E) {
+      const int rank = rank_of(pl, (E + 3) / 4, e, v[i]);
+      if (rank < top) {
+        idx[t * top + rank] = e;
+        if (renorm) sel[rank] = v[i]; else weight[t * top + rank] = v[i];
+      }
+    }
+  }
+  if (!renorm) return;
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < top) {
+    float chosen = 0.f;
+    for (int k = 0; k < top; ++k) chosen += sel[k];
+    weight[t * top + threadIdx.x] = sel[threadIdx.x] / chosen;
+  }
+}
+
 // The same for up to 64 PER experts, a wave per row.
 template <int PER>
 __global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight, int64_t rows, int E,
@@ -656,12 +714,13 @@ int gbxm_route_topk(const float* logits, int32_t* idx, float* weight, int64_t T_
   if (top > NT) return fail(GBXM_ERR_UNSUPPORTED, "route_topk: top > %d", NT);
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (choice_by_wave(E, top)) {
+  if (choice_by_wave(E, top, most_of_softmax(E))) {
     const unsigned blocks = choice_blocks(T_), threads = choice_threads(T_);
     if (E <= 64) route_topk_wave_kernel<1><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
     else if (E <= 128) route_topk_wave_kernel<2><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
     else route_topk_wave_kernel<4><<<blocks, threads, 0, s>>>(logits, idx, weight, T_, E, top, renorm);
-  } else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
+  } else if (choice_by_rank(E, top)) route_topk_rank_kernel<<<dim3(T_), NT, 0, s>>>(logits, idx, weight, E, top, renorm);
+  else route_topk_kernel<<<dim3(T_), NT, E * sizeof(float), s>>>(logits, idx, weight, E, top, renorm);
   return after_launch("route_topk");
 }
 

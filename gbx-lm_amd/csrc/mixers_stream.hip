@@ -270,6 +270,70 @@ __global__ __launch_bounds__(64) void route_sigmoid_groups_kernel(const float* _
   for (int k = lane; k < top; k += 64) weight[t * top + k] = sl[idx[t * top + k]] * mul;
 }
 
+// The same by rank: scores, groups and their order as above.  A group with fewer than two experts that can be chosen scores
+// -inf and is never struck out, here as there.
+__global__ __launch_bounds__(NT) void route_sigmoid_rank_kernel(const float* __restrict__ logits, const float* __restrict__ correction,
+                                                               int* __restrict__ idx, float* __restrict__ weight, int E, int top, int n_groups,
+                                                               int keep_groups, int renorm, float scale) {
+  __shared__ __attribute__((aligned(16))) float cl[RANK_EXPERTS];
+  __shared__ __attribute__((aligned(16))) float gl[RANK_EXPERTS];
+  __shared__ float sel[RANK_EXPERTS];
+  const int64_t t = blockIdx.x;
+  const int nth = blockDim.x, tid = threadIdx.x;
+  constexpr int PER = RANK_EXPERTS / NT;
+  float sc[PER], c[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = tid + i * nth, ec = min(e, E - 1);
+    sc[i] = 1.f / (1.f + expf(-logits[t * E + ec]));
+    c[i] = sc[i] + correction[ec];
+    if (e >= E || c[i] != c[i]) c[i] = -INFINITY;
+    if (e < (E + 3) / 4 * 4) cl[e] = c[i];
+  }
+  __syncthreads();
+  if (n_groups > 0) {
+    const int size = E / n_groups, g4 = (n_groups + 3) / 4;
+    for (int g = tid; g < 4 * g4; g += nth) {
+      float a = -INFINITY, b = -INFINITY;          // the two largest
+      if (g < n_groups)
+#pragma unroll 8
+        for (int e = g * size; e < (g + 1) * size; ++e) {
+          const float v = cl[e];
+          b = fmaxf(b, fminf(a, v));
+          a = fmaxf(a, v);
+        }
+      gl[g] = size > 1 ? a + b : a;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = tid + i * nth;
+      if (e < E) {
+        const int g = e / size;
+        const float x = gl[g];
+        if (x != -INFINITY && rank_of(gl, g4, g, x) >= keep_groups) cl[e] = c[i] = -INFINITY;
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = tid + i * nth;
+    if (e < E) {
+      const int rank = rank_of(cl, (E + 3) / 4, e, c[i]);
+      if (rank < top) {
+        idx[t * top + rank] = e;
+        sel[rank] = sc[i];
+      }
+    }
+  }
+  __syncthreads();
+  float chosen = 0.f;
+  for (int k = 0; k < top; ++k) chosen += sel[k];
+  const float mul = renorm ? scale / (chosen + 1e-20f) : scale;
+  for (int k = tid; k < top; k += nth) weight[t * top + k] = sel[k] * mul;
+}
+
 // The same for up to 64 PER experts, a wave per row.  A group with fewer than two experts that can be chosen scores -inf and is never struck out, here
 // as there.
 template <int PER>
@@ -392,12 +456,14 @@ int gbxm_route_sigmoid_groups(const float* logits, const float* correction, int3
   if (E > 4096) return fail(GBXM_ERR_UNSUPPORTED, "route_sigmoid_groups: more than 4096 experts");
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (choice_by_wave(E, top) && n_groups <= 64) {
+  if (choice_by_wave(E, top, most_of_logits(E), n_groups, keep_groups)) {
     const unsigned blocks = choice_blocks(T_), threads = choice_threads(T_);
     if (E <= 64) route_sigmoid_wave_kernel<1><<<blocks, threads, 0, s>>>(logits, correction, idx, weight, T_, E, top, n_groups, keep_groups, renorm, scale);
     else if (E <= 128) route_sigmoid_wave_kernel<2><<<blocks, threads, 0, s>>>(logits, correction, idx, weight, T_, E, top, n_groups, keep_groups, renorm, scale);
     else route_sigmoid_wave_kernel<4><<<blocks, threads, 0, s>>>(logits, correction, idx, weight, T_, E, top, n_groups, keep_groups, renorm, scale);
-  } else
+  } else if (choice_by_rank(E, top + (n_groups > 0 ? keep_groups : 0)))
+    route_sigmoid_rank_kernel<<<dim3(T_), min((E + 63) / 64 * 64, NT), 0, s>>>(logits, correction, idx, weight, E, top, n_groups, keep_groups, renorm, scale);
+  else
     route_sigmoid_groups_kernel<<<dim3(T_), 64, (2 * E + (n_groups > 0 ? n_groups : 1)) * sizeof(float), s>>>(logits, correction, idx, weight, E, top,
                                                                                                             n_groups, keep_groups, renorm, scale);
   return after_launch("route_sigmoid_groups");

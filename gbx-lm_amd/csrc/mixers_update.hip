@@ -166,7 +166,7 @@ __global__ __launch_bounds__(NT) void router_rows_kernel(const T* __restrict__ h
   if (lane == 0) logits[t * E + e] = s;
 }
 
-// One workgroup per row (more than 256 experts or 64 choices; others: route_groups_wave_kernel).  The choice runs on the logits (softmax keeps their order) and by RANK: an expert counts the candidates in front
+// One workgroup per row (few choices: route_groups_wave_kernel).  The choice runs on the logits (softmax keeps their order) and by RANK: an expert counts the candidates in front
 // of it -- larger, or equal with a lower index -- so no round waits for another; ranks are a permutation (a logit that is not a number
 // counts as the smallest).  LDS: candidate logits [E, padded to 4 with -inf], group maxima [n_groups, padded], partial sums.
 __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restrict__ logits, int64_t row, int* __restrict__ idx, float* __restrict__ weight,
@@ -176,13 +176,13 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
   float* cl = lds;
   float* gl = lds + (E + 3) / 4 * 4;
   const int64_t t = blockIdx.x;
-  const int tid = threadIdx.x;
+  const int nth = blockDim.x, tid = threadIdx.x;
   const float* lr = logits + t * row;
   auto at = [&](int e) { const float v = lr[e]; return v == v ? v : -INFINITY; };
-  for (int e = tid; e < (E + 3) / 4 * 4; e += NT) cl[e] = e < E ? at(e) : -INFINITY;
+  for (int e = tid; e < (E + 3) / 4 * 4; e += nth) cl[e] = e < E ? at(e) : -INFINITY;
   __syncthreads();
   if (sigmoid) {                                       // (its order is the logits' order)
-    for (int e = tid; e < E; e += NT) {
+    for (int e = tid; e < E; e += nth) {
       const int rank = rank_of(cl, (E + 3) / 4, e, cl[e]);
       if (rank < top) {
         idx[t * top + rank] = e;
@@ -192,18 +192,27 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
     return;
   }
   float mx = -INFINITY;
-  for (int e = tid; e < E; e += NT) mx = fmaxf(mx, cl[e]);
+  for (int e = tid; e < E; e += nth) mx = fmaxf(mx, cl[e]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  if ((tid & 63) == 0) red[tid >> 6] = mx;
-  __syncthreads();
-  for (int i = 0; i < NW; ++i) mx = fmaxf(mx, red[i]);
+  if (nth > 64) {
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    for (int i = 0; i < nth / 64; ++i) mx = fmaxf(mx, red[i]);
+    __syncthreads();
+  }
   float sum = 0.f;
-  for (int e = tid; e < E; e += NT) sum += expf(cl[e] - mx);
-  sum = block_sum<NW>(sum, red);
+  for (int e = tid; e < E; e += nth) sum += expf(cl[e] - mx);
+  sum = wave_sum(sum);
+  if (nth > 64) {
+    if ((tid & 63) == 0) red[tid >> 6] = sum;
+    __syncthreads();
+    sum = 0.f;
+    for (int i = 0; i < nth / 64; ++i) sum += red[i];
+  }
   if (n_groups > 0) {
     const int size = E / n_groups, g4 = (n_groups + 3) / 4;
-    for (int g = tid; g < 4 * g4; g += NT) {
+    for (int g = tid; g < 4 * g4; g += nth) {
       float a = -INFINITY;
       if (g < n_groups)
 #pragma unroll 8
@@ -211,13 +220,13 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
       gl[g] = a;
     }
     __syncthreads();
-    for (int e = tid; e < E; e += NT) {
+    for (int e = tid; e < E; e += nth) {
       const int g = e / size;
       if (rank_of(gl, g4, g, gl[g]) >= keep_groups) cl[e] = -INFINITY;      // (only this thread reads cl[e] until the barrier)
     }
     __syncthreads();
   }
-  for (int e = tid; e < E; e += NT) {
+  for (int e = tid; e < E; e += nth) {
     const float x = cl[e];
     const int rank = rank_of(cl, (E + 3) / 4, e, x);
     if (rank < top) {
@@ -342,7 +351,7 @@ int gbxm_route_groups(const float* logits, int64_t row, int32_t* idx, float* wei
   if (E > 8192) return fail(GBXM_ERR_UNSUPPORTED, "route_groups: more than 8192 experts");
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (choice_by_wave(E, top) && n_groups <= 64) {
+  if (choice_by_wave(E, top, most_of_logits(E), n_groups, keep_groups)) {
     const unsigned blocks = choice_blocks(T_), threads = choice_threads(T_);
 #define GBXM_CHOOSE(PER_) \
   route_groups_wave_kernel<PER_><<<blocks, threads, 0, s>>>(logits, row, idx, weight, weight_row, T_, E, top, n_groups, keep_groups, gate, sigmoid)
@@ -352,7 +361,7 @@ int gbxm_route_groups(const float* logits, int64_t row, int32_t* idx, float* wei
 #undef GBXM_CHOOSE
   } else {
     const size_t lds = ((E + 3) / 4 * 4 + (n_groups + 3) / 4 * 4 + 4) * sizeof(float);
-    route_groups_kernel<<<dim3(T_), NT, lds, s>>>(logits, row, idx, weight, weight_row, E, top, n_groups, keep_groups, gate, sigmoid);
+    route_groups_kernel<<<dim3(T_), E <= 64 ? 64 : (E <= 128 ? 128 : NT), lds, s>>>(logits, row, idx, weight, weight_row, E, top, n_groups, keep_groups, gate, sigmoid);
   }
   return after_launch("route_groups");
 }

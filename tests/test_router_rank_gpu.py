@@ -117,6 +117,20 @@ def test_sigmoid_choice_of_odd_logits(e, top, groups):
             assert all(a != a if v > 0 else abs(a + v) < 1e-6 for a, (v, _) in zip(got, key))
 
 
+@pytest.mark.parametrize("e,top", [(16, 16), (32, 26), (32, 27), (64, 46), (64, 47), (64, 64), (128, 64), (128, 65), (129, 70), (256, 64), (256, 65), (256, 256), (300, 70)])
+def test_softmax_choice_of_many(e, top):
+    """Both sides of the rule between rounds of a wave and ranks, and all experts chosen."""
+    for t, renorm in ((3, True), (1030, False)):
+        test_softmax_choice(e, top, t, torch.float32, renorm)
+
+
+@pytest.mark.parametrize("e,top,groups", [(16, 10, None), (16, 11, None), (64, 28, None), (64, 29, None), (130, 70, None), (256, 64, None), (256, 65, None), (256, 200, (4, 4)), (64, 16, (32, 32)),
+                                          (64, 17, (32, 32)), (64, 29, (32, 2 * 8)), (128, 8, (128, 40)), (256, 2, (128, 4)), (256, 8, (256, 128)), (300, 70, (100, 50))])
+def test_grouped_sigmoid_choice_of_many(e, top, groups):
+    """The same, and more groups than a wave has lanes: few of their rounds, and many."""
+    test_grouped_sigmoid_choice(e, top, groups, 33, torch.float32, True)
+
+
 CHOICES = [(1, 1, None), (63, 4, (9, 2)), (64, 64, None), (65, 8, None), (128, 8, (8, 4)), (129, 65, None), (192, 6, (64, 40)), (256, 8, (8, 4)), (256, 64, (128, 64)),
            (260, 8, (4, 2))]
 
