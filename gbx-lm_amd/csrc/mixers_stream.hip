@@ -367,8 +367,9 @@ __global__ __launch_bounds__(256) void route_sigmoid_wave_kernel(const float* __
         a = fmaxf(a, v);
       }
     const float both = size > 1 ? a + b : a;
-    unsigned long long stays = __builtin_amdgcn_ballot_w64(lane < n_groups && both == -INFINITY);
-    unsigned key[1] = {lane < n_groups ? order_key(both) : 0u};
+    const bool odd = both != both;                                       // (infinities of both signs: stays beside those that are kept)
+    unsigned long long stays = __builtin_amdgcn_ballot_w64(lane < n_groups && (odd || both == -INFINITY));
+    unsigned key[1] = {lane < n_groups && !odd ? order_key(both) : 0u};
     wave_choose(key, keep_groups, [&](int, int g, unsigned) { stays |= 1ull << g; });
 #pragma unroll
     for (int i = 0; i < PER; ++i)

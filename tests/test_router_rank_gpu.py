@@ -131,6 +131,19 @@ def test_grouped_sigmoid_choice_of_many(e, top, groups):
     test_grouped_sigmoid_choice(e, top, groups, 33, torch.float32, True)
 
 
+@pytest.mark.parametrize("e,top,keep", [(64, 6, 3), (64, 32, 24), (128, 4, 2)])
+def test_a_group_whose_score_is_no_number(e, top, keep):
+    """An expert that is always chosen beside one that never is: their group stays and takes no other's place, by rounds and by rank."""
+    rows, correction = torch.randn((3, e), generator=torch.Generator().manual_seed(e)), torch.zeros(e)
+    correction[10], correction[11] = float("inf"), float("-inf")
+    idx, _ = choose(rows, top, (e // 2, keep), correction)
+    for r in range(3):
+        c = torch.sigmoid(rows[r].double()) + correction
+        best = c.view(-1, 2).sum(-1).nan_to_num(-1.0).topk(keep).indices.tolist()
+        alive = [i for i in range(e) if i // 2 in best or i // 2 == 5]
+        assert idx[r].tolist() == sorted(alive, key=lambda i: (-c[i].item(), i))[:top]
+
+
 CHOICES = [(1, 1, None), (63, 4, (9, 2)), (64, 64, None), (65, 8, None), (128, 8, (8, 4)), (129, 65, None), (192, 6, (64, 40)), (256, 8, (8, 4)), (256, 64, (128, 64)),
            (260, 8, (4, 2))]
 
