@@ -15,7 +15,7 @@
 // The matrix-core kernel for bf16 prompt portions is in mixers_sink_mfma.hip.
 #include <algorithm>
 #include <climits>
-#include "mixers_common.h"
+#include "mixers_mfma.h"
 
 namespace gbxm {
 namespace {
@@ -527,23 +527,24 @@ __global__ __launch_bounds__(NT) void stream_add_norm_kernel(float* __restrict__
 template <typename T, bool FAST>
 struct HeadOut {
   const gbxm_head_project_args& a;
+  int64_t row;
   const T* ip;
   T* op;
   const T* gp;                                     // this row and head's gates, or null
-  __device__ __forceinline__ HeadOut(const gbxm_head_project_args& a_) : a(a_) {
-    ip = static_cast<const T*>(a.in) + blockIdx.x * a.in_row + blockIdx.y * a.in_head;
-    op = static_cast<T*>(a.out) + blockIdx.x * a.out_row + blockIdx.y * a.out_head;
-    gp = a.gate ? static_cast<const T*>(a.gate) + blockIdx.x * a.gate_row + static_cast<int64_t>(blockIdx.y) * a.n_out : nullptr;
+  __device__ __forceinline__ HeadOut(const gbxm_head_project_args& a_, int64_t row_) : a(a_), row(row_) {
+    ip = static_cast<const T*>(a.in) + row * a.in_row + blockIdx.y * a.in_head;
+    op = static_cast<T*>(a.out) + row * a.out_row + blockIdx.y * a.out_head;
+    gp = a.gate ? static_cast<const T*>(a.gate) + row * a.gate_row + static_cast<int64_t>(blockIdx.y) * a.n_out : nullptr;
   }
   __device__ __forceinline__ void put(int j, float s) const { op[j] = from_f32<T>(gp ? s * sigmoid_<FAST>(to_f32(gp[j])) : s); }
   __device__ __forceinline__ void tail() const {
     if (!a.freq) {
-      for (int c = threadIdx.x; c < a.n_tail; c += NT) op[a.n_out + c] = ip[a.n_in + c];
+      for (int c = threadIdx.x; c < a.n_tail; c += blockDim.x) op[a.n_out + c] = ip[a.n_in + c];
       return;
     }
     const int half = a.n_tail / 2;
-    const float pos = static_cast<float>(a.positions[blockIdx.x * a.pos_stride]);
-    for (int i = threadIdx.x; i < half; i += NT) {
+    const float pos = static_cast<float>(a.positions[row * a.pos_stride]);
+    for (int i = threadIdx.x; i < half; i += blockDim.x) {
       const int c0 = a.interleaved ? 2 * i : i, c1 = a.interleaved ? 2 * i + 1 : i + half;
       float sn, cs;
       sincosf(pos * a.freq[i], &sn, &cs);
@@ -558,7 +559,7 @@ struct HeadOut {
 template <typename T, bool FAST>
 __global__ __launch_bounds__(NT) void head_project_kernel(const gbxm_head_project_args a) {
   extern __shared__ float xin[];                   // [n_in]
-  const HeadOut<T, FAST> o(a);
+  const HeadOut<T, FAST> o(a, blockIdx.x);
   const T* ip = o.ip;
   const int n_in = a.n_in, n_out = a.n_out;
   const T* wp = static_cast<const T*>(a.w) + static_cast<int64_t>(blockIdx.y) * n_in * n_out;
@@ -577,112 +578,131 @@ __global__ __launch_bounds__(NT) void head_project_kernel(const gbxm_head_projec
   o.tail();
 }
 
-// The same with 16-byte loads of w: a thread owns a run of PER outputs and every IS-th input channel (IS = 256 / (outputs / PER):
-// all threads stream w, many loads in flight each); the IS partial sums of an output meet in LDS in a fixed order.
-template <typename T, bool FAST>
-__global__ __launch_bounds__(NT) void head_project_vec_kernel(const gbxm_head_project_args a) {
-  constexpr int PER = 16 / sizeof(T);
-  extern __shared__ float xin[];                   // [n_in], then the partial sums [NT * PER]
-  const HeadOut<T, FAST> o(a);
-  const T* ip = o.ip;
-  const int n_in = a.n_in, n_out = a.n_out;
-  float* red = xin + n_in;
-  const T* wp = static_cast<const T*>(a.w) + static_cast<int64_t>(blockIdx.y) * n_in * n_out;
-  const int tid = threadIdx.x;
-  for (int i = tid; i < n_in; i += NT) xin[i] = to_f32(ip[i]);
-  for (int jb = 0; jb < n_out; jb += NT * PER) {
-    const int jn = min(n_out - jb, NT * PER);
-    const int JC = jn / PER, IS = NT / JC;
-    const int jc = tid % JC, is = tid / JC;
-    float acc[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) acc[u] = 0.f;
-    __syncthreads();                               // xin is there; red is free
-    if (is < IS) {
-      const T* col = wp + jb + jc * PER;
-#pragma unroll 8
-      for (int i = is; i < n_in; i += IS) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(col + static_cast<int64_t>(i) * n_out);
-        const float x = xin[i];
-        if constexpr (sizeof(T) == 2) {
-          const unsigned u4[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            acc[2 * u] += x * __uint_as_float(u4[u] << 16);
-            acc[2 * u + 1] += x * __uint_as_float(u4[u] & 0xFFFF0000u);
-          }
-        } else {
-          acc[0] += x * __uint_as_float(raw.x); acc[1] += x * __uint_as_float(raw.y);
-          acc[2] += x * __uint_as_float(raw.z); acc[3] += x * __uint_as_float(raw.w);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < PER; ++u) red[is * jn + jc * PER + u] = acc[u];
-    }
-    __syncthreads();
-    for (int j = tid; j < jn; j += NT) {
-      float s = 0.f;
-      for (int k = 0; k < IS; ++k) s += red[k * jn + j];
-      o.put(jb + j, s);
-    }
-  }
-  o.tail();
-}
-
-// The same for steps of fewer rows times heads than CUs, a workgroup per (row, head, JC runs of PER outputs): a thread owns a run and every IS-th input channel (IS = 256 / JC),
-// eight of them in flight; the partial sums of a run meet within the waves and then in LDS, in a fixed order.  A workgroup of its own
-// copies or turns the tail.  Bound by one trip to memory; a workgroup for all of a head's outputs makes four trips one after the other, on T H of the
-// CUs.  That | this, us: 2 rows, 16 heads, 128 -> 512 channels 5.1 | 3.8, 512 -> 128 5.4 | 4.5, 1 row, 8 heads, 64 -> 256 3.6 | 3.3; 32 rows, 16 heads 6.1 | 8.7.
-template <typename T, bool FAST>
-__global__ __launch_bounds__(NT) void head_project_cut_kernel(const gbxm_head_project_args a, int JC) {
-  constexpr int PER = 16 / sizeof(T);
-  __shared__ __attribute__((aligned(16))) float red[NW][64 * PER];
-  const HeadOut<T, FAST> o(a);
+// The same with 16-byte loads of w, a workgroup per (row, head, JC runs of PER outputs): a thread owns a run and every IS-th input channel (IS = 256 / JC), eight of
+// them in flight, the first ones asked for before the row is parked in LDS.  An output is 32 sums -- sum m over the channels m, m + 32, ... in turn -- which meet by
+// halves, m and m + 16, then m and m + 8, and so on: in a thread's registers, across the waves in LDS, within a wave.  The same sums in the same order whatever JC,
+// so a row does not depend on how many others the step has.  Channels past the last one are zeros on either side: no test in the loop.  Bound by the trip to memory
+// while rows are few, then by the weights' way from L2.  Many rows go two a workgroup (ROWS), which halves that way.  A workgroup a (row, head), sums in its own order | that,
+// and outputs cut into runs with sums in an order of the step's below 256 rows times heads | this, us, bf16, 16 heads: 128 -> 512 channels, 2 rows 5.0 | 3.5 | 3.0, 15 rows 5.2 | 5.5 |
+// 4.0, 64 rows 8.5 | 8.5 | 8.4, 512 rows 45 | 46 | 42; 512 -> 128, 2 rows 5.0 | 4.1 | 3.4, 15 rows 5.2 | 5.8 | 4.1, 64 rows 8.5 | 8.4 | 6.8, 512 rows 45 | 44 | 30; 192 -> 1 024, 8 rows
+// 12.1 | 18.3 | 9.9; fp32, 512 -> 128, 15 rows 7.1 | 10.8 | 5.5.  128 heads of 128 -> 512, 32 rows, are the one size found slower: 28 | 28 | 32.  Sums two at a time in few registers, 16 sums,
+// 32 channels in flight a thread: slower at few rows or at many.
+template <typename T, bool FAST, int JC, int ROWS>
+__global__ __launch_bounds__(NT) void head_project_runs_kernel(const gbxm_head_project_args a, int own_tail) {
+  constexpr int PER = 16 / sizeof(T), IS = NT / JC, SUMS = 32 / IS, PART = PER / NW;
+  extern __shared__ float xin[];                   // [ROWS][n_in, in whole steps of 8 IS]
+  __shared__ __attribute__((aligned(16))) float red[NW][NW][64][PART];
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
   const int n_in = a.n_in, n_out = a.n_out, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j0 = blockIdx.z * JC * PER;
-  if (j0 >= n_out) {
-    o.tail();
+  if (j0 >= n_out) {                               // (a workgroup of its own copies or turns the tail)
+    HeadOut<T, FAST>(a, row0).tail();
     return;
   }
-  const int jc = tid & (JC - 1), IS = NT / JC, first = tid / JC;
-  const bool on = j0 + jc * PER < n_out;
-  const T* col = static_cast<const T*>(a.w) + static_cast<int64_t>(blockIdx.y) * n_in * n_out + (on ? j0 + jc * PER : 0);
-  float acc[PER];
+  const int jc = tid & (JC - 1), first = tid / JC, bytes = n_out * static_cast<int>(sizeof(T)), steps = (n_in + 8 * IS - 1) / (8 * IS), padded = steps * 8 * IS;
+  const T* w = static_cast<const T*>(a.w) + static_cast<int64_t>(blockIdx.y) * n_in * n_out;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w), 0, n_in * bytes, 0x00020000);
+  int at = first * bytes + min(j0 + jc * PER, n_out - PER) * static_cast<int>(sizeof(T));
+  u32x4 raw[8];
+  auto load = [&]() {
 #pragma unroll
-  for (int u = 0; u < PER; ++u) acc[u] = 0.f;
-  for (int i0 = first; i0 < n_in; i0 += 8 * IS) {
-    uint4 raw[8];
-    float x[8];
+    for (int k = 0; k < 8; ++k) raw[k] = __builtin_amdgcn_raw_buffer_load_b128(rw, at + k * IS * bytes, 0, 0);
+    at += 8 * IS * bytes;
+  };
+  load();
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int i = min(i0 + k * IS, n_in - 1);
-      raw[k] = *reinterpret_cast<const uint4*>(col + static_cast<int64_t>(i) * n_out);
-      x[k] = to_f32(o.ip[i]);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if (i0 + k * IS >= n_in) break;
-      if constexpr (sizeof(T) == 2) {
-        const unsigned u4[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          acc[2 * u] += x[k] * __uint_as_float(u4[u] << 16);
-          acc[2 * u + 1] += x[k] * __uint_as_float(u4[u] & 0xFFFF0000u);
-        }
-      } else {
-        acc[0] += x[k] * __uint_as_float(raw[k].x); acc[1] += x[k] * __uint_as_float(raw[k].y);
-        acc[2] += x[k] * __uint_as_float(raw[k].z); acc[3] += x[k] * __uint_as_float(raw[k].w);
-      }
-    }
-  }
-  for (int m = JC; m < 64; m <<= 1)
-#pragma unroll
-    for (int u = 0; u < PER; ++u) acc[u] += __shfl_xor(acc[u], m, 64);
-  if (lane < JC) {
-#pragma unroll
-    for (int u = 0; u < PER; u += 4) *reinterpret_cast<float4*>(&red[wave][lane * PER + u]) = float4{acc[u], acc[u + 1], acc[u + 2], acc[u + 3]};
+  for (int r = 0; r < ROWS; ++r) {                 // (a row behind the last one is the last one again; nobody writes it)
+    const T* ip = HeadOut<T, FAST>(a, min(row0 + r, a.T - 1)).ip;
+    for (int i = tid; i < padded; i += NT) xin[r * padded + i] = i < n_in ? to_f32(ip[i]) : 0.f;
   }
   __syncthreads();
-  for (int j = tid; j < JC * PER && j0 + j < n_out; j += NT) o.put(j0 + j, (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]));
+  float acc[ROWS][SUMS][PER];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < SUMS; ++c)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) acc[r][c][u] = 0.f;
+  const float* xp = xin + first;
+  for (int t = 0; t < steps; ++t, xp += 8 * IS) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const float x = xp[r * padded + k * IS];
+        float* to = acc[r][k % SUMS];
+        if constexpr (sizeof(T) == 2) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            to[2 * u] += x * __uint_as_float(raw[k][u] << 16);
+            to[2 * u + 1] += x * __uint_as_float(raw[k][u] & 0xFFFF0000u);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) to[u] += x * __uint_as_float(raw[k][u]);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);             // (hoisted among the products, loads cost a wave a SIMD)
+    if (t + 1 < steps) load();
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    if (row0 + r >= a.T) break;
+    const HeadOut<T, FAST> o(a, row0 + r);
+#pragma unroll
+    for (int c = SUMS / 2; c > 0; c /= 2)
+#pragma unroll
+      for (int k = 0; k < c; ++k)
+#pragma unroll
+        for (int u = 0; u < PER; ++u) acc[r][k][u] += acc[r][k + c][u];
+    // wave w finishes the outputs w PART .. w PART + PART - 1 of every run
+    if (r > 0) __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+#pragma unroll
+      for (int u = 0; u < PART; ++u) red[v][wave][lane][u] = acc[r][0][v * PART + u];
+    __syncthreads();
+    float s[PART];
+#pragma unroll
+    for (int u = 0; u < PART; ++u) {
+      s[u] = (red[wave][0][lane][u] + red[wave][2][lane][u]) + (red[wave][1][lane][u] + red[wave][3][lane][u]);
+#pragma unroll
+      for (int m = 32; m >= JC; m >>= 1) s[u] += __shfl_xor(s[u], m, 64);
+    }
+    if (lane < JC && j0 + jc * PER < n_out) {
+#pragma unroll
+      for (int u = 0; u < PART; ++u) o.put(j0 + jc * PER + wave * PART + u, s[u]);
+    }
+    if (!own_tail && blockIdx.z == gridDim.z - 1) o.tail();
+  }
+}
+
+// rows times heads from which a workgroup takes two rows.  One | two, us, bf16, 16 heads, 32 | 64 rows: 128 -> 512 5.4 | 9.2 against 5.5 | 8.4, 512 -> 128 5.2 | 7.6 against 5.6 | 6.8
+constexpr int64_t PAIRS_FROM = 1024;
+
+template <typename T, bool FAST>
+int launch_head_project(const gbxm_head_project_args& a, hipStream_t s) {
+  constexpr int PER = 16 / sizeof(T);
+  // runs of outputs a workgroup takes: fewer while that leaves CUs without one and lines of 128 bytes whole
+  const int64_t units = a.T * a.H;
+  const auto cuts = [&](int runs) { return (a.n_out + runs * PER - 1) / (runs * PER); };
+  const bool pairs = units >= PAIRS_FROM && a.n_in <= 4096;
+  int runs = pairs ? 32 : 64;
+  while (runs > 8 && (runs / 2 * PER >= a.n_out || units * cuts(runs) < 256)) runs /= 2;
+  const int own_tail = a.n_tail > 0 && units < 256, step = 8 * NT / runs;
+  const dim3 grid(pairs ? (a.T + 1) / 2 : a.T, a.H, cuts(runs) + own_tail);
+  const size_t lds = (a.n_in + step - 1) / step * step * sizeof(float) * (pairs ? 2 : 1);
+#define GBXM_RUNS(JC_)                                                                                       \
+  do {                                                                                                       \
+    if (pairs) head_project_runs_kernel<T, FAST, JC_, 2><<<grid, NT, lds, s>>>(a, own_tail);                 \
+    else head_project_runs_kernel<T, FAST, JC_, 1><<<grid, NT, lds, s>>>(a, own_tail);                       \
+  } while (0)
+  if (runs == 64) head_project_runs_kernel<T, FAST, 64, 1><<<grid, NT, lds, s>>>(a, own_tail);
+  else if (runs == 32) GBXM_RUNS(32);
+  else if (runs == 16) GBXM_RUNS(16);
+  else GBXM_RUNS(8);
+#undef GBXM_RUNS
+  return after_launch("head_project");
 }
 
 __device__ __forceinline__ float activation(float v, int kind) {
@@ -786,22 +806,10 @@ int gbxm_head_project(const gbxm_head_project_args* a, void* stream) {
   if (a->T == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int per = a->act == GBXM_BF16 ? 8 : 4;
+  const bool near = static_cast<int64_t>(a->n_in + 256) * a->n_out < (1 << 29);      // (a head's matrix, and a step beyond it, by 32-bit byte offsets)
+  if (a->n_out % per == 0 && near && reinterpret_cast<uintptr_t>(a->w) % 16 == 0)
+    return a->act == GBXM_BF16 ? launch_head_project<bf16_t, true>(*a, s) : launch_head_project<float, false>(*a, s);
   const dim3 grid(a->T, a->H);
-  if (a->n_out % per == 0 && reinterpret_cast<uintptr_t>(a->w) % 16 == 0) {
-    if (a->T * a->H < 256) {
-      // runs of outputs a workgroup takes: a wave's worth, fewer while that leaves CUs without one and lines of 64 bytes whole
-      int runs = 64;
-      while (runs > 4 && (runs / 2 * per >= a->n_out || a->T * a->H * ((a->n_out + runs * per - 1) / (runs * per)) < 256)) runs /= 2;
-      const dim3 cut(a->T, a->H, (a->n_out + runs * per - 1) / (runs * per) + (a->n_tail > 0));
-      if (a->act == GBXM_BF16) head_project_cut_kernel<bf16_t, true><<<cut, NT, 0, s>>>(*a, runs);
-      else head_project_cut_kernel<float, false><<<cut, NT, 0, s>>>(*a, runs);
-      return after_launch("head_project");
-    }
-    const size_t lds = (a->n_in + NT * per) * sizeof(float);
-    if (a->act == GBXM_BF16) head_project_vec_kernel<bf16_t, true><<<grid, NT, lds, s>>>(*a);
-    else head_project_vec_kernel<float, false><<<grid, NT, lds, s>>>(*a);
-    return after_launch("head_project");
-  }
   if (a->act == GBXM_BF16) head_project_kernel<bf16_t, true><<<grid, NT, a->n_in * sizeof(float), s>>>(*a);
   else head_project_kernel<float, false><<<grid, NT, a->n_in * sizeof(float), s>>>(*a);
   return after_launch("head_project");

@@ -184,6 +184,18 @@ def test_a_matrix_per_head(rows, heads, n_in, n_out, tail, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,n_in,n_out,tail", [(16, 128, 512, 64), (16, 512, 128, 0), (3, 33, 72, 8), (8, 1, 1032, 2), (5, 100, 40, 0), (4, 4100, 24, 0)])
+def test_a_matrix_per_head_of_any_number_of_rows(heads, n_in, n_out, tail, dt):
+    """A row's bits do not depend on how many others the step has: outputs cut into runs of every length, rows alone and in pairs."""
+    from gbx_lm_amd import mixer_ops as M
+    g = torch.Generator().manual_seed(n_in)
+    x, w = torch.randn((260, heads, n_in + tail), generator=g).to(dt).to(DEV), torch.randn((heads, n_in, n_out), generator=g).to(dt).to(DEV)
+    whole = M.head_project(x, w, tail)
+    for rows in (1, 2, 5, 15, 16, 33, 64, 65, 86, 129):
+        assert torch.equal(M.head_project(x[:rows], w, tail), whole[:rows])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("k,v,off", [(8, 4, 0), (576, 0, 0), (6, 4, 0), (8, 6, 0), (8, 8, 1), (1028, 512, 0)])
 @pytest.mark.parametrize("window,keep", [(None, 0), (5, 3)])
 def test_rows_appended_to_slots(k, v, off, dt, window, keep):
