@@ -13,8 +13,8 @@
 //
 // Bound by what a wave's own chain leaves idle (of a tile's time the matrix cores work a third, vector instructions a third: one exponential and
 // four others a score) and, in short prompts, by how few tiles there are.  Before (one buffer, every row found by itself, tiles from both ends of
-// a prompt in one workgroup) | now, us: 16 heads of <192, 128>, 8 192 rows 545 | 395, 10 000 rows 1 169 | 620, 2 000 + 777 rows 73 | 58; <128, 128>,
-// 8 192 rows 400 | 302, 4 000 rows 117 | 92, 1 501 + 700 + 65 rows 44 | 35; <64, 64>, 3 000 + 500 rows 54 | 44; 8 heads of <256, 256>, 3 000 rows 324 | 188.
+// a prompt in one workgroup) | now, us: 16 heads of <192, 128>, 8 192 rows 542 | 389, 2 000 + 777 rows 73 | 59, 7 500 rows 483 | 335; <128, 128>,
+// 8 192 rows 404 | 301, 4 000 rows 116 | 91, 1 501 + 700 + 65 rows 43 | 33; <64, 64>, 2 000 + 777 rows 37 | 30; 8 heads of <256, 256>, 4 000 rows 425 | 248.
 //
 // Head sizes are run-time numbers (multiples of 8) inside a compiled capacity <DK, DV>: channels beyond them are staged as zeros.
 #include <algorithm>
@@ -568,50 +568,74 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
   return launch_sink_reduce(a, splits, s);
 }
 
-// A workgroup = a query tile of a head; tiles that see many keys, at the end of the step's list, go first.  Heads are the fast index, those of a
-// key / value head G apart, so that an XCD's workgroups (every eighth) meet in few heads' keys.
-template <int DK, int DV, int GROUPS, int KT, int BUFS>
+// A workgroup = a query tile of a head, or (PAIRS, one group) two, one from each end of the list; tiles that see many keys, at the end of the step's list, go
+// first.  Heads are the fast index, those of a key / value head G apart, so that an XCD's workgroups (every eighth) meet in few heads' keys.
+template <int DK, int DV, int GROUPS, int KT, int BUFS, bool PAIRS>
 __global__ __launch_bounds__((256 * GROUPS), (SinkShape<DK, DV, GROUPS, KT, BUFS>::WAVES)) void sink_tile_kernel(const SinkTileArgs a, const int n_tiles) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int place = blockIdx.x % a.H, head = place % a.G * (a.H / a.G) + place / a.G;
-  sink_tile<DK, DV, GROUPS, KT, BUFS>(a, n_tiles - 1 - blockIdx.x / a.H, head, lds);
+  const int place = blockIdx.x % a.H, head = place % a.G * (a.H / a.G) + place / a.G, at = blockIdx.x / a.H;
+  sink_tile<DK, DV, GROUPS, KT, BUFS>(a, n_tiles - 1 - at, head, lds);
+  if constexpr (PAIRS) {
+    if (2 * at == n_tiles - 1) return;
+    __syncthreads();                                         // (the first tile's last keys have been read)
+    sink_tile<DK, DV, GROUPS, KT, BUFS>(a, at, head, lds);
+  }
 }
 
-template <int DK, int DV, int GROUPS, int KT, int BUFS>
+template <int DK, int DV, int GROUPS, int KT, int BUFS, bool PAIRS = false>
 int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
+  static_assert(!PAIRS || GROUPS == 1, "a second group leaves before the second tile");
   constexpr int bytes = SinkShape<DK, DV, GROUPS, KT, BUFS>::LDS;
   static OncePerDevice once;
   if (once.pending()) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT, BUFS>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sink_tile_kernel<DK, DV, GROUPS, KT, BUFS, PAIRS>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return hip_fail(e, "sink_attention (tiles)");
     once.done();
   }
-  sink_tile_kernel<DK, DV, GROUPS, KT, BUFS><<<static_cast<unsigned>(t.H) * n_tiles, 256 * GROUPS, bytes, s>>>(t, n_tiles);
+  const unsigned grid = static_cast<unsigned>(t.H) * (PAIRS ? (n_tiles + 1) / 2 : n_tiles);
+  sink_tile_kernel<DK, DV, GROUPS, KT, BUFS, PAIRS><<<grid, 256 * GROUPS, bytes, s>>>(t, n_tiles);
   return after_launch("sink_attention (tiles)");
 }
 
-// Which form, by tiles times heads n and the longest sequence's keys (0: unknown, long).  Measured in a replayed graph, us.
-// Up to 64 keys: one group, 32 keys, one buffer, the form with most waves (start-up is all there is: 1 x 20 rows, 16 heads of <128, 128> 6.4 | one
-// group of two buffers 7.8 | two groups 8.5; 64 x 20 rows 10.4 | 16.2 | 30.8); up to 224 also where there is more than a tile a CU: 64 x 200 60 | 70 |
-// 94, <64, 64> 64 x 100 17.7 | 23.9 | 33.4.
+// Which form, by tiles times heads n, the longest sequence's keys (0: unknown, long) and whether the others are about as long (even).  Measured in a
+// replayed graph, us, 16 heads of <128, 128> unless named.
+// Up to 64 keys: one group, 32 keys, one buffer, the form with most waves (start-up is all there is: 1 x 20 rows 6.4 | one group of two buffers 7.8 |
+// two groups 8.5; 64 x 20 rows 9.9 | 15.6 | 29.7); up to 224 also where there is more than a tile a CU: 64 x 200 60 | 70 | 94, 8 .. 163 rows x 32
+// 17.1 | 19.2 | 27.5, <64, 64> 32 heads, 64 x 128 32 | 35 | 60.
 // Two groups halve the chain of key tiles behind the last query tile, at one workgroup a CU.  Two groups | one of two buffers: 4 x 256 rows 13.3 |
 // 14.2, 2 x 500 17.8 | 21.0; small heads of few keys are done before a second buffer pays: two groups of one buffer | of two, <64, 64> 8 x 100 7.9 |
-// 8.6, <32, 32> 16 x 200 8.5 | 9.5.  Beyond a tile a CU only long chains gain: 8 x 500 37.5 | 31.4, 8 x 300 26.6 | 20.1, 4 x 1000 53.5 | 48.9, 2 x 1300
-// 34.8 | 46.9, 2 x 2000 61.9 | 78.2, 4 000 rows 93 | 125, <192, 128> 2 000 + 777 rows 58 | 90; a chip full of tiles has none to wait for: 7 000 rows
+// 8.6, <32, 32> 16 x 200 8.5 | 9.5.  Beyond a tile a CU only long chains gain: 8 x 500 36.8 | 31.1, 4 x 1000 49.5 | 45.8, 2 x 1300 33.0 | 42.6, 2 x 2000 58 |
+// 72, 4 000 rows 91 | 123, <192, 128> 2 000 + 777 rows 59 | 90; a chip full of tiles has none to wait for: 7 000 rows
 // 251 | 234, 8 192 332 | 301, <192, 128> 8 192 457 | 390, 10 000 669 | 617.
-constexpr int TWO_GROUPS = 960;
+// Two tiles a workgroup where tiles of sequences of one length would fill the places twice: one tile | two, 32 heads, 32 x 128 rows 31.9 | 31.1 (32 keys, one
+// buffer 34.7), 8 x 500 48.6 | 43.0, 4 x 1000 67.7 | 58.8, 3 x 1100 62 | 59, 16 x 500 56.7 | 45.3, 32 x 256 41.3 | 35.7, <192, 128> 16 x 500 68 | 55, <256, 256> 8 heads 16 x 500 87 |
+// 65, <64, 64> 16 x 500 37.8 | 34.3; of many lengths the long ones first even out better: 60 .. 810 rows x 16 46.6 | 53.3, 100 .. 660 x 8, 32 heads 38.3 | 44.9; so do fewer or
+// more tiles: 32 heads, 8 x 300 31 | 34, 4 x 700 46.7 | 47.6, 12 x 400 57.8 | 67.1.  Heads of 32: two groups of one buffer instead, 4 x 1000 40.7 | 32.8, 8 x 500 26.8 | 23.9, and pairs of
+// one buffer at twice as many tiles, 16 x 500 44.4 | 39.1, 32 x 256 32.7 | 29.4.
+constexpr int FEW_TILES = 960;
 template <int DK, int DV>
-int launch(const SinkTileArgs& t, int n_tiles, int longest, hipStream_t s) {
+int launch(const SinkTileArgs& t, int n_tiles, int longest, bool even, hipStream_t s) {
   constexpr int KT = DK + DV > 256 ? 32 : 64;                // (larger heads: 64 would cost the second wave per SIMD)
+  constexpr int PLACES = DK + DV <= 320 ? 512 : 256;
+  constexpr bool SMALL = DK + DV <= 64;
   const int64_t n = static_cast<int64_t>(t.H) * n_tiles;
   const int keys = longest > 0 ? longest : 1 << 30;
-  if (keys <= 64 || (keys <= 224 && n > (DK + DV > 64 ? 256 : TWO_GROUPS))) return launch_groups<DK, DV, 1, 32, 1>(t, n_tiles, s);
+  const auto twice = [&](int places) { return even && keys > 64 && keys <= 1100 && 8 * n > 13 * places && n <= 2 * places; };
+  if constexpr (DK + DV > 128) {
+    if (twice(PLACES)) return launch_groups<DK, DV, 1, KT, 2, true>(t, n_tiles, s);
+  }
+  if (keys <= 64 || (keys <= 224 && n > (SMALL ? FEW_TILES : 256))) return launch_groups<DK, DV, 1, 32, 1>(t, n_tiles, s);
   if constexpr (DK + DV < 256) {
-    if (keys <= (DK + DV > 64 ? 128 : 256) && n <= TWO_GROUPS) return launch_groups<DK, DV, 2, KT, 1>(t, n_tiles, s);
+    if ((keys <= (SMALL ? 256 : 128) && n <= FEW_TILES) || (SMALL && twice(PLACES))) return launch_groups<DK, DV, 2, KT, 1>(t, n_tiles, s);
+  }
+  if constexpr (SMALL) {
+    if (twice(2 * PLACES)) return launch_groups<DK, DV, 1, KT, 1, true>(t, n_tiles, s);
+  } else if constexpr (DK + DV <= 128) {
+    if (twice(PLACES)) return launch_groups<DK, DV, 1, KT, 2, true>(t, n_tiles, s);
   }
   if constexpr (DK + DV <= 320) {
-    if (n <= 256 || (n <= TWO_GROUPS && keys > 1024)) return launch_groups<DK, DV, 2, KT, 2>(t, n_tiles, s);
+    if (n <= 256 || (n <= FEW_TILES && keys > 1024)) return launch_groups<DK, DV, 2, KT, 2>(t, n_tiles, s);
   }
   return launch_groups<DK, DV, 1, KT, 2>(t, n_tiles, s);
 }
@@ -649,7 +673,8 @@ static SinkTileArgs tile_args(const gbxm_sink_attn_args& a) {
 int launch_sink_tiles(const gbxm_sink_attn_args& a, hipStream_t s) {
   if (!sink_tiles_shape(a.dk, a.dv) || a.q_tile != 128 || static_cast<int64_t>(a.H) * a.n_tiles > 0x7fffffff || !tile_operands(a)) return GBXM_ERR_UNSUPPORTED;
   const SinkTileArgs t = tile_args(a);
-#define GBXM_TILE(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch<DK_, DV_>(t, a.n_tiles, a.longest, s)
+  const bool even = a.longest > 0 && 8 * a.T >= 7 * static_cast<int64_t>(a.B) * a.longest;
+#define GBXM_TILE(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch<DK_, DV_>(t, a.n_tiles, a.longest, even, s)
   GBXM_TILE(32, 32); GBXM_TILE(64, 64); GBXM_TILE(64, 128); GBXM_TILE(96, 96); GBXM_TILE(128, 128); GBXM_TILE(192, 128); GBXM_TILE(256, 256);
 #undef GBXM_TILE
   return GBXM_ERR_UNSUPPORTED;

@@ -54,6 +54,13 @@ def portions(lens, dk, dv, window):
         r0 += n
 
 
+@pytest.mark.parametrize("count,rows,dk,dv", [(128, 120, 128, 128), (113, 128, 192, 128), (61, 250, 72, 64), (43, 257, 64, 64), (40, 300, 32, 32), (30, 1000, 32, 32), (63, 128, 256, 256),
+                                              (13, 1100, 96, 96), (12, 1200, 96, 96)])
+def test_sequences_of_one_length(count, rows, dk, dv):
+    """Two tiles a workgroup -- odd and even numbers of them, one and several a sequence -- and the forms that small heads take instead."""
+    portions([rows] * (count - 1) + [rows - 7], dk, dv, None)
+
+
 @pytest.mark.parametrize("window,keep", [(None, 0), (256, 0), (200, 5), (96, 70), (33, 0)])
 @pytest.mark.parametrize("dk,dv,H", [(64, 64, 8), (192, 128, 8), (128, 120, 8), (128, 128, 48)])
 def test_portions_behind_a_history(window, keep, dk, dv, H):
