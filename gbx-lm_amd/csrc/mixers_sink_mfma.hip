@@ -606,14 +606,15 @@ int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
 // Two groups halve the chain of key tiles behind the last query tile, at one workgroup a CU.  Two groups | one of two buffers: 4 x 256 rows 13.3 |
 // 14.2, 2 x 500 17.8 | 21.0; small heads of few keys are done before a second buffer pays: two groups of one buffer | of two, <64, 64> 8 x 100 7.9 |
 // 8.6, <32, 32> 16 x 200 8.5 | 9.5.  Beyond a tile a CU only long chains gain: 8 x 500 36.8 | 31.1, 4 x 1000 49.5 | 45.8, 2 x 1300 33.0 | 42.6, 2 x 2000 58 |
-// 72, 4 000 rows 91 | 123, <192, 128> 2 000 + 777 rows 59 | 90; a chip full of tiles has none to wait for: 7 000 rows
-// 251 | 234, 8 192 332 | 301, <192, 128> 8 192 457 | 390, 10 000 669 | 617.
+// 72, 4 000 rows 91 | 123, <192, 128> 2 000 + 777 rows 59 | 90; a chip whose two places a CU fill has less to wait for: 32 heads 2 x 1300 60 | 52, 3 000 rows
+// 117 | 108, 3 700 157 | 147, <64, 64> 2 500 62 | 59, <192, 128> 2 500 114 | 117, 3 000 148 | 138, 16 heads 7 500 374 | 335; heads of 32 are long at their chain: 32
+// heads 2 x 1300 28.7 | 31.3, 3 x 1100 30.3 | 35.5.
 // Two tiles a workgroup where tiles of sequences of one length would fill the places twice: one tile | two, 32 heads, 32 x 128 rows 31.9 | 31.1 (32 keys, one
 // buffer 34.7), 8 x 500 48.6 | 43.0, 4 x 1000 67.7 | 58.8, 3 x 1100 62 | 59, 16 x 500 56.7 | 45.3, 32 x 256 41.3 | 35.7, <192, 128> 16 x 500 68 | 55, <256, 256> 8 heads 16 x 500 87 |
 // 65, <64, 64> 16 x 500 37.8 | 34.3; of many lengths the long ones first even out better: 60 .. 810 rows x 16 46.6 | 53.3, 100 .. 660 x 8, 32 heads 38.3 | 44.9; so do fewer or
 // more tiles: 32 heads, 8 x 300 31 | 34, 4 x 700 46.7 | 47.6, 12 x 400 57.8 | 67.1.  Heads of 32: two groups of one buffer instead, 4 x 1000 40.7 | 32.8, 8 x 500 26.8 | 23.9, and pairs of
 // one buffer at twice as many tiles, 16 x 500 44.4 | 39.1, 32 x 256 32.7 | 29.4.
-constexpr int FEW_TILES = 960;
+constexpr int FEW_TILES = 960, LONG_TILES = 640;
 template <int DK, int DV>
 int launch(const SinkTileArgs& t, int n_tiles, int longest, bool even, hipStream_t s) {
   constexpr int KT = DK + DV > 256 ? 32 : 64;                // (larger heads: 64 would cost the second wave per SIMD)
@@ -635,7 +636,7 @@ int launch(const SinkTileArgs& t, int n_tiles, int longest, bool even, hipStream
     if (twice(PLACES)) return launch_groups<DK, DV, 1, KT, 2, true>(t, n_tiles, s);
   }
   if constexpr (DK + DV <= 320) {
-    if (n <= 256 || (n <= FEW_TILES && keys > 1024)) return launch_groups<DK, DV, 2, KT, 2>(t, n_tiles, s);
+    if (n <= 256 || (n <= (SMALL ? FEW_TILES : LONG_TILES) && keys > 1024)) return launch_groups<DK, DV, 2, KT, 2>(t, n_tiles, s);
   }
   return launch_groups<DK, DV, 1, KT, 2>(t, n_tiles, s);
 }
