@@ -488,16 +488,19 @@ int launch_group(const GroupArgs& g, int tiles, hipStream_t s) {
 size_t align16(size_t n) { return (n + 15) & ~static_cast<size_t>(15); }
 constexpr int64_t MIN_PAIRS = 64;         // below this the weight-streaming row kernels read less
 // Pairs per expert (on average) up to which the skinny form is taken.  Measured at 4 | 8 | 16 | 64 pairs per expert, skinny against grouped, us:
-// 128 experts of 3 x 2048 x 768  215 | 223 | 235 | 389  against 220 | 219 | 223 | 255;  64 of 2 x 2048 x 2048  187 | 196 | 211 | 374  against
-// 191 | 194 | 199 | 218;  32 of 3 x 1024 x 512  28 | 28 | 28 | 41  against 29 | 29 | 29 | 36.
+// 128 experts of 3 x 2048 x 768  215 | 221 | 237 | 383  against 215 | 224 | 228 | 259;  64 of 2 x 2048 x 2048  192 | 202 | 208 | 361  against
+// 192 | 195 | 193 | 215;  32 of 3 x 1024 x 512  27 | 27 | 28 | 40  against 30 | 30 | 30 | 38.
 constexpr int64_t SKINNY_PAIRS = 8;
-// ... and, where the grouped form's first product has at most half a chip of workgroups, each of them a chain over the whole contraction, up to 64.  Skinny |
-// grouped, us: without a gate, 16 experts of 2 x 1024 x 512, 4 | 32 | 64 pairs per expert 18 | 20 | 23 against 26 | 28 | 32; 8 of 2 x 4096 x 2048, 16 | 32 | 64
-// 58 | 76 | 111 against 79 | 81 | 96; gated, 4 of 3 x 512 x 2048, 32 | 64 | 128 pairs 26 | 27 | 32 against 37 | 46 | 56.
-constexpr int64_t SKINNY_PAIRS_FEW = 64, FEW_GROUPS = 128;
-int rows_of(int64_t P, int E, int F, bool gated) {
+// ... and, where the grouped form's first product has at most half a chip of workgroups, each of them a chain over the whole contraction, up to 64, while the skinny form's
+// -- one per tile and 128 channels, about half an expert's tile more than the pairs fill -- do not come to more than one a CU of 4 096 channels: every tile reads its
+// expert's weights anew.  Skinny | grouped, us: without a gate, 16 experts of 2 x 1024 x 512, 4 | 32 | 64 pairs per expert 18 | 18 | 24 against 27 | 27 | 33; 8 of 2 x 4096 x 2048,
+// 16 | 48 | 64 pairs 58 | 74 | 107 against 79 | 85 | 96; 4 of 2 x 4096 x 4096, 16 | 48 | 64 67 | 69 | 120 against 97 | 105 | 121 (the line lies behind 48 in both); 16 of 2 x 2048 x 1792,
+// 16 | 32 | 48 43 | 61 | 51 against 51 | 51 | 51 (many experts of one tile and a little, which the line does not see); gated, 4 of 3 x 512 x 2048, 32 | 64 pairs 26 | 27 against 37 | 45.
+constexpr int64_t SKINNY_PAIRS_FEW = 64, FEW_GROUPS = 128, FEW_CHANNELS = 256 * 4096;
+int rows_of(int64_t P, int E, int K, int F, bool gated) {
   const int64_t groups = (P / GR + E) * (gated ? (F + 127) / 128 : (F + 255) / 256);
-  return P <= (groups <= FEW_GROUPS ? SKINNY_PAIRS_FEW : SKINNY_PAIRS) * E ? RS : GR;
+  const bool few = groups <= FEW_GROUPS && (P / RS + E / 2) * ((F + 127) / 128) * K <= FEW_CHANNELS;
+  return P <= (few ? SKINNY_PAIRS_FEW : SKINNY_PAIRS) * E ? RS : GR;
 }
 
 
@@ -561,7 +564,7 @@ int launch_expert_grouped(const gbxm_expert_args& a, hipStream_t s) {
   const int P = static_cast<int>(a.T * top);
   ExpertBuckets k;
   const bool gated = a.kind != GBXM_EXPERT_RELU2;
-  const int rows = rows_of(P, E, F, gated);
+  const int rows = rows_of(P, E, K, F, gated);
   int rc = expert_buckets(a.idx, P, rows, E, a.ws, &k, s);
   if (rc != GBXM_OK) return rc;
   const int *offsets = k.offsets, *sorted = k.sorted, tiles = k.tiles;

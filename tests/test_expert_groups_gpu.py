@@ -51,6 +51,12 @@ def test_skinny_tiles(kind, width, ff, counts):
     tiles(counts, kind, width, ff)
 
 
+@pytest.mark.parametrize("pairs", [48, 56, 64])
+def test_few_workgroups_of_long_contractions(pairs):
+    """Both sides of the rule for steps of few experts: one tile of an expert's pairs, or several that read its weights anew."""
+    tiles([pairs + d for d in (-9, 0, 3, 6)] * 2, "relu2", 4096, 2048)
+
+
 def tiles(counts, kind, width, ff):
     from gbx_lm_amd import mixer_ops as M
     gen = torch.Generator(device="cuda").manual_seed(width + ff)
