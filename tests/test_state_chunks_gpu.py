@@ -142,3 +142,55 @@ def test_carried_states_that_are_not_numbers(what, delta):
     assert torch.equal(out.isnan(), out1.isnan()) and torch.equal(state.isnan(), state1.isnan())
     assert float((out - out1).view(n, H, dv)[:, heads].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
     assert float((state - state1)[0, heads].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["nothing", "nan value", "inf value", "nan key", "growing decay", "large key", "nan beta"])
+def test_which_form_ran(what, delta):
+    """The flags that lead the workspace, [heads][places]: zero for a head of ordinary numbers, and its sums are the chunks'; raised only for the head and the
+    sequence whose inputs are not, and what that one gives -- rows before the odd number, later ones and the state -- is the token-by-token form's to the bit.
+    A workspace that is a byte short leaves every sequence to that form."""
+    if what == "nan beta" and not delta:
+        pytest.skip("no betas without the delta rule")
+    from gbx_lm_amd import _lib
+    L, H, dk, dv, counts = _lib.mixers(), 4, 128, 32, [40, 150, 144, 9, 200]
+    T, B, g = sum(counts), len(counts), torch.Generator().manual_seed(11)
+    first = [sum(counts[:b]) for b in range(B)]
+    odd, at = 2, first[2] + 37
+    width = 3 * H * dk + H * dv
+    r = torch.rand((T, width + (H if delta else 0)), generator=g) * 0.9
+    r[:, :2 * H * dk] /= dk ** 0.5
+    head = {"value": 2 * H * dk + dv + 3, "key": H * dk + dk + 70, "decay": 2 * H * dk + H * dv + dk + 5, "beta": width + 1}
+    if what != "nothing":
+        kind, name = what.split()
+        r[at, head[name]] = {"nan": float("nan"), "inf": float("inf"), "growing": 1.5, "large": 1e13}[kind]
+    start = torch.randn((B, H, dv, dk), generator=g)
+    seq = torch.tensor([[b, b % 2 * 5, counts[b], first[b]] for b in range(B)], dtype=torch.int32, device=DEV)
+    rd, need = r.to(DEV), L.gbxm_state_scan_workspace(B, T, max(counts), H, dk, dv)
+    places = T // 16 + B
+    assert need > 4 * H * places
+
+    def scan(nbytes):
+        state, out, ws = start.to(DEV), torch.empty((T, H * dv), device=DEV), torch.full((need,), 0x5a, dtype=torch.uint8, device=DEV)
+        _lib.check_mixers(L.gbxm_state_scan_ws(rd.data_ptr(), rd.stride(0), state.data_ptr(), out.data_ptr(), seq.data_ptr(), B, T, H, H, dk, dv, int(delta),
+                                               ws.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream))
+        return out.cpu().view(T, H, dv), state.cpu(), ws.cpu()
+
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+    out, state, ws = scan(need)
+    token, kept, _ = scan(0)
+    short, shorts, untouched = scan(need - 1)
+    assert same(short, token) and same(shorts, kept) and bool((untouched == 0x5a).all())
+    flags = ws[:4 * H * places].view(torch.int32).view(H, places)
+    for b, n in enumerate(counts):
+        rows = slice(first[b], first[b] + n)
+        for h in range(H):
+            if n >= 128:
+                raised = flags[h, first[b] // 16 + b:][:(n + 15) // 16] != 0
+                assert bool(raised.any()) == (what != "nothing" and (b, h) == (odd, 1))
+            if n < 128 or (what != "nothing" and (b, h) == (odd, 1)):
+                assert same(out[rows, h], token[rows, h]) and same(state[b, h], kept[b, h])
+            else:
+                assert not torch.equal(out[rows, h], token[rows, h])          # (other orders of sums)
+                assert float((out - token)[rows, h].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
+                assert float((state - kept)[b, h].abs().max()) < (dk + 60) * 2.0 ** -22 * 32
