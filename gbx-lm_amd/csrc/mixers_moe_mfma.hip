@@ -10,26 +10,25 @@
 // channels of one pair (8-byte stores) and the gate / up pair of a channel sits in the same lane for the activation.
 // What bounds it: a few hundred pairs per expert, so the weights are a stream of their own (1.2 GB at 128 experts of 3 x 2048 x 768: 0.24 ms)
 // beside about as much matrix-core work; both operands therefore go memory -> LDS by DMA, stages of 64 elements, two of activations and three of
-// weights (which come from memory, two stages ahead; with two of either, one ahead: 64 experts of 2 x 2048 x 2048, 16 384 pairs 420 us for 389,
-// 128 of 3 x 2048 x 768, 2 048 pairs 252 for 236, 27 848 415 for 410), and a weight row is fetched once per 256 pairs.  Eight waves, a wave 128 pairs x 64 weight rows (16 x 16 x 32 products); four phases a stage, two wave groups
+// weights (which come from memory, two stages ahead; with two of either, one ahead), and a weight row is fetched once per 256 pairs.  Eight waves, a wave 128 pairs x 64 weight rows (16 x 16 x 32 products); four phases a stage, two wave groups
 // a barrier apart, so that one group multiplies while the other reads fragments and issues requests.  Stages of 64 elements, because a row
 // piece is then a whole 128-byte line: 256 x 128 tiles with stages of 32 elements and two workgroups per CU spent their time on twice the L2
 // requests (536 us for the first line below).  A tile is as high as its expert's pairs need, in steps of 64 (32 NR).
-// Measured (us, first + second products with the sort; 256-pair tiles with results from the registers -> results by rows, in turn on one card, uniform choices, the least of
-// four places of the weights in memory, which move these times by up to a tenth):
-//   27 848 pairs, 128 experts, 2048 x 768 gated:  448 -> 423 (now 406: 650 TFLOP/s, 3.0 TB/s of weights)
-//   18 128 pairs of the same:                       340 -> 326 (now 306: 3.9 TB/s)
-//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 437 -> 422 (now 389); a factor of the weights' way from memory (one expert's for all: 150 less) and of the results' (kept back:
-//   75 less), which tiles of one round write at the same time
-//    8 192 pairs,   8 experts, 4096 x 2048 gated:   461 -> 457 (900 TFLOP/s)
+// Measured (us, first + second products with the sort, uniform choices, mean over four places of the weights in memory, which move these times by up to a tenth;
+// two stages of weights, all from the contraction's start -> as it is now, in turn on one card):
+//   27 848 pairs, 128 experts, 2048 x 768 gated:  399 -> 395 (665 TFLOP/s, 3.1 TB/s of weights)
+//   18 128 pairs of the same:                     337 -> 320 (3.8 TB/s);  2 048 pairs: 262 -> 232 (5.2 TB/s)
+//   16 384 pairs,  64 experts, 2048 x 2048, no gate: 421 -> 400;  2 000 pairs: 274 -> 202.  At 16 384 the weights' way from memory is a factor (one expert's for all: 150 less) and
+//   the results' (kept back: 75 less), which tiles of one round write at the same time
+//    8 192 pairs,   8 experts, 4096 x 2048 gated: 473 -> 480 (860 TFLOP/s): the one form that the walk of the contraction costs, by 1 %
 // The table keeps a lower tile beside its expert's others.  By falling height, so that the last round is short, tiles read their weights anew: 256 pairs an
 // expert 454 us against 410 (64 experts), 531 against 476 (128), 288 pairs 595 against 467.  A stage's lines ordered into L2 before gain nothing; nor does
 // it matter how many rows a request spans (256 x 128 B, 64 x 512 B or 32 KB in one piece: 4.4 to 4.7 TB/s).
 // An expert's tiles walk the contraction from a stage of their own (expert % stages, so that a pair's sums do not depend on the step's other pairs): rows of
 // a power of two of bytes put a column of every row on the same memory channels, and workgroups that started together stayed there together.  All from the
-// first stage | this, us: 64 experts of 2 x 2048 x 2048, 2 000 pairs 259 | 200 (5.4 TB/s), 64 of 3 x 2048 x 1024, 6 000 pairs 208 | 178, 128 of 3 x 2048 x
-// 768, 2 048 pairs 237 | 228, 18 128 318 | 306; offsets by column
-// block as well lose the activation rows that its workgroups share in L2 (8 experts of 3 x 4096 x 2048, 8 192 pairs 449 | 446 | 479 by both).
+// first stage | this, us: 64 experts of 2 x 2048 x 2048, 2 000 pairs 259 | 202 (5.3 TB/s), 64 of 3 x 2048 x 1024, 6 000 pairs 208 | 185, 128 of 3 x 2048 x
+// 768, 2 048 pairs 237 | 232; offsets by column
+// block as well lose the activation rows that its workgroups share in L2 (8 experts of 3 x 4096 x 2048, 8 192 pairs 7 % slower).
 // The grid is sized for the worst case sum_e ceil(n_e / 256) <= P / 256 + E; surplus workgroups leave at once.
 // Steps with few pairs per expert (a batch that decodes) stream weights and little else: expert_skinny_kernel takes tiles of 32 pairs, a
 // wave per 32 output channels and no barrier.  A wave moves its own rows -- eight lanes to a row's 128 bytes, so an access touches eight

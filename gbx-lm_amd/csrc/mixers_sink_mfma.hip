@@ -121,7 +121,7 @@ __device__ __forceinline__ void sink_tile(const SinkTileArgs& a, const int tile,
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float scale2 = (a.head_scale ? a.scale * a.head_scale[head] : a.scale) * LOG2E;
-  // what the weights are measured from: the largest score when it last moved, and 8 more, so that no weight exceeds 1 until a score is 2^8 times that one
+  // what the weights are measured from: the largest score when it last moved, and 8 more, so that no weight exceeds 1 before the sums move again
   constexpr float ROOM = 8.f;
   float m = a.sink && group == 0 ? a.sink[head] * LOG2E + ROOM : -INFINITY;
   float l = (a.sink && group == 0 && hb == 0) ? 1.f / (1 << static_cast<int>(ROOM)) : 0.f;      // the sink counts once per query
@@ -610,7 +610,7 @@ int launch_groups(const SinkTileArgs& t, int n_tiles, hipStream_t s) {
 // 117 | 108, 3 700 157 | 147, <64, 64> 2 500 62 | 59, <192, 128> 2 500 114 | 117, 3 000 148 | 138, 16 heads 7 500 374 | 335; heads of 32 are long at their chain: 32
 // heads 2 x 1300 28.7 | 31.3, 3 x 1100 30.3 | 35.5.
 // Two tiles a workgroup where tiles of sequences of one length would fill the places twice: one tile | two, 32 heads, 32 x 128 rows 31.9 | 31.1 (32 keys, one
-// buffer 34.7), 8 x 500 48.6 | 43.0, 4 x 1000 67.7 | 58.8, 3 x 1100 62 | 59, 16 x 500 56.7 | 45.3, 32 x 256 41.3 | 35.7, <192, 128> 16 x 500 68 | 55, <256, 256> 8 heads 16 x 500 87 |
+// buffer 34.7), 8 x 500 48.6 | 43.0, 4 x 1000 67.7 | 58.8, 3 x 1100 62 | 59, 16 heads, 16 x 500 56.7 | 45.3, 32 x 256 41.3 | 35.7, <192, 128> 16 x 500 68 | 55, <256, 256> 8 heads 16 x 500 87 |
 // 65, <64, 64> 16 x 500 37.8 | 34.3; of many lengths the long ones first even out better: 60 .. 810 rows x 16 46.6 | 53.3, 100 .. 660 x 8, 32 heads 38.3 | 44.9; so do fewer or
 // more tiles: 32 heads, 8 x 300 31 | 34, 4 x 700 46.7 | 47.6, 12 x 400 57.8 | 67.1.  Heads of 32: two groups of one buffer instead, 4 x 1000 40.7 | 32.8, 8 x 500 26.8 | 23.9, and pairs of
 // one buffer at twice as many tiles, 16 x 500 44.4 | 39.1, 32 x 256 32.7 | 29.4.
