@@ -890,6 +890,24 @@ int gbx_dense_forward(const void* x, const void* w, const void* bias, void* y, i
   return GBX_OK;
 }
 
+int gbx_dense_forward_multi(const void* x, int32_t mats, const void* const* w, const void* const* bias, void* const* y, const int32_t* N, int64_t M, int32_t K,
+                            int32_t act_dtype, void* hip_stream) {
+  if (act_dtype != GBX_F16 && act_dtype != GBX_BF16) return fail(GBX_ERR_INVALID, "act_dtype must be GBX_F16 or GBX_BF16");
+  if (mats < 1 || mats > 3 || !w || !bias || !y || !N) return fail(GBX_ERR_INVALID, "one to three matrices (got %d) with their pointers and row counts", mats);
+  if (M < 0 || K <= 0) return fail(GBX_ERR_INVALID, "bad shape M=%lld K=%d", (long long)M, K);
+  if (M == 0) return GBX_OK;
+  if (!x || !aligned(x, 16)) return fail(GBX_ERR_INVALID, "x must be a 16-byte aligned device pointer");
+  for (int g = 0; g < mats; ++g) {
+    if (N[g] <= 0 || !w[g] || !y[g]) return fail(GBX_ERR_INVALID, "matrix %d: bad row count %d or null device pointer", g, N[g]);
+    if (!aligned(w[g], 16) || !aligned(y[g], (N[g] % 8) == 0 ? 16 : 2)) return fail(GBX_ERR_INVALID, "matrix %d: w must be 16-byte aligned (and y too when N %% 8 == 0)", g);
+    if (M > 2147483647LL || !gbx::gemm_dense_supported(static_cast<int>(M), N[g], K))
+      return fail(GBX_ERR_UNSUPPORTED, "dense matrix-core GEMM needs K %% 64 == 0 and M*K, N*K < 2^30 elements (M=%lld N=%d K=%d)", (long long)M, N[g], K);
+  }
+  const hipError_t e = gbx::launch_gemm_dense_multi(x, mats, w, bias, y, N, static_cast<int>(M), K, act_dtype == GBX_BF16, static_cast<hipStream_t>(hip_stream));
+  if (e != hipSuccess) return hip_fail(e, "gbx_dense_forward_multi launch");
+  return GBX_OK;
+}
+
 int gbx_dense_swiglu_forward(const void* x, const void* w_gate_up, void* y, int64_t M, int32_t N, int32_t K, int32_t act_dtype,
                              void* hip_stream) {
   if (act_dtype != GBX_F16 && act_dtype != GBX_BF16) return fail(GBX_ERR_INVALID, "act_dtype must be GBX_F16 or GBX_BF16");

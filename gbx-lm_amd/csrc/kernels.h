@@ -48,6 +48,8 @@ hipError_t launch_qgemm_mfma(const void* x, const uint32_t* qw, const void* sc, 
                              int M, int N, int K, int bits, int log2g, bool bf16, hipStream_t s, float* ws = nullptr);
 size_t qgemm_batch_workspace_bytes(int M, int N, int K, int bits, int log2g);
 bool gemm_dense_supported(int M, int N, int K);
+// the same GEMM for up to three matrices of one x in one launch (mfma_dense.hip)
+hipError_t launch_gemm_dense_multi(const void* x, int mats, const void* const* w, const void* const* bias, void* const* y, const int* N, int M, int K, bool bf16, hipStream_t s);
 hipError_t launch_gemm_dense(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, bool bf16, hipStream_t s,
                              bool swiglu = false, float* part = nullptr);
 // k split of the dense GEMM for few-tile shapes (fp32 slices in caller scratch + the summing launch): slices (1: none) and scratch bytes

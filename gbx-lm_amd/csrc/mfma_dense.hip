@@ -44,6 +44,12 @@ struct DenseArgs2 {
   // (caller scratch) and a second launch sums the slices, adds the bias and rounds (launch_splitk_finish)
   float* part;
   int ksplit;
+  // up to two more matrices of the same x (q, k and v of a block): their tile columns follow the first one's, each matrix starts a column of its own.  Alone, k and v
+  // are 48 tiles each at 3001 rows x 1024 outputs: split over k and summed by a second launch, 36 us each beside q's 55; together 74 (1.28 PFLOP/s).
+  int nseg;                    // 0 or 1: one matrix
+  const unsigned short *w_x[2], *bias_x[2];
+  unsigned short* y_x[2];
+  int N_x[2];
 };
 
 // Tiles of 32 RT x 64 CT: a wave owns 16 RT rows and 16 CT columns; of an operand with 192 rows a tile (RT = 6, CT = 3) the second request is 64 rows.
@@ -64,23 +70,36 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave >> 2, wcn = wave & 3;          // wave row (M half) / wave column (64 of the 256 N)
-  const int M = a.M, N = a.N, K = a.K;
+  const int M = a.M, K = a.K;
+  int N = a.N;
+  const unsigned short *w = a.w, *bias = a.bias;
+  unsigned short* y = a.y;
   const int ksplit = a.part ? a.ksplit : 1;
   const int nk = K / DK / ksplit;                    // K tiles of this workgroup's slice
 
   // XCD-aware tile order (as mfma_gemm.hip): every XCD walks a contiguous run of (tile, k slice) units, M-tile major
-  const int tiles_n = (N + TN - 1) / TN, tiles_m = (M + TM - 1) / TM, tiles = tiles_m * tiles_n * ksplit;
+  const int cols0 = (N + TN - 1) / TN, cols1 = a.nseg > 1 ? (a.N_x[0] + TN - 1) / TN : 0, cols2 = a.nseg > 2 ? (a.N_x[1] + TN - 1) / TN : 0;
+  const int tiles_n = cols0 + cols1 + cols2, tiles_m = (M + TM - 1) / TM, tiles = tiles_m * tiles_n * ksplit;
   const int per_xcd = (tiles + 7) / 8;
   const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (unit >= tiles) return;
   const int tile = unit / ksplit, kslice = unit % ksplit;
-  const int m0 = (tile / tiles_n) * TM, n0 = (tile % tiles_n) * TN;
+  int col = tile % tiles_n;
+  if (col >= cols0) {                                // (uniform) a further matrix
+    const int g = col >= cols0 + cols1;
+    col -= g ? cols0 + cols1 : cols0;
+    N = a.N_x[g];
+    w = a.w_x[g];
+    bias = a.bias_x[g];
+    y = a.y_x[g];
+  }
+  const int m0 = (tile / tiles_n) * TM, n0 = col * TN;
   const int kbase = kslice * nk * (DK * 2);          // byte offset of the slice inside a row
 
   // ---- DMA side: piece p = tid + 512 i (i = 0, 1) of a half-tile = (row p >> 3, 16-byte column p & 7); LDS linear, the
   // swizzle on the source column: slot (row, c) holds logical column c ^ ((row >> 1) & 7)
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(a.x), 0, 0x7FFFFFFF, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(a.w), 0, 0x7FFFFFFF, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(w), 0, 0x7FFFFFFF, 0x00020000);
   int voa[2][2], vob[2][2];                          // [half][i] byte offsets of this lane's pieces at k = 0
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -240,13 +259,13 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int n = min(nb + ct * 16 + fr, N - 1);
-    const float b = a.bias ? act_to_f32<BF16>(a.bias[n]) : 0.f;
+    const float b = bias ? act_to_f32<BF16>(bias[n]) : 0.f;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {                  // C/D layout of the 16x16 tile: row = 4 (lane >> 4) + e, column = lane & 15
         float v = acc[rt][ct][e];
-        if (a.bias) v = act_to_f32<BF16>(f32_to_act<BF16>(v)) + b;
+        if (bias) v = act_to_f32<BF16>(f32_to_act<BF16>(v)) + b;
         *reinterpret_cast<unsigned short*>(et + (rt * 16 + 4 * fk + e) * EROW + (ct * 16 + fr) * 2) = f32_to_act<BF16>(v);
       }
   }
@@ -277,7 +296,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
         o[j] = static_cast<unsigned>(f32_to_act<BF16>(s0 * act_lo<BF16>(uw[j]))) |
                (static_cast<unsigned>(f32_to_act<BF16>(s1 * act_hi<BF16>(uw[j]))) << 16);
       }
-      *reinterpret_cast<u32x4*>(a.y + static_cast<size_t>(m) * NO + ob + c * 8) = u32x4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<u32x4*>(y + static_cast<size_t>(m) * NO + ob + c * 8) = u32x4{o[0], o[1], o[2], o[3]};
     }
     return;
   }
@@ -288,7 +307,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseArgs2 a) {
     const int m = mb + row;
     if (m >= M) continue;
     const u32x4 v = *reinterpret_cast<const u32x4*>(et + row * EROW + c * 16);
-    unsigned short* dst = a.y + static_cast<size_t>(m) * N + nb + c * 8;
+    unsigned short* dst = y + static_cast<size_t>(m) * N + nb + c * 8;
     if (full_n) {
       *reinterpret_cast<u32x4*>(dst) = v;
     } else {
@@ -421,7 +440,9 @@ hipError_t launch_dense_tiles(const DenseArgs2& a, bool bf16, hipStream_t s) {
     if (e != hipSuccess) return e;
     once.done();
   }
-  const int tiles = ((a.N + Shape::TN - 1) / Shape::TN) * ((a.M + Shape::TM - 1) / Shape::TM) * (a.part ? a.ksplit : 1);
+  int cols = (a.N + Shape::TN - 1) / Shape::TN;
+  for (int g = 1; g < a.nseg; ++g) cols += (a.N_x[g - 1] + Shape::TN - 1) / Shape::TN;
+  const int tiles = cols * ((a.M + Shape::TM - 1) / Shape::TM) * (a.part ? a.ksplit : 1);
   dim3 grid(8 * ((tiles + 7) / 8)), block(512);
   if (bf16) hipLaunchKernelGGL((gemm_dense_kernel<true, RT, CT>), grid, block, Shape::LDS, s, a);
   else hipLaunchKernelGGL((gemm_dense_kernel<false, RT, CT>), grid, block, Shape::LDS, s, a);
@@ -432,18 +453,25 @@ hipError_t launch_dense_tiles(const DenseArgs2& a, bool bf16, hipStream_t s) {
 // 0.62 + 0.38 n / 256 of a full one (what is alone on the chip runs faster).  Every output sums its products in the same order in all four.  Measured, us, 256 x 256 | 256 x 192 |
 // 192 x 256 | 192 x 192: 3001 x 3072, K 3072 69 | 60 | 60 | 55, K 8192 173 | 160 | 161 | 152; 3001 x 5120, K 3072 82 | 115 | 109 | 110; 6000 x 4096, K 4096 171 | 214 |
 // 158 | 191; 6000 x 3072, K 8192 315 | 267 | 270 | 249; 2048 x 6144, K 4096 90 | 84 | 136 | 123; 2500 x 28672, K 4096 488 | 512 | 561 | 607.
-int gemm_dense_shape(int M, int N, bool swiglu) {
+int gemm_dense_shape(int M, const int* N, int mats, bool swiglu) {
   constexpr float cost[4] = {1.f, 0.8f, 0.8f, 0.66f};                    // 256 x 256, 256 x 192, 192 x 256, 192 x 192
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < 4; ++i) {
     if (swiglu && (i & 1)) continue;                                     // (gate and up meet in tiles of 256 columns)
     const int tm = i & 2 ? 192 : 256, tn = i & 1 ? 192 : 256;
-    const long long tiles = static_cast<long long>((N + tn - 1) / tn) * ((M + tm - 1) / tm), rest = tiles % 256;
+    long long cols = 0;
+    for (int g = 0; g < mats; ++g) cols += (N[g] + tn - 1) / tn;
+    const long long tiles = cols * ((M + tm - 1) / tm), rest = tiles % 256;
     const float t = cost[i] * (tiles / 256 + (rest ? 0.62f + 0.38f * rest / 256 : 0.f));
     if (i == 0 || t < least) { best = i; least = i == 0 ? 0.97f * t : t; }  // (what gains less than three in a hundred is not sure to gain)
   }
   return best;
+}
+
+hipError_t launch_dense_shape(const DenseArgs2& a, int shape, bool bf16, hipStream_t s) {
+  return shape == 0 ? launch_dense_tiles<8, 4>(a, bf16, s) : shape == 1 ? launch_dense_tiles<8, 3>(a, bf16, s)
+         : shape == 2 ? launch_dense_tiles<6, 4>(a, bf16, s) : launch_dense_tiles<6, 3>(a, bf16, s);
 }
 
 template <int NWV>
@@ -495,17 +523,28 @@ hipError_t launch_gemm_dense(const void* x, const void* w, const void* bias, voi
   static const bool skinny = env_switch("GBX_DENSE_SKINNY") != 0;
   if (skinny && !swiglu && M <= 32 && K % SK == 0 && N >= 128 * 256) {        // a stream of weight rows: one pass, no padding rows
     DenseArgs2 a{static_cast<const unsigned short*>(x), static_cast<const unsigned short*>(w), static_cast<const unsigned short*>(bias),
-                 static_cast<unsigned short*>(y), M, N, K, 0, nullptr, 1};
+                 static_cast<unsigned short*>(y), M, N, K, 0, nullptr, 1, 1, {}, {}, {}, {}};
     return launch_dense_batch(a, bf16, s);
   }
   const int ksplit = (part && !swiglu && N % 4 == 0) ? gemm_dense_ksplit(M, N, K) : 1;
   DenseArgs2 a{static_cast<const unsigned short*>(x), static_cast<const unsigned short*>(w), static_cast<const unsigned short*>(bias),
-               static_cast<unsigned short*>(y), M, N, K, swiglu ? 1 : 0, ksplit > 1 ? part : nullptr, ksplit};
-  const int shape = ksplit > 1 ? 0 : gemm_dense_shape(M, N, swiglu);
-  const hipError_t e = shape == 0 ? launch_dense_tiles<8, 4>(a, bf16, s) : shape == 1 ? launch_dense_tiles<8, 3>(a, bf16, s)
-                     : shape == 2 ? launch_dense_tiles<6, 4>(a, bf16, s) : launch_dense_tiles<6, 3>(a, bf16, s);
+               static_cast<unsigned short*>(y), M, N, K, swiglu ? 1 : 0, ksplit > 1 ? part : nullptr, ksplit, 1, {}, {}, {}, {}};
+  const int shape = ksplit > 1 ? 0 : gemm_dense_shape(M, &N, 1, swiglu);
+  const hipError_t e = launch_dense_shape(a, shape, bf16, s);
   if (e != hipSuccess || ksplit <= 1) return e;
   return launch_splitk_finish(part, static_cast<const unsigned short*>(bias), static_cast<unsigned short*>(y), ksplit, M, N, bf16, s);
+}
+
+hipError_t launch_gemm_dense_multi(const void* x, int mats, const void* const* w, const void* const* bias, void* const* y, const int* N, int M, int K, bool bf16, hipStream_t s) {
+  DenseArgs2 a{static_cast<const unsigned short*>(x), static_cast<const unsigned short*>(w[0]), static_cast<const unsigned short*>(bias[0]),
+               static_cast<unsigned short*>(y[0]), M, N[0], K, 0, nullptr, 1, mats, {}, {}, {}, {}};
+  for (int g = 1; g < mats; ++g) {
+    a.w_x[g - 1] = static_cast<const unsigned short*>(w[g]);
+    a.bias_x[g - 1] = static_cast<const unsigned short*>(bias[g]);
+    a.y_x[g - 1] = static_cast<unsigned short*>(y[g]);
+    a.N_x[g - 1] = N[g];
+  }
+  return launch_dense_shape(a, gemm_dense_shape(M, N, mats, false), bf16, s);
 }
 
 }  // namespace gbx

@@ -362,6 +362,58 @@ def _pack_scales_zeros(mod, mod2=None) -> torch.Tensor:
     return out
 
 
+def _dense_image(mod, m: int, dtype: torch.dtype, device):
+    """The resident 16-bit image of a module's weight where ``quantized_matmul`` on ``m`` rows would multiply by it (256 rows on: one that is there already;
+    from 1024 rows on, where the dense path is the rule, built now); None: it would not."""
+    w, scales, zeros = src = mod.qweight, mod.scales, mod.zeros
+    n, k, bits, group_size = mod.output_dims, mod.input_dims, mod.bits, mod.group_size
+    if _dense_cache.budget < n * k * 2 or scales is None or scales.dtype != dtype or zeros.dtype != dtype or k % 64 or not all(t.is_cuda and t.is_contiguous() for t in src):
+        return None
+    L, ckey = _lib.lib(), (n, k, bits, group_size, dtype, device.index)
+    rule = (m >= 1024 and m <= 61440 and L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) >= n * k * 2
+            and 31 <= L.gbx_qlinear_kernel_id(m, n, k, bits, group_size, 1) <= 33)
+    if not rule and not 256 <= m < 4096:
+        return None
+    dense = _dense_cache.get(src, ckey)
+    if dense is None and rule:
+        dense = _alloc_dense((n, k), dtype, device)
+        if dense is not None:
+            _lib.check(L.gbx_dequantize(w.data_ptr(), scales.data_ptr(), zeros.data_ptr(), dense.data_ptr(), n, k, bits, group_size, _DT[dtype], _DT[dtype],
+                                        _stream_ptr(device)))
+            _dense_cache.put(src, ckey, dense)
+    return dense
+
+
+def quantized_matmul_prompt(x: torch.Tensor, mods) -> Optional[list]:
+    """[m(x) for m in mods] for the two or three QuantizedLinear modules that read a prompt's rows together (q, k and v), in ONE launch of the dense GEMM on
+    their resident images: k and v alone are a few tiles each.  None where one of them would not take that path (the caller then calls each)."""
+    from .models.quantized_linear_gba import QuantizedLinear
+    k = x.shape[-1]
+    m = x.numel() // k if k else 0
+    if not (x.is_cuda and m >= 256 and x.dtype in _DT and 2 <= len(mods) <= 3 and not torch.cuda.is_current_stream_capturing()
+            and all(type(q) is QuantizedLinear and q.input_dims == k and not q._forward_hooks and not q._forward_pre_hooks for q in mods)
+            and all(q.bias is None or (q.bias.dtype == x.dtype and q.bias.is_cuda and q.bias.is_contiguous()) for q in mods)):
+        return None
+    # A matrix of 176 tiles fills the chip by itself (and is not split over k there): one launch for all of such gains nothing.  Each alone, k split where that helps | one
+    # launch, us: 3072 + 1024 + 1024 outputs of 3072, 256 rows 59 | 42, 1024 81 | 46, 3001 118 | 74, 8000 234 | 209; 4096 + 1024 + 1024 of 4096, 1500 rows 118 | 72, 3001
+    # 155 | 137; three of 4096 x 4096, 1024 146 | 84, 2500 (160 tiles) 224 | 193, 3001 (192 tiles) 237 | 253, 8000 591 | 599.
+    if -(-m // 256) * min(-(-q.output_dims // 256) for q in mods) >= 176:
+        return None
+    images = [_dense_image(q, m, x.dtype, x.device) for q in mods]
+    if any(t is None for t in images):
+        return None
+    x2 = x.reshape(-1, k).contiguous()
+    ys = [x2.new_empty((m, q.output_dims)) for q in mods]
+    n = len(mods)
+    VP, I32 = ctypes.c_void_p * n, ctypes.c_int32 * n
+    rc = _lib.lib().gbx_dense_forward_multi(x2.data_ptr(), n, VP(*[t.data_ptr() for t in images]), VP(*[None if q.bias is None else q.bias.data_ptr() for q in mods]),
+                                            VP(*[y.data_ptr() for y in ys]), I32(*[q.output_dims for q in mods]), m, k, _DT[x.dtype], _stream_ptr(x.device))
+    if rc == _lib.GBX_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc)
+    return [y.reshape(*x.shape[:-1], q.output_dims) for y, q in zip(ys, mods)]
+
+
 def quantized_matmul_multi(x: torch.Tensor, mods, pre_norm=None) -> list:
     """[m(x) for m in mods] for 2-3 QuantizedLinear modules that share ``x`` (q/k/v, gate/up) -- ONE launch of the
     split-K matrix-core kernel when the batch is decode-sized (gbx_qlinear_forward_multi), else one call per module.
