@@ -890,7 +890,9 @@ int gbx_dense_forward(const void* x, const void* w, const void* bias, void* y, i
   return GBX_OK;
 }
 
-int gbx_dense_forward_multi(const void* x, int32_t mats, const void* const* w, const void* const* bias, void* const* y, const int32_t* N, int64_t M, int32_t K,
+// gbx_dense_forward (without a split of k) for one to three matrices w[g] [N[g], K] of ONE x in one launch, y[g] [M, N[g]]: the q, k and v of a block, of which k and v alone
+// are too few tiles for the chip.  bias: an array, its entries null where a matrix has none.  For this package's own Python layer; not part of the public header.
+extern "C" int gbx_dense_forward_multi(const void* x, int32_t mats, const void* const* w, const void* const* bias, void* const* y, const int32_t* N, int64_t M, int32_t K,
                             int32_t act_dtype, void* hip_stream) {
   if (act_dtype != GBX_F16 && act_dtype != GBX_BF16) return fail(GBX_ERR_INVALID, "act_dtype must be GBX_F16 or GBX_BF16");
   if (mats < 1 || mats > 3 || !w || !bias || !y || !N) return fail(GBX_ERR_INVALID, "one to three matrices (got %d) with their pointers and row counts", mats);

@@ -428,11 +428,6 @@ size_t gbx_dense_workspace_bytes(int64_t M, int32_t N, int32_t K);
 int gbx_dense_forward_ws(const void* x, const void* w, const void* bias, void* y, int64_t M, int32_t N, int32_t K, int32_t act_dtype,
                          void* workspace, size_t workspace_bytes, void* hip_stream);
 
-/* The same GEMM (without a split of k) for one to three matrices w[g] [N[g], K] of ONE x in one launch, y[g] [M, N[g]]: the q, k and v of a block, of which k and v
- * alone are too few tiles for the chip.  bias: an array, its entries null where a matrix has none. */
-int gbx_dense_forward_multi(const void* x, int32_t mats, const void* const* w, const void* const* bias, void* const* y, const int32_t* N, int64_t M, int32_t K,
-                            int32_t act_dtype, void* hip_stream);
-
 /* The same GEMM over TWO matrices in one dense image with the SwiGLU in its epilogue: w_gate_up [2 * N, K] holds gate rows and up
  * rows in alternating blocks of 128 (rows [256 t, 256 t + 128) = gate rows [128 t, +128), the next 128 = the same up rows -- the
  * image gbx_qlinear_swiglu_forward_ws leaves in its workspace, which a caller may keep and reuse); y [M, N] = silu(x . gate^T) *
