@@ -111,7 +111,8 @@ class _DecodeGraph:
         self.batch = StepBatch(list(slots), [0] * b, [1] * b, b, i32[2 * b:6 * b].view(b, 4), i32[6 * b:8 * b].view(b, 2), 128,
                                i32[8 * b:10 * b].view(b, 2))
         self.graph = None
-        self.logits = None
+        self.logits = None                               # rows of the output head (``BatchScheduler._head``)
+        self.at: Optional[List[int]] = None              # positions that the static tables hold
 
     def fill(self, tokens: Sequence[int], pos0: Sequence[int]) -> None:
         k = self.turn % 2
@@ -125,14 +126,22 @@ class _DecodeGraph:
         seq_pos[:] = tok_pos[:] = pos0
         self.static.copy_(self.pinned[k], non_blocking=True)
         self.copied[k].record(torch.cuda.current_stream(self.static.device))
-        self.batch.pos0 = list(pos0)
+        self.batch.pos0 = self.at = list(pos0)
+
+    def advance(self, tokens: torch.Tensor) -> None:
+        """The next token of every sequence, from the device: one small launch instead of a copy from the host that has read them there first."""
+        from . import _lib, ops
+        b = len(self.slots)
+        _lib.check_mixers(_lib.mixers().gbxm_step_advance(tokens.data_ptr(), tokens.element_size(), self.static.data_ptr(), self.batch.seq.data_ptr(),
+                                                          self.batch.tok.data_ptr(), b, ops._stream_ptr(self.static.device)))
+        self.batch.pos0 = self.at = [p + 1 for p in self.at]
 
     def run(self, sched: "BatchScheduler") -> torch.Tensor:
         if self.graph is None:
             torch.cuda.synchronize(sched.device)
             g = torch.cuda.CUDAGraph()
             with graphs.capture(g):
-                self.logits = sched.model.logits(sched.model.forward_tokens(self.tokens, self.batch, sched.caches))
+                self.logits = sched._head(sched.model.forward_tokens(self.tokens, self.batch, sched.caches))
             self.graph = g
         self.graph.replay()
         return self.logits
@@ -157,6 +166,18 @@ class BatchScheduler:
         self._seen: Dict[Tuple[int, ...], int] = {}
         self._buffers = None
 
+    def _whole_head(self) -> bool:
+        """Whether a model's logits are ``finish_logits`` of ``head_rows``, which then may be finished where they are read."""
+        from .models.step_model import RaggedStepModel as R
+        m, t = self.model, type(self.model)
+        return (isinstance(m, R) and t.logits is R.logits and t.finish_logits is R.finish_logits and not {"logits", "finish_logits"} & vars(m).keys())
+
+    def _head(self, hidden: torch.Tensor) -> torch.Tensor:
+        return self.model.head_rows(hidden) if self._whole_head() else self.model.logits(hidden)
+
+    def _finish(self, rows: torch.Tensor) -> torch.Tensor:
+        return self.model.finish_logits(rows) if self._whole_head() else rows
+
     def position(self, seq_id) -> int:
         return self.slots.length[self.slot_of[seq_id]]
 
@@ -170,8 +191,9 @@ class BatchScheduler:
         [wanted, vocab]."""
         return self._step(entries, want)
 
-    def _step(self, entries, want=None, keep: bool = True) -> torch.Tensor:
-        """``keep`` False: the caller is done with the logits before the next step, whose replay may overwrite them."""
+    def _step(self, entries, want=None, raw: bool = False) -> torch.Tensor:
+        """``raw``: the output head's rows as they are, of every entry's last token; the caller finishes them and is done with them before the next step, whose
+        replay may overwrite them."""
         if not entries:
             return torch.empty((0, 0))
         new_tokens = sum(len(t) for _, t in entries)
@@ -190,13 +212,16 @@ class BatchScheduler:
             if logits is not None:
                 for s in slot:
                     self.slots.length[s] += 1
+                if raw:
+                    return logits
+                buffer, logits = logits, self._finish(logits)
                 rows = [i for i in range(len(slot)) if want is None or len(want[i])]
                 if any(p != 0 for i in rows if want is not None for p in want[i]):
                     raise ValueError("a wanted place lies outside the entry's tokens")
                 if not rows:
                     return torch.empty((0, self.model.args.vocab), dtype=torch.float32, device=self.device)
                 if len(rows) == len(slot):
-                    return logits.float() if logits.dtype != torch.float32 else logits.clone() if keep else logits      # (the graph's buffer is overwritten by the next replay)
+                    return logits.float() if logits.dtype != torch.float32 else logits.clone() if logits is buffer else logits      # (the graph's buffer is overwritten by the next replay)
                 return logits.index_select(0, torch.tensor(rows, dtype=torch.long, device=self.device)).float()
         batch = StepBatch.build(slot, pos0, n_new, self.device)
         try:
@@ -222,11 +247,11 @@ class BatchScheduler:
         if not rows:
             return torch.empty((0, self.model.args.vocab), dtype=torch.float32, device=self.device)
         idx = torch.tensor(rows, dtype=torch.long, device=self.device)
-        return self.model.logits(hidden.index_select(0, idx)).float()
+        out = self._head(hidden.index_select(0, idx))
+        return out if raw else self._finish(out).float()
 
-    def _graph_step(self, slots: Tuple[int, ...], tokens: Sequence[int], pos0: Sequence[int]) -> Optional[torch.Tensor]:
-        """Replay (or, at the third step of this set of slots, capture) the decode graph; None: run the step eagerly."""
-        longest = max(pos0) + 1
+    def _current_graph(self, slots: Tuple[int, ...], longest: int) -> Optional["_DecodeGraph"]:
+        """The captured step of these slots, dropped with all others where a table it reads has moved."""
         for c in self.caches:                            # tables without a window grow on the host, never inside a replay
             if hasattr(c, "ensure"):
                 c.ensure(longest)
@@ -236,9 +261,37 @@ class BatchScheduler:
             self._graphs.clear()
             self._seen.clear()
             self._buffers = buffers
-        if 0 in buffers:
+        return self._graphs.get(slots)
+
+    def _step_ahead(self, ids: Sequence[object], tokens: torch.Tensor):
+        """The next step of the sequences ``ids``, enqueued before the host has seen their tokens: (the tokens on their way to the host, the event behind that copy,
+        the output head's rows), or None where that step has to be laid out on the host."""
+        if not (self.use_graphs and 0 < len(ids) <= 256 and isinstance(tokens, torch.Tensor) and tokens.device == self.device and tokens.dtype in (torch.int64, torch.int32)
+                and tokens.numel() == len(ids) and all(i in self.slot_of for i in ids)):
             return None
-        g = self._graphs.get(slots)
+        if self.max_tokens is not None and self.slots.live_tokens() + len(ids) > self.max_tokens:
+            return None
+        slots = tuple(self.slot_of[i] for i in ids)
+        at = [self.slots.length[s] - 1 for s in slots]
+        g = self._current_graph(slots, max(at) + 2)
+        if g is None or g.graph is None or g.at != at:
+            return None
+        tokens = tokens.contiguous()
+        host = torch.empty((len(ids),), dtype=tokens.dtype, pin_memory=True)
+        host.copy_(tokens, non_blocking=True)
+        there = torch.cuda.Event()
+        there.record(torch.cuda.current_stream(self.device))
+        g.advance(tokens)
+        rows = g.run(self)
+        for s in slots:
+            self.slots.length[s] += 1
+        return host, there, rows
+
+    def _graph_step(self, slots: Tuple[int, ...], tokens: Sequence[int], pos0: Sequence[int]) -> Optional[torch.Tensor]:
+        """Replay (or, at the third step of this set of slots, capture) the decode graph; None: run the step eagerly."""
+        g = self._current_graph(slots, max(pos0) + 1)
+        if 0 in self._buffers:
+            return None
         if g is None:
             self._seen[slots] = self._seen.get(slots, 0) + 1
             if self._seen[slots] < 3:
@@ -264,20 +317,37 @@ class BatchScheduler:
         out: List[List[int]] = [[] for _ in prompts]
         live = list(range(len(prompts)))
         feed = {i: list(prompts[i]) for i in live}
+        rows = None                                     # the output head's rows of a step that is under way already
         while live:
-            entries = [(ids[i], feed[i]) for i in live]
-            # log-probabilities are a tensor of their own: the plain step's logits need not outlive its next replay.  A step that someone put in its place is called as it is.
+            # log-probabilities are a tensor of their own: the plain step's rows need not outlive its next replay.  A step that someone put in its place is called as it is.
             plain = getattr(self.step, "__func__", None) is _PLAIN_STEP
-            logprobs = log_probabilities(self._step(entries, keep=False) if plain else self.step(entries))
-            toks = sampler(logprobs).reshape(-1).tolist()
-            nxt = []
-            for i, t in zip(live, toks):
+            if plain:
+                rows = self._step([(ids[i], feed[i]) for i in live], raw=True) if rows is None else rows
+                whole = self._whole_head()
+                logprobs = log_probabilities(rows, (1.0 if self.model.logit_scale is None else self.model.logit_scale) if whole else 1.0)
+            else:
+                logprobs = log_probabilities(self.step([(ids[i], feed[i]) for i in live]))
+            toks = sampler(logprobs).reshape(-1)
+            # Where every sequence goes on, unless a token ends it, the next step is enqueued behind the tokens before the host reads them: the chip does not wait for the host's
+            # turn (some 40 us a step).  A sequence that a token has ended then has run one step too many, in a slot that is given back.
+            ahead = self._step_ahead([ids[i] for i in live], toks) if plain and all(len(out[i]) + 1 < max_tokens for i in live) else None
+            if ahead is None:
+                values, rows = toks.tolist(), None
+            else:
+                host, there, rows = ahead
+                there.synchronize()
+                values = host.tolist()
+            nxt, kept = [], []
+            for at, (i, t) in enumerate(zip(live, values)):
                 out[i].append(int(t))
                 if int(t) in stop or len(out[i]) >= max_tokens:
                     self.release(ids[i])
                 else:
                     feed[i] = [int(t)]
                     nxt.append(i)
+                    kept.append(at)
+            if rows is not None and len(kept) < len(live) and kept:
+                rows = rows.index_select(0, torch.tensor(kept, dtype=torch.long, device=rows.device))
             live = nxt
         return out
 

@@ -91,28 +91,28 @@ template <typename T> __device__ __forceinline__ int lsm_step(int vec) { return 
 template <typename T> __device__ __forceinline__ int lsm_first(int vec) { return blockIdx.x * LSM_SLICE + threadIdx.x * (lsm_step<T>(vec) == 1 ? 8 : 1); }
 
 template <typename T>
-__device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int n, int vec, float* v) {
+__device__ __forceinline__ void lsm_load8(const T* __restrict__ row, int k, int n, int vec, float scale, float* v) {
   if (vec) {                                                  // (n is a multiple of 8: all of them are in the row, or none)
     constexpr int PER = 16 / sizeof(T);
     uint4 u[8 / PER];
 #pragma unroll
     for (int i = 0; i < 8 / PER; ++i) u[i] = *reinterpret_cast<const uint4*>(row + min(k, n - 8) + i * PER);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = k < n ? lsm_get<T>(u[j / PER], j % PER) : -INFINITY;
+    for (int j = 0; j < 8; ++j) v[j] = k < n ? lsm_get<T>(u[j / PER], j % PER) * scale : -INFINITY;
   } else {
     const int step = lsm_step<T>(0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = k + j * step < n ? static_cast<float>(row[k + j * step]) : -INFINITY;
+    for (int j = 0; j < 8; ++j) v[j] = k + j * step < n ? static_cast<float>(row[k + j * step]) * scale : -INFINITY;
   }
 }
 
 // (maximum, sum of exponentials against it or against 0 where it is infinite) of one slice
 template <typename T>
-__global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n, int vec) {
+__global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restrict__ x, float2* __restrict__ part, int n, int vec, float scale) {
   __shared__ float top[4], red[4];
   const int k = lsm_first<T>(vec), step = lsm_step<T>(vec);
   float v[8], m = -INFINITY, s = 0.f;
-  lsm_load8(x + static_cast<int64_t>(blockIdx.y) * n, k, n, vec, v);
+  lsm_load8(x + static_cast<int64_t>(blockIdx.y) * n, k, n, vec, scale, v);
 #pragma unroll
   for (int j = 0; j < 8; ++j) m = fmaxf(m, v[j]);
 #pragma unroll
@@ -127,14 +127,14 @@ __global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restr
   if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = float2{m, s};
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, T* __restrict__ out, int n, int vec) {
+template <typename T, typename O>
+__global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restrict__ x, const float2* __restrict__ part, O* __restrict__ out, int n, int vec, float scale) {
   __shared__ float top[4], red[4];
   const float2* p = part + blockIdx.y * gridDim.x;
   const int parts = gridDim.x, k = lsm_first<T>(vec);
   const int64_t base = static_cast<int64_t>(blockIdx.y) * n;
   float v[8], m = -INFINITY, s = 0.f;
-  lsm_load8(x + base, k, n, vec, v);
+  lsm_load8(x + base, k, n, vec, scale, v);
   for (int i = threadIdx.x; i < parts; i += 256) m = fmaxf(m, p[i].x);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
@@ -145,32 +145,32 @@ __global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restr
   // (an infinite maximum: the slice's sum is 0, infinite or no number against any shift -- the shift's own exponential may be infinite, and 0 times that is
   // no number)
   for (int i = threadIdx.x; i < parts; i += 256) s += isinf(p[i].x) ? p[i].y : p[i].y * expf(p[i].x - shift);
-  const float lse = lsm_round<T>(logf(block_sum<4>(s, red)) + shift);
+  const float lse = lsm_round<O>(logf(block_sum<4>(s, red)) + shift);
   if (vec) {
     if (k >= n) return;
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (sizeof(O) == 4) {
       float* o = reinterpret_cast<float*>(out) + base + k;
 #pragma unroll
       for (int i = 0; i < 2; ++i) *reinterpret_cast<float4*>(o + 4 * i) = float4{v[4 * i] - lse, v[4 * i + 1] - lse, v[4 * i + 2] - lse, v[4 * i + 3] - lse};
     } else {
       unsigned w[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = static_cast<unsigned>(lsm_bits<T>(v[2 * j] - lse)) | (static_cast<unsigned>(lsm_bits<T>(v[2 * j + 1] - lse)) << 16);
+      for (int j = 0; j < 4; ++j) w[j] = static_cast<unsigned>(lsm_bits<O>(v[2 * j] - lse)) | (static_cast<unsigned>(lsm_bits<O>(v[2 * j + 1] - lse)) << 16);
       *reinterpret_cast<uint4*>(out + base + k) = uint4{w[0], w[1], w[2], w[3]};
     }
   } else {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (k + j * lsm_step<T>(0) < n) out[base + k + j * lsm_step<T>(0)] = static_cast<T>(v[j] - lse);
+      if (k + j * lsm_step<T>(0) < n) out[base + k + j * lsm_step<T>(0)] = static_cast<O>(v[j] - lse);
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict__ x, T* __restrict__ out, int n, int vec) {
+template <typename T, typename O>
+__global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict__ x, O* __restrict__ out, int n, int vec, float scale) {
   constexpr int PER = 16 / sizeof(T), NWV = LSM_NT / 64;
   __shared__ float red[NWV];
   const T* row = x + static_cast<int64_t>(blockIdx.x) * n;
-  T* orow = out + static_cast<int64_t>(blockIdx.x) * n;
+  O* orow = out + static_cast<int64_t>(blockIdx.x) * n;
   const int nv = vec ? n / PER : 0;                          // whole 16-byte pieces; the rest (all of it where rows are not aligned) one by one
   const uint4* rv = reinterpret_cast<const uint4*>(row);
   const int tid = threadIdx.x;
@@ -182,15 +182,15 @@ __global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict
     if (k < nv) {
       v[i] = rv[k];
 #pragma unroll
-      for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(v[i], j));
+      for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(v[i], j) * scale);
     }
   }
   for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) {
     const uint4 u = rv[k];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(u, j));
+    for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(u, j) * scale);
   }
-  for (int k = nv * PER + tid; k < n; k += LSM_NT) m = fmaxf(m, static_cast<float>(row[k]));
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) m = fmaxf(m, static_cast<float>(row[k]) * scale);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   if ((tid & 63) == 0) red[tid >> 6] = m;
@@ -203,34 +203,36 @@ __global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict
   for (int i = 0; i < LSM_VR; ++i)
     if (tid + i * LSM_NT < nv) {
 #pragma unroll
-      for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(v[i], j) - m);
+      for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(v[i], j) * scale - m);
     }
   for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) {
     const uint4 u = rv[k];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(u, j) - m);
+    for (int j = 0; j < PER; ++j) s += expf(lsm_get<T>(u, j) * scale - m);
   }
-  for (int k = nv * PER + tid; k < n; k += LSM_NT) s += expf(static_cast<float>(row[k]) - m);
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) s += expf(static_cast<float>(row[k]) * scale - m);
   s = block_sum<NWV>(s, red);
-  const float lse = lsm_round<T>(logf(s) + m);
+  const float lse = lsm_round<O>(logf(s) + m);
   auto put = [&](int k, const uint4& u) {
-    uint4 r;
-    unsigned* w = &r.x;
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (sizeof(O) == 4) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = __float_as_uint(lsm_get<T>(u, j) - lse);
+      for (int i = 0; i < PER; i += 4)
+        reinterpret_cast<float4*>(orow)[(k * PER + i) / 4] = float4{lsm_get<T>(u, i) * scale - lse, lsm_get<T>(u, i + 1) * scale - lse, lsm_get<T>(u, i + 2) * scale - lse,
+                                                                    lsm_get<T>(u, i + 3) * scale - lse};
     } else {
+      uint4 r;
+      unsigned* w = &r.x;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        w[j] = static_cast<unsigned>(lsm_bits<T>(lsm_get<T>(u, 2 * j) - lse)) | (static_cast<unsigned>(lsm_bits<T>(lsm_get<T>(u, 2 * j + 1) - lse)) << 16);
+        w[j] = static_cast<unsigned>(lsm_bits<O>(lsm_get<T>(u, 2 * j) * scale - lse)) | (static_cast<unsigned>(lsm_bits<O>(lsm_get<T>(u, 2 * j + 1) * scale - lse)) << 16);
+      reinterpret_cast<uint4*>(orow)[k] = r;
     }
-    reinterpret_cast<uint4*>(orow)[k] = r;
   };
 #pragma unroll
   for (int i = 0; i < LSM_VR; ++i)
     if (tid + i * LSM_NT < nv) put(tid + i * LSM_NT, v[i]);
   for (int k = tid + LSM_VR * LSM_NT; k < nv; k += LSM_NT) put(k, rv[k]);
-  for (int k = nv * PER + tid; k < n; k += LSM_NT) orow[k] = static_cast<T>(static_cast<float>(row[k]) - lse);
+  for (int k = nv * PER + tid; k < n; k += LSM_NT) orow[k] = static_cast<O>(static_cast<float>(row[k]) * scale - lse);
 }
 
 // The tables of a step's rows and query tiles, from its sequences' (slot, first position, rows, first row) and first tiles.  Written on the host, entry by entry, they kept the
@@ -257,21 +259,33 @@ __global__ __launch_bounds__(256) void step_tables_kernel(const int* __restrict_
   }
 }
 
-template <typename T>
-void launch_log_softmax(const void* x, void* out, int64_t rows, int n, float* part, hipStream_t s) {
+// The tokens of the next step of the same sequences, from where they were chosen, and every position one further: what a step needs that is enqueued before the host has
+// read them.  A step of the 4-layer models in batching.py's loop, us, tokens through the host | ahead of it: one sequence, several streams of 1024 244 | 219; two, latent attention 387 |
+// 362; 32, sandwich norms 1124 | 1080 (a replay of the step alone: 200, 332 and 1043).
+template <typename I>
+__global__ __launch_bounds__(256) void step_advance_kernel(const I* __restrict__ from, int64_t* __restrict__ tokens, int* __restrict__ seq, int* __restrict__ tok, int B) {
+  const int b = threadIdx.x;
+  if (b >= B) return;
+  tokens[b] = from[b];
+  seq[4 * b + 1] += 1;
+  tok[2 * b + 1] += 1;
+}
+
+template <typename T, typename O = T>
+void launch_log_softmax(const void* x, void* out, int64_t rows, int n, float* part, float scale, hipStream_t s) {
   constexpr int PER = 16 / sizeof(T);
   const T* xt = static_cast<const T*>(x);
-  T* ot = static_cast<T*>(out);
+  O* ot = static_cast<O*>(out);
   const bool aligned = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   if (part) {
     const dim3 grid((n + LSM_SLICE - 1) / LSM_SLICE, static_cast<unsigned>(rows));
     const int vec = aligned && n % 8 == 0;
-    log_softmax_slice_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<float2*>(part), n, vec);
-    log_softmax_write_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<const float2*>(part), ot, n, vec);
+    log_softmax_slice_kernel<T><<<grid, 256, 0, s>>>(xt, reinterpret_cast<float2*>(part), n, vec, scale);
+    log_softmax_write_kernel<T, O><<<grid, 256, 0, s>>>(xt, reinterpret_cast<const float2*>(part), ot, n, vec, scale);
     return;
   }
   const int vec = aligned && (rows == 1 || n % PER == 0);
-  log_softmax_kernel<T><<<static_cast<unsigned>(rows), LSM_NT, 0, s>>>(xt, ot, n, vec);
+  log_softmax_kernel<T, O><<<static_cast<unsigned>(rows), LSM_NT, 0, s>>>(xt, ot, n, vec, scale);
 }
 
 template <typename T>
@@ -659,16 +673,33 @@ extern "C" size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n) {
 }
 
 extern "C" int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream) {
-  if (rows < 0 || n <= 0 || (type != GBXM_BF16 && type != GBXM_F32 && type != GBXM_F16) || rows > 0x7fffffff) return fail(GBXM_ERR_INVALID, "log_softmax: bad argument");
+  return gbxm_log_softmax_scaled(x, out, rows, n, type, type, 1.f, ws, ws_bytes, stream);
+}
+
+extern "C" int gbxm_log_softmax_scaled(const void* x, void* out, int64_t rows, int32_t n, int32_t type, int32_t out_type, float scale, void* ws, size_t ws_bytes, void* stream) {
+  if (rows < 0 || n <= 0 || (type != GBXM_BF16 && type != GBXM_F32 && type != GBXM_F16) || (out_type != type && out_type != GBXM_F32) || rows > 0x7fffffff)
+    return fail(GBXM_ERR_INVALID, "log_softmax: bad argument");
   if (rows == 0) return GBXM_OK;
   const size_t need = gbxm_log_softmax_workspace(rows, n);
   if (!x || !out || (need && (!ws || ws_bytes < need || reinterpret_cast<uintptr_t>(ws) % 8))) return fail(GBXM_ERR_INVALID, "log_softmax: null pointer or workspace");
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* part = need ? static_cast<float*>(ws) : nullptr;
-  if (type == GBXM_F32) launch_log_softmax<float>(x, out, rows, n, part, s);
-  else if (type == GBXM_BF16) launch_log_softmax<__bf16>(x, out, rows, n, part, s);
-  else launch_log_softmax<_Float16>(x, out, rows, n, part, s);
+  if (type == GBXM_F32) launch_log_softmax<float>(x, out, rows, n, part, scale, s);
+  else if (type == GBXM_BF16 && out_type == GBXM_F32) launch_log_softmax<__bf16, float>(x, out, rows, n, part, scale, s);
+  else if (type == GBXM_BF16) launch_log_softmax<__bf16>(x, out, rows, n, part, scale, s);
+  else if (out_type == GBXM_F32) launch_log_softmax<_Float16, float>(x, out, rows, n, part, scale, s);
+  else launch_log_softmax<_Float16>(x, out, rows, n, part, scale, s);
   return after_launch("log_softmax");
+}
+
+extern "C" int gbxm_step_advance(const void* from, int32_t from_bytes, int64_t* tokens, int32_t* seq, int32_t* tok, int32_t B, void* stream) {
+  if (!from || !tokens || !seq || !tok || B < 1 || B > 256 || (from_bytes != 4 && from_bytes != 8) || reinterpret_cast<uintptr_t>(from) % from_bytes ||
+      reinterpret_cast<uintptr_t>(tokens) % 8 || (reinterpret_cast<uintptr_t>(seq) | reinterpret_cast<uintptr_t>(tok)) % 4)
+    return fail(GBXM_ERR_INVALID, "step_advance: bad argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (from_bytes == 8) step_advance_kernel<int64_t><<<1, 256, 0, s>>>(static_cast<const int64_t*>(from), tokens, seq, tok, B);
+  else step_advance_kernel<int><<<1, 256, 0, s>>>(static_cast<const int*>(from), tokens, seq, tok, B);
+  return after_launch("step_advance");
 }
 
 int gbxm_segment_rmsnorm(void* rows, int64_t T_, int64_t row_stride, int32_t n0, int32_t n1, const float* w0, const float* w1, float eps,

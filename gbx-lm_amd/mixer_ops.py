@@ -188,20 +188,22 @@ _EXPERT = {"silu": 1, "clamped_swish": 2, "relu2": 16}
 _LSM = {torch.bfloat16: _lib.GBXM_BF16, torch.float32: _lib.GBXM_F32, torch.float16: _lib.GBXM_F16}
 
 
-def log_probabilities(logits: torch.Tensor) -> torch.Tensor:
+def log_probabilities(logits: torch.Tensor, scale: Optional[float] = None) -> torch.Tensor:
     """``logits - logsumexp(logits)`` over the last axis, the logarithm formed in fp32 (fp64 for fp64) and rounded to the logits' dtype: one launch
-    on the GPU (two for a few long rows), torch elsewhere."""
+    on the GPU (two for a few long rows), torch elsewhere.  With ``scale`` (rows of an output head): of ``logits.float() * scale``, in fp32."""
     if not (logits.is_cuda and logits.dtype in _LSM and logits.numel() and outside_torch(logits)):
+        if scale is not None:
+            logits = logits.float() * scale if scale != 1.0 else logits.float()
         wide = logits if logits.dtype == torch.float64 else logits.float()
         return logits - torch.logsumexp(wide, dim=-1, keepdim=True).to(logits.dtype)
     x = logits.contiguous()
     n = x.shape[-1]
-    out = torch.empty_like(x)
+    out = torch.empty_like(x) if scale is None else torch.empty(x.shape, dtype=torch.float32, device=x.device)
     L, rows = _lib.mixers(), x.numel() // n
     need = L.gbxm_log_softmax_workspace(rows, n)
     ws = torch.empty((need,), dtype=torch.uint8, device=x.device) if need else None
-    _lib.check_mixers(L.gbxm_log_softmax(x.data_ptr(), out.data_ptr(), rows, n, _LSM[x.dtype], None if ws is None else ws.data_ptr(), need,
-                                         _stream(x.device)))
+    _lib.check_mixers(L.gbxm_log_softmax_scaled(x.data_ptr(), out.data_ptr(), rows, n, _LSM[x.dtype], _LSM[out.dtype], 1.0 if scale is None else float(scale),
+                                         None if ws is None else ws.data_ptr(), need, _stream(x.device)))
     return out
 
 

@@ -63,10 +63,19 @@ class RaggedStepModel(nn.Module):
     def forward_tokens(self, tokens: torch.Tensor, batch: StepBatch, caches) -> torch.Tensor:
         raise NotImplementedError
 
-    def logits(self, x: torch.Tensor) -> torch.Tensor:
-        """Last norm and output head on rows of the stream."""
+    logit_scale: Optional[float] = None     # applied to the output head's rows in fp32
+
+    def head_rows(self, x: torch.Tensor) -> torch.Tensor:
+        """Last norm and output head on rows of the stream: the logits before ``finish_logits``."""
         w = self.lm_head.weight
         return project(self.model.norm(x, w.dtype), w)
+
+    def finish_logits(self, rows: torch.Tensor) -> torch.Tensor:
+        return rows if self.logit_scale is None else rows.float() * self.logit_scale
+
+    def logits(self, x: torch.Tensor) -> torch.Tensor:
+        """Last norm, output head and the logit scale, if there is one, on rows of the stream."""
+        return self.finish_logits(self.head_rows(x))
 
     def _run(self, inputs: torch.Tensor, cache):
         b, l = inputs.shape

@@ -24,7 +24,6 @@ from ..batching import StepBatch
 from .base import BaseModelArgs
 from .cache import SequenceSlots
 from .feed_forward import GatedDenseFeedForward
-from .projection import project
 from .recurrent_mixers import ChannelDeltaRule, GatedLinearAttention
 from .residual import StreamLayerNorm, hyper_step_
 from .sink_attention import LatentAttention
@@ -164,11 +163,6 @@ class Model(RaggedStepModel):
             if self.trace_layers is not None:
                 self.trace_layers.append(streams.sum(1))
         return h
-
-    def logits(self, x: torch.Tensor) -> torch.Tensor:
-        """Last norm, output head and the logit scale (applied in fp32) on rows of the summed stream."""
-        w = self.lm_head.weight
-        return project(self.model.norm(x, w.dtype), w).float() * self.logit_scale
 
     @staticmethod
     def shapes_from(weights: Dict[str, torch.Tensor], config: Dict[str, Any]) -> Dict[int, Dict[str, int]]:

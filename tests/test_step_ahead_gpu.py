@@ -1,0 +1,83 @@
+"""Generation whose next step is enqueued before the host has read the tokens (BatchScheduler._step_ahead), and log-probabilities straight from the output head's rows."""
+import pytest
+import torch
+
+from gbx_lm_amd import synthetic as S
+from gbx_lm_amd.batching import BatchScheduler
+from gbx_lm_amd.mixer_ops import log_probabilities
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(name):
+    if name == "tugolix":
+        cfg = S.tugolix_config(width=256, delta=dict(heads=4, kv_heads=2, dim=64, vdim=64, conv=4), gla=dict(heads=2, dim=64, vdim=128, tau=16.0),
+                               latent=dict(heads=4, dim=64, vdim=64, kv_rank=128), ff=512, moe=dict(experts=8, top=2, ff=128, groups=(4, 2)), pattern="dgls")
+        return S.build_tugolix(cfg, device="cuda:0", seed=3), cfg["vocab"]
+    cfg = S.gibalorn_config(width=256, latent=dict(heads=4, dim=64, rot_dim=32, vdim=64, kv_rank=128, q_rank=128),
+                            mamba2=dict(heads=8, vdim=64, state=64, groups=1, conv=4, norm_groups=1), attention=dict(heads=4, kv_heads=2, dim=64, rot_dims=32),
+                            moe=dict(experts=8, top=2, ff=128), pattern="mla")
+    return S.build_gibalorn(cfg, device="cuda:0", seed=3), cfg["vocab"]
+
+
+@pytest.mark.parametrize("name", ["tugolix", "gibalorn"])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("stops", [{}, {1: 9}, {0: 8, 2: 8}, {0: 7, 1: 8, 2: 9}])
+def test_the_same_tokens_and_log_probabilities(name, dtype, stops):
+    """Odd numbers of sequences (tables off the grid of 16 bytes), sequences that a token ends at different steps and all at once; a continuation that the caller
+    supplies, so that both orders of host and device compute the same rows."""
+    model, vocab = _model(name)
+    steps, stop = 14, vocab - 1
+    gen = torch.Generator().manual_seed(5)
+    prompts = [torch.randint(0, stop, (n,), generator=gen).tolist() for n in (5, 1, 12)]
+    forced = torch.randint(0, stop, (steps, 3), generator=gen)
+    for seq, at in stops.items():
+        forced[at, seq] = stop
+    runs = []
+    for ahead in (True, False):
+        engine = BatchScheduler(model)
+        took = []
+        inner = engine._step_ahead
+
+        def counted(ids, toks):
+            got = inner(ids, toks) if ahead else None
+            took.append(got is not None)
+            return got
+
+        engine._step_ahead = counted
+        rows = []
+        for again in range(2):                                    # the second time replays what the first captured
+            live, n = [0, 1, 2], [0]
+
+            def sampler(lp):
+                row = forced[n[0], live].clone()
+                rows.append((list(live), lp))
+                live[:] = [i for i in live if forced[n[0], i] != stop]
+                n[0] += 1
+                return row.to("cuda:0", dtype)
+
+            out = engine.generate(prompts, max_tokens=steps, sampler=sampler, stop_tokens=[stop])
+            for i in range(3):
+                want = forced[:stops.get(i, steps - 1) + 1, i].tolist()
+                assert out[i] == want
+        assert any(took) == ahead
+        assert not engine.slot_of and all(v < 0 for v in engine.slots.length)      # every slot was given back
+        runs.append(rows)
+    assert len(runs[0]) == len(runs[1])
+    for (a, x), (b, y) in zip(*runs):
+        assert a == b and x.shape == y.shape
+        # bf16 activations: a step that still holds a sequence which has ended may take another kernel for its rows
+        assert (x - y).abs().max() <= 0.05 * y.std()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,n", [(1, 8), (1, 32000), (2, 24584), (3, 24579), (15, 30001), (16, 1003), (33, 8192), (1, 151936)])
+@pytest.mark.parametrize("scale", [1.0, 0.25, 3.0])
+def test_rows_of_the_head(dtype, rows, n, scale):
+    x = (torch.randn((rows, n), generator=torch.Generator(device="cuda").manual_seed(n + rows), device="cuda") * 4).to(dtype)
+    got = log_probabilities(x, scale)
+    assert got.dtype == torch.float32
+    y = x.double() * scale
+    want = y - torch.logsumexp(y, -1, keepdim=True)
+    # fp32: a product, a difference and a logarithm, each within an ulp of values up to 2^6; n exponentials sum to a relative 2^-24 sqrt(n) at most 2^-15
+    assert ((got.double() - want).abs() <= 2.0 ** -17 * want.abs().clamp(min=1.0) + 2.0 ** -15).all()
