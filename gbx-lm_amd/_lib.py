@@ -408,6 +408,30 @@ def build_mixers(force: bool = False, jobs: int = 8) -> str:
     return _MSO
 
 
+_host = None
+
+
+def host():
+    """The host side of small calls as a native module (csrc/host_linear.cpp), bound to the library's entry points; None where it is not built (it is compiled against one
+    torch and one interpreter), and the calls then go through ctypes."""
+    global _host
+    if _host is None:
+        _host = False
+        path = os.path.join(_CSRC, "_gbx_host.so")
+        if os.path.exists(path):
+            import importlib.util
+            L = lib()
+            spec = importlib.util.spec_from_file_location("_gbx_host", path)
+            try:
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+            except ImportError:
+                return None
+            mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.gbx_qlinear_forward, L.gbx_qlinear_forward_ws, L.gbx_qlinear_workspace_bytes)))
+            _host = mod
+    return _host or None
+
+
 def mixers() -> ctypes.CDLL:
     """The ragged-step kernel library; compiled on first use when the checkout holds no built copy.  No fallback: raises."""
     global _mlib

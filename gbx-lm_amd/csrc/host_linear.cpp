@@ -1,0 +1,105 @@
+// One packed product of few rows from Python in one call: the checks of ops.quantized_matmul, the result's allocation and the library's entry point.  Through the interpreter (reads of
+// shapes and addresses, an allocation, a foreign call of fourteen arguments) a module's call took 10.8 us, here 6.7, where the kernel of one row of 4096 x 4096 takes 5.4; 27 rows of
+// 8192 x 3072, whose kernel takes 8: 11.7 -> 8.6.
+// Whatever is not plain -- other layouts, types that want a cast, subclasses, transforms, modes, traces, more rows -- is answered with None: the general path then takes or refuses it.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+namespace {
+
+// entry points of the library that the package has loaded (_lib.py hands their addresses over)
+typedef int (*ForwardFn)(const void*, const void*, const void*, const void*, const void*, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t, void*);
+typedef int (*ForwardWsFn)(const void*, const void*, const void*, const void*, const void*, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t, void*, size_t, void*);
+typedef size_t (*WorkspaceFn)(int64_t, int32_t, int32_t, int32_t, int32_t);
+ForwardFn forward_fn = nullptr;
+ForwardWsFn forward_ws_fn = nullptr;
+WorkspaceFn workspace_fn = nullptr;
+
+constexpr int64_t FEW_ROWS = 256;          // from here on a resident image of the weight may be the faster operand (ops.py decides)
+constexpr int F16 = 0, BF16 = 1;
+
+bool plain(const at::Tensor& t, at::Device device) {
+  static const uint64_t usual = (c10::DispatchKeySet(c10::DispatchKey::CUDA) | c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) |
+                                 c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) | c10::DispatchKeySet(c10::DispatchKey::AutocastCUDA)).raw_repr();
+  return (t.key_set().raw_repr() & ~usual) == 0 && t.device() == device && t.is_contiguous() && t.has_storage();
+}
+
+bool watched() {                            // something is to see every operation
+  return c10::impl::dispatch_mode_enabled() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
+}
+
+PyObject* bind(PyObject*, PyObject* args) {
+  unsigned long long f, w, s;
+  if (!PyArg_ParseTuple(args, "KKK", &f, &w, &s)) return nullptr;
+  forward_fn = reinterpret_cast<ForwardFn>(static_cast<uintptr_t>(f));
+  forward_ws_fn = reinterpret_cast<ForwardWsFn>(static_cast<uintptr_t>(w));
+  workspace_fn = reinterpret_cast<WorkspaceFn>(static_cast<uintptr_t>(s));
+  Py_RETURN_NONE;
+}
+
+// few_rows(x, qweight, scales, zeros, group_size, bits, bias or None) -> y, None (not a call for this path) or the library's error code
+PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 7 || !forward_fn) Py_RETURN_NONE;
+  for (int i = 0; i < 4; ++i)
+    if (!THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
+  const bool has_bias = args[6] != Py_None;
+  if ((has_bias && !THPVariable_CheckExact(args[6])) || !PyLong_CheckExact(args[4]) || !PyLong_CheckExact(args[5]) || watched()) Py_RETURN_NONE;
+  const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &sc = THPVariable_Unpack(args[2]), &ze = THPVariable_Unpack(args[3]);
+  const auto type = x.scalar_type();
+  if (!x.is_cuda() || (type != at::kBFloat16 && type != at::kHalf) || (w.scalar_type() != at::kInt && w.scalar_type() != at::ScalarType::UInt32) || sc.scalar_type() != type ||
+      ze.scalar_type() != type)
+    Py_RETURN_NONE;
+  const at::Device device = x.device();
+  if (!plain(x, device) || !plain(w, device) || !plain(sc, device) || !plain(ze, device)) Py_RETURN_NONE;
+  const int64_t group = PyLong_AsLongLong(args[4]), bits = PyLong_AsLongLong(args[5]);
+  if (x.dim() < 1 || w.dim() != 2 || sc.dim() != 2 || ze.dim() != 2 || group < 1 || bits < 1 || group > 1024 || bits > 32) Py_RETURN_NONE;
+  const int64_t n = w.size(0), words = w.size(1);
+  if (words * 32 % bits) Py_RETURN_NONE;
+  const int64_t k = words * 32 / bits;
+  if (k < 1 || n < 1 || k > 0x7fffffff || n > 0x7fffffff || x.size(-1) != k || k % group || sc.size(0) != n || sc.size(1) != k / group || ze.size(0) != n || ze.size(1) != k / group)
+    Py_RETURN_NONE;
+  const int64_t m = x.numel() / k;
+  if (m < 1 || m >= FEW_ROWS) Py_RETURN_NONE;
+  const void* bias = nullptr;
+  if (has_bias) {
+    const at::Tensor& b = THPVariable_Unpack(args[6]);
+    if (b.scalar_type() != type || b.dim() != 1 || b.size(0) != n || !plain(b, device)) Py_RETURN_NONE;
+    bias = b.const_data_ptr();
+  }
+  auto shape = x.sizes().vec();
+  shape.back() = n;
+  at::Tensor y = at::empty(shape, x.options().requires_grad(false));
+  if (!plain(y, device)) Py_RETURN_NONE;
+  void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+  const int act = type == at::kBFloat16 ? BF16 : F16;
+  const int32_t N = static_cast<int32_t>(n), K = static_cast<int32_t>(k), B = static_cast<int32_t>(bits), G = static_cast<int32_t>(group);
+  // scratch: decode batches and short prompts split k across workgroups
+  const size_t need = (m >= 2 && m <= 32) || m > 64 ? workspace_fn(m, N, K, B, G) : 0;
+  int rc;
+  if (need) {
+    at::Tensor ws = at::empty({static_cast<int64_t>(need)}, x.options().dtype(at::kByte).requires_grad(false));
+    rc = forward_ws_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, ws.mutable_data_ptr(), need, stream);
+  } else {
+    rc = forward_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, stream);
+  }
+  if (rc) return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
+                         {"few_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(few_rows)), METH_FASTCALL, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_gbx_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__gbx_host(void) { return PyModule_Create(&module); }

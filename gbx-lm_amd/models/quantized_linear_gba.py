@@ -28,6 +28,9 @@ _STRATEGY_KEYS = ['kv_a_proj_with_mqa', 'kv_b_proj', 'q_a_proj', 'q_b_proj', 'q_
 _DQ_NAMES = ("qstatistic", "qzeros_zeros", "qzeros_scales", "qscales_zeros", "qscales_scales")
 
 
+_ASK = object()
+
+
 def _is_gba_linear(m) -> bool:
     return isinstance(m, QuantizedLinear)
 
@@ -124,12 +127,15 @@ class QuantizedLinear(nn.Module):
 
     # ------------------------------------------------------------------ forward (:179-207)
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        scales, zeros = self.scales, self.zeros
+        held = self._buffers                                  # (a module's attributes cost a search each; what is no buffer is found that way)
+        scales, zeros = held.get("scales", _ASK), held.get("zeros", _ASK)
+        qweight, bias = held.get("qweight", _ASK), held.get("bias", _ASK)
+        if scales is _ASK or zeros is _ASK or qweight is _ASK:
+            scales, zeros, qweight = self.scales, self.zeros, self.qweight
         if scales is None or zeros is None:
             raise RuntimeError("QuantizedLinear: double-quantised statistics not expanded; call prepare_scales_zeros")
         # channel_scale / q_perm are intentionally NOT applied (commented out in the reference, :187-192)
-        return ops.quantized_matmul(x, self.qweight, scales=scales, biases=zeros, transpose=True,
-                                    group_size=self.group_size, bits=self.bits, bias=self.bias)
+        return ops.quantized_matmul(x, qweight, scales, zeros, True, self.group_size, self.bits, self.bias if bias is _ASK else bias)
 
     # ------------------------------------------------------------------ loader hooks (:210-324)
     @classmethod

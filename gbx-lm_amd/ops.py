@@ -186,6 +186,19 @@ def _alloc_dense(shape, dtype, device):
             return None
 
 
+_few_rows = None
+
+
+def _bind_few_rows():
+    """The native call of up to 255 rows (csrc/host_linear.cpp); without it nothing is taken there."""
+    global _few_rows
+    mod = _lib.host() if torch.cuda.is_available() else None
+    few = mod.few_rows if mod is not None else lambda *a: None
+    if torch.cuda.is_available():
+        _few_rows = few
+    return few
+
+
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                      transpose: bool = True, group_size: int = 64, bits: int = 4,
                      bias: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -197,6 +210,13 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """
     if not transpose:
         raise NotImplementedError("quantized_matmul(transpose=False) is not on the QuantizedLinear path")
+    if out is None:
+        few = _few_rows or _bind_few_rows()
+        y = few(x, w, scales, biases, group_size, bits, bias)
+        if y is not None:
+            if type(y) is int:
+                _lib.check(y)
+            return y
     if not (x.is_cuda and w.is_cuda and scales.is_cuda and biases.is_cuda):
         for t, nm in ((x, "x"), (w, "w"), (scales, "scales"), (biases, "biases")):
             _require_cuda(t, nm)
