@@ -54,9 +54,39 @@ template <> struct Lanes<bf16_t, 4> {
   }
 };
 
+// One step of a sum over a wave, every lane: v of this lane plus that of the lane 2^k away.  Register moves: a trip through LDS (__shfl_xor) is what a row kernel
+// of a decode step waits for otherwise (by __shfl_xor | this, the same bits, us a token: 1 row of 4 streams x 1024 over 4 layers 197.5 | 192.0, 2 rows of 2048 over 4
+// 332.6 | 329.6).  FROM 32, 16: halves and rows of 16 trade places; 8: any values; 4: values that step 8 has made alike.
+template <int FROM> __device__ __forceinline__ float lanes_apart_sum(float v) {
+  if constexpr (FROM >= 16) {
+    const unsigned b = __float_as_uint(v);
+    if constexpr (FROM == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+      return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+      return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+  } else {
+    constexpr int MOVE = FROM == 8 ? 0x128 : FROM == 4 ? 0x124 : FROM == 2 ? 0x4E : 0xB1;       // row_ror:8, row_ror:4, quad_perm [2,3,0,1], [1,0,3,2]
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), MOVE, 0xf, 0xf, false));
+  }
+}
+// The sum of a wave's values, the same bits in every lane: halves first, neighbours last.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = lanes_apart_sum<16>(lanes_apart_sum<32>(v));
+  v = lanes_apart_sum<4>(lanes_apart_sum<8>(v));
+  return lanes_apart_sum<1>(lanes_apart_sum<2>(v));
+}
+// The same over aligned groups of `lanes` (a power of two, the same for a whole wave), neighbours first.
+__device__ __forceinline__ float group_sum(float v, int lanes) {
+  const auto plus = [&](auto move) { v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(move)::value, 0xf, 0xf, false)); };
+  if (lanes > 1) plus(std::integral_constant<int, 0xB1>{});          // quad_perm [1,0,3,2]
+  if (lanes > 2) plus(std::integral_constant<int, 0x4E>{});          // quad_perm [2,3,0,1]
+  if (lanes > 4) plus(std::integral_constant<int, 0x141>{});         // row_half_mirror
+  if (lanes > 8) plus(std::integral_constant<int, 0x140>{});         // row_mirror
+  if (lanes > 16) v = lanes_apart_sum<16>(v);
+  if (lanes > 32) v = lanes_apart_sum<32>(v);
   return v;
 }
 // Sum over the 16 lanes of a row; every lane of the row gets the same bits (each step adds the two halves of a mirrored pair).
@@ -86,8 +116,17 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
+  const int waves = blockDim.x >> 6;
   float s = 0.f;
-  for (int i = 0; i < static_cast<int>(blockDim.x >> 6); ++i) s += red[i];
+#pragma unroll
+  for (int i = 0; i < 16; i += 4)                  // (four at a time: a loop waits for LDS once a wave)
+    if (i < waves) {
+      const float r[4] = {red[i], red[i + 1], red[i + 2], red[i + 3]};
+      s += r[0];
+#pragma unroll
+      for (int k = 1; k < 4; ++k)
+        if (i + k < waves) s += r[k];
+    }
   return s;
 }
 

@@ -115,8 +115,7 @@ __global__ __launch_bounds__(256) void log_softmax_slice_kernel(const T* __restr
   lsm_load8(x + static_cast<int64_t>(blockIdx.y) * n, k, n, vec, scale, v);
 #pragma unroll
   for (int j = 0; j < 8; ++j) m = fmaxf(m, v[j]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
@@ -136,8 +135,7 @@ __global__ __launch_bounds__(256) void log_softmax_write_kernel(const T* __restr
   float v[8], m = -INFINITY, s = 0.f;
   lsm_load8(x + base, k, n, vec, scale, v);
   for (int i = threadIdx.x; i < parts; i += 256) m = fmaxf(m, p[i].x);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
@@ -191,8 +189,7 @@ __global__ __launch_bounds__(LSM_NT) void log_softmax_kernel(const T* __restrict
     for (int j = 0; j < PER; ++j) m = fmaxf(m, lsm_get<T>(u, j) * scale);
   }
   for (int k = nv * PER + tid; k < n; k += LSM_NT) m = fmaxf(m, static_cast<float>(row[k]) * scale);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((tid & 63) == 0) red[tid >> 6] = m;
   __syncthreads();
 #pragma unroll
@@ -477,8 +474,7 @@ __global__ __launch_bounds__(NT) void route_topk_kernel(const float* __restrict_
   __syncthreads();
   float mx = -INFINITY;
   for (int e = threadIdx.x; e < E; e += NT) mx = fmaxf(mx, lg[e]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
   if (lane == 0) red[wave] = mx;
   __syncthreads();
   mx = red[0];
@@ -534,8 +530,7 @@ __global__ __launch_bounds__(NT) void route_topk_rank_kernel(const float* __rest
     v[i] = e < E ? logits[t * E + e] : -INFINITY;
     mx = fmaxf(mx, v[i]);
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
   if ((threadIdx.x & 63) == 0) mxs[threadIdx.x >> 6] = mx;
   __syncthreads();
 #pragma unroll

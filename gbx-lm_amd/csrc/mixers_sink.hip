@@ -121,8 +121,7 @@ __global__ __launch_bounds__(NT) void sink_rows_kernel(const T* __restrict__ q, 
     for (int r = wave; r < nr; r += NW) {           // a wave per head: the tile's maximum, the weights, their sum
       const float s = gl[r * KT + lane];
       float mx = s;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
       const float m_old = ml[r], m_new = fmaxf(m_old, mx);            // mx is finite: a tile holds at least one key
       const float p = exp_<FAST>(s - m_new);
       gl[r * KT + lane] = p;
@@ -666,8 +665,9 @@ __global__ __launch_bounds__(NT) void head_project_runs_kernel(const gbxm_head_p
 #pragma unroll
     for (int u = 0; u < PART; ++u) {
       s[u] = (red[wave][0][lane][u] + red[wave][2][lane][u]) + (red[wave][1][lane][u] + red[wave][3][lane][u]);
-#pragma unroll
-      for (int m = 32; m >= JC; m >>= 1) s[u] += __shfl_xor(s[u], m, 64);
+      if constexpr (JC <= 32) s[u] = lanes_apart_sum<32>(s[u]);
+      if constexpr (JC <= 16) s[u] = lanes_apart_sum<16>(s[u]);
+      if constexpr (JC <= 8) s[u] = lanes_apart_sum<8>(s[u]);
     }
     if (lane < JC && j0 + jc * PER < n_out) {
 #pragma unroll

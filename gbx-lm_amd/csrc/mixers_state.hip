@@ -140,8 +140,7 @@ __global__ __launch_bounds__(NT) void recurrent_prep_rows_kernel(gbxm_recurrent_
         float mul = c < nq ? p.q_scale : 1.f;
         if (p.unit) {
           float ss = v[0] * v[0] + v[1] * v[1] + (v[2] * v[2] + v[3] * v[3]);
-          for (int o = 1; o < p.dk / 4; o <<= 1) ss += __shfl_xor(ss, o, 64);
-          mul *= 1.f / sqrtf(ss + 1e-6f);
+          mul *= 1.f / sqrtf(group_sum(ss, p.dk / 4) + 1e-6f);
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] *= mul;
@@ -266,8 +265,7 @@ __global__ __launch_bounds__(NT) void head_norm_gate_vec_kernel(const float* __r
     for (int k = 0; k < 4; ++k) m[k] = w[(c & (dv - 1)) + k];
   }
   float ss = x[0] * x[0] + x[1] * x[1] + (x[2] * x[2] + x[3] * x[3]);
-  for (int d = 1; d < dv / 4; d <<= 1) ss += __shfl_xor(ss, d, 64);
-  const float r = 1.f / sqrtf(ss / dv + eps);
+  const float r = 1.f / sqrtf(group_sum(ss, dv / 4) / dv + eps);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const float s = sigmoid_<FAST>(g[k]);

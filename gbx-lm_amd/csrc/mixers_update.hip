@@ -193,8 +193,7 @@ __global__ __launch_bounds__(NT) void route_groups_kernel(const float* __restric
   }
   float mx = -INFINITY;
   for (int e = tid; e < E; e += nth) mx = fmaxf(mx, cl[e]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
   if (nth > 64) {
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
