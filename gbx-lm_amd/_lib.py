@@ -335,6 +335,13 @@ class SinkAttnArgs(ctypes.Structure):
                 ("longest", ctypes.c_int32)]
 
 
+class SlotRows(ctypes.Structure):
+    """Mirror of ``gbxm_slot_rows``."""
+    _fields_ = [("k", ctypes.c_void_p), ("k_stride", ctypes.c_int64), ("k_width", ctypes.c_int32),
+                ("v", ctypes.c_void_p), ("v_stride", ctypes.c_int64), ("v_width", ctypes.c_int32),
+                ("kcache", ctypes.c_void_p), ("vcache", ctypes.c_void_p)]
+
+
 class HeadProjectArgs(ctypes.Structure):
     """Mirror of ``gbxm_head_project_args``."""
     _fields_ = [("in_", ctypes.c_void_p), ("in_row", ctypes.c_int64), ("in_head", ctypes.c_int64), ("w", ctypes.c_void_p), ("out", ctypes.c_void_p),
@@ -464,6 +471,7 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_rotate_norm_heads.argtypes = [p, i64, i64, p, i64, ctypes.POINTER(HeadSegment), i32, f32, i32, p]
         L.gbxm_slot_append.argtypes = [p, i64, i32, p, i64, i32, p, p, p, p, i64, i32, i32, i32, p]
         L.gbxm_sink_attention.argtypes = [ctypes.POINTER(SinkAttnArgs), p]
+        L.gbxm_sink_attention_append.argtypes = [ctypes.POINTER(SinkAttnArgs), ctypes.POINTER(SlotRows), p]
         L.gbxm_sink_attention_tiled.argtypes = [i32, i32, i32, i32]
         L.gbxm_hyper_step.argtypes = [p, p, p, p, p, p, p, p, p, p, i64, i32, i32, i32, f32, i32, p]
         L.gbxm_glu.argtypes = [p, i64, p, i64, p, i64, i64, i32, i32, f32, f32, i32, p]

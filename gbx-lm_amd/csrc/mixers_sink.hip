@@ -15,6 +15,7 @@
 // The matrix-core kernel for bf16 prompt portions is in mixers_sink_mfma.hip.
 #include <algorithm>
 #include <climits>
+#include <utility>
 #include "mixers_mfma.h"
 
 namespace gbxm {
@@ -211,14 +212,50 @@ __global__ __launch_bounds__(NT) void sink_rows_kernel(const T* __restrict__ q, 
   }
 }
 
+// The step's rows on their way into the slot tables; k null: none.
+template <typename T> struct SlotRows {
+  const T *k, *v;
+  T *kc, *vc;
+  int64_t k_stride, v_stride;
+  int k_width, v_width, keep, ring, fours;
+  const int *seq, *tok;
+};
+template <typename T> SlotRows<T> slot_rows(const gbxm_slot_rows& r, const int32_t* seq, const int32_t* tok, int keep, int ring) {
+  const bool fours = (r.k_width | (r.v ? r.v_width : 0)) % 4 == 0 && r.k_stride % 4 == 0 && (!r.v || r.v_stride % 4 == 0) &&
+                     all_aligned(4 * sizeof(T), static_cast<const char*>(r.k), static_cast<const char*>(r.v), static_cast<const char*>(r.kcache),
+                                 static_cast<const char*>(r.v ? r.vcache : nullptr));
+  return {static_cast<const T*>(r.k), static_cast<const T*>(r.v), static_cast<T*>(r.kcache), static_cast<T*>(r.vcache), r.k_stride, r.v_stride,
+          r.k_width, r.v ? r.v_width : 0, keep, ring, fours, seq, tok};
+}
+// A workgroup copies row t, four channels a thread where rows, tables and their strides are in groups of four.
+template <typename T, int V> __device__ __forceinline__ void copy_row(const SlotRows<T>& r, int64_t t, int64_t row) {
+  struct alignas(V * sizeof(T)) Group { T v[V]; };
+  for (int c = threadIdx.x * V; c < r.k_width + r.v_width; c += NT * V)
+    *reinterpret_cast<Group*>(c < r.k_width ? r.kc + row * r.k_width + c : r.vc + row * r.v_width + (c - r.k_width)) =
+        *reinterpret_cast<const Group*>(c < r.k_width ? r.k + t * r.k_stride + c : r.v + t * r.v_stride + (c - r.k_width));
+}
+template <typename T> __device__ __forceinline__ void append_row(const SlotRows<T>& r, int64_t t) {
+  const int b = r.tok[2 * t], pos = r.tok[2 * t + 1];
+  const int slot = r.seq[4 * b], pos0 = r.seq[4 * b + 1], n = r.seq[4 * b + 2];
+  if (pos >= r.keep && pos + r.ring < pos0 + n) return;  // a later row of this step takes the same ring row
+  const int64_t row = static_cast<int64_t>(slot) * (r.keep + r.ring) + (pos < r.keep + r.ring ? pos : r.keep + (pos - r.keep) % r.ring);
+  if (r.fours) copy_row<T, 4>(r, t, row);
+  else copy_row<T, 1>(r, t, row);
+}
+
 // Joins the key splits' (sum, maximum, denominator), adds the sink, applies the gate; one workgroup per (row, head, 128 channels).  Rows of `partial`
 // are partial_width(dv) floats (the sums, padding to a multiple of four, maximum, denominator), so a thread reads four channels at once; eight
 // groups of 32 threads take every eighth split, all of it (at most 64) in flight beside the splits' weights -- one trip to memory, where two
-// halves of a workgroup for all channels made eight -- and meet in LDS in a fixed order.
+// halves of a workgroup for all channels made eight -- and meet in LDS in a fixed order.  Workgroups behind the last head append the step's rows: no query
+// reads the tables any more, and a launch of its own costs a step more than the copy (a launch behind | here, us a token: 2 rows, three such layers 328.9 | 322.5).
 template <typename T, bool FAST>
 __global__ __launch_bounds__(256) void sink_reduce_kernel(const float* __restrict__ partial, T* __restrict__ out, const float* __restrict__ sink,
                                                          const T* __restrict__ gate, int64_t gate_row, int gate_channels, int64_t T_, int H, int dv,
-                                                         int splits, int64_t out_row) {
+                                                         int splits, int64_t out_row, const SlotRows<T> rows) {
+  if (static_cast<int>(blockIdx.y) == H) {
+    if (blockIdx.z == 0) append_row(rows, blockIdx.x);
+    return;
+  }
   __shared__ float wz[64];
   __shared__ float den;
   __shared__ float4 part[8][32];
@@ -264,8 +301,18 @@ __global__ __launch_bounds__(256) void sink_reduce_kernel(const float* __restric
     out[t * out_row + head * dv + d + c] = from_f32<T>(gate && gate_channels ? r[c] * sigmoid_<FAST>(to_f32(gate[t * gate_row + head * dv + d + c])) : r[c]);
 }
 
+// `rows`: appended in the same launch.
 template <typename T, bool FAST>
-int launch_rows(const gbxm_sink_attn_args& a, const SinkGeo& g, int rc, int chunks, size_t lds, hipStream_t s) {
+int launch_reduce(const gbxm_sink_attn_args& a, int splits, int64_t out_row, const gbxm_slot_rows* rows, hipStream_t s) {
+  const SlotRows<T> r = rows ? slot_rows<T>(*rows, a.seq, a.tok, a.keep, a.ring) : SlotRows<T>{};
+  sink_reduce_kernel<T, FAST><<<dim3(a.T, a.H + (rows ? 1 : 0), (a.dv + 127) / 128), 256, 0, s>>>(
+      static_cast<const float*>(a.partial), static_cast<T*>(a.out), a.sink, static_cast<const T*>(a.gate), a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits, out_row, r);
+  return after_launch("sink_attention (join of key splits)");
+}
+
+// Launches that join key splits take `rows` with them and clear it for the caller.
+template <typename T, bool FAST>
+int launch_rows(const gbxm_sink_attn_args& a, const SinkGeo& g, int rc, int chunks, size_t lds, const gbxm_slot_rows*& rows, hipStream_t s) {
   constexpr int PER = 16 / sizeof(T);
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   bool vec = a.dk % PER == 0 && a.k_row % PER == 0 && a.k_head % PER == 0 && al(a.k_new) && a.v_row % 2 == 0 && a.v_head % 2 == 0 &&
@@ -296,8 +343,10 @@ int launch_rows(const gbxm_sink_attn_args& a, const SinkGeo& g, int rc, int chun
     if (vec) go(sink_rows_kernel<T, FAST, true, NCH_MAX>);
     else go(sink_rows_kernel<T, FAST, false, NCH_MAX>);
   }
-  if (splits > 1) sink_reduce_kernel<T, FAST><<<dim3(a.T, a.H, (a.dv + 127) / 128), 256, 0, s>>>(part, out, a.sink, gate, a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits,
-                                                                                       g.out_row);
+  if (splits > 1) {
+    const int rc2 = after_launch("sink_attention (rows)");
+    return rc2 != GBXM_OK ? rc2 : launch_reduce<T, FAST>(a, splits, g.out_row, std::exchange(rows, nullptr), s);
+  }
   return after_launch("sink_attention (rows)");
 }
 
@@ -737,36 +786,20 @@ __global__ __launch_bounds__(NT) void activate_vec_kernel(T* __restrict__ z, int
   *p = uint4{u[0], u[1], u[2], u[3]};
 }
 
-// V: channels a thread copies at a time (4: rows, tables and their strides in groups of four)
-template <typename T, int V>
-__global__ __launch_bounds__(NT) void slot_append_kernel(const T* __restrict__ k, int64_t k_stride, int k_width, const T* __restrict__ v,
-                                                        int64_t v_stride, int v_width, T* __restrict__ kc, T* __restrict__ vc,
-                                                        const int* __restrict__ seq, const int* __restrict__ tok, int keep, int ring) {
-  const int64_t t = blockIdx.x;
-  const int b = tok[2 * t], pos = tok[2 * t + 1];
-  const int slot = seq[4 * b], pos0 = seq[4 * b + 1], n = seq[4 * b + 2];
-  if (pos >= keep && pos + ring < pos0 + n) return;      // a later row of this step takes the same ring row
-  const int64_t row = static_cast<int64_t>(slot) * (keep + ring) + (pos < keep + ring ? pos : keep + (pos - keep) % ring);
-  struct alignas(V * sizeof(T)) Group { T v[V]; };
-  const int all = k_width + (v ? v_width : 0);
-  for (int c = threadIdx.x * V; c < all; c += NT * V)
-    *reinterpret_cast<Group*>(c < k_width ? kc + row * k_width + c : vc + row * v_width + (c - k_width)) =
-        *reinterpret_cast<const Group*>(c < k_width ? k + t * k_stride + c : v + t * v_stride + (c - k_width));
-}
+// grid (rows)
+template <typename T>
+__global__ __launch_bounds__(NT) void slot_append_kernel(const SlotRows<T> r) { append_row(r, blockIdx.x); }
 
 bool act_ok(int act) { return act == GBXM_BF16 || act == GBXM_F32; }
 
 }  // namespace
 
 int launch_sink_tiles(const gbxm_sink_attn_args& a, hipStream_t s);     // mixers_sink_mfma.hip; GBXM_ERR_UNSUPPORTED: not its shape
-int launch_sink_group(const gbxm_sink_attn_args& a, hipStream_t s);     // the same for steps of single rows
+int launch_sink_group(const gbxm_sink_attn_args& a, const gbxm_slot_rows*& rows, hipStream_t s);     // the same for steps of single rows
 bool sink_tiles_shape(int dk, int dv);
 
-int launch_sink_reduce(const gbxm_sink_attn_args& a, int splits, hipStream_t s) {
-  sink_reduce_kernel<bf16_t, true><<<dim3(a.T, a.H, (a.dv + 127) / 128), 256, 0, s>>>(static_cast<const float*>(a.partial), static_cast<bf16_t*>(a.out), a.sink,
-                                                                  static_cast<const bf16_t*>(a.gate), a.gate_row, a.gate_channels, a.T, a.H, a.dv, splits,
-                                                                  a.out_row > 0 ? a.out_row : static_cast<int64_t>(a.H) * a.dv);
-  return after_launch("sink_attention (join of key splits)");
+int launch_sink_reduce(const gbxm_sink_attn_args& a, int splits, const gbxm_slot_rows* rows, hipStream_t s) {
+  return launch_reduce<bf16_t, true>(a, splits, a.out_row > 0 ? a.out_row : static_cast<int64_t>(a.H) * a.dv, rows, s);
 }
 
 }  // namespace gbxm
@@ -868,14 +901,8 @@ int gbxm_slot_append(const void* k, int64_t k_stride, int32_t k_width, const voi
     return fail(GBXM_ERR_INVALID, "slot_append: bad argument");
   if (T_ == 0) return GBXM_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool fours = (k_width | v_width) % 4 == 0 && k_stride % 4 == 0 && (!v || v_stride % 4 == 0) &&
-                     all_aligned(act == GBXM_BF16 ? 8 : 16, static_cast<const char*>(k), static_cast<const char*>(v), static_cast<const char*>(kcache),
-                                 static_cast<const char*>(v ? vcache : nullptr));
-#define GBXM_APPEND(V_) slot_append_kernel<T, V_><<<dim3(T_), NT, 0, s>>>(static_cast<const T*>(k), k_stride, k_width, static_cast<const T*>(v), v_stride, v_width, \
-                                                                         static_cast<T*>(kcache), static_cast<T*>(vcache), seq, tok, keep, ring)
-  if (fours) GBXM_DISPATCH(act, GBXM_APPEND(4));
-  else GBXM_DISPATCH(act, GBXM_APPEND(1));
-#undef GBXM_APPEND
+  const gbxm_slot_rows rows{k, k_stride, k_width, v, v_stride, v_width, kcache, vcache};
+  GBXM_DISPATCH(act, (slot_append_kernel<T><<<dim3(T_), NT, 0, s>>>(slot_rows<T>(rows, seq, tok, keep, ring))));
   return after_launch("slot_append");
 }
 
@@ -883,7 +910,7 @@ int gbxm_sink_attention_tiled(int32_t dk, int32_t dv, int32_t act, int32_t decod
   return act == GBXM_BF16 && sink_tiles_shape(dk, dv);          // (steps of single rows: the grouped form of the same products)
 }
 
-int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream) {
+static int sink_attention(const gbxm_sink_attn_args* a, const gbxm_slot_rows*& rows, void* stream) {
   if (!a || !a->q || !a->k_new || !a->v_new || !a->seq || !a->tok || !a->out) return fail(GBXM_ERR_INVALID, "sink_attention: null argument");
   if (!act_ok(a->act)) return fail(GBXM_ERR_INVALID, "sink_attention: dtype");
   if (a->H <= 0 || a->G <= 0 || a->H % a->G || a->dk <= 0 || a->dv <= 0 || a->keep < 0 || a->ring < 1 || a->T < 0 || a->B < 0 ||
@@ -900,7 +927,7 @@ int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream) {
     if (rc != GBXM_ERR_UNSUPPORTED) return rc;
   }
   if (a->decode_only && a->act == GBXM_BF16 && a->H <= 65535) {
-    const int rc = launch_sink_group(*a, s);
+    const int rc = launch_sink_group(*a, rows, s);
     if (rc != GBXM_ERR_UNSUPPORTED) return rc;
   }
   SinkGeo g{a->H, a->G, a->dk, a->dv, a->window, a->keep, a->ring, a->chunk, a->gate_channels, a->scale, a->head_scale,
@@ -916,7 +943,24 @@ int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream) {
   if (lds_of(rc) > 60 * 1024) return fail(GBXM_ERR_UNSUPPORTED, "sink_attention: head sizes dk=%d dv=%d are beyond the row kernel", a->dk, a->dv);
   const int chunks = (R + rc - 1) / rc;
   if (a->T > 0x7fffffffLL || a->G * chunks > 65535 || a->H > 65535) return fail(GBXM_ERR_UNSUPPORTED, "sink_attention: grid");
-  return a->act == GBXM_BF16 ? launch_rows<bf16_t, true>(*a, g, rc, chunks, lds_of(rc), s) : launch_rows<float, false>(*a, g, rc, chunks, lds_of(rc), s);
+  return a->act == GBXM_BF16 ? launch_rows<bf16_t, true>(*a, g, rc, chunks, lds_of(rc), rows, s) : launch_rows<float, false>(*a, g, rc, chunks, lds_of(rc), rows, s);
+}
+
+int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream) {
+  const gbxm_slot_rows* none = nullptr;
+  return sink_attention(a, none, stream);
+}
+
+int gbxm_sink_attention_append(const gbxm_sink_attn_args* a, const gbxm_slot_rows* rows, void* stream) {
+  if (!a || !rows || !rows->k || !rows->kcache || rows->k_width <= 0 || rows->k_stride < rows->k_width ||
+      (rows->v && (!rows->vcache || rows->v_width <= 0 || rows->v_stride < rows->v_width)))
+    return fail(GBXM_ERR_INVALID, "sink_attention_append: bad argument");
+  const bool apart = a->H >= 65535;                             // (a grid has one place more)
+  const gbxm_slot_rows* left = apart ? nullptr : rows;
+  const int rc = sink_attention(a, left, stream);
+  if (rc != GBXM_OK || !(left || apart)) return rc;
+  return gbxm_slot_append(rows->k, rows->k_stride, rows->k_width, rows->v, rows->v_stride, rows->v_width, rows->kcache, rows->vcache, a->seq, a->tok, a->T, a->keep,
+                          a->ring, a->act, stream);
 }
 
 }  // extern "C"

@@ -18,11 +18,12 @@
 //
 // Head sizes are run-time numbers (multiples of 8) inside a compiled capacity <DK, DV>: channels beyond them are staged as zeros.
 #include <algorithm>
+#include <utility>
 #include "mixers_mfma.h"
 
 namespace gbxm {
 
-int launch_sink_reduce(const gbxm_sink_attn_args& a, int splits, hipStream_t s);      // mixers_sink.hip
+int launch_sink_reduce(const gbxm_sink_attn_args& a, int splits, const gbxm_slot_rows* rows, hipStream_t s);      // mixers_sink.hip
 
 namespace {
 
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(256) void sink_group_kernel(const SinkTileArgs a, c
 }
 
 template <int DK, int DV, bool ALIAS>
-int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_t s) {
+int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, const gbxm_slot_rows*& rows, hipStream_t s) {
   const int R = a.H / a.G, chunks = (R + 31) / 32;
   int splits = 1;
   const int64_t groups = a.T * a.G * chunks;
@@ -565,7 +566,7 @@ int launch_group(const SinkTileArgs& t, const gbxm_sink_attn_args& a, hipStream_
   else sink_group_kernel<DK, DV, ALIAS, false><<<grid, 256, 0, s>>>(t, a.tok, R, splits, static_cast<float*>(a.partial));
   const int rc = after_launch("sink_attention (grouped rows)");
   if (rc != GBXM_OK || splits == 1) return rc;
-  return launch_sink_reduce(a, splits, s);
+  return launch_sink_reduce(a, splits, std::exchange(rows, nullptr), s);
 }
 
 // A workgroup = a query tile of a head, or (PAIRS, one group) two, one from each end of the list; tiles that see many keys, at the end of the step's list, go
@@ -693,19 +694,19 @@ bool sink_group_shape(int dk, int dv, bool alias) {
   return sink_tiles_shape(dk, dv);
 }
 
-int launch_sink_group(const gbxm_sink_attn_args& a, hipStream_t s) {
+int launch_sink_group(const gbxm_sink_attn_args& a, const gbxm_slot_rows*& rows, hipStream_t s) {
   const bool alias = values_alias_keys(a);
   const int chunks = (a.H / a.G + 31) / 32;
   if (!sink_group_shape(a.dk, a.dv, alias) || a.G * chunks > 65535 || !tile_operands(a)) return GBXM_ERR_UNSUPPORTED;
   const SinkTileArgs t = tile_args(a);
   if (alias) {
-#define GBXM_GROUP(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch_group<DK_, DV_, true>(t, a, s)
+#define GBXM_GROUP(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch_group<DK_, DV_, true>(t, a, rows, s)
     // (latent rows without rotated channels have capacities of their own, which they fill: 62 launches of 256 / 256 as 320 / 256 308 us | 296)
     GBXM_GROUP(96, 96); GBXM_GROUP(160, 128); GBXM_GROUP(256, 256); GBXM_GROUP(320, 256); GBXM_GROUP(512, 512); GBXM_GROUP(576, 512);
 #undef GBXM_GROUP
     return GBXM_ERR_UNSUPPORTED;
   }
-#define GBXM_GROUP(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch_group<DK_, DV_, false>(t, a, s)
+#define GBXM_GROUP(DK_, DV_) if (a.dk <= DK_ && a.dv <= DV_) return launch_group<DK_, DV_, false>(t, a, rows, s)
   GBXM_GROUP(32, 32); GBXM_GROUP(64, 64); GBXM_GROUP(64, 128); GBXM_GROUP(96, 96); GBXM_GROUP(128, 128); GBXM_GROUP(192, 128); GBXM_GROUP(256, 256);
 #undef GBXM_GROUP
   return GBXM_ERR_UNSUPPORTED;

@@ -354,25 +354,29 @@ def rotate_norm_heads_(rows: torch.Tensor, positions: torch.Tensor, segments, ep
                                                           segs, len(segments), float(eps), act, _stream(rows.device)))
 
 
-def slot_append(cache, k_rows: torch.Tensor, v_rows: Optional[torch.Tensor], batch) -> None:
-    act = _act(k_rows, "k_rows")
+def _slot_rows(cache, k_rows: torch.Tensor, v_rows: Optional[torch.Tensor], batch) -> "_lib.SlotRows":
     if k_rows.stride(1) != 1 or k_rows.shape[1] != cache.k_width or cache.keys.dtype != k_rows.dtype or cache.keys.shape[0] <= max(batch.slot):
         raise ValueError("slot_append: key rows do not fit the table")
     two = v_rows is not None
     if two != bool(cache.v_width) or (two and (v_rows.stride(1) != 1 or v_rows.shape[1] != cache.v_width)):
         raise ValueError("slot_append: value rows do not fit the table")
-    _lib.check_mixers(_lib.mixers().gbxm_slot_append(k_rows.data_ptr(), k_rows.stride(0), cache.k_width, v_rows.data_ptr() if two else None,
-                                                    v_rows.stride(0) if two else 0, cache.v_width, cache.keys.data_ptr(),
-                                                    cache.values.data_ptr() if two else None, batch.seq.data_ptr(), batch.tok.data_ptr(), batch.total,
-                                                    cache.keep, cache.ring, act, _stream(k_rows.device)))
+    return _lib.SlotRows(k_rows.data_ptr(), k_rows.stride(0), cache.k_width, v_rows.data_ptr() if two else None, v_rows.stride(0) if two else 0,
+                         cache.v_width, cache.keys.data_ptr(), cache.values.data_ptr() if two else None)
+
+
+def slot_append(cache, k_rows: torch.Tensor, v_rows: Optional[torch.Tensor], batch) -> None:
+    act, r = _act(k_rows, "k_rows"), _slot_rows(cache, k_rows, v_rows, batch)
+    _lib.check_mixers(_lib.mixers().gbxm_slot_append(r.k, r.k_stride, r.k_width, r.v, r.v_stride, r.v_width, r.kcache, r.vcache, batch.seq.data_ptr(),
+                                                    batch.tok.data_ptr(), batch.total, cache.keep, cache.ring, act, _stream(k_rows.device)))
 
 
 def sink_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, cache, batch, scale: float, window: Optional[int], keep: int,
                    sink: Optional[torch.Tensor], gate: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
-                   head_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   head_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, append=None) -> torch.Tensor:
     """Context rows [T, H * dv]; q [T, H, dk], k_new [T, G, dk], v_new [T, G, dv] views with unit channel stride, gate [T, H] or None;
     ``cache`` (models/cache.py:SlotKVCache, or None for a step without history) holds the positions before the step.  ``chunk``: a row
-    sees its own chunk of positions only; ``head_scale`` fp32 [H]: a factor of every score per query head; ``out``: rows to write into."""
+    sees its own chunk of positions only; ``head_scale`` fp32 [H]: a factor of every score per query head; ``out``: rows to write into;
+    ``append`` (key rows, value rows or None): what goes into the table of ``cache`` once every query has read it."""
     act = _act(q, "q")
     t, heads, dk = q.shape
     groups, dv = v_new.shape[1], v_new.shape[2]
@@ -432,7 +436,13 @@ def sink_attention(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, ca
         if splits > 1:
             partial = torch.empty((splits, t, heads, (dv + 3) // 4 * 4 + 4), dtype=torch.float32, device=q.device)
             a.partial, a.partial_splits = partial.data_ptr(), splits
-    _lib.check_mixers(_lib.mixers().gbxm_sink_attention(ctypes.byref(a), _stream(q.device)))
+    if append is None:
+        _lib.check_mixers(_lib.mixers().gbxm_sink_attention(ctypes.byref(a), _stream(q.device)))
+        return out
+    if _act(append[0], "append") != act or a.keep != cache.keep or a.ring != cache.ring or append[0].shape[0] != t:
+        raise ValueError("sink_attention: the rows to append do not fit the step or the table")
+    rows = _slot_rows(cache, append[0], append[1], batch)
+    _lib.check_mixers(_lib.mixers().gbxm_sink_attention_append(ctypes.byref(a), ctypes.byref(rows), _stream(q.device)))
     return out
 
 

@@ -130,13 +130,14 @@ def _attend_one(q, k, v, pos_q, pos_k, scale, window, keep, sink, gate, chunk=No
 
 def sink_attend(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, cache: Optional[SlotKVCache], batch, scale: float,
                 window: Optional[int], keep: int, sink: Optional[torch.Tensor], gate: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
-                head_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                head_scale: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, append=None) -> torch.Tensor:
     """q [T, H, dk], k_new [T, G, dk], v_new [T, G, dv] (views with unit inner stride), gate [T, H], [T, H * dv] or None -> [T, H * dv].
     ``cache`` (or None when no sequence of the step has history) holds the positions before the step; with ``chunk`` its table is one
-    of ``window = chunk`` rows.  ``head_scale`` fp32 [H]; ``out``: rows to write into (any row stride)."""
+    of ``window = chunk`` rows.  ``head_scale`` fp32 [H]; ``out``: rows to write into (any row stride); ``append`` (key rows [T, k_width],
+    value rows or None): into the table of ``cache`` after every query of the step has attended."""
     if q.is_cuda:
         from .. import mixer_ops as M
-        return M.sink_attention(q, k_new, v_new, cache, batch, scale, window, keep, sink, gate, chunk, head_scale, out)
+        return M.sink_attention(q, k_new, v_new, cache, batch, scale, window, keep, sink, gate, chunk, head_scale, out, append)
     t, heads, _ = q.shape
     groups, dv = v_new.shape[1], v_new.shape[2]
     if out is None:
@@ -155,6 +156,8 @@ def sink_attend(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, cache
                         None if gate is None else gate[r0:r0 + n], chunk, head_scale)
         out[r0:r0 + n] = o.reshape(n, heads * dv).to(q.dtype)
         r0 += n
+    if append is not None:
+        cache_append(cache, append[0], append[1], batch)
     return out
 
 
@@ -223,9 +226,9 @@ class RotatedValueWindowAttention(nn.Module):
         cache.reserve(max(p + n for p, n in zip(batch.pos0, batch.n_new)), qkv.dtype, qkv.device)
         k_rows, v_rows = qkv[:, self.nq:self.nq + self.nk], qkv[:, self.nq + self.nk:]
         ctx = sink_attend(qkv[:, :self.nq].view(t, self.heads, self.dim), k_rows.view(t, self.kv_heads, self.dim),
-                          v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, self.keep_first, self.sink)
+                          v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, self.keep_first, self.sink,
+                          append=(k_rows, v_rows))
         rotate_norm_heads_(ctx, pos, [HeadSegment(0, self.heads, self.vdim, 0, self.vdim, self.vfreq, sign=-1.0)], self.eps)
-        cache_append(cache, k_rows, v_rows, batch)
         return project(ctx, self.o.weight)
 
 
@@ -270,7 +273,6 @@ class GatedSinkWindowAttention(nn.Module):
         return w, b
 
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
-        from .feed_forward import gate_mul
         t = h.shape[0]
         y = project(h, self.inp.weight, self.inp.bias)
         pos = batch.tok[:, 1]
@@ -281,9 +283,9 @@ class GatedSinkWindowAttention(nn.Module):
         cache.reserve(max(p + n for p, n in zip(batch.pos0, batch.n_new)), y.dtype, y.device)
         k_rows, v_rows = y[:, self.nq:self.nq + self.nk], y[:, self.nq + self.nk:self.nq + self.nk + self.nv]
         ctx = sink_attend(y[:, :self.nq].view(t, self.heads, self.dim), k_rows.view(t, self.kv_heads, self.dim),
-                          v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, 0, self.sink)
-        cache_append(cache, k_rows, v_rows, batch)
-        return project(gate_mul(y[:, self.off_gate:self.off_gate + self.ng], ctx, "sigmoid"), self.o.weight, self.o.bias)
+                          v_rows.view(t, self.kv_heads, self.vdim), cache, batch, self.scale, self.window, 0, self.sink,
+                          y[:, self.off_gate:self.off_gate + self.ng], append=(k_rows, v_rows))
+        return project(ctx, self.o.weight, self.o.bias)
 
 
 class ChunkedAttention(nn.Module):
@@ -328,8 +330,7 @@ class ChunkedAttention(nn.Module):
         k_rows, v_rows = y[:, self.nq:self.nq + self.nk], y[:, self.nq + self.nk:self.off_gate]
         ctx = sink_attend(y[:, :self.nq].unflatten(1, (self.heads, self.dim)), k_rows.unflatten(1, (self.kv_heads, self.dim)),
                           v_rows.unflatten(1, (self.kv_heads, self.vdim)), cache, batch, self.scale, None, 0, None,
-                          y[:, self.off_gate:self.off_gate + self.heads], self.chunk, self.temp, out)
-        cache_append(cache, k_rows, v_rows, batch)
+                          y[:, self.off_gate:self.off_gate + self.heads], self.chunk, self.temp, out, (k_rows, v_rows))
         return ctx
 
     def forward(self, h: torch.Tensor, batch, cache: SlotKVCache) -> torch.Tensor:
@@ -383,8 +384,8 @@ class SharedKeyValueAttention(nn.Module):
         cache.reserve(max(p + n for p, n in zip(batch.pos0, batch.n_new)), y.dtype, y.device)
         rows = y[:, self.off_k:self.off_k + self.nk]
         heads = rows.unflatten(1, (self.kv_heads, self.head_row))
-        ctx = sink_attend(y[:, :self.nq].unflatten(1, (self.heads, d)), heads[:, :, r:], heads[:, :, :d], cache, batch, self.scale, None, 0, self.sink)
-        cache_append(cache, rows, None, batch)
+        ctx = sink_attend(y[:, :self.nq].unflatten(1, (self.heads, d)), heads[:, :, r:], heads[:, :, :d], cache, batch, self.scale, None, 0, self.sink,
+                          append=(rows, None))
         return project(ctx, self.o.weight)
 
 
@@ -493,13 +494,14 @@ class LatentAttention(nn.Module):
             if turn is not None:
                 rotate_norm_heads_(q.flatten(1), pos, [turn], self.eps)
             ctx = sink_attend(q, keys, kv[:, self.nq:].view(t, hd, dv), None, batch, self.scale, None, 0, self.sink, gate)
+            if self.own_latent:
+                cache_append(cache, latent, None, batch)
         else:
             qa = head_project(q, self.uk_heads, r, turn, pos)                      # W_uk^T q | rotated part, per head
             per_channel = gate if self.gate_channels else None                     # (meets the value channels, behind W_uv)
             mixed = sink_attend(qa, latent.view(t, 1, self.nl), latent[:, :rank].view(t, 1, rank), table, batch, self.scale, None, 0,
-                                self.sink, None if self.gate_channels else gate)
+                                self.sink, None if self.gate_channels else gate, append=(latent, None) if self.own_latent else None)
             ctx = head_project(mixed.view(t, hd, rank), self.uv_heads_t, gate=per_channel).view(t, hd * dv)
         if self.own_latent:
-            cache_append(cache, latent, None, batch)
             cache.step_rows = latent                                # for mixers that attend over these rows later in the step
         return project(ctx, self.o.weight)

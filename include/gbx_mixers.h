@@ -168,6 +168,14 @@ typedef struct {
   int32_t longest;              /* positions of the step's longest sequence, its new ones included; 0: unknown.  Chooses among forms of the prompt kernel */
 } gbxm_sink_attn_args;
 int gbxm_sink_attention(const gbxm_sink_attn_args* a, void* stream);
+
+/* The same, and the step's rows into the tables (gbxm_slot_append with the call's seq, tok, T, keep, ring and act) once every query has read them. */
+typedef struct {
+  const void* k; int64_t k_stride; int32_t k_width;
+  const void* v; int64_t v_stride; int32_t v_width;      /* v null: a table without value rows */
+  void *kcache, *vcache;                                 /* the tables themselves */
+} gbxm_slot_rows;
+int gbxm_sink_attention_append(const gbxm_sink_attn_args* a, const gbxm_slot_rows* rows, void* stream);
 int gbxm_sink_attention_tiled(int32_t dk, int32_t dv, int32_t act, int32_t decode_only);
 
 /* ---- several residual streams, layer norm, gated activations, grouped sigmoid router (gbx-lm_amd/models/residual.py:hyper_step_,
