@@ -111,12 +111,12 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
-// The same over a workgroup of blockDim.x threads (whole waves, at most 16 of them); `red` is 16 floats of LDS that no earlier call used.
-__device__ __forceinline__ float row_sum(float v, float* red) {
+// The same over the workgroup of a row of `width` channels (row_threads); `red` is 16 floats of LDS that no earlier call used.
+__device__ __forceinline__ float row_sum(float v, float* red, int width) {
+  const int waves = (width / 4 + 63) >> 6;
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  const int waves = blockDim.x >> 6;
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; i += 4)                  // (four at a time: a loop waits for LDS once a wave)
@@ -211,25 +211,72 @@ inline bool choice_by_rank(int E, int rounds) { return E <= RANK_EXPERTS && E <=
 inline unsigned choice_threads(int64_t rows) { return rows > 1024 ? 256 : 64; }
 inline unsigned choice_blocks(int64_t rows) { return static_cast<unsigned>(rows > 1024 ? (rows + 3) / 4 : rows); }
 
-// z = a row of a sublayer's output, or sum_k mix[k] (candidate row k), at channels c .. c + 3; eight candidates in flight at a time.
-template <typename T>
-__device__ __forceinline__ void candidate_sum(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c, float* z) {
-  if (!mix) { Lanes<T, 4>::load(y + c, z); return; }
+// Four neighbouring elements as they lie in memory, so that a load in a branch does not wait there for its own conversion.
+template <typename T> struct Raw4;
+template <> struct Raw4<float> {
+  float4 r;
+  __device__ __forceinline__ void load(const float* p) { r = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ void get(float* v) const { v[0] = r.x; v[1] = r.y; v[2] = r.z; v[3] = r.w; }
+};
+template <> struct Raw4<bf16_t> {
+  uint2 r;
+  __device__ __forceinline__ void load(const bf16_t* p) { r = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ void get(float* v) const {
+    v[0] = __uint_as_float(r.x << 16); v[1] = __uint_as_float(r.x & 0xFFFF0000u);
+    v[2] = __uint_as_float(r.y << 16); v[3] = __uint_as_float(r.y & 0xFFFF0000u);
+  }
+};
+// Numbers that are the same for a whole wave, here and now: left to itself the compiler asks for each where it is first used, behind the trip of the rows.
+__device__ __forceinline__ void at_hand(float& x) { asm volatile("" : "+v"(x)); }
+template <typename P> __device__ __forceinline__ void at_hand(P* p) { asm volatile("" ::"s"(p)); }
+template <typename P, typename... Q> __device__ __forceinline__ void at_hand(P* p, Q*... q) { at_hand(p); at_hand(q...); }
+
+// z = a row of a sublayer's output, or sum_k mix[k] (candidate row k) (mix null: the sum alone where `sum` says so), at channels c .. c + 3; eight candidates in
+// flight at a time, the first ones (FEW: and their weights) from ask() on.
+template <typename T, bool FEW = false> struct Candidates {
+  Raw4<T> u[8];
+  float m[8];
+  __device__ __forceinline__ void ask(const T* __restrict__ y, const float* __restrict__ mix, int first, int top, int width, int c) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) z[i] = 0.f;
-  for (int k0 = 0; k0 < top; k0 += 8) {
-    float u[8][4];
+    for (int k = 0; k < 8; ++k) u[k].load(y + static_cast<int64_t>(min(first + k, top - 1)) * width + c);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) Lanes<T, 4>::load(y + static_cast<int64_t>(min(k0 + k, top - 1)) * width + c, u[k]);
+    for (int k = 0; k < 8; ++k) m[k] = mix ? mix[min(first + k, top - 1)] : 1.f;
+  }
+  __device__ __forceinline__ void add(int first, int top, float* z) {
+    if constexpr (FEW) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) at_hand(m[k]);
+    }
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (k0 + k < top) {
-        const float m = mix[k0 + k];
+      if (first + k < top) {
+        float v[4];
+        u[k].get(v);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z[i] += m * u[k][i];
+        for (int i = 0; i < 4; ++i) z[i] += m[k] * v[i];
       }
   }
-}
+  __device__ __forceinline__ void rest(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c, float* z) {
+    for (int k0 = 8; k0 < top; k0 += 8) {
+      ask(y, mix, k0, top, width, c);
+      add(k0, top, z);
+    }
+  }
+};
+template <typename T, bool FEW = false> struct Branch : Candidates<T, FEW> {
+  using Candidates<T, FEW>::u;
+  __device__ __forceinline__ void ask(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c) {
+    if (mix) Candidates<T, FEW>::ask(y, mix, 0, top, width, c);
+    else u[0].load(y + c);
+  }
+  __device__ __forceinline__ void sum(const T* __restrict__ y, const float* __restrict__ mix, int top, int width, int c, float* z) {
+    if (!mix) { u[0].get(z); return; }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] = 0.f;
+    this->add(0, top, z);
+    this->rest(y, mix, top, width, c, z);
+  }
+};
 
 // Transcendentals: exact library forms for fp32 models, hardware approximations (a few ulp) where activations are bf16.
 template <bool FAST> __device__ __forceinline__ float exp_(float x) { if constexpr (FAST) return __expf(x); else return expf(x); }

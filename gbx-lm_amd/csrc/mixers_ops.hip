@@ -428,13 +428,17 @@ __global__ __launch_bounds__(1024) void residual_norm_add_row_kernel(float* __re
   const int64_t t = blockIdx.x;
   const int c = threadIdx.x * 4;
   const bool on = c < width;
+  const T* y = branch + t * top * width;
+  const float* m = mix ? mix + t * top : nullptr;
   float z[4] = {0.f, 0.f, 0.f, 0.f}, v[4], f[4];
   if (on) {
+    Branch<T> b;
     Lanes<float, 4>::load(x + t * width + c, v);
     Lanes<float, 4>::load(w + c, f);
-    candidate_sum(branch + t * top * width, mix ? mix + t * top : nullptr, top, width, c, z);
+    b.ask(y, m, top, width, c);
+    b.sum(y, m, top, width, c, z);
   }
-  const float r = 1.f / sqrtf(row_sum(z[0] * z[0] + z[1] * z[1] + z[2] * z[2] + z[3] * z[3], red) / width + eps);
+  const float r = 1.f / sqrtf(row_sum(z[0] * z[0] + z[1] * z[1] + z[2] * z[2] + z[3] * z[3], red, width) / width + eps);
   if (!on) return;
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] += mult * (z[i] * r * f[i]);
@@ -453,7 +457,7 @@ __global__ __launch_bounds__(1024) void stream_rmsnorm_row_kernel(const float* _
     Lanes<float, 4>::load(x + t * width + c, v);
     Lanes<float, 4>::load(w + c, f);
   }
-  const float r = 1.f / sqrtf(row_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], red) / width + eps);
+  const float r = 1.f / sqrtf(row_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], red, width) / width + eps);
   if (!on) return;
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = v[i] * r * f[i];

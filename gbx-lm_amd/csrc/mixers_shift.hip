@@ -105,9 +105,9 @@ __global__ __launch_bounds__(1024) void norm_shift_row_kernel(const float* __res
   Lanes<float, 4>::load(x + (first ? static_cast<int64_t>(row0) + n - 1 : t) * width + c, xl);
   Lanes<float, 4>::load(st, kept);
   auto square = [&](const float* v) { return live ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f; };
-  const float rc = 1.f / sqrtf(row_sum(square(xc), red) / width + eps);
-  const float rp = 1.f / sqrtf(row_sum(square(xp), red + 16) / width + eps);
-  const float rl = first ? 1.f / sqrtf(row_sum(square(xl), red + 32) / width + eps) : rc;
+  const float rc = 1.f / sqrtf(row_sum(square(xc), red, width) / width + eps);
+  const float rp = 1.f / sqrtf(row_sum(square(xp), red + 16, width) / width + eps);
+  const float rl = first ? 1.f / sqrtf(row_sum(square(xl), red + 32, width) / width + eps) : rc;
   float last[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -130,22 +130,33 @@ __global__ __launch_bounds__(1024) void branch_norm_add_norm_row_kernel(float* _
   const int64_t t = blockIdx.x;
   const bool live = static_cast<int>(threadIdx.x) * 4 < width;
   const int c = live ? threadIdx.x * 4 : width - 4;
-  float v[4], wc[4], nw[4], e[4] = {0.f, 0.f, 0.f, 0.f}, z[4];
+  const T* y = branch + t * top * width;
+  const float* m = mix ? mix + t * top : nullptr;
+  at_hand(x, y, m, extra, w, next_w, h);
+  float v[4], wc[4], nw[4], e[4], z[4];
+  Raw4<T> ex;
+  Branch<T> b;
+  b.ask(y, m, top, width, c);
   Lanes<float, 4>::load(x + t * width + c, v);
+  if (extra) ex.load(extra + t * width + c);
   Lanes<float, 4>::load(w + c, wc);
   if (next_w) Lanes<float, 4>::load(next_w + c, nw);
-  if (extra) Lanes<T, 4>::load(extra + t * width + c, e);
-  candidate_sum(branch + t * top * width, mix ? mix + t * top : nullptr, top, width, c, z);
+  b.sum(y, m, top, width, c, z);
+  if (extra) {
+    ex.get(e);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z[i] += e[i];
+  }
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { if (extra) z[i] += e[i]; ss += z[i] * z[i]; }
-  const float r = 1.f / sqrtf(row_sum(live ? ss : 0.f, red) / width + eps);
+  for (int i = 0; i < 4; ++i) ss += z[i] * z[i];
+  const float r = 1.f / sqrtf(row_sum(live ? ss : 0.f, red, width) / width + eps);
   float s2 = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) { v[i] += z[i] * r * wc[i]; s2 += v[i] * v[i]; }
   if (live) Lanes<float, 4>::store(x + t * width + c, v);
   if (!next_w) return;
-  const float r2 = 1.f / sqrtf(row_sum(live ? s2 : 0.f, red + 16) / width + eps);
+  const float r2 = 1.f / sqrtf(row_sum(live ? s2 : 0.f, red + 16, width) / width + eps);
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] *= r2 * nw[i];
   if (live) Lanes<T, 4>::store(h + t * width + c, v);

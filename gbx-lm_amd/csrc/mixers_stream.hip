@@ -106,7 +106,9 @@ __global__ __launch_bounds__(NT) void hyper_step_kernel(float* __restrict__ X, c
 // The same for rows whose channels fit a workgroup in groups of four (row_threads): latency-bound in decode steps, memory-bound in prompts.
 // One trip to memory: the streams, the sublayer's output and the norm's weights are loaded together.
 // (1 row of 4 streams x 1024 channels: 8.5 -> 3.8 us; 2266 rows x 2048: 42.5 -> 29.9 us.)
-template <typename T, int S>
+// FEW: every number of the step is asked for at the start, one trip instead of three, for the registers of a third fewer waves, which many rows would miss
+// (each where it is first used | this, us: a token of 59 launches, ten of them this one, 1 row of 4 streams x 1024, 187.7 | 185.2; a prompt of 2266 rows x 2048 2675 | 2686).
+template <typename T, int S, bool FEW>
 __global__ __launch_bounds__(1024) void hyper_step_row_kernel(float* __restrict__ X, const T* __restrict__ y, const float* __restrict__ y_mix,
                                                              const float* __restrict__ mix, const float* __restrict__ write, const float* __restrict__ read,
                                                              const float* __restrict__ norm_w, const float* __restrict__ norm_b, T* __restrict__ h,
@@ -116,24 +118,52 @@ __global__ __launch_bounds__(1024) void hyper_step_row_kernel(float* __restrict_
   const bool live = static_cast<int>(threadIdx.x) * 4 < width;
   const int c = live ? threadIdx.x * 4 : width - 4;
   float* xr = X + t * S * width + c;
-  float xs[S][4], z[4], nw[4], nb[4], u[4];
+  const T* yt = y ? y + t * top * width : nullptr;
+  const float* ym = y_mix ? y_mix + t * top : nullptr;
+  if constexpr (FEW) at_hand(X, yt, ym, mix, write, read, norm_w, norm_b, h, out_u);
+  float xs[S][4], nw[4], nb[4], u[4];
+  Branch<T, FEW> b;
+  if (FEW && y) b.ask(yt, ym, top, width, c);
 #pragma unroll
   for (int i = 0; i < S; ++i) Lanes<float, 4>::load(xr + i * width, xs[i]);
   if (norm_w) {
     Lanes<float, 4>::load(norm_w + c, nw);
     Lanes<float, 4>::load(norm_b + c, nb);
   }
+  const auto reads = [&](int j) { return read ? read[j] : 1.f; };
+  float rd[S], wr[S], mx[S][S], z[4];
+  if constexpr (FEW) {
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+      rd[j] = reads(j);
+      if (y) {
+        wr[j] = write[j];
+#pragma unroll
+        for (int i = 0; i < S; ++i) mx[i][j] = mix[i * S + j];
+      }
+    }
+  }
 #pragma unroll
   for (int k = 0; k < 4; ++k) u[k] = 0.f;
   if (y) {
-    candidate_sum(y + t * top * width, y_mix ? y_mix + t * top : nullptr, top, width, c, z);
+    if constexpr (FEW) {
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        at_hand(rd[j]);
+        at_hand(wr[j]);
+#pragma unroll
+        for (int i = 0; i < S; ++i) at_hand(mx[i][j]);
+      }
+    }
+    if constexpr (!FEW) b.ask(yt, ym, top, width, c);
+    b.sum(yt, ym, top, width, c, z);
 #pragma unroll
     for (int j = 0; j < S; ++j) {
-      const float wj = write[j], rj = read ? read[j] : 1.f;
+      const float wj = FEW ? wr[j] : write[j], rj = FEW ? rd[j] : reads(j);
       float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < S; ++i) {
-        const float m = mix[i * S + j];
+        const float m = FEW ? mx[i][j] : mix[i * S + j];
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] += m * xs[i][k];
       }
@@ -147,7 +177,7 @@ __global__ __launch_bounds__(1024) void hyper_step_row_kernel(float* __restrict_
   } else {
 #pragma unroll
     for (int j = 0; j < S; ++j) {
-      const float rj = read ? read[j] : 1.f;
+      const float rj = FEW ? rd[j] : reads(j);
 #pragma unroll
       for (int k = 0; k < 4; ++k) u[k] += rj * xs[j][k];
     }
@@ -156,23 +186,27 @@ __global__ __launch_bounds__(1024) void hyper_step_row_kernel(float* __restrict_
     if (live) Lanes<float, 4>::store(out_u + t * width + c, u);
     return;
   }
-  const float mean = row_sum(live ? (u[0] + u[1]) + (u[2] + u[3]) : 0.f, red) / width;
+  const float mean = row_sum(live ? (u[0] + u[1]) + (u[2] + u[3]) : 0.f, red, width) / width;
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) { u[k] -= mean; ss += u[k] * u[k]; }
-  const float r = 1.f / sqrtf(row_sum(live ? ss : 0.f, red + 16) / width + eps);
+  const float r = 1.f / sqrtf(row_sum(live ? ss : 0.f, red + 16, width) / width + eps);
 #pragma unroll
   for (int k = 0; k < 4; ++k) u[k] = u[k] * r * nw[k] + nb[k];
   if (live) Lanes<T, 4>::store(h + t * width + c, u);
 }
 
+constexpr unsigned FEW_ROWS = 256;        // a workgroup a CU at most: nothing else hides a trip
 template <typename T>
 void launch_hyper_step(int S, dim3 grid, size_t lds, hipStream_t s, float* X, const void* y, const float* y_mix, const float* mix, const float* write,
                        const float* read, const float* norm_w, const float* norm_b, void* h, float* out_u, int width, int top, float eps) {
   const int nt = all_aligned(16, X, norm_w, norm_b, out_u) && all_aligned(4 * sizeof(T), static_cast<const T*>(y), static_cast<const T*>(h)) ? row_threads(width) : 0;
+  const bool few = S <= 4 && grid.x <= FEW_ROWS;
+#define GBXM_HS_ROW(N, FEW_) \
+  hyper_step_row_kernel<T, N, FEW_><<<grid, nt, 0, s>>>(X, static_cast<const T*>(y), y_mix, mix, write, read, norm_w, norm_b, static_cast<T*>(h), out_u, width, top, eps)
 #define GBXM_HS(N)                                                                                                                                    \
-  if (nt) hyper_step_row_kernel<T, N><<<grid, nt, 0, s>>>(X, static_cast<const T*>(y), y_mix, mix, write, read, norm_w, norm_b, static_cast<T*>(h), out_u, \
-                                                          width, top, eps);                                                                           \
+  if (nt && few) GBXM_HS_ROW(N, N <= 4);                                                                                                              \
+  else if (nt) GBXM_HS_ROW(N, false);                                                                                                                 \
   else hyper_step_kernel<T, N><<<grid, NT, lds, s>>>(X, static_cast<const T*>(y), y_mix, mix, write, read, norm_w, norm_b, static_cast<T*>(h), out_u, width, \
                                                      top, eps)
   switch (S) {
@@ -186,6 +220,7 @@ void launch_hyper_step(int S, dim3 grid, size_t lds, hipStream_t s, float* X, co
     default: GBXM_HS(8); break;
   }
 #undef GBXM_HS
+#undef GBXM_HS_ROW
 }
 
 // V channels per thread and pass; with `scale` row t is also multiplied by scale[t * scale_row] before it is rounded.

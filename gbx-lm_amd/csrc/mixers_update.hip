@@ -103,38 +103,36 @@ template <typename T>
 __global__ __launch_bounds__(1024) void layer_update_row_kernel(gbxm_layer_update_args p) {
   __shared__ float red[16];
   const int64_t t = blockIdx.x;
-  const int width = p.width, c = threadIdx.x * 4;
+  const int width = p.width, top = p.top, c = threadIdx.x * 4;
   const bool on = c < width;
+  const T* y = p.cand ? static_cast<const T*>(p.cand) + t * top * width : nullptr;
+  const float* m = p.mix ? p.mix + t * p.mix_row : nullptr;
+  at_hand(p.x, p.branch, y, m, p.extra, p.norm_w, p.h, p.image);
   float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4];
   if (on) {
-    float x[4] = {0.f, 0.f, 0.f, 0.f}, ex[4] = {0.f, 0.f, 0.f, 0.f};
-    if (!p.replace) Lanes<float, 4>::load(p.x + t * width + c, x);
+    Candidates<T> cand;
+    Raw4<T> br, ex;
+    Raw4<float> old;
+    if (p.cand) cand.ask(y, m, 0, top, width, c);
+    if (p.branch) br.load(static_cast<const T*>(p.branch) + t * p.branch_row + c);
+    if (p.extra) ex.load(static_cast<const T*>(p.extra) + t * width + c);
+    if (!p.replace) old.load(p.x + t * width + c);
     if (p.norm_w) Lanes<float, 4>::load(p.norm_w + c, w);
-    if (p.branch) Lanes<T, 4>::load(static_cast<const T*>(p.branch) + t * p.branch_row + c, v);
-    if (p.extra) Lanes<T, 4>::load(static_cast<const T*>(p.extra) + t * width + c, ex);
+    if (p.branch) br.get(v);
     if (p.cand) {
-      const T* cand = static_cast<const T*>(p.cand) + t * p.top * width + c;
-      const float* mix = p.mix ? p.mix + t * p.mix_row : nullptr;
-      for (int k0 = 0; k0 < p.top; k0 += 8) {
-        float u[8][4];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) Lanes<T, 4>::load(cand + static_cast<int64_t>(min(k0 + k, p.top - 1)) * width, u[k]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (k0 + k < p.top) {
-            const float m = mix ? mix[k0 + k] : 1.f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] += m * u[k][i];
-          }
-      }
+      cand.add(0, top, v);
+      cand.rest(y, m, top, width, c, v);
     }
+    float x[4] = {0.f, 0.f, 0.f, 0.f}, e[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.extra) ex.get(e);
+    if (!p.replace) old.get(x);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = (v[i] + ex[i]) + x[i];
+    for (int i = 0; i < 4; ++i) v[i] = (v[i] + e[i]) + x[i];
     Lanes<float, 4>::store(p.x + t * width + c, v);
     if (p.image) Lanes<T, 4>::store(static_cast<T*>(p.image) + t * p.image_row + c, v);
   }
   if (!p.norm_w) return;
-  const float r = 1.f / sqrtf(row_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], red) / width + p.eps);
+  const float r = 1.f / sqrtf(row_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], red, width) / width + p.eps);
   if (!on) return;
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] *= w[i] * r;
