@@ -65,3 +65,16 @@ def test_modules_share_a_launch(rows):
         assert ops.quantized_matmul_prompt(x, mods) is None               # what watches a module sees its call
         handle.remove()
     ops.dense_cache_clear()
+
+
+def test_a_batch_keeps_its_sums(monkeypatch):
+    """Several sequences' rows take each product alone, one sequence's together."""
+    from gbx_lm_amd import synthetic as S
+    from gbx_lm_amd.models.cache import make_prompt_cache
+    model = S.build_model(S.TINY, S.make_strategy("S40", 2), device="cuda:0", seed=0)
+    calls = []
+    monkeypatch.setattr(ops, "quantized_matmul_prompt", lambda x, mods: calls.append(x.shape[0]))
+    with torch.no_grad():
+        for rows, length in ((4, 300), (1, 300)):
+            model(torch.ones((rows, length), dtype=torch.long, device="cuda:0"), cache=make_prompt_cache(model))
+    assert calls and set(calls) == {1}
