@@ -309,6 +309,11 @@ int gbx_gather_qlinear_forward(const void* x, const uint32_t* qweight, const voi
   if ((K % 128) != 0 || K > max_k)
     return fail(GBX_ERR_UNSUPPORTED, "gather path needs K %% 128 == 0 and K <= %d at %d bits (K = %d)", max_k, bits, K);
   if ((static_cast<long long>(N) * (K / 32 * bits) * 4) % 16 != 0) return fail(GBX_ERR_UNSUPPORTED, "expert stride must keep 16-byte alignment");
+  if (gbx::gemv_pairs_takes(N, K, bits)) {
+    const hipError_t pe = gbx::launch_gemv_pairs(x, &qweight, &scales, &zeros, 1, bias, indices, y, pairs, x_div, num_experts, N, K, bits, log2_group(group_size),
+                                                 act_dtype == GBX_BF16, static_cast<hipStream_t>(hip_stream));
+    return pe == hipSuccess ? GBX_OK : hip_fail(pe, "gbx_gather_qlinear_forward launch");
+  }
   gbx::GemvArgs a{};
   a.x = x;
   a.seg[0] = gbx::GemvSeg{qweight, static_cast<const unsigned short*>(scales), static_cast<const unsigned short*>(zeros),
@@ -347,6 +352,13 @@ int gbx_gather_swiglu_forward(const void* x, const uint32_t* gate_qweight, const
   if ((K % 128) != 0 || K > max_k)
     return fail(GBX_ERR_UNSUPPORTED, "gather path needs K %% 128 == 0 and K <= %d at %d bits (K = %d)", max_k, bits, K);
   if ((static_cast<long long>(N) * (K / 32 * bits) * 4) % 16 != 0) return fail(GBX_ERR_UNSUPPORTED, "expert stride must keep 16-byte alignment");
+  if (gbx::gemv_pairs_takes(N, K, bits)) {
+    const uint32_t* const qs[2] = {gate_qweight, up_qweight};
+    const void *const ss[2] = {gate_scales, up_scales}, *const zs[2] = {gate_zeros, up_zeros};
+    const hipError_t pe = gbx::launch_gemv_pairs(x, qs, ss, zs, 2, nullptr, indices, y, pairs, x_div, num_experts, N, K, bits, log2_group(group_size),
+                                                 act_dtype == GBX_BF16, static_cast<hipStream_t>(hip_stream));
+    return pe == hipSuccess ? GBX_OK : hip_fail(pe, "gbx_gather_swiglu_forward launch");
+  }
   gbx::GemvArgs a{};
   a.x = x;
   a.seg[0] = gbx::GemvSeg{gate_qweight, static_cast<const unsigned short*>(gate_scales), static_cast<const unsigned short*>(gate_zeros),

@@ -149,6 +149,10 @@ hipError_t launch_eminf(const void* logits, float* cur, float* nxt, float* out_e
                         float threshold, int num_steps, hipStream_t s);
 hipError_t launch_attn_static(const void* q, const void* kcache, const void* vcache, const long long* pos, void* out, int batch,
                               int n_heads, int n_kv, int head_dim, int capacity, float sm_scale, bool bf16, hipStream_t s);
+// a few (token, slot) pairs of experts, rows of one slot a lane (gemv_pairs.hip): one matrix, or gate and up of a SwiGLU
+bool gemv_pairs_takes(int N, int K, int bits);
+hipError_t launch_gemv_pairs(const void* x, const uint32_t* const* w, const void* const* scales, const void* const* zeros, int matrices, const void* bias,
+                             const int32_t* idx, void* y, int pairs, int x_div, int E, int N, int K, int bits, int log2g, bool bf16, hipStream_t s);
 hipError_t launch_moe_route(const void* logits, int* inds, void* scores, int T, int E, int k, int mode, int renorm, bool bf16,
                             hipStream_t s);
 hipError_t launch_moe_combine(const void* y, const void* scores, void* out, int T, int k, int D, bool bf16, hipStream_t s,
