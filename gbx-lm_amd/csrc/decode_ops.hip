@@ -308,46 +308,78 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
   const int d0 = (lane % LP) * 8, sub = lane / LP;
   const unsigned short* kbase = a.kcache + static_cast<size_t>(kvh) * a.capacity * HD;
   const unsigned short* vbase = a.vcache + static_cast<size_t>(kvh) * a.capacity * HD;
-  // Slice form (batched decode): loads return in order, and RoPE needs this thread's 2 x 8 slice values (12 KB per workgroup), not the
-  // 64 KB of speculative cache rows -- so the slices are requested FIRST (one (head, pair) item per thread when the workgroup is wide
-  // enough; the v values by the first HD threads) and summed when RoPE gets to them.
+  // Loads return in order, and RoPE needs this thread's own values (slices: 12 KB per workgroup), not the 64 KB of cache rows -- so they are requested FIRST
+  // (one (head, pair) item per thread when the workgroup is wide enough; the v values by the first HD threads) and summed when RoPE gets to them.
   constexpr int NIT = (REP + 1) * (HD / 2);
-  const bool pre = !STATIC && a.qkv_ws != nullptr && NT >= NIT && NT >= HD;
+  constexpr bool ONE = !STATIC && NT >= NIT && NT >= HD;
+  const bool pre = ONE && a.qkv_ws != nullptr;
   float ps1[8], ps2[8], psv[8];
-  if (pre) {
-    const float* wsrow0 = a.qkv_ws + static_cast<size_t>(blockIdx.y) * ((a.n_heads + 2 * a.n_kv) * HD);
+  unsigned short e1 = 0, e2 = 0, ev = 0, w1 = 0, w2 = 0;
+  float freq = 0.f;
+  if constexpr (ONE) {
     const int pp = min(tid, NIT - 1);
     const int hh = pp / (HD / 2), i = pp % (HD / 2);
-    const int col = hh == REP ? a.n_heads * HD + kvh * HD : (hq0 + hh) * HD;
     const int i1 = a.traditional ? 2 * i : i, i2 = a.traditional ? 2 * i + 1 : i + HD / 2;
-    const float* pv = wsrow0 + (a.n_heads + a.n_kv) * HD + kvh * HD + min(tid, HD - 1);
+    if (pre) {
+      const float* wsrow0 = a.qkv_ws + static_cast<size_t>(blockIdx.y) * ((a.n_heads + 2 * a.n_kv) * HD);
+      const int col = hh == REP ? a.n_heads * HD + kvh * HD : (hq0 + hh) * HD;
+      const float* pv = wsrow0 + (a.n_heads + a.n_kv) * HD + kvh * HD + min(tid, HD - 1);
 #pragma unroll
-    for (int sl = 0; sl < 8; ++sl) {
-      const size_t so = static_cast<size_t>(min(sl, a.qkv_slices - 1)) * a.qkv_mn;
-      ps1[sl] = wsrow0[col + i1 + so];
-      ps2[sl] = wsrow0[col + i2 + so];
-      psv[sl] = pv[so];
+      for (int sl = 0; sl < 8; ++sl) {
+        const size_t so = static_cast<size_t>(min(sl, a.qkv_slices - 1)) * a.qkv_mn;
+        ps1[sl] = wsrow0[col + i1 + so];
+        ps2[sl] = wsrow0[col + i2 + so];
+        psv[sl] = pv[so];
+      }
+    } else {
+      const unsigned short* src = hh == REP ? a.k + static_cast<size_t>(kvh) * HD : a.q + (static_cast<size_t>(hq0) + hh) * HD;
+      e1 = src[i1];
+      e2 = src[i2];
+      ev = a.v[static_cast<size_t>(kvh) * HD + min(tid, HD - 1)];
     }
+    if (a.qn_w) {
+      const unsigned short* w = hh == REP ? a.kn_w : a.qn_w;
+      w1 = w[i1];
+      w2 = w[i2];
+    }
+    freq = a.inv_freq[i];
   }
+  const int nsplit = a.ws ? static_cast<int>(gridDim.z) : 1, sp = a.ws ? static_cast<int>(blockIdx.z) : 0;
   u32x4 k0[UB0], v0[UB0];
 #pragma unroll
-  for (int u = 0; u < UB0; ++u) {                   // first 4 * 4 * PPW positions requested before *pos is known
-    const int tc = min(wave * PPW + u * NW * PPW + sub, a.capacity - 1);
+  for (int u = 0; u < UB0; ++u) {                   // first 4 * 4 * PPW positions requested before *pos is known (further slices of a context: one row)
+    const int tc = sp == 0 ? min(wave * PPW + u * NW * PPW + sub, a.capacity - 1) : 0;
     k0[u] = *reinterpret_cast<const u32x4*>(kbase + static_cast<size_t>(tc) * HD + d0);
     v0[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(tc) * HD + d0);
   }
   const int pos = static_cast<int>(*a.pos);
   const int nctx = STATIC ? pos + 1 : pos;          // cached positions to visit
   // this workgroup's slice of them (all of them unless the launch splits the context)
-  const int nsplit = a.ws ? static_cast<int>(gridDim.z) : 1, sp = a.ws ? static_cast<int>(blockIdx.z) : 0;
   const int per = nsplit > 1 ? (((nctx + nsplit - 1) / nsplit + NW * PPW - 1) / (NW * PPW)) * (NW * PPW) : nctx;
   const int tb = sp * per, te = min(nctx, tb + per);
   const bool last_split = sp == nsplit - 1;
+  // ... and the first block of the sweep behind them: its trip to memory runs beside the norms and RoPE (behind their barrier it was one more in the chain).  The
+  // eight waves of the wide form have it behind the barrier: a batch's 64 KB of slices a workgroup keep the memory pipe busy until then (32 sequences of a whole model 0.5 %
+  // slower).  A head's sum of squares stays in its wave (before: LDS atomics and a barrier).  Before | now, us a launch, heads of 128: one sequence with q / k norms, 32 heads on
+  // 4, context 130 7.8 | 6.4, 530 9.1 | 7.4, 1500 10.9 | 8.7; eight of 300, 24 on 8 10.8 | 9.2; 32 of 250 from slices, 24 on 8 12.9 | 10.7, 32 on 8 13.4 | 12.7;
+  // two of 3000, 32 on 8 15.0 | 13.2.
+  constexpr int UB = 4;
+  const int tm = (sp == 0 ? UB0 * NW * PPW : tb) + wave * PPW;
+  u32x4 kv4[UB], vv4[UB];
+  auto ask = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < UB; ++u) {
+      const int t = t0 + u * NW * PPW + sub, tc = t < te ? t : max(te - 1, 0);
+      kv4[u] = *reinterpret_cast<const u32x4*>(kbase + static_cast<size_t>(tc) * HD + d0);
+      vv4[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(tc) * HD + d0);
+    }
+  };
+  constexpr bool EARLY = NW == 4;
+  if constexpr (EARLY) ask(tm);
 
   if constexpr (STATIC) {
     for (int p = tid; p < REP * HD; p += NT) q_s[p / HD][p % HD] = act_to_f32<BF16>(a.q[static_cast<size_t>(hq0) * HD + p]) * a.sm_scale;
   } else {
-  __shared__ float ssq_s[REP + 1];
   // projection output (+ bias, rounded to the activation dtype like the projection's own `+ bias`)
   // (`col`: first column of this head inside the concatenated q | k | v row, for the slice form)
   const int qkv_n = (a.n_heads + 2 * a.n_kv) * HD;
@@ -374,26 +406,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
         x = sum8(t);
       }
     } else {
-      x = act_to_f32<BF16>(src[i]);
+      x = act_to_f32<BF16>(!ONE || which == 0 ? src[i] : which == 1 ? e1 : which == 2 ? e2 : ev);
     }
     return bias ? act_to_f32<BF16>(f32_to_act<BF16>(x + act_to_f32<BF16>(bias[i]))) : x;
   };
   const int col_k = a.n_heads * HD + kvh * HD, col_v = (a.n_heads + a.n_kv) * HD + kvh * HD;
   const bool normed = a.qn_w != nullptr;
   const bool writer = blockIdx.x % parts == 0 && blockIdx.z == 0;   // one workgroup of the kv group appends k, v
-  if (normed) {                                     // sum of squares per head (q heads of this part, then the k head)
-    if (tid <= REP) ssq_s[tid] = 0.f;
-    __syncthreads();
-    for (int p = tid; p < (REP + 1) * (HD / 2); p += NT) {
-      const int hh = p / (HD / 2), i = p % (HD / 2);
-      const unsigned short* src = hh == REP ? a.k + static_cast<size_t>(kvh) * HD : a.q + (static_cast<size_t>(hq0) + hh) * HD;
-      const unsigned short* bsrc = !a.q_bias ? nullptr : hh == REP ? a.k_bias + static_cast<size_t>(kvh) * HD : a.q_bias + (static_cast<size_t>(hq0) + hh) * HD;
-      const int col = hh == REP ? col_k : (hq0 + hh) * HD;
-      const float x1 = ldb(col, src, bsrc, 2 * i), x2 = ldb(col, src, bsrc, 2 * i + 1);
-      atomicAdd(&ssq_s[hh], x1 * x1 + x2 * x2);
-    }
-    __syncthreads();
-  }
   // RoPE on the REP query heads and the kv head's k; append k, v to the cache
   for (int p = tid; p < (REP + 1) * (HD / 2); p += NT) {
     const int hh = p / (HD / 2), i = p % (HD / 2);   // hh == REP: the k head
@@ -403,14 +422,23 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
     const int i2 = a.traditional ? 2 * i + 1 : i + HD / 2;
     const unsigned short* bsrc = !a.q_bias ? nullptr : isk ? a.k_bias + static_cast<size_t>(kvh) * HD : a.q_bias + (static_cast<size_t>(hq0) + hh) * HD;
     const int col = isk ? col_k : (hq0 + hh) * HD;
-    float x1 = ldb(col, src, bsrc, i1, pre ? 1 : 0), x2 = ldb(col, src, bsrc, i2, pre ? 2 : 0);     // (pre: one item per thread, p == tid)
+    float x1 = ldb(col, src, bsrc, i1, ONE ? 1 : 0), x2 = ldb(col, src, bsrc, i2, ONE ? 2 : 0);     // (ONE: one item per thread, p == tid)
     if (normed) {                                   // RMSNorm output rounded to the activation dtype, like the separate op
-      const float rstd = rsqrtf(ssq_s[hh] / static_cast<float>(HD) + a.norm_eps);
+      float ssq = x1 * x1 + x2 * x2;                // (a head's pairs lie in HD / 2 neighbouring lanes of one wave)
+      if constexpr (HD == 128) ssq = wave_sum(ssq);
+      else {
+        ssq += dpp_f32<0xB1>(ssq);
+        ssq += dpp_f32<0x4E>(ssq);
+        ssq += dpp_f32<0x141>(ssq);
+        ssq += dpp_f32<0x140>(ssq);
+        ssq += __shfl_xor(ssq, 16, 64);
+      }
+      const float rstd = rsqrtf(ssq / static_cast<float>(HD) + a.norm_eps);
       const unsigned short* w = isk ? a.kn_w : a.qn_w;
-      x1 = act_to_f32<BF16>(f32_to_act<BF16>(x1 * rstd * act_to_f32<BF16>(w[i1])));
-      x2 = act_to_f32<BF16>(f32_to_act<BF16>(x2 * rstd * act_to_f32<BF16>(w[i2])));
+      x1 = act_to_f32<BF16>(f32_to_act<BF16>(x1 * rstd * act_to_f32<BF16>(ONE ? w1 : w[i1])));
+      x2 = act_to_f32<BF16>(f32_to_act<BF16>(x2 * rstd * act_to_f32<BF16>(ONE ? w2 : w[i2])));
     }
-    const float rev = static_cast<float>(pos) * a.rope_scale * a.inv_freq[i] * 0.15915494309189535f;
+    const float rev = static_cast<float>(pos) * a.rope_scale * (ONE ? freq : a.inv_freq[i]) * 0.15915494309189535f;
     const float fr = rev - floorf(rev);
     const float sn = __builtin_amdgcn_sinf(fr), cs = __builtin_amdgcn_cosf(fr);
     const unsigned short r1 = f32_to_act<BF16>(x1 * cs - x2 * sn), r2 = f32_to_act<BF16>(x1 * sn + x2 * cs);
@@ -428,7 +456,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
     }
   }
   if (tid < HD) {
-    const unsigned short vb = f32_to_act<BF16>(ldb(col_v, a.v + static_cast<size_t>(kvh) * HD, a.v_bias ? a.v_bias + static_cast<size_t>(kvh) * HD : nullptr, tid, pre ? 3 : 0));
+    const unsigned short vb = f32_to_act<BF16>(ldb(col_v, a.v + static_cast<size_t>(kvh) * HD, a.v_bias ? a.v_bias + static_cast<size_t>(kvh) * HD : nullptr, tid, ONE ? 3 : 0));
     vn_s[tid] = act_to_f32<BF16>(vb);
     if (writer) a.vcache[(static_cast<size_t>(kvh) * a.capacity + pos) * HD + tid] = vb;
   }
@@ -469,24 +497,18 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
       m[r] = mn;
     }
   };
+  if constexpr (!EARLY) ask(tm);
+  if (sp == 0) {                                    // (the speculative first positions)
 #pragma unroll
-  // (the speculative first positions belong to split 0; the other splits start their own slice below)
-  for (int u = 0; u < UB0; ++u) consume(k0[u], v0[u], sp == 0 && wave * PPW + u * NW * PPW + sub < te);
+    for (int u = 0; u < UB0; ++u) consume(k0[u], v0[u], wave * PPW + u * NW * PPW + sub < te);
+  }
   // Main loop: UB positions per lane group as ONE block of the online softmax -- UB independent dot / DPP chains, one
   // rescale of the accumulators per block instead of per position (per position the chain dot -> DPP -> max -> exp ->
   // acc * corr ran serially UB times with a single wave or two per SIMD to hide it: 1.2 TB/s of cache at long contexts).
-  constexpr int UB = 4;
-  for (int t0 = (sp == 0 ? UB0 * NW * PPW : tb) + wave * PPW; t0 < te; t0 += NW * PPW * UB) {
-    u32x4 kv4[UB], vv4[UB];
+  for (int t0 = tm; t0 < te; t0 += NW * PPW * UB) {
     bool valid[UB];
 #pragma unroll
-    for (int u = 0; u < UB; ++u) {
-      const int t = t0 + u * NW * PPW + sub;
-      valid[u] = t < te;
-      const int tc = valid[u] ? t : max(te - 1, 0);
-      kv4[u] = *reinterpret_cast<const u32x4*>(kbase + static_cast<size_t>(tc) * HD + d0);
-      vv4[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(tc) * HD + d0);
-    }
+    for (int u = 0; u < UB; ++u) valid[u] = t0 + u * NW * PPW + sub < te;
     float sc[REP][UB];
 #pragma unroll
     for (int u = 0; u < UB; ++u) {
@@ -526,6 +548,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_gqa_kernel(AttnArgs a) {
         }
       }
     }
+    ask(t0 + NW * PPW * UB);                        // (behind the last block: one row)
   }
   // the new token itself (k, v in LDS)
   if (!STATIC && last_split && wave == 0 && sub == 0) {
