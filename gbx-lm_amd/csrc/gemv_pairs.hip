@@ -26,26 +26,27 @@ struct PairArgs {
   const unsigned short* bias;     // [E, N] or null
   unsigned short* y;              // [pairs, N]
   int N, K, log2g, div, E;
+  // pair_mix_kernel: y [pairs / top, N] = residual + the sum of a token's slots by their weights
+  const unsigned short *mix, *residual;
+  int top;
 };
 
-// LPR: lanes a row.  B: batches of a wave, two accumulators each: a gate and an up row, or two plain rows.
+// LPR: lanes a row.  B: batches of a wave from row `first` on, two accumulators each: a gate and an up row, or two plain rows.  The totals: with LPR 64 in every
+// lane, with LPR 32 those of a half's row in its last lane.
 template <int BITS, bool BF16, bool SPLIT, int LPR, bool SWIGLU, int B>
-__global__ __launch_bounds__(256) void pair_rows_kernel(const PairArgs a) {
+__device__ __forceinline__ void pair_totals(const PairArgs& a, int p, int e, int first, float (&t)[B][2]) {
   using F = Fmt<BITS>;
   using WT = typename SlotWords<BITS>::type;
   constexpr int NSUB = F::NSUB, PAIRS = F::VPL / 2, UP = F::UNIT_PAIRS, UPSUB = 32 / F::UNIT_VALS, NG = SPLIT ? 2 : 1;
   constexpr int RW = 64 / LPR, STEP = SWIGLU ? RW : 2 * RW;             // rows of y a batch
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int N = a.N, K = a.K, p = blockIdx.y, nslots = K / F::VPL;
+  const int lane = threadIdx.x & 63, N = a.N, K = a.K, nslots = K / F::VPL;
   const int half = lane / LPR, sub = lane % LPR, slot = min(sub, nslots - 1);
-  const int e = min(max(a.idx[p], 0), a.E - 1);                         // (a bad index cannot leave the tensors)
   const u32x4* xs4 = reinterpret_cast<const u32x4*>(a.x + static_cast<size_t>(p / a.div) * K + slot * F::VPL);
   u32x4 xr[F::VPL / 8];
 #pragma unroll
   for (int i = 0; i < F::VPL / 8; ++i) xr[i] = xs4[i];
   const int W = K / 32 * BITS, G = K >> a.log2g;
   const int64_t ew = static_cast<int64_t>(e) * N * W, eg = static_cast<int64_t>(e) * N * G;
-  const int first = (blockIdx.x * 4 + wave) * B * STEP;                 // the wave's rows are neighbours
   const int gat = (slot * NSUB) >> (a.log2g - 5);
   WT w[B][2];
   unsigned short sc[B][2][NG], ze[B][2][NG];
@@ -116,12 +117,10 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const PairArgs a) {
         }
       }
     }
-    // totals: LPR 64 wave-uniform; LPR 32 those of a half in its last lane
-    float t[2];
     if constexpr (LPR == 64) {
       const float tot = wave_sum2(acc[0], acc[1]);
-      t[0] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(tot), 31));
-      t[1] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(tot), 63));
+      t[b][0] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(tot), 31));
+      t[b][1] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(tot), 63));
     } else {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -130,29 +129,74 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const PairArgs a) {
         v += dpp_f32<0x4E>(v);
         v += dpp_f32<0x141>(v);
         v += dpp_f32<0x140>(v);
-        t[i] = v + dpp_f32<0x142, 0xA>(v);
+        t[b][i] = v + dpp_f32<0x142, 0xA>(v);
       }
     }
-    const int row = first + b * STEP + half;
-    unsigned short* y = a.y + static_cast<size_t>(p) * N;
-    if (sub == LPR - 1) {
-      if constexpr (SWIGLU) {                                           // every step rounded, as the three operations do
-        const float g = round_bf16_or_f16(t[0], BF16), u = round_bf16_or_f16(t[1], BF16);
-        const float sl = round_bf16_or_f16(g / (1.f + __expf(-g)), BF16);
-        if (row < N) y[row] = f32_to_act<BF16>(sl * u);
-      } else {
+  }
+}
+
+__device__ __forceinline__ int expert_of(const PairArgs& a, int p) { return min(max(a.idx[p], 0), a.E - 1); }      // (a bad index cannot leave the tensors)
+
+template <int BITS, bool BF16, bool SPLIT, int LPR, bool SWIGLU, int B>
+__global__ __launch_bounds__(256) void pair_rows_kernel(const PairArgs a) {
+  constexpr int RW = 64 / LPR, STEP = SWIGLU ? RW : 2 * RW;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = blockIdx.y, e = expert_of(a, p), N = a.N;
+  const int first = (blockIdx.x * 4 + wave) * B * STEP;                 // the wave's rows are neighbours
+  float t[B][2];
+  pair_totals<BITS, BF16, SPLIT, LPR, SWIGLU, B>(a, p, e, first, t);
+  if (lane % LPR != LPR - 1) return;
+  unsigned short* y = a.y + static_cast<size_t>(p) * N;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int r = row + i * RW;
-          if (r < N) {
-            unsigned short v = f32_to_act<BF16>(t[i]);
-            if (a.bias) v = f32_to_act<BF16>(act_to_f32<BF16>(v) + act_to_f32<BF16>(a.bias[static_cast<int64_t>(e) * N + r]));
-            y[r] = v;
-          }
+  for (int b = 0; b < B; ++b) {
+    const int row = first + b * STEP + lane / LPR;
+    if constexpr (SWIGLU) {                                             // every step rounded, as the three operations do
+      const float g = round_bf16_or_f16(t[b][0], BF16), u = round_bf16_or_f16(t[b][1], BF16);
+      const float sl = round_bf16_or_f16(g / (1.f + __expf(-g)), BF16);
+      if (row < N) y[row] = f32_to_act<BF16>(sl * u);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = row + i * RW;
+        if (r < N) {
+          unsigned short v = f32_to_act<BF16>(t[b][i]);
+          if (a.bias) v = f32_to_act<BF16>(act_to_f32<BF16>(v) + act_to_f32<BF16>(a.bias[static_cast<int64_t>(e) * N + r]));
+          y[r] = v;
         }
       }
     }
   }
+}
+
+// The last products of a token's up to eight experts with their weighted sum and the block's residual, every step rounded as moe_combine_kernel does: a wave a slot, the
+// same few rows in each, which meet in LDS.  A launch less in a chain of launches that take one trip to memory each.  Two launches | this, us, 8 slots of 128
+// experts, 2048 x 768 at 3 bits, 1 token 7.5 | 4.1, 8 tokens 17.0 | 15.0.
+constexpr int MIX_ROWS = 8;
+template <int BITS, bool BF16, bool SPLIT, int LPR>
+__global__ __launch_bounds__(512) void pair_mix_kernel(const PairArgs a) {
+  constexpr int RW = 64 / LPR, B = MIX_ROWS / (2 * RW);
+  __shared__ float part[8][MIX_ROWS];
+  const int lane = threadIdx.x & 63, slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), N = a.N, first = blockIdx.x * MIX_ROWS;
+  const int64_t token = blockIdx.y;
+  const int row = first + min(static_cast<int>(threadIdx.x), MIX_ROWS - 1);
+  const float res = a.residual && threadIdx.x < MIX_ROWS ? act_to_f32<BF16>(a.residual[token * N + min(row, N - 1)]) : 0.f;
+  if (slot < a.top) {
+    const int p = blockIdx.y * a.top + slot;
+    const float w = act_to_f32<BF16>(a.mix[p]);
+    float t[B][2];
+    pair_totals<BITS, BF16, SPLIT, LPR, false, B>(a, p, expert_of(a, p), first, t);
+    if (lane % LPR == LPR - 1) {
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) part[slot][(b * 2 + i) * RW + lane / LPR] = round_bf16_or_f16(w * round_bf16_or_f16(t[b][i], BF16), BF16);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x >= MIX_ROWS || row >= N) return;
+  float v = 0.f;
+  for (int s = 0; s < a.top; ++s) v += part[s][threadIdx.x];
+  if (a.residual) v = res + round_bf16_or_f16(v, BF16);
+  a.y[token * N + row] = f32_to_act<BF16>(v);
 }
 
 template <int BITS, bool BF16, bool SPLIT, int LPR, bool SWIGLU>
@@ -170,6 +214,12 @@ void launch_pairs(const PairArgs& a, int pairs, hipStream_t s) {
 template <int BITS, bool BF16, bool SPLIT>
 void launch_pairs_rows(const PairArgs& a, int pairs, bool swiglu, hipStream_t s) {
   const bool two = a.K / Fmt<BITS>::VPL <= 32;
+  if (a.mix) {
+    const dim3 grid((a.N + MIX_ROWS - 1) / MIX_ROWS, pairs / a.top);
+    if (two) hipLaunchKernelGGL((pair_mix_kernel<BITS, BF16, SPLIT, 32>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((pair_mix_kernel<BITS, BF16, SPLIT, 64>), grid, dim3(512), 0, s, a);
+    return;
+  }
   if (swiglu) two ? launch_pairs<BITS, BF16, SPLIT, 32, true>(a, pairs, s) : launch_pairs<BITS, BF16, SPLIT, 64, true>(a, pairs, s);
   else two ? launch_pairs<BITS, BF16, SPLIT, 32, false>(a, pairs, s) : launch_pairs<BITS, BF16, SPLIT, 64, false>(a, pairs, s);
 }
@@ -187,6 +237,13 @@ bool gemv_pairs_takes(int N, int K, int bits) {
   return K / (bits == 2 ? 64 : 32) <= 64 && static_cast<int64_t>(N) * (K / 32 * bits) * 4 <= INT32_MAX;      // (one slot a lane; 32-bit offsets in an expert)
 }
 
+static hipError_t launch_pairs_args(const PairArgs& a, int pairs, int bits, bool swiglu, bool bf16, hipStream_t s) {
+  if (bits == 2) launch_pairs_bits<2>(a, pairs, swiglu, bf16, s);
+  else if (bits == 3) launch_pairs_bits<3>(a, pairs, swiglu, bf16, s);
+  else launch_pairs_bits<4>(a, pairs, swiglu, bf16, s);
+  return hipGetLastError();
+}
+
 hipError_t launch_gemv_pairs(const void* x, const uint32_t* const* w, const void* const* scales, const void* const* zeros, int matrices, const void* bias,
                              const int32_t* idx, void* y, int pairs, int x_div, int E, int N, int K, int bits, int log2g, bool bf16, hipStream_t s) {
   PairArgs a{};
@@ -196,11 +253,27 @@ hipError_t launch_gemv_pairs(const void* x, const uint32_t* const* w, const void
   a.bias = static_cast<const unsigned short*>(bias);
   a.y = static_cast<unsigned short*>(y);
   a.N = N; a.K = K; a.log2g = log2g; a.div = x_div; a.E = E;
-  const bool swiglu = matrices == 2;
-  if (bits == 2) launch_pairs_bits<2>(a, pairs, swiglu, bf16, s);
-  else if (bits == 3) launch_pairs_bits<3>(a, pairs, swiglu, bf16, s);
-  else launch_pairs_bits<4>(a, pairs, swiglu, bf16, s);
-  return hipGetLastError();
+  return launch_pairs_args(a, pairs, bits, matrices == 2, bf16, s);
 }
 
 }  // namespace gbx
+
+// y[t] = residual[t] (or nothing) + sum_s mix[t, s] * (expert idx[t, s] of the stacked [E, N, ...] matrices times x[t, s]), rounded like the product, the elementwise
+// multiply, the sum and the add.  For this package's own Python layer; not part of the public header.  Non-zero: the caller runs the steps (nothing was launched).
+extern "C" int gbx_gather_mix_forward(const void* x, const uint32_t* qweight, const void* scales, const void* zeros, const int32_t* indices, const void* mix,
+                                      const void* residual, void* y, int32_t tokens, int32_t top, int32_t num_experts, int32_t N, int32_t K, int32_t bits,
+                                      int32_t group_size, int32_t bf16, void* hip_stream) {
+  const auto off = [](const void* p, unsigned n) { return reinterpret_cast<uintptr_t>(p) % n != 0; };
+  if (!x || !qweight || !scales || !zeros || !indices || !mix || !y || tokens < 1 || tokens > 65535 || top < 1 || top > 8 || num_experts < 1 || N < 1) return 1;
+  if (bits < 2 || bits > 4 || (group_size != 32 && group_size != 64 && group_size != 128) || K < 128 || K % 128 || !gbx::gemv_pairs_takes(N, K, bits)) return 1;
+  if (off(x, 16) || off(qweight, 16) || (static_cast<int64_t>(N) * (K / 32 * bits) * 4) % 16) return 1;
+  gbx::PairArgs a{};
+  a.x = static_cast<const unsigned short*>(x);
+  a.m[0] = gbx::PairMatrix{qweight, static_cast<const unsigned short*>(scales), static_cast<const unsigned short*>(zeros)};
+  a.idx = indices;
+  a.mix = static_cast<const unsigned short*>(mix);
+  a.residual = static_cast<const unsigned short*>(residual);
+  a.y = static_cast<unsigned short*>(y);
+  a.N = N; a.K = K; a.log2g = group_size == 32 ? 5 : group_size == 64 ? 6 : 7; a.div = 1; a.E = num_experts; a.top = top;
+  return gbx::launch_pairs_args(a, tokens * top, bits, false, bf16 != 0, static_cast<hipStream_t>(hip_stream)) == hipSuccess ? 0 : 2;
+}

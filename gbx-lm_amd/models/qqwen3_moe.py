@@ -22,7 +22,7 @@ from .projection import RowLinear
 from .qllama import RMSNorm
 from .quantized_linear_gba import QuantizedLinear
 from .rope_utils import RoPE
-from .switch_layers import SwitchGLU
+from .switch_layers import SwitchGLU, mixed_experts
 
 
 @dataclass
@@ -124,9 +124,9 @@ class Qwen3MoeSparseMoeBlock(nn.Module):
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``residual`` (decode fast path): returns residual + block(x), the add fused into the mixing launch."""
         if _device_routing(x, self.num_experts, self.top_k):
-            # routing decisions and the weighted sum as two launches (gbx_moe_route / gbx_moe_combine)
+            # routing decisions as one launch (gbx_moe_route), the weighted sum as another or with the last products
             inds, scores = ops.moe_route(self.gate(x), self.top_k, 0, self.norm_topk_prob)
-            return ops.moe_combine(self.switch_mlp(x, inds), scores, residual)
+            return mixed_experts(self.switch_mlp, x, inds, scores, residual)
         if residual is not None:
             return residual + self.forward(x)
         gates = torch.softmax(self.gate(x).float(), dim=-1).to(x.dtype)

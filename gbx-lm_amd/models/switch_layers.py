@@ -103,7 +103,7 @@ class SwitchGLU(nn.Module):
         self.down_proj = cls(hidden_dims, input_dims, num_experts, bias=bias)
         self.activation = activation if activation is not None else SwiGLU()
 
-    def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
+    def _activated(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         x = x.unsqueeze(-2).unsqueeze(-3)                          # [..., 1, 1, D]: one row shared by the k slots
         act = None
         if (isinstance(self.activation, SwiGLU) and isinstance(self.gate_proj, QuantizedSwitchLinear)
@@ -113,8 +113,23 @@ class SwitchGLU(nn.Module):
             x_up = self.up_proj(x, indices)
             x_gate = self.gate_proj(x, indices)
             act = self.activation(x_up, x_gate)
-        y = self.down_proj(act, indices)                            # [..., k, 1, D]
+        return act
+
+    def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
+        y = self.down_proj(self._activated(x, indices), indices)    # [..., k, 1, D]
         return y.squeeze(-2)
+
+
+def mixed_experts(experts: nn.Module, x: torch.Tensor, indices: torch.Tensor, scores: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``moe_combine(experts(x, indices), scores, residual)``; of a few tokens the last products and their sum in one launch, unless something watches or
+    replaces a module on the way."""
+    down = getattr(experts, "down_proj", None)
+    if (type(experts) is SwitchGLU and type(down) is QuantizedSwitchLinear and x.is_cuda and indices.numel() <= 64
+            and not any(m._forward_hooks or m._forward_pre_hooks for m in (experts, down))):
+        act = experts._activated(x, indices)
+        y = ops.gather_mix(act, down, indices, scores, residual)
+        return y if y is not None else ops.moe_combine(down(act, indices).squeeze(-2), scores, residual)
+    return ops.moe_combine(experts(x, indices), scores, residual)
 
 
 class DenseRoutedGLU(nn.Module):

@@ -618,6 +618,26 @@ def gather_swiglu(x: torch.Tensor, gate, up, rhs_indices: torch.Tensor):
     return y.reshape(*rhs_indices.shape[:-1], k, 1, N)
 
 
+def gather_mix(x: torch.Tensor, down, rhs_indices: torch.Tensor, scores: torch.Tensor, residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``moe_combine(down(x, indices), scores, residual)`` of a decode-sized set of (token, slot) pairs in ONE launch (gbx_gather_mix_forward), x [..., k, 1, K],
+    ``down`` a QuantizedSwitchLinear.  None where the launch does not take the call (the caller then runs the two)."""
+    K, N, k = x.shape[-1], down.output_dims, rhs_indices.shape[-1]
+    pairs, lead = rhs_indices.numel(), tuple(rhs_indices.shape[:-1])
+    if not (x.is_cuda and x.dtype in _DT and 0 < pairs <= 64 and k <= 8 and tuple(x.shape) == (*lead, k, 1, K) and K == down.input_dims and K % 128 == 0
+            and K <= 64 * (64 if down.bits == 2 else 32) and down.bias is None and rhs_indices.dtype == torch.int32 and down.scales.dtype == x.dtype
+            and down.zeros.dtype == x.dtype and scores.dtype == x.dtype and tuple(scores.shape) == tuple(rhs_indices.shape)
+            and all(t.is_cuda and t.is_contiguous() for t in (down.qweight, down.scales, down.zeros))
+            and (residual is None or (residual.is_cuda and residual.dtype == x.dtype and tuple(residual.shape) == (*lead, N)))):
+        return None
+    xr, idx, mix = x.reshape(-1, K).contiguous(), rhs_indices.reshape(-1).contiguous(), scores.contiguous()
+    res = None if residual is None else residual.contiguous()
+    y = torch.empty((*lead, N), dtype=x.dtype, device=x.device)
+    rc = _lib.lib().gbx_gather_mix_forward(xr.data_ptr(), down.qweight.data_ptr(), down.scales.data_ptr(), down.zeros.data_ptr(), idx.data_ptr(), mix.data_ptr(),
+                                           None if res is None else res.data_ptr(), y.data_ptr(), pairs // k, k, down.qweight.shape[0], N, K, down.bits,
+                                           down.group_size, int(x.dtype == torch.bfloat16), _stream_ptr(x.device))
+    return y if rc == 0 else None
+
+
 def quantized_swiglu(x: torch.Tensor, gate, up) -> Optional[torch.Tensor]:
     """``silu(gate_proj(x)) * up_proj(x)`` for a decode-sized batch (2..64 rows) in ONE launch (gbx_qlinear_swiglu_forward:
     the no-dequant matrix-core GEMM with the SwiGLU in its epilogue) or for a long prompt (the dense path of >= 1024 / 4096 rows:

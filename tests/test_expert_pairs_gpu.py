@@ -69,3 +69,33 @@ def test_bad_index_and_infinity():
     assert torch.equal(y[0, 0], y[0, 1]) and torch.equal(y[0, 3], y[0, 2])                 # the nearest expert's row
     x[..., 7] = float("inf")
     assert not torch.isfinite(m(x.to(DEV), torch.tensor([[1]]).to(DEV)).float()).any()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,group,K", [(2, 32, 128), (2, 128, 2176), (3, 64, 1152), (3, 128, 768), (4, 32, 1024), (4, 128, 2048)])
+@pytest.mark.parametrize("N,T,top", [(128, 1, 1), (76, 3, 2), (264, 8, 8), (2048, 1, 8)])
+def test_mixed(dt, bits, group, K, N, T, top):
+    """The last products with their weighted sum and residual in one launch: the bits of the two launches."""
+    m = _layer(5, N, K, bits, group, dt, K + N)
+    gen = torch.Generator().manual_seed(T)
+    idx = torch.randint(0, 5, (T, top), generator=gen).to(torch.int32).to(DEV)
+    act = torch.randn((T, top, 1, K), generator=gen).to(dt).to(DEV)
+    scores = torch.softmax(torch.randn((T, top), generator=gen), -1).to(dt).to(DEV)
+    for residual in (None, torch.randn((T, N), generator=gen).to(dt).to(DEV)):
+        both = ops.gather_mix(act, m, idx, scores, residual)
+        assert both is not None and torch.equal(both, ops.moe_combine(m(act, idx).squeeze(-2), scores, residual))
+
+
+def test_what_watches_a_module_sees_its_call():
+    from gbx_lm_amd.models.switch_layers import SwitchGLU, mixed_experts
+    glu = SwitchGLU(256, 128, 4)
+    for name, n, k in (("gate_proj", 128, 256), ("up_proj", 128, 256), ("down_proj", 256, 128)):
+        src, dst = _layer(4, n, k, 4, 64, torch.bfloat16, n), getattr(glu, name)
+        dst.qweight, dst.scales, dst.zeros = src.qweight, src.scales, src.zeros
+    x = torch.randn((1, 3, 256), generator=torch.Generator().manual_seed(0)).bfloat16().to(DEV)
+    idx = torch.tensor([[[0, 1], [3, 2], [1, 1]]], dtype=torch.int32).to(DEV)
+    scores = torch.full((1, 3, 2), 0.5).bfloat16().to(DEV)
+    y, seen = mixed_experts(glu, x, idx, scores, x), []
+    handle = glu.down_proj.register_forward_hook(lambda *a: seen.append(1))
+    assert torch.equal(mixed_experts(glu, x, idx, scores, x), y) and seen == [1]
+    handle.remove()
