@@ -77,6 +77,7 @@ def lib() -> ctypes.CDLL:
             L.gbx_p2p_inbox_bytes.restype = ctypes.c_size_t
         L.gbx_dense_swiglu_forward.argtypes = [p, p, p, i64, i32, i32, i32, p]
         L.gbx_dense_forward_multi.argtypes = [p, i32, p, p, p, p, i64, i32, i32, p]
+        L.gbx_rope_qkv.argtypes = [p, p, p, p, p, p, p, i64, i32, i32, i32, i32, i32, p, i32, i32, ctypes.c_float, i32, i32, p]
         L.gbx_gather_mix_forward.argtypes = [p, p, p, p, p, p, p, p, i32, i32, i32, i32, i32, i32, i32, i32, p]
         L.gbx_dense_workspace_bytes.argtypes = [i64, i32, i32]
         L.gbx_dense_workspace_bytes.restype = ctypes.c_size_t

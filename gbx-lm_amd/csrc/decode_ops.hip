@@ -1632,6 +1632,114 @@ hipError_t launch_rope_kv_write(const void* k, const void* v, void* kcache, void
   return hipGetLastError();
 }
 
+// RoPE of a prompt chunk's queries and of its keys straight into the key cache, and the value rows into theirs, as ONE launch: rope(q), rope(k) and
+// cache.update_and_fetch(k, v) of a block (qllama.py:84-91).  A workgroup takes a token of one sequence; its angles serve all heads.  In rope_tokens_kernel's arithmetic.
+// Bound by a launch's start for few tokens and by the rows' bytes for many.  Two launches | this, us: 17 tokens, 32 heads of 128 on 8 4.8 | 3.1; 3001, 24 on 8 13.4 | 11.1.
+struct RopeRows {
+  const unsigned short* x;
+  unsigned short* y;
+  long long sb, sh, sl;        // of x, in elements
+  long long rows;              // of y per (sequence, head)
+  int heads, t0;               // y's row of token 0
+};
+// (by value: a choice among named variables is one among their addresses, which puts them into scratch memory: 47 us for the last of these)
+template <typename T> __device__ __forceinline__ T choose3(bool first, bool second, T a, T b, T c) { return first ? a + 0 : second ? b + 0 : c + 0; }
+template <bool BF16>
+__global__ __launch_bounds__(256) void rope_qkv_kernel(const RopeRows q, const RopeRows k, const RopeRows v, const float* __restrict__ inv_freq, long long pos0, int D,
+                                                       float scale, int traditional) {
+  __shared__ float sn_s[128], cs_s[128];
+  const int t = blockIdx.x, b = blockIdx.y, half = D / 2, cph = D / 16;
+  if (threadIdx.x < half) {
+    const float ang = static_cast<float>(pos0 + t) * scale * inv_freq[threadIdx.x];
+    float sn, cs;
+    sincosf(ang, &sn, &cs);
+    sn_s[threadIdx.x] = sn;
+    cs_s[threadIdx.x] = cs;
+  }
+  const int nq = q.heads * cph, nk = k.heads * cph, items = nq + 2 * nk;
+  // an item: the 8-channel chunks c and c + D / 16 of a head (traditional: chunks 2 c and 2 c + 1), asked for before the angles are there
+  const unsigned short *xq = q.x + b * q.sb + t * q.sl, *xk = k.x + b * k.sb + t * k.sl, *xv = v.x + b * v.sb + t * v.sl;
+  unsigned short* yq = q.y + (static_cast<long long>(b) * q.heads * q.rows + q.t0 + t) * D;
+  unsigned short *yk = k.y + (static_cast<long long>(b) * k.heads * k.rows + k.t0 + t) * D, *yv = v.y + (static_cast<long long>(b) * v.heads * v.rows + v.t0 + t) * D;
+  const long long hq = q.sh, hk = k.sh, hv = v.sh, oq = q.rows * D, ok = k.rows * D;
+  auto place = [&](int w, bool& turn, const unsigned short*& xr, unsigned short*& yr, int& c) {
+    const bool isq = w < nq, isk = w < nq + nk;
+    const int i = isq ? w : isk ? w - nq : w - nq - nk, h = i / cph;
+    c = i - h * cph;
+    turn = isk;
+    xr = choose3(isq, isk, xq, xk, xv) + h * choose3(isq, isk, hq, hk, hv);
+    yr = choose3(isq, isk, yq, yk, yv) + h * choose3(isq, isk, oq, ok, ok);
+  };
+  bool first = true;
+  for (int w = threadIdx.x; w - static_cast<int>(threadIdx.x) < items; w += 256) {
+    bool turn;
+    const unsigned short* xr;
+    unsigned short* yr;
+    int c;
+    place(min(w, items - 1), turn, xr, yr, c);
+    const int ea = traditional ? 16 * c : 8 * c, eb = traditional ? 16 * c + 8 : half + 8 * c;
+    const u32x4 va = *reinterpret_cast<const u32x4*>(xr + ea), vb = *reinterpret_cast<const u32x4*>(xr + eb);
+    if (first) __syncthreads();
+    first = false;
+    unsigned wa[4] = {va.x, va.y, va.z, va.w}, wb[4] = {vb.x, vb.y, vb.z, vb.w};
+    if (turn && traditional) {                            // pairs (2i, 2i+1)
+      auto rotate = [&](unsigned (&o)[4], int e0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = e0 / 2 + j;
+          float o1, o2;
+          rope_rot(act_lo<BF16>(o[j]), act_hi<BF16>(o[j]), sn_s[i], cs_s[i], o1, o2);
+          o[j] = static_cast<unsigned>(f32_to_act<BF16>(o1)) | (static_cast<unsigned>(f32_to_act<BF16>(o2)) << 16);
+        }
+      };
+      rotate(wa, ea);
+      rotate(wb, eb);
+    } else if (turn) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = c * 8 + 2 * j;
+        float p0, q0, p1, q1;
+        rope_rot(act_lo<BF16>(wa[j]), act_lo<BF16>(wb[j]), sn_s[i], cs_s[i], p0, q0);
+        rope_rot(act_hi<BF16>(wa[j]), act_hi<BF16>(wb[j]), sn_s[i + 1], cs_s[i + 1], p1, q1);
+        wa[j] = static_cast<unsigned>(f32_to_act<BF16>(p0)) | (static_cast<unsigned>(f32_to_act<BF16>(p1)) << 16);
+        wb[j] = static_cast<unsigned>(f32_to_act<BF16>(q0)) | (static_cast<unsigned>(f32_to_act<BF16>(q1)) << 16);
+      }
+    }
+    if (w < items) {
+      *reinterpret_cast<u32x4*>(yr + ea) = u32x4{wa[0], wa[1], wa[2], wa[3]};
+      *reinterpret_cast<u32x4*>(yr + eb) = u32x4{wb[0], wb[1], wb[2], wb[3]};
+    }
+  }
+}
+
+}  // namespace gbx
+
+// For this package's own Python layer; not part of the public header.  q [B, Hq, L, D], k / v [B, H, L, D] through strides (elements), rows D apart by any multiple of 8;
+// qout [B, Hq, L, D], caches [B, H, capacity, D], rows t0 .. t0 + L - 1 written.  Non-zero: nothing was launched (1: not a call for this launch).
+extern "C" int gbx_rope_qkv(const void* q, const void* k, const void* v, void* qout, void* kcache, void* vcache, const float* inv_freq, int64_t pos0, int32_t B, int32_t Hq,
+                            int32_t H, int32_t L, int32_t D, const int64_t* strides, int32_t capacity, int32_t t0, float scale, int32_t traditional, int32_t bf16,
+                            void* hip_stream) {
+  if (!q || !k || !v || !qout || !kcache || !vcache || !inv_freq || !strides || B < 1 || B > 65535 || Hq < 1 || H < 1 || L < 1 || t0 < 0 || capacity - L < t0) return 1;
+  if (D % 16 || D < 16 || D > 256 || static_cast<int64_t>(Hq) + 2 * static_cast<int64_t>(H) > (1 << 20)) return 1;
+  uintptr_t bits = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(qout) |
+                   reinterpret_cast<uintptr_t>(kcache) | reinterpret_cast<uintptr_t>(vcache);
+  if (bits % 16) return 1;
+  for (int i = 0; i < 9; ++i)
+    if (strides[i] % 8) return 1;
+  typedef const unsigned short* In;
+  typedef unsigned short* Out;
+  const gbx::RopeRows rq{static_cast<In>(q), static_cast<Out>(qout), strides[0], strides[1], strides[2], L, Hq, 0};
+  const gbx::RopeRows rk{static_cast<In>(k), static_cast<Out>(kcache), strides[3], strides[4], strides[5], capacity, H, t0};
+  const gbx::RopeRows rv{static_cast<In>(v), static_cast<Out>(vcache), strides[6], strides[7], strides[8], capacity, H, t0};
+  const dim3 grid(L, B);
+  hipStream_t s = static_cast<hipStream_t>(hip_stream);
+  if (bf16) hipLaunchKernelGGL((gbx::rope_qkv_kernel<true>), grid, dim3(256), 0, s, rq, rk, rv, inv_freq, pos0, D, scale, traditional);
+  else hipLaunchKernelGGL((gbx::rope_qkv_kernel<false>), grid, dim3(256), 0, s, rq, rk, rv, inv_freq, pos0, D, scale, traditional);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+namespace gbx {
+
 // ------------------------------------------------------------------------------------------------ batched RoPE + cache append
 // One launch for a synchronous batched decode step (every sequence at position *pos): q is rotated in place, k is rotated
 // into kcache[b, kvh, pos, :], v is copied into vcache[b, kvh, pos, :].  Replaces rope(q), rope(k) and

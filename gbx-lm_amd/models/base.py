@@ -87,28 +87,56 @@ def fused_decode_attention(q, k, v, cache, rope, scale: float, n_heads: int, n_k
     return out.reshape(bsz, 1, -1)
 
 
+def _rope_in_launch(rope, k: torch.Tensor, v: torch.Tensor, cache, start) -> bool:
+    """A prompt chunk on the GPU with a plain full-width RoPE and a plain KVCache: rotated keys can go straight into the cache."""
+    from .cache import KVCache
+    from .rope_utils import RoPE, Llama3RoPE
+    D = k.shape[3]
+    return (type(cache) is KVCache and not cache.static_active and k.is_cuda and k.shape[2] >= 16 and type(rope) in (RoPE, Llama3RoPE)
+            and isinstance(start, int) and rope.inv_freq.numel() * 2 == D and D % 16 == 0 and D <= 256 and v.shape[3] == D
+            and k.dtype in (torch.bfloat16, torch.float16) and v.dtype == k.dtype and k.stride(3) == 1 and v.stride(3) == 1
+            and all(t.stride(i) % 8 == 0 for t in (k, v) for i in (0, 1, 2)) and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0
+            and rope.inv_freq.is_cuda and rope.inv_freq.dtype == torch.float32)
+
+
+def _cache_takes(cache, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether a launch that indexes the cache with k's batch and head counts may write it: a reused cache of another geometry takes the
+    generic path, whose update_and_fetch raises the shape error."""
+    D = k.shape[3]
+    return (cache.keys.dtype == k.dtype and cache.values.dtype == k.dtype and cache.keys.is_contiguous() and cache.values.is_contiguous()
+            and cache.keys.shape[3] == D and cache.values.shape[3] == D
+            and tuple(cache.keys.shape[:2]) == tuple(k.shape[:2]) and tuple(cache.values.shape[:2]) == tuple(v.shape[:2]))
+
+
+def rope_and_update_cache(rope, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache, start):
+    """``q, k = rope(q, offset=start), rope(k, offset=start); k, v = cache.update_and_fetch(k, v)`` (qllama.py:84-91).  A prompt chunk on
+    the GPU does all of it in ONE launch (gbx_rope_qkv), the same bits; what that does not take goes step by step."""
+    if (_rope_in_launch(rope, k, v, cache, start) and q.dtype == k.dtype and q.device == k.device and v.device == k.device and q.shape[0] == k.shape[0]
+            and q.shape[2:] == k.shape[2:] and v.shape == k.shape and q.stride(3) == 1 and all(q.stride(i) % 8 == 0 for i in (0, 1, 2))
+            and q.data_ptr() % 16 == 0 and not rope._forward_hooks and not rope._forward_pre_hooks):
+        prev = cache.offset
+        cache.reserve(k.shape[2], k, v)
+        if _cache_takes(cache, k, v):
+            from .. import ops
+            out = ops.rope_qkv(q, k, v, cache.keys, cache.values, rope.inv_freq, start, prev, getattr(rope, "scale", 1.0), rope.traditional)
+            if out is not None:
+                cache.offset = prev + k.shape[2]
+                return out, cache.keys[..., :cache.offset, :], cache.values[..., :cache.offset, :]
+        cache.offset = prev
+    return (rope(q, offset=start), *rope_keys_and_update_cache(rope, k, v, cache, start))
+
+
 def rope_keys_and_update_cache(rope, k: torch.Tensor, v: torch.Tensor, cache, start):
     """``k = rope(k, offset=start); k, v = cache.update_and_fetch(k, v)`` (qllama.py:88-91).  A prompt chunk on the GPU with a plain
     full-width RoPE and a plain KVCache does both in ONE launch: the rotated keys go straight into the cache (gbx_rope_kv_write:
     the same arithmetic as the stand-alone RoPE launch, so the cache contents are bit-identical), no temporary, no copy launches."""
-    from .cache import KVCache
-    from .rope_utils import RoPE, Llama3RoPE
-    L, D = k.shape[2], k.shape[3]
-    if (type(cache) is KVCache and not cache.static_active and k.is_cuda and L >= 16 and type(rope) in (RoPE, Llama3RoPE)
-            and isinstance(start, int) and rope.inv_freq.numel() * 2 == D and D % 16 == 0 and D <= 256 and v.shape[3] == D
-            and k.dtype in (torch.bfloat16, torch.float16) and v.dtype == k.dtype and k.stride(3) == 1 and v.stride(3) == 1
-            and all(t.stride(i) % 8 == 0 for t in (k, v) for i in (0, 1, 2)) and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0
-            and rope.inv_freq.is_cuda and rope.inv_freq.dtype == torch.float32):
+    if _rope_in_launch(rope, k, v, cache, start):
         prev = cache.offset
-        cache.reserve(L, k, v)
-        # (the kernel indexes the cache with k's batch and head counts: a reused cache of another geometry takes the generic path,
-        # whose update_and_fetch raises the shape error)
-        if (cache.keys.dtype == k.dtype and cache.values.dtype == k.dtype and cache.keys.is_contiguous() and cache.values.is_contiguous()
-                and cache.keys.shape[3] == D and cache.values.shape[3] == D
-                and tuple(cache.keys.shape[:2]) == tuple(k.shape[:2]) and tuple(cache.values.shape[:2]) == tuple(v.shape[:2])):
+        cache.reserve(k.shape[2], k, v)
+        if _cache_takes(cache, k, v):
             from .. import ops
             ops.rope_kv_write(k, v, cache.keys, cache.values, rope.inv_freq, start, prev, getattr(rope, "scale", 1.0), rope.traditional)
-            cache.offset = prev + L
+            cache.offset = prev + k.shape[2]
             return cache.keys[..., :cache.offset, :], cache.values[..., :cache.offset, :]
         cache.offset = prev                              # fast path not taken: hand an untouched offset to the generic path
     k = rope(k, offset=start)

@@ -15,7 +15,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from .base import (BaseModelArgs, cache_offset, create_attention_mask, rope_keys_and_update_cache, scaled_dot_product_attention,
+from .base import (BaseModelArgs, cache_offset, create_attention_mask, rope_and_update_cache, scaled_dot_product_attention,
                    swiglu)
 from .projection import RowLinear
 from .qllama import RMSNorm
@@ -85,8 +85,7 @@ class Attention(nn.Module):
         k = k.reshape(b, l, self.n_kv_heads, -1).permute(0, 2, 1, 3)
         v = v.reshape(b, l, self.n_kv_heads, -1).permute(0, 2, 1, 3)
         start = cache_offset(cache)
-        q = self.rope(q, offset=start)
-        k, v = rope_keys_and_update_cache(self.rope, k, v, cache, start)
+        q, k, v = rope_and_update_cache(self.rope, q, k, v, cache, start)
         ctx = scaled_dot_product_attention(q, k, v, cache=cache, scale=self.scale, mask=mask)
         return self.o_proj(ctx.permute(0, 2, 1, 3).reshape(b, l, -1))
 

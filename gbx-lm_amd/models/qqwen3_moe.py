@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import ops
-from .base import (BaseModelArgs, cache_offset, create_attention_mask, fused_decode_attention, rope_keys_and_update_cache,
+from .base import (BaseModelArgs, cache_offset, create_attention_mask, fused_decode_attention, rope_and_update_cache,
                    scaled_dot_product_attention, swiglu)
 from .projection import RowLinear
 from .qllama import RMSNorm
@@ -87,8 +87,7 @@ class Attention(nn.Module):
         k = self.k_norm(k.view(b, l, self.n_kv_heads, -1)).permute(0, 2, 1, 3)
         v = v.view(b, l, self.n_kv_heads, -1).permute(0, 2, 1, 3)
         start = cache_offset(cache)
-        q = self.rope(q, offset=start)
-        k, v = rope_keys_and_update_cache(self.rope, k, v, cache, start)
+        q, k, v = rope_and_update_cache(self.rope, q, k, v, cache, start)
         ctx = scaled_dot_product_attention(q, k, v, cache=cache, scale=self.scale, mask=mask)
         out = self.o_proj(ctx.permute(0, 2, 1, 3).reshape(b, l, -1))
         return out if residual is None else residual + out

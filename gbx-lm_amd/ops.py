@@ -1554,6 +1554,19 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, kcache: torch.Tensor, vcache
                                             _stream_ptr(k.device)))
 
 
+def rope_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, inv_freq: torch.Tensor, pos0: int, t0: int,
+             scale: float = 1.0, traditional: bool = False) -> Optional[torch.Tensor]:
+    """``rope(q)`` returned, RoPE(k) and v into rows t0.. of their caches, one launch (gbx_rope_qkv).  q [B, Hq, L, D], k / v [B, H, L, D] views with a
+    unit feature stride; caches [B, H, capacity, D] contiguous.  None: not a call for that launch, nothing was done."""
+    B, Hq, L, D = q.shape
+    out = torch.empty((B, Hq, L, D), dtype=q.dtype, device=q.device)
+    strides = (ctypes.c_int64 * 9)(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3])
+    rc = _lib.lib().gbx_rope_qkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), inv_freq.data_ptr(), int(pos0), B, Hq,
+                                 k.shape[1], L, D, strides, kcache.shape[2], int(t0), float(scale), int(bool(traditional)), int(q.dtype == torch.bfloat16),
+                                 _stream_ptr(q.device))
+    return out if rc == 0 else None
+
+
 def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 inv_freq: torch.Tensor, pos: torch.Tensor, n_heads: int, n_kv: int, head_dim: int,
                 rope_scale: float, traditional: bool) -> None:
