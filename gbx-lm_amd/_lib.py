@@ -78,6 +78,8 @@ def lib() -> ctypes.CDLL:
         L.gbx_dense_swiglu_forward.argtypes = [p, p, p, i64, i32, i32, i32, p]
         L.gbx_dense_forward_multi.argtypes = [p, i32, p, p, p, p, i64, i32, i32, p]
         L.gbx_rope_qkv.argtypes = [p, p, p, p, p, p, p, i64, i32, i32, i32, i32, i32, p, i32, i32, ctypes.c_float, i32, i32, p]
+        L.gbx_step_feed.argtypes = [p, p, i32, p, i64, p]
+        L.gbx_step_words.argtypes = [p, p, p, p, p, p]
         L.gbx_gather_mix_forward.argtypes = [p, p, p, p, p, p, p, p, i32, i32, i32, i32, i32, i32, i32, i32, p]
         L.gbx_dense_workspace_bytes.argtypes = [i64, i32, i32]
         L.gbx_dense_workspace_bytes.restype = ctypes.c_size_t

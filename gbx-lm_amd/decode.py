@@ -230,8 +230,7 @@ class DecodeRunner:
     def _step_local(self, token: torch.Tensor) -> torch.Tensor:
         off = self.caches[0].offset
         self._check_room(off)
-        self.tok.copy_(token.reshape(-1))
-        self.pos.fill_(off)
+        ops.step_feed(token, self.tok, self.pos, off)
         if self.use_graph:
             self.graph.replay()
         else:
@@ -286,8 +285,7 @@ class GraphDecodeRunner:
         off = self.caches[0].offset
         if off >= self.capacity:
             raise RuntimeError(f"KV cache is full ({off} of {self.capacity} positions): grow it and build a new runner")
-        self.tok.copy_(token.reshape(self.batch, 1))
-        self.pos.fill_(off)
+        ops.step_feed(token, self.tok, self.pos, off)
         self.graph.replay()
         for c in self.caches:
             c.offset = off + 1
@@ -713,13 +711,11 @@ class FusedDecodeRunner(DecodeRunner):
             if first:
                 self._capture_other_mode("gen")
             if not fed_back:
-                self.tok.copy_(token.reshape(self.tok.shape))
-                self.pos.fill_(off - 1)                               # the embedding launch advances it to `off`
+                ops.step_feed(token, self.tok, self.pos, off - 1)    # the embedding launch advances it to `off`
             graph.replay()
         else:
             if not fed_back:
-                self.tok.copy_(token.reshape(self.tok.shape))
-                self.pos.fill_(off - 1)
+                ops.step_feed(token, self.tok, self.pos, off - 1)
             self.chain, self.long_mode = "gen", long
             with torch.no_grad():
                 self._forward()
@@ -739,12 +735,10 @@ class FusedDecodeRunner(DecodeRunner):
             graph, out = self._graph_for(False, long)
             if first:
                 self._capture_other_mode(False)
-            self.tok.copy_(token.reshape(-1))
-            self.pos.fill_(off)
+            ops.step_feed(token, self.tok, self.pos, off)
             graph.replay()
         else:
-            self.tok.copy_(token.reshape(-1))
-            self.pos.fill_(off)
+            ops.step_feed(token, self.tok, self.pos, off)
             self.long_mode = long
             with torch.no_grad():
                 out = self.logits = self._forward()

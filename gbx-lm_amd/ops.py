@@ -1375,6 +1375,26 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, offset: int,
     return out
 
 
+def step_feed(token: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor, value: int) -> None:
+    """``tok.copy_(token); pos.fill_(value)``: what a captured decode step reads, as one launch (gbx_step_feed)."""
+    if (tok.is_cuda and token.device == tok.device and token.dtype == torch.int64 and token.numel() == tok.numel() and token.is_contiguous() and tok.is_contiguous()
+            and tok.dtype == torch.int64 and pos.dtype == torch.int64 and pos.numel() == 1 and pos.device == tok.device):
+        _lib.check(_lib.lib().gbx_step_feed(token.data_ptr(), tok.data_ptr(), tok.numel(), pos.data_ptr(), int(value), _stream_ptr(tok.device)))
+        return
+    tok.copy_(token.reshape(-1) if tok.dim() == 1 else token.reshape(tok.shape))
+    pos.fill_(value)
+
+
+def step_words(token: torch.Tensor, words, out: torch.Tensor) -> bool:
+    """A token and up to three status words (int32 device scalars) side by side into ``out`` int64 [4], one launch (gbx_step_words).  False: not a call for it."""
+    if not (token.is_cuda and token.dtype == torch.int64 and token.numel() >= 1 and len(words) <= 3 and out.device == token.device
+            and all(w.device == token.device and w.dtype == torch.int32 for w in words)):
+        return False
+    w = [t.data_ptr() for t in words] + [None] * (3 - len(words))
+    _lib.check(_lib.lib().gbx_step_words(token.data_ptr(), *w, out.data_ptr(), _stream_ptr(token.device)))
+    return True
+
+
 def moe_route(logits: torch.Tensor, top_k: int, mode: int = 0, renormalize: bool = True):
     """Router logits [..., E] -> (indices int32 [..., k], scores [..., k]) in one launch (gbx_moe_route)."""
     _require_cuda(logits, "logits")

@@ -369,7 +369,7 @@ def generate_step(prompt: torch.Tensor, model: nn.Module, *, max_tokens: int = 2
     # The status words of the decode runner's fused launches (in-launch hand-offs that can time out: another tenant on the GPU, a CU
     # mask) travel with the id: a non-zero word means the step's stream was poisoned (NaN logits) -- the model then falls back to the
     # five-launch block for good and the step is REPLAYED, so the caller never sees a token of a faulted step.
-    ring, fring, pring, slot = [], [], [], [0]
+    ring, fring, pring, side_by_side, slot = [], [], [], [], [0]
     fault_words = getattr(model, "decode_fault_words", None) if fast_decode is not None else None
 
     class _HandoffFault(Exception):
@@ -389,8 +389,18 @@ def generate_step(prompt: torch.Tensor, model: nn.Module, *, max_tokens: int = 2
             pinned.copy_(step_words[0], non_blocking=True)
             fpin = pinned[1:]
         else:
-            pinned.copy_(t.reshape(-1)[:1], non_blocking=True)
+            from . import ops
             words = fault_words() if fault_words is not None else []
+            if words and not side_by_side:
+                side_by_side.append(torch.empty((4,), dtype=torch.long, device=t.device))
+            if words and ops.step_words(t, words, side_by_side[0]):
+                if not pring:
+                    pring.extend(torch.zeros((4,), dtype=torch.long, pin_memory=True) for _ in range(3))
+                pinned, words = pring[slot[0] % 3], []
+                pinned.copy_(side_by_side[0], non_blocking=True)
+                fpin = pinned[1:]
+            else:
+                pinned.copy_(t.reshape(-1)[:1], non_blocking=True)
             if words:
                 fpin = fring[slot[0] % 3][:len(words)]
                 for i, w in enumerate(words):
