@@ -621,13 +621,15 @@ def gather_swiglu(x: torch.Tensor, gate, up, rhs_indices: torch.Tensor):
 def gather_mix(x: torch.Tensor, down, rhs_indices: torch.Tensor, scores: torch.Tensor, residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``moe_combine(down(x, indices), scores, residual)`` of a decode-sized set of (token, slot) pairs in ONE launch (gbx_gather_mix_forward), x [..., k, 1, K],
     ``down`` a QuantizedSwitchLinear.  None where the launch does not take the call (the caller then runs the two)."""
-    K, N, k = x.shape[-1], down.output_dims, rhs_indices.shape[-1]
+    K, N, k, bits, g = x.shape[-1], down.output_dims, rhs_indices.shape[-1], down.bits, down.group_size
     pairs, lead = rhs_indices.numel(), tuple(rhs_indices.shape[:-1])
     if not (x.is_cuda and x.dtype in _DT and 0 < pairs <= 64 and k <= 8 and tuple(x.shape) == (*lead, k, 1, K) and K == down.input_dims and K % 128 == 0
-            and K <= 64 * (64 if down.bits == 2 else 32) and down.bias is None and rhs_indices.dtype == torch.int32 and down.scales.dtype == x.dtype
-            and down.zeros.dtype == x.dtype and scores.dtype == x.dtype and tuple(scores.shape) == tuple(rhs_indices.shape)
-            and all(t.is_cuda and t.is_contiguous() for t in (down.qweight, down.scales, down.zeros))
-            and (residual is None or (residual.is_cuda and residual.dtype == x.dtype and tuple(residual.shape) == (*lead, N)))):
+            and K <= 64 * (64 if bits == 2 else 32) and g in (32, 64, 128) and down.bias is None and rhs_indices.dtype == torch.int32 and tuple(scores.shape) == tuple(rhs_indices.shape)
+            and down.qweight.dtype in (torch.uint32, torch.int32) and tuple(down.qweight.shape[1:]) == (N, K // 32 * bits)
+            and all(tuple(t.shape) == (down.qweight.shape[0], N, K // g) and t.dtype == x.dtype for t in (down.scales, down.zeros))
+            and all(t.device == x.device for t in (rhs_indices, down.qweight, down.scales, down.zeros)) and down.qweight.is_contiguous() and down.scales.is_contiguous()
+            and down.zeros.is_contiguous() and all(t is None or (t.device == x.device and t.dtype == x.dtype) for t in (scores, residual))
+            and (residual is None or tuple(residual.shape) == (*lead, N))):
         return None
     xr, idx, mix = x.reshape(-1, K).contiguous(), rhs_indices.reshape(-1).contiguous(), scores.contiguous()
     res = None if residual is None else residual.contiguous()
