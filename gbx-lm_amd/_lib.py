@@ -489,6 +489,9 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_packed_experts.argtypes = [ctypes.POINTER(PackedExpertsArgs), p]
         L.gbxm_expert_ff.argtypes = [ctypes.POINTER(ExpertArgs), p]
         L.gbxm_recurrent_prepare.argtypes = [ctypes.POINTER(RecurrentPrepArgs), p]
+        L.gbxm_recurrent_prepare_keep.argtypes = [ctypes.POINTER(RecurrentPrepArgs), p]
+        L.gbxm_embed_streams.argtypes = [p, p, p, i64, i32, i32, i32, p]
+        L.gbxm_linear_rows_pair.argtypes = [p, i64, p, p, i32, p, i64, p, p, i32, i64, i32, p]
         L.gbxm_conv_tail_update.argtypes = [p, i64, p, p, i32, i32, i32, i32, p]
         L.gbxm_state_scan.argtypes = [p, i64, p, p, p, i32, i64, i32, i32, i32, i32, i32, p]
         L.gbxm_state_scan_ws.argtypes = [p, i64, p, p, p, i32, i64, i32, i32, i32, i32, i32, p, sz, p]

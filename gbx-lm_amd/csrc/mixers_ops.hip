@@ -22,12 +22,12 @@ constexpr int NT = 256, NW = NT / 64;
 
 template <typename T>
 __global__ __launch_bounds__(NT) void embed_kernel(const T* __restrict__ table, const int64_t* __restrict__ tokens, float* __restrict__ x,
-                                                   T* __restrict__ h, int64_t h_row, int width, float scale) {
+                                                   T* __restrict__ h, int64_t h_row, int width, float scale, int copies) {
   const int64_t t = blockIdx.x;
   const T* row = table + tokens[t] * width;
   for (int c = threadIdx.x; c < width; c += NT) {
     const float v = to_f32(row[c]) * scale;
-    x[t * width + c] = v;
+    for (int i = 0; i < copies; ++i) x[(t * copies + i) * width + c] = v;
     if (h) h[t * h_row + c] = from_f32<T>(v);
   }
 }
@@ -38,7 +38,7 @@ __global__ __launch_bounds__(NT) void embed_kernel(const T* __restrict__ table, 
 // 4.0 | 2.7.
 template <typename T>
 __global__ __launch_bounds__(1024) void embed_row_kernel(const T* __restrict__ table, const int64_t* __restrict__ tokens, float* __restrict__ x, T* __restrict__ h,
-                                                         int64_t h_row, int width, float scale) {
+                                                         int64_t h_row, int width, float scale, int copies) {
   const int64_t t = blockIdx.x;
   const int c = threadIdx.x * 4;
   if (c >= width) return;
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(1024) void embed_row_kernel(const T* __restrict__ t
   Lanes<T, 4>::load(table + tokens[t] * width + c, v);
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] *= scale;
-  Lanes<float, 4>::store(x + t * width + c, v);
+  for (int i = 0; i < copies; ++i) Lanes<float, 4>::store(x + (t * copies + i) * width + c, v);
   if (h) Lanes<T, 4>::store(h + t * h_row + c, v);
 }
 
@@ -644,7 +644,7 @@ const char* gbxm_last_error(void) { return g_err; }
     if ((act) == GBXM_BF16) { using T = bf16_t; CALL; } else { using T = float; CALL; } \
   } while (0)
 
-int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* h, int64_t h_row, int64_t T_, int32_t width, float scale, int32_t act,
+static int embed_rows(const void* table, const int64_t* tokens, float* x, void* h, int64_t h_row, int64_t T_, int32_t width, float scale, int32_t copies, int32_t act,
                       void* stream) {
   if (!act_ok(act) || !table || !tokens || !x || width <= 0 || T_ < 0 || (h && h_row < width)) return fail(GBXM_ERR_INVALID, "embed_scaled: bad argument");
   if (T_ == 0) return GBXM_OK;
@@ -652,10 +652,21 @@ int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* 
   const int threads = row_threads(width);
   const size_t group = act == GBXM_BF16 ? 8 : 16;
   if (threads && all_aligned(16, x) && all_aligned(group, static_cast<const char*>(table)) && (!h || (h_row % 4 == 0 && all_aligned(group, static_cast<const char*>(h)))))
-    GBXM_DISPATCH(act, (embed_row_kernel<T><<<dim3(T_), threads, 0, s>>>(static_cast<const T*>(table), tokens, x, static_cast<T*>(h), h_row, width, scale)));
+    GBXM_DISPATCH(act, (embed_row_kernel<T><<<dim3(T_), threads, 0, s>>>(static_cast<const T*>(table), tokens, x, static_cast<T*>(h), h_row, width, scale, copies)));
   else
-    GBXM_DISPATCH(act, (embed_kernel<T><<<dim3(T_), NT, 0, s>>>(static_cast<const T*>(table), tokens, x, static_cast<T*>(h), h_row, width, scale)));
+    GBXM_DISPATCH(act, (embed_kernel<T><<<dim3(T_), NT, 0, s>>>(static_cast<const T*>(table), tokens, x, static_cast<T*>(h), h_row, width, scale, copies)));
   return after_launch("embed_scaled");
+}
+
+int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* h, int64_t h_row, int64_t T_, int32_t width, float scale, int32_t act,
+                      void* stream) {
+  return embed_rows(table, tokens, x, h, h_row, T_, width, scale, 1, act, stream);
+}
+
+// x [T, copies, width]: the embedding in every residual stream (a launch to spread it: 3 us and a row).  For this package's own Python layer; not part of the public header.
+extern "C" int gbxm_embed_streams(const void* table, const int64_t* tokens, float* x, int64_t T_, int32_t width, int32_t copies, int32_t act, void* stream) {
+  if (copies < 1 || copies > 64) return fail(GBXM_ERR_INVALID, "embed_streams: %d streams", copies);
+  return embed_rows(table, tokens, x, nullptr, 0, T_, width, 1.f, copies, act, stream);
 }
 
 extern "C" int gbxm_step_tables(const int32_t* seq, const int32_t* tile0, int32_t* tok, int32_t* tiles, int32_t B, int32_t T_, int32_t n_tiles, int32_t q_tile, void* stream) {

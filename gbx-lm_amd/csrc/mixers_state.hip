@@ -88,7 +88,7 @@ __global__ __launch_bounds__(NT) void recurrent_prep_kernel(gbxm_recurrent_prep_
 // Bound by the fp32 rows it writes (12 320 numbers a token in the first line) and the decays' logarithms and exponentials.  Measured, us: 2 266 rows, 32 heads of 128 with 16
 // of q / k and a convolution 184 -> 67; without one, 8 heads of 128 x 256 29 -> 27; one row of the former kind, 8 heads of 64 x 128 6.4 -> 3.5.
 template <typename T, bool CONV, int R>
-__global__ __launch_bounds__(NT) void recurrent_prep_rows_kernel(gbxm_recurrent_prep_args p) {
+__global__ __launch_bounds__(NT) void recurrent_prep_rows_kernel(gbxm_recurrent_prep_args p, T* tails) {
   const int nq = p.G * p.dk, nv = p.H * p.dv, nd = p.H * p.dk, C = 2 * nq + nv;
   const int c = (blockIdx.y * NT + threadIdx.x) * 4;
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * R;
@@ -131,6 +131,11 @@ __global__ __launch_bounds__(NT) void recurrent_prep_rows_kernel(gbxm_recurrent_
           acc += w[k][3] * x[i][k];
           v[k] = acc * sigmoid_<false>(acc);
           h[0][k] = h[1][k]; h[1][k] = h[2][k]; h[2][k] = x[i][k];
+        }
+        if (tails && pos == pos0 + p.seq[4 * b + 2] - 1) {   // (every sequence brings one row: nobody else reads these channels of the slot)
+          T* to = tails + static_cast<int64_t>(p.seq[4 * b]) * 3 * C + c;
+#pragma unroll
+          for (int j = 0; j < 3; ++j) Lanes<T, 4>::store(to + static_cast<int64_t>(j) * C, h[j]);
         }
       } else {
 #pragma unroll
@@ -192,11 +197,12 @@ bool prep_rows_shape(const gbxm_recurrent_prep_args& a) {
 }
 
 template <typename T, bool CONV>
-void launch_prep_rows(const gbxm_recurrent_prep_args& a, hipStream_t s) {
+void launch_prep_rows(const gbxm_recurrent_prep_args& a, bool keep, hipStream_t s) {
+  T* tails = keep ? static_cast<T*>(const_cast<void*>(a.tail)) : nullptr;
   const unsigned cols = (2 * a.G * a.dk + a.H * a.dv + a.H * a.dk + 4 * NT - 1) / (4 * NT);
   // eight rows a thread where that leaves the chip full, else one
-  if (a.T * cols >= 8 * 1024) recurrent_prep_rows_kernel<T, CONV, 8><<<dim3((a.T + 7) / 8, cols), NT, 0, s>>>(a);
-  else recurrent_prep_rows_kernel<T, CONV, 1><<<dim3(a.T, cols), NT, 0, s>>>(a);
+  if (a.T * cols >= 8 * 1024) recurrent_prep_rows_kernel<T, CONV, 8><<<dim3((a.T + 7) / 8, cols), NT, 0, s>>>(a, tails);
+  else recurrent_prep_rows_kernel<T, CONV, 1><<<dim3(a.T, cols), NT, 0, s>>>(a, tails);
 }
 
 template <typename T>
@@ -361,9 +367,7 @@ bool act_ok(int act) { return act == GBXM_BF16 || act == GBXM_F32; }
 
 using namespace gbxm;
 
-extern "C" {
-
-int gbxm_recurrent_prepare(const gbxm_recurrent_prep_args* a, void* stream) {
+static int prepare(const gbxm_recurrent_prep_args* a, bool keep, void* stream) {
   if (!a || !act_ok(a->act) || !a->y || (a->a && !a->decay_bias) || !a->decay_rate || !a->seq || !a->tok || !a->out || a->T < 0 || a->H < 1 || a->G < 1 ||
       a->H % a->G || a->dk < 1 || a->dv < 1 || a->off_q < 0 || a->off_k < 0 || a->off_v < 0)
     return fail(GBXM_ERR_INVALID, "recurrent_prepare: bad argument");
@@ -376,10 +380,10 @@ int gbxm_recurrent_prepare(const gbxm_recurrent_prep_args* a, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool bf = a->act == GBXM_BF16;
   if (bf ? prep_rows_shape<bf16_t>(*a) : prep_rows_shape<float>(*a)) {
-    if (bf && a->conv) launch_prep_rows<bf16_t, true>(*a, s);
-    else if (bf) launch_prep_rows<bf16_t, false>(*a, s);
-    else if (a->conv) launch_prep_rows<float, true>(*a, s);
-    else launch_prep_rows<float, false>(*a, s);
+    if (bf && a->conv) launch_prep_rows<bf16_t, true>(*a, keep, s);
+    else if (bf) launch_prep_rows<bf16_t, false>(*a, keep, s);
+    else if (a->conv) launch_prep_rows<float, true>(*a, keep, s);
+    else launch_prep_rows<float, false>(*a, keep, s);
     return after_launch("recurrent_prepare");
   }
   // splits of a row: enough workgroups for the chip when the step has few rows, never more than the row has work for
@@ -391,7 +395,23 @@ int gbxm_recurrent_prepare(const gbxm_recurrent_prep_args* a, void* stream) {
   const dim3 grid(a->T, static_cast<unsigned>(splits));
   if (a->act == GBXM_BF16) recurrent_prep_kernel<bf16_t, false><<<grid, NT, 0, s>>>(*a);
   else recurrent_prep_kernel<float, false><<<grid, NT, 0, s>>>(*a);
+  if (keep) {
+    const dim3 grid((C + NT - 1) / NT, static_cast<unsigned>(a->T));
+    if (bf) conv_tail_kernel<bf16_t><<<grid, NT, 0, s>>>(static_cast<const bf16_t*>(a->y) + a->off_q, a->y_stride, static_cast<bf16_t*>(const_cast<void*>(a->tail)), a->seq, C, a->taps);
+    else conv_tail_kernel<float><<<grid, NT, 0, s>>>(static_cast<const float*>(a->y) + a->off_q, a->y_stride, static_cast<float*>(const_cast<void*>(a->tail)), a->seq, C, a->taps);
+  }
   return after_launch("recurrent_prepare");
+}
+
+extern "C" {
+
+int gbxm_recurrent_prepare(const gbxm_recurrent_prep_args* a, void* stream) { return prepare(a, false, stream); }
+
+// The same and gbxm_conv_tail_update behind it, for a step whose every sequence brings one row (T sequences): the convolution's inputs go on into the slots from the registers that
+// hold them (a launch of its own: 3.3 us).  For this package's own Python layer; not part of the public header.
+int gbxm_recurrent_prepare_keep(const gbxm_recurrent_prep_args* a, void* stream) {
+  if (!a || !a->conv || a->taps < 2 || a->T > 65535) return fail(GBXM_ERR_INVALID, "recurrent_prepare_keep: a convolution of two taps at least");
+  return prepare(a, true, stream);
 }
 
 int gbxm_conv_tail_update(const void* y, int64_t y_stride, void* tail, const int32_t* seq, int32_t B, int32_t C, int32_t taps, int32_t act,

@@ -61,6 +61,16 @@ def embed_scaled(table: torch.Tensor, tokens: torch.Tensor, scale: float, image=
     return x, h
 
 
+def embed_streams(table: torch.Tensor, tokens: torch.Tensor, streams: int) -> torch.Tensor:
+    """fp32 [T, streams, W]: the tokens' rows of the table in every stream, one launch."""
+    act = _act(table, "table")
+    t, w = tokens.numel(), table.shape[1]
+    tokens = tokens.reshape(-1).to(torch.long).contiguous()
+    x = torch.empty((t, streams, w), dtype=torch.float32, device=table.device)
+    _lib.check_mixers(_lib.mixers().gbxm_embed_streams(table.data_ptr(), tokens.data_ptr(), x.data_ptr(), t, w, streams, act, _stream(table.device)))
+    return x
+
+
 def segment_rmsnorm_(rows: torch.Tensor, n0: int, n1: int, w0: torch.Tensor, w1: torch.Tensor, eps: float) -> None:
     act = _act(rows, "rows")
     if rows.dim() != 2 or rows.stride(1) != 1:
@@ -122,6 +132,20 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]) 
     _lib.check_mixers(_lib.mixers().gbxm_linear_rows(x.data_ptr(), stride, w.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), n, t, n,
                                                     k, _stream(x.device)))
     return y
+
+
+def linear_rows_pair(x0: torch.Tensor, w0: torch.Tensor, x1: torch.Tensor, w1: torch.Tensor):
+    """``(x0 @ w0.T, x1 @ w1.T)`` of few bf16 rows and one short contraction length as one launch, or None for what it does not take."""
+    if not all(t.dim() == 2 and t.is_cuda and t.dtype == torch.bfloat16 and t.device == x0.device and t.data_ptr() % 16 == 0 for t in (x0, w0, x1, w1)):
+        return None
+    t, k = x0.shape
+    if (x1.shape != x0.shape or w0.shape[1] != k or w1.shape[1] != k or not 0 < t <= 32 or k % 64 or not 0 < k <= 512 or not (0 < w0.shape[0] <= 1 << 20 and 0 < w1.shape[0] <= 1 << 20)
+            or any(x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k for x in (x0, x1)) or not w0.is_contiguous() or not w1.is_contiguous()):
+        return None
+    y0, y1 = (torch.empty((t, w.shape[0]), dtype=torch.bfloat16, device=x0.device) for w in (w0, w1))
+    _lib.check_mixers(_lib.mixers().gbxm_linear_rows_pair(x0.data_ptr(), x0.stride(0), w0.data_ptr(), y0.data_ptr(), w0.shape[0], x1.data_ptr(), x1.stride(0), w1.data_ptr(),
+                                                         y1.data_ptr(), w1.shape[0], t, k, _stream(x0.device)))
+    return y0, y1
 
 
 # Rows up to which a router's logits are one launch on the rows as they are -- every (row, expert) reads its router row again, so a router that the
@@ -518,7 +542,7 @@ def route_sigmoid_groups(h: torch.Tensor, router: torch.Tensor, correction: torc
 
 # ------------------------------------------------------------------------------- recurrent mixers (models/recurrent_mixers.py)
 def recurrent_prepare(y: torch.Tensor, a: Optional[torch.Tensor], lay, decay_bias: Optional[torch.Tensor], decay_rate: torch.Tensor, sign: float,
-                      conv: Optional[torch.Tensor], cache, batch, unit: bool, q_scale: float, qkv_silu: bool = False) -> torch.Tensor:
+                      conv: Optional[torch.Tensor], cache, batch, unit: bool, q_scale: float, qkv_silu: bool = False, keep_tail: bool = False) -> torch.Tensor:
     act = _act(y, "y")
     t = y.shape[0]
     if y.dim() != 2 or y.stride(1) != 1 or t != batch.total or (a is not None and (a.dim() != 2 or a.stride(1) != 1 or a.dtype != y.dtype or a.shape != (t, lay.nd))):
@@ -550,7 +574,8 @@ def recurrent_prepare(y: torch.Tensor, a: Optional[torch.Tensor], lay, decay_bia
     p.H, p.G, p.dk, p.dv = lay.heads, lay.groups, lay.dk, lay.dv
     p.off_q, p.off_k, p.off_v, p.off_beta = lay.off_q, lay.off_k, lay.off_v, lay.off_beta
     p.unit, p.sign, p.q_scale, p.act = int(bool(unit)), float(sign), float(q_scale), act
-    _lib.check_mixers(_lib.mixers().gbxm_recurrent_prepare(ctypes.byref(p), _stream(y.device)))
+    L = _lib.mixers()
+    _lib.check_mixers((L.gbxm_recurrent_prepare_keep if keep_tail else L.gbxm_recurrent_prepare)(ctypes.byref(p), _stream(y.device)))
     return out
 
 

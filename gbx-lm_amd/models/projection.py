@@ -20,6 +20,15 @@ def project(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = Non
     return F.linear(x, w, bias)
 
 
+def project_pair(x0: torch.Tensor, w0: torch.Tensor, x1: torch.Tensor, w1: torch.Tensor):
+    """``project(x0, w0), project(x1, w1)``: of few rows and short contractions of one length in one launch."""
+    if isinstance(x0, torch.Tensor) and x0.is_cuda and x0.dim() == 2 and 0 < x0.shape[0] <= 32 and M.outside_torch(x0, w0, None) and M.outside_torch(x1, w1, None):
+        y = M.linear_rows_pair(x0, w0, x1, w1)
+        if y is not None:
+            return y
+    return project(x0, w0), project(x1, w1)
+
+
 class RowLinear(nn.Linear):
     """``nn.Linear`` whose product is ``project``."""
 

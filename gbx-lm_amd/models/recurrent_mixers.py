@@ -37,7 +37,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .cache import SlotStateCache
-from .projection import project
+from .projection import project, project_pair
 
 GATE_SILU, GATE_SIGMOID = 1, 2
 
@@ -264,10 +264,14 @@ class _RecurrentMixer(nn.Module):
     def _mix(self, y: torch.Tensor, a: torch.Tensor, gate: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
         lay = self.layout
         cache.reserve(y.dtype, y.device)
-        r = recurrent_prepare(y, a, lay, self.decay_bias, self.decay_rate, self.decay_sign, self.conv if self.taps else None, cache, batch,
-                              self.unit, self.q_scale, self.qkv_silu)
-        if self.taps > 1:
-            conv_tail_update(y, 2 * lay.nq + lay.nv, cache, batch)
+        args = (y, a, lay, self.decay_bias, self.decay_rate, self.decay_sign, self.conv if self.taps else None, cache, batch, self.unit, self.q_scale, self.qkv_silu)
+        if y.is_cuda and self.taps > 1 and lay.off_q == 0 and all(n == 1 for n in batch.n_new) and batch.total == len(batch.slot):
+            from .. import mixer_ops as M                             # a row a sequence: the launch that reads the inputs in front of it moves them on
+            r = M.recurrent_prepare(*args, keep_tail=True)
+        else:
+            r = recurrent_prepare(*args)
+            if self.taps > 1:
+                conv_tail_update(y, 2 * lay.nq + lay.nv, cache, batch)
         o = decayed_state_scan(r, lay, cache, batch, self.delta)
         return project(head_norm_gate(o, gate, self.out_norm, 1 if self.norm_heads_together else lay.heads, self.eps, self.gate_kind), self.o.weight)
 
@@ -369,8 +373,7 @@ class ChannelDeltaRule(_RecurrentMixer):
 
     def forward(self, h: torch.Tensor, batch, cache: SlotStateCache) -> torch.Tensor:
         y = project(h, self.inp.weight)
-        a = project(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight)
-        gate = project(y[:, self.off_g1:self.off_g1 + self.gate_rank], self.g2.weight)
+        a, gate = project_pair(y[:, self.off_a1:self.off_a1 + self.decay_rank], self.a2.weight, y[:, self.off_g1:self.off_g1 + self.gate_rank], self.g2.weight)
         return self._mix(y, a, gate, batch, cache)
 
 

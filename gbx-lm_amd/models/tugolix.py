@@ -130,9 +130,8 @@ class TugolixModel(nn.Module):
         w = self.embed_tokens.weight
         if tokens.is_cuda:
             from .. import mixer_ops as M
-            x = M.embed_scaled(w, tokens, 1.0, image=False)[0]
-        else:
-            x = w[tokens].float()
+            return M.embed_streams(w, tokens, self.streams)
+        x = w[tokens].float()
         return x.unsqueeze(1).repeat(1, self.streams, 1)
 
 
