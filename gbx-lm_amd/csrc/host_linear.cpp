@@ -20,6 +20,8 @@ typedef size_t (*WorkspaceFn)(int64_t, int32_t, int32_t, int32_t, int32_t);
 ForwardFn forward_fn = nullptr;
 ForwardWsFn forward_ws_fn = nullptr;
 WorkspaceFn workspace_fn = nullptr;
+typedef int (*GroupsFn)(const void*, const void*, const void*, const void*, const void*, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, void*);
+GroupsFn groups_fn = nullptr;
 
 constexpr int64_t FEW_ROWS = 256;          // from here on a resident image of the weight may be the faster operand (ops.py decides)
 constexpr int F16 = 0, BF16 = 1;
@@ -36,11 +38,12 @@ bool watched() {                            // something is to see every operati
 }
 
 PyObject* bind(PyObject*, PyObject* args) {
-  unsigned long long f, w, s;
-  if (!PyArg_ParseTuple(args, "KKK", &f, &w, &s)) return nullptr;
+  unsigned long long f, w, s, g;
+  if (!PyArg_ParseTuple(args, "KKKK", &f, &w, &s, &g)) return nullptr;
   forward_fn = reinterpret_cast<ForwardFn>(static_cast<uintptr_t>(f));
   forward_ws_fn = reinterpret_cast<ForwardWsFn>(static_cast<uintptr_t>(w));
   workspace_fn = reinterpret_cast<WorkspaceFn>(static_cast<uintptr_t>(s));
+  groups_fn = reinterpret_cast<GroupsFn>(static_cast<uintptr_t>(g));
   Py_RETURN_NONE;
 }
 
@@ -81,6 +84,12 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
   const int act = type == at::kBFloat16 ? BF16 : F16;
   const int32_t N = static_cast<int32_t>(n), K = static_cast<int32_t>(k), B = static_cast<int32_t>(bits), G = static_cast<int32_t>(group);
+  // rows of several sequences keep the order of sums that they had (see ops.quantized_matmul)
+  if (m > 32 && !(x.dim() == 3 && x.size(0) > 1)) {
+    const int rc = groups_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, 0, stream);
+    if (rc == 0) return THPVariable_Wrap(std::move(y));
+    if (rc != 1) return PyLong_FromLong(rc);
+  }
   // scratch: decode batches and short prompts split k across workgroups
   const size_t need = (m >= 2 && m <= 32) || m > 64 ? workspace_fn(m, N, K, B, G) : 0;
   int rc;

@@ -1,4 +1,4 @@
-// Quantised products of up to 32 rows that fit the registers, contractions of 1024 to 4096 (kernel: mfma_slab_impl.h, one unit per width; launch: mfma_rows.hip).
+// Quantised products of up to 32 rows (one matrix: 1023, in groups) that fit the registers, contractions of 1024 to 4096 (kernel: mfma_slab_impl.h, one unit per width; launch: mfma_rows.hip).
 #pragma once
 #include "mfma_common.h"
 

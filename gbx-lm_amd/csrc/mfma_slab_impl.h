@@ -1,4 +1,5 @@
-// Quantised products of 2 to 32 rows: the rows stay in registers, the packed weights stream past them.
+// Quantised products of 2 to 32 rows: the rows stay in registers, the packed weights stream past them.  More rows are groups of up to 32, which share the chip out between
+// them (grid.y; the weights come from memory for the first and from the L2 for the others): gbx_qlinear_groups, mfma_rows.hip.
 //   y[m, n] = sum_g s[n, g] (sum_k x (C + q)) + (z[n, g] - C s[n, g]) sum_k x
 // A workgroup owns the whole contraction (up to 4096) for up to 8 (16 rows of x: 16) tiles of 16 outputs.  Each of its eight waves owns CW
 // neighbouring chunks of 128 of it: it brings its part of the rows into registers once (LDS-DMA in row order, then fragments), and walks the tiles with
@@ -36,6 +37,7 @@ struct SlabArgs {
   unsigned short* y[3];
   int N[3], block0[3];                     // rows of a matrix, first workgroup of it
   int M, K, tpb;                           // tpb: tiles of a workgroup
+  int rows;                                // of a group of x's rows (at most 32), grid.y of them
 };
 
 // s_waitcnt: at most n vector memory accesses outstanding
@@ -67,7 +69,9 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   const int c0 = wave * CW, own = chunks - c0;                         // the wave's first chunk, and how many there are from it on
   // (every argument is asked for at once: one trip to memory instead of one per use)
   asm volatile("" ::"s"(a.qw[0]), "s"(a.qw[1]), "s"(a.qw[2]), "s"(a.sc[0]), "s"(a.sc[1]), "s"(a.sc[2]), "s"(a.ze[0]), "s"(a.ze[1]), "s"(a.ze[2]), "s"(a.x), "s"(a.N[0]), "s"(a.N[1]), "s"(a.N[2]),
-               "s"(a.block0[1]), "s"(a.block0[2]), "s"(a.M), "s"(a.K), "s"(a.tpb));
+               "s"(a.block0[1]), "s"(a.block0[2]), "s"(a.M), "s"(a.K), "s"(a.tpb), "s"(a.rows));
+  const int m_first = blockIdx.y * a.rows, M = min(a.rows, a.M - m_first);
+  const unsigned short* xg = a.x + static_cast<int64_t>(m_first) * K;
   const int seg = (blockIdx.x >= a.block0[1]) + (blockIdx.x >= a.block0[2]);
   const int N = pick(seg, a.N[0], a.N[1], a.N[2]), tile0 = (blockIdx.x - pick(seg, a.block0[0], a.block0[1], a.block0[2])) * a.tpb, nt = min(a.tpb, ((N + 15) >> 4) - tile0);
 
@@ -92,7 +96,7 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
     // different banks; four rows a request, in pieces of 256 bytes
     packed_x4 x[CW][MT][4];
     float xs[NF][MT];                                                  // lane (m, f): the sum of row m over a group of chunk f
-    const __amdgpu_buffer_rsrc_t rx = slab_buffer(a.x, 0, static_cast<int64_t>(a.M) * K * 2);
+    const __amdgpu_buffer_rsrc_t rx = slab_buffer(xg, 0, static_cast<int64_t>(M) * K * 2);
     int from[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) from[i] = f * K * 2 + ((fr ^ f ^ (4 * i)) << 4);
@@ -218,7 +222,7 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   };
   const int places = nt * MT * 64, n0 = tile0 * 16;
   const unsigned short* bias = a.bias[seg];
-  unsigned short* y = a.y[seg];
+  unsigned short* y = a.y[seg] + static_cast<int64_t>(m_first) * N;
   auto write = [&](int n, int m, float r) {
     const size_t at = static_cast<size_t>(m) * N + n;
     unsigned short o = f32_to_act<BF16>(r);
@@ -233,7 +237,7 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       finite &= __builtin_isfinite(s[v]);
-      if (n < N && m0 + v < a.M) write(n, m0 + v, s[v]);
+      if (n < N && m0 + v < M) write(n, m0 + v, s[v]);
     }
   }
   if (finite) return;
@@ -242,11 +246,11 @@ __device__ __forceinline__ void qgemm_slab(const SlabArgs& a) {
   for (int q = 0; tid + (q >> 2) * 64 * SLAB_WAVES < places; ++q) {
     const int p = tid + (q >> 2) * 64 * SLAB_WAVES, v = q & 3, m = (p >> 6) % MT * 16 + 4 * f + v;
     const int64_t n = n0 + p / (MT * 64) * 16 + fr;
-    if (n >= N || m >= a.M) continue;
+    if (n >= N || m >= M) continue;
     float r = 0.f;
     for (int w = 0; w < SLAB_WAVES; ++w) r += *reinterpret_cast<const float*>(slab_lds + w * SLAB_BYTES + p * 16 + v * 4);
     if (!__builtin_isfinite(r))
-      write(n, m, expanded_dot<BITS, GRP, BF16>(a.x + static_cast<int64_t>(m) * K, a.qw[seg] + n * words, a.sc[seg] + n * groups, a.ze[seg] + n * groups, K));
+      write(n, m, expanded_dot<BITS, GRP, BF16>(xg + static_cast<int64_t>(m) * K, a.qw[seg] + n * words, a.sc[seg] + n * groups, a.ze[seg] + n * groups, K));
   }
 }
 
@@ -264,7 +268,7 @@ hipError_t launch_slab_shape(const MfmaArgs& a, hipStream_t s) {
     done.done();
   }
   SlabArgs t{a.x, {a.qweight, a.qweight_x[0], a.qweight_x[1]}, {a.scales, a.scales_x[0], a.scales_x[1]}, {a.zeros, a.zeros_x[0], a.zeros_x[1]},
-             {a.bias, a.bias_x[0], a.bias_x[1]}, {a.y, a.y_x[0], a.y_x[1]}, {a.N, 0, 0}, {0, 0x7FFFFFFF, 0x7FFFFFFF}, a.M, a.K, 0};
+             {a.bias, a.bias_x[0], a.bias_x[1]}, {a.y, a.y_x[0], a.y_x[1]}, {a.N, 0, 0}, {0, 0x7FFFFFFF, 0x7FFFFFFF}, a.M, a.K, 0, 0};
   constexpr int most = SLAB_BYTES / (MT * 1024);
   // a workgroup fills a CU: as many tiles a workgroup as spread them evenly over as few rounds of 256 as their sums' place in LDS allows
   int tiles = 0;
@@ -272,14 +276,16 @@ hipError_t launch_slab_shape(const MfmaArgs& a, hipStream_t s) {
     if (a.nseg > 1) t.N[g] = a.n_seg[g];
     tiles += (t.N[g] + 15) / 16;
   }
-  const int rounds = (tiles + 256 * most - 1) / (256 * most);
-  t.tpb = (tiles + 256 * rounds - 1) / (256 * rounds);
+  const int groups = (a.M + 31) / 32, wgs = std::max(256 / groups, 1);         // (groups of rows share the chip)
+  t.rows = (a.M + groups - 1) / groups;
+  const int rounds = (tiles + wgs * most - 1) / (wgs * most);
+  t.tpb = (tiles + wgs * rounds - 1) / (wgs * rounds);
   int blocks = 0;
   for (int g = 0; g < std::max(a.nseg, 1); ++g) {
     t.block0[g] = blocks;
     blocks += ((t.N[g] + 15) / 16 + t.tpb - 1) / t.tpb;
   }
-  qgemm_slab_kernel<BITS, GRP, BF16, MT, CW><<<blocks, 64 * SLAB_WAVES, SLAB_LDS, s>>>(t);
+  qgemm_slab_kernel<BITS, GRP, BF16, MT, CW><<<dim3(blocks, groups), 64 * SLAB_WAVES, SLAB_LDS, s>>>(t);
   return hipGetLastError();
 }
 
@@ -301,7 +307,8 @@ hipError_t launch_slab_chunks(const MfmaArgs& a, bool bf16, hipStream_t s) {
 
 template <int BITS, int GRP>
 hipError_t launch_slab_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
-  return a.M <= 16 ? launch_slab_chunks<BITS, GRP, 1>(a, bf16, s) : launch_slab_chunks<BITS, GRP, 2>(a, bf16, s);
+  const int groups = (a.M + 31) / 32;
+  return (a.M + groups - 1) / groups <= 16 ? launch_slab_chunks<BITS, GRP, 1>(a, bf16, s) : launch_slab_chunks<BITS, GRP, 2>(a, bf16, s);
 }
 
 }  // namespace slab

@@ -258,6 +258,15 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise ValueError("out must be a contiguous [M, N] tensor of the activation dtype")
     bias_ptr = bias.data_ptr() if bias is not None else None
     L = _lib.lib()
+    # 33 to 1023 rows as groups of 32 side by side, where that is faster and no resident image is there to multiply by.  Rows of several sequences (a leading size over 1) keep the
+    # kernel and the order of sums that they had: a batch's caches are what its later steps are compared by, and two roundings drift apart over a stack of layers.
+    grouped = 32 < m < 1024 and not (len(xshape) == 3 and xshape[0] > 1)
+    if grouped and m < 256:
+        rc = L.gbx_qlinear_groups(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits, group_size, act, 0,
+                                  _stream_ptr(x.device))
+        if rc != 1:
+            _lib.check(rc)
+            return out if len(xshape) == 2 else out.reshape(*xshape[:-1], n)
     # scratch: decode batches / short prompts split k across workgroups, long prompts dequantise once
     need = L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) if (2 <= m <= 32 or m > 64) else 0
     if m < 256:                                         # no resident images at these sizes: nothing more to decide
@@ -301,6 +310,12 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                                         m, n, k, _DT[x.dtype], scratch.data_ptr() if part else None, part, _stream_ptr(x.device))
             if rc == _lib.GBX_OK:
                 return out.reshape(*x.shape[:-1], n)
+    if grouped:
+        rc = L.gbx_qlinear_groups(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits, group_size, act, 0,
+                                  _stream_ptr(x.device))
+        if rc != 1:
+            _lib.check(rc)
+            return out.reshape(*xshape[:-1], n)
     if need:
         ws = torch.empty((need,), dtype=torch.uint8, device=x.device)
         rc = L.gbx_qlinear_forward_ws(
