@@ -81,6 +81,8 @@ def lib() -> ctypes.CDLL:
         L.gbx_step_feed.argtypes = [p, p, i32, p, i64, p]
         L.gbx_step_words.argtypes = [p, p, p, p, p, p]
         L.gbx_qlinear_groups.argtypes = [p, p, p, p, p, p, i64, i32, i32, i32, i32, i32, i32, p]
+        L.gbx_qlinear_groups_multi.argtypes = [p, i32, p, p, p, p, p, p, i64, i32, i32, i32, i32, p]
+        L.gbx_qlinear_groups_win.argtypes = [i64, i32, i32, i32, i32]
         L.gbx_gather_mix_forward.argtypes = [p, p, p, p, p, p, p, p, i32, i32, i32, i32, i32, i32, i32, i32, p]
         L.gbx_dense_workspace_bytes.argtypes = [i64, i32, i32]
         L.gbx_dense_workspace_bytes.restype = ctypes.c_size_t
@@ -439,7 +441,8 @@ def host():
                 spec.loader.exec_module(mod)
             except ImportError:
                 return None
-            mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.gbx_qlinear_forward, L.gbx_qlinear_forward_ws, L.gbx_qlinear_workspace_bytes, L.gbx_qlinear_groups)))
+            mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.gbx_qlinear_forward, L.gbx_qlinear_forward_ws, L.gbx_qlinear_workspace_bytes, L.gbx_qlinear_groups,
+                                                                          L.gbx_qlinear_groups_win)))
             _host = mod
     return _host or None
 

@@ -22,6 +22,8 @@ ForwardWsFn forward_ws_fn = nullptr;
 WorkspaceFn workspace_fn = nullptr;
 typedef int (*GroupsFn)(const void*, const void*, const void*, const void*, const void*, void*, int64_t, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, void*);
 GroupsFn groups_fn = nullptr;
+typedef int (*GroupsWinFn)(int64_t, int32_t, int32_t, int32_t, int32_t);
+GroupsWinFn groups_win_fn = nullptr;
 
 constexpr int64_t FEW_ROWS = 256;          // from here on a resident image of the weight may be the faster operand (ops.py decides)
 constexpr int F16 = 0, BF16 = 1;
@@ -38,19 +40,20 @@ bool watched() {                            // something is to see every operati
 }
 
 PyObject* bind(PyObject*, PyObject* args) {
-  unsigned long long f, w, s, g;
-  if (!PyArg_ParseTuple(args, "KKKK", &f, &w, &s, &g)) return nullptr;
+  unsigned long long f, w, s, g, gw;
+  if (!PyArg_ParseTuple(args, "KKKKK", &f, &w, &s, &g, &gw)) return nullptr;
   forward_fn = reinterpret_cast<ForwardFn>(static_cast<uintptr_t>(f));
   forward_ws_fn = reinterpret_cast<ForwardWsFn>(static_cast<uintptr_t>(w));
   workspace_fn = reinterpret_cast<WorkspaceFn>(static_cast<uintptr_t>(s));
   groups_fn = reinterpret_cast<GroupsFn>(static_cast<uintptr_t>(g));
+  groups_win_fn = reinterpret_cast<GroupsWinFn>(static_cast<uintptr_t>(gw));
   Py_RETURN_NONE;
 }
 
-// few_rows(x, qweight, scales, zeros, group_size, bits, bias or None) -> y, None (not a call for this path) or the library's error code
+// few_rows(x, qweight, scales, zeros, group_size, bits, bias or None[, whether 256 rows and more may go as groups of 32]) -> y, None (not a call for this path) or the library's error code
 PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 7 || !forward_fn) Py_RETURN_NONE;
+  if ((n_args != 7 && n_args != 8) || !forward_fn) Py_RETURN_NONE;
   for (int i = 0; i < 4; ++i)
     if (!THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
   const bool has_bias = args[6] != Py_None;
@@ -70,7 +73,9 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (k < 1 || n < 1 || k > 0x7fffffff || n > 0x7fffffff || x.size(-1) != k || k % group || sc.size(0) != n || sc.size(1) != k / group || ze.size(0) != n || ze.size(1) != k / group)
     Py_RETURN_NONE;
   const int64_t m = x.numel() / k;
-  if (m < 1 || m >= FEW_ROWS) Py_RETURN_NONE;
+  // rows of several sequences keep the order of sums that they had (see quantized_matmul in ops.py)
+  const bool grouped = m > 32 && !(x.dim() == 3 && x.size(0) > 1) && groups_win_fn(m, static_cast<int32_t>(n), static_cast<int32_t>(k), static_cast<int32_t>(bits), static_cast<int32_t>(group));
+  if (m < 1 || (m >= FEW_ROWS && (!grouped || n_args < 8 || args[7] != Py_True))) Py_RETURN_NONE;
   const void* bias = nullptr;
   if (has_bias) {
     const at::Tensor& b = THPVariable_Unpack(args[6]);
@@ -84,11 +89,11 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
   const int act = type == at::kBFloat16 ? BF16 : F16;
   const int32_t N = static_cast<int32_t>(n), K = static_cast<int32_t>(k), B = static_cast<int32_t>(bits), G = static_cast<int32_t>(group);
-  // rows of several sequences keep the order of sums that they had (see ops.quantized_matmul)
-  if (m > 32 && !(x.dim() == 3 && x.size(0) > 1)) {
+  if (grouped) {
     const int rc = groups_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, 0, stream);
     if (rc == 0) return THPVariable_Wrap(std::move(y));
     if (rc != 1) return PyLong_FromLong(rc);
+    if (m >= FEW_ROWS) Py_RETURN_NONE;
   }
   // scratch: decode batches and short prompts split k across workgroups
   const size_t need = (m >= 2 && m <= 32) || m > 64 ? workspace_fn(m, N, K, B, G) : 0;

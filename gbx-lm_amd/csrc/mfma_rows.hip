@@ -179,13 +179,13 @@ hipError_t launch_rows(const MfmaArgs& a, bool bf16, hipStream_t s) {
 
 }  // namespace
 
-constexpr int SLAB_ROWS = 1023;             // in groups of 32
+constexpr int SLAB_ROWS = 4096;             // in groups of 32
 
-// (contractions under 1024: see below; one row: what is left of 33, by the kernel of the other 32)
+// (contractions under 1024 of up to 32 rows: see below; one row: what is left of 33, by the kernel of the other 32)
 hipError_t launch_qgemm_slab(const MfmaArgs& a, int bits, bool bf16, hipStream_t s) {
   uintptr_t affine = reinterpret_cast<uintptr_t>(a.scales) | reinterpret_cast<uintptr_t>(a.zeros);
   for (int g = 1; g < a.nseg; ++g) affine |= reinterpret_cast<uintptr_t>(a.scales_x[g - 1]) | reinterpret_cast<uintptr_t>(a.zeros_x[g - 1]);
-  if (a.swiglu || a.ws || a.M < 1 || a.M > (a.nseg > 1 ? 32 : SLAB_ROWS) || a.K % 128 || a.K < 1024 || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
+  if (a.swiglu || a.ws || a.M < 1 || a.M > (a.nseg > 1 ? 64 : SLAB_ROWS) || a.K % 128 || (a.M <= 32 && a.K < 1024) || a.log2g < 5 || a.log2g > 7 || affine % (256u >> a.log2g)) return hipErrorInvalidValue;
   return bits == 2 ? launch_slab_bits<2>(a, bf16, s) : bits == 3 ? launch_slab_bits<3>(a, bf16, s) : bits == 4 ? launch_slab_bits<4>(a, bf16, s) : hipErrorInvalidValue;
 }
 
@@ -215,28 +215,40 @@ hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t
   return bits == 2 ? launch_rows<2>(a, bf16, s) : bits == 3 ? launch_rows<3>(a, bf16, s) : bits == 4 ? launch_rows<4>(a, bf16, s) : hipErrorInvalidValue;
 }
 
-// Where products of 33 to 1023 rows are faster as groups of up to 32 on the slab kernel than as tiles of dequantised weights (or, up to 64 rows, on the other few-row kernels).
-// Both grow with their tiles; here a tile of 16 outputs x 32 rows takes a CU 0.8 to 2.3 us, by the length of the contraction and by how dear the fields and scales are to take
-// apart, behind a start of 5 us, there the chip is filled by tiles of 64 rows and more.  So the line is a number of tiles a CU.  There | here, us:
+// Where products of 33 to 4096 rows are faster as groups of up to 32 on the slab kernel than as tiles of dequantised weights (up to 64 rows: than on the other few-row kernels;
+// from 1024 on: than by a 16-bit image).  Both grow with their tiles; here a tile of 16 outputs x 32 rows takes a CU 0.5 to 2.3 us, by the length of the contraction and by how dear
+// the fields and scales are to take apart, behind a start of 5 us, there the chip is filled by tiles of 64 rows and more.  So the line is a number of tiles a CU.  There | here, us:
 //   33 rows 4096 x 4096, 4 bits, group 128 14.8 | 8.6, 3 bits, group 64 19.1 | 9.3; 8192 x 3072 23.8 | 9.0, 24.2 | 10.9; 14336 x 4096 33.9 | 14.7, group 32 50 | 21
 //   200 rows 1024 x 4096 18.6 | 8.6; 2048 x 2048 19.5 | 7.2; 4096 x 4096 28.5 | 16.3, 3 bits, group 64 29.8 | 20.8, 4 bits, group 32 29.4 | 23.6; 700 x 1280 15.2 | 5.5
 //   K from 3072 on, groups of 64 and 128, 32 tiles a CU: 1000 rows 4096 x 4096 77.5 | 60.1, 512 8192 x 3072 60.0 | 49.3; more: 700 8192 x 3072 63.8 | 71.1, 450 11008 x 4096 79 | 92
 //   shorter: 16 tiles 255 rows 8192 x 1536 28.8 | 19.6 to 21.5, 32 tiles 36.6 | 36.6 to 39.3; K 1152, 12 to 16 tiles 18.6 | 17.0 to 19.4, 28 tiles 30 | 33 to 38
+//   K 256 and 768, 16 tiles: 100 rows of 16384 17.3 | 10.3 to 15.4, 20.4 | 12.9 to 20.0; 32 tiles 16.6 | 19.1 to 28.9, 24.6 | 24.6 to 38.1
 //   3 bits, group 64, 16 tiles: 512 rows 4096 x 4096 41.5 | 39.3, 1000 2048 x 2048 32.8 | 25.7; 19 to 24 tiles 52 | 54, 55 | 67; K 1152, 12 tiles 18.6 | 20.8
 //   groups of 32: 8 tiles 128 rows 8192 x 3072 27.6 | 21.1, 65 11008 x 4096 33.2 | 33.3; 10 tiles 36.6 | 38.2; 3 bits, 5 tiles 29.5 | 27.8, 8 tiles 30.3 | 32.3
+//   from 1024 rows on, where few outputs leave the image's tiles few: 1024 rows 1024 x 4096 (8 tiles) 26.3 | 21.3, 2000 200 x 3072 (3) 24.7 | 13.2; 1500 1024 x 4096 (12) 31.5 | 33.4
 static bool groups_win(int64_t M, int N, int K, int bits, int log2g) {
   const int64_t groups = (M + 31) / 32, tiles = (N + 15) / 16;
-  const int a_cu = log2g == 5 ? (bits == 3 ? 5 : 8) : bits == 3 && log2g == 6 ? (K >= 2048 ? 16 : 8) : K >= 3072 ? 32 : K >= 1536 ? 16 : 8;
+  const int dear = log2g == 5 ? (bits == 3 ? 5 : 8) : bits == 3 && log2g == 6 ? (K >= 2048 ? 16 : 8) : K >= 3072 ? 32 : K >= 1536 ? 16 : 8;
+  const int a_cu = M >= 1024 ? (log2g == 5 ? 5 : 8) : K < 1024 && (bits != 3 || log2g != 5) ? 16 : dear;
   return groups <= 2 || groups * tiles <= 256 * a_cu;
 }
 
 }  // namespace gbx
 
-// Products of 33 to 1023 rows as groups of up to 32 that the slab kernel takes side by side, where that is the faster form (`always`: wherever it can).  1: not a call for it,
+static bool groups_force_generic() {
+  static const bool force = gbx::env_switch("GBX_FORCE_GENERIC") != 0;
+  return force;
+}
+
+// Products of 33 to 4096 rows as groups of up to 32 that the slab kernel takes side by side, where that is the faster form (`always`: wherever it can).  1: not a call for it,
 // nothing was launched.  For this package's own Python layer; not part of the public header.
+extern "C" int gbx_qlinear_groups_win(int64_t M, int32_t N, int32_t K, int32_t bits, int32_t group_size) {
+  return M >= 33 && M <= gbx::SLAB_ROWS && N >= 1 && K >= 128 && K <= 4096 && K % 128 == 0 && bits >= 2 && bits <= 4 && (group_size == 32 || group_size == 64 || group_size == 128) &&
+         gbx::groups_win(M, N, K, bits, group_size == 32 ? 5 : group_size == 64 ? 6 : 7);
+}
 extern "C" int gbx_qlinear_groups(const void* x, const uint32_t* qweight, const void* scales, const void* zeros, const void* bias, void* y, int64_t M, int32_t N, int32_t K,
                                   int32_t bits, int32_t group_size, int32_t act_dtype, int32_t always, void* hip_stream) {
-  if (!x || !qweight || !scales || !zeros || !y || M < 33 || M >= 1024 || N < 1 || K < 1024 || K > 4096 || K % 128 || bits < 2 || bits > 4 || (group_size != 32 && group_size != 64 && group_size != 128) ||
+  if (!x || !qweight || !scales || !zeros || !y || M < 33 || M > gbx::SLAB_ROWS || N < 1 || K < 128 || K > 4096 || K % 128 || bits < 2 || bits > 4 || (group_size != 32 && group_size != 64 && group_size != 128) ||
       (act_dtype != 0 && act_dtype != 1) || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(qweight) % 16)
     return 1;
   gbx::MfmaArgs a{};
@@ -244,8 +256,33 @@ extern "C" int gbx_qlinear_groups(const void* x, const uint32_t* qweight, const 
   a.qweight = qweight; a.scales = static_cast<const unsigned short*>(scales); a.zeros = static_cast<const unsigned short*>(zeros);
   a.bias = static_cast<const unsigned short*>(bias); a.y = static_cast<unsigned short*>(y);
   a.M = static_cast<int>(M); a.N = N; a.K = K; a.log2g = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
-  static const bool force_generic = gbx::env_switch("GBX_FORCE_GENERIC") != 0;
-  if (force_generic || (!always && !gbx::groups_win(M, N, K, bits, a.log2g))) return 1;
+  if (groups_force_generic() || (!always && !gbx::groups_win(M, N, K, bits, a.log2g))) return 1;
+  const hipError_t e = gbx::launch_qgemm_slab(a, bits, act_dtype == 1, static_cast<hipStream_t>(hip_stream));
+  return e == hipSuccess ? 0 : e == hipErrorInvalidValue ? 1 : 2;
+}
+
+// The same for 33 to 64 rows of two or three layers of one input (q, k, v): one launch, with the sums of a call per layer (from 65 rows on every layer is a call).  Split contraction
+// of dequantised weights | here, us, 33 and 64 rows: 4096, 512 and 512 x 2048, 4 bits, group 128 9.8 9.8 | 6.0 6.3, 3 bits, group 64 12.6 12.9 | 7.0 7.5; 2048, 1024 and 1024 x 1024,
+// 2 bits 8.1 8.5 | 4.1 4.3; three of 4096 x 4096, 4 bits 32.7 30.5 | 22.5 22.9; two of 12288 x 4096, 2 bits, in two passes of the batch kernel 22.0 25.6 | 23.0 23.7.
+extern "C" int gbx_qlinear_groups_multi(const void* x, int32_t nseg, const void* const* qweight, const void* const* scales, const void* const* zeros, const void* const* bias,
+                                        void* const* y, const int32_t* N, int64_t M, int32_t K, int32_t bits, int32_t group_size, int32_t act_dtype, void* hip_stream) {
+  if (!x || nseg < 2 || nseg > 3 || M < 33 || M > 64 || K < 128 || K > 4096 || K % 128 || bits < 2 || bits > 4 || (group_size != 32 && group_size != 64 && group_size != 128) ||
+      (act_dtype != 0 && act_dtype != 1) || reinterpret_cast<uintptr_t>(x) % 16 || groups_force_generic())
+    return 1;
+  gbx::MfmaArgs a{};
+  a.x = static_cast<const unsigned short*>(x);
+  a.M = static_cast<int>(M); a.N = N[0]; a.K = K; a.log2g = group_size == 32 ? 5 : group_size == 64 ? 6 : 7; a.nseg = nseg;
+  for (int g = 0; g < nseg; ++g) {
+    if (!qweight[g] || !scales[g] || !zeros[g] || !y[g] || N[g] < 1 || reinterpret_cast<uintptr_t>(qweight[g]) % 16) return 1;
+    const auto half = [](const void* p) { return static_cast<const unsigned short*>(p); };
+    const auto w = static_cast<const uint32_t*>(qweight[g]);
+    a.n_seg[g] = N[g];
+    if (g == 0) {
+      a.qweight = w; a.scales = half(scales[0]); a.zeros = half(zeros[0]); a.bias = half(bias[0]); a.y = static_cast<unsigned short*>(y[0]);
+    } else {
+      a.qweight_x[g - 1] = w; a.scales_x[g - 1] = half(scales[g]); a.zeros_x[g - 1] = half(zeros[g]); a.bias_x[g - 1] = half(bias[g]); a.y_x[g - 1] = static_cast<unsigned short*>(y[g]);
+    }
+  }
   const hipError_t e = gbx::launch_qgemm_slab(a, bits, act_dtype == 1, static_cast<hipStream_t>(hip_stream));
   return e == hipSuccess ? 0 : e == hipErrorInvalidValue ? 1 : 2;
 }

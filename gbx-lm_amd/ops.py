@@ -212,7 +212,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise NotImplementedError("quantized_matmul(transpose=False) is not on the QuantizedLinear path")
     if out is None:
         few = _few_rows or _bind_few_rows()
-        y = few(x, w, scales, biases, group_size, bits, bias)
+        y = few(x, w, scales, biases, group_size, bits, bias, not _dense_cache.entries)      # (256 rows on: only while no weight has a resident image)
         if y is not None:
             if type(y) is int:
                 _lib.check(y)
@@ -258,15 +258,19 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise ValueError("out must be a contiguous [M, N] tensor of the activation dtype")
     bias_ptr = bias.data_ptr() if bias is not None else None
     L = _lib.lib()
-    # 33 to 1023 rows as groups of 32 side by side, where that is faster and no resident image is there to multiply by.  Rows of several sequences (a leading size over 1) keep the
-    # kernel and the order of sums that they had: a batch's caches are what its later steps are compared by, and two roundings drift apart over a stack of layers.
-    grouped = 32 < m < 1024 and not (len(xshape) == 3 and xshape[0] > 1)
-    if grouped and m < 256:
-        rc = L.gbx_qlinear_groups(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits, group_size, act, 0,
-                                  _stream_ptr(x.device))
+    # 33 rows on as groups of 32 side by side, where that is faster and the weight has no resident image.  Rows of several sequences (a leading size over 1) keep the kernel and the
+    # order of sums that they had: a batch's caches are what its later steps are compared by, and two roundings drift apart over a stack of layers.
+    several = len(xshape) == 3 and xshape[0] > 1
+
+    def groups() -> bool:
+        rc = 1 if several or m < 33 else L.gbx_qlinear_groups(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits,
+                                                              group_size, act, 0, _stream_ptr(x.device))
         if rc != 1:
             _lib.check(rc)
-            return out if len(xshape) == 2 else out.reshape(*xshape[:-1], n)
+        return rc == 0
+
+    if m < 256 and groups():
+        return out if len(xshape) == 2 else out.reshape(*xshape[:-1], n)
     # scratch: decode batches / short prompts split k across workgroups, long prompts dequantise once
     need = L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) if (2 <= m <= 32 or m > 64) else 0
     if m < 256:                                         # no resident images at these sizes: nothing more to decide
@@ -297,6 +301,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         # prompt-sized call on the dense path: the [N, K] image is built once (gbx_dequantize), kept resident, and every call
         # runs the GEMM alone (gbx_dense_forward_ws: k split over workgroups with fp32 scratch for few-tile shapes)
         dense = _dense_cache.get(src, ckey)
+        if dense is None and groups():
+            return out.reshape(*xshape[:-1], n)
         if dense is None:
             dense = _alloc_dense((n, k), x.dtype, x.device)
             if dense is not None:
@@ -310,12 +316,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                                         m, n, k, _DT[x.dtype], scratch.data_ptr() if part else None, part, _stream_ptr(x.device))
             if rc == _lib.GBX_OK:
                 return out.reshape(*x.shape[:-1], n)
-    if grouped:
-        rc = L.gbx_qlinear_groups(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, bits, group_size, act, 0,
-                                  _stream_ptr(x.device))
-        if rc != 1:
-            _lib.check(rc)
-            return out.reshape(*xshape[:-1], n)
+    if not cacheable and groups():
+        return out.reshape(*xshape[:-1], n)
     if need:
         ws = torch.empty((need,), dtype=torch.uint8, device=x.device)
         rc = L.gbx_qlinear_forward_ws(
@@ -487,11 +489,13 @@ def quantized_matmul_multi(x: torch.Tensor, mods, pre_norm=None) -> list:
     ys = [torch.empty((rows, m.output_dims), dtype=x.dtype, device=x.device) for m in mods]
     n = len(mods)
     VP, I32 = ctypes.c_void_p * n, ctypes.c_int32 * n
-    _lib.check(_lib.lib().gbx_qlinear_forward_multi(
-        x2.data_ptr(), n, VP(*[m.qweight.data_ptr() for m in mods]), VP(*[m.scales.data_ptr() for m in mods]),
-        VP(*[m.zeros.data_ptr() for m in mods]), VP(*[(m.bias.data_ptr() if m.bias is not None else None) for m in mods]),
-        VP(*[y.data_ptr() for y in ys]), I32(*[m.output_dims for m in mods]), rows, k, m0.bits, m0.group_size,
-        _DT[x.dtype], _stream_ptr(x.device)))
+    args = (x2.data_ptr(), n, VP(*[m.qweight.data_ptr() for m in mods]), VP(*[m.scales.data_ptr() for m in mods]),
+            VP(*[m.zeros.data_ptr() for m in mods]), VP(*[(m.bias.data_ptr() if m.bias is not None else None) for m in mods]),
+            VP(*[y.data_ptr() for y in ys]), I32(*[m.output_dims for m in mods]), rows, k, m0.bits, m0.group_size,
+            _DT[x.dtype], _stream_ptr(x.device))
+    # over 32 rows of one sequence: the kernel that a call per module takes (quantized_matmul)
+    rc = _lib.lib().gbx_qlinear_groups_multi(*args) if rows > 32 and not (x.dim() == 3 and x.shape[0] > 1) else 1
+    _lib.check(rc if rc != 1 else _lib.lib().gbx_qlinear_forward_multi(*args))
     return [y.reshape(*x.shape[:-1], m.output_dims) for y, m in zip(ys, mods)]
 
 

@@ -1,4 +1,4 @@
-"""Packed products of 33 to 1023 rows as groups of up to 32 (gbx_qlinear_groups): rows and outputs that end inside a group or a tile, every width, group and type, a bias, infinities in
+"""Packed products of 33 to 4096 rows as groups of up to 32 (gbx_qlinear_groups): rows and outputs that end inside a group or a tile, every width, group and type, a bias, infinities in
 one group's rows; against float64.  And the calls: what takes that way, what keeps the one it had."""
 import numpy as np
 import pytest
@@ -36,7 +36,7 @@ def _groups(x, w, s, z, bias, bits, group, always=1):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits,group", [(b, g) for b in (2, 3, 4) for g in (32, 64, 128)])
-@pytest.mark.parametrize("rows,n,k", [(33, 16, 1024), (64, 17, 4096), (65, 700, 1152), (97, 1, 2048), (511, 4111, 1280), (1023, 31, 3072), (200, 9000, 1024)])
+@pytest.mark.parametrize("rows,n,k", [(33, 16, 1024), (64, 17, 4096), (65, 700, 1152), (97, 1, 2048), (511, 4111, 1280), (1023, 31, 3072), (200, 9000, 1024), (4096, 40, 128), (70, 300, 640)])
 def test_against_float64(dt, bits, group, rows, n, k):
     w, s, z, bias = _layer(n, k, bits, group, dt, rows + n, bias=n == 700)
     x = torch.randn((rows, k), generator=torch.Generator().manual_seed(k)).to(dt).to(DEV)
@@ -68,7 +68,7 @@ def test_infinities_stay_in_their_rows():
 
 
 def test_what_it_does_not_take():
-    for rows, n, k, bits, group in ((32, 64, 1024, 4, 64), (1024, 64, 1024, 4, 64), (64, 64, 896, 4, 64), (64, 64, 4224, 4, 64)):
+    for rows, n, k, bits, group in ((32, 64, 1024, 4, 64), (4097, 64, 1024, 4, 64), (64, 64, 1088, 4, 64), (64, 64, 4224, 4, 64)):
         w, s, z, _ = _layer(n, k, bits, group, torch.bfloat16, 3)
         assert _groups(torch.zeros((rows, k), device=DEV).bfloat16(), w, s, z, None, bits, group) == 1
     w, s, z, _ = _layer(11008, 4096, 3, 32, torch.bfloat16, 3)
@@ -76,7 +76,7 @@ def test_what_it_does_not_take():
     assert _groups(x, w, s, z, None, 3, 32, always=0) == 1 and torch.is_tensor(_groups(x, w, s, z, None, 3, 32)) and torch.is_tensor(_groups(x[:64], w, s, z, None, 3, 32, always=0))
 
 
-@pytest.mark.parametrize("rows", [33, 100, 255, 256, 600])
+@pytest.mark.parametrize("rows", [33, 100, 255, 256, 600, 2000])
 @pytest.mark.parametrize("native", [True, False])
 def test_calls(monkeypatch, rows, native):
     """Rows of one sequence go that way, by the native call and by the general one; those of several keep theirs, and 256 rows on whose weight has a resident image."""
@@ -89,7 +89,38 @@ def test_calls(monkeypatch, rows, native):
     want = _groups(x, w, s, z, bias, 4, 128, always=0)
     call = lambda t: ops.quantized_matmul(t, w, s, z, group_size=128, bits=4, bias=bias)
     assert torch.equal(call(x), want) and torch.equal(call(x[None]), want[None]) and torch.equal(call(x[:, None].transpose(0, 1)), want[None])
+    assert ops._dense_cache.get((w, s, z), (n, k, 4, 128, x.dtype, x.device.index)) is None       # (no image was built for it)
     if rows % 2 == 0:
         other = call(x.view(2, rows // 2, k)).view(rows, n)
         assert ((other.double() - want.double()).abs() <= 2.0 ** -6 * want.double().abs() + 0.05).all()
         assert not torch.equal(other, want)
+        ops.dense_cache_clear()
+    if rows == 600:
+        image = ops.dequantize(w, s, z, 128, 4)
+        ops._dense_cache.put((w, s, z), (n, k, 4, 128, x.dtype, x.device.index), image)
+        dense, exact = call(x), x.double() @ image.double().t()
+        assert not torch.equal(dense, want)
+        # two roundings to 8 bits, of the product and of its sum with the bias
+        assert ((dense.double() - exact - bias.double()).abs() <= 2.0 ** -8 * (exact.abs() + (exact + bias.double()).abs()) + 1e-4).all()
+        ops.dense_cache_clear()
+
+
+@pytest.mark.parametrize("bits,group,k", [(2, 128, 4096), (3, 64, 1152), (4, 32, 640)])
+@pytest.mark.parametrize("rows", [33, 64])
+def test_layers_of_one_input(bits, group, k, rows):
+    """Two or three layers in one launch: the bits of a call each; rows of several sequences keep the launch that they had."""
+    from gbx_lm_amd.models.quantized_linear_gba import QuantizedLinear
+    mods = []
+    for i, n in enumerate((544, 32, 96)):
+        w, s, z, bias = _layer(n, k, bits, group, torch.bfloat16, 7 * i + rows, bias=i == 1)
+        q = QuantizedLinear(k, n, i == 1, group, bits)
+        q._buffers.update(qweight=w, scales=s, zeros=z, **({"bias": bias} if i == 1 else {}))
+        mods.append(q)
+    x = torch.randn((rows, k), generator=torch.Generator().manual_seed(rows)).bfloat16().to(DEV)
+    for some in (mods, mods[:2]):
+        for y, q in zip(ops.quantized_matmul_multi(x, some), some):
+            assert torch.equal(y, q(x)) and torch.equal(y, _groups(x, q.qweight, q.scales, q.zeros, q.bias, bits, group, always=0))
+    one = ops.quantized_matmul_multi(x[None], mods)
+    assert all(torch.equal(y[0], q(x)) for y, q in zip(one, mods))
+    for y, v in zip(ops.quantized_matmul_multi(x[:, None], mods), one):
+        assert ((y[:, 0].double() - v[0].double()).abs() <= 2.0 ** -6 * v[0].double().abs() + 0.05).all()
