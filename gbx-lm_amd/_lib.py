@@ -488,7 +488,7 @@ def mixers() -> ctypes.CDLL:
         L.gbxm_log_softmax_workspace.argtypes, L.gbxm_log_softmax_workspace.restype = [i64, i32], sz
         L.gbxm_log_softmax.argtypes = [p, p, i64, i32, i32, p, sz, p]
         L.gbxm_log_softmax_scaled.argtypes = [p, p, i64, i32, i32, i32, f32, p, sz, p]
-        L.gbxm_step_advance.argtypes = [p, i32, p, p, p, i32, p]
+        L.gbxm_step_advance.argtypes = [p, i32, i64, p, p, p, i32, p]
         L.gbxm_packed_experts_workspace.argtypes, L.gbxm_packed_experts_workspace.restype = [i64, i32, i32], sz
         L.gbxm_packed_experts.argtypes = [ctypes.POINTER(PackedExpertsArgs), p]
         L.gbxm_expert_ff.argtypes = [ctypes.POINTER(ExpertArgs), p]

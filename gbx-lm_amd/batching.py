@@ -128,11 +128,12 @@ class _DecodeGraph:
         self.copied[k].record(torch.cuda.current_stream(self.static.device))
         self.batch.pos0 = self.at = list(pos0)
 
-    def advance(self, tokens: torch.Tensor) -> None:
-        """The next token of every sequence, from the device: one small launch instead of a copy from the host that has read them there first."""
+    def advance(self, tokens: torch.Tensor, rows: int) -> None:
+        """The next token of every sequence, from the device: one small launch instead of a copy from the host that has read them there first.  What is no row of an
+        embedding of ``rows`` goes on as token 0."""
         from . import _lib, ops
         b = len(self.slots)
-        _lib.check_mixers(_lib.mixers().gbxm_step_advance(tokens.data_ptr(), tokens.element_size(), self.static.data_ptr(), self.batch.seq.data_ptr(),
+        _lib.check_mixers(_lib.mixers().gbxm_step_advance(tokens.data_ptr(), tokens.element_size(), rows, self.static.data_ptr(), self.batch.seq.data_ptr(),
                                                           self.batch.tok.data_ptr(), b, ops._stream_ptr(self.static.device)))
         self.batch.pos0 = self.at = [p + 1 for p in self.at]
 
@@ -271,6 +272,9 @@ class BatchScheduler:
             return None
         if self.max_tokens is not None and self.slots.live_tokens() + len(ids) > self.max_tokens:
             return None
+        table = getattr(self.model, "token_rows", None)              # (tokens that nobody has looked at yet stay inside the embedding)
+        if table is None:
+            return None
         slots = tuple(self.slot_of[i] for i in ids)
         at = [self.slots.length[s] - 1 for s in slots]
         g = self._current_graph(slots, max(at) + 2)
@@ -281,7 +285,7 @@ class BatchScheduler:
         host.copy_(tokens, non_blocking=True)
         there = torch.cuda.Event()
         there.record(torch.cuda.current_stream(self.device))
-        g.advance(tokens)
+        g.advance(tokens, table)
         rows = g.run(self)
         for s in slots:
             self.slots.length[s] += 1
@@ -342,6 +346,8 @@ class BatchScheduler:
                 out[i].append(int(t))
                 if int(t) in stop or len(out[i]) >= max_tokens:
                     self.release(ids[i])
+                elif ahead is not None and not 0 <= t < self.model.token_rows:
+                    raise ValueError(f"the sampler chose token {t}, which is neither a stop token nor one of the model's {self.model.token_rows}")
                 else:
                     feed[i] = [int(t)]
                     nxt.append(i)

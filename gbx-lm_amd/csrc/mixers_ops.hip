@@ -259,11 +259,14 @@ __global__ __launch_bounds__(256) void step_tables_kernel(const int* __restrict_
 // The tokens of the next step of the same sequences, from where they were chosen, and every position one further: what a step needs that is enqueued before the host has
 // read them.  A step of the 4-layer models in batching.py's loop, us, tokens through the host | ahead of it: one sequence, several streams of 1024 244 | 219; two, latent attention 387 |
 // 362; 32, sandwich norms 1124 | 1080 (a replay of the step alone: 200, 332 and 1043).
+// The host has not yet looked at the tokens: one that is no row of the embedding (a sampler's end mark) goes on as token 0, in a step whose row the host then drops.
 template <typename I>
-__global__ __launch_bounds__(256) void step_advance_kernel(const I* __restrict__ from, int64_t* __restrict__ tokens, int* __restrict__ seq, int* __restrict__ tok, int B) {
+__global__ __launch_bounds__(256) void step_advance_kernel(const I* __restrict__ from, int64_t rows, int64_t* __restrict__ tokens, int* __restrict__ seq, int* __restrict__ tok,
+                                                           int B) {
   const int b = threadIdx.x;
   if (b >= B) return;
-  tokens[b] = from[b];
+  const int64_t v = from[b];
+  tokens[b] = v >= 0 && v < rows ? v : 0;
   seq[4 * b + 1] += 1;
   tok[2 * b + 1] += 1;
 }
@@ -702,13 +705,13 @@ extern "C" int gbxm_log_softmax_scaled(const void* x, void* out, int64_t rows, i
   return after_launch("log_softmax");
 }
 
-extern "C" int gbxm_step_advance(const void* from, int32_t from_bytes, int64_t* tokens, int32_t* seq, int32_t* tok, int32_t B, void* stream) {
-  if (!from || !tokens || !seq || !tok || B < 1 || B > 256 || (from_bytes != 4 && from_bytes != 8) || reinterpret_cast<uintptr_t>(from) % from_bytes ||
+extern "C" int gbxm_step_advance(const void* from, int32_t from_bytes, int64_t rows, int64_t* tokens, int32_t* seq, int32_t* tok, int32_t B, void* stream) {
+  if (!from || rows < 1 || !tokens || !seq || !tok || B < 1 || B > 256 || (from_bytes != 4 && from_bytes != 8) || reinterpret_cast<uintptr_t>(from) % from_bytes ||
       reinterpret_cast<uintptr_t>(tokens) % 8 || (reinterpret_cast<uintptr_t>(seq) | reinterpret_cast<uintptr_t>(tok)) % 4)
     return fail(GBXM_ERR_INVALID, "step_advance: bad argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (from_bytes == 8) step_advance_kernel<int64_t><<<1, 256, 0, s>>>(static_cast<const int64_t*>(from), tokens, seq, tok, B);
-  else step_advance_kernel<int><<<1, 256, 0, s>>>(static_cast<const int*>(from), tokens, seq, tok, B);
+  if (from_bytes == 8) step_advance_kernel<int64_t><<<1, 256, 0, s>>>(static_cast<const int64_t*>(from), rows, tokens, seq, tok, B);
+  else step_advance_kernel<int><<<1, 256, 0, s>>>(static_cast<const int*>(from), rows, tokens, seq, tok, B);
   return after_launch("step_advance");
 }
 

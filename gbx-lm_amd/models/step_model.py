@@ -49,6 +49,11 @@ class RaggedStepModel(nn.Module):
     def layers(self):
         return [self.model.layers[i] for i in self.layer_runs]
 
+    @property
+    def token_rows(self) -> int:
+        """Rows of the token embedding: ids outside [0, token_rows) are none."""
+        return self.model.embed_tokens.weight.shape[0]
+
     def required_kernels(self) -> None:
         """Load (and, in a checkout without built files, first compile) the one kernel library these models run on."""
         from .. import _lib

@@ -35,9 +35,9 @@ int gbxm_embed_scaled(const void* table, const int64_t* tokens, float* x, void* 
 size_t gbxm_log_softmax_workspace(int64_t rows, int32_t n);
 int gbxm_log_softmax(const void* x, void* out, int64_t rows, int32_t n, int32_t type, void* ws, size_t ws_bytes, void* stream);
 int gbxm_log_softmax_scaled(const void* x, void* out, int64_t rows, int32_t n, int32_t type, int32_t out_type, float scale, void* ws, size_t ws_bytes, void* stream);
-/* The next step of the same B <= 256 sequences, one token each: tokens[b] <- from[b] (whole numbers of 4 or 8 bytes), the positions in seq [B][4] and tok [B][2] (of
- * gbxm_step_tables) one further. */
-int gbxm_step_advance(const void* from, int32_t from_bytes, int64_t* tokens, int32_t* seq, int32_t* tok, int32_t B, void* stream);
+/* The next step of the same B <= 256 sequences, one token each: tokens[b] <- from[b] (whole numbers of 4 or 8 bytes; 0 for one outside [0, rows), the embedding's
+ * rows), the positions in seq [B][4] and tok [B][2] (of gbxm_step_tables) one further. */
+int gbxm_step_advance(const void* from, int32_t from_bytes, int64_t rows, int64_t* tokens, int32_t* seq, int32_t* tok, int32_t B, void* stream);
 /* In place: rows[t][0:n0] and rows[t][n0:n0+n1] each RMS-normalised over the whole segment (fp32 statistics), times w0 / w1. */
 int gbxm_segment_rmsnorm(void* rows, int64_t T, int64_t row_stride, int32_t n0, int32_t n1, const float* w0, const float* w1,
                          float eps, int32_t act, void* stream);

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from gbx_lm_amd import synthetic as S
+from gbx_lm_amd import _lib, ops, synthetic as S
 from gbx_lm_amd.batching import BatchScheduler
 from gbx_lm_amd.mixer_ops import log_probabilities
 
@@ -81,3 +81,70 @@ def test_rows_of_the_head(dtype, rows, n, scale):
     want = y - torch.logsumexp(y, -1, keepdim=True)
     # fp32: a product, a difference and a logarithm, each within an ulp of values up to 2^6; n exponentials sum to a relative 2^-24 sqrt(n) at most 2^-15
     assert ((got.double() - want).abs() <= 2.0 ** -17 * want.abs().clamp(min=1.0) + 2.0 ** -15).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("b", [1, 5, 256])
+def test_tokens_ahead_of_the_host_stay_inside_the_embedding(dtype, b):
+    """Ids just outside the table and far from it become token 0; positions go on by one."""
+    rows, far = 1000, torch.iinfo(dtype)
+    ids = torch.tensor([-1, rows, rows - 1, 0, far.max, far.min, rows + 1, 1, 2 ** 31 - 1, -rows], dtype=dtype).repeat(26)[:b]
+    seq, tok = torch.arange(4 * b, dtype=torch.int32), torch.arange(2 * b, dtype=torch.int32)
+    dev = [t.to("cuda:0") for t in (ids, torch.full((b,), 7, dtype=torch.int64), seq, tok)]
+    L = _lib.mixers()
+    call = lambda n: L.gbxm_step_advance(dev[0].data_ptr(), ids.element_size(), n, dev[1].data_ptr(), dev[2].data_ptr(), dev[3].data_ptr(), b, ops._stream_ptr(dev[0].device))
+    assert call(0) == _lib.GBX_ERR_INVALID and call(-1) == _lib.GBX_ERR_INVALID
+    assert call(rows) == _lib.GBX_OK
+    assert torch.equal(dev[1].cpu(), torch.where((ids >= 0) & (ids < rows), ids, 0).long())
+    seq[1::4] += 1
+    tok[1::2] += 1
+    assert torch.equal(dev[2].cpu(), seq) and torch.equal(dev[3].cpu(), tok)
+
+
+@pytest.mark.parametrize("stop", [-1, "rows", 2 ** 40])
+def test_stop_tokens_that_are_no_tokens(stop):
+    """A sampler's end mark that the embedding has no row for ends its sequence, and the others get what they get from a loop that waits for the host."""
+    model, vocab = _model("tugolix")
+    assert model.token_rows == vocab
+    stop = vocab if stop == "rows" else stop
+    steps = 12
+    gen = torch.Generator().manual_seed(6)
+    forced = torch.randint(0, vocab, (steps, 2), generator=gen)
+    forced[9, 1] = stop
+    runs = []
+    for ahead in (True, False):
+        engine = BatchScheduler(model)
+        took, inner = [], engine._step_ahead
+
+        def counted(ids, toks):
+            got = inner(ids, toks) if ahead else None
+            took.append(got is not None)
+            return got
+
+        engine._step_ahead = counted
+        rows, n = [], [0]
+
+        def sampler(lp):
+            rows.append(lp)
+            n[0] += 1
+            return forced[n[0] - 1, :lp.shape[0]].to("cuda:0")
+
+        out = engine.generate([[5, 6], [7]], max_tokens=steps, sampler=sampler, stop_tokens=[stop])
+        assert out == [forced[:, 0].tolist(), forced[:10, 1].tolist()]
+        assert took[9] == ahead and not engine.slot_of
+        runs.append(rows)
+    for x, y in zip(*runs):
+        assert x.shape == y.shape and (x - y).abs().max() <= 0.05 * y.std()      # (the bound of the comparison above)
+
+
+def test_a_token_that_is_none_and_does_not_stop_raises():
+    model, vocab = _model("tugolix")
+    engine, n = BatchScheduler(model), [0]
+
+    def sampler(lp):
+        n[0] += 1
+        return torch.tensor([vocab if n[0] == 8 else 3], device="cuda:0")
+
+    with pytest.raises(ValueError, match="neither a stop token"):
+        engine.generate([[1, 2, 3]], max_tokens=20, sampler=sampler)
+    assert n[0] == 8
