@@ -404,7 +404,11 @@ def _dense_image(mod, m: int, dtype: torch.dtype, device):
     from 1024 rows on, where the dense path is the rule, built now); None: it would not."""
     w, scales, zeros = src = mod.qweight, mod.scales, mod.zeros
     n, k, bits, group_size = mod.output_dims, mod.input_dims, mod.bits, mod.group_size
-    if _dense_cache.budget < n * k * 2 or scales is None or scales.dtype != dtype or zeros.dtype != dtype or k % 64 or not all(t.is_cuda and t.is_contiguous() for t in src):
+    if any(t is None for t in src) or not all(t.is_cuda and t.device == device and t.is_contiguous() for t in src):
+        return None
+    # (what the module says of itself against what it holds: the launches go by the former)
+    if (w.dtype not in (torch.uint32, torch.int32) or scales.dtype != dtype or zeros.dtype != dtype or bits < 1 or group_size < 1 or k % 64 or k % group_size
+            or w.shape != (n, k * bits // 32) or scales.shape != (n, k // group_size) or zeros.shape != scales.shape or _dense_cache.budget < n * k * 2):
         return None
     L, ckey = _lib.lib(), (n, k, bits, group_size, dtype, device.index)
     rule = (m >= 1024 and m <= 61440 and L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) >= n * k * 2
@@ -429,16 +433,19 @@ def quantized_matmul_prompt(x: torch.Tensor, mods) -> Optional[list]:
     m = x.numel() // k if k else 0
     if not (x.is_cuda and m >= 256 and x.dtype in _DT and 2 <= len(mods) <= 3 and not torch.cuda.is_current_stream_capturing()
             and all(type(q) is QuantizedLinear and q.input_dims == k and not q._forward_hooks and not q._forward_pre_hooks for q in mods)
-            and all(q.bias is None or (q.bias.dtype == x.dtype and q.bias.is_cuda and q.bias.is_contiguous()) for q in mods)):
+            and all(q.bias is None or (q.bias.dtype == x.dtype and q.bias.is_cuda and q.bias.device == x.device and q.bias.shape == (q.output_dims,)
+                                       and q.bias.is_contiguous()) for q in mods)):
         return None
     # A matrix of 176 tiles fills the chip by itself (and is not split over k there): one launch for all of such gains nothing.  Each alone, k split where that helps | one
     # launch, us: 3072 + 1024 + 1024 outputs of 3072, 256 rows 59 | 42, 1024 81 | 46, 3001 118 | 74, 8000 234 | 209; 4096 + 1024 + 1024 of 4096, 1500 rows 118 | 72, 3001
     # 155 | 137; three of 4096 x 4096, 1024 146 | 84, 2500 (160 tiles) 224 | 193, 3001 (192 tiles) 237 | 253, 8000 591 | 599.
     if -(-m // 256) * min(-(-q.output_dims // 256) for q in mods) >= 176:
         return None
-    images = [_dense_image(q, m, x.dtype, x.device) for q in mods]
-    if any(t is None for t in images):
-        return None
+    images = []
+    for q in mods:
+        images.append(_dense_image(q, m, x.dtype, x.device))
+        if images[-1] is None:
+            return None
     x2 = x.reshape(-1, k).contiguous()
     ys = [x2.new_empty((m, q.output_dims)) for q in mods]
     n = len(mods)

@@ -133,6 +133,57 @@ def test_experts_of_many_pairs_leave_what_they_cannot_take_to_one_expert_at_a_ti
         ops.gather_quantized_matmul(x, m.qweight, m.scales, m.zeros, dev(idx), group_size=64, bits=4, bias=bias)
 
 
+def packed_layer(n=64, k=256, g=64, bits=4, **buffers):
+    """A packed layer whose buffers say that they are the GPU's; ``buffers`` take the places of those that fit it."""
+    from gbx_lm_amd.models.quantized_linear_gba import QuantizedLinear
+    m = QuantizedLinear(k, n, "bias" in buffers, g, bits)
+    fits = dict(qweight=torch.zeros((n, k // 32 * bits), dtype=torch.int32), scales=bf16(n, k // g), zeros=bf16(n, k // g))
+    for name, t in {**fits, **buffers}.items():
+        m._buffers[name] = t if t is None else dev(t)
+    return m
+
+
+MISFITS = {
+    "too few outputs": dict(qweight=torch.zeros((60, 32), dtype=torch.int32)),
+    "too few words": dict(qweight=torch.zeros((64, 24), dtype=torch.int32)),
+    "words of another type": dict(qweight=torch.zeros((64, 32))),
+    "words of 64 bits": dict(qweight=torch.zeros((64, 32), dtype=torch.int64)),
+    "too few groups": dict(scales=bf16(64, 2)),
+    "scales of too few outputs": dict(scales=bf16(32, 4), zeros=bf16(32, 4)),
+    "zeros of another shape": dict(zeros=bf16(64, 2)),
+    "scales of one rank": dict(scales=bf16(256)),
+    "scales of another type": dict(scales=torch.randn(64, 4)),
+    "no zeros": dict(zeros=None),
+    "words on another device": dict(qweight=torch.zeros((64, 32), dtype=torch.int32, device="meta")),
+    "scales on another device": dict(scales=torch.empty((64, 4), dtype=torch.bfloat16, device="meta")),
+    "short bias": dict(bias=bf16(32)),
+    "long bias": dict(bias=bf16(65)),
+    "column as bias": dict(bias=bf16(64, 1)),
+    "bias on another device": dict(bias=torch.empty((64,), dtype=torch.bfloat16, device="meta")),
+}
+
+
+@pytest.mark.parametrize("rows", [300, 1024])
+@pytest.mark.parametrize("name", list(MISFITS))
+def test_products_of_a_prompt_leave_misfits_to_each_layer(no_launch, monkeypatch, name, rows):
+    """q, k and v together: a layer that does not hold what its sizes say is left to its own call, which refuses it."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops._dense_cache, "get", lambda *a: pytest.fail("an image was asked for") if "bias" not in name else torch.empty(0))
+    mods = [packed_layer(**MISFITS[name]), packed_layer(), packed_layer()]
+    assert ops.quantized_matmul_prompt(dev(bf16(1, rows, 256)), mods) is None
+
+
+def test_products_of_a_prompt_of_fitting_layers_ask_for_their_images(no_launch, monkeypatch):
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    asked = []
+    monkeypatch.setattr(ops._dense_cache, "get", lambda src, key: asked.append(key))
+    for mods in ([packed_layer(), packed_layer()], [packed_layer(bias=bf16(64)), packed_layer()], [packed_layer(bits=3), packed_layer()]):
+        assert ops.quantized_matmul_prompt(dev(bf16(1, 300, 256)), mods) is None      # nothing is resident
+    assert [key[2] for key in asked] == [4, 4, 3]
+    with pytest.raises(AssertionError, match="was reached"):
+        ops.quantized_matmul_prompt(dev(bf16(1, 1024, 256)), [packed_layer(), packed_layer()])
+
+
 @pytest.mark.parametrize("rows", [1, 300, 1024])
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64, torch.int32])
 def test_activations_of_a_packed_product_are_16_bits(no_launch, monkeypatch, rows, dt):
