@@ -111,7 +111,8 @@ class _DecodeGraph:
         self.batch = StepBatch(list(slots), [0] * b, [1] * b, b, i32[2 * b:6 * b].view(b, 4), i32[6 * b:8 * b].view(b, 2), 128,
                                i32[8 * b:10 * b].view(b, 2))
         self.graph = None
-        self.logits = None                               # rows of the output head (``BatchScheduler._head``)
+        self.logits = None                               # rows of the output head (``BatchScheduler._head``) ...
+        self.whole = False                               # ... as it was when they were captured: whether ``_finish`` has to follow
         self.at: Optional[List[int]] = None              # positions that the static tables hold
 
     def fill(self, tokens: Sequence[int], pos0: Sequence[int]) -> None:
@@ -141,8 +142,9 @@ class _DecodeGraph:
         if self.graph is None:
             torch.cuda.synchronize(sched.device)
             g = torch.cuda.CUDAGraph()
+            self.whole = sched._whole_head()
             with graphs.capture(g):
-                self.logits = sched._head(sched.model.forward_tokens(self.tokens, self.batch, sched.caches))
+                self.logits = sched._head(sched.model.forward_tokens(self.tokens, self.batch, sched.caches), self.whole)
             self.graph = g
         self.graph.replay()
         return self.logits
@@ -173,11 +175,13 @@ class BatchScheduler:
         m, t = self.model, type(self.model)
         return (isinstance(m, R) and t.logits is R.logits and t.finish_logits is R.finish_logits and not {"logits", "finish_logits"} & vars(m).keys())
 
-    def _head(self, hidden: torch.Tensor) -> torch.Tensor:
-        return self.model.head_rows(hidden) if self._whole_head() else self.model.logits(hidden)
+    def _head(self, hidden: torch.Tensor, whole: bool) -> torch.Tensor:
+        return self.model.head_rows(hidden) if whole else self.model.logits(hidden)
 
-    def _finish(self, rows: torch.Tensor) -> torch.Tensor:
-        return self.model.finish_logits(rows) if self._whole_head() else rows
+    def _finish(self, rows: torch.Tensor, whole: bool) -> torch.Tensor:
+        """The logits of ``_head``'s rows, by what was decided when these were made (a wrapper put over ``logits`` since then has not seen them)."""
+        from .models.step_model import RaggedStepModel
+        return RaggedStepModel.finish_logits(self.model, rows) if whole else rows
 
     def position(self, seq_id) -> int:
         return self.slots.length[self.slot_of[seq_id]]
@@ -192,9 +196,9 @@ class BatchScheduler:
         [wanted, vocab]."""
         return self._step(entries, want)
 
-    def _step(self, entries, want=None, raw: bool = False) -> torch.Tensor:
-        """``raw``: the output head's rows as they are, of every entry's last token; the caller finishes them and is done with them before the next step, whose
-        replay may overwrite them."""
+    def _step(self, entries, want=None, raw: bool = False):
+        """``raw``: the output head's rows as they are, of every entry's last token, and whether they are still to be finished; the caller is done with them before the
+        next step, whose replay may overwrite them."""
         if not entries:
             return torch.empty((0, 0))
         new_tokens = sum(len(t) for _, t in entries)
@@ -209,13 +213,13 @@ class BatchScheduler:
         pos0 = [self.slots.length[s] for s in slot]
         n_new = [len(t) for _, t in entries]
         if self.use_graphs and all(n == 1 for n in n_new) and len(slot) <= 256:
-            logits = self._graph_step(tuple(slot), [ts[0] for _, ts in entries], pos0)
-            if logits is not None:
+            g = self._graph_step(tuple(slot), [ts[0] for _, ts in entries], pos0)
+            if g is not None:
                 for s in slot:
                     self.slots.length[s] += 1
                 if raw:
-                    return logits
-                buffer, logits = logits, self._finish(logits)
+                    return g.logits, g.whole
+                buffer, logits = g.logits, self._finish(g.logits, g.whole)
                 rows = [i for i in range(len(slot)) if want is None or len(want[i])]
                 if any(p != 0 for i in rows if want is not None for p in want[i]):
                     raise ValueError("a wanted place lies outside the entry's tokens")
@@ -248,8 +252,9 @@ class BatchScheduler:
         if not rows:
             return torch.empty((0, self.model.args.vocab), dtype=torch.float32, device=self.device)
         idx = torch.tensor(rows, dtype=torch.long, device=self.device)
-        out = self._head(hidden.index_select(0, idx))
-        return out if raw else self._finish(out).float()
+        whole = self._whole_head()
+        out = self._head(hidden.index_select(0, idx), whole)
+        return (out, whole) if raw else self._finish(out, whole).float()
 
     def _current_graph(self, slots: Tuple[int, ...], longest: int) -> Optional["_DecodeGraph"]:
         """The captured step of these slots, dropped with all others where a table it reads has moved."""
@@ -266,7 +271,7 @@ class BatchScheduler:
 
     def _step_ahead(self, ids: Sequence[object], tokens: torch.Tensor):
         """The next step of the sequences ``ids``, enqueued before the host has seen their tokens: (the tokens on their way to the host, the event behind that copy,
-        the output head's rows), or None where that step has to be laid out on the host."""
+        the output head's rows, whether they are still to be finished), or None where that step has to be laid out on the host."""
         if not (self.use_graphs and 0 < len(ids) <= 256 and isinstance(tokens, torch.Tensor) and tokens.device == self.device and tokens.dtype in (torch.int64, torch.int32)
                 and tokens.numel() == len(ids) and all(i in self.slot_of for i in ids)):
             return None
@@ -289,9 +294,9 @@ class BatchScheduler:
         rows = g.run(self)
         for s in slots:
             self.slots.length[s] += 1
-        return host, there, rows
+        return host, there, rows, g.whole
 
-    def _graph_step(self, slots: Tuple[int, ...], tokens: Sequence[int], pos0: Sequence[int]) -> Optional[torch.Tensor]:
+    def _graph_step(self, slots: Tuple[int, ...], tokens: Sequence[int], pos0: Sequence[int]) -> Optional["_DecodeGraph"]:
         """Replay (or, at the third step of this set of slots, capture) the decode graph; None: run the step eagerly."""
         g = self._current_graph(slots, max(pos0) + 1)
         if 0 in self._buffers:
@@ -305,7 +310,8 @@ class BatchScheduler:
             g = self._graphs[slots] = _DecodeGraph(self, slots)
             self._seen.pop(slots, None)
         g.fill(tokens, pos0)
-        return g.run(self)
+        g.run(self)
+        return g
 
     @torch.no_grad()
     def generate(self, prompts: Sequence[Sequence[int]], max_tokens: int = 64,
@@ -321,24 +327,25 @@ class BatchScheduler:
         out: List[List[int]] = [[] for _ in prompts]
         live = list(range(len(prompts)))
         feed = {i: list(prompts[i]) for i in live}
-        rows = None                                     # the output head's rows of a step that is under way already
+        rows, whole = None, False                       # the output head's rows of a step that is under way already, and whether they are still to be finished
+        # A step that someone put in the place of the scheduler's is called as it is, from the first on that is not under way.
+        plain = lambda: getattr(self.step, "__func__", None) is _PLAIN_STEP
         while live:
-            # log-probabilities are a tensor of their own: the plain step's rows need not outlive its next replay.  A step that someone put in its place is called as it is.
-            plain = getattr(self.step, "__func__", None) is _PLAIN_STEP
-            if plain:
-                rows = self._step([(ids[i], feed[i]) for i in live], raw=True) if rows is None else rows
-                whole = self._whole_head()
-                logprobs = log_probabilities(rows, (1.0 if self.model.logit_scale is None else self.model.logit_scale) if whole else 1.0)
+            # log-probabilities are a tensor of their own: the plain step's rows need not outlive its next replay
+            if rows is None and plain():
+                rows, whole = self._step([(ids[i], feed[i]) for i in live], raw=True)
+            if rows is not None:
+                logprobs = log_probabilities(rows, self.model.logit_scale if whole and self.model.logit_scale is not None else 1.0)
             else:
                 logprobs = log_probabilities(self.step([(ids[i], feed[i]) for i in live]))
             toks = sampler(logprobs).reshape(-1)
             # Where every sequence goes on, unless a token ends it, the next step is enqueued behind the tokens before the host reads them: the chip does not wait for the host's
             # turn (some 40 us a step).  A sequence that a token has ended then has run one step too many, in a slot that is given back.
-            ahead = self._step_ahead([ids[i] for i in live], toks) if plain and all(len(out[i]) + 1 < max_tokens for i in live) else None
+            ahead = self._step_ahead([ids[i] for i in live], toks) if plain() and all(len(out[i]) + 1 < max_tokens for i in live) else None
             if ahead is None:
                 values, rows = toks.tolist(), None
             else:
-                host, there, rows = ahead
+                host, there, rows, whole = ahead
                 there.synchronize()
                 values = host.tolist()
             nxt, kept = [], []

@@ -148,3 +148,54 @@ def test_a_token_that_is_none_and_does_not_stop_raises():
     with pytest.raises(ValueError, match="neither a stop token"):
         engine.generate([[1, 2, 3]], max_tokens=20, sampler=sampler)
     assert n[0] == 8
+
+
+@pytest.mark.parametrize("at_capture", [False, True])
+def test_a_captured_step_is_finished_as_it_was_captured(at_capture):
+    """``logits`` set on a model whose step is captured already, or taken off again: what the replay's rows still lack does not change."""
+    cfg = S.tugolix_config(width=256, delta=dict(heads=4, kv_heads=2, dim=64, vdim=64, conv=4), gla=dict(heads=2, dim=64, vdim=128, tau=16.0),
+                           latent=dict(heads=4, dim=64, vdim=64, kv_rank=128), ff=512, moe=dict(experts=8, top=2, ff=128, groups=(4, 2)), pattern="dgls")
+    cfg["logit_scale"] = 0.5
+    model = S.build_tugolix(cfg, device="cuda:0", seed=3)
+    assert model.logit_scale == 0.5
+    plain = model.logits
+
+    def toggle(on):
+        if on:
+            model.logits = lambda x: plain(x)
+        else:
+            model.__dict__.pop("logits", None)
+
+    toggle(at_capture)
+    engine, twin = BatchScheduler(model), BatchScheduler(model)
+    twin.use_graphs = False
+    for i in range(8):
+        if i == 5:                                                # (a graph replays from the third single-token step on)
+            assert engine._graphs and all(g.graph is not None for g in engine._graphs.values())
+            toggle(not at_capture)
+        entries = [("a", [3 + i]), ("b", [40 - i])]
+        got, want = engine.step(entries), twin.step(entries)
+        assert torch.equal(got, want)
+
+
+def test_a_step_replaced_on_the_way():
+    """A step that a sampler puts in place of the scheduler's takes over at once, and each token is consumed once."""
+    model, vocab = _model("tugolix")
+    forced = torch.randint(0, vocab, (12,), generator=torch.Generator().manual_seed(8)).tolist()
+    seen = {}
+    for replace in (False, True):
+        engine, n = BatchScheduler(model), [0]
+        rows, fed = seen.setdefault(replace, []), []
+
+        def sampler(lp):
+            rows.append(lp)
+            n[0] += 1
+            if replace and n[0] == 8:
+                inner = engine.step
+                engine.step = lambda entries: (fed.extend(t for _, ts in entries for t in ts), inner(entries))[1]
+            return torch.tensor([forced[n[0] - 1]], device="cuda:0")
+
+        assert engine.generate([[5, 6, 7]], max_tokens=12, sampler=sampler) == [forced]
+        assert fed == ([] if not replace else forced[7:11])
+    for x, y in zip(*seen.values()):
+        assert (x - y).abs().max() <= 0.05 * y.std()              # (the bound of the comparison above)
