@@ -282,7 +282,11 @@ class BatchScheduler:
             return None
         slots = tuple(self.slot_of[i] for i in ids)
         at = [self.slots.length[s] - 1 for s in slots]
-        g = self._current_graph(slots, max(at) + 2)
+        # tables grow, and captured steps are dropped, behind the host's look at the tokens: a sequence that ends here needs no row more, and nothing runs then
+        longest = max(at) + 2
+        if not all(c.holds(longest) if hasattr(c, "holds") else not hasattr(c, "ensure") for c in self.caches):
+            return None
+        g = self._current_graph(slots, longest)
         if g is None or g.graph is None or g.at != at:
             return None
         tokens = tokens.contiguous()

@@ -231,6 +231,10 @@ class SlotKVCache:
         if self.keys is not None:
             self.reserve(longest, self.keys.dtype, self.keys.device)
 
+    def holds(self, longest: int) -> bool:
+        """Whether ``ensure(longest)`` leaves the table where it is."""
+        return self.keys is None or self.window is not None or longest <= self.ring
+
     def grow(self, n_slots: int) -> None:
         if self.keys is not None and self.keys.shape[0] < n_slots:
             old_k, old_v = self.keys, self.values
@@ -285,6 +289,9 @@ class SharedLatentRows:
 
     def ensure(self, longest: int) -> None:
         self.source.ensure(longest)
+
+    def holds(self, longest: int) -> bool:
+        return self.source.holds(longest)
 
     def is_trimmable(self):
         return False
@@ -411,6 +418,9 @@ class CacheGroup:
         for c in self._leaves():
             if hasattr(c, "ensure"):
                 c.ensure(longest)
+
+    def holds(self, longest: int) -> bool:
+        return all(c.holds(longest) if hasattr(c, "holds") else not hasattr(c, "ensure") for c in self._leaves())
 
     def is_trimmable(self):
         return False

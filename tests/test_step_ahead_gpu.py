@@ -199,3 +199,59 @@ def test_a_step_replaced_on_the_way():
         assert fed == ([] if not replace else forced[7:11])
     for x, y in zip(*seen.values()):
         assert (x - y).abs().max() <= 0.05 * y.std()              # (the bound of the comparison above)
+
+
+def _ring(engine):
+    leaves = [leaf for c in engine.caches for leaf in (c._leaves() if hasattr(c, "_leaves") else [c])]
+    rings = {leaf.ring for leaf in leaves if getattr(leaf, "window", 0) is None}
+    assert len(rings) == 1
+    return rings.pop()
+
+
+@pytest.mark.parametrize("name", ["tugolix", "gibalorn"])
+def test_tables_do_not_grow_for_a_token_that_ends_the_last_sequence(name):
+    """A table of 256 rows holds a sequence whose last fed token takes row 255; the end mark behind it needs none."""
+    model, vocab = _model(name)
+    stop, engine, n = vocab - 1, BatchScheduler(model), [0]
+
+    def sampler(lp):
+        n[0] += 1
+        return torch.tensor([stop if n[0] == 7 else n[0]], device="cuda:0")
+
+    assert engine.generate([list(range(1, 251))], max_tokens=20, sampler=sampler, stop_tokens=[stop]) == [[1, 2, 3, 4, 5, 6, stop]]
+    assert _ring(engine) == 256
+
+
+@pytest.mark.parametrize("name", ["tugolix", "gibalorn"])
+def test_sequences_outgrow_their_tables_while_steps_go_ahead(name):
+    """The step that needs the 257th row waits for the host, which moves the tables; the steps behind it go ahead again."""
+    model, vocab = _model(name)
+    steps = 24
+    gen = torch.Generator().manual_seed(11)
+    prompts = [torch.randint(0, vocab, (n,), generator=gen).tolist() for n in (247, 31)]
+    forced = torch.randint(0, vocab, (steps, 2), generator=gen)
+    runs = []
+    for ahead in (True, False):
+        engine = BatchScheduler(model)
+        took, inner = [], engine._step_ahead
+
+        def counted(ids, toks):
+            got = inner(ids, toks) if ahead else None
+            took.append(got is not None)
+            return got
+
+        engine._step_ahead = counted
+        rows, n = [], [0]
+
+        def sampler(lp):
+            rows.append(lp)
+            n[0] += 1
+            return forced[n[0] - 1].to("cuda:0")
+
+        assert engine.generate(prompts, max_tokens=steps, sampler=sampler) == forced.t().tolist()
+        assert _ring(engine) == 512
+        # token i is fed at place 247 + i; a set of slots is captured at its third single-token step, before and after the tables have moved
+        assert [i for i, t in enumerate(took) if t] == ([3, 4, 5, 6, 7, 8] + list(range(12, steps - 1)) if ahead else [])
+        runs.append(rows)
+    for x, y in zip(*runs):
+        assert (x - y).abs().max() <= 0.05 * y.std()              # (the bound of the comparison above)
