@@ -111,13 +111,14 @@ def _cache_takes(cache, k: torch.Tensor, v: torch.Tensor) -> bool:
 def rope_and_update_cache(rope, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache, start):
     """``q, k = rope(q, offset=start), rope(k, offset=start); k, v = cache.update_and_fetch(k, v)`` (qllama.py:84-91).  A prompt chunk on
     the GPU does all of it in ONE launch (gbx_rope_qkv), the same bits; what that does not take goes step by step."""
+    from .. import ops
+    from .rope_utils import PLAIN_FORWARDS
     if (_rope_in_launch(rope, k, v, cache, start) and q.dtype == k.dtype and q.device == k.device and v.device == k.device and q.shape[0] == k.shape[0]
             and q.shape[2:] == k.shape[2:] and v.shape == k.shape and q.stride(3) == 1 and all(q.stride(i) % 8 == 0 for i in (0, 1, 2))
-            and q.data_ptr() % 16 == 0 and not rope._forward_hooks and not rope._forward_pre_hooks):
+            and q.data_ptr() % 16 == 0 and ops.plain_call(rope, PLAIN_FORWARDS[type(rope)])):
         prev = cache.offset
         cache.reserve(k.shape[2], k, v)
         if _cache_takes(cache, k, v):
-            from .. import ops
             out = ops.rope_qkv(q, k, v, cache.keys, cache.values, rope.inv_freq, start, prev, getattr(rope, "scale", 1.0), rope.traditional)
             if out is not None:
                 cache.offset = prev + k.shape[2]

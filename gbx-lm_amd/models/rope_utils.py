@@ -79,6 +79,9 @@ class Llama3RoPE(nn.Module):
         return apply_rope(x, self.inv_freq, offset, 1.0, self.traditional)
 
 
+PLAIN_FORWARDS = {cls: cls.forward for cls in (RoPE, Llama3RoPE)}      # (as they are written here: see ops.plain_call)
+
+
 class SuScaledRotaryEmbedding(nn.Module):
     """Phi-3 "su" / longrope embedding (gbx_lm/models/su_rope.py:11-65): per-frequency ``long_factor`` stretches the
     rotary periods and the input is scaled by sqrt(1 + ln(max / original) / ln(original)) (or ``long_mscale``) before

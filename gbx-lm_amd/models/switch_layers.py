@@ -120,12 +120,15 @@ class SwitchGLU(nn.Module):
         return y.squeeze(-2)
 
 
+_GLU_FORWARD, _PACKED_FORWARD = SwitchGLU.forward, QuantizedSwitchLinear.forward
+
+
 def mixed_experts(experts: nn.Module, x: torch.Tensor, indices: torch.Tensor, scores: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``moe_combine(experts(x, indices), scores, residual)``; of a few tokens the last products and their sum in one launch, unless something watches or
     replaces a module on the way."""
     down = getattr(experts, "down_proj", None)
     if (type(experts) is SwitchGLU and type(down) is QuantizedSwitchLinear and x.is_cuda and indices.numel() <= 64
-            and not any(m._forward_hooks or m._forward_pre_hooks for m in (experts, down))):
+            and ops.plain_call(experts, _GLU_FORWARD) and ops.plain_call(down, _PACKED_FORWARD)):
         act = experts._activated(x, indices)
         y = ops.gather_mix(act, down, indices, scores, residual)
         return y if y is not None else ops.moe_combine(down(act, indices).squeeze(-2), scores, residual)
