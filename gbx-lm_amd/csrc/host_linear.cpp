@@ -25,7 +25,8 @@ GroupsFn groups_fn = nullptr;
 typedef int (*GroupsWinFn)(int64_t, int32_t, int32_t, int32_t, int32_t);
 GroupsWinFn groups_win_fn = nullptr;
 
-constexpr int64_t FEW_ROWS = 256;          // from here on a resident image of the weight may be the faster operand (ops.py decides)
+// From the first on a resident image of the weight goes before groups of 32, from the second on these do wherever they win; what they do not take is decided in ops.py.
+constexpr int64_t FEW_ROWS = 256, MANY_ROWS = 1024;
 constexpr int F16 = 0, BF16 = 1;
 
 bool plain(const at::Tensor& t, at::Device device) {
@@ -50,7 +51,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-// few_rows(x, qweight, scales, zeros, group_size, bits, bias or None[, whether 256 rows and more may go as groups of 32]) -> y, None (not a call for this path) or the library's error code
+// few_rows(x, qweight, scales, zeros, group_size, bits, bias or None[, whether 256 to 1023 rows may go as groups of 32]) -> y, None (not a call for this path) or the library's error code
 PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   if ((n_args != 7 && n_args != 8) || !forward_fn) Py_RETURN_NONE;
@@ -75,7 +76,7 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   const int64_t m = x.numel() / k;
   // rows of several sequences keep the order of sums that they had (see quantized_matmul in ops.py)
   const bool grouped = m > 32 && !(x.dim() == 3 && x.size(0) > 1) && groups_win_fn(m, static_cast<int32_t>(n), static_cast<int32_t>(k), static_cast<int32_t>(bits), static_cast<int32_t>(group));
-  if (m < 1 || (m >= FEW_ROWS && (!grouped || n_args < 8 || args[7] != Py_True))) Py_RETURN_NONE;
+  if (m < 1 || (m >= FEW_ROWS && (!grouped || (m < MANY_ROWS && (n_args < 8 || args[7] != Py_True))))) Py_RETURN_NONE;
   const void* bias = nullptr;
   if (has_bias) {
     const at::Tensor& b = THPVariable_Unpack(args[6]);

@@ -225,7 +225,9 @@ hipError_t launch_qgemm_rows(const MfmaArgs& a, int bits, bool bf16, hipStream_t
 //   K 256 and 768, 16 tiles: 100 rows of 16384 17.3 | 10.3 to 15.4, 20.4 | 12.9 to 20.0; 32 tiles 16.6 | 19.1 to 28.9, 24.6 | 24.6 to 38.1
 //   3 bits, group 64, 16 tiles: 512 rows 4096 x 4096 41.5 | 39.3, 1000 2048 x 2048 32.8 | 25.7; 19 to 24 tiles 52 | 54, 55 | 67; K 1152, 12 tiles 18.6 | 20.8
 //   groups of 32: 8 tiles 128 rows 8192 x 3072 27.6 | 21.1, 65 11008 x 4096 33.2 | 33.3; 10 tiles 36.6 | 38.2; 3 bits, 5 tiles 29.5 | 27.8, 8 tiles 30.3 | 32.3
-//   from 1024 rows on, where few outputs leave the image's tiles few: 1024 rows 1024 x 4096 (8 tiles) 26.3 | 21.3, 2000 200 x 3072 (3) 24.7 | 13.2; 1500 1024 x 4096 (12) 31.5 | 33.4
+//   from 1024 rows on, where few outputs leave the image's tiles few: 1024 rows 1024 x 4096 (8 tiles) 26.3 | 21.3, 2000 200 x 3072 (3) 24.7 | 13.2; 1500 1024 x 4096 (12) 31.5 | 33.4;
+//   by an image that is there already, 4 bits, group 128 and 3 bits, group 64: 1024 rows 1024 x 4096 26.5 | 21.6, 25.9 | 25.4; 1024 x 1024 18.6 | 9.0, 18.6 | 10.8; 1024 x 256 9.8 |
+//   5.6, 9.8 | 6.9; 4096 rows 256 x 4096 26.2 | 21.1, 25.8 | 25.0; 64 x 4096, group 32, 23.3 | 15.8, 3 bits 23.3 | 23.4
 static bool groups_win(int64_t M, int N, int K, int bits, int log2g) {
   const int64_t groups = (M + 31) / 32, tiles = (N + 15) / 16;
   const int dear = log2g == 5 ? (bits == 3 ? 5 : 8) : bits == 3 && log2g == 6 ? (K >= 2048 ? 16 : 8) : K >= 3072 ? 32 : K >= 1536 ? 16 : 8;

@@ -212,7 +212,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise NotImplementedError("quantized_matmul(transpose=False) is not on the QuantizedLinear path")
     if out is None:
         few = _few_rows or _bind_few_rows()
-        y = few(x, w, scales, biases, group_size, bits, bias, not _dense_cache.entries)      # (256 rows on: only while no weight has a resident image)
+        y = few(x, w, scales, biases, group_size, bits, bias, not _dense_cache.entries)      # (256 to 1023 rows: only while no weight has a resident image)
         if y is not None:
             if type(y) is int:
                 _lib.check(y)
@@ -258,7 +258,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise ValueError("out must be a contiguous [M, N] tensor of the activation dtype")
     bias_ptr = bias.data_ptr() if bias is not None else None
     L = _lib.lib()
-    # 33 rows on as groups of 32 side by side, where that is faster and the weight has no resident image.  Rows of several sequences (a leading size over 1) keep the kernel and the
+    # 33 rows on as groups of 32 side by side, where that is faster.  Rows of several sequences (a leading size over 1) keep the kernel and the
     # order of sums that they had: a batch's caches are what its later steps are compared by, and two roundings drift apart over a stack of layers.
     several = len(xshape) == 3 and xshape[0] > 1
 
@@ -269,7 +269,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
             _lib.check(rc)
         return rc == 0
 
-    if m < 256 and groups():
+    # (from 1024 rows on whether an image is resident or not, so that a layer's way and its bits do not depend on what ran before; below, the image of an earlier call is taken first)
+    if (m < 256 or m >= 1024) and groups():
         return out if len(xshape) == 2 else out.reshape(*xshape[:-1], n)
     # scratch: decode batches / short prompts split k across workgroups, long prompts dequantise once
     need = L.gbx_qlinear_workspace_bytes(m, n, k, bits, group_size) if (2 <= m <= 32 or m > 64) else 0
@@ -301,8 +302,6 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         # prompt-sized call on the dense path: the [N, K] image is built once (gbx_dequantize), kept resident, and every call
         # runs the GEMM alone (gbx_dense_forward_ws: k split over workgroups with fp32 scratch for few-tile shapes)
         dense = _dense_cache.get(src, ckey)
-        if dense is None and groups():
-            return out.reshape(*xshape[:-1], n)
         if dense is None:
             dense = _alloc_dense((n, k), x.dtype, x.device)
             if dense is not None:
@@ -316,7 +315,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
                                         m, n, k, _DT[x.dtype], scratch.data_ptr() if part else None, part, _stream_ptr(x.device))
             if rc == _lib.GBX_OK:
                 return out.reshape(*x.shape[:-1], n)
-    if not cacheable and groups():
+    if m < 1024 and groups():
         return out.reshape(*xshape[:-1], n)
     if need:
         ws = torch.empty((need,), dtype=torch.uint8, device=x.device)

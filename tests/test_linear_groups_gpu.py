@@ -79,7 +79,7 @@ def test_what_it_does_not_take():
 @pytest.mark.parametrize("rows", [33, 100, 255, 256, 600, 2000])
 @pytest.mark.parametrize("native", [True, False])
 def test_calls(monkeypatch, rows, native):
-    """Rows of one sequence go that way, by the native call and by the general one; those of several keep theirs, and 256 rows on whose weight has a resident image."""
+    """Rows of one sequence go that way, by the native call and by the general one; those of several keep theirs, and 256 to 1023 rows whose weight has a resident image."""
     k, n = 2048, 512
     w, s, z, bias = _layer(n, k, 4, 128, torch.bfloat16, rows, bias=True)
     if not native:
@@ -124,3 +124,22 @@ def test_layers_of_one_input(bits, group, k, rows):
     assert all(torch.equal(y[0], q(x)) for y, q in zip(one, mods))
     for y, v in zip(ops.quantized_matmul_multi(x[:, None], mods), one):
         assert ((y[:, 0].double() - v[0].double()).abs() <= 2.0 ** -6 * v[0].double().abs() + 0.05).all()
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("rows,n,k,bits,group", [(1024, 1024, 1024, 4, 128), (2000, 200, 3072, 3, 64), (4096, 64, 4096, 2, 32), (1025, 500, 128, 4, 32)])
+def test_many_rows_go_one_way_whatever_is_resident(monkeypatch, native, rows, n, k, bits, group):
+    """From 1024 rows on the bits of a layer do not depend on an image that an earlier call has left, its own or another's."""
+    w, s, z, _ = _layer(n, k, bits, group, torch.bfloat16, rows)
+    if not native:
+        monkeypatch.setattr(ops, "_few_rows", lambda *a: None)
+    x = torch.randn((rows, k), generator=torch.Generator().manual_seed(rows)).bfloat16().to(DEV)
+    call = lambda: ops.quantized_matmul(x, w, s, z, group_size=group, bits=bits)
+    ops.dense_cache_clear()
+    want = _groups(x, w, s, z, None, bits, group, always=0)
+    assert torch.equal(call(), want) and ops.dense_cache_bytes() == 0
+    other = _layer(n, k, bits, group, torch.bfloat16, rows + 1)[:3]
+    for t in (other, (w, s, z)):
+        ops._dense_cache.put(t, (n, k, bits, group, x.dtype, x.device.index), ops.dequantize(*t, group, bits))
+        assert torch.equal(call(), want)
+    ops.dense_cache_clear()
