@@ -40,6 +40,12 @@ bool watched() {                            // something is to see every operati
          c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
+// A launch waits where the queue is full: other threads run meanwhile, as they do during a foreign call.
+struct WithoutLock {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutLock() { PyEval_RestoreThread(state); }
+};
+
 PyObject* bind(PyObject*, PyObject* args) {
   unsigned long long f, w, s, g, gw;
   if (!PyArg_ParseTuple(args, "KKKKK", &f, &w, &s, &g, &gw)) return nullptr;
@@ -90,20 +96,28 @@ PyObject* few_rows(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
   const int act = type == at::kBFloat16 ? BF16 : F16;
   const int32_t N = static_cast<int32_t>(n), K = static_cast<int32_t>(k), B = static_cast<int32_t>(bits), G = static_cast<int32_t>(group);
+  const void *px = x.const_data_ptr(), *pw = w.const_data_ptr(), *ps = sc.const_data_ptr(), *pz = ze.const_data_ptr();
+  void* py = y.mutable_data_ptr();
+  int rc;
   if (grouped) {
-    const int rc = groups_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, 0, stream);
+    {
+      WithoutLock free;
+      rc = groups_fn(px, pw, ps, pz, bias, py, m, N, K, B, G, act, 0, stream);
+    }
     if (rc == 0) return THPVariable_Wrap(std::move(y));
     if (rc != 1) return PyLong_FromLong(rc);
     if (m >= FEW_ROWS) Py_RETURN_NONE;
   }
   // scratch: decode batches and short prompts split k across workgroups
   const size_t need = (m >= 2 && m <= 32) || m > 64 ? workspace_fn(m, N, K, B, G) : 0;
-  int rc;
   if (need) {
     at::Tensor ws = at::empty({static_cast<int64_t>(need)}, x.options().dtype(at::kByte).requires_grad(false));
-    rc = forward_ws_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, ws.mutable_data_ptr(), need, stream);
+    void* pws = ws.mutable_data_ptr();
+    WithoutLock free;
+    rc = forward_ws_fn(px, pw, ps, pz, bias, py, m, N, K, B, G, act, pws, need, stream);
   } else {
-    rc = forward_fn(x.const_data_ptr(), w.const_data_ptr(), sc.const_data_ptr(), ze.const_data_ptr(), bias, y.mutable_data_ptr(), m, N, K, B, G, act, stream);
+    WithoutLock free;
+    rc = forward_fn(px, pw, ps, pz, bias, py, m, N, K, B, G, act, stream);
   }
   if (rc) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(y));

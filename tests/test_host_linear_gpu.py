@@ -86,3 +86,21 @@ def test_other_streams():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(held, ops.quantized_matmul(x, w, s, z, group_size=128, bits=4))
+
+
+@pytest.mark.parametrize("rows,k", [(1, 256), (16, 4096), (40, 256), (100, 8192)])
+def test_other_threads_run_during_a_launch(rows, k):
+    """The launch is called without the interpreter's lock: a stand-in answers whether its thread holds it (0: no error, the call's result; 1: an error code)."""
+    import ctypes
+    L, host = _lib.lib(), _lib.host()
+    w, s, z = _layer(64, k, 4, 64, torch.bfloat16)
+    x = torch.randn((rows, k), device="cuda", dtype=torch.bfloat16)
+    at = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    holds = at(ctypes.pythonapi.PyGILState_Check)
+    real = [at(f) for f in (L.gbx_qlinear_forward, L.gbx_qlinear_forward_ws, L.gbx_qlinear_workspace_bytes, L.gbx_qlinear_groups, L.gbx_qlinear_groups_win)]
+    try:
+        host.bind(holds, holds, real[2], holds, real[4])
+        got = host.few_rows(x, w, s, z, 64, 4, None)
+    finally:
+        host.bind(*real)
+    assert isinstance(got, torch.Tensor)
