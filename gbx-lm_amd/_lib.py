@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import os
 import subprocess
+import sys
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 from . import env as _env  # noqa: E402
@@ -24,7 +25,7 @@ _xlib = None
 
 def build(force: bool = False, jobs: int = 8) -> str:
     """Compile every HIP source for gfx950 in-tree (hipcc cross-compiles without a GPU)."""
-    cmd = ["make", "-C", _CSRC, f"-j{jobs}"]
+    cmd = ["make", "-C", _CSRC, f"-j{jobs}", f"PY={sys.executable}"]
     if force:
         cmd.append("-B")
     subprocess.check_call(cmd, stdout=subprocess.DEVNULL)
@@ -425,13 +426,20 @@ def build_mixers(force: bool = False, jobs: int = 8) -> str:
 _host = None
 
 
+def host_so_path() -> str:
+    """The native module's file for this torch and this interpreter (csrc/Makefile gives it that name)."""
+    import sysconfig
+    import torch
+    return os.path.join(_CSRC, f"_gbx_host-{torch.__version__}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
 def host():
-    """The host side of small calls as a native module (csrc/host_linear.cpp), bound to the library's entry points; None where it is not built (it is compiled against one
-    torch and one interpreter), and the calls then go through ctypes."""
+    """The host side of small calls as a native module (csrc/host_linear.cpp), bound to the library's entry points; None, with a warning, where it is not built for this torch
+    and this interpreter or does not load, and the calls then go through ctypes."""
     global _host
     if _host is None:
-        _host = False
-        path = os.path.join(_CSRC, "_gbx_host.so")
+        path, why = host_so_path(), "is not built (`make -C gbx-lm_amd/csrc`)"
+        mod = None
         if os.path.exists(path):
             import importlib.util
             L = lib()
@@ -439,8 +447,13 @@ def host():
             try:
                 mod = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(mod)
-            except ImportError:
-                return None
+            except ImportError as e:
+                mod, why = None, f"does not load ({e})"
+        if mod is None:
+            import warnings
+            warnings.warn(f"gbx_lm_amd: {os.path.basename(path)} {why}; calls of few rows go through ctypes, slower", RuntimeWarning, stacklevel=2)
+            _host = False
+        else:
             mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.gbx_qlinear_forward, L.gbx_qlinear_forward_ws, L.gbx_qlinear_workspace_bytes, L.gbx_qlinear_groups,
                                                                           L.gbx_qlinear_groups_win)))
             _host = mod
