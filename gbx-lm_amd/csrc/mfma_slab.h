@@ -1,4 +1,5 @@
-// Quantised products of up to 32 rows (one matrix: 1023, in groups) that fit the registers, contractions of 1024 to 4096 (kernel: mfma_slab_impl.h, one unit per width; launch: mfma_rows.hip).
+// Quantised products whose rows fit the registers (kernel: mfma_slab_impl.h, one unit per width; launch: mfma_rows.hip): up to 32 rows with contractions of 1024 to 4096, more in groups of
+// up to 32 with contractions of 128 to 4096 -- 4096 rows of one matrix, 64 of two or three.
 #pragma once
 #include "mfma_common.h"
 

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(NT) void sink_rows_kernel(const T* __restrict__ q, 
     for (int r = wave; r < nr; r += NW) {           // a wave per head: the tile's maximum, the weights, their sum
       const float s = gl[r * KT + lane];
       float mx = s;
-  mx = wave_max(mx);
+      mx = wave_max(mx);
       const float m_old = ml[r], m_new = fmaxf(m_old, mx);            // mx is finite: a tile holds at least one key
       const float p = exp_<FAST>(s - m_new);
       gl[r * KT + lane] = p;

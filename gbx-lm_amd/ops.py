@@ -190,7 +190,7 @@ _few_rows = None
 
 
 def _bind_few_rows():
-    """The native call of up to 255 rows (csrc/host_linear.cpp); without it nothing is taken there."""
+    """The native call (csrc/host_linear.cpp): up to 255 rows, and up to 4096 where they go as groups of 32; without it nothing is taken there."""
     global _few_rows
     mod = _lib.host() if torch.cuda.is_available() else None
     few = mod.few_rows if mod is not None else lambda *a: None
@@ -207,6 +207,8 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     ``w`` is the packed uint32 ``qweight [N, K*bits/32]``; ``biases`` are the GBA "zeros"
     (already MLX-signed, quantized_linear_gba.py:151-155).  Only ``transpose=True`` exists on
     this path.  Raises ValueError on shape/bits/group violations like the reference's asserts.
+    From 33 rows on x [B > 1, L, K] and the same rows as [B L, K] may take different kernels, whose
+    results agree to the rounding of 16-bit weights and not bit by bit.
     """
     if not transpose:
         raise NotImplementedError("quantized_matmul(transpose=False) is not on the QuantizedLinear path")
@@ -258,8 +260,10 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
         raise ValueError("out must be a contiguous [M, N] tensor of the activation dtype")
     bias_ptr = bias.data_ptr() if bias is not None else None
     L = _lib.lib()
-    # 33 rows on as groups of 32 side by side, where that is faster.  Rows of several sequences (a leading size over 1) keep the kernel and the
-    # order of sums that they had: a batch's caches are what its later steps are compared by, and two roundings drift apart over a stack of layers.
+    # 33 rows on as groups of 32 side by side, where that is faster.  Rows of several sequences ([B > 1, L, K]) keep the tiles of weights rounded to 16 bits and their order of sums: the line
+    # is one of comparability, not of speed or accuracy.  Behind 28 layers of 2 bits another order moves a batch's logits by 0.039 of their norm (4 bits 0.030, 8 layers 0.021), so a batch
+    # would no longer agree to 0.03 with what it gave before.  Tiles | groups: 48 rows of 4096 x 4096, 4 bits, 15.0 | 8.4 us, 100 rows 22.8 | 10.9, 512 rows 38.3 | 30.2; error of the
+    # product against 64 bits 2.2e-3 | 1.7e-3, of the logits behind 8 layers 0.0190 | 0.0176.
     several = len(xshape) == 3 and xshape[0] > 1
 
     def groups() -> bool:
@@ -508,7 +512,7 @@ def quantized_matmul_multi(x: torch.Tensor, mods, pre_norm=None) -> list:
             VP(*[m.zeros.data_ptr() for m in mods]), VP(*[(m.bias.data_ptr() if m.bias is not None else None) for m in mods]),
             VP(*[y.data_ptr() for y in ys]), I32(*[m.output_dims for m in mods]), rows, k, m0.bits, m0.group_size,
             _DT[x.dtype], _stream_ptr(x.device))
-    # over 32 rows of one sequence: the kernel that a call per module takes (quantized_matmul)
+    # over 32 rows of one sequence: the kernel that a call per module takes (quantized_matmul, which says why not those of several)
     rc = _lib.lib().gbx_qlinear_groups_multi(*args) if rows > 32 and not (x.dim() == 3 and x.shape[0] > 1) else 1
     _lib.check(rc if rc != 1 else _lib.lib().gbx_qlinear_forward_multi(*args))
     return [y.reshape(*x.shape[:-1], m.output_dims) for y, m in zip(ys, mods)]
